@@ -5,6 +5,7 @@
 // results (RowsIn::sq): W (r x) = r (W x), so no launch of its own stands between the two.
 #pragma once
 #include "elem.h"
+#include <algorithm>
 
 namespace ad {
 
@@ -101,24 +102,122 @@ __global__ __launch_bounds__(256) void row_kernel(RowsPair rp, E e) {
         if (t == 0) e.sums[blockIdx.x] = (red[4] + red[5]) + (red[6] + red[7]);
     }
 }
-// 2 .. 16 tokens: a workgroup per 16 RG weight rows, its NW waves on interleaved 128-column blocks of the reduction.  Tokens are the
-// rows of A, weight rows the columns of B: both k-contiguous in memory, so fragments come straight from global memory, and the matrix pipe takes the
-// multiply-adds of all tokens at the price of one.  RG = 2 reads the tokens once for 32 weight rows: at 16 tokens they are as many bytes as 16 rows;
-// PAIR: the second 16 are the up rows of the same outputs.
-// (Plain loads: a fragment touches half a cache line of 16 rows and the next one the other half, which a non-temporal hint fetches twice -- 157
-// against 123 us for a 514 MB head at 8 tokens.)
-template <int NW, int RG, class E, bool PAIR>
-__global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, E e) {
-    static_assert(!PAIR || RG == 2, "gate rows beside up rows");
+// 2 .. 16 tokens: a workgroup of NW waves runs through the groups [g0, g1) of 16 weight rows (PAIR: 16 gate rows, then the 16 up rows of the same
+// outputs).  Tokens are the rows of A, weight rows the columns of B: both k-contiguous in memory, so fragments come straight from global memory, and
+// the matrix pipe takes the multiply-adds of all tokens at the price of one.  Wave w owns the KS 32-column steps of the reduction that start at
+// column 32 KS w: its part of the tokens is loaded ONCE and stays in registers, and a weight fragment's register is refilled with the next group's as
+// soon as it is used, so up to 16 kilobytes a wave are in flight without a break between the groups.  The NW partial results meet in LDS (two images in
+// turn: one barrier a group), where a quarter of the threads at a time sums them and calls out(value, up value, token row, weight row, group).
+// (Plain loads: a fragment touches half a cache line of 16 rows and the next one the other half, which a non-temporal hint fetches twice.)
+template <int NW, bool PAIR>
+struct RowsRed {
+    float v[2][PAIR ? 2 : 1][NW][16][17];
+};
+template <int NW, int KS, bool PAIR, class Out>
+__device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, int K, int N, const bf16_t* xp, int g0, int g1, RowsRed<NW, PAIR>& red,
+                                            const Out& out) {
+    constexpr int SUB = PAIR ? 2 : 1, DEPTH = KS <= 16 ? KS : KS / 2;   // fragments in flight
+    static_assert(KS % DEPTH == 0, "a step keeps its register");
+    const int t = threadIdx.x, l = t & 63, w = t >> 6, q4 = l >> 4, c16 = l & 15;
+    // the last waves' windows are moved down into the row, the columns that another wave owns zeroed in the tokens: every address is base + constant
+    const int own = w * KS * 32, k0 = min(own, K - KS * 32) + q4 * 8;
+    xp += k0;
+    u32x4 x[KS], b[DEPTH];
+    const bf16_t* wp = W + (long long)min(g0 * 16 + c16, N - 1) * K + k0;
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) b[u] = ld16(wp + 32 * u);
+#pragma unroll
+    for (int u = 0; u < KS; ++u) x[u] = ld16(xp + 32 * u);
+#pragma unroll
+    for (int u = 0; u < KS; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[u][q] = k0 + 32 * u >= own ? x[u][q] : 0u;
+    for (int g = g0; g < g1; ++g) {
+        const int ph = (g - g0) & 1;
+#pragma unroll
+        for (int sub = 0; sub < SUB; ++sub) {
+            f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+            const bool up_next = PAIR && sub == 0, more = up_next || g + 1 < g1;
+            const bf16_t *cur = wp, *nxt = (up_next ? W2 : W) + (long long)min((up_next ? g : g + 1) * 16 + c16, N - 1) * K + k0;
+            wp = nxt;
+            if (more) {
+#pragma unroll
+                for (int u = 0; u < KS; ++u) {
+                    acc[u & 1] = mfma16(__builtin_bit_cast(s16x8, x[u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[u & 1]);
+                    b[u % DEPTH] = ld16(u + DEPTH < KS ? cur + 32 * (u + DEPTH) : nxt + 32 * (u + DEPTH - KS));
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < KS; ++u) {
+                    acc[u & 1] = mfma16(__builtin_bit_cast(s16x8, x[u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[u & 1]);
+                    if (u + DEPTH < KS) b[u % DEPTH] = ld16(cur + 32 * (u + DEPTH));
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red.v[ph][sub][w][4 * q4 + r][c16] = acc[0][r] + acc[1][r];
+        }
+        sync();
+        if ((t >> 8) == ((g - g0) & (NW / 4 - 1))) {   // (whole waves: 256 sums)
+            const int tok = (t >> 4) & 15, n = t & 15;
+            float v = 0.f, u = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww) {
+                v += red.v[ph][0][ww][tok][n];
+                if (PAIR) u += red.v[ph][SUB - 1][ww][tok][n];
+            }
+            out(v, u, tok, g * 16 + n, g);
+        }
+    }
+}
+// 1 / rms of sixteen tokens from their partial sums of squares, a wave per token
+__device__ __forceinline__ void token_rms(float* rms, const RowsIn& in, int t0, int n_tok, int waves) {
+    const int l = threadIdx.x & 63;
+    for (int i = threadIdx.x >> 6; i < 16 && t0 + i < n_tok; i += waves) {
+        float s = 0.f;
+        for (int j = l; j < in.sq_n; j += 64) s += in.sq[(long long)(t0 + i) * in.sq_n + j];
+        s = wave_sum_bcast(s);
+        if (l == 0) rms[i] = 1.f / sqrtf(s * in.inv_n + in.eps);
+    }
+}
+template <int NW, int KS, class E, bool PAIR>
+__global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, int per, E e) {
+    ARIA_SMEM_STATIC RowsRed<NW, PAIR> red;
+    ARIA_SMEM_STATIC float rms[16];
+    const RowsIn& in = rp.in[blockIdx.z];
+    const int c16 = threadIdx.x & 15, t0 = blockIdx.y * 16, groups = (in.N + 15) / 16, g0 = blockIdx.x * per;
+    if (in.sq) token_rms(rms, in, t0, n_tok, NW);   // (published by the first group's barrier)
+    stream_rows<NW, KS, PAIR>(in.W, in.W2, in.K, in.N, in.X + (long long)min(t0 + c16, n_tok - 1) * in.ldx, g0, min(groups, g0 + per), red,
+                              [&](float v, float u, int tok, int n, int g) {
+                                  const bool in_range = t0 + tok < n_tok && n < in.N;
+                                  float s = 0.f;
+                                  if (in_range) {
+                                      if (in.sq) {
+                                          v *= rms[tok];
+                                          u *= rms[tok];
+                                      }
+                                      if constexpr (PAIR)
+                                          e(v, u, t0 + tok, n);
+                                      else
+                                          s = e(v, t0 + tok, n, int(blockIdx.z));
+                                  }
+                                  if constexpr (E::SUMSQ) {   // sixteen lanes hold a token's outputs
+                                      s = group_sum<16>(s);
+                                      if ((n & 15) == 0 && t0 + tok < n_tok) e.sums[(long long)(t0 + tok) * groups + g] = s;
+                                  }
+                              });
+}
+// any reduction (below a wave's window of stream_rows or beyond what it holds in registers): the 8 waves on interleaved 128-column blocks of it, a workgroup per 16 rows
+template <class E, bool PAIR>
+__global__ __launch_bounds__(512) void rows_long_kernel(RowsPair rp, int n_tok, E e) {
+    constexpr int NW = 8, RG = PAIR ? 2 : 1;
     ARIA_SMEM_STATIC float red[NW][16][16 * RG + 1];
     ARIA_SMEM_STATIC float rms[16];
     const RowsIn& in = rp.in[blockIdx.z];
     const int t = threadIdx.x, l = t & 63, w = t >> 6, q4 = l >> 4, c16 = l & 15, K = in.K, N = in.N;
-    constexpr int OUT = PAIR ? 16 : 16 * RG;
-    const int n0 = blockIdx.x * OUT, t0 = blockIdx.y * 16;
+    const int n0 = blockIdx.x * 16, t0 = blockIdx.y * 16;
     const bf16_t* wp[RG];
 #pragma unroll
-    for (int g = 0; g < RG; ++g) wp[g] = (PAIR && g ? in.W2 : in.W) + (long long)min(n0 + (PAIR ? 0 : 16 * g) + c16, N - 1) * K;
+    for (int g = 0; g < RG; ++g) wp[g] = (g ? in.W2 : in.W) + (long long)min(n0 + c16, N - 1) * K;
     const bf16_t* xp = in.X + (long long)min(t0 + c16, n_tok - 1) * in.ldx;
     f32x4 acc[RG][2];
 #pragma unroll
@@ -144,74 +243,99 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, E
 #pragma unroll
             for (int g = 0; g < RG; ++g) acc[g][u & 1] = mfma16(__builtin_bit_cast(s16x8, a[u]), __builtin_bit_cast(s16x8, b[g][u]), acc[g][u & 1]);
     }
-    if (in.sq) {   // 1 / rms of the tokens, a wave per token
-        for (int i = w; i < 16 && t0 + i < n_tok; i += NW) {
-            float s = 0.f;
-            for (int j = l; j < in.sq_n; j += 64) s += in.sq[(long long)(t0 + i) * in.sq_n + j];
-            s = wave_sum_bcast(s);
-            if (l == 0) rms[i] = 1.f / sqrtf(s * in.inv_n + in.eps);
-        }
-    }
+    if (in.sq) token_rms(rms, in, t0, n_tok, NW);
 #pragma unroll
     for (int g = 0; g < RG; ++g)
 #pragma unroll
         for (int r = 0; r < 4; ++r) red[w][4 * q4 + r][16 * g + c16] = acc[g][0][r] + acc[g][1][r];
     sync();
-    for (int i = t; i < 16 * OUT; i += NW * 64) {   // (whole waves: 16 OUT is a multiple of 64)
-        const int tok = i / OUT, n = i % OUT;
-        const bool in_range = t0 + tok < n_tok && n0 + n < N;
-        float v = 0.f, u = 0.f;
+    if (t >= 256) return;
+    const int tok = t >> 4, n = t & 15;
+    const bool in_range = t0 + tok < n_tok && n0 + n < N;
+    float v = 0.f, u = 0.f, s = 0.f;
 #pragma unroll
-        for (int ww = 0; ww < NW; ++ww) {
-            v += red[ww][tok][n];
-            if (PAIR) u += red[ww][tok][16 + n];
-        }
-        if (in.sq && in_range) {
+    for (int ww = 0; ww < NW; ++ww) {
+        v += red[ww][tok][n];
+        if (PAIR) u += red[ww][tok][16 * (RG - 1) + n];
+    }
+    if (in_range) {
+        if (in.sq) {
             v *= rms[tok];
             u *= rms[tok];
         }
-        float s = 0.f;
-        if (in_range) {
-            if (PAIR)
-                e(v, u, t0 + tok, n0 + n);
-            else
-                s = e(v, t0 + tok, n0 + n, int(blockIdx.z));
-        }
-        if (E::SUMSQ) {
-            static_assert(!E::SUMSQ || OUT == 16, "sixteen lanes hold a token's outputs");
-            s = group_sum<16>(s);
-            if (n == 0 && t0 + tok < n_tok) e.sums[(long long)(t0 + tok) * gridDim.x + blockIdx.x] = s;
-        }
+        if constexpr (PAIR)
+            e(v, u, t0 + tok, n0 + n);
+        else
+            s = e(v, t0 + tok, n0 + n, int(blockIdx.z));
+    }
+    if constexpr (E::SUMSQ) {
+        s = group_sum<16>(s);
+        if (n == 0 && t0 + tok < n_tok) e.sums[(long long)(t0 + tok) * gridDim.x + blockIdx.x] = s;
     }
 }
 
 // workgroups of one problem, i.e. the partial sums per token that an epilogue with SUMSQ leaves
 inline int rows_parts(int64_t T, int64_t N) { return int(T == 1 ? (N + 7) / 8 : (N + 15) / 16); }
 
+// Row groups per workgroup: one round of the 256 CUs.  More workgroups read the tokens more often (7680 x 2560, 16 tokens: 240 workgroups 10.4 us, 480
+// 13.1), fewer leave CUs idle (4448 rows: two groups each on 139 workgroups 9.5 us, one each on 278 -- a second, nearly empty round -- 12.1).
+inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std::max<int64_t>(1, (groups * problems + 255) / 256)); }
+
+// stream_rows' shape for a reduction of K columns: CALL(waves, steps per wave).  The steps of a wave are registers (4 a step for the tokens, as many for
+// up to 16 fragments in flight), rounded up to a few values; OTHER runs beyond 6656 columns, and below 128 (a wave's window).
+// One launch, 16 tokens, this form against rows_long_kernel: 100352 x 2560 112 us (4.6 TB/s) against 147, 7680 x 2560 10.4 against 15.8, 2560 x 2560 6.7
+// against 8.9, 6656 x 2560 9.9 against 15.6; at 2 tokens 97 against 117, 9.1 against 10.6, 5.3 against 6.3, 8.5 against 10.4.  What is left beside the
+// 6.1 TB/s of a plain read is the launch itself (about 4 us until the first results) and the tokens' rows from the L2, once per workgroup.
+#define ARIA_ROWS_SHAPE(K, CALL, OTHER) \
+    if ((K) < 128)                      \
+        OTHER                           \
+    else if ((K) <= 1024)               \
+        CALL(8, 4)                      \
+    else if ((K) <= 1792)               \
+        CALL(8, 7)                      \
+    else if ((K) <= 2560)               \
+        CALL(8, 10)                     \
+    else if ((K) <= 3328)               \
+        CALL(8, 13)                     \
+    else if ((K) <= 4096)               \
+        CALL(8, 16)                     \
+    else if ((K) <= 6656)               \
+        CALL(8, 26)                     \
+    else                                \
+        OTHER
+
+template <bool PAIR, class E>
+int launch_rows_of(const RowsPair& rp, int problems, int64_t T, const E& e, void* stream) {
+    const int64_t groups = (rp.in[0].N + 15) / 16;
+    const int per = rows_per_workgroup(groups, problems), other = rp.in[problems - 1].K;
+    const int K = std::max(rp.in[0].K, other), least = std::min(rp.in[0].K, other);
+    const dim3 grid(unsigned((groups + per - 1) / per), unsigned((T + 15) / 16), unsigned(problems));
+#define ARIA_ROWS_LONG ARIA_LAUNCH((rows_long_kernel<E, PAIR>), dim3(unsigned(groups), grid.y, grid.z), dim3(512), 0, stream, rp, int(T), e);
+#define ARIA_ROWS(NW, KS)                                                                                                     \
+    {                                                                                                                         \
+        if (least >= KS * 32) /* (a wave's window lies inside the shorter reduction too) */                                   \
+            ARIA_LAUNCH((rows_kernel<NW, KS, E, PAIR>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);                  \
+        else                                                                                                                  \
+            ARIA_ROWS_LONG                                                                                                    \
+    }
+    ARIA_ROWS_SHAPE(K, ARIA_ROWS, ARIA_ROWS_LONG)
+#undef ARIA_ROWS
+#undef ARIA_ROWS_LONG
+    return aria_check_launch();
+}
+
 template <class E>
 int launch_rows(const RowsPair& rp, int problems, int64_t T, const E& e, void* stream) {
-    const int64_t N = rp.in[0].N;
-    const unsigned z = unsigned(problems), groups = unsigned((T + 15) / 16);
-    if constexpr (!E::SUMSQ) {
-        if (T > 1 && N > 16 * 1024) {
-            ARIA_LAUNCH((rows_kernel<4, 2, E, false>), dim3(unsigned((N + 31) / 32), groups, z), dim3(256), 0, stream, rp, int(T), e);
-            return aria_check_launch();
-        }
-    }
-    if (T == 1)
-        ARIA_LAUNCH((row_kernel<E, false>), dim3(unsigned((N + 7) / 8), 1, z), dim3(256), 0, stream, rp, e);
-    else   // few row groups: more waves per group
-        ARIA_LAUNCH((rows_kernel<8, 1, E, false>), dim3(unsigned((N + 15) / 16), groups, z), dim3(512), 0, stream, rp, int(T), e);
+    if (T > 1) return launch_rows_of<false>(rp, problems, T, e, stream);
+    ARIA_LAUNCH((row_kernel<E, false>), dim3(unsigned((rp.in[0].N + 7) / 8), 1, unsigned(problems)), dim3(256), 0, stream, rp, e);
     return aria_check_launch();
 }
 // gated pair: outputs e(gate, up, token, row)
 template <class E>
 int launch_row_pairs(const RowsIn& in, int64_t T, const E& e, void* stream) {
     const RowsPair rp{{in, in}};
-    if (T == 1)
-        ARIA_LAUNCH((row_kernel<E, true>), dim3(unsigned((in.N + 3) / 4)), dim3(256), 0, stream, rp, e);
-    else
-        ARIA_LAUNCH((rows_kernel<8, 2, E, true>), dim3(unsigned((in.N + 15) / 16), unsigned((T + 15) / 16)), dim3(512), 0, stream, rp, int(T), e);
+    if (T > 1) return launch_rows_of<true>(rp, 1, T, e, stream);
+    ARIA_LAUNCH((row_kernel<E, true>), dim3(unsigned((in.N + 3) / 4)), dim3(256), 0, stream, rp, e);
     return aria_check_launch();
 }
 
