@@ -6,7 +6,7 @@
 // never expands: the query moves into latent space once (q W_uk, per head), scores are dot products with the cache rows as they lie in memory, and
 // the weighted sum of latents is expanded through W_uv at the end.  A cache row is then read ONCE for 16 or 32 heads, which makes decode
 // attention a matrix product with the heads as rows (v_mfma_f32_16x16x32_bf16) whose operand streams from HBM.
-#include "rows.h"
+#include "experts.h"
 #include "tile_attn.h"
 #include <cstdlib>
 
@@ -334,7 +334,8 @@ struct LatentRows {
     }
 };
 
-// routed up-projection of one (token, slot): act = silu(gate . h) * (up . h); the routing runs in front of the rows, workgroup x = 0 publishes it
+// Routed experts of one token (of several: experts.h, with the routing as a launch of its own in front):
+// up-projection of one (token, slot): act = silu(gate . h) * (up . h); the routing runs in front of the rows, workgroup x = 0 publishes it
 __global__ __launch_bounds__(256) void mix_up_kernel(const float* logits, const float* correction, int E, int ldl, int groups, int keep, int k,
                                                      const bf16_t* Wg, const bf16_t* Wu, const bf16_t* X, int K, int F, bf16_t* act, float* weights,
                                                      int32_t* idx) {
@@ -370,6 +371,51 @@ __global__ __launch_bounds__(256) void mix_down_kernel(const bf16_t* Wd, const f
         y1 += wj * acc[1][0];
     }
     if (l < 2 && row0 + l < D) stream_step(l ? y1 : y0, ro.post, ro.next, ro.x, ro.h, (long long)tok * D + row0 + l, row0 + l);
+}
+
+// Several tokens.  Routing and expert lists, one workgroup of 16 waves: a wave per token.
+__global__ __launch_bounds__(1024) void mix_lists_kernel(const float* logits, const float* correction, int E, int ldl, int groups, int keep, int k, int T,
+                                                         float* weights, ExpertLists lists) {
+    ARIA_SMEM_STATIC float lds[16][768];
+    ARIA_SMEM_STATIC ListsLds sl;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int tok = w; tok < T; tok += 16) {
+        float my_w;
+        int my_e;
+        route_group_limited(logits + (long long)tok * ldl, correction, E, groups, keep, k, lds[w], l, 0, my_w, my_e);
+        if (l < k) {
+            weights[tok * k + l] = my_w;
+            sl.idx[tok * k + l] = my_e;
+        }
+        wave_barrier();
+    }
+    write_lists(lists, sl, T * k);
+}
+struct MixAct {
+    bf16_t* act;
+    long long F;
+    __device__ __forceinline__ void operator()(float g, float u, int entry, int n) const { act[entry * F + n] = f2bf(silu_fast(g) * u); }
+};
+struct MixPartial {   // a (token, slot)'s expert output, in 32 bits until the weighted sum
+    float* out;
+    long long D;
+    __device__ __forceinline__ void operator()(float v, float, int entry, int n) const { out[entry * D + n] = v; }
+};
+// the weighted sum of a token's k experts, residual and norms; a thread per stream column
+__global__ __launch_bounds__(256) void mix_combine_kernel(const float* part, const float* weights, int k, int D, RowsOut ro) {
+    const int n = blockIdx.x * 256 + threadIdx.x, tok = blockIdx.y;
+    if (n >= D) return;
+    const float* p = part + (long long)tok * k * D + n;
+    float y = 0.f;
+    for (int j0 = 0; j0 < k; j0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = p[(long long)min(j0 + j, k - 1) * D];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j0 + j < k) y += weights[tok * k + j0 + j] * v[j];
+    }
+    stream_step(y, ro.post, ro.next, ro.x, ro.h, (long long)tok * D + n, n);
 }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -485,9 +531,9 @@ int aria_latent_expand(const float* part_o, const float* part_ml, const AriaLate
 namespace {
 
 struct Scratch {
-    float *x, *part_o, *part_ml, *logits, *weights;
+    float *x, *part_o, *part_ml, *logits, *weights, *eo;
     bf16_t *h, *proj, *qa, *ao, *act;
-    int32_t* idx;
+    int32_t *idx, *table;
     int64_t bytes;
 };
 Scratch layout(const AriaLatentStack& st, const AriaLatentLayer* L, int64_t T, int64_t max_len, char* base) {
@@ -524,6 +570,8 @@ Scratch layout(const AriaLatentStack& st, const AriaLatentLayer* L, int64_t T, i
     z.logits = reinterpret_cast<float*>(take(4 * T * E));
     z.weights = reinterpret_cast<float*>(take(4 * T * k));
     z.idx = reinterpret_cast<int32_t*>(take(4 * T * k));
+    z.table = reinterpret_cast<int32_t*>(take(T > 1 ? 4 * ExpertLists::table_ints(E) : 0));
+    z.eo = reinterpret_cast<float*>(take(T > 1 ? 4 * T * k * st.D : 0));
     z.bytes = at;
     return z;
 }
@@ -581,6 +629,21 @@ int aria_latent_decode(const AriaLatentStack* st, const AriaLatentLayer* L, int6
             RowsOut lg{z.logits, (long long)ldl, none, none, nullptr, nullptr};
             rc = rows<ROWS_F32>(y.w_router, z.h, D, D, y.E, T, lg, stream);
             if (rc != ARIA_OK) break;
+            if (expert_rows_take(D, y.ff, y.E, y.k, T)) {
+                const ExpertLists lists{z.table, z.idx, int(y.E)};
+                ARIA_LAUNCH(mix_lists_kernel, dim3(1), dim3(1024), 0, stream, (const float*)z.logits, y.correction, int(y.E), int(ldl), int(y.groups),
+                            int(y.keep), int(y.k), int(T), z.weights, lists);
+                const ExpertIn up{static_cast<const bf16_t*>(y.w_gate), static_cast<const bf16_t*>(y.w_up), z.h, (long long)D, int(y.k), int(D), int(y.ff)};
+                const ExpertIn down{static_cast<const bf16_t*>(y.w_down), nullptr, z.act, (long long)y.ff, 1, int(y.ff), int(D)};
+                rc = aria_check_launch();
+                if (rc == ARIA_OK) rc = launch_expert_rows<true>(up, lists, y.k, T, MixAct{z.act, (long long)y.ff}, stream);
+                if (rc == ARIA_OK) rc = launch_expert_rows<false>(down, lists, y.k, T, MixPartial{z.eo, (long long)D}, stream);
+                if (rc != ARIA_OK) break;
+                ARIA_LAUNCH(mix_combine_kernel, dim3(unsigned((D + 255) / 256), unsigned(T)), dim3(256), 0, stream, (const float*)z.eo,
+                            (const float*)z.weights, int(y.k), int(D), out);
+                rc = aria_check_launch();
+                continue;
+            }
             ARIA_LAUNCH(mix_up_kernel, dim3(unsigned((y.ff + 3) / 4), unsigned(y.k), unsigned(T)), dim3(256), 0, stream, (const float*)z.logits,
                         y.correction, int(y.E), int(ldl), int(y.groups), int(y.keep), int(y.k), static_cast<const bf16_t*>(y.w_gate),
                         static_cast<const bf16_t*>(y.w_up), (const bf16_t*)z.h, int(D), int(y.ff), z.act, z.weights, z.idx);

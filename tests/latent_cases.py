@@ -523,6 +523,23 @@ def case_long_decode(dev, dtype, prompt=3, steps=150, name="sharp"):
     assert logit_err(torch.cat(got), want[prompt - 1:]) < model_tol(cfg, w, [toks], dtype)
 
 
+def case_decode_batch(dev, width, ff, requests):
+    """Single tokens of several requests (the row-streaming projections and the gathered experts) at reductions on both sides of every register window of
+    the kernels: ``width`` and ``ff`` below one window, between windows, a window's columns plus 8, beyond the last one."""
+    from aria_amd.serving import Scheduler
+
+    mix = mixer(heads=2, dim=16, rot_dim=8, vdim=16, kv_rank=32)
+    cfg = config([(mix, moe(ff=ff, experts=6, top=3, count=2, keep=2)), (mix, dense(ff=ff))], width=width, vocab=70)
+    w = checkpoint(cfg, seed=width)
+    m = build(cfg, w, dev, bf16)
+    toks = [clear_tokens(cfg, w, 2, seed=i) for i in range(requests)]
+    want = [O.forward(cfg, w, t) for t in toks]
+    sched = Scheduler(m, 4)
+    for step in range(2):
+        got = sched.step(list(range(requests)), [[t[step]] for t in toks])
+        assert logit_err(got, torch.stack([x[step] for x in want])) < model_tol(cfg, w, toks[:2], bf16)
+
+
 def case_graph_replay(dev, name="mixed", n=70, steps=3):
     """The one-call decode step captured into a HIP graph: every replay, with eager work between, equals the eager step bit for bit."""
     from aria_amd.serving import Scheduler, StepBatch

@@ -69,6 +69,11 @@ def test_model(dtype, name):
     C.case_model(DEV, dtype, name, lens=(4, 1, 2), tail=2)
 
 
+@pytest.mark.parametrize("width,ff,requests", [(136, 120, 3), (264, 128, 16), (1032, 136, 2)])
+def test_decode_batch(width, ff, requests):
+    C.case_decode_batch(DEV, width, ff, requests)
+
+
 def test_portions():
     C.case_portions(DEV, f32, "equal", n=15)
 

@@ -104,6 +104,11 @@ def test_rows_do_not_depend_on_company(dtype, name):
     C.case_rows_do_not_depend_on_company(DEV, dtype, name)
 
 
+@pytest.mark.parametrize("width,ff,requests", [(136, 120, 3), (264, 128, 16), (1032, 1792, 2), (1800, 2568, 5), (3328, 3336, 16), (4104, 6656, 3), (6664, 136, 2)])
+def test_decode_batch(width, ff, requests):
+    C.case_decode_batch(DEV, width, ff, requests)
+
+
 @both
 def test_borrowed_layers_keep_their_own_cache(dtype):
     C.case_borrowed_layers_keep_their_own_cache(DEV, dtype)
