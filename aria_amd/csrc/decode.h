@@ -1,0 +1,19 @@
+// What the one-token decode engine (decode.hip) shares with the step of several sequences (batch.hip).  Hidden: not part of the C ABI.
+#pragma once
+#include "aria_device.h"
+#include "aria_hip.h"
+#include <algorithm>
+
+#define ARIA_HIDDEN __attribute__((visibility("hidden")))
+
+// Splits of the keys of one head: a round of three workgroups a CU over all heads and tokens, one pass of 128 keys at least.  Up to 256 keys one workgroup
+// of 16 waves per head is as fast and needs no merge.
+ARIA_HIDDEN int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len);
+// RoPE, cache write and attention of T tokens of T sequences: qkv [T, 3 H hd], caches [slots, Smax, H hd], part: T H splits (hd + 2) floats, out [T, H hd]
+ARIA_HIDDEN int aria_decode_rows_attn(const ad::bf16_t* qkv, const ad::bf16_t* freqs, const int32_t* slot, const int32_t* pos, ad::bf16_t* kc, ad::bf16_t* vc,
+                                      ad::bf16_t* out, float* part, int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, void* stream);
+ARIA_HIDDEN int aria_decode_dims_ok(const int64_t* dims);
+// One sequence's step by the engine's kernels
+ARIA_HIDDEN int64_t aria_decode_one_scratch(const int64_t* dims);
+ARIA_HIDDEN int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+                                int64_t max_len, float* logits, char* scratch, void* stream);

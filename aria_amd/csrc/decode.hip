@@ -19,8 +19,7 @@
 //   * sampling (gptfast/generate.py:35-58) is one launch as well (aria_sample_topk).
 // Rounding points mirror the tile path (GEMM outputs, norm, SwiGLU, residual adds are each rounded to bf16 where the reference
 // materialises a bf16 tensor); only the fp32 summation ORDER inside a dot product differs from the MFMA kernels.
-#include "aria_device.h"
-#include "aria_hip.h"
+#include "decode.h"
 #include <cmath>
 #include <cstdlib>
 
@@ -115,7 +114,7 @@ __device__ __forceinline__ void dot_rows(float (&acc)[R], const bf16_t* w, long 
 // y[n] = bf16(W[n,:] . xn) (+ residual[n], added to the ROUNDED product like the stand-alone add kernel)
 template <int R, int NC>
 __global__ __launch_bounds__(256) void gemv_kernel(const bf16_t* W, long long ldw, const bf16_t* x, const bf16_t* norm_w, float eps, int K,
-                                                   int N, const bf16_t* residual, bf16_t* y) {
+                                                   int N, const bf16_t* residual, bf16_t* y, float* y32) {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int row0 = (blockIdx.x * 4 + w) * R;
     if (row0 >= N) return;
@@ -127,7 +126,12 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16_t* W, long long ld
     if (l == 0) {
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            if (row0 + r < N) y[row0 + r] = residual ? f2bf(bf2f(residual[row0 + r]) + rbf(acc[r])) : f2bf(acc[r]);
+            if (row0 + r < N) {
+                if (y32)
+                    y32[row0 + r] = acc[r];
+                else
+                    y[row0 + r] = residual ? f2bf(bf2f(residual[row0 + r]) + rbf(acc[r])) : f2bf(acc[r]);
+            }
     }
 }
 
@@ -546,19 +550,21 @@ struct DecodeAttn {
 constexpr int DECODE_ATTN_WAVES = 16;
 template <int HD>
 __global__ __launch_bounds__(DECODE_ATTN_WAVES * 64) void decode_attn_kernel(const bf16_t* qkv, const bf16_t* fc, const int32_t* pos,
-                                                                            bf16_t* k_cache, bf16_t* v_cache, bf16_t* out, int D, float scale) {
+                                                                            const int32_t* slot, long long slot_stride, bf16_t* k_cache,
+                                                                            bf16_t* v_cache, bf16_t* out, int D, float scale) {
     using A = DecodeAttn<HD, DECODE_ATTN_WAVES>;
     ARIA_SMEM_STATIC float red[DECODE_ATTN_WAVES][A::LPK][10];
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, sub = l % A::LPK, grp = l / A::LPK, head = blockIdx.x;
-    const int ps = pos[0];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, sub = l % A::LPK, grp = l / A::LPK, head = blockIdx.x, tok = blockIdx.y;
+    const int ps = pos[tok];
+    const long long at = slot ? slot[tok] * slot_stride : 0;
     float m, lsum, o[8];
-    A::run(qkv, fc, ps, k_cache, v_cache, D, scale, head, 0, ps + 1, true, red, m, lsum, o);
+    A::run(qkv + tok * 3ll * D, fc, ps, k_cache + at, v_cache + at, D, scale, head, 0, ps + 1, true, red, m, lsum, o);
     if (w == 0 && grp == 0) {
         const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
         u32x4 r;
 #pragma unroll
         for (int q = 0; q < 4; ++q) r[q] = pack2bf(o[2 * q] * inv, o[2 * q + 1] * inv);
-        st16(out + (long long)head * HD + sub * 8, r);
+        st16(out + (long long)tok * D + head * HD + sub * 8, r);
     }
 }
 
@@ -571,19 +577,21 @@ __global__ __launch_bounds__(DECODE_ATTN_WAVES * 64) void decode_attn_kernel(con
 constexpr int DECODE_MAX_SPLITS = 32;
 
 template <int HD>
-__global__ __launch_bounds__(256) void decode_attn_split_kernel(const bf16_t* qkv, const bf16_t* fc, const int32_t* pos, bf16_t* k_cache,
-                                                                bf16_t* v_cache, float* part, int D, float scale) {
+__global__ __launch_bounds__(256) void decode_attn_split_kernel(const bf16_t* qkv, const bf16_t* fc, const int32_t* pos, const int32_t* slot,
+                                                                long long slot_stride, bf16_t* k_cache, bf16_t* v_cache, float* part, int D,
+                                                                float scale) {
     using A = DecodeAttn<HD>;
     ARIA_SMEM_STATIC float red[4][A::LPK][10];
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, sub = l % A::LPK, grp = l / A::LPK, head = blockIdx.x, split = blockIdx.y;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, sub = l % A::LPK, grp = l / A::LPK, head = blockIdx.x, split = blockIdx.y, tok = blockIdx.z;
     const int NS = gridDim.y;
-    const int ps = pos[0], nkeys = ps + 1;
+    const int ps = pos[tok], nkeys = ps + 1;
+    const long long at = slot ? slot[tok] * slot_stride : 0;
     const int chunk = ((nkeys + NS - 1) / NS + A::PER_ITER - 1) / A::PER_ITER * A::PER_ITER;
     const int kbeg = split * chunk, kend = min(nkeys, kbeg + chunk);
     float m, lsum, o[8];
-    A::run(qkv, fc, ps, k_cache, v_cache, D, scale, head, kbeg, kend, ps >= kbeg && ps < kend, red, m, lsum, o);
+    A::run(qkv + tok * 3ll * D, fc, ps, k_cache + at, v_cache + at, D, scale, head, kbeg, kend, ps >= kbeg && ps < kend, red, m, lsum, o);
     if (w == 0 && grp == 0) {
-        float* dst = part + ((long long)head * NS + split) * (HD + 2);
+        float* dst = part + (((long long)tok * gridDim.x + head) * NS + split) * (HD + 2);
         if (sub == 0) {
             dst[0] = m;
             dst[1] = lsum;
@@ -595,8 +603,8 @@ __global__ __launch_bounds__(256) void decode_attn_split_kernel(const bf16_t* qk
 
 // grid = heads, HD threads: thread f folds feature f of the NS partial states of its head (m, l are read by every thread: broadcast loads)
 __global__ void decode_attn_merge_kernel(const float* part, bf16_t* out, int NS, int HD) {
-    const int head = blockIdx.x, f = threadIdx.x;
-    const float* src = part + (long long)head * NS * (HD + 2);
+    const int head = blockIdx.x, f = threadIdx.x, tok = blockIdx.y;
+    const float* src = part + ((long long)tok * gridDim.x + head) * NS * (HD + 2);
     float mm = -INFINITY;
     for (int s = 0; s < NS; ++s) mm = fmaxf(mm, src[s * (HD + 2)]);
     float lsum = 0.f, acc = 0.f;
@@ -607,7 +615,12 @@ __global__ void decode_attn_merge_kernel(const float* part, bf16_t* out, int NS,
         acc += src[s * (HD + 2) + 2 + f] * wgt;
     }
     const float r = lsum > 0.f ? acc * (1.f / lsum) : 0.f;
-    out[(long long)head * HD + f] = f2bf(r);
+    out[((long long)tok * gridDim.x + head) * HD + f] = f2bf(r);
+}
+
+__global__ __launch_bounds__(256) void embedding_row_kernel(const int32_t* id, const bf16_t* table, bf16_t* x, int nch, int V) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c < nch) st16(x + c * 8, ld16(table + ((long long)min(max(id[0], 0), V - 1) * nch + c) * 8));
 }
 
 struct Scratch {
@@ -762,26 +775,30 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_topk_kernel(const bf16_
     }
 }
 
-// splits == 1: the one-workgroup-per-head kernel; otherwise the split form + merge (part: H * splits * (hd + 2) floats)
+// splits == 1: the one-workgroup-per-head kernel; otherwise the split form + merge (part: T * H * splits * (hd + 2) floats).  T tokens of T sequences, each on
+// its own slot of the caches (slot NULL: one sequence)
 int launch_decode_attn(void* stream, const bf16_t* qkv, const bf16_t* freqs, const int32_t* pos, bf16_t* kc, bf16_t* vc, bf16_t* out,
-                       float* part, int64_t H, int64_t hd, int64_t D, int splits) {
+                       float* part, int64_t H, int64_t hd, int64_t D, int splits, int64_t T = 1, const int32_t* slot = nullptr,
+                       int64_t slot_stride = 0) {
     const float sc = 1.0f / sqrtf(float(hd));
+    const unsigned h = unsigned(H), t = unsigned(T);
+    const long long ss = slot_stride;
     if (splits <= 1) {
+        const dim3 block(DECODE_ATTN_WAVES * 64);
         if (hd == 128)
-            ARIA_LAUNCH((decode_attn_kernel<128>), dim3(unsigned(H)), dim3(DECODE_ATTN_WAVES * 64), 0, stream, qkv, freqs, pos, kc, vc, out, int(D), sc);
+            ARIA_LAUNCH((decode_attn_kernel<128>), dim3(h, t), block, 0, stream, qkv, freqs, pos, slot, ss, kc, vc, out, int(D), sc);
         else
-            ARIA_LAUNCH((decode_attn_kernel<64>), dim3(unsigned(H)), dim3(DECODE_ATTN_WAVES * 64), 0, stream, qkv, freqs, pos, kc, vc, out, int(D), sc);
+            ARIA_LAUNCH((decode_attn_kernel<64>), dim3(h, t), block, 0, stream, qkv, freqs, pos, slot, ss, kc, vc, out, int(D), sc);
         return aria_check_launch();
     }
+    const dim3 grid(h, unsigned(splits), t);
     if (hd == 128)
-        ARIA_LAUNCH((decode_attn_split_kernel<128>), dim3(unsigned(H), unsigned(splits)), dim3(256), 0, stream, qkv, freqs, pos, kc, vc, part,
-                    int(D), sc);
+        ARIA_LAUNCH((decode_attn_split_kernel<128>), grid, dim3(256), 0, stream, qkv, freqs, pos, slot, ss, kc, vc, part, int(D), sc);
     else
-        ARIA_LAUNCH((decode_attn_split_kernel<64>), dim3(unsigned(H), unsigned(splits)), dim3(256), 0, stream, qkv, freqs, pos, kc, vc, part,
-                    int(D), sc);
+        ARIA_LAUNCH((decode_attn_split_kernel<64>), grid, dim3(256), 0, stream, qkv, freqs, pos, slot, ss, kc, vc, part, int(D), sc);
     int rc = aria_check_launch();
     if (rc != ARIA_OK) return rc;
-    ARIA_LAUNCH(decode_attn_merge_kernel, dim3(unsigned(H)), dim3(unsigned(hd)), 0, stream, (const float*)part, out, splits, int(hd));
+    ARIA_LAUNCH(decode_attn_merge_kernel, dim3(h, t), dim3(unsigned(hd)), 0, stream, (const float*)part, out, splits, int(hd));
     return aria_check_launch();
 }
 
@@ -819,14 +836,14 @@ bool decode_fuse_enabled() {
 inline int chunks_per_lane(long long K) { return int((K / 8 + 63) / 64); }
 
 int launch_gemv(int N, void* stream, const bf16_t* W, long long ldw, const bf16_t* x, const bf16_t* norm_w, float eps, int K,
-                const bf16_t* residual, bf16_t* y) {
+                const bf16_t* residual, bf16_t* y, float* y32 = nullptr) {
     // rows per wave: 4 when that still leaves well over a thousand waves, else 2 (small N must still cover 256 CUs)
     if (N >= 4096) {
-#define CALL(NC) ARIA_LAUNCH((gemv_kernel<4, NC>), dim3((N + 15) / 16), dim3(256), 0, stream, W, ldw, x, norm_w, eps, K, N, residual, y)
+#define CALL(NC) ARIA_LAUNCH((gemv_kernel<4, NC>), dim3((N + 15) / 16), dim3(256), 0, stream, W, ldw, x, norm_w, eps, K, N, residual, y, y32)
         ARIA_NC_SWITCH(chunks_per_lane(K), CALL)
 #undef CALL
     } else {
-#define CALL(NC) ARIA_LAUNCH((gemv_kernel<2, NC>), dim3((N + 7) / 8), dim3(256), 0, stream, W, ldw, x, norm_w, eps, K, N, residual, y)
+#define CALL(NC) ARIA_LAUNCH((gemv_kernel<2, NC>), dim3((N + 7) / 8), dim3(256), 0, stream, W, ldw, x, norm_w, eps, K, N, residual, y, y32)
         ARIA_NC_SWITCH(chunks_per_lane(K), CALL)
 #undef CALL
     }
@@ -859,43 +876,28 @@ Scratch carve(char* base, int64_t L, int64_t D, int64_t H, int64_t hd, int64_t E
     return s;
 }
 
-}  // namespace
-
-extern "C" {
-
-int aria_decode_trace_layout(const int64_t* dims, int64_t* out) {
-    if (!dims || !out) return ARIA_ERR_INVALID;
-    char* const base = reinterpret_cast<char*>(uintptr_t(1) << 20);  // (never dereferenced: carve only does address arithmetic)
-    const Scratch s = carve(base, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
-    out[0] = reinterpret_cast<char*>(s.rl) - base, out[1] = int64_t(s.rl_stride) * 2;      // router logits: bf16 [L][E], row stride in bytes
-    out[2] = reinterpret_cast<char*>(s.idx) - base, out[3] = int64_t(s.idx_stride) * 4;    // expert ids: int32 [L][k]
-    out[4] = reinterpret_cast<char*>(s.scores) - base, out[5] = int64_t(s.sc_stride) * 2;  // scores: bf16 [L][k]
-    return ARIA_OK;
-}
-
-int64_t aria_decode_scratch_bytes(const int64_t* dims) {
-    if (!dims) return 0;
-    return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes);
-}
-
-int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, void* stream) {
-    if (!ptrs || !dims) return ARIA_ERR_INVALID;
-    const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8],
-                  Smax = dims[9];
+// what a decode step of one token needs besides its weights' layer table
+struct OneToken {
+    const bf16_t *freqs, *final_norm, *out_w, *x;
+    const void* const* layers;
+    const int32_t *pos, *slot;   // slot NULL: the caches hold one sequence
+    bf16_t* logits;
+    float* logits32;             // instead of logits
+    int splits;
+};
+int dims_ok(const int64_t* d) {
+    const int64_t L = d[0], D = d[1], H = d[2], hd = d[3], E = d[4], k = d[5], I = d[6], Is = d[7];
     if (L <= 0 || D <= 0 || H * hd != D || (D & 7) || (I & 7) || (Is & 7) || D > 4096 || I > 4096 || Is > 4096 || k > 8 || E > 256)  // 8 chunks/lane
         return ARIA_ERR_UNSUPPORTED;
     if (hd != 64 && hd != 128) return ARIA_ERR_UNSUPPORTED;
-    if (Is % I) return ARIA_ERR_UNSUPPORTED;  // the shared expert is handled as Is / I further experts of width I
-    const int ns = int(Is / I);
-    for (int i = 0; i < ARIA_DECODE_HEADER_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
-        if (!ptrs[i]) return ARIA_ERR_INVALID;
-    const bf16_t* freqs = static_cast<const bf16_t*>(ptrs[0]);
-    const bf16_t* final_norm = static_cast<const bf16_t*>(ptrs[1]);
-    const bf16_t* out_w = static_cast<const bf16_t*>(ptrs[2]);
-    const Scratch s = carve(static_cast<char*>(const_cast<void*>(ptrs[3])), L, D, H, hd, E, k, I, Is);
-    const int32_t* pos = static_cast<const int32_t*>(ptrs[4]);
-    const bf16_t* x = static_cast<const bf16_t*>(ptrs[5]);
-    bf16_t* logits = static_cast<bf16_t*>(const_cast<void*>(ptrs[6]));
+    return Is % I ? ARIA_ERR_UNSUPPORTED : ARIA_OK;  // the shared expert is handled as Is / I further experts of width I
+}
+int decode_one(const OneToken& one, const Scratch& s, const int64_t* dims, float eps, void* stream) {
+    const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8],
+                  Smax = dims[9];
+    const int ns = int(Is / I), splits = one.splits;
+    const int32_t* pos = one.pos;
+    const bf16_t* x = one.x;
     int rc;
 #define ARIA_TRY(call)              \
     do {                            \
@@ -904,7 +906,7 @@ int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, v
     } while (0)
     const bool fuse = decode_fuse_enabled();
     for (int64_t li = 0; li < L; ++li) {
-        const void* const* lp = ptrs + ARIA_DECODE_HEADER_PTRS + ARIA_DECODE_LAYER_PTRS * li;
+        const void* const* lp = one.layers + ARIA_DECODE_LAYER_PTRS * li;
         const bf16_t *attn_norm = static_cast<const bf16_t*>(lp[0]), *wqkv = static_cast<const bf16_t*>(lp[1]),
                      *wo = static_cast<const bf16_t*>(lp[2]), *ffn_norm = static_cast<const bf16_t*>(lp[3]),
                      *gate = static_cast<const bf16_t*>(lp[4]), *w1 = static_cast<const bf16_t*>(lp[5]),
@@ -917,11 +919,10 @@ int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, v
         int32_t* const idx = s.idx + li * s.idx_stride;
         // attention block: h = x + wo( attn( rope(wqkv(norm(x))) ) )
         ARIA_TRY(launch_gemv(int(3 * D), stream, wqkv, (long long)D, x, attn_norm, eps, int(D), nullptr, s.qkv));
-        const int splits = decode_splits_for(Smax);
-        if (Smax <= 16384 || splits > 1) {  // one workgroup per head walks the whole context, or (opt-in) heads x splits workgroups
-            ARIA_TRY(launch_decode_attn(stream, (const bf16_t*)s.qkv, freqs, pos, kc, vc, s.ao, s.part, H, hd, D, splits));
+        if (one.slot || Smax <= 16384 || splits > 1) {  // one workgroup per head walks the whole context, or (opt-in) heads x splits workgroups
+            ARIA_TRY(launch_decode_attn(stream, (const bf16_t*)s.qkv, one.freqs, pos, kc, vc, s.ao, s.part, H, hd, D, splits, 1, one.slot, Smax * D));
         } else {
-            ARIA_LAUNCH(rope_cache_kernel, dim3(unsigned((3 * D / 8 + 255) / 256)), dim3(256), 0, stream, s.qkv, freqs, pos, kc, vc, int(D),
+            ARIA_LAUNCH(rope_cache_kernel, dim3(unsigned((3 * D / 8 + 255) / 256)), dim3(256), 0, stream, s.qkv, one.freqs, pos, kc, vc, int(D),
                         int(hd), s.kv_len);
             ARIA_TRY(aria_check_launch());
             ARIA_TRY(aria_attn_fwd(s.qkv, kc, vc, s.ao, nullptr, s.kv_len, nullptr, 1, 1, Smax, H, hd, D, D, D, D, 1.0f / sqrtf(float(hd)),
@@ -988,9 +989,66 @@ int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, v
         ARIA_TRY(aria_check_launch());
         x = s.xb;  // the next layer reads x = xb and writes its h into xa again (h is dead once this add has run)
     }
-    ARIA_TRY(launch_gemv(int(V), stream, out_w, (long long)D, x, final_norm, eps, int(D), nullptr, logits));
+    ARIA_TRY(launch_gemv(int(V), stream, one.out_w, (long long)D, x, one.final_norm, eps, int(D), nullptr, one.logits, one.logits32));
 #undef ARIA_TRY
     return ARIA_OK;
+}
+
+}  // namespace
+
+int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len) {
+    if (max_len <= 256) return 1;
+    const int64_t fill = (768 + H * T - 1) / (H * T), passes = (max_len + 127) / 128;
+    return int(std::max<int64_t>(1, std::min<int64_t>(std::min(fill, passes), DECODE_MAX_SPLITS)));
+}
+int aria_decode_rows_attn(const bf16_t* qkv, const bf16_t* freqs, const int32_t* slot, const int32_t* pos, bf16_t* kc, bf16_t* vc, bf16_t* out, float* part,
+                          int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, void* stream) {
+    return launch_decode_attn(stream, qkv, freqs, pos, kc, vc, out, part, H, hd, H * hd, splits, T, slot, Smax * H * hd);
+}
+int aria_decode_dims_ok(const int64_t* dims) { return dims_ok(dims); }
+int64_t aria_decode_one_scratch(const int64_t* dims) {
+    return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes) + 2 * dims[1];
+}
+int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const int32_t* ids, const int32_t* slot, const int32_t* pos, int64_t max_len,
+                    float* logits, char* scratch, void* stream) {
+    const int64_t D = dims[1];
+    const Scratch s = carve(scratch, dims[0], D, dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
+    bf16_t* x = reinterpret_cast<bf16_t*>(scratch + s.bytes);
+    ARIA_LAUNCH(embedding_row_kernel, dim3(unsigned((D / 8 + 255) / 256)), dim3(256), 0, stream, ids, static_cast<const bf16_t*>(ptrs[3]), x, int(D / 8),
+                int(dims[8]));
+    if (const int rc = aria_check_launch()) return rc;
+    const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]), x,
+                       ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len)};
+    return decode_one(one, s, dims, eps, stream);
+}
+
+extern "C" {
+
+int aria_decode_trace_layout(const int64_t* dims, int64_t* out) {
+    if (!dims || !out) return ARIA_ERR_INVALID;
+    char* const base = reinterpret_cast<char*>(uintptr_t(1) << 20);  // (never dereferenced: carve only does address arithmetic)
+    const Scratch s = carve(base, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
+    out[0] = reinterpret_cast<char*>(s.rl) - base, out[1] = int64_t(s.rl_stride) * 2;      // router logits: bf16 [L][E], row stride in bytes
+    out[2] = reinterpret_cast<char*>(s.idx) - base, out[3] = int64_t(s.idx_stride) * 4;    // expert ids: int32 [L][k]
+    out[4] = reinterpret_cast<char*>(s.scores) - base, out[5] = int64_t(s.sc_stride) * 2;  // scores: bf16 [L][k]
+    return ARIA_OK;
+}
+
+int64_t aria_decode_scratch_bytes(const int64_t* dims) {
+    if (!dims) return 0;
+    return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes);
+}
+
+int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, void* stream) {
+    if (!ptrs || !dims) return ARIA_ERR_INVALID;
+    if (const int rc = dims_ok(dims)) return rc;
+    for (int i = 0; i < ARIA_DECODE_HEADER_PTRS + ARIA_DECODE_LAYER_PTRS * dims[0]; ++i)
+        if (!ptrs[i]) return ARIA_ERR_INVALID;
+    const Scratch s = carve(static_cast<char*>(const_cast<void*>(ptrs[3])), dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
+    const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]),
+                       static_cast<const bf16_t*>(ptrs[5]), ptrs + ARIA_DECODE_HEADER_PTRS, static_cast<const int32_t*>(ptrs[4]), nullptr,
+                       static_cast<bf16_t*>(const_cast<void*>(ptrs[6])), nullptr, decode_splits_for(dims[9])};
+    return decode_one(one, s, dims, eps, stream);
 }
 
 int aria_sample_topk(const void* logits, const float* q, int64_t V, int64_t top_k, float temperature, int32_t* out, void* stream) {

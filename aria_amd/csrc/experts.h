@@ -71,6 +71,10 @@ struct ExpertIn {
     const bf16_t* X;        // row of an entry: X + (entry / div) ldx
     long long ldx;
     int div, K, N;
+    // experts that every token uses, E, E + 1, ... in the lists: their rows have the stride s_ld, the next one begins s_step further on
+    const bf16_t *S = nullptr, *S2 = nullptr;
+    long long s_step = 0, s_ld = 0;
+    int E = 1 << 30;
 };
 
 namespace {
@@ -87,12 +91,15 @@ __global__ __launch_bounds__(NW * 64) void expert_rows_kernel(ExpertIn in, Exper
     while (g < end) {
         const int a = g / groups, g0 = g - a * groups, g1 = min(groups, g0 + end - g);
         const int first = lists.table[1 + lists.E + a], m = lists.table[2 + lists.E + a] - first;
-        const long long at = (long long)lists.table[1 + a] * in.N * in.K;
+        const int id = lists.table[1 + a];
+        const bool all = id >= in.E;
+        const long long at = all ? (id - in.E) * in.s_step : (long long)id * in.N * in.K;
+        const bf16_t *W = (all ? in.S : in.W) + at, *W2 = PAIR ? (all ? in.S2 : in.W2) + at : nullptr;
         for (int t0 = 0; t0 < m; t0 += 16) {   // (more than 16 only where tokens chose an expert several times: NaN logits)
             sync();                            // (red and entries of the piece before are read)
             const int mine = lists.list[first + min(t0 + (t & 15), m - 1)];
             if (t < 16) entries[t] = mine;     // (published by the first group's barrier)
-            stream_rows<NW, KS, PAIR>(in.W + at, PAIR ? in.W2 + at : nullptr, in.K, in.N, in.X + (long long)(mine / in.div) * in.ldx, g0, g1, red,
+            stream_rows<NW, KS, PAIR>(W, W2, all ? in.s_ld : (long long)in.K, in.K, in.N, in.X + (long long)(mine / in.div) * in.ldx, g0, g1, red,
                                       [&](float v, float u, int tok, int n, int) {
                                           if (t0 + tok < m && n < in.N) e(v, u, entries[tok], n);
                                       });
@@ -106,8 +113,11 @@ __global__ __launch_bounds__(NW * 64) void expert_rows_kernel(ExpertIn in, Exper
 // choices fall on an expert that another token has chosen already.  Up + down + the extra launches against a projection per choice, us: 64 experts of
 // 2560 x 1664, 6 a token: 4 tokens (13 % fall together) 114 / 107, 6 (20 %) 149 / 157, 16 (50 %) 220 / 394; 32 of 1536 x 1024, 4 a token: 8 tokens
 // 54 / 60, 16 67 / 103; 16 of 1024 x 768, 2 a token: 12 tokens 29 / 31, 16 30 / 36.  At 16 tokens the weights of the experts in use arrive at 5.9 TB/s.
+inline bool expert_rows_can(int64_t K0, int64_t K1, int64_t E, int64_t k, int64_t T) {
+    return T * k <= LISTS_MAX && E <= 256 && k <= E && std::min(K0, K1) >= 128 && std::max(K0, K1) <= 6656;
+}
 inline bool expert_rows_take(int64_t K0, int64_t K1, int64_t E, int64_t k, int64_t T) {
-    if (T < 2 || T * k > LISTS_MAX || E > 256 || k > E || std::min(K0, K1) < 128 || std::max(K0, K1) > 6656) return false;
+    if (T < 2 || !expert_rows_can(K0, K1, E, k, T)) return false;
     const double reached = double(E) * (1.0 - std::pow(1.0 - double(k) / double(E), double(T)));
     return reached * 6.0 <= 5.0 * double(T * k);
 }

@@ -114,7 +114,7 @@ struct RowsRed {
     float v[2][PAIR ? 2 : 1][NW][16][17];
 };
 template <int NW, int KS, bool PAIR, class Out>
-__device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, int K, int N, const bf16_t* xp, int g0, int g1, RowsRed<NW, PAIR>& red,
+__device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, long long ldw, int K, int N, const bf16_t* xp, int g0, int g1, RowsRed<NW, PAIR>& red,
                                             const Out& out) {
     constexpr int SUB = PAIR ? 2 : 1, DEPTH = KS <= 16 ? KS : KS / 2;   // fragments in flight
     static_assert(KS % DEPTH == 0, "a step keeps its register");
@@ -123,7 +123,7 @@ __device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, i
     const int own = w * KS * 32, k0 = min(own, K - KS * 32) + q4 * 8;
     xp += k0;
     u32x4 x[KS], b[DEPTH];
-    const bf16_t* wp = W + (long long)min(g0 * 16 + c16, N - 1) * K + k0;
+    const bf16_t* wp = W + (long long)min(g0 * 16 + c16, N - 1) * ldw + k0;
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) b[u] = ld16(wp + 32 * u);
 #pragma unroll
@@ -138,7 +138,7 @@ __device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, i
         for (int sub = 0; sub < SUB; ++sub) {
             f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
             const bool up_next = PAIR && sub == 0, more = up_next || g + 1 < g1;
-            const bf16_t *cur = wp, *nxt = (up_next ? W2 : W) + (long long)min((up_next ? g : g + 1) * 16 + c16, N - 1) * K + k0;
+            const bf16_t *cur = wp, *nxt = (up_next ? W2 : W) + (long long)min((up_next ? g : g + 1) * 16 + c16, N - 1) * ldw + k0;
             wp = nxt;
             if (more) {
 #pragma unroll
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, i
     const RowsIn& in = rp.in[blockIdx.z];
     const int c16 = threadIdx.x & 15, t0 = blockIdx.y * 16, groups = (in.N + 15) / 16, g0 = blockIdx.x * per;
     if (in.sq) token_rms(rms, in, t0, n_tok, NW);   // (published by the first group's barrier)
-    stream_rows<NW, KS, PAIR>(in.W, in.W2, in.K, in.N, in.X + (long long)min(t0 + c16, n_tok - 1) * in.ldx, g0, min(groups, g0 + per), red,
+    stream_rows<NW, KS, PAIR>(in.W, in.W2, in.K, in.K, in.N, in.X + (long long)min(t0 + c16, n_tok - 1) * in.ldx, g0, min(groups, g0 + per), red,
                               [&](float v, float u, int tok, int n, int g) {
                                   const bool in_range = t0 + tok < n_tok && n < in.N;
                                   float s = 0.f;

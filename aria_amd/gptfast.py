@@ -22,6 +22,7 @@ from . import hip, ops
 from .vision import AriaProjector, AriaVisionConfig, AriaVisionModel
 
 bf16 = torch.bfloat16
+DECODE_ROWS = 16   # single tokens that one serving step takes at once
 
 
 @dataclass
@@ -258,6 +259,7 @@ class Transformer(nn.Module):
         self.decode_graph = False         # ... optionally replayed from a natively captured HIP graph (measured SLOWER than the plain
         #                                   enqueue on ROCm 7.2: 6.2 vs 4.8 ms/token -- graph kernel nodes cost more than stream launches)
         self._engine: Optional["DecodeEngine"] = None
+        self._tables: Optional["_StepTables"] = None
         # bumped by whatever may re-home a weight (module.to / .cuda / casts; load_state_dict, also through a parent module, also assign=True):
         # the decode engine re-checks its whole pointer table only then
         self._weights_version = 0
@@ -292,7 +294,7 @@ class Transformer(nn.Module):
             return   # same geometry: the buffers are re-used as they are (positions beyond the cursor are never read; gptfast/model.py:67-93
             #          overwrites rows in place as well) and the decode engine's pointer table stays valid
         self.max_batch_size, self.max_seq_length = max_batch_size, rounded
-        self._engine = None   # it holds raw addresses of the tensors replaced below
+        self._engine = self._tables = None   # they hold raw addresses of the tensors replaced below
         for b in self.layers:
             b.attention.kv_cache = None if training else KVCache(max_batch_size, self.max_seq_length, self.config.n_head,
                                                                  b.attention.hdp, dev)
@@ -335,7 +337,19 @@ class Transformer(nn.Module):
             return ops.gemm(h, self.output.weight).view(B, 1, -1)
         return ops.gemm(h, self.output.weight).view(B, S, -1)
 
-    # ---- the serving protocol (serving.py): sequences of a batch run one after the other, each on its own cache slot with its own decode engine
+    # ---- the serving protocol (serving.py).  Single tokens of up to DECODE_ROWS sequences are one library call; where the library does not serve the
+    # sizes, and for portions of prompts, the sequences of a batch run one after the other, each on its own cache slot
+    def _step_tables(self, batch) -> Optional["_StepTables"]:
+        """Tables of the one-call step on the caches as they are; None where this model does not go through it."""
+        cache = self.layers[0].attention.kv_cache
+        if cache is None or not self.use_decode_engine or self.decode_graph or not self._engine_capable():
+            return None
+        if batch.max_len > self.max_seq_length or max(batch.slots) >= cache.k.shape[0]:
+            raise ValueError("the batch does not fit the caches")
+        if self._tables is None or not self._tables.valid_for(self):
+            self._tables = _StepTables(self)
+        return self._tables
+
     @property
     def vocab(self) -> int:
         return self.config.vocab_size
@@ -347,6 +361,11 @@ class Transformer(nn.Module):
     @torch.no_grad()
     def step(self, batch) -> torch.Tensor:
         """Run a ``serving.StepBatch`` -> float32 logits [wanted rows, vocab]."""
+        tables = self._step_tables(batch)
+        if tables is not None and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS:
+            logits = tables.run(batch.ids, batch.slot, batch.pos, batch.max_len)
+            if logits is not None:
+                return logits if batch.wanted is None or batch.wanted.numel() == len(logits) else logits[batch.wanted.long()]
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:
@@ -358,7 +377,7 @@ class Transformer(nn.Module):
                 rows, self._engine = self._slot_state.get(slot) or ([c.row(slot) for c in whole], None)
                 for b, r in zip(self.layers, rows):
                     b.attention.kv_cache = r
-                toks = ids[at:at + n].view(1, n)
+                toks, first = ids[at:at + n].view(1, n), at
                 at += n
                 if start == 0 and n > 1:
                     last = list(want) == [n - 1]
@@ -366,6 +385,11 @@ class Transformer(nn.Module):
                     out.append(logits if last else logits[list(want)])
                 else:
                     for j in range(n):      # (on a cache: token by token)
+                        token = slice(first + j, first + j + 1)
+                        logits = tables.run(batch.ids[token], batch.slot[token], batch.pos[token], start + j + 1) if tables is not None else None
+                        if logits is not None:
+                            out += [logits] * list(want).count(j)
+                            continue
                         logits = self.forward(toks[:, j:j + 1], torch.tensor([start + j], dtype=torch.int32, device=ids.device))
                         out += [logits[0].float().clone()] * list(want).count(j)
                 self._slot_state[slot] = (rows, self._engine)
@@ -374,6 +398,53 @@ class Transformer(nn.Module):
                 b.attention.kv_cache = c
             self._engine = engine
         return torch.cat(out) if out else torch.empty((0, self.vocab), dtype=torch.float32, device=ids.device)
+
+
+class _StepTables:
+    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches (re-made when either moves), and its scratch."""
+
+    def __init__(self, model: "Transformer"):
+        import ctypes
+
+        import numpy as np
+
+        c = model.config
+        self.version, self.key, self.eps = model._weights_version, DecodeEngine._cheap_key(model), float(c.norm_eps)
+        self.dims = np.array([c.n_layer, c.dim, c.n_head, c.head_dim, c.num_experts, c.router_topk, c.intermediate_size,
+                              c.intermediate_size * c.num_shared_experts, c.vocab_size, model.max_seq_length], dtype=np.int64)
+        self.dims_p = self.dims.ctypes.data_as(ctypes.c_void_p)
+        self.tensors = [model.freqs_cis, model.norm.weight, model.output.weight, model.tok_embeddings.weight] + _layer_table(model)
+        self.served = all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in self.tensors)
+        self.ptrs = (ctypes.c_void_p * len(self.tensors))(*(t.data_ptr() for t in self.tensors))
+        self.scratch: Optional[torch.Tensor] = None
+
+    def valid_for(self, model: "Transformer") -> bool:
+        return model._weights_version == self.version and DecodeEngine._cheap_key(model) == self.key
+
+    def run(self, ids, slot, pos, max_len: int) -> Optional[torch.Tensor]:
+        """logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""
+        lib, T = hip.get_lib(), ids.numel()
+        need = int(lib.cdll.aria_decode_step_scratch(self.dims_p, T, max_len)) if self.served else 0
+        if need == 0:
+            return None
+        if self.scratch is None or self.scratch.numel() < need:
+            self.scratch = torch.empty(need, dtype=torch.uint8, device=ids.device)
+        logits = torch.empty((T, int(self.dims[8])), dtype=torch.float32, device=ids.device)
+        for t in (ids, slot, pos):
+            assert t.dtype == torch.int32 and t.is_contiguous() and t.numel() == T
+        lib.call("aria_decode_step", self.ptrs, self.dims_p, self.eps, T, ids.data_ptr(), slot.data_ptr(), pos.data_ptr(), max_len, logits.data_ptr(),
+                 self.scratch.data_ptr(), self.scratch.numel(), ops._stream(logits))
+        return logits
+
+
+def _layer_table(model: "Transformer") -> List[torch.Tensor]:
+    """the tensors of every layer in the order of the decode engine's pointer tables"""
+    out = []
+    for blk in model.layers:
+        a, f = blk.attention, blk.feed_forward
+        out += [blk.attention_norm.weight, a.wqkv.weight, a.wo.weight, blk.ffn_norm.weight, f.gate.weight, f.cond_ffn.w1, f.cond_ffn.w3, f.cond_ffn.w2,
+                f.shared_ffn.w1.weight, f.shared_ffn.w3.weight, f.shared_ffn.w2.weight, a.kv_cache.k, a.kv_cache.v]
+    return out
 
 
 class DecodeEngine:
@@ -424,13 +495,7 @@ class DecodeEngine:
 
     def _table(self, model: "Transformer"):
         """The pointer table of aria_decode_token, read from the MODEL's current tensors (weights, freqs_cis, KV cache) + the engine's own."""
-        tensors = [model.freqs_cis, model.norm.weight, model.output.weight, self.scratch, self.pos, self.x_in, self.logits, self.pos]
-        for blk in model.layers:
-            a, f = blk.attention, blk.feed_forward
-            tensors += [blk.attention_norm.weight, a.wqkv.weight, a.wo.weight, blk.ffn_norm.weight, f.gate.weight, f.cond_ffn.w1,
-                        f.cond_ffn.w3, f.cond_ffn.w2, f.shared_ffn.w1.weight, f.shared_ffn.w3.weight, f.shared_ffn.w2.weight,
-                        a.kv_cache.k, a.kv_cache.v]
-        return tensors
+        return [model.freqs_cis, model.norm.weight, model.output.weight, self.scratch, self.pos, self.x_in, self.logits, self.pos] + _layer_table(model)
 
     def valid_for(self, model: "Transformer") -> bool:
         """The recorded addresses against what the model holds NOW: ``setup_caches`` allocates new K/V tensors and a fresh ``freqs_cis``,

@@ -417,6 +417,16 @@ int aria_cross_entropy(const void* logits, const int32_t* labels, float* loss_su
 #define ARIA_DECODE_LAYER_PTRS 13
 int64_t aria_decode_scratch_bytes(const int64_t* dims);
 int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, void* stream);
+/* One serving step of T sequences, one token each (token ids, cache slots, positions: int32 [T] on the device; max_len >= largest position + 1, known to
+ * the host): embedding rows to fp32 logits [T, V].  One sequence runs the kernels of aria_decode_token, several the batched ones (batch.hip: every weight
+ * read once for all tokens; meant for T up to 16).
+ * ptrs: [0] freqs_cis   [1] final norm weight   [2] output weight [V, D]   [3] embedding [vocab, D]   then the 13 of a layer as above, caches
+ *   [slots, S_max, D].  dims as above.
+ * scratch: 16-byte aligned; 0 bytes from aria_decode_step_scratch: these sizes are not served (aria_decode_step: ARIA_ERR_UNSUPPORTED). */
+#define ARIA_DECODE_STEP_PTRS 4
+int64_t aria_decode_step_scratch(const int64_t* dims, int64_t T, int64_t max_len);
+int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+                     int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
 /* Where, inside the scratch buffer, the last aria_decode_token call left every layer's routing record (TopKRouter of
  * gptfast/model.py:355-366 as the engine evaluated it): out[0], out[1] = byte offset and per-layer byte stride of the router logits (bf16 [L][E]),
  * out[2], out[3] = the chosen expert ids (int32 [L][top_k]), out[4], out[5] = their scores (bf16 [L][top_k]).  Read by the full-depth parity

@@ -55,6 +55,47 @@ def case_gptfast_batch(dev, engine=True):
             sched.finish(r)
 
 
+def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
+    """Steps of several requests in one call (every weight read once) against each request alone, one token at a time: requests of unequal lengths on any
+    slots, experts that one, several and all of them chose.  Embeddings carry the directions of their experts, so that no choice is a close call.  Both
+    sides round the same tensors to bf16; a logit differs by the order of fp32 sums and by roundings that then fall the other way, about 2^-9 a layer's
+    residual step, four of them."""
+    from aria_amd import gptfast as G
+    from aria_amd.serving import Scheduler
+
+    E, k, V = 16, 3, 264
+    args = G.ModelArgs(block_size=longest + 16, vocab_size=V, n_layer=2, n_head=dim // head_dim, dim=dim, intermediate_size=inter, rope_base=10000.0, norm_eps=1e-5,
+                       num_experts=E, router_topk=k, num_shared_experts=2)
+    m, g = G.Transformer(args), L.gen(5)
+    unit = torch.nn.functional.normalize(torch.randn(E, dim, generator=g), dim=-1)
+    chosen = torch.zeros(V, E).scatter_(1, torch.rand(V, E, generator=g).topk(k, -1).indices, 1.0)
+    with torch.no_grad():
+        for n, p in m.named_parameters():
+            p.copy_((1 + 0.1 * torch.randn(p.shape, generator=g)).to(bf16) if "norm" in n else (torch.randn(p.shape, generator=g) * p.shape[-1] ** -0.5).to(bf16))
+        m.tok_embeddings.weight.copy_((torch.randn(V, dim, generator=g) + 8.0 * chosen @ unit).to(bf16))
+        for b in m.layers:
+            b.feed_forward.gate.weight.copy_(unit[torch.randperm(E, generator=g)].to(bf16))
+    m = m.to(dev).eval()
+    toks = [torch.randint(0, V, (max(3, longest - 5 * i),), generator=L.gen(i)).tolist() for i in range(requests)]
+
+    def alone(t):
+        s = Scheduler(m, longest + 1)
+        s.step(["x"], [t[:-2]], [[]])
+        return torch.cat([s.step(["x"], [[i]]) for i in t[-2:]]).cpu().double()
+
+    want = [alone(t) for t in toks]
+    sched = Scheduler(m, longest + 1)
+    for i, t in enumerate(toks):      # (prompts as in the single runs: the caches then hold the same rows)
+        if i == 0:
+            m.setup_caches(requests, longest + 1)
+            sched.slots, sched.free = requests, list(range(requests))[::-1]
+        sched.step([i], [t[:-2]], [[]])
+    for step in range(2):
+        order = list(range(requests))[::-1] if step else list(range(requests))
+        got = sched.step(order, [[toks[i][len(toks[i]) - 2 + step]] for i in order])
+        assert L.logit_err(got, torch.stack([want[i][step] for i in order])) < 4 * 2 ** -8
+
+
 def case_gptfast_generate(dev):
     """serving.generate on the gptfast decoder: greedy continuation equals arg-max over full prefills wherever that is not a tie."""
     from aria_amd import serving

@@ -15,6 +15,10 @@ def emu():
     emu_lib.uninstall()
 
 
+def test_gptfast_decode_batch():
+    C.case_gptfast_decode_batch(DEV, 128, 64, 128, 3)
+
+
 def test_gptfast_batch():
     C.case_gptfast_batch(DEV, engine=False)   # (the engine's emulated form takes a minute: on hardware only)
 

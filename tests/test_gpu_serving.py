@@ -21,6 +21,12 @@ def real_library():
     yield
 
 
+@pytest.mark.parametrize("dim,head_dim,inter,requests,longest", [(128, 64, 128, 2, 9), (512, 128, 1024, 16, 30), (2560, 128, 1664, 5, 400),
+                                                                    (640, 64, 264, 3, 9), (1920, 64, 1800, 16, 300)])
+def test_gptfast_decode_batch(dim, head_dim, inter, requests, longest):
+    C.case_gptfast_decode_batch(DEV, dim, head_dim, inter, requests, longest)
+
+
 @pytest.mark.parametrize("engine", [False, True])
 def test_gptfast_batch(engine):
     C.case_gptfast_batch(DEV, engine)
