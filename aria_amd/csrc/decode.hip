@@ -601,21 +601,37 @@ __global__ __launch_bounds__(256) void decode_attn_split_kernel(const bf16_t* qk
     }
 }
 
-// grid = heads, HD threads: thread f folds feature f of the NS partial states of its head (m, l are read by every thread: broadcast loads)
+// grid = (heads, tokens), HD threads: thread f folds feature f of the NS <= 32 partial states of its head.  Wave 0 turns the states' (m, l) into
+// weights, a lane per split, while every thread already has its features of 16 splits on the way.
 __global__ void decode_attn_merge_kernel(const float* part, bf16_t* out, int NS, int HD) {
+    ARIA_SMEM_STATIC float wt[DECODE_MAX_SPLITS];
     const int head = blockIdx.x, f = threadIdx.x, tok = blockIdx.y;
     const float* src = part + ((long long)tok * gridDim.x + head) * NS * (HD + 2);
-    float mm = -INFINITY;
-    for (int s = 0; s < NS; ++s) mm = fmaxf(mm, src[s * (HD + 2)]);
-    float lsum = 0.f, acc = 0.f;
-    for (int s = 0; s < NS; ++s) {
-        const float ms = src[s * (HD + 2)];
-        const float wgt = ms == -INFINITY ? 0.f : exp2_fast(ms - mm);
-        lsum += src[s * (HD + 2) + 1] * wgt;
-        acc += src[s * (HD + 2) + 2 + f] * wgt;
+    float v[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) v[s] = src[min(s, NS - 1) * (HD + 2) + 2 + f];
+    if (f < 64) {
+        const int s = min(f, NS - 1);
+        const float m = f < NS ? src[s * (HD + 2)] : -INFINITY, l = f < NS ? src[s * (HD + 2) + 1] : 0.f;
+        const float mm = wave_max_bcast(m);
+        const float w = m == -INFINITY ? 0.f : exp2_fast(m - mm);   // (an empty range)
+        const float lsum = wave_sum_bcast(l * w);
+        if (f < NS) wt[f] = lsum > 0.f ? w * (1.f / lsum) : 0.f;
     }
-    const float r = lsum > 0.f ? acc * (1.f / lsum) : 0.f;
-    out[((long long)tok * gridDim.x + head) * HD + f] = f2bf(r);
+    sync();
+    float acc = 0.f;
+    for (int s0 = 0; s0 < NS; s0 += 16) {
+        if (s0) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) v[s] = src[min(s0 + s, NS - 1) * (HD + 2) + 2 + f];
+        }
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const float w = s0 + s < NS ? wt[min(s0 + s, NS - 1)] : 0.f;
+            acc += w != 0.f ? w * v[s] : 0.f;   // (selected, not multiplied: an empty range's state is not finite by itself)
+        }
+    }
+    out[((long long)tok * gridDim.x + head) * HD + f] = f2bf(acc);
 }
 
 __global__ __launch_bounds__(256) void embedding_row_kernel(const int32_t* id, const bf16_t* table, bf16_t* x, int nch, int V) {
@@ -998,7 +1014,7 @@ int decode_one(const OneToken& one, const Scratch& s, const int64_t* dims, float
 
 int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len) {
     if (max_len <= 256) return 1;
-    const int64_t fill = (768 + H * T - 1) / (H * T), passes = (max_len + 127) / 128;
+    const int64_t fill = (2048 + H * T - 1) / (H * T), passes = (max_len + 127) / 128;
     return int(std::max<int64_t>(1, std::min<int64_t>(std::min(fill, passes), DECODE_MAX_SPLITS)));
 }
 int aria_decode_rows_attn(const bf16_t* qkv, const bf16_t* freqs, const int32_t* slot, const int32_t* pos, bf16_t* kc, bf16_t* vc, bf16_t* out, float* part,

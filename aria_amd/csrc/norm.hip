@@ -280,6 +280,33 @@ __global__ __launch_bounds__(256) void rope_interleaved_kernel(bf16_t* x, const 
     }
 }
 
+// The same rotation for the packed prompts of several sequences, with the cache write (gptfast/model.py:67-93) in the same pass: q and k of a [T, 3 D]
+// projection rotated in place (the attention reads them there), k and v also into row pos of the sequence's slot.
+__global__ __launch_bounds__(256) void rope_cache_rows_kernel(bf16_t* qkv, const bf16_t* fc, const int32_t* slot, const int32_t* pos, bf16_t* kc, bf16_t* vc,
+                                                              long long nitems, int nch, int cph, long long S) {
+    for (long long it = (long long)blockIdx.x * blockDim.x + threadIdx.x; it < nitems; it += (long long)gridDim.x * blockDim.x) {
+        const int c = int(it % nch), part = int(it / nch % 3);
+        const long long t = it / nch / 3;
+        const int ps = pos[t];
+        bf16_t* p = qkv + ((t * 3 + part) * nch + c) * 8;
+        const long long row = ((slot[t] * S + ps) * nch + c) * 8;
+        const u32x4 a = ld16(p);
+        if (part == 2) {
+            st16(vc + row, a);
+            continue;
+        }
+        const u32x4 f = ld16(fc + ((long long)ps * cph + c % cph) * 8);
+        u32x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float x0 = bflo(a[q]), x1 = bfhi(a[q]), cs = bflo(f[q]), sn = bfhi(f[q]);
+            o[q] = pack2bf(x0 * cs - x1 * sn, x1 * cs + x0 * sn);
+        }
+        st16(p, o);
+        if (part == 1) st16(kc + row, o);
+    }
+}
+
 // AdamW with fp32 master weights (decoupled weight decay, bias correction), one pass over HBM:
 //   g = grad (bf16) * grad_scale; m, v updated; master -= lr * (m_hat / (sqrt(v_hat) + eps) + wd * master); param = bf16(master)
 __global__ __launch_bounds__(256) void adamw_kernel(bf16_t* param, const bf16_t* grad, float* master, float* m, float* v,
@@ -589,6 +616,18 @@ int aria_rope_interleaved_inplace(void* x, const void* freqs_cis, const int32_t*
     const long long nitems = T * n_heads * (hd / 8);
     ARIA_LAUNCH(rope_interleaved_kernel, dim3(grid1d(nitems, 256)), dim3(256), 0, stream, static_cast<bf16_t*>(x),
                 static_cast<const bf16_t*>(freqs_cis), pos, nitems, int(S), int(n_heads), int(hd), (long long)ld);
+    return aria_check_launch();
+}
+
+int aria_rope_cache_rows(void* qkv, const void* freqs_cis, const int32_t* slot, const int32_t* pos, void* k_cache, void* v_cache, int64_t T, int64_t H, int64_t hd,
+                         int64_t S_max, void* stream) {
+    if (!qkv || !freqs_cis || !slot || !pos || !k_cache || !v_cache || T < 0 || H <= 0 || hd <= 0 || S_max <= 0) return ARIA_ERR_INVALID;
+    if (hd & 7) return ARIA_ERR_ALIGN;
+    if (T == 0) return ARIA_OK;
+    const int64_t nch = H * hd / 8;
+    const long long nitems = T * 3 * nch;
+    ARIA_LAUNCH(rope_cache_rows_kernel, dim3(grid1d(nitems, 256)), dim3(256), 0, stream, static_cast<bf16_t*>(qkv), static_cast<const bf16_t*>(freqs_cis), slot, pos,
+                static_cast<bf16_t*>(k_cache), static_cast<bf16_t*>(v_cache), nitems, int(nch), int(hd / 8), (long long)S_max);
     return aria_check_launch();
 }
 

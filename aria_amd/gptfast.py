@@ -172,6 +172,16 @@ class Attention(nn.Module):
         return ops.gemm(o, self.wo.weight)
 
 
+    def packed(self, x2d, freqs_cis, batch):
+        """Whole prompts of several sequences (``serving.StepBatch``), packed: one projection, rotation and cache write for all of them, attention within
+        each sequence."""
+        c = self.config
+        D, H, hd = c.dim, c.n_head, c.head_dim
+        qkv = ops.rope_cache_rows_(ops.gemm(x2d, self.wqkv.weight), freqs_cis, batch.slot, batch.pos, self.kv_cache.k, self.kv_cache.v, H, hd)
+        o = ops.attention_varlen(qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:], batch.cu, batch.longest, H, hd, hd, hd ** -0.5)
+        return ops.gemm(o, self.wo.weight)
+
+
 class ConditionalFeedForward(nn.Module):
     def __init__(self, config: ModelArgs):
         super().__init__()
@@ -231,16 +241,18 @@ class TransformerBlock(nn.Module):
         self.ffn_norm = RMSNorm(config.dim, config.norm_eps)
         self.attention_norm = RMSNorm(config.dim, config.norm_eps)
 
-    def forward(self, res, delta, B, S, freqs_cis, pos32, kv_len, prefill, pos_is_arange=False):
+    def forward(self, res, delta, B, S, freqs_cis, pos32, kv_len, prefill, pos_is_arange=False, packed=None):
         """gptfast/model.py:236-260 with the two residual adds folded into the norm that follows each (``rmsnorm`` with a residual: the
         sum is rounded to bf16 and written once, then normalised -- the same bits as ``add`` followed by ``rmsnorm``, two launches and two
         passes over [T, D] less per layer).  The block's input is ``res + delta`` (``delta`` None for the first block); it returns
-        (h, ffn_out), the two halves of its output, for the next block's attention_norm -- or the model's final norm -- to sum."""
+        (h, ffn_out), the two halves of its output, for the next block's attention_norm -- or the model's final norm -- to sum.  ``packed``: a
+        batch of whole prompts, packed, instead of the B x S arguments."""
         if delta is None:
             x, xn = res, self.attention_norm(res)
         else:
             xn, x, _ = ops.rmsnorm(delta, self.attention_norm.weight, self.attention_norm.eps, residual=res, want_rstd=False)
-        a = self.attention(xn, B, S, freqs_cis, pos32, kv_len, prefill, pos_is_arange)
+        a = (self.attention(xn, B, S, freqs_cis, pos32, kv_len, prefill, pos_is_arange) if packed is None else
+             self.attention.packed(xn, freqs_cis, packed))
         hn, h, _ = ops.rmsnorm(a, self.ffn_norm.weight, self.ffn_norm.eps, residual=x, want_rstd=False)
         return h, self.feed_forward(hn)
 
@@ -358,6 +370,26 @@ class Transformer(nn.Module):
     def device(self):
         return self.output.weight.device
 
+    def _packs(self, batch) -> bool:
+        """Whole prompts of several sequences run packed, every weight read once for all of them, where the experts' projections are the gathering launches
+        (a kernel per expert and projection would not share more) and the batch is no larger than one long prompt."""
+        f = self.layers[0].feed_forward
+        return (batch.fresh and len(batch.lengths) > 1 and batch.longest > 1 and batch.ids.numel() <= 65536 and _glu_pair_ready(f.cond_ffn.w1, f.cond_ffn.w3)
+                and ops.gather_fusable(self.config.dim) and self.freqs_cis.shape[0] >= self.max_seq_length)
+
+    def _prompts(self, batch) -> torch.Tensor:
+        if batch.wanted is not None and batch.wanted.numel() == 0:
+            wanted = None
+        else:
+            wanted = slice(None) if batch.wanted is None else batch.wanted.long()
+        res, delta = self.tok_embeddings(batch.ids.long()), None
+        for layer in self.layers:
+            res, delta = layer(res, delta, None, None, self.freqs_cis, None, None, True, packed=batch)
+        if wanted is None:
+            return torch.empty((0, self.vocab), dtype=torch.float32, device=self.device)
+        h = ops.rmsnorm(delta[wanted], self.norm.weight, self.norm.eps, residual=res[wanted], want_rstd=False)[0]
+        return ops.gemm(h, self.output.weight).float()
+
     @torch.no_grad()
     def step(self, batch) -> torch.Tensor:
         """Run a ``serving.StepBatch`` -> float32 logits [wanted rows, vocab]."""
@@ -366,6 +398,8 @@ class Transformer(nn.Module):
             logits = tables.run(batch.ids, batch.slot, batch.pos, batch.max_len)
             if logits is not None:
                 return logits if batch.wanted is None or batch.wanted.numel() == len(logits) else logits[batch.wanted.long()]
+        if tables is not None and self._packs(batch):
+            return self._prompts(batch)
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:

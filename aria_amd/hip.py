@@ -86,6 +86,7 @@ SIGNATURES = {
     "aria_rmsnorm_bwd": [P, P, P, P, P, P, P, I64, I64, I64, P],
     "aria_colsum_f32": [P, P, I64, I64, I32, P],
     "aria_rope_inplace": [P, P, P, I64, I64, I64, I64, I64, I32, P],
+    "aria_rope_cache_rows": [P, P, P, P, P, P, I64, I64, I64, I64, P],
     "aria_rope_interleaved_inplace": [P, P, P, I64, I64, I64, I64, I64, P],
     "aria_adamw_step": [P, P, P, P, P, I64, F32, F32, F32, F32, F32, I64, F32, P],
     "aria_sumsq_bf16": [P, I64, P, I32, P, P],

@@ -790,6 +790,20 @@ def rope_interleaved_(x: torch.Tensor, freqs_cis: torch.Tensor, n_heads: int, hd
     return x
 
 
+def rope_cache_rows_(qkv: torch.Tensor, freqs_cis: torch.Tensor, slot: torch.Tensor, pos: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, H: int,
+                     hd: int) -> torch.Tensor:
+    """``rope_interleaved_`` on q and k of ``qkv`` [T, 3 H hd] (packed tokens of several sequences), and k and v into row pos[t] of slot[t] of the caches
+    [slots, S, H hd]."""
+    _chk(qkv, name="qkv"), _chk(freqs_cis, name="freqs_cis"), _chk(slot, torch.int32, "slot"), _chk(pos, torch.int32, "pos")
+    assert qkv.is_contiguous() and qkv.shape[1] == 3 * H * hd and slot.numel() == pos.numel() == qkv.shape[0]
+    assert freqs_cis.is_contiguous() and freqs_cis.shape[1] * 2 == hd and freqs_cis.shape[0] >= k_cache.shape[1]
+    for c in (k_cache, v_cache):
+        assert c.is_contiguous() and c.shape == k_cache.shape and c.shape[2] == H * hd and c.dtype == bf16
+    hip.get_lib().call("aria_rope_cache_rows", _p(qkv), _p(freqs_cis), _p(slot), _p(pos), _p(k_cache), _p(v_cache), qkv.shape[0], H, hd, k_cache.shape[1],
+                       _stream(qkv))
+    return qkv
+
+
 def adamw_step_(param: torch.Tensor, grad: torch.Tensor, master: torch.Tensor, m: torch.Tensor, v: torch.Tensor, *, lr: float,
                 beta1: float, beta2: float, eps: float, weight_decay: float, step: int, grad_scale: float = 1.0):
     """In-place AdamW on flat contiguous views (bf16 param/grad, fp32 master/m/v) of equal, even length."""

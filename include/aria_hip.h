@@ -292,6 +292,10 @@ int aria_rope_inplace(void* x, const void* cos, const void* sin, int64_t T, int6
  * pos int32[T] (device; the decode cursor) or NULL (position = t % S). */
 int aria_rope_interleaved_inplace(void* x, const void* freqs_cis, const int32_t* pos, int64_t T, int64_t S, int64_t n_heads,
                                   int64_t hd, int64_t ld, void* stream);
+/* The same for the packed tokens of several sequences, with the cache write: qkv [T, 3 H hd] contiguous, q and k rotated in place, k and v also into row pos[t] of
+ * slot[t] of the caches [slots, S_max, H hd] (slot, pos: int32 [T] on the device). */
+int aria_rope_cache_rows(void* qkv, const void* freqs_cis, const int32_t* slot, const int32_t* pos, void* k_cache, void* v_cache, int64_t T, int64_t H, int64_t hd,
+                         int64_t S_max, void* stream);
 
 /* AdamW step with fp32 master weights on a contiguous (shard of a) parameter: the optimizer the reference's recipe runs through
  * DeepSpeed ZeRO-2 (recipes/config_full.yaml:25-29 lr 5e-6, weight_decay 0.1, adam_beta2 0.95; accelerate_configs/zero2.yaml).

@@ -55,16 +55,12 @@ def case_gptfast_batch(dev, engine=True):
             sched.finish(r)
 
 
-def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
-    """Steps of several requests in one call (every weight read once) against each request alone, one token at a time: requests of unequal lengths on any
-    slots, experts that one, several and all of them chose.  Embeddings carry the directions of their experts, so that no choice is a close call.  Both
-    sides round the same tensors to bf16; a logit differs by the order of fp32 sums and by roundings that then fall the other way, about 2^-9 a layer's
-    residual step, four of them."""
+def gptfast_routed(dev, dim, head_dim, inter, block):
+    """Embeddings carry the directions of their experts, so that no choice is a close call."""
     from aria_amd import gptfast as G
-    from aria_amd.serving import Scheduler
 
     E, k, V = 16, 3, 264
-    args = G.ModelArgs(block_size=longest + 16, vocab_size=V, n_layer=2, n_head=dim // head_dim, dim=dim, intermediate_size=inter, rope_base=10000.0, norm_eps=1e-5,
+    args = G.ModelArgs(block_size=block, vocab_size=V, n_layer=2, n_head=dim // head_dim, dim=dim, intermediate_size=inter, rope_base=10000.0, norm_eps=1e-5,
                        num_experts=E, router_topk=k, num_shared_experts=2)
     m, g = G.Transformer(args), L.gen(5)
     unit = torch.nn.functional.normalize(torch.randn(E, dim, generator=g), dim=-1)
@@ -75,8 +71,18 @@ def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
         m.tok_embeddings.weight.copy_((torch.randn(V, dim, generator=g) + 8.0 * chosen @ unit).to(bf16))
         for b in m.layers:
             b.feed_forward.gate.weight.copy_(unit[torch.randperm(E, generator=g)].to(bf16))
-    m = m.to(dev).eval()
-    toks = [torch.randint(0, V, (max(3, longest - 5 * i),), generator=L.gen(i)).tolist() for i in range(requests)]
+    return m.to(dev).eval()
+
+
+def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
+    """Steps of several requests in one call (every weight read once) against each request alone, one token at a time: requests of unequal lengths on any
+    slots, experts that one, several and all of them chose.  Embeddings carry the directions of their experts, so that no choice is a close call.  Both
+    sides round the same tensors to bf16; a logit differs by the order of fp32 sums and by roundings that then fall the other way, about 2^-9 a layer's
+    residual step, four of them."""
+    from aria_amd.serving import Scheduler
+
+    m = gptfast_routed(dev, dim, head_dim, inter, longest + 16)
+    toks = [torch.randint(0, 264, (max(3, longest - 5 * i),), generator=L.gen(i)).tolist() for i in range(requests)]
 
     def alone(t):
         s = Scheduler(m, longest + 1)
@@ -94,6 +100,28 @@ def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
         order = list(range(requests))[::-1] if step else list(range(requests))
         got = sched.step(order, [[toks[i][len(toks[i]) - 2 + step]] for i in order])
         assert L.logit_err(got, torch.stack([want[i][step] for i in order])) < 4 * 2 ** -8
+
+
+def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17)):
+    """Prompts of several requests packed into one step against each prompt alone, logits at places inside and at the end, and a step on the caches that they
+    left; rounding as in ``case_gptfast_decode_batch`` (the flash kernel's probabilities included)."""
+    from aria_amd.serving import Scheduler
+
+    m = gptfast_routed(dev, dim, 64, 128, max(lens) + 8)
+    toks = [torch.randint(0, 264, (n + 1,), generator=L.gen(n)).tolist() for n in lens]
+    places = [sorted({0, n // 2, n - 1}) for n in lens]
+    want = []
+    for t, p in zip(toks, places):
+        s = Scheduler(m, max(lens) + 2)
+        want.append((s.step(["x"], [t[:-1]], [p]).cpu().double(), s.step(["x"], [t[-1:]]).cpu().double()))
+    sched = Scheduler(m, max(lens) + 2)
+    ids = list(range(len(lens)))
+    assert m.layers[0].attention.kv_cache.k.shape[0] == 1      # (set up again for the batch)
+    got = sched.step(ids, [t[:-1] for t in toks], places)
+    assert L.logit_err(got, torch.cat([w[0] for w in want])) < 4 * 2 ** -8
+    got = sched.step(ids, [t[-1:] for t in toks])
+    assert L.logit_err(got, torch.cat([w[1] for w in want])) < 4 * 2 ** -8
+    assert sched.step(ids[:1], [[1]], [[]]) is None
 
 
 def case_gptfast_generate(dev):

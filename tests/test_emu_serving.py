@@ -19,6 +19,10 @@ def test_gptfast_decode_batch():
     C.case_gptfast_decode_batch(DEV, 128, 64, 128, 3)
 
 
+def test_gptfast_packed_prompts():
+    C.case_gptfast_packed_prompts(DEV, 128, (5, 1, 9))
+
+
 def test_gptfast_batch():
     C.case_gptfast_batch(DEV, engine=False)   # (the engine's emulated form takes a minute: on hardware only)
 

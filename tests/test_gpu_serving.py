@@ -27,6 +27,11 @@ def test_gptfast_decode_batch(dim, head_dim, inter, requests, longest):
     C.case_gptfast_decode_batch(DEV, dim, head_dim, inter, requests, longest)
 
 
+def test_gptfast_packed_prompts():
+    C.case_gptfast_packed_prompts(DEV)
+    C.case_gptfast_packed_prompts(DEV, 1024, (300, 64, 65, 2, 129))
+
+
 @pytest.mark.parametrize("engine", [False, True])
 def test_gptfast_batch(engine):
     C.case_gptfast_batch(DEV, engine)
