@@ -251,6 +251,19 @@ __device__ __forceinline__ f32x16 mfma32(s16x8 a, s16x8 b, f32x16 c) {
 // D = A(16x32) * B(32x16) + C.
 //   A fragment: lane l holds A[l & 15][8 * (l >> 4) + 0..7];  B: B[8 * (l >> 4) + 0..7][l & 15]
 //   C/D: reg r of lane l is C[4 * (l >> 4) + r][l & 15]
+// v_mfma_f32_16x16x4_f32, true 32-bit: a = A[l & 15][l >> 4], b = B[l >> 4][l & 15]; the result lies as mfma16's
+__device__ __forceinline__ f32x4 mfma16_f32(float a, float b, f32x4 c) {
+#ifdef ARIA_EMU
+    const int l = emu::lane();
+    for (int k = 0; k < 4; ++k) {
+        const float bk = emu::shfl(b, 16 * k + (l & 15));
+        for (int r = 0; r < 4; ++r) c[r] = std::fma(emu::shfl(a, 16 * k + 4 * (l >> 4) + r), bk, c[r]);
+    }
+    return c;
+#else
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+#endif
+}
 __device__ __forceinline__ f32x4 mfma16(s16x8 a, s16x8 b, f32x4 c) {
 #ifdef ARIA_EMU
     struct AB { s16x8 a, b; };
