@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void embedding_rows_kernel(const int32_t* ids,
 }
 
 struct StoreBf16 {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     bf16_t* out;
     long long ld;
     float* sums = nullptr;
@@ -48,7 +48,7 @@ struct StoreBf16 {
     }
 };
 struct StoreF32 {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     float* out;
     long long ld;
     float* sums = nullptr;
@@ -58,7 +58,7 @@ struct StoreF32 {
     }
 };
 struct Residual {   // x += the rounded product; the next norm's input beside it
-    static constexpr bool SUMSQ = true;
+    static constexpr bool SUMSQ = true, WAVES = false;
     bf16_t *x, *h;
     const bf16_t* norm;
     long long D;

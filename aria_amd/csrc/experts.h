@@ -83,26 +83,29 @@ namespace {
 // 512 places: 110 us; as one sequence 93).
 template <int NW, int KS, class Ep, bool PAIR>
 __global__ __launch_bounds__(NW * 64) void expert_rows_kernel(ExpertIn in, ExpertLists lists, Ep e) {
-    ARIA_SMEM_STATIC RowsRed<NW, PAIR> red;
+    ARIA_SMEM_STATIC RowsRed<NW, 1> red;
     ARIA_SMEM_STATIC int entries[16];
-    const int groups = (in.N + 15) / 16, total = lists.table[0] * groups, per = (total + int(gridDim.x) - 1) / int(gridDim.x), t = threadIdx.x;
-    const int end = min(total, (int(blockIdx.x) + 1) * per);
+    constexpr int OUT = PAIR ? 8 : 16;
+    const int groups = (in.N + OUT - 1) / OUT, total = lists.table[0] * groups, per = (total + int(gridDim.x) - 1) / int(gridDim.x), t = threadIdx.x;
+    const int end = min(total, (int(blockIdx.x) + 1) * per), c16 = t & 15;
     int g = int(blockIdx.x) * per;
     while (g < end) {
         const int a = g / groups, g0 = g - a * groups, g1 = min(groups, g0 + end - g);
         const int first = lists.table[1 + lists.E + a], m = lists.table[2 + lists.E + a] - first;
         const int id = lists.table[1 + a];
         const bool all = id >= in.E;
-        const long long at = all ? (id - in.E) * in.s_step : (long long)id * in.N * in.K;
-        const bf16_t *W = (all ? in.S : in.W) + at, *W2 = PAIR ? (all ? in.S2 : in.W2) + at : nullptr;
+        const long long at = all ? (id - in.E) * in.s_step : (long long)id * in.N * in.K, ldw = all ? in.s_ld : (long long)in.K;
+        const bf16_t* W = (PAIR && c16 >= 8 ? (all ? in.S2 : in.W2) : (all ? in.S : in.W)) + at;
         for (int t0 = 0; t0 < m; t0 += 16) {   // (more than 16 only where tokens chose an expert several times: NaN logits)
             sync();                            // (red and entries of the piece before are read)
-            const int mine = lists.list[first + min(t0 + (t & 15), m - 1)];
+            const int mine = lists.list[first + min(t0 + c16, m - 1)];
             if (t < 16) entries[t] = mine;     // (published by the first group's barrier)
-            stream_rows<NW, KS, PAIR>(W, W2, all ? in.s_ld : (long long)in.K, in.K, in.N, in.X + (long long)(mine / in.div) * in.ldx, g0, g1, red,
-                                      [&](float v, float u, int tok, int n, int) {
-                                          if (t0 + tok < m && n < in.N) e(v, u, entries[tok], n);
-                                      });
+            stream_rows<NW, KS, 1>(
+                in.K, [&](int gg) { return W + (long long)min(gg * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * ldw; },
+                [&](int) { return in.X + (long long)(mine / in.div) * in.ldx; }, g0, g1, red, [&](float v, int tok, int n, int gg) {
+                    const float u = PAIR ? shfl_xor(v, 8) : 0.f;
+                    if (t0 + tok < m && gg * OUT + n < in.N && n < OUT) e(v, u, entries[tok], gg * OUT + n);
+                });
         }
         g += g1 - g0;
     }
@@ -124,7 +127,7 @@ inline bool expert_rows_take(int64_t K0, int64_t K1, int64_t E, int64_t k, int64
 
 template <bool PAIR, class Ep>
 int launch_expert_rows(const ExpertIn& in, const ExpertLists& lists, int64_t k, int64_t T, const Ep& e, void* stream) {
-    const int64_t most = (in.N + 15) / 16 * std::min<int64_t>(lists.E, T * k);
+    const int64_t most = (in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16) * std::min<int64_t>(lists.E, T * k);
     const dim3 grid(unsigned(std::min<int64_t>(512, most)));   // two workgroups a CU are resident
 #define ARIA_ROWS(NW, KS) ARIA_LAUNCH((expert_rows_kernel<NW, KS, Ep, PAIR>), grid, dim3(NW * 64), 0, stream, in, lists, e);
     ARIA_ROWS_SHAPE(in.K, ARIA_ROWS, return ARIA_ERR_UNSUPPORTED;)

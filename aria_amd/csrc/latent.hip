@@ -321,7 +321,7 @@ struct RowsOut {
 };
 template <int MODE>
 struct LatentRows {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     RowsOut ro;
     float* sums = nullptr;
     __device__ __forceinline__ float operator()(float v, int tok, int n, int) const {

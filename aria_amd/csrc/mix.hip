@@ -15,7 +15,7 @@ using namespace ad;
 typedef AriaChunkShape Chunk;
 
 struct StoreRows {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     bf16_t* out[2];   // per problem
     long long ldo;
     float* sums = nullptr;
@@ -26,7 +26,7 @@ struct StoreRows {
 };
 // input projection of a layer with chunk attention: keys and values also go to the token's cache row
 struct StoreRowsAndCache {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     bf16_t *out, *cache;
     Chunk s;
     const int32_t *slot, *pos;
@@ -45,7 +45,7 @@ struct StoreRowsAndCache {
 };
 // x += mult v (+ embedding rows); h = x times the next norm's weight, 1 / rms left to the reader
 struct ResidualRows {
-    static constexpr bool SUMSQ = true;
+    static constexpr bool SUMSQ = true, WAVES = false;
     float *x, *sums;
     bf16_t* h;
     const float* w;
@@ -63,7 +63,7 @@ struct ResidualRows {
     }
 };
 struct ReluGate {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     bf16_t* act;
     long long ff;
     float* sums = nullptr;
@@ -74,7 +74,7 @@ struct ReluGate {
     __device__ __forceinline__ float operator()(float, int, int, int) const { return 0.f; }
 };
 struct CappedLogits {
-    static constexpr bool SUMSQ = false;
+    static constexpr bool SUMSQ = false, WAVES = false;
     float* out;
     long long V;
     float cap;

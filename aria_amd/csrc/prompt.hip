@@ -1,0 +1,113 @@
+// A serving step over short prompts of the gptfast (Aria) decoder in one call: packed tokens of one or several sequences, every product by the row-streaming
+// kernels of wide.hip.  At these sizes a layer is fifteen launches of 5 .. 230 us; enqueued one by one from Python they take longer than they run (four
+// layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
+#include "decode.h"
+#include <algorithm>
+
+namespace {
+using namespace ad;
+
+__global__ __launch_bounds__(256) void prompt_rows_kernel(const int32_t* ids, const bf16_t* table, bf16_t* x, int nch, int T, int V, int32_t* counts, int n_counts) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n_counts) counts[i] = 0;
+    if (i >= T * nch) return;
+    const int t = i / nch, c = i - t * nch;
+    st16(x + (long long)i * 8, ld16(table + ((long long)min(max(ids[t], 0), V - 1) * nch + c) * 8));
+}
+
+struct Scratch {
+    bf16_t *x, *y, *h, *qkv, *ao, *d, *logits, *scores, *act, *eo, *sact, *sh;
+    int32_t *idx, *counts, *offsets, *src, *inv, *rows;
+    int64_t bytes;
+};
+Scratch layout(const int64_t* dims, int64_t T, char* base) {
+    const int64_t L = dims[0], D = dims[1], E = dims[4], k = dims[5], I = dims[6], Is = dims[7];
+    Scratch z{};
+    int64_t at = 0;
+    auto take = [&](int64_t bytes) {
+        char* p = base + at;
+        at += (bytes + 255) & ~int64_t(255);
+        return p;
+    };
+    auto rows = [&](int64_t n) { return reinterpret_cast<bf16_t*>(take(2 * T * n)); };
+    z.x = rows(D), z.y = rows(D), z.h = rows(D), z.qkv = rows(3 * D), z.ao = rows(D), z.d = rows(D), z.logits = rows(E), z.scores = rows(k);
+    z.act = rows(k * I), z.eo = rows(k * D), z.sact = rows(Is), z.sh = rows(D);
+    auto ints = [&](int64_t n) { return reinterpret_cast<int32_t*>(take(4 * n)); };
+    z.idx = ints(T * k), z.counts = ints(L * E), z.offsets = ints(E + 1), z.src = ints(T * k), z.inv = ints(T * k), z.rows = ints(T * k);
+    z.bytes = at;
+    return z;
+}
+bool prompt_ok(const int64_t* d, int64_t T) {
+    const int64_t D = d[1], E = d[4], k = d[5], I = d[6], Is = d[7];
+    return aria_decode_dims_ok(d) == ARIA_OK && E <= 64 && k >= 1 && k <= E && T * k <= std::min<int64_t>(8192, 27 * E) && D >= 512 && D <= 2560 && I >= 512 && I <= 2560 && Is <= 4096 &&
+           D % 16 == 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t aria_prompt_step_scratch(const int64_t* dims, int64_t T) {
+    return dims && T > 0 && prompt_ok(dims, T) ? layout(dims, T, nullptr).bytes : 0;
+}
+
+int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+                     const int32_t* cu, int64_t n_seq, int64_t longest, const int32_t* wanted, int64_t n_wanted, float* logits, void* scratch,
+                     int64_t scratch_bytes, void* stream) {
+    if (!ptrs || !dims || !ids || !slot || !pos || !cu || !scratch || T < 0 || n_seq <= 0 || longest <= 0 || n_wanted < 0 || (n_wanted && (!wanted || !logits)))
+        return ARIA_ERR_INVALID;
+    if (T == 0) return ARIA_OK;
+    if (reinterpret_cast<uintptr_t>(scratch) & 15) return ARIA_ERR_ALIGN;
+    const int64_t need = aria_prompt_step_scratch(dims, T);
+    if (need == 0) return ARIA_ERR_UNSUPPORTED;
+    const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8], Smax = dims[9];
+    if (scratch_bytes < need || longest > Smax || n_wanted > T) return ARIA_ERR_INVALID;
+    for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
+        if (!ptrs[i]) return ARIA_ERR_INVALID;
+    const Scratch z = layout(dims, T, static_cast<char*>(scratch));
+    const int64_t items = std::max(T * (D / 8), L * E);
+    ARIA_LAUNCH(prompt_rows_kernel, dim3(unsigned((items + 255) / 256)), dim3(256), 0, stream, ids, static_cast<const bf16_t*>(ptrs[3]), z.x, int(D / 8), int(T), int(V),
+                z.counts, int(L * E));
+    int rc = aria_check_launch();
+    bf16_t *x = z.x, *y = z.y;   // the residual before and behind the sum that comes next
+    const bf16_t* delta = nullptr;
+#define ARIA_TRY(call) \
+    if (rc == ARIA_OK) rc = (call)
+    for (int64_t li = 0; li < L; ++li) {
+        const void* const* p = ptrs + ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * li;
+        void *kc = const_cast<void*>(p[11]), *vc = const_cast<void*>(p[12]);
+        if (delta) {
+            ARIA_TRY(aria_rmsnorm_fwd(delta, x, p[0], y, z.h, nullptr, T, D, eps, stream));
+            std::swap(x, y);
+        } else {
+            ARIA_TRY(aria_rmsnorm_fwd(x, nullptr, p[0], nullptr, z.h, nullptr, T, D, eps, stream));
+        }
+        ARIA_TRY(aria_rows_gemm(z.h, p[1], z.qkv, 0, T, 3 * D, D, D, 3 * D, stream));
+        ARIA_TRY(aria_rope_cache_rows(z.qkv, ptrs[0], slot, pos, kc, vc, T, H, hd, Smax, stream));
+        ARIA_TRY(aria_attn_varlen_fwd(z.qkv, z.qkv + D, z.qkv + 2 * D, z.ao, cu, nullptr, n_seq, longest, H, H, hd, hd, 3 * D, 3 * D, 3 * D, D, 0,
+                                      1.0f / sqrtf(float(hd)), stream));
+        ARIA_TRY(aria_rows_gemm(z.ao, p[2], z.d, 0, T, D, D, D, D, stream));
+        ARIA_TRY(aria_rmsnorm_fwd(z.d, x, p[3], y, z.h, nullptr, T, D, eps, stream));
+        std::swap(x, y);
+        ARIA_TRY(aria_rows_gemm(z.h, p[4], z.logits, 0, T, E, D, D, E, stream));
+        ARIA_TRY(aria_route_and_sort(z.logits, z.scores, z.idx, z.counts + li * E, z.offsets, z.src, z.inv, z.rows, int(T), int(E), int(k), stream));
+        ARIA_TRY(aria_rows_experts(z.h, z.rows, z.offsets, p[5], p[6], z.act, E, T * k, I, D, D, I, stream));
+        if (T * k <= 4 * E) {   // (beyond: the tiles, see wide.hip)
+            ARIA_TRY(aria_rows_experts(z.act, nullptr, z.offsets, p[7], nullptr, z.eo, E, T * k, D, I, I, D, stream));
+        } else {
+            ARIA_TRY(aria_grouped_gemm_bf16(z.act, p[7], z.eo, z.offsets, E, T * k, D, I, 0, I, I, D * I, D, stream));
+        }
+        ARIA_TRY(aria_rows_swiglu(z.h, p[8], p[9], z.sact, T, Is, D, D, Is, stream));
+        ARIA_TRY(aria_rows_gemm(z.sact, p[10], z.sh, 0, T, D, Is, Is, D, stream));
+        ARIA_TRY(aria_moe_unpermute(z.eo, z.inv, z.scores, z.sh, z.d, T, D, k, stream));
+        delta = z.d;
+    }
+    if (n_wanted == 0) return rc;
+    ARIA_TRY(aria_rmsnorm_fwd(delta, x, ptrs[1], y, z.h, nullptr, T, D, eps, stream));
+    ARIA_TRY(aria_moe_permute(z.h, wanted, z.ao, n_wanted, D, 1, D, stream));
+    ARIA_TRY(aria_rows_gemm(z.ao, ptrs[2], logits, 1, n_wanted, V, D, D, V, stream));
+#undef ARIA_TRY
+    return rc;
+}
+
+}  // extern "C"

@@ -1,6 +1,6 @@
 // Row-streaming projections of 1 .. 16 tokens (bf16): the decode steps' matrix products, each with its consumer's elementwise work as an epilogue.
 //
-// An epilogue E is called once per output, e(value, token, row, problem).  E::SUMSQ: it returns the square of what it stored and offers `sums`, which
+// An epilogue E is called once per output, e(value, token, row, problem) (E::WAVES: by whole waves, e(value, token, row, in range)).  E::SUMSQ: it returns the square of what it stored and offers `sums`, which
 // receives per token and workgroup the sum of those squares -- partial sums for an RMS norm whose 1 / rms the CONSUMER of the stored rows applies to its
 // results (RowsIn::sq): W (r x) = r (W x), so no launch of its own stands between the two.
 #pragma once
@@ -102,70 +102,74 @@ __global__ __launch_bounds__(256) void row_kernel(RowsPair rp, E e) {
         if (t == 0) e.sums[blockIdx.x] = (red[4] + red[5]) + (red[6] + red[7]);
     }
 }
-// 2 .. 16 tokens: a workgroup of NW waves runs through the groups [g0, g1) of 16 weight rows (PAIR: 16 gate rows, then the 16 up rows of the same
-// outputs).  Tokens are the rows of A, weight rows the columns of B: both k-contiguous in memory, so fragments come straight from global memory, and
-// the matrix pipe takes the multiply-adds of all tokens at the price of one.  Wave w owns the KS 32-column steps of the reduction that start at
-// column 32 KS w: its part of the tokens is loaded ONCE and stays in registers, and a weight fragment's register is refilled with the next group's as
-// soon as it is used, so up to 16 kilobytes a wave are in flight without a break between the groups.  The NW partial results meet in LDS (two images in
-// turn: one barrier a group), where a quarter of the threads at a time sums them and calls out(value, up value, token row, weight row, group).
+// Several tokens: a workgroup of NW waves runs through the groups [g0, g1) of 16 weight rows with MT x 16 tokens.  Tokens are the rows of A, weight rows
+// the columns of B: both k-contiguous in memory, so fragments come straight from global memory, and the matrix pipe takes the multiply-adds of sixteen tokens
+// at the price of one.  Wave w owns the KS 32-column steps of the reduction that start at column 32 KS w: its part of the tokens is loaded ONCE and stays
+// in registers, and a weight fragment's register is refilled with the next group's as soon as it is used, so up to 16 kilobytes a wave are in flight
+// without a break between the groups.  The NW partial results meet in LDS (two images in turn: one barrier a group), where whole waves sum them and call
+// out(value, token, column of the group, group).  wrow(g): this lane's weight row of group g, xrow(i): its token row of tile i; both from column 0.
 // (Plain loads: a fragment touches half a cache line of 16 rows and the next one the other half, which a non-temporal hint fetches twice.)
-template <int NW, bool PAIR>
+template <int NW, int MT>
 struct RowsRed {
-    float v[2][PAIR ? 2 : 1][NW][16][17];
+    float v[2][NW][16 * MT][17];
 };
-template <int NW, int KS, bool PAIR, class Out>
-__device__ __forceinline__ void stream_rows(const bf16_t* W, const bf16_t* W2, long long ldw, int K, int N, const bf16_t* xp, int g0, int g1, RowsRed<NW, PAIR>& red,
-                                            const Out& out) {
-    constexpr int SUB = PAIR ? 2 : 1, DEPTH = KS <= 16 ? KS : KS / 2;   // fragments in flight
+template <int NW, int KS, int MT, class WRow, class XRow, class Out>
+__device__ __forceinline__ void stream_rows(int K, const WRow& wrow, const XRow& xrow, int g0, int g1, RowsRed<NW, MT>& red, const Out& out) {
+    constexpr int DEPTH = KS <= 16 ? KS : KS / 2;   // fragments in flight
     static_assert(KS % DEPTH == 0, "a step keeps its register");
     const int t = threadIdx.x, l = t & 63, w = t >> 6, q4 = l >> 4, c16 = l & 15;
     // the last waves' windows are moved down into the row, the columns that another wave owns zeroed in the tokens: every address is base + constant
     const int own = w * KS * 32, k0 = min(own, K - KS * 32) + q4 * 8;
-    xp += k0;
-    u32x4 x[KS], b[DEPTH];
-    const bf16_t* wp = W + (long long)min(g0 * 16 + c16, N - 1) * ldw + k0;
+    u32x4 x[MT][KS], b[DEPTH];
+    const bf16_t* wp = wrow(g0) + k0;
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) b[u] = ld16(wp + 32 * u);
 #pragma unroll
-    for (int u = 0; u < KS; ++u) x[u] = ld16(xp + 32 * u);
+    for (int i = 0; i < MT; ++i) {
+        const bf16_t* xp = xrow(i) + k0;
 #pragma unroll
-    for (int u = 0; u < KS; ++u)
+        for (int u = 0; u < KS; ++u) x[i][u] = ld16(xp + 32 * u);
+    }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[u][q] = k0 + 32 * u >= own ? x[u][q] : 0u;
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int u = 0; u < KS; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[i][u][q] = k0 + 32 * u >= own ? x[i][u][q] : 0u;
     for (int g = g0; g < g1; ++g) {
         const int ph = (g - g0) & 1;
+        f32x4 acc[MT];   // (one chain a tile whatever MT is: a token's sums do not depend on how many tokens there are)
 #pragma unroll
-        for (int sub = 0; sub < SUB; ++sub) {
-            f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-            const bool up_next = PAIR && sub == 0, more = up_next || g + 1 < g1;
-            const bf16_t *cur = wp, *nxt = (up_next ? W2 : W) + (long long)min((up_next ? g : g + 1) * 16 + c16, N - 1) * ldw + k0;
-            wp = nxt;
-            if (more) {
+        for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const bf16_t* cur = wp;
+        if (g + 1 < g1) {
+            wp = wrow(g + 1) + k0;
 #pragma unroll
-                for (int u = 0; u < KS; ++u) {
-                    acc[u & 1] = mfma16(__builtin_bit_cast(s16x8, x[u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[u & 1]);
-                    b[u % DEPTH] = ld16(u + DEPTH < KS ? cur + 32 * (u + DEPTH) : nxt + 32 * (u + DEPTH - KS));
-                }
-            } else {
+            for (int u = 0; u < KS; ++u) {
 #pragma unroll
-                for (int u = 0; u < KS; ++u) {
-                    acc[u & 1] = mfma16(__builtin_bit_cast(s16x8, x[u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[u & 1]);
-                    if (u + DEPTH < KS) b[u % DEPTH] = ld16(cur + 32 * (u + DEPTH));
-                }
+                for (int i = 0; i < MT; ++i) acc[i] = mfma16(__builtin_bit_cast(s16x8, x[i][u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[i]);
+                b[u % DEPTH] = ld16(u + DEPTH < KS ? cur + 32 * (u + DEPTH) : wp + 32 * (u + DEPTH - KS));
             }
+        } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red.v[ph][sub][w][4 * q4 + r][c16] = acc[0][r] + acc[1][r];
+            for (int u = 0; u < KS; ++u) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[i] = mfma16(__builtin_bit_cast(s16x8, x[i][u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[i]);
+                if (u + DEPTH < KS) b[u % DEPTH] = ld16(cur + 32 * (u + DEPTH));
+            }
         }
-        sync();
-        if ((t >> 8) == ((g - g0) & (NW / 4 - 1))) {   // (whole waves: 256 sums)
-            const int tok = (t >> 4) & 15, n = t & 15;
-            float v = 0.f, u = 0.f;
 #pragma unroll
-            for (int ww = 0; ww < NW; ++ww) {
-                v += red.v[ph][0][ww][tok][n];
-                if (PAIR) u += red.v[ph][SUB - 1][ww][tok][n];
-            }
-            out(v, u, tok, g * 16 + n, g);
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red.v[ph][w][16 * i + 4 * q4 + r][c16] = acc[i][r];
+        sync();
+        // (whole waves; one tile of sums: the halves of the workgroup in turn)
+        for (int i = MT == 1 ? ((t >> 8) == ((g - g0) & (NW / 4 - 1)) ? t & 255 : 256) : t; i < 256 * MT; i += NW * 64) {
+            const int tok = i >> 4, n = i & 15;
+            float v = 0.f;
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww) v += red.v[ph][ww][tok][n];
+            out(v, tok, n, g);
         }
     }
 }
@@ -179,32 +183,37 @@ __device__ __forceinline__ void token_rms(float* rms, const RowsIn& in, int t0, 
         if (l == 0) rms[i] = 1.f / sqrtf(s * in.inv_n + in.eps);
     }
 }
-template <int NW, int KS, class E, bool PAIR>
+// PAIR: a group is 8 gate rows and the 8 up rows of the same outputs
+template <int NW, int KS, int MT, class E, bool PAIR>
 __global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, int per, E e) {
-    ARIA_SMEM_STATIC RowsRed<NW, PAIR> red;
+    ARIA_SMEM_STATIC RowsRed<NW, MT> red;
     ARIA_SMEM_STATIC float rms[16];
+    constexpr int OUT = PAIR ? 8 : 16;
     const RowsIn& in = rp.in[blockIdx.z];
-    const int c16 = threadIdx.x & 15, t0 = blockIdx.y * 16, groups = (in.N + 15) / 16, g0 = blockIdx.x * per;
-    if (in.sq) token_rms(rms, in, t0, n_tok, NW);   // (published by the first group's barrier)
-    stream_rows<NW, KS, PAIR>(in.W, in.W2, in.K, in.K, in.N, in.X + (long long)min(t0 + c16, n_tok - 1) * in.ldx, g0, min(groups, g0 + per), red,
-                              [&](float v, float u, int tok, int n, int g) {
-                                  const bool in_range = t0 + tok < n_tok && n < in.N;
-                                  float s = 0.f;
-                                  if (in_range) {
-                                      if (in.sq) {
-                                          v *= rms[tok];
-                                          u *= rms[tok];
-                                      }
-                                      if constexpr (PAIR)
-                                          e(v, u, t0 + tok, n);
-                                      else
-                                          s = e(v, t0 + tok, n, int(blockIdx.z));
-                                  }
-                                  if constexpr (E::SUMSQ) {   // sixteen lanes hold a token's outputs
-                                      s = group_sum<16>(s);
-                                      if ((n & 15) == 0 && t0 + tok < n_tok) e.sums[(long long)(t0 + tok) * groups + g] = s;
-                                  }
-                              });
+    const int c16 = threadIdx.x & 15, t0 = blockIdx.y * 16 * MT, groups = (in.N + OUT - 1) / OUT, g0 = blockIdx.x * per;
+    if (MT == 1 && in.sq) token_rms(rms, in, t0, n_tok, NW);   // (published by the first group's barrier)
+    const bf16_t* W = PAIR && c16 >= 8 ? in.W2 : in.W;
+    stream_rows<NW, KS, MT>(
+        in.K, [&](int g) { return W + (long long)min(g * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * in.K; },
+        [&](int i) { return in.X + (long long)min(t0 + 16 * i + c16, n_tok - 1) * in.ldx; }, g0, min(groups, g0 + per), red,
+        [&](float v, int tok, int n, int g) {
+            const float u = PAIR ? shfl_xor(v, 8) : 0.f;
+            const int row = g * OUT + n;
+            const bool in_range = t0 + tok < n_tok && row < in.N && n < OUT;
+            const float r = MT == 1 && in.sq && in_range ? rms[tok] : 1.f;
+            float s = 0.f;
+            if constexpr (PAIR) {
+                if (in_range) e(v * r, u * r, t0 + tok, row);
+            } else if constexpr (E::WAVES) {   // (all lanes: the epilogue exchanges values)
+                e(v, t0 + tok, row, in_range);
+            } else if (in_range) {
+                s = e(v * r, t0 + tok, row, int(blockIdx.z));
+            }
+            if constexpr (E::SUMSQ) {   // sixteen lanes hold a token's outputs
+                s = group_sum<16>(s);
+                if (n == 0 && t0 + tok < n_tok) e.sums[(long long)(t0 + tok) * groups + g] = s;
+            }
+        });
 }
 // any reduction (below a wave's window of stream_rows or beyond what it holds in registers): the 8 waves on interleaved 128-column blocks of it, a workgroup per 16 rows
 template <class E, bool PAIR>
@@ -304,17 +313,60 @@ inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std
     else                                \
         OTHER
 
+// The same for up to a few hundred tokens: 16, 32 or 64 at a time past the weights, as many as the registers hold beside a wave's window of the
+// reduction.  K < 128 or > 4096: not served.
+inline int rows_tiles(int64_t K, int64_t T) {
+    const int most = K <= 2560 ? 4 : 2, need = int((T + 15) / 16);
+    return need <= 1 ? 1 : need <= 2 ? 2 : most;
+}
+template <bool PAIR, class E>
+int launch_rows_wide(const RowsIn& in, int64_t T, const E& e, void* stream) {
+    const RowsPair rp{{in, in}};
+    const int mt = rows_tiles(in.K, T);
+    const int64_t groups = (in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), ty = (T + 16 * mt - 1) / (16 * mt);
+    const int per = rows_per_workgroup(groups, ty);
+    const dim3 grid(unsigned((groups + per - 1) / per), unsigned(ty));
+#define ARIA_WIDE(KS, MT) ARIA_LAUNCH((rows_kernel<8, KS, MT, E, PAIR>), grid, dim3(512), 0, stream, rp, int(T), per, e)
+#define ARIA_WIDE_TILES(KS)  \
+    if (mt == 1)             \
+        ARIA_WIDE(KS, 1);    \
+    else if (mt == 2)        \
+        ARIA_WIDE(KS, 2);    \
+    else                     \
+        ARIA_WIDE(KS, 4)
+    if (in.K < 128 || in.K > 4096) return ARIA_ERR_UNSUPPORTED;
+    if (in.K <= 1024) {
+        ARIA_WIDE_TILES(4);
+    } else if (in.K <= 1792) {
+        ARIA_WIDE_TILES(7);
+    } else if (in.K <= 2560) {
+        ARIA_WIDE_TILES(10);
+    } else if (in.K <= 3328) {
+        if (mt == 1)
+            ARIA_WIDE(13, 1);
+        else
+            ARIA_WIDE(13, 2);
+    } else if (mt == 1) {
+        ARIA_WIDE(16, 1);
+    } else {
+        ARIA_WIDE(16, 2);
+    }
+#undef ARIA_WIDE
+#undef ARIA_WIDE_TILES
+    return aria_check_launch();
+}
+
 template <bool PAIR, class E>
 int launch_rows_of(const RowsPair& rp, int problems, int64_t T, const E& e, void* stream) {
-    const int64_t groups = (rp.in[0].N + 15) / 16;
+    const int64_t groups = (rp.in[0].N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), long_groups = (rp.in[0].N + 15) / 16;
     const int per = rows_per_workgroup(groups, problems), other = rp.in[problems - 1].K;
     const int K = std::max(rp.in[0].K, other), least = std::min(rp.in[0].K, other);
     const dim3 grid(unsigned((groups + per - 1) / per), unsigned((T + 15) / 16), unsigned(problems));
-#define ARIA_ROWS_LONG ARIA_LAUNCH((rows_long_kernel<E, PAIR>), dim3(unsigned(groups), grid.y, grid.z), dim3(512), 0, stream, rp, int(T), e);
+#define ARIA_ROWS_LONG ARIA_LAUNCH((rows_long_kernel<E, PAIR>), dim3(unsigned(long_groups), grid.y, grid.z), dim3(512), 0, stream, rp, int(T), e);
 #define ARIA_ROWS(NW, KS)                                                                                                     \
     {                                                                                                                         \
         if (least >= KS * 32) /* (a wave's window lies inside the shorter reduction too) */                                   \
-            ARIA_LAUNCH((rows_kernel<NW, KS, E, PAIR>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);                  \
+            ARIA_LAUNCH((rows_kernel<NW, KS, 1, E, PAIR>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);                  \
         else                                                                                                                  \
             ARIA_ROWS_LONG                                                                                                    \
     }

@@ -100,6 +100,11 @@ def _glu_pair_ready(w_gate: nn.Parameter, w_up: nn.Parameter) -> bool:
     return False
 
 
+def _project(x2d: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T: the row-streaming kernel for few tokens, the tile product beyond"""
+    return ops.rows_gemm(x2d, w) if ops.rows_take(*x2d.shape) and w.is_contiguous() else ops.gemm(x2d, w)
+
+
 class RMSNorm(nn.Module):
     def __init__(self, dim: int, eps: float):
         super().__init__()
@@ -145,10 +150,13 @@ class Attention(nn.Module):
             # rotation nor the cache row depends on a device tensor nobody validated.  A prompt longer than the cache takes the
             # path below, whose copy raises.
             cache = self.kv_cache
-            q = ops.gemm_qkv_rope_cache(x2d, self.wqkv.weight, freqs_cis, None, cache.k, cache.v, S, hd)
+            if ops.rows_take(S, D) and self.wqkv.weight.is_contiguous():
+                q = ops.rows_qkv_rope_cache(x2d, self.wqkv.weight, freqs_cis, cache.k[:1], cache.v[:1], hd)
+            else:
+                q = ops.gemm_qkv_rope_cache(x2d, self.wqkv.weight, freqs_cis, None, cache.k, cache.v, S, hd)
             o, _ = ops.attention_fwd(q, cache.k[0, :S], cache.v[0, :S], 1, S, H, hd, hd ** -0.5, True)
-            return ops.gemm(o, self.wo.weight)
-        qkv = ops.gemm(x2d, self.wqkv.weight)
+            return _project(o, self.wo.weight)
+        qkv = _project(x2d, self.wqkv.weight)
         ops.rope_interleaved_(qkv[:, :2 * D], freqs_cis, 2 * H, hd, pos32)
         q, k, v = qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:]
         if hdp != hd:  # toy head dims only (tests)
@@ -169,7 +177,7 @@ class Attention(nn.Module):
                                      kv_len=kv_len, Skv=Smax)
         if hdp != hd:
             o = Fn._unpad_heads(o, H, hd, hdp).contiguous()
-        return ops.gemm(o, self.wo.weight)
+        return _project(o, self.wo.weight)
 
 
     def packed(self, x2d, freqs_cis, batch):
@@ -177,9 +185,9 @@ class Attention(nn.Module):
         each sequence."""
         c = self.config
         D, H, hd = c.dim, c.n_head, c.head_dim
-        qkv = ops.rope_cache_rows_(ops.gemm(x2d, self.wqkv.weight), freqs_cis, batch.slot, batch.pos, self.kv_cache.k, self.kv_cache.v, H, hd)
+        qkv = ops.rope_cache_rows_(_project(x2d, self.wqkv.weight), freqs_cis, batch.slot, batch.pos, self.kv_cache.k, self.kv_cache.v, H, hd)
         o = ops.attention_varlen(qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:], batch.cu, batch.longest, H, hd, hd, hd ** -0.5)
-        return ops.gemm(o, self.wo.weight)
+        return _project(o, self.wo.weight)
 
 
 class ConditionalFeedForward(nn.Module):
@@ -205,14 +213,19 @@ class MOEFeedForward(nn.Module):
 
     def forward(self, x2d):
         k = self.config.router_topk
-        if ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
+        few = ops.rows_take(*x2d.shape)   # few tokens: every product is bound by its weights
+        if not few and ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
             logits, scores, idx, counts = ops.moe_router_fused(x2d, self.gate.weight, k)
         else:
-            logits = ops.gemm(x2d, self.gate.weight)
+            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 45 us for 280 tokens, 12 in two launches)
             scores, idx, counts = ops.moe_route(logits, k)             # topk + softmax (model.py:359-363)
         offsets, sorted_src, inv = ops.moe_sort(idx, counts)           # token_permutation (:243-254)
         cf = self.cond_ffn
-        if _glu_pair_ready(cf.w1, cf.w3) and ops.gather_fusable(x2d.shape[1]):
+        E, I, D = cf.w1.shape
+        contiguous = all(w.is_contiguous() for w in (cf.w1, cf.w2, cf.w3))
+        if contiguous and ops.rows_experts_take(sorted_src.numel(), E, D, I):
+            act = ops.rows_experts(x2d, cf.w1, offsets, ops.permuted_token_rows(sorted_src, k), cf.w3)
+        elif _glu_pair_ready(cf.w1, cf.w3) and ops.gather_fusable(x2d.shape[1]):
             # K2 + K3: the dispatcher's row gather (model.py:243-254) in the A loader of the fused w1 / w3 / SwiGLU launch -- no permuted copy
             # of the tokens ([6T, D]: 1.6 GB written and read per layer of a 53 K-token prefill), no h1 / h3 round trip
             act = ops.grouped_gemm_swiglu_split_gather(x2d, ops.permuted_token_rows(sorted_src, k), cf.w1, cf.w3, offsets)[1]
@@ -223,13 +236,16 @@ class MOEFeedForward(nn.Module):
             h1 = ops.grouped_gemm(perm, cf.w1, offsets, w_is_kn=False)     # sequential_gemm(w1) (:278-297): w1[e] is [I, D] = rc form
             h3 = ops.grouped_gemm(perm, cf.w3, offsets, w_is_kn=False)
             act = ops.swiglu(h1, h3)
-        eo = ops.grouped_gemm(act, cf.w2, offsets, w_is_kn=False)
+        by_rows = contiguous and ops.rows_experts_take(sorted_src.numel(), E, I, D, down=True)
+        eo = ops.rows_experts(act, cf.w2, offsets) if by_rows else ops.grouped_gemm(act, cf.w2, offsets, w_is_kn=False)
         sf = self.shared_ffn
-        if _glu_pair_ready(sf.w1.weight, sf.w3.weight):
+        if few and sf.w1.weight.is_contiguous() and sf.w3.weight.is_contiguous():
+            sact = ops.rows_swiglu(x2d, sf.w1.weight, sf.w3.weight)
+        elif _glu_pair_ready(sf.w1.weight, sf.w3.weight):
             sact = ops.gemm_swiglu_split(x2d, sf.w1.weight, sf.w3.weight)[1]
         else:
             sact = ops.swiglu(ops.gemm(x2d, sf.w1.weight), ops.gemm(x2d, sf.w3.weight))
-        sh = ops.gemm(sact, sf.w2.weight)
+        sh = _project(sact, sf.w2.weight)
         return ops.moe_unpermute(eo, inv, scores, k, add=sh)
 
 
@@ -346,8 +362,8 @@ class Transformer(nn.Module):
         h = ops.rmsnorm(delta, self.norm.weight, self.norm.eps, residual=res, want_rstd=False)[0] if delta is not None else self.norm(res)
         if last_only:
             h = h.view(B, S, D)[:, -1].contiguous()
-            return ops.gemm(h, self.output.weight).view(B, 1, -1)
-        return ops.gemm(h, self.output.weight).view(B, S, -1)
+            return _project(h, self.output.weight).view(B, 1, -1)
+        return _project(h, self.output.weight).view(B, S, -1)
 
     # ---- the serving protocol (serving.py).  Single tokens of up to DECODE_ROWS sequences are one library call; where the library does not serve the
     # sizes, and for portions of prompts, the sequences of a batch run one after the other, each on its own cache slot
@@ -388,7 +404,7 @@ class Transformer(nn.Module):
         if wanted is None:
             return torch.empty((0, self.vocab), dtype=torch.float32, device=self.device)
         h = ops.rmsnorm(delta[wanted], self.norm.weight, self.norm.eps, residual=res[wanted], want_rstd=False)[0]
-        return ops.gemm(h, self.output.weight).float()
+        return _project(h, self.output.weight).float()
 
     @torch.no_grad()
     def step(self, batch) -> torch.Tensor:
@@ -398,8 +414,12 @@ class Transformer(nn.Module):
             logits = tables.run(batch.ids, batch.slot, batch.pos, batch.max_len)
             if logits is not None:
                 return logits if batch.wanted is None or batch.wanted.numel() == len(logits) else logits[batch.wanted.long()]
-        if tables is not None and self._packs(batch):
-            return self._prompts(batch)
+        if tables is not None and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length:
+            logits = tables.prompts(batch) if batch.n_wanted <= batch.ids.numel() else None
+            if logits is not None:
+                return logits
+            if self._packs(batch):
+                return self._prompts(batch)
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:
@@ -461,13 +481,34 @@ class _StepTables:
         need = int(lib.cdll.aria_decode_step_scratch(self.dims_p, T, max_len)) if self.served else 0
         if need == 0:
             return None
-        if self.scratch is None or self.scratch.numel() < need:
-            self.scratch = torch.empty(need, dtype=torch.uint8, device=ids.device)
+        self._room(need, ids.device)
         logits = torch.empty((T, int(self.dims[8])), dtype=torch.float32, device=ids.device)
         for t in (ids, slot, pos):
             assert t.dtype == torch.int32 and t.is_contiguous() and t.numel() == T
         lib.call("aria_decode_step", self.ptrs, self.dims_p, self.eps, T, ids.data_ptr(), slot.data_ptr(), pos.data_ptr(), max_len, logits.data_ptr(),
                  self.scratch.data_ptr(), self.scratch.numel(), ops._stream(logits))
+        return logits
+
+
+    def _room(self, need: int, device) -> None:
+        if self.scratch is None or self.scratch.numel() < need:
+            self.scratch = torch.empty(need, dtype=torch.uint8, device=device)
+
+    def prompts(self, batch) -> Optional[torch.Tensor]:
+        """logits float32 [wanted rows, vocab] of a batch of whole short prompts; None: not served in one call"""
+        lib, T = hip.get_lib(), batch.ids.numel()
+        need = int(lib.cdll.aria_prompt_step_scratch(self.dims_p, T)) if self.served and T <= ops.ROWS_TOKENS else 0
+        if need == 0:
+            return None
+        self._room(need, batch.ids.device)
+        wanted = torch.arange(T, dtype=torch.int32, device=batch.ids.device) if batch.wanted is None else batch.wanted
+        logits = torch.empty((wanted.numel(), int(self.dims[8])), dtype=torch.float32, device=batch.ids.device)
+        for t in (batch.ids, batch.slot, batch.pos, batch.cu, wanted):
+            assert t.dtype == torch.int32 and t.is_contiguous()
+        n = wanted.numel()
+        lib.call("aria_prompt_step", self.ptrs, self.dims_p, self.eps, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.cu.data_ptr(),
+                 len(batch.lengths), batch.longest, wanted.data_ptr() if n else None, n, logits.data_ptr() if n else None, self.scratch.data_ptr(),
+                 self.scratch.numel(), ops._stream(self.scratch))
         return logits
 
 

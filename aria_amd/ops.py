@@ -44,6 +44,80 @@ def _rowmajor_2d(t: torch.Tensor, name="tensor") -> int:
 ACTIVATIONS = {None: 0, "gelu_tanh": 1, "relu_squared": 2}
 
 
+# Products of few tokens are bound by their weights; up to these sizes the row-streaming kernels (csrc/wide.hip) are ahead of the tiles.
+ROWS_TOKENS = 320      # 280 tokens x 7680 x 2560: 37 us, tiles 58; 400: 54, tiles 58
+ROWS_PER_EXPERT = 27       # on average, gate and up pairs: 280 tokens, 6 of 64 experts of 1664 x 2560: 234 us, tiles 270; 350: 373, tiles 271
+ROWS_PER_EXPERT_DOWN = 4   # down projections: 32 tokens 97 us, tiles 103; 64: 134, tiles 104
+
+
+def rows_take(M: int, K: int) -> bool:
+    """(Below 512 columns a launch costs more than the weights in either form.)"""
+    return 0 < M <= ROWS_TOKENS and 512 <= K <= 4096 and K % 8 == 0
+
+
+def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> bool:
+    """``rows_experts`` for M rows sorted by expert, w [E, N, K]"""
+    return (0 < M <= (ROWS_PER_EXPERT_DOWN if down else ROWS_PER_EXPERT) * E and E <= 256 and min(K, N) >= 512 and max(K, N) <= 2560 and K % 8 == 0
+            and N % 8 == 0)
+
+
+def rows_gemm(x: torch.Tensor, w: torch.Tensor, out_dtype=bf16) -> torch.Tensor:
+    """x [M, K] w^T for a contiguous w [N, K], M of a few hundred at most."""
+    _chk(x, name="x"), _chk(w, name="w")
+    (M, K), N = x.shape, w.shape[0]
+    if w.shape[1] != K or not w.is_contiguous():
+        raise ValueError("rows_gemm: w must be a contiguous [N, K] tensor of x's reduction")
+    out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+    hip.get_lib().call("aria_rows_gemm", _p(x), _p(w), _p(out), {bf16: 0, torch.float32: 1}[out_dtype], M, N, K, _rowmajor_2d(x, "x"), N, _stream(x))
+    return out
+
+
+def rows_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:
+    """silu(x w_gate^T) * (x w_up^T)"""
+    _chk(x, name="x"), _chk(w_gate, name="w_gate"), _chk(w_up, name="w_up")
+    (M, K), I = x.shape, w_gate.shape[0]
+    if w_gate.shape != w_up.shape or w_gate.shape[1] != K or not w_gate.is_contiguous() or not w_up.is_contiguous():
+        raise ValueError("rows_swiglu: contiguous [I, K] weights of x's reduction")
+    act = torch.empty((M, I), dtype=bf16, device=x.device)
+    hip.get_lib().call("aria_rows_swiglu", _p(x), _p(w_gate), _p(w_up), _p(act), M, I, K, _rowmajor_2d(x, "x"), I, _stream(x))
+    return act
+
+
+def rows_qkv_rope_cache(x: torch.Tensor, wqkv: torch.Tensor, freqs_cis: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, hd: int,
+                        slot: Optional[torch.Tensor] = None, pos: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Projection, rotation and cache write of tokens at pos of slot of the caches [slots, S, D] (default: positions 0 .. of the only slot) -> q [M, D]."""
+    _chk(x, name="x"), _chk(wqkv, name="wqkv"), _chk(freqs_cis, name="freqs_cis")
+    (M, K), D = x.shape, wqkv.shape[0] // 3
+    if wqkv.shape != (3 * D, K) or not wqkv.is_contiguous() or not freqs_cis.is_contiguous() or freqs_cis.shape[1] * 2 != hd:
+        raise ValueError("rows_qkv_rope_cache: wqkv [3 D, K], freqs_cis [S, hd / 2, 2], contiguous")
+    for c in (k_cache, v_cache):
+        if c.dtype != bf16 or not c.is_contiguous() or c.shape != k_cache.shape or c.shape[2] != D:
+            raise ValueError("rows_qkv_rope_cache: contiguous bf16 caches [slots, S, D]")
+    if slot is None and (k_cache.shape[0] != 1 or M > k_cache.shape[1] or M > freqs_cis.shape[0]) or freqs_cis.shape[0] < (k_cache.shape[1] if slot is not None else M):
+        raise ValueError("rows_qkv_rope_cache: the tokens do not fit the cache or the rotation table")
+    if slot is not None:
+        _chk(slot, torch.int32, "slot"), _chk(pos, torch.int32, "pos")
+        assert slot.numel() == pos.numel() == M
+    q = torch.empty((M, D), dtype=bf16, device=x.device)
+    hip.get_lib().call("aria_rows_qkv_rope_cache", _p(x), _p(wqkv), _p(q), _p(k_cache), _p(v_cache), _p(freqs_cis), _p(slot), _p(pos), M, D, K, hd,
+                       k_cache.shape[1], _rowmajor_2d(x, "x"), _stream(x))
+    return q
+
+
+def rows_experts(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, rows: Optional[torch.Tensor] = None, w_up: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Rows sorted by expert (offsets int32 [E + 1]) times w[e]^T, w [E, N, K]: row i is x[rows[i]] (default x[i]); with ``w_up`` the SwiGLU pair."""
+    _chk(x, name="x"), _chk(w, name="w"), _chk(offsets, torch.int32, "offsets")
+    E, N, K = w.shape
+    M = x.shape[0] if rows is None else rows.numel()
+    if x.shape[1] != K or offsets.numel() != E + 1 or any(not t.is_contiguous() or t.shape != w.shape for t in (w, w_up) if t is not None):
+        raise ValueError("rows_experts: contiguous [E, N, K] weights of x's reduction, offsets [E + 1]")
+    if rows is not None:
+        _chk(rows, torch.int32, "rows")
+    out = torch.empty((M, N), dtype=bf16, device=x.device)
+    hip.get_lib().call("aria_rows_experts", _p(x), _p(rows), _p(offsets), _p(w), _p(w_up), _p(out), E, M, N, K, _rowmajor_2d(x, "x"), N, _stream(x))
+    return out
+
+
 def gemm(a: torch.Tensor, b: torch.Tensor, *, a_oc: bool = False, b_oc: bool = False, bias: Optional[torch.Tensor] = None,
          out: Optional[torch.Tensor] = None, out_dtype=bf16, accumulate: bool = False, act: Optional[str] = None) -> torch.Tensor:
     """C[M,N] = op(A) op(B) (+bias) (+C).  a: [M,K] (a_oc=False) or [K,M] (a_oc=True);
@@ -1012,6 +1086,8 @@ def linear_any(a: torch.Tensor, w: torch.Tensor, out_dtype=None, relu_squared: b
     """a [M, K] w^T (then max(z, 0)^2) for a weight [N, K] of the same dtype: the MFMA GEMM for bf16 (the activation in its epilogue), the 32-bit
     kernel for float32."""
     if not _f32(a):
+        if not relu_squared and rows_take(*a.shape) and w.dtype == bf16 and w.is_contiguous():
+            return rows_gemm(a, w, out_dtype or bf16)
         return gemm(a, w, out_dtype=out_dtype or bf16, act="relu_squared" if relu_squared else None)
     _chk(w, torch.float32, "w")
     M, K = a.shape

@@ -401,6 +401,21 @@ int aria_cross_entropy(const void* logits, const int32_t* labels, float* loss_su
                        int64_t T, int64_t V, int64_t ld, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
+ * Weight-bound products of up to a few hundred tokens (wide.hip): the same functions as the tile products above, the weights streamed past 16 .. 64 tokens at a
+ * time with the reduction split over a workgroup's waves.  bf16, W [N, K] contiguous, 128 <= K <= 4096 (experts: 2560), K % 8 == 0.
+ * aria_rows_gemm: out [M, N] = X W^T, bf16 or fp32.   aria_rows_swiglu: act [M, I] = silu(X Wg^T) * (X Wu^T).
+ * aria_rows_qkv_rope_cache: as aria_gemm_qkv_rope_cache_bf16 on caches [slots, S_cache, D]: token t is position pos[t] of slot[t] (both NULL: position t of
+ *   the only slot); Q [M, D].
+ * aria_rows_experts: rows sorted by expert (offsets int32 [E + 1] on the device), place i reads X row rows[i] (NULL: i); W [E, N, K]; with Wu the
+ *   SwiGLU pair. */
+int aria_rows_gemm(const void* X, const void* W, void* out, int out_f32, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldo, void* stream);
+int aria_rows_swiglu(const void* X, const void* Wg, const void* Wu, void* act, int64_t M, int64_t I, int64_t K, int64_t ldx, int64_t ldact, void* stream);
+int aria_rows_qkv_rope_cache(const void* X, const void* Wqkv, void* Q, void* Kc, void* Vc, const void* freqs_cis, const int32_t* slot, const int32_t* pos,
+                             int64_t M, int64_t D, int64_t K, int64_t hd, int64_t S_cache, int64_t ldx, void* stream);
+int aria_rows_experts(const void* X, const int32_t* rows, const int32_t* offsets, const void* W, const void* Wu, void* out, int64_t E, int64_t M, int64_t N,
+                      int64_t K, int64_t ldx, int64_t ldo, void* stream);
+
+/* ------------------------------------------------------------------------------------------------
  * Single-token decode engine (decode.hip) -- gptfast/model.py:178-234 (Transformer.forward, one new token, batch 1),
  * :318-366 (MOEFeedForward, T < 50 path), :67-93 (KVCache.update), :413-447 (Attention with the static cache).
  * ONE call enqueues every kernel of every layer for one token: GEMV projections with RMSNorm / residual / SwiGLU folded in,
@@ -431,6 +446,13 @@ int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, v
 int64_t aria_decode_step_scratch(const int64_t* dims, int64_t T, int64_t max_len);
 int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
                      int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
+/* One serving step over T packed tokens of n_seq whole prompts (sequence b = rows cu[b] .. cu[b + 1), positions from 0; ids, slot, pos, cu, wanted: int32 on the
+ * device; longest: the host's maximum length): keys and values into the caches, fp32 logits [n_wanted, V] of the wanted rows.  ptrs, dims as
+ * aria_decode_step.  For prompts of a few hundred tokens together (prompt.hip); scratch: 0 bytes from aria_prompt_step_scratch as above. */
+int64_t aria_prompt_step_scratch(const int64_t* dims, int64_t T);
+int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+                     const int32_t* cu, int64_t n_seq, int64_t longest, const int32_t* wanted, int64_t n_wanted, float* logits, void* scratch,
+                     int64_t scratch_bytes, void* stream);
 /* Where, inside the scratch buffer, the last aria_decode_token call left every layer's routing record (TopKRouter of
  * gptfast/model.py:355-366 as the engine evaluated it): out[0], out[1] = byte offset and per-layer byte stride of the router logits (bf16 [L][E]),
  * out[2], out[3] = the chosen expert ids (int32 [L][top_k]), out[4], out[5] = their scores (bf16 [L][top_k]).  Read by the full-depth parity

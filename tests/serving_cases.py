@@ -102,12 +102,54 @@ def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
         assert L.logit_err(got, torch.stack([want[i][step] for i in order])) < 4 * 2 ** -8
 
 
-def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17)):
+def case_rows_products(dev, M, N, K, E=3):
+    """The weight-streaming products at edges of their token tiles, row groups and windows of the reduction against float64; bf16 results: half an ulp, 2^-9,
+    and twice that behind the rounded gate and up of SwiGLU."""
+    from aria_amd import ops
+
+    x, w, u = (L.rnd(n, K, seed=i, scale=K ** -0.5 if i else 1.0) for i, n in enumerate((M, N, N)))
+    xd, wd, ud = (t.to(dev) for t in (x, w, u))
+    want, up = x.double() @ w.double().T, x.double() @ u.double().T
+    assert L.rel(ops.rows_gemm(xd, wd, f32), want) < 2e-6 and L.rel(ops.rows_gemm(xd, wd), want) < 2 ** -8
+    assert L.rel(ops.rows_swiglu(xd, wd, ud), torch.nn.functional.silu(want) * up) < 2 ** -7
+    if K > 2560:
+        return
+    cuts = sorted([0, 0, M // 3, M])          # the first expert has no rows
+    off = torch.tensor(cuts, dtype=torch.int32, device=dev)
+    rows = torch.randperm(M, generator=L.gen(M)).to(torch.int32)
+    we, ue = (L.rnd(E, N, K, seed=5 + i, scale=K ** -0.5) for i in range(2))
+    for idx in (None, rows):
+        xs = x if idx is None else x[idx.long()]
+        y, z = (torch.cat([xs[a:b].double() @ m[e].double().T for e, (a, b) in enumerate(zip(cuts, cuts[1:]))]) for m in (we, ue))
+        kw = {} if idx is None else dict(rows=idx.to(dev))
+        assert L.rel(ops.rows_experts(xd, we.to(dev), off, **kw), y) < 2 ** -8
+        assert L.rel(ops.rows_experts(xd, we.to(dev), off, w_up=ue.to(dev), **kw), torch.nn.functional.silu(y) * z) < 2 ** -7
+
+
+def case_rows_qkv(dev, M, D, hd, S):
+    """Projection, rotation and cache write in one launch against the separate ones on the same product, bit for bit: positions 0 .. and any slots."""
+    from aria_amd import gptfast as G
+    from aria_amd import ops
+
+    x, w = L.rnd(M, D, seed=1).to(dev), L.rnd(3 * D, D, seed=2, scale=D ** -0.5).to(dev)
+    fc = G.precompute_freqs_cis(S, hd, 10000.0).to(dev).contiguous()
+    for slots in (1, 3):
+        slot = torch.arange(M, dtype=torch.int32) % slots
+        pos = torch.arange(M, dtype=torch.int32) // slots
+        k, v = (torch.zeros(slots, S, D, dtype=bf16, device=dev) for _ in range(2))
+        k2, v2 = torch.zeros_like(k), torch.zeros_like(v)
+        where = dict(slot=slot.to(dev), pos=pos.to(dev)) if slots > 1 else {}
+        q = ops.rows_qkv_rope_cache(x, w, fc, k, v, hd, **where)
+        qkv = ops.rope_cache_rows_(ops.rows_gemm(x, w), fc, slot.to(dev), pos.to(dev), k2, v2, D // hd, hd)
+        assert torch.equal(q, qkv[:, :D]) and torch.equal(k, k2) and torch.equal(v, v2)
+
+
+def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17), inter=128):
     """Prompts of several requests packed into one step against each prompt alone, logits at places inside and at the end, and a step on the caches that they
     left; rounding as in ``case_gptfast_decode_batch`` (the flash kernel's probabilities included)."""
     from aria_amd.serving import Scheduler
 
-    m = gptfast_routed(dev, dim, 64, 128, max(lens) + 8)
+    m = gptfast_routed(dev, dim, 64, inter, max(lens) + 8)
     toks = [torch.randint(0, 264, (n + 1,), generator=L.gen(n)).tolist() for n in lens]
     places = [sorted({0, n // 2, n - 1}) for n in lens]
     want = []
@@ -116,7 +158,6 @@ def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17)):
         want.append((s.step(["x"], [t[:-1]], [p]).cpu().double(), s.step(["x"], [t[-1:]]).cpu().double()))
     sched = Scheduler(m, max(lens) + 2)
     ids = list(range(len(lens)))
-    assert m.layers[0].attention.kv_cache.k.shape[0] == 1      # (set up again for the batch)
     got = sched.step(ids, [t[:-1] for t in toks], places)
     assert L.logit_err(got, torch.cat([w[0] for w in want])) < 4 * 2 ** -8
     got = sched.step(ids, [t[-1:] for t in toks])

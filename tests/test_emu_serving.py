@@ -19,6 +19,15 @@ def test_gptfast_decode_batch():
     C.case_gptfast_decode_batch(DEV, 128, 64, 128, 3)
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 20, 136), (70, 9, 520)])
+def test_rows_products(M, N, K):
+    C.case_rows_products(DEV, M, N, K)
+
+
+def test_rows_qkv():
+    C.case_rows_qkv(DEV, 37, 128, 64, 40)
+
+
 def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV, 128, (5, 1, 9))
 

@@ -27,6 +27,21 @@ def test_gptfast_decode_batch(dim, head_dim, inter, requests, longest):
     C.case_gptfast_decode_batch(DEV, dim, head_dim, inter, requests, longest)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 100, 128), (16, 33, 1024), (17, 264, 1032), (33, 16, 1800), (64, 1000, 2560), (65, 7, 1792), (320, 40, 2568), (40, 130, 3336), (15, 24, 4096)])
+def test_rows_products(M, N, K):
+    C.case_rows_products(DEV, M, N, K)
+
+
+@pytest.mark.parametrize("M,D,hd,S", [(5, 512, 64, 8), (100, 2560, 128, 104), (37, 768, 64, 40)])
+def test_rows_qkv(M, D, hd, S):
+    C.case_rows_qkv(DEV, M, D, hd, S)
+
+
+@pytest.mark.parametrize("dim,inter,lens", [(512, 512, (9, 1, 20, 7)), (1024, 1664, (20,)), (1536, 1024, (2, 3, 5, 2, 17, 1)), (2560, 1664, (33, 30, 8))])
+def test_gptfast_packed_prompts_in_one_call(dim, inter, lens):
+    C.case_gptfast_packed_prompts(DEV, dim, lens, inter)
+
+
 def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV)
     C.case_gptfast_packed_prompts(DEV, 1024, (300, 64, 65, 2, 129))
