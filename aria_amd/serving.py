@@ -13,6 +13,7 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from . import gptfast as G
@@ -94,15 +95,32 @@ class StepBatch:
         """tokens: one list of ids per sequence, or an int32 device tensor with one id per sequence (a decode step whose ids never visited the host)."""
         on_device = isinstance(tokens, torch.Tensor)
         lengths = [1] * len(slots) if on_device else [len(t) for t in tokens]
-        cu, slot, pos, seq = [0], [], [], []
-        for i, (n, s, p) in enumerate(zip(lengths, slots, starts)):
-            cu.append(cu[-1] + n)
-            slot += [s] * n
-            pos += range(p, p + n)
-            seq += [i] * n
-        T = cu[-1]
-        host = ([] if on_device else [i for t in tokens for i in t]) + slot + pos + seq + cu + (list(wanted) if wanted is not None else [])
-        buf = torch.tensor(host, dtype=torch.int32).to(device)      # one copy to the device per step
+        T, n = sum(lengths), len(lengths)
+        # one copy to the device per step, from pinned memory: it waits for nothing that runs there (the pinned block is the allocator's again when the
+        # copy is done)
+        size = (0 if on_device else T) + 3 * T + n + 1 + (len(wanted) if wanted is not None else 0)
+        cuda = torch.device(device).type == "cuda"
+        host = torch.empty(size, dtype=torch.int32, device="cpu", pin_memory=cuda)
+        fill, at = host.numpy(), 0
+
+        def put(values, count):
+            nonlocal at
+            fill[at:at + count] = values
+            at += count
+
+        if not on_device:
+            for t in tokens:
+                put(t, len(t))
+        each = np.asarray(lengths)
+        ends = np.cumsum(each)
+        put(np.repeat(np.asarray(slots), each), T)
+        put(np.arange(T) + np.repeat(np.asarray(starts) - (ends - each), each), T)
+        put(np.repeat(np.arange(n), each), T)
+        put(0, 1)
+        put(ends, n)
+        if wanted is not None:
+            put(list(wanted), len(wanted))
+        buf = host.to(device, non_blocking=True) if cuda else host
         at = 0
 
         def take(n):
