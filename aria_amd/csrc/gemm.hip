@@ -262,6 +262,69 @@ int launch_gemm(const GemmParams& p, int a_oc, int b_oc, int grid_x, int grid_y,
     return aria_check_launch();
 }
 
+// C (+)= A B for a reduction of 8 or 16 (an adapter's second projection): one pass over C, no tile.  A thread holds its 8 columns of B and runs through
+// rows; bound by C's bytes.  4096 x 2560, K = 8, accumulated: the 128 x 128 tile kernel 69 us, this 17.
+template <int KC, bool B_OC, bool ACC>
+__global__ __launch_bounds__(256) void gemm_thin_kernel(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, long long lda, long long ldb, long long ldc) {
+    constexpr int ROWS = 32;
+    const int c = blockIdx.x * 64 + (threadIdx.x & 63), n0 = c * 8, m_end = min(M, (int(blockIdx.y) + 1) * ROWS);
+    if (n0 >= N) return;
+    float b[KC * 8][8];
+#pragma unroll
+    for (int i = 0; i < (B_OC ? KC * 8 : 8); ++i)
+#pragma unroll
+        for (int j = 0; j < (B_OC ? 1 : KC); ++j) {   // B_OC: row k, its 8 columns; else: column n0 + i's 8 KC reduction indices
+            const u32x4 v = B_OC ? ld16(B + i * ldb + n0) : ld16(B + (n0 + i) * ldb + 8 * j);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                (B_OC ? b[i][2 * q] : b[8 * j + 2 * q][i]) = bflo(v[q]);
+                (B_OC ? b[i][2 * q + 1] : b[8 * j + 2 * q + 1][i]) = bfhi(v[q]);
+            }
+        }
+    for (int m = blockIdx.y * ROWS + (threadIdx.x >> 6); m < m_end; m += 4) {
+        bf16_t* dst = C + m * ldc + n0;
+        u32x4 old;
+        if (ACC) old = ld16(dst);
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = 0.f;
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+            const u32x4 a = ld16(A + m * lda + 8 * j);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float av = k & 1 ? bfhi(a[k >> 1]) : bflo(a[k >> 1]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) y[e] = fmaf(av, b[8 * j + k][e], y[e]);
+            }
+        }
+        if (ACC) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                y[2 * q] += bflo(old[q]);
+                y[2 * q + 1] += bfhi(old[q]);
+            }
+        }
+        st16(dst, u32x4{pack2bf(y[0], y[1]), pack2bf(y[2], y[3]), pack2bf(y[4], y[5]), pack2bf(y[6], y[7])});
+    }
+}
+template <int KC>
+int launch_thin(const GemmParams& p, bool b_oc, void* stream) {
+    const dim3 grid(unsigned((p.N / 8 + 63) / 64), unsigned((p.M + 31) / 32)), block(256);
+    const bf16_t *A = static_cast<const bf16_t*>(p.A), *B = static_cast<const bf16_t*>(p.B);
+    bf16_t* C = static_cast<bf16_t*>(p.C);
+    const long long lda = p.lda, ldb = p.ldb, ldc = p.ldc;
+    if (b_oc && p.accumulate)
+        ARIA_LAUNCH((gemm_thin_kernel<KC, true, true>), grid, block, 0, stream, A, B, C, p.M, p.N, lda, ldb, ldc);
+    else if (b_oc)
+        ARIA_LAUNCH((gemm_thin_kernel<KC, true, false>), grid, block, 0, stream, A, B, C, p.M, p.N, lda, ldb, ldc);
+    else if (p.accumulate)
+        ARIA_LAUNCH((gemm_thin_kernel<KC, false, true>), grid, block, 0, stream, A, B, C, p.M, p.N, lda, ldb, ldc);
+    else
+        ARIA_LAUNCH((gemm_thin_kernel<KC, false, false>), grid, block, 0, stream, A, B, C, p.M, p.N, lda, ldb, ldc);
+    return aria_check_launch();
+}
+
 thread_local int g_last_variant = 0;
 constexpr int GROUPED_V3_DEFAULT = 3;  // r02 in-bench A/B with the wide epilogue: v3 for both weight forms 702 ms/step, v2 for the [K,N] form 710
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -277,12 +340,16 @@ bool use_v2(long long tiles256) {
 
 // v3 (LDS-DMA staged, phase-scheduled 256x256 tile, gemm3.hip): the operand byte offsets must fit 32 bits.
 // ARIA_GEMM_FORCE=3 pins it where eligible.
-bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB, long long extentA, long long extentB) {
+bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB, long long extentA, long long extentB, long long least = 192) {
     if (K < 64 || bytesA >= (1ll << 32) || bytesB >= (1ll << 32) || extentA < 8 || extentB < 8) return false;
     const char* force = std::getenv("ARIA_GEMM_FORCE");
     if (force) return force[0] == '3';
-    return tiles256 >= 192;
+    return tiles256 >= least;
 }
+// Fewest 256 x 256 tiles that v3 takes in one partly filled round: its time there is the reduction's (about 1.45 us per 64 columns), the 128 x 128 kernel's
+// grows with the tiles -- 4096 x 2560 x 2560 (160 tiles): 137 us against 70.  Short reductions stay with the small tiles.
+constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150;
+long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
 }  // namespace
 
@@ -333,6 +400,10 @@ int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, 
     p.c_f32 = c_f32;
     p.accumulate = accumulate;
     p.act = act;
+    // (whole 16-byte pieces of C; an output of a few columns stays with the tiles)
+    if ((K == 8 || K == 16) && !a_oc && !c_f32 && !bias && act == ARIA_ACT_NONE && N >= 512 && (N & 7) == 0 && (ldc & 7) == 0 && aligned16(C) &&
+        (M + 31) / 32 <= 65535 && !std::getenv("ARIA_GEMM_FORCE"))
+        return g_last_variant = 1, K == 8 ? launch_thin<1>(p, b_oc, stream) : launch_thin<2>(p, b_oc, stream);
     p.ntn = int((N + BN - 1) / BN);
     const int ntm = int((M + BM - 1) / BM);
     const long long t256 = ((M + 255) / 256) * ((N + 255) / 256);
@@ -340,7 +411,7 @@ int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, 
     // with a workspace the partly filled last round of tiles is split along K (gemm3.hip), so small outputs fill the chip too
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
-    if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, bytesA, bytesB, M, N))
+    if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
         return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
@@ -376,7 +447,8 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const int gmask = gsel ? std::atoi(gsel) : GROUPED_V3_DEFAULT;
     const char* gforce = std::getenv("ARIA_GEMM_FORCE");
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
-    if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N))
+    if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
+                      v3_least(K, V3_FEW_TILES_GROUPED)))
         return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc, int(M_total / 256 + E), stream);
     if (use_v2((M_total / 256 + 1) * ((N + 255) / 256))) return g_last_variant = 2, aria_launch_gemm2(p, 0, b_oc, int(M_total / 256 + E), 1, stream);
     return g_last_variant = 1, launch_gemm(p, 0, b_oc, p.ntn * max_tm, 1, stream);

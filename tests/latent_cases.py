@@ -210,6 +210,19 @@ def case_gemm_relu_squared(dev, M, N, K):
     assert rel(got, O.relu_squared(a.cpu().double() @ w.cpu().double().T)) < 1e-2
 
 
+def case_gemm_thin(dev, M, N, K):
+    """A reduction of 8 or 16 in both layouts of the right operand, stored and accumulated: one bf16 rounding of the exact result (2^-9), two when the sum
+    with the old value cancels part of it."""
+    from aria_amd import ops
+
+    a, b, c = rnd(M, K, seed=1), rnd(N, K, seed=2), rnd(M, N, seed=3)
+    want = a.double() @ b.double().T
+    ad, bd, bt = a.to(dev), b.to(dev), b.T.contiguous().to(dev)
+    assert rel(ops.gemm(ad, bd), want) < 2 ** -8 and rel(ops.gemm(ad, bt, b_oc=True), want) < 2 ** -8
+    assert rel(ops.gemm(ad, bd, out=c.to(dev), accumulate=True), want + c.double()) < 2 ** -8
+    assert rel(ops.gemm(ad, bt, b_oc=True, out=c.to(dev), accumulate=True), want + c.double()) < 2 ** -8
+
+
 def case_gemm_f32(dev, M, N, K):
     from aria_amd import ops
 

@@ -33,6 +33,11 @@ def test_gemm_relu_squared(M, N, K):
     C.case_gemm_relu_squared(DEV, M, N, K)
 
 
+def test_gemm_thin():
+    C.case_gemm_thin(DEV, 33, 520, 8)
+    C.case_gemm_thin(DEV, 5, 512, 16)
+
+
 @pytest.mark.parametrize("M,N,K", [(5, 9, 4), (70, 66, 20)])
 def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)

@@ -37,6 +37,11 @@ def test_gemm_relu_squared(M, N, K):
     C.case_gemm_relu_squared(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 512, 8), (33, 1032, 8), (300, 2560, 16), (31, 520, 16)])
+def test_gemm_thin(M, N, K):
+    C.case_gemm_thin(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(5, 9, 4), (70, 66, 20), (300, 257, 516), (16, 33, 1028), (17, 31, 88), (64, 130, 636), (65, 95, 132), (2100, 1030, 72)])
 def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)
