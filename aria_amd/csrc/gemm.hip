@@ -263,7 +263,7 @@ int launch_gemm(const GemmParams& p, int a_oc, int b_oc, int grid_x, int grid_y,
 }
 
 // C (+)= A B for a reduction of 8 or 16 (an adapter's second projection): one pass over C, no tile.  A thread holds its 8 columns of B and runs through
-// rows; bound by C's bytes.  4096 x 2560, K = 8, accumulated: the 128 x 128 tile kernel 69 us, this 17.
+// rows; bound by C's bytes.  4096 x 2560, K = 8, us as a 128 x 128 tile / here: accumulated 16.5 / 9.2, stored 12.3 / 10.0.
 template <int KC, bool B_OC, bool ACC>
 __global__ __launch_bounds__(256) void gemm_thin_kernel(const bf16_t* A, const bf16_t* B, bf16_t* C, int M, int N, long long lda, long long ldb, long long ldc) {
     constexpr int ROWS = 32;
@@ -347,7 +347,8 @@ bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB,
     return tiles256 >= least;
 }
 // Fewest 256 x 256 tiles that v3 takes in one partly filled round: its time there is the reduction's (about 1.45 us per 64 columns), the 128 x 128 kernel's
-// grows with the tiles -- 4096 x 2560 x 2560 (160 tiles): 137 us against 70.  Short reductions stay with the small tiles.
+// grows with the tiles.  us as 128 x 128 / 256 x 256: 4096 x 2560 outputs (160 tiles), K = 2560 86 / 58, K = 1664 57 / 40, K = 512 27 / 19; 2100 x 2560 (90
+// tiles), K = 2560 54 / 54.  Shorter reductions stay with the small tiles.
 constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150;
 long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 

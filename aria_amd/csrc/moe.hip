@@ -284,7 +284,7 @@ __global__ __launch_bounds__(64) void sort_scatter_kernel(const int32_t* idx, co
 }
 
 // Up to SORT_SMALL entries: the three passes as one launch of one workgroup, its 16 waves on sixteen ranges of the entries (a chunk of 2048 entries per wave and
-// launch took 9 + 4 + 9 us for the 1680 entries of 280 tokens; 6 us here).  counts NULL: taken from the entries; rows: the token of every place.
+// launch took 9 + 4 + 9 us for the 1680 entries of 280 tokens; 5 us here).  counts NULL: taken from the entries; rows: the token of every place.
 constexpr int SORT_SMALL = 8192;
 __global__ __launch_bounds__(1024) void sort_small_kernel(const int32_t* idx, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv,
                                                           int32_t* rows, int E, int M, int k) {

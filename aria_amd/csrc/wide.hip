@@ -2,9 +2,9 @@
 //
 // A 256 x 256 tile of the matrix product leaves most of the chip idle there: 280 tokens x 7680 outputs are 60 tiles, each with the whole reduction to itself
 // (58 us for 39 MB of weights).  The row-streaming kernels of the decode step (rows.h) split the reduction over a workgroup's waves instead and take
-// up to 64 tokens at a time past the weights; further tokens find the weights in the L2 / MALL.  280 tokens, us as tiles / here: q | k | v with rotation
-// and cache write 58 / 37, gate and up with SwiGLU (2 x 3328) 56 / 38, 2560 x 2560 34 / 21; 64 tokens: 58 / 17, 56 / 17, 34 / 13; lm_head of one token
-// 140 / 97.  From about 400 tokens on the tiles are ahead.
+// up to 64 tokens at a time past the weights; further tokens find the weights in the L2 / MALL.  280 tokens, us as tiles / here: q | k | v 58 / 39
+// (with rotation and cache write in the epilogue 58 / 42), gate and up with SwiGLU (2 x 3328) 56 / 40, 2560 x 2560 34 / 22; 64 tokens: 58 / 17, 56 / 17,
+// 34 / 13; lm_head of one token 140 / 86.  From about 400 tokens on the tiles are ahead.
 // Routed experts: with n tokens an expert's matrix meets n k / E rows (26 at 280 tokens, 6 of 64 experts); its rows are read once per 64 of them.  Up pairs
 // (64 experts of 2 x 1664 x 2560), tiles / here: 32 tokens 238 / 182, 280 tokens 270 / 234, 350 tokens (92 rows for the most popular expert: read twice)
 // 271 / 373.  Down (2560 x 1664): 32 tokens 103 / 97, from 64 tokens on the tiles are ahead (104 / 134).

@@ -217,7 +217,7 @@ class MOEFeedForward(nn.Module):
         if not few and ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
             logits, scores, idx, counts = ops.moe_router_fused(x2d, self.gate.weight, k)
         else:
-            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 45 us for 280 tokens, 12 in two launches)
+            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 45 us for 280 tokens, 22 in two launches)
             scores, idx, counts = ops.moe_route(logits, k)             # topk + softmax (model.py:359-363)
         offsets, sorted_src, inv = ops.moe_sort(idx, counts)           # token_permutation (:243-254)
         cf = self.cond_ffn
@@ -366,7 +366,7 @@ class Transformer(nn.Module):
         return _project(h, self.output.weight).view(B, S, -1)
 
     # ---- the serving protocol (serving.py).  Single tokens of up to DECODE_ROWS sequences are one library call; where the library does not serve the
-    # sizes, and for portions of prompts, the sequences of a batch run one after the other, each on its own cache slot
+    # sizes the sequences of a batch run one after the other, each on its own cache slot
     def _step_tables(self, batch) -> Optional["_StepTables"]:
         """Tables of the one-call step on the caches as they are; None where this model does not go through it."""
         cache = self.layers[0].attention.kv_cache

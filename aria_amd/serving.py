@@ -7,7 +7,9 @@ that ends leaves its cache slot to a later batch.  A model serves through three 
 * ``step(batch) -> float32 [wanted, vocab]`` -- run the batch's tokens from and into the caches, logits at the wanted rows;
 * ``vocab``, ``device`` -- columns of the logits, where tensors live.
 
-``duguzen.DuguzenForCausalLM`` and ``kozipel.KozipelForCausalLM`` run a batch as one; ``gptfast.Transformer`` (Aria) runs its sequences one after the other on the slots' caches.  The same ``step`` is what ``generate`` and the trace runner (bin/trace_run) drive."""
+All three decoders (``gptfast.Transformer`` = Aria, ``duguzen.DuguzenForCausalLM``, ``kozipel.KozipelForCausalLM``) run a batch as one; Aria falls back to one
+sequence after the other for continued prompts and for sizes its kernels do not take.  The same ``step`` is what ``generate`` and the trace runner
+(bin/trace_run) drive."""
 from __future__ import annotations
 
 from dataclasses import dataclass, field
