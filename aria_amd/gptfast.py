@@ -102,7 +102,7 @@ def _glu_pair_ready(w_gate: nn.Parameter, w_up: nn.Parameter) -> bool:
 
 def _project(x2d: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x w^T: the row-streaming kernel for few tokens, the tile product beyond"""
-    return ops.rows_gemm(x2d, w) if ops.rows_take(*x2d.shape) and w.is_contiguous() else ops.gemm(x2d, w)
+    return ops.rows_gemm(x2d, w) if ops.rows_take(*x2d.shape) and w.is_contiguous() and w.shape[0] % 2 == 0 else ops.gemm(x2d, w)
 
 
 class RMSNorm(nn.Module):
@@ -455,7 +455,8 @@ class Transformer(nn.Module):
 
 
 class _StepTables:
-    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches (re-made when either moves), and its scratch."""
+    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches (re-made when either moves).  The scratch is a step's own:
+    steps of other streams never share it, and the allocator knows whose stream it was used on."""
 
     def __init__(self, model: "Transformer"):
         import ctypes
@@ -470,7 +471,6 @@ class _StepTables:
         self.tensors = [model.freqs_cis, model.norm.weight, model.output.weight, model.tok_embeddings.weight] + _layer_table(model)
         self.served = all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in self.tensors)
         self.ptrs = (ctypes.c_void_p * len(self.tensors))(*(t.data_ptr() for t in self.tensors))
-        self.scratch: Optional[torch.Tensor] = None
 
     def valid_for(self, model: "Transformer") -> bool:
         return model._weights_version == self.version and DecodeEngine._cheap_key(model) == self.key
@@ -481,18 +481,13 @@ class _StepTables:
         need = int(lib.cdll.aria_decode_step_scratch(self.dims_p, T, max_len)) if self.served else 0
         if need == 0:
             return None
-        self._room(need, ids.device)
+        scratch = torch.empty(need, dtype=torch.uint8, device=ids.device)
         logits = torch.empty((T, int(self.dims[8])), dtype=torch.float32, device=ids.device)
         for t in (ids, slot, pos):
             assert t.dtype == torch.int32 and t.is_contiguous() and t.numel() == T
         lib.call("aria_decode_step", self.ptrs, self.dims_p, self.eps, T, ids.data_ptr(), slot.data_ptr(), pos.data_ptr(), max_len, logits.data_ptr(),
-                 self.scratch.data_ptr(), self.scratch.numel(), ops._stream(logits))
+                 scratch.data_ptr(), need, ops._stream(logits))
         return logits
-
-
-    def _room(self, need: int, device) -> None:
-        if self.scratch is None or self.scratch.numel() < need:
-            self.scratch = torch.empty(need, dtype=torch.uint8, device=device)
 
     def prompts(self, batch) -> Optional[torch.Tensor]:
         """logits float32 [wanted rows, vocab] of a batch of whole short prompts; None: not served in one call"""
@@ -500,15 +495,15 @@ class _StepTables:
         need = int(lib.cdll.aria_prompt_step_scratch(self.dims_p, T)) if self.served and T <= ops.ROWS_TOKENS else 0
         if need == 0:
             return None
-        self._room(need, batch.ids.device)
+        scratch = torch.empty(need, dtype=torch.uint8, device=batch.ids.device)
         wanted = torch.arange(T, dtype=torch.int32, device=batch.ids.device) if batch.wanted is None else batch.wanted
         logits = torch.empty((wanted.numel(), int(self.dims[8])), dtype=torch.float32, device=batch.ids.device)
         for t in (batch.ids, batch.slot, batch.pos, batch.cu, wanted):
             assert t.dtype == torch.int32 and t.is_contiguous()
         n = wanted.numel()
         lib.call("aria_prompt_step", self.ptrs, self.dims_p, self.eps, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.cu.data_ptr(),
-                 len(batch.lengths), batch.longest, wanted.data_ptr() if n else None, n, logits.data_ptr() if n else None, self.scratch.data_ptr(),
-                 self.scratch.numel(), ops._stream(self.scratch))
+                 len(batch.lengths), batch.longest, wanted.data_ptr() if n else None, n, logits.data_ptr() if n else None, scratch.data_ptr(),
+                 need, ops._stream(scratch))
         return logits
 
 

@@ -1086,7 +1086,7 @@ def linear_any(a: torch.Tensor, w: torch.Tensor, out_dtype=None, relu_squared: b
     """a [M, K] w^T (then max(z, 0)^2) for a weight [N, K] of the same dtype: the MFMA GEMM for bf16 (the activation in its epilogue), the 32-bit
     kernel for float32."""
     if not _f32(a):
-        if not relu_squared and rows_take(*a.shape) and w.dtype == bf16 and w.is_contiguous():
+        if not relu_squared and rows_take(*a.shape) and w.dtype == bf16 and w.is_contiguous() and w.shape[0] % 2 == 0:   # (odd: gemm raises)
             return rows_gemm(a, w, out_dtype or bf16)
         return gemm(a, w, out_dtype=out_dtype or bf16, act="relu_squared" if relu_squared else None)
     _chk(w, torch.float32, "w")
