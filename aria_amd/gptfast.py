@@ -298,6 +298,7 @@ class Transformer(nn.Module):
 
     def _apply(self, fn, *a, **k):
         self._weights_version = getattr(self, "_weights_version", 0) + 1
+        self._tables = None      # (they keep the storage that is given up here)
         return super()._apply(fn, *a, **k)
 
     def _engine_capable(self) -> bool:
@@ -328,10 +329,7 @@ class Transformer(nn.Module):
                                                                  b.attention.hdp, dev)
         self.freqs_cis = precompute_freqs_cis(max(self.config.block_size, self.max_seq_length), self.config.head_dim,
                                               self.config.rope_base).to(dev).contiguous()
-        for b in self.layers:  # gate / up pairs into one allocation each NOW (the decode engine records parameter addresses later)
-            ff = b.feed_forward
-            _glu_pair_ready(ff.cond_ffn.w1, ff.cond_ffn.w3)
-            _glu_pair_ready(ff.shared_ffn.w1.weight, ff.shared_ffn.w3.weight)
+        _pair_weights(self)
 
     def forward(self, idx: Optional[torch.Tensor], input_pos: Optional[torch.Tensor] = None,
                 input_embeds: Optional[torch.Tensor] = None, last_only: bool = False) -> torch.Tensor:
@@ -454,9 +452,19 @@ class Transformer(nn.Module):
         return torch.cat(out) if out else torch.empty((0, self.vocab), dtype=torch.float32, device=ids.device)
 
 
+def _pair_weights(model: "Transformer") -> None:
+    """Gate / up pairs into one allocation each before anybody records parameter addresses: the layers, which pair lazily, then find nothing to move."""
+    for b in model.layers:
+        ff = b.feed_forward
+        _glu_pair_ready(ff.cond_ffn.w1, ff.cond_ffn.w3)
+        _glu_pair_ready(ff.shared_ffn.w1.weight, ff.shared_ffn.w3.weight)
+
+
 class _StepTables:
-    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches (re-made when either moves).  The scratch is a step's own:
-    steps of other streams never share it, and the allocator knows whose stream it was used on."""
+    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches.  Every step compares them with the tensors that the model
+    holds then (assigned, moved or replaced weights and modules: about 0.1 us a tensor, beside a device that is busy with the step before), and
+    the tables keep the storage alive that they point to.  The scratch is a step's own: steps of other streams never share it, and the allocator
+    knows whose stream it was used on."""
 
     def __init__(self, model: "Transformer"):
         import ctypes
@@ -464,16 +472,42 @@ class _StepTables:
         import numpy as np
 
         c = model.config
-        self.version, self.key, self.eps = model._weights_version, DecodeEngine._cheap_key(model), float(c.norm_eps)
+        _pair_weights(model)
+        self.key, self.eps = DecodeEngine._cheap_key(model), float(c.norm_eps)
         self.dims = np.array([c.n_layer, c.dim, c.n_head, c.head_dim, c.num_experts, c.router_topk, c.intermediate_size,
                               c.intermediate_size * c.num_shared_experts, c.vocab_size, model.max_seq_length], dtype=np.int64)
         self.dims_p = self.dims.ctypes.data_as(ctypes.c_void_p)
-        self.tensors = [model.freqs_cis, model.norm.weight, model.output.weight, model.tok_embeddings.weight] + _layer_table(model)
-        self.served = all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in self.tensors)
-        self.ptrs = (ctypes.c_void_p * len(self.tensors))(*(t.data_ptr() for t in self.tensors))
+        tensors = [model.freqs_cis, model.norm.weight, model.output.weight, model.tok_embeddings.weight] + _layer_table(model)
+        self.tensors = [t.detach() for t in tensors]      # (a parameter's storage may be exchanged, a detached tensor's not)
+        D, I, Is, E, cache = c.dim, c.intermediate_size, c.intermediate_size * c.num_shared_experts, c.num_experts, tuple(model.layers[0].attention.kv_cache.k.shape)
+        layer = [(D,), (3 * D, D), (D, D), (D,), (E, D), (E, I, D), (E, I, D), (E, D, I), (Is, D), (Is, D), (D, Is), cache, cache]
+        shapes = [(model.freqs_cis.shape[0], c.head_dim // 2, 2), (D,), (c.vocab_size, D), (c.vocab_size, D)] + layer * c.n_layer
+        self.served = (all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in tensors) and [tuple(t.shape) for t in tensors] == shapes
+                       and cache[1:] == (model.max_seq_length, D) and model.freqs_cis.shape[0] >= model.max_seq_length)
+        self.ptrs = (ctypes.c_void_p * len(tensors))(*(t.data_ptr() for t in tensors))
+        # ways to the weights: (modules of the parent, name, module), (parameters of the module, name); addresses and sizes of these
+        self.modules, self.ways, seen = [], [], set()
+        for path in [("norm", "weight"), ("output", "weight"), ("tok_embeddings", "weight")] + [("layers", str(i)) + w for i in range(c.n_layer) for w in _LAYER_WEIGHTS]:
+            at = model
+            for name in path[:-1]:
+                parent, at = at, at._modules[name]
+                if (id(parent), name) not in seen:
+                    seen.add((id(parent), name))
+                    self.modules.append((parent._modules, name, at))
+            self.ways.append((at._parameters, path[-1]))
+        weights = [of.get(name) for of, name in self.ways]
+        self.served = self.served and all(t is not None for t in weights)       # (one that is computed from other parameters has no address of its own)
+        if self.served:
+            self.where, self.sizes = [t.data_ptr() for t in weights], [t.numel() for t in weights]
 
     def valid_for(self, model: "Transformer") -> bool:
-        return model._weights_version == self.version and DecodeEngine._cheap_key(model) == self.key
+        if not self.served or DecodeEngine._cheap_key(model) != self.key:      # (tensors that the library does not take: looked at again with every step)
+            return False
+        if [None for of, name, module in self.modules if of.get(name) is not module]:
+            return False
+        weights = [of.get(name) for of, name in self.ways]
+        return (not [None for t in weights if t is None] and list(map(torch.Tensor.data_ptr, weights)) == self.where and list(map(torch.Tensor.numel, weights)) == self.sizes
+                and all(map(torch.Tensor.is_contiguous, weights)))
 
     def run(self, ids, slot, pos, max_len: int) -> Optional[torch.Tensor]:
         """logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""
@@ -507,13 +541,22 @@ class _StepTables:
         return logits
 
 
+# a layer's weights in the order of the decode engine's pointer tables (the caches behind them)
+_LAYER_WEIGHTS = (("attention_norm", "weight"), ("attention", "wqkv", "weight"), ("attention", "wo", "weight"), ("ffn_norm", "weight"),
+                  ("feed_forward", "gate", "weight"), ("feed_forward", "cond_ffn", "w1"), ("feed_forward", "cond_ffn", "w3"), ("feed_forward", "cond_ffn", "w2"),
+                  ("feed_forward", "shared_ffn", "w1", "weight"), ("feed_forward", "shared_ffn", "w3", "weight"), ("feed_forward", "shared_ffn", "w2", "weight"))
+
+
 def _layer_table(model: "Transformer") -> List[torch.Tensor]:
     """the tensors of every layer in the order of the decode engine's pointer tables"""
     out = []
     for blk in model.layers:
-        a, f = blk.attention, blk.feed_forward
-        out += [blk.attention_norm.weight, a.wqkv.weight, a.wo.weight, blk.ffn_norm.weight, f.gate.weight, f.cond_ffn.w1, f.cond_ffn.w3, f.cond_ffn.w2,
-                f.shared_ffn.w1.weight, f.shared_ffn.w3.weight, f.shared_ffn.w2.weight, a.kv_cache.k, a.kv_cache.v]
+        for path in _LAYER_WEIGHTS:
+            t = blk
+            for name in path:
+                t = getattr(t, name)
+            out.append(t)
+        out += [blk.attention.kv_cache.k, blk.attention.kv_cache.v]
     return out
 
 
@@ -545,6 +588,7 @@ class DecodeEngine:
         self.x_in = torch.zeros(c.dim, dtype=bf16, device=dev)
         self.logits = torch.zeros(c.vocab_size, dtype=bf16, device=dev)
         self.eps = float(c.norm_eps)
+        _pair_weights(model)
         tensors = self._table(model)
         for t in tensors:
             assert t.is_contiguous() and t.device == dev

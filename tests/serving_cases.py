@@ -4,6 +4,7 @@ import io
 import json
 import os
 
+import pytest
 import torch
 
 from tests import kozipel_cases as K
@@ -100,6 +101,63 @@ def case_gptfast_decode_batch(dev, dim, head_dim, inter, requests, longest=9):
         order = list(range(requests))[::-1] if step else list(range(requests))
         got = sched.step(order, [[toks[i][len(toks[i]) - 2 + step]] for i in order])
         assert L.logit_err(got, torch.stack([want[i][step] for i in order])) < 4 * 2 ** -8
+
+
+def gptfast_moved_weights(dev, names):
+    """(name, model, what changes its weights, a model that has had them from the beginning), each change by another way in"""
+    from torch import nn
+
+    def copies():
+        return gptfast_routed(dev, 128, 64, 128, 32), gptfast_routed(dev, 128, 64, 128, 32)
+
+    def assign(m):
+        m.load_state_dict({k: v.clone() for k, v in m.state_dict().items()}, assign=True)
+
+    def parameter(m):
+        m.output.weight = nn.Parameter(m.output.weight.detach() * 2, requires_grad=False)
+
+    def data(m):
+        m.layers[1].attention.wo.weight.data = m.layers[1].attention.wo.weight.data.T.contiguous()
+
+    def module(m):
+        other = gptfast_routed(dev, 128, 64, 128, 32).layers[0].feed_forward
+        with torch.no_grad():
+            other.shared_ffn.w2.weight.mul_(-1)
+        m.layers[0].feed_forward = other
+
+    for change in (c for c in (assign, parameter, data, module) if c.__name__ in names):
+        m, want = copies()
+        change(want)
+        yield change.__name__, m, change, want
+
+
+def case_gptfast_moved_weights(dev, names=("assign", "parameter", "data", "module")):
+    """Weights that are assigned, exchanged or re-homed between steps (by the caller, and by the packed prompts' own pairing of gate and up): every later step
+    runs on the new ones, to the bit as a model that was made with them."""
+    from aria_amd.serving import Scheduler
+
+    prompts = [torch.randint(0, 264, (n,), generator=L.gen(n)).tolist() for n in (5, 3)]
+
+    def session(s):
+        out = [s.step(["a", "b"], prompts), s.step(["a", "b"], [[7], [8]])]
+        s.finish("a"), s.finish("b")
+        return torch.cat(out).cpu()
+
+    for name, m, change, other in gptfast_moved_weights(dev, names):
+        want = session(Scheduler(other, 16))
+        sched = Scheduler(m, 16)
+        for first in (False, True):
+            if first:
+                session(sched)                                # (tables exist when the weights change)
+            else:
+                m.setup_caches(2, 16)
+                sched.slots, sched.free = 2, [0, 1]
+            if first or name == "assign":
+                change(m)
+                assert torch.equal(session(sched), want), name
+    m.layers[1].attention.wo.weight.data = m.layers[1].attention.wo.weight.data.T      # (refused by every path)
+    with pytest.raises(ValueError):
+        sched.step(["a", "b"], prompts)
 
 
 def case_rows_products(dev, M, N, K, E=3):
@@ -236,8 +294,6 @@ def case_trace_run(dev, tmp, dtype="float32", design="duguzen"):
 
 
 def case_registry():
-    import pytest
-
     from aria_amd import registry
 
     assert registry.architecture({"architecture": "Duguzen"}) == "Duguzen"

@@ -19,6 +19,10 @@ def test_gptfast_decode_batch():
     C.case_gptfast_decode_batch(DEV, 128, 64, 128, 3)
 
 
+def test_gptfast_moved_weights():
+    C.case_gptfast_moved_weights(DEV, ("assign", "module"))
+
+
 @pytest.mark.parametrize("M,N,K", [(5, 20, 136), (70, 9, 520)])
 def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)

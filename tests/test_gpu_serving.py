@@ -27,6 +27,10 @@ def test_gptfast_decode_batch(dim, head_dim, inter, requests, longest):
     C.case_gptfast_decode_batch(DEV, dim, head_dim, inter, requests, longest)
 
 
+def test_gptfast_moved_weights():
+    C.case_gptfast_moved_weights(DEV)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 100, 128), (16, 33, 1024), (17, 264, 1032), (33, 16, 1800), (64, 1000, 2560), (65, 7, 1792), (320, 40, 2568), (40, 130, 3336), (15, 24, 4096)])
 def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)
