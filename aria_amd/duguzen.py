@@ -158,7 +158,7 @@ class DuguzenForCausalLM(nn.Module):
             if self._decode is None:
                 self._decode = _DecodeTables(self)
             logits = self._decode.run(batch)
-            return logits if batch.wanted is None or batch.wanted.numel() == T else logits[batch.wanted.long()]
+            return logits if batch.every_row else logits[batch.wanted.long()]
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.dyt_stream(x, None, self.layer(0).norm1.params(), ids=batch.ids, table=self.embed)
         for i in range(len(self.config.layers)):

@@ -408,11 +408,12 @@ class Transformer(nn.Module):
     def step(self, batch) -> torch.Tensor:
         """Run a ``serving.StepBatch`` -> float32 logits [wanted rows, vocab]."""
         tables = self._step_tables(batch)
-        if tables is not None and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS:
+        together = tables is not None and batch.by_sequence
+        if together and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS:
             logits = tables.run(batch.ids, batch.slot, batch.pos, batch.max_len)
             if logits is not None:
-                return logits if batch.wanted is None or batch.wanted.numel() == len(logits) else logits[batch.wanted.long()]
-        if tables is not None and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length:
+                return logits if batch.every_row else logits[batch.wanted.long()]
+        if together and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length:
             logits = tables.prompts(batch) if batch.n_wanted <= batch.ids.numel() else None
             if logits is not None:
                 return logits

@@ -170,7 +170,7 @@ class KozipelForCausalLM(nn.Module):
             if self._decode is None:
                 self._decode = _DecodeTables(self)
             logits = self._decode.run(batch)
-            return logits if batch.wanted is None or batch.wanted.numel() == T else logits[batch.wanted.long()]
+            return logits if batch.every_row else logits[batch.wanted.long()]
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.rms_stream(x, c.width, c.eps, self.layers[c.runs[0].layer].norm1.weight, ids=batch.ids, table=self.embed, scale=c.embedding_scale)
         for i, run in enumerate(c.runs):

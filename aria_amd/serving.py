@@ -75,6 +75,21 @@ class StepBatch:
         return out
 
     @property
+    def every_row(self) -> bool:
+        """the logits of every row are asked for, in order (as many rows in another order, or some of them twice, are not)"""
+        return self.wanted is None or self.rows == list(range(self.ids.numel()))
+
+    @property
+    def by_sequence(self) -> bool:
+        """the wanted rows are the batch's own, sequence after sequence"""
+        if self.rows is None or self.wanted is None:
+            return self.rows is self.wanted
+        if not self.rows or (self.rows[0] >= 0 and self.rows[-1] < self.ids.numel() and sorted(self.rows) == self.rows):
+            return True
+        firsts = [at - n for at, n in zip(np.cumsum(self.lengths).tolist(), self.lengths)]
+        return self.rows == [first + j for first, want in zip(firsts, self.wanted_by_sequence()) for j in want]
+
+    @property
     def fresh(self) -> bool:
         """every sequence starts at its first token"""
         return not any(self.starts)

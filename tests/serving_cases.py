@@ -160,6 +160,50 @@ def case_gptfast_moved_weights(dev, names=("assign", "parameter", "data", "modul
         sched.step(["a", "b"], prompts)
 
 
+def toy(design, dev):
+    """A small decoder whose steps of several requests are one call."""
+    if design == "gptfast":
+        return gptfast_routed(dev, 128, 64, 128, 32)
+    cases, name = DESIGNS[design]
+    cfg = cases.CONFIGS[name]
+    return cases.build(cfg, cases.checkpoint(cfg, seed=3), dev, bf16)
+
+
+def case_wanted_rows(dev, design):
+    """Wanted places named twice, none of a request's, all but not in order: the rows of the step that asks for each once."""
+    from aria_amd.serving import Scheduler
+
+    m, prompts = toy(design, dev), [[5, 3, 7], [4, 9]]
+
+    def session(prompt_places, places):
+        s = Scheduler(m, 8)
+        out = [s.step("ab", prompts, prompt_places), s.step("ab", [[11], [12]], places)]
+        s.finish("a"), s.finish("b")
+        return [t.cpu() for t in out]
+
+    one, two = session([[0, 1, 2], [0, 1]], [[0], [0]])
+    got = session([[2, 0, 0, 1], [0]], [[0, 0], []])
+    assert torch.equal(got[0], one[[2, 0, 0, 1, 3]]) and torch.equal(got[1], two[[0, 0]])
+    got = session([[], [1, 0]], [[], [0, 0]])
+    assert torch.equal(got[0], one[[4, 3]]) and torch.equal(got[1], two[[1, 1]])
+
+
+def case_gptfast_wanted_outside(dev, dim=128, inter=128):
+    """Places that a request does not have are left out, in single steps as in packed prompts and in the prompts' one call."""
+    from aria_amd.serving import StepBatch
+
+    m = gptfast_routed(dev, dim, 64, inter, 32)
+    m.setup_caches(2, 8)
+
+    def step(tokens, starts, rows):
+        return m.step(StepBatch.build(tokens, [0, 1], starts, rows, dev)).cpu()
+
+    for tokens, starts in (([[5, 3, 7], [4, 9]], [0, 0]), ([[11], [12]], [3, 2])):
+        last = sum(map(len, tokens)) - 1
+        both, n = step(tokens, starts, [0, last]), 4 * 2 ** -8
+        assert L.logit_err(step(tokens, starts, [-1, 0]), both[:1]) < n and L.logit_err(step(tokens, starts, [last, last + 1]), both[1:]) < n
+
+
 def case_rows_products(dev, M, N, K, E=3):
     """The weight-streaming products at edges of their token tiles, row groups and windows of the reduction against float64; bf16 results: half an ulp, 2^-9,
     and twice that behind the rounded gate and up of SwiGLU."""

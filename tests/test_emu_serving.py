@@ -19,6 +19,15 @@ def test_gptfast_decode_batch():
     C.case_gptfast_decode_batch(DEV, 128, 64, 128, 3)
 
 
+@pytest.mark.parametrize("design", ["duguzen", "gptfast", "kozipel"])
+def test_wanted_rows(design):
+    C.case_wanted_rows(DEV, design)
+
+
+def test_gptfast_wanted_outside():
+    C.case_gptfast_wanted_outside(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 

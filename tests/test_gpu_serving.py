@@ -27,6 +27,16 @@ def test_gptfast_decode_batch(dim, head_dim, inter, requests, longest):
     C.case_gptfast_decode_batch(DEV, dim, head_dim, inter, requests, longest)
 
 
+@pytest.mark.parametrize("design", ["duguzen", "gptfast", "kozipel"])
+def test_wanted_rows(design):
+    C.case_wanted_rows(DEV, design)
+
+
+def test_gptfast_wanted_outside():
+    C.case_gptfast_wanted_outside(DEV)
+    C.case_gptfast_wanted_outside(DEV, 512, 512)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV)
 
