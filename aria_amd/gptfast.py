@@ -437,14 +437,15 @@ class Transformer(nn.Module):
                     logits = self.forward(toks, last_only=last)[0].float()
                     out.append(logits if last else logits[list(want)])
                 else:
+                    made = {}
                     for j in range(n):      # (on a cache: token by token)
                         token = slice(first + j, first + j + 1)
                         logits = tables.run(batch.ids[token], batch.slot[token], batch.pos[token], start + j + 1) if tables is not None else None
-                        if logits is not None:
-                            out += [logits] * list(want).count(j)
-                            continue
-                        logits = self.forward(toks[:, j:j + 1], torch.tensor([start + j], dtype=torch.int32, device=ids.device))
-                        out += [logits[0].float().clone()] * list(want).count(j)
+                        if logits is None:
+                            logits = self.forward(toks[:, j:j + 1], torch.tensor([start + j], dtype=torch.int32, device=ids.device))
+                            logits = logits[0].float().clone() if j in want else None
+                        made[j] = logits if j in want else None
+                    out += [made[j] for j in want]
                 self._slot_state[slot] = (rows, self._engine)
         finally:
             for b, c in zip(self.layers, whole):

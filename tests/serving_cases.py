@@ -188,6 +188,21 @@ def case_wanted_rows(dev, design):
     assert torch.equal(got[0], one[[4, 3]]) and torch.equal(got[1], two[[1, 1]])
 
 
+def case_gptfast_portion_order(dev):
+    """A portion of a prompt: logits in the order in which its places are named."""
+    from aria_amd.serving import Scheduler
+
+    m = gptfast_toy(dev)
+    m.use_decode_engine = False
+
+    def portion(places):
+        s = Scheduler(m, 8)
+        s.step(["a"], [[5, 3]], [[]])
+        return s.step(["a"], [[9, 2, 77]], [places]).cpu()
+
+    assert torch.equal(portion([2, 0, 2]), portion([0, 1, 2])[[2, 0, 2]])
+
+
 def case_gptfast_wanted_outside(dev, dim=128, inter=128):
     """Places that a request does not have are left out, in single steps as in packed prompts and in the prompts' one call."""
     from aria_amd.serving import StepBatch

@@ -28,6 +28,10 @@ def test_gptfast_wanted_outside():
     C.case_gptfast_wanted_outside(DEV)
 
 
+def test_gptfast_portion_order():
+    C.case_gptfast_portion_order(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 

@@ -37,6 +37,10 @@ def test_gptfast_wanted_outside():
     C.case_gptfast_wanted_outside(DEV, 512, 512)
 
 
+def test_gptfast_portion_order():
+    C.case_gptfast_portion_order(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV)
 
