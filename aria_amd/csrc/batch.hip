@@ -23,12 +23,12 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     sync();
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
-__global__ __launch_bounds__(256) void embedding_rows_kernel(const int32_t* ids, const bf16_t* table, const bf16_t* norm, bf16_t* x, bf16_t* h, float* sums, int D, int V) {
+__global__ __launch_bounds__(256) void embedding_rows_kernel(const bf16_t* rows, const bf16_t* norm, bf16_t* x, bf16_t* h, float* sums, int D) {
     ARIA_SMEM_STATIC float red[4];
     const int n = blockIdx.x * STREAM_COLS + threadIdx.x, tok = blockIdx.y;
     float v = 0.f;
     if (n < D) {
-        const bf16_t b = table[(long long)min(max(ids[tok], 0), V - 1) * D + n];
+        const bf16_t b = rows[(long long)tok * D + n];
         v = bf2f(b);
         x[(long long)tok * D + n] = b;
         h[(long long)tok * D + n] = f2bf(v * bf2f(norm[n]));
@@ -171,18 +171,18 @@ int64_t aria_decode_step_scratch(const int64_t* dims, int64_t T, int64_t max_len
     return batch_ok(dims, T) ? layout(dims, T, max_len, nullptr).bytes : 0;
 }
 
-int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const void* x, const int32_t* slot, const int32_t* pos,
                      int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream) {
-    if (!ptrs || !dims || !ids || !slot || !pos || !logits || !scratch || T < 0 || max_len <= 0) return ARIA_ERR_INVALID;
+    if (!ptrs || !dims || !x || !slot || !pos || !logits || !scratch || T < 0 || max_len <= 0) return ARIA_ERR_INVALID;
     if (T == 0) return ARIA_OK;
-    if (reinterpret_cast<uintptr_t>(scratch) & 15) return ARIA_ERR_ALIGN;
+    if ((reinterpret_cast<uintptr_t>(scratch) | reinterpret_cast<uintptr_t>(x)) & 15) return ARIA_ERR_ALIGN;
     const int64_t need = aria_decode_step_scratch(dims, T, max_len);
     if (need == 0) return ARIA_ERR_UNSUPPORTED;
     const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8], Smax = dims[9];
     if (scratch_bytes < need || max_len > Smax) return ARIA_ERR_INVALID;
     for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
         if (!ptrs[i]) return ARIA_ERR_INVALID;
-    if (T == 1) return aria_decode_one(ptrs, dims, eps, ids, slot, pos, max_len, logits, static_cast<char*>(scratch), stream);
+    if (T == 1) return aria_decode_one(ptrs, dims, eps, x, slot, pos, max_len, logits, static_cast<char*>(scratch), stream);
     const Scratch z = layout(dims, T, max_len, static_cast<char*>(scratch));
     auto weight = [&](int64_t i) { return static_cast<const bf16_t*>(ptrs[i]); };
     const int64_t ns = Is / I;
@@ -192,8 +192,8 @@ int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, in
     int sq_n = parts;   // partial sums a token has beside h
     auto input = [&](const bf16_t* W, int64_t N) { return RowsIn{W, nullptr, z.h, (long long)D, int(D), int(N), z.sums, sq_n, inv_n, eps}; };
     auto rows = [&](const RowsIn& in, const auto& e) { return launch_rows(RowsPair{{in, in}}, 1, T, e, stream); };
-    ARIA_LAUNCH(embedding_rows_kernel, stream_grid, dim3(256), 0, stream, ids, weight(3), weight(ARIA_DECODE_STEP_PTRS), z.x, z.h, z.sums, int(D),
-                int(V));
+    ARIA_LAUNCH(embedding_rows_kernel, stream_grid, dim3(256), 0, stream, static_cast<const bf16_t*>(x), weight(ARIA_DECODE_STEP_PTRS), z.x, z.h, z.sums,
+                int(D));
     int rc = aria_check_launch();
     const ExpertLists lists{z.table, z.list, int(E + ns)};
     for (int64_t li = 0; li < L && rc == ARIA_OK; ++li) {

@@ -18,5 +18,5 @@ ARIA_HIDDEN int aria_route_and_sort(const ad::bf16_t* logits, ad::bf16_t* scores
 ARIA_HIDDEN int aria_decode_dims_ok(const int64_t* dims);
 // One sequence's step by the engine's kernels
 ARIA_HIDDEN int64_t aria_decode_one_scratch(const int64_t* dims);
-ARIA_HIDDEN int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+ARIA_HIDDEN int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const void* x, const int32_t* slot, const int32_t* pos,
                                 int64_t max_len, float* logits, char* scratch, void* stream);

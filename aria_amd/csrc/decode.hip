@@ -634,11 +634,6 @@ __global__ void decode_attn_merge_kernel(const float* part, bf16_t* out, int NS,
     out[((long long)tok * gridDim.x + head) * HD + f] = f2bf(acc);
 }
 
-__global__ __launch_bounds__(256) void embedding_row_kernel(const int32_t* id, const bf16_t* table, bf16_t* x, int nch, int V) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c < nch) st16(x + c * 8, ld16(table + ((long long)min(max(id[0], 0), V - 1) * nch + c) * 8));
-}
-
 struct Scratch {
     bf16_t *xa, *xb, *qkv, *ao, *rl, *scores, *act, *eo;
     int32_t *idx, *kv_len;
@@ -1023,17 +1018,12 @@ int aria_decode_rows_attn(const bf16_t* qkv, const bf16_t* freqs, const int32_t*
 }
 int aria_decode_dims_ok(const int64_t* dims) { return dims_ok(dims); }
 int64_t aria_decode_one_scratch(const int64_t* dims) {
-    return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes) + 2 * dims[1];
+    return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes);
 }
-int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const int32_t* ids, const int32_t* slot, const int32_t* pos, int64_t max_len,
+int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const void* x, const int32_t* slot, const int32_t* pos, int64_t max_len,
                     float* logits, char* scratch, void* stream) {
-    const int64_t D = dims[1];
-    const Scratch s = carve(scratch, dims[0], D, dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
-    bf16_t* x = reinterpret_cast<bf16_t*>(scratch + s.bytes);
-    ARIA_LAUNCH(embedding_row_kernel, dim3(unsigned((D / 8 + 255) / 256)), dim3(256), 0, stream, ids, static_cast<const bf16_t*>(ptrs[3]), x, int(D / 8),
-                int(dims[8]));
-    if (const int rc = aria_check_launch()) return rc;
-    const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]), x,
+    const Scratch s = carve(scratch, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
+    const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]), static_cast<const bf16_t*>(x),
                        ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len)};
     return decode_one(one, s, dims, eps, stream);
 }

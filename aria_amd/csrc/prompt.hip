@@ -7,12 +7,9 @@
 namespace {
 using namespace ad;
 
-__global__ __launch_bounds__(256) void prompt_rows_kernel(const int32_t* ids, const bf16_t* table, bf16_t* x, int nch, int T, int V, int32_t* counts, int n_counts) {
+__global__ __launch_bounds__(256) void clear_counts_kernel(int32_t* counts, int n) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n_counts) counts[i] = 0;
-    if (i >= T * nch) return;
-    const int t = i / nch, c = i - t * nch;
-    st16(x + (long long)i * 8, ld16(table + ((long long)min(max(ids[t], 0), V - 1) * nch + c) * 8));
+    if (i < n) counts[i] = 0;
 }
 
 struct Scratch {
@@ -51,13 +48,13 @@ int64_t aria_prompt_step_scratch(const int64_t* dims, int64_t T) {
     return dims && T > 0 && prompt_ok(dims, T) ? layout(dims, T, nullptr).bytes : 0;
 }
 
-int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const void* embedded, const int32_t* slot, const int32_t* pos,
                      const int32_t* cu, int64_t n_seq, int64_t longest, const int32_t* wanted, int64_t n_wanted, float* logits, void* scratch,
                      int64_t scratch_bytes, void* stream) {
-    if (!ptrs || !dims || !ids || !slot || !pos || !cu || !scratch || T < 0 || n_seq <= 0 || longest <= 0 || n_wanted < 0 || (n_wanted && (!wanted || !logits)))
+    if (!ptrs || !dims || !embedded || !slot || !pos || !cu || !scratch || T < 0 || n_seq <= 0 || longest <= 0 || n_wanted < 0 || (n_wanted && (!wanted || !logits)))
         return ARIA_ERR_INVALID;
     if (T == 0) return ARIA_OK;
-    if (reinterpret_cast<uintptr_t>(scratch) & 15) return ARIA_ERR_ALIGN;
+    if ((reinterpret_cast<uintptr_t>(scratch) | reinterpret_cast<uintptr_t>(embedded)) & 15) return ARIA_ERR_ALIGN;
     const int64_t need = aria_prompt_step_scratch(dims, T);
     if (need == 0) return ARIA_ERR_UNSUPPORTED;
     const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8], Smax = dims[9];
@@ -65,12 +62,14 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
     for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
         if (!ptrs[i]) return ARIA_ERR_INVALID;
     const Scratch z = layout(dims, T, static_cast<char*>(scratch));
-    const int64_t items = std::max(T * (D / 8), L * E);
-    ARIA_LAUNCH(prompt_rows_kernel, dim3(unsigned((items + 255) / 256)), dim3(256), 0, stream, ids, static_cast<const bf16_t*>(ptrs[3]), z.x, int(D / 8), int(T), int(V),
-                z.counts, int(L * E));
+    ARIA_LAUNCH(clear_counts_kernel, dim3(unsigned((L * E + 255) / 256)), dim3(256), 0, stream, z.counts, int(L * E));
     int rc = aria_check_launch();
-    bf16_t *x = z.x, *y = z.y;   // the residual before and behind the sum that comes next
-    const bf16_t* delta = nullptr;
+    const bf16_t *x = static_cast<const bf16_t*>(embedded), *delta = nullptr;   // the residual before the sum that comes next; y: behind it
+    bf16_t *y = z.x, *spare = z.y;
+    auto summed = [&] {
+        x = y;
+        std::swap(y, spare);
+    };
 #define ARIA_TRY(call) \
     if (rc == ARIA_OK) rc = (call)
     for (int64_t li = 0; li < L; ++li) {
@@ -78,7 +77,7 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         void *kc = const_cast<void*>(p[11]), *vc = const_cast<void*>(p[12]);
         if (delta) {
             ARIA_TRY(aria_rmsnorm_fwd(delta, x, p[0], y, z.h, nullptr, T, D, eps, stream));
-            std::swap(x, y);
+            summed();
         } else {
             ARIA_TRY(aria_rmsnorm_fwd(x, nullptr, p[0], nullptr, z.h, nullptr, T, D, eps, stream));
         }
@@ -88,7 +87,7 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
                                       1.0f / sqrtf(float(hd)), stream));
         ARIA_TRY(aria_rows_gemm(z.ao, p[2], z.d, 0, T, D, D, D, D, stream));
         ARIA_TRY(aria_rmsnorm_fwd(z.d, x, p[3], y, z.h, nullptr, T, D, eps, stream));
-        std::swap(x, y);
+        summed();
         ARIA_TRY(aria_rows_gemm(z.h, p[4], z.logits, 0, T, E, D, D, E, stream));
         ARIA_TRY(aria_route_and_sort(z.logits, z.scores, z.idx, z.counts + li * E, z.offsets, z.src, z.inv, z.rows, int(T), int(E), int(k), stream));
         ARIA_TRY(aria_rows_experts(z.h, z.rows, z.offsets, p[5], p[6], z.act, E, T * k, I, D, D, I, stream));

@@ -391,12 +391,22 @@ class Transformer(nn.Module):
         return (batch.fresh and len(batch.lengths) > 1 and batch.longest > 1 and batch.ids.numel() <= 65536 and _glu_pair_ready(f.cond_ffn.w1, f.cond_ffn.w3)
                 and ops.gather_fusable(self.config.dim) and self.freqs_cis.shape[0] >= self.max_seq_length)
 
-    def _prompts(self, batch) -> torch.Tensor:
+    def _embedded(self, batch) -> Optional[torch.Tensor]:
+        """The batch's embedding rows as the one-call steps read them, [T, D] (None: another type or place than theirs).  The module makes them: it takes what
+        integers it takes and refuses what is not in its vocabulary."""
+        ids, D = batch.ids.reshape(-1), self.config.dim
+        x = self.tok_embeddings(ids if ids.dtype in (torch.int32, torch.int64) else ids.long())
+        if x.dtype != bf16 or tuple(x.shape) != (ids.numel(), D) or x.device != self.device:
+            return None
+        x = x.contiguous()
+        return x if x.data_ptr() % 16 == 0 else x.clone()
+
+    def _prompts(self, batch, x) -> torch.Tensor:
         if batch.wanted is not None and batch.wanted.numel() == 0:
             wanted = None
         else:
             wanted = slice(None) if batch.wanted is None else batch.wanted.long()
-        res, delta = self.tok_embeddings(batch.ids.long()), None
+        res, delta = x, None
         for layer in self.layers:
             res, delta = layer(res, delta, None, None, self.freqs_cis, None, None, True, packed=batch)
         if wanted is None:
@@ -408,23 +418,32 @@ class Transformer(nn.Module):
     def step(self, batch) -> torch.Tensor:
         """Run a ``serving.StepBatch`` -> float32 logits [wanted rows, vocab]."""
         tables = self._step_tables(batch)
+        if tables is not None:
+            batch = batch.tables_for(self.device)
         together = tables is not None and batch.by_sequence
-        if together and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS:
-            logits = tables.run(batch.ids, batch.slot, batch.pos, batch.max_len)
+        made = []
+
+        def embed():
+            if not made:
+                made.append(self._embedded(batch))
+            return made[0]
+
+        if together and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS and embed() is not None:
+            logits = tables.run(embed(), batch.slot, batch.pos, batch.max_len)
             if logits is not None:
                 return logits if batch.every_row else logits[batch.wanted.long()]
         if together and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length:
-            logits = tables.prompts(batch) if batch.n_wanted <= batch.ids.numel() else None
+            logits = tables.prompts(batch, embed) if batch.n_wanted <= batch.ids.numel() else None
             if logits is not None:
                 return logits
-            if self._packs(batch):
-                return self._prompts(batch)
+            if self._packs(batch) and embed() is not None:
+                return self._prompts(batch, embed())
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:
             self._slot_key, self._slot_state = key, {}      # slot -> (per-layer cache rows, decode engine)
         out, at, engine = [], 0, self._engine
-        ids = batch.ids.long()
+        ids = batch.ids.reshape(-1).long()
         try:
             for n, start, slot, want in zip(batch.lengths, batch.starts, batch.slots, batch.wanted_by_sequence()):
                 rows, self._engine = self._slot_state.get(slot) or ([c.row(slot) for c in whole], None)
@@ -440,7 +459,8 @@ class Transformer(nn.Module):
                     made = {}
                     for j in range(n):      # (on a cache: token by token)
                         token = slice(first + j, first + j + 1)
-                        logits = tables.run(batch.ids[token], batch.slot[token], batch.pos[token], start + j + 1) if tables is not None else None
+                        logits = (tables.run(embed()[token], batch.slot[token], batch.pos[token], start + j + 1) if tables is not None and embed() is not None
+                                  else None)
                         if logits is None:
                             logits = self.forward(toks[:, j:j + 1], torch.tensor([start + j], dtype=torch.int32, device=ids.device))
                             logits = logits[0].float().clone() if j in want else None
@@ -479,17 +499,17 @@ class _StepTables:
         self.dims = np.array([c.n_layer, c.dim, c.n_head, c.head_dim, c.num_experts, c.router_topk, c.intermediate_size,
                               c.intermediate_size * c.num_shared_experts, c.vocab_size, model.max_seq_length], dtype=np.int64)
         self.dims_p = self.dims.ctypes.data_as(ctypes.c_void_p)
-        tensors = [model.freqs_cis, model.norm.weight, model.output.weight, model.tok_embeddings.weight] + _layer_table(model)
+        tensors = [model.freqs_cis, model.norm.weight, model.output.weight] + _layer_table(model)
         self.tensors = [t.detach() for t in tensors]      # (a parameter's storage may be exchanged, a detached tensor's not)
         D, I, Is, E, cache = c.dim, c.intermediate_size, c.intermediate_size * c.num_shared_experts, c.num_experts, tuple(model.layers[0].attention.kv_cache.k.shape)
         layer = [(D,), (3 * D, D), (D, D), (D,), (E, D), (E, I, D), (E, I, D), (E, D, I), (Is, D), (Is, D), (D, Is), cache, cache]
-        shapes = [(model.freqs_cis.shape[0], c.head_dim // 2, 2), (D,), (c.vocab_size, D), (c.vocab_size, D)] + layer * c.n_layer
+        shapes = [(model.freqs_cis.shape[0], c.head_dim // 2, 2), (D,), (c.vocab_size, D)] + layer * c.n_layer
         self.served = (all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in tensors) and [tuple(t.shape) for t in tensors] == shapes
                        and cache[1:] == (model.max_seq_length, D) and model.freqs_cis.shape[0] >= model.max_seq_length)
         self.ptrs = (ctypes.c_void_p * len(tensors))(*(t.data_ptr() for t in tensors))
         # ways to the weights: (modules of the parent, name, module), (parameters of the module, name); addresses and sizes of these
         self.modules, self.ways, seen = [], [], set()
-        for path in [("norm", "weight"), ("output", "weight"), ("tok_embeddings", "weight")] + [("layers", str(i)) + w for i in range(c.n_layer) for w in _LAYER_WEIGHTS]:
+        for path in [("norm", "weight"), ("output", "weight")] + [("layers", str(i)) + w for i in range(c.n_layer) for w in _LAYER_WEIGHTS]:
             at = model
             for name in path[:-1]:
                 parent, at = at, at._modules[name]
@@ -511,33 +531,30 @@ class _StepTables:
         return (not [None for t in weights if t is None] and list(map(torch.Tensor.data_ptr, weights)) == self.where and list(map(torch.Tensor.numel, weights)) == self.sizes
                 and all(map(torch.Tensor.is_contiguous, weights)))
 
-    def run(self, ids, slot, pos, max_len: int) -> Optional[torch.Tensor]:
-        """logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""
-        lib, T = hip.get_lib(), ids.numel()
+    def run(self, x, slot, pos, max_len: int) -> Optional[torch.Tensor]:
+        """embedding rows x [T, D] -> logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""
+        lib, T = hip.get_lib(), x.shape[0]
         need = int(lib.cdll.aria_decode_step_scratch(self.dims_p, T, max_len)) if self.served else 0
         if need == 0:
             return None
-        scratch = torch.empty(need, dtype=torch.uint8, device=ids.device)
-        logits = torch.empty((T, int(self.dims[8])), dtype=torch.float32, device=ids.device)
-        for t in (ids, slot, pos):
-            assert t.dtype == torch.int32 and t.is_contiguous() and t.numel() == T
-        lib.call("aria_decode_step", self.ptrs, self.dims_p, self.eps, T, ids.data_ptr(), slot.data_ptr(), pos.data_ptr(), max_len, logits.data_ptr(),
+        scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+        logits = torch.empty((T, int(self.dims[8])), dtype=torch.float32, device=x.device)
+        lib.call("aria_decode_step", self.ptrs, self.dims_p, self.eps, T, x.data_ptr(), slot.data_ptr(), pos.data_ptr(), max_len, logits.data_ptr(),
                  scratch.data_ptr(), need, ops._stream(logits))
         return logits
 
-    def prompts(self, batch) -> Optional[torch.Tensor]:
-        """logits float32 [wanted rows, vocab] of a batch of whole short prompts; None: not served in one call"""
+    def prompts(self, batch, embed) -> Optional[torch.Tensor]:
+        """logits float32 [wanted rows, vocab] of a batch of whole short prompts (embed: makes its embedding rows [T, D]); None: not served in one call"""
         lib, T = hip.get_lib(), batch.ids.numel()
         need = int(lib.cdll.aria_prompt_step_scratch(self.dims_p, T)) if self.served and T <= ops.ROWS_TOKENS else 0
-        if need == 0:
+        x = embed() if need else None
+        if x is None:
             return None
-        scratch = torch.empty(need, dtype=torch.uint8, device=batch.ids.device)
-        wanted = torch.arange(T, dtype=torch.int32, device=batch.ids.device) if batch.wanted is None else batch.wanted
-        logits = torch.empty((wanted.numel(), int(self.dims[8])), dtype=torch.float32, device=batch.ids.device)
-        for t in (batch.ids, batch.slot, batch.pos, batch.cu, wanted):
-            assert t.dtype == torch.int32 and t.is_contiguous()
+        scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+        wanted = torch.arange(T, dtype=torch.int32, device=x.device) if batch.wanted is None else batch.wanted
         n = wanted.numel()
-        lib.call("aria_prompt_step", self.ptrs, self.dims_p, self.eps, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.cu.data_ptr(),
+        logits = torch.empty((n, int(self.dims[8])), dtype=torch.float32, device=x.device)
+        lib.call("aria_prompt_step", self.ptrs, self.dims_p, self.eps, T, x.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.cu.data_ptr(),
                  len(batch.lengths), batch.longest, wanted.data_ptr() if n else None, n, logits.data_ptr() if n else None, scratch.data_ptr(),
                  need, ops._stream(scratch))
         return logits

@@ -12,7 +12,7 @@ sequence after the other for continued prompts and for sizes its kernels do not 
 (bin/trace_run) drive."""
 from __future__ import annotations
 
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
@@ -74,6 +74,16 @@ class StepBatch:
             first += n
         return out
 
+    def tables_for(self, device) -> "StepBatch":
+        """This batch with its tables as a library call reads them (one made by hand may hold other integers, strides, places)."""
+        T = self.ids.numel()
+        if self.slot.numel() != T or self.pos.numel() != T or sum(self.lengths) != T or self.cu.numel() != len(self.lengths) + 1:
+            raise ValueError(f"{T} tokens, lengths {self.lengths}, tables of {self.slot.numel()}, {self.pos.numel()} and {self.cu.numel()} entries")
+        own = {n: getattr(self, n) for n in ("slot", "pos", "cu", "wanted")}
+        odd = {n: t.to(device, torch.int32).contiguous() for n, t in own.items()
+               if t is not None and (t.dtype != torch.int32 or t.device != device or not t.is_contiguous())}
+        return replace(self, **odd) if odd else self
+
     @property
     def every_row(self) -> bool:
         """the logits of every row are asked for, in order (as many rows in another order, or some of them twice, are not)"""
@@ -109,7 +119,8 @@ class StepBatch:
 
     @classmethod
     def build(cls, tokens: Sequence, slots: Sequence[int], starts: Sequence[int], wanted: Optional[Sequence[int]], device) -> "StepBatch":
-        """tokens: one list of ids per sequence, or an int32 device tensor with one id per sequence (a decode step whose ids never visited the host)."""
+        """tokens: one list of ids per sequence, or an int32 device tensor with one id per sequence (a decode step whose ids never visited the host; Aria
+        takes any integers and strides)."""
         on_device = isinstance(tokens, torch.Tensor)
         lengths = [1] * len(slots) if on_device else [len(t) for t in tokens]
         T, n = sum(lengths), len(lengths)

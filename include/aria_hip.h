@@ -436,21 +436,20 @@ int aria_rows_experts(const void* X, const int32_t* rows, const int32_t* offsets
 #define ARIA_DECODE_LAYER_PTRS 13
 int64_t aria_decode_scratch_bytes(const int64_t* dims);
 int aria_decode_token(const void* const* ptrs, const int64_t* dims, float eps, void* stream);
-/* One serving step of T sequences, one token each (token ids, cache slots, positions: int32 [T] on the device; max_len >= largest position + 1, known to
- * the host): embedding rows to fp32 logits [T, V].  One sequence runs the kernels of aria_decode_token, several the batched ones (batch.hip: every weight
+/* One serving step of T sequences, one token each: x, the tokens' embedding rows (bf16 [T, D], 16-byte aligned), to fp32 logits [T, V] (cache slots, positions:
+ * int32 [T] on the device; max_len >= largest position + 1, known to the host).  One sequence runs the kernels of aria_decode_token, several the batched ones (batch.hip: every weight
  * read once for all tokens; meant for T up to 16).
- * ptrs: [0] freqs_cis   [1] final norm weight   [2] output weight [V, D]   [3] embedding [vocab, D]   then the 13 of a layer as above, caches
- *   [slots, S_max, D].  dims as above.
+ * ptrs: [0] freqs_cis   [1] final norm weight   [2] output weight [V, D]   then the 13 of a layer as above, caches [slots, S_max, D].  dims as above.
  * scratch: 16-byte aligned; 0 bytes from aria_decode_step_scratch: these sizes are not served (aria_decode_step: ARIA_ERR_UNSUPPORTED). */
-#define ARIA_DECODE_STEP_PTRS 4
+#define ARIA_DECODE_STEP_PTRS 3
 int64_t aria_decode_step_scratch(const int64_t* dims, int64_t T, int64_t max_len);
-int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const void* x, const int32_t* slot, const int32_t* pos,
                      int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
-/* One serving step over T packed tokens of n_seq whole prompts (sequence b = rows cu[b] .. cu[b + 1), positions from 0; ids, slot, pos, cu, wanted: int32 on the
+/* One serving step over T packed tokens of n_seq whole prompts (sequence b = rows cu[b] .. cu[b + 1), positions from 0; x as above; slot, pos, cu, wanted: int32 on the
  * device; longest: the host's maximum length): keys and values into the caches, fp32 logits [n_wanted, V] of the wanted rows.  ptrs, dims as
  * aria_decode_step.  For prompts of a few hundred tokens together (prompt.hip); scratch: 0 bytes from aria_prompt_step_scratch as above. */
 int64_t aria_prompt_step_scratch(const int64_t* dims, int64_t T);
-int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, int64_t T, const void* x, const int32_t* slot, const int32_t* pos,
                      const int32_t* cu, int64_t n_seq, int64_t longest, const int32_t* wanted, int64_t n_wanted, float* logits, void* scratch,
                      int64_t scratch_bytes, void* stream);
 /* Where, inside the scratch buffer, the last aria_decode_token call left every layer's routing record (TopKRouter of

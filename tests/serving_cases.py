@@ -188,6 +188,32 @@ def case_wanted_rows(dev, design):
     assert torch.equal(got[0], one[[4, 3]]) and torch.equal(got[1], two[[1, 1]])
 
 
+def case_gptfast_ids(dev, dim=128, inter=128):
+    """Steps take the ids of any integer type and stride on the device, and refuse on the CPU, where that can be looked at, the same ids as a model's embedding:
+    outside the vocabulary, in prompts of one call, packed prompts and decoded tokens."""
+    from aria_amd.serving import Scheduler
+
+    m = gptfast_routed(dev, dim, 64, inter, 32)
+
+    def session(second, prompts=([5, 3, 7], [4, 9])):
+        s = Scheduler(m, 8)
+        out = [s.step("ab", list(prompts)), s.step("ab", second)]
+        s.finish("a"), s.finish("b")
+        return torch.cat(out).cpu()
+
+    want = session([[11], [12]])
+    ids = torch.tensor([11, 12], device=dev)
+    strided = torch.stack([ids, ids + 1], 1)[:, 0]
+    for second in (ids, ids.int(), ids.short(), strided, strided.int(), ids.view(2, 1)):
+        assert torch.equal(session(second), want), (second.dtype, second.shape, second.stride())
+    if str(dev) == "cpu":
+        for bad in ([[264], [12]], [[11], [-1]], ids + 256):
+            with pytest.raises(IndexError):
+                session(bad)
+        with pytest.raises(IndexError):
+            session([[11], [12]], ([5, 264, 7], [4, 9]))
+
+
 def case_gptfast_portion_order(dev):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

@@ -32,6 +32,10 @@ def test_gptfast_portion_order():
     C.case_gptfast_portion_order(DEV)
 
 
+def test_gptfast_ids():
+    C.case_gptfast_ids(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 
