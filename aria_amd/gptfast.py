@@ -421,12 +421,12 @@ class Transformer(nn.Module):
         if tables is not None:
             batch = batch.tables_for(self.device)
         together = tables is not None and batch.by_sequence
-        made = []
+        embedded = []
 
         def embed():
-            if not made:
-                made.append(self._embedded(batch))
-            return made[0]
+            if not embedded:
+                embedded.append(self._embedded(batch))
+            return embedded[0]
 
         if together and batch.longest == 1 and batch.ids.numel() <= DECODE_ROWS and embed() is not None:
             logits = tables.run(embed(), batch.slot, batch.pos, batch.max_len)

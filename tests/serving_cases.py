@@ -214,12 +214,12 @@ def case_gptfast_ids(dev, dim=128, inter=128):
             session([[11], [12]], ([5, 264, 7], [4, 9]))
 
 
-def case_gptfast_portion_order(dev):
+def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler
 
     m = gptfast_toy(dev)
-    m.use_decode_engine = False
+    m.use_decode_engine = engine
 
     def portion(places):
         s = Scheduler(m, 8)

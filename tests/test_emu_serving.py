@@ -28,8 +28,9 @@ def test_gptfast_wanted_outside():
     C.case_gptfast_wanted_outside(DEV)
 
 
-def test_gptfast_portion_order():
-    C.case_gptfast_portion_order(DEV)
+@pytest.mark.parametrize("engine", [False, True])
+def test_gptfast_portion_order(engine):
+    C.case_gptfast_portion_order(DEV, engine)
 
 
 def test_gptfast_ids():
