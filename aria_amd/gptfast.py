@@ -370,7 +370,7 @@ class Transformer(nn.Module):
         cache = self.layers[0].attention.kv_cache
         if cache is None or not self.use_decode_engine or self.decode_graph or not self._engine_capable():
             return None
-        if batch.max_len > self.max_seq_length or max(batch.slots) >= cache.k.shape[0]:
+        if batch.max_len > self.max_seq_length or max(batch.slots) >= cache.k.shape[0] or min(batch.slots) < 0 or min(batch.starts) < 0:
             raise ValueError("the batch does not fit the caches")
         if self._tables is None or not self._tables.valid_for(self):
             self._tables = _StepTables(self)
@@ -420,7 +420,8 @@ class Transformer(nn.Module):
         tables = self._step_tables(batch)
         if tables is not None:
             batch = batch.tables_for(self.device)
-        together = tables is not None and batch.by_sequence
+        # (a slot that the batch names twice: its second part reads what the first one writes)
+        together = tables is not None and batch.by_sequence and len(set(batch.slots)) == len(batch.slots)
         embedded = []
 
         def embed():

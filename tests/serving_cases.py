@@ -214,6 +214,26 @@ def case_gptfast_ids(dev, dim=128, inter=128):
             session([[11], [12]], ([5, 264, 7], [4, 9]))
 
 
+def case_gptfast_slot_twice(dev, dim=128, inter=128):
+    """A batch that names a slot twice runs its parts in order, the second one on the rows of the first; slots and positions before the first are refused."""
+    from aria_amd.serving import StepBatch
+
+    m = gptfast_routed(dev, dim, 64, inter, 32)
+    m.setup_caches(2, 8)
+
+    def step(tokens, slots, starts):
+        return m.step(StepBatch.build(tokens, slots, starts, None, dev)).cpu()
+
+    step([[5, 3], [9, 9]], [0, 1], [0, 0])
+    want = [step([[t]], [0], [2 + i]) for i, t in enumerate((7, 4))]
+    for c in m.layers[0].attention.kv_cache.k, m.layers[1].attention.kv_cache.v:
+        c[0, 2:].fill_(float("nan"))
+    assert torch.equal(step([[7], [4]], [0, 0], [2, 3]), torch.cat(want))
+    for slots, starts in (([0, -1], [2, 2]), ([0, 1], [2, -1]), ([0, 2], [2, 2]), ([0, 1], [2, 8])):
+        with pytest.raises(ValueError):
+            step([[7], [4]], slots, starts)
+
+
 def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

@@ -37,6 +37,10 @@ def test_gptfast_ids():
     C.case_gptfast_ids(DEV)
 
 
+def test_gptfast_slot_twice():
+    C.case_gptfast_slot_twice(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 
