@@ -433,7 +433,7 @@ class Transformer(nn.Module):
             logits = tables.run(embed(), batch.slot, batch.pos, batch.max_len)
             if logits is not None:
                 return logits if batch.every_row else logits[batch.wanted.long()]
-        if together and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length:
+        if together and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length and not tables.watched(self):
             logits = tables.prompts(batch, embed) if batch.n_wanted <= batch.ids.numel() else None
             if logits is not None:
                 return logits
@@ -483,6 +483,12 @@ def _pair_weights(model: "Transformer") -> None:
         _glu_pair_ready(ff.shared_ffn.w1.weight, ff.shared_ffn.w3.weight)
 
 
+def _own_layers(model: "Transformer") -> bool:
+    """Layers of other classes run as modules: the library knows nothing of what they compute."""
+    return all(type(b) is TransformerBlock and type(b.attention) is Attention and type(b.feed_forward) is MOEFeedForward and
+               type(b.attention_norm) is type(b.ffn_norm) is RMSNorm for b in model.layers)
+
+
 class _StepTables:
     """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches.  Every step compares them with the tensors that the model
     holds then (assigned, moved or replaced weights and modules: about 0.1 us a tensor, beside a device that is busy with the step before), and
@@ -495,6 +501,9 @@ class _StepTables:
         import numpy as np
 
         c = model.config
+        self.modules, self.served = [], False
+        if not _own_layers(model):
+            return
         _pair_weights(model)
         self.key, self.eps = DecodeEngine._cheap_key(model), float(c.norm_eps)
         self.dims = np.array([c.n_layer, c.dim, c.n_head, c.head_dim, c.num_experts, c.router_topk, c.intermediate_size,
@@ -509,7 +518,7 @@ class _StepTables:
                        and cache[1:] == (model.max_seq_length, D) and model.freqs_cis.shape[0] >= model.max_seq_length)
         self.ptrs = (ctypes.c_void_p * len(tensors))(*(t.data_ptr() for t in tensors))
         # ways to the weights: (modules of the parent, name, module), (parameters of the module, name); addresses and sizes of these
-        self.modules, self.ways, seen = [], [], set()
+        self.ways, seen = [], set()
         for path in [("norm", "weight"), ("output", "weight")] + [("layers", str(i)) + w for i in range(c.n_layer) for w in _LAYER_WEIGHTS]:
             at = model
             for name in path[:-1]:
@@ -531,6 +540,13 @@ class _StepTables:
         weights = [of.get(name) for of, name in self.ways]
         return (not [None for t in weights if t is None] and list(map(torch.Tensor.data_ptr, weights)) == self.where and list(map(torch.Tensor.numel, weights)) == self.sizes
                 and all(map(torch.Tensor.is_contiguous, weights)))
+
+    def watched(self, model: "Transformer") -> bool:
+        """Somebody looks at or changes what the model's modules do with a prompt (forward hooks, other forwards): it then runs module by module.  (Single
+        tokens have never done that on the decode engine.)"""
+        everywhere = nn.modules.module
+        return not _own_layers(model) or bool(everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks or
+                                              [None for _, _, m in self.modules if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__])
 
     def run(self, x, slot, pos, max_len: int) -> Optional[torch.Tensor]:
         """embedding rows x [T, D] -> logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""

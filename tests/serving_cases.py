@@ -234,6 +234,41 @@ def case_gptfast_slot_twice(dev, dim=128, inter=128):
             step([[7], [4]], slots, starts)
 
 
+def case_gptfast_hooks(dev, dim=128, inter=128):
+    """Hooks on the modules see every prompt by itself, as do replaced forwards and layers of other classes; logits as without them."""
+    from aria_amd import gptfast as G
+    from aria_amd.serving import Scheduler
+
+    m, prompts = gptfast_routed(dev, dim, 64, inter, 32), [[5, 3, 7], [4, 9]]
+
+    def prompt():
+        s = Scheduler(m, 8)
+        out = s.step("ab", prompts).cpu().double()
+        s.finish("a"), s.finish("b")
+        return out
+
+    want, seen = prompt(), []
+    block = m.layers[1]
+    for part in (block, block.attention, block.feed_forward):
+        for register in (part.register_forward_hook, part.register_forward_pre_hook):
+            hook = register(lambda m, a, *out: seen.append(a[0].shape[0]))
+            assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2]
+            hook.remove()
+            seen.clear()
+    plain = block.feed_forward.forward
+    block.feed_forward.forward = lambda x: seen.append(x.shape[0]) or plain(x)
+    assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2]
+    del block.feed_forward.forward
+
+    class Other(G.MOEFeedForward):
+        def forward(self, x):
+            seen.append(-x.shape[0])
+            return super().forward(x)
+
+    block.feed_forward.__class__ = Other
+    assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2, -3, -2]
+
+
 def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

@@ -50,6 +50,11 @@ def test_gptfast_slot_twice():
     C.case_gptfast_slot_twice(DEV)
 
 
+def test_gptfast_hooks():
+    C.case_gptfast_hooks(DEV)
+    C.case_gptfast_hooks(DEV, 512, 512)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV)
 
