@@ -417,11 +417,13 @@ class Transformer(nn.Module):
     @torch.no_grad()
     def step(self, batch) -> torch.Tensor:
         """Run a ``serving.StepBatch`` -> float32 logits [wanted rows, vocab]."""
+        if not batch.lengths:
+            return torch.empty((0, self.vocab), dtype=torch.float32, device=self.device)
         tables = self._step_tables(batch)
         if tables is not None:
             batch = batch.tables_for(self.device)
         # (a slot that the batch names twice: its second part reads what the first one writes)
-        together = tables is not None and batch.by_sequence and len(set(batch.slots)) == len(batch.slots)
+        together = tables is not None and min(batch.lengths) > 0 and batch.by_sequence and len(set(batch.slots)) == len(batch.slots)
         embedded = []
 
         def embed():

@@ -21,6 +21,22 @@ import torch
 from . import gptfast as G
 
 
+def _numbers(values, kinds: str = "iufb") -> np.ndarray:
+    """Numbers, tensors of one element (on any device), or an array or tensor of them"""
+    if isinstance(values, torch.Tensor):
+        values = values.reshape(-1).tolist()
+    try:
+        a = np.asarray(values)
+        plain = a.ndim == 1 and a.dtype.kind != "O"
+    except (TypeError, ValueError, RuntimeError):
+        plain = False
+    if not plain:
+        a = np.asarray([int(v) for v in values], dtype=object)
+    elif a.size and a.dtype.kind not in kinds:
+        raise TypeError(f"integers expected, not {a.dtype}")
+    return a
+
+
 @dataclass
 class StepBatch:
     """Tokens of one step, packed sequence after sequence.  Device tensors are int32; ``lengths`` / ``starts`` / ``slots`` are the host's copy (one
@@ -129,7 +145,7 @@ class StepBatch:
         size = (0 if on_device else T) + 3 * T + n + 1 + (len(wanted) if wanted is not None else 0)
         cuda = torch.device(device).type == "cuda"
         host = torch.empty(size, dtype=torch.int32, device="cpu", pin_memory=cuda)
-        fill, at = host.numpy(), 0
+        fill, at = np.empty(size, dtype=np.int64), 0
 
         def put(values, count):
             nonlocal at
@@ -137,17 +153,20 @@ class StepBatch:
             at += count
 
         if not on_device:
-            for t in tokens:
-                put(t, len(t))
-        each = np.asarray(lengths)
+            for t in ([[t[0] for t in tokens]] if T == n and max(lengths, default=0) == 1 else tokens):
+                put(_numbers(t), len(t))
+        each = np.asarray(lengths, dtype=np.int64)
         ends = np.cumsum(each)
-        put(np.repeat(np.asarray(slots), each), T)
-        put(np.arange(T) + np.repeat(np.asarray(starts) - (ends - each), each), T)
+        put(np.repeat(_numbers(slots), each), T)
+        put(np.arange(T) + np.repeat(_numbers(starts, "iub") - (ends - each), each), T)
         put(np.repeat(np.arange(n), each), T)
         put(0, 1)
         put(ends, n)
         if wanted is not None:
-            put(list(wanted), len(wanted))
+            put(_numbers(wanted), len(wanted))
+        if fill.min() < -2 ** 31 or fill.max() >= 2 ** 31:     # (the assignment would wrap)
+            raise RuntimeError("value cannot be converted to type int32 without overflow")
+        host.numpy()[:] = fill
         buf = host.to(device, non_blocking=True) if cuda else host
         at = 0
 

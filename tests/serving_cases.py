@@ -269,6 +269,32 @@ def case_gptfast_hooks(dev, dim=128, inter=128):
     assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2, -3, -2]
 
 
+def case_build(dev):
+    """Ids as lists, ranges, arrays, tensors on any device and tensors of one element make the same tables; what 32 bits do not hold is refused; no sequences
+    make an empty batch, which Aria answers with no rows."""
+    import numpy as np
+
+    from aria_amd.serving import StepBatch
+
+    def tables(tokens, slots=(1, 0), starts=(3, 0), wanted=(2, 0)):
+        b = StepBatch.build(tokens, slots, starts, wanted, dev)
+        return [t.tolist() for t in (b.ids, b.slot, b.pos, b.cu, b.wanted, b.seq)]
+
+    want = [[5, 6, 9], [1, 1, 0], [3, 4, 0], [0, 2, 3], [2, 0], [0, 0, 1]]
+    t = torch.tensor([5, 6, 9], device=dev)
+    for tokens in ([[5, 6], [9]], [range(5, 7), (9,)], [np.array([5, 6]), np.array([9], dtype=np.uint8)], [t[:2], t[2:]], [[t[0], t[1]], [t[2]]], [t[:2].view(2, 1), [9]]):
+        assert tables(tokens) == want
+    assert tables([[5], [9]], wanted=t[:0]) == tables([t[:1], [t[2]]], wanted=()) and tables([[5], [9]], torch.tensor([1, 0]), np.array([3, 0])) == tables([[5], [9]])
+    for tokens, slots, starts in (([[2 ** 31]], [0], [0]), ([np.array([2 ** 40])], [0], [0]), ([torch.tensor([2 ** 40])], [0], [0]), ([[1]], [2 ** 32], [0]), ([[1]], [0], [2 ** 31])):
+        with pytest.raises((RuntimeError, OverflowError)):
+            tables(tokens, slots, starts, [0])
+    empty = StepBatch.build([], [], [], None, dev)
+    assert empty.ids.numel() == 0 and empty.cu.tolist() == [0]
+    m = gptfast_routed(dev, 128, 64, 128, 32)
+    m.setup_caches(1, 8)
+    assert m.step(empty).shape == (0, 264)
+
+
 def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

@@ -45,6 +45,10 @@ def test_gptfast_hooks():
     C.case_gptfast_hooks(DEV)
 
 
+def test_build():
+    C.case_build(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 
