@@ -147,7 +147,7 @@ Scratch layout(const int64_t* d, int64_t T, int64_t max_len, char* base) {
     z.logits = reinterpret_cast<bf16_t*>(take(2 * T * E));
     z.act = reinterpret_cast<bf16_t*>(take(2 * T * ks * I));
     z.sums = reinterpret_cast<float*>(take(4 * T * std::max(rows_parts(T, D), stream_parts(D))));
-    z.part = reinterpret_cast<float*>(take(4 * T * H * aria_decode_rows_splits(H, T, max_len) * (hd + 2)));
+    z.part = reinterpret_cast<float*>(take(4 * T * H * aria_decode_rows_splits(H, T, max_len, d[9]) * (hd + 2)));
     z.scores = reinterpret_cast<float*>(take(4 * T * k));
     z.rinv = reinterpret_cast<float*>(take(4 * T));
     z.eo = reinterpret_cast<float*>(take(4 * T * ks * D));
@@ -186,7 +186,7 @@ int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, in
     const Scratch z = layout(dims, T, max_len, static_cast<char*>(scratch));
     auto weight = [&](int64_t i) { return static_cast<const bf16_t*>(ptrs[i]); };
     const int64_t ns = Is / I;
-    const int parts = stream_parts(D), splits = aria_decode_rows_splits(H, T, max_len);
+    const int parts = stream_parts(D), splits = aria_decode_rows_splits(H, T, max_len, Smax);
     const dim3 stream_grid = dim3(unsigned(parts), unsigned(T));
     const float inv_n = 1.f / float(D);
     int sq_n = parts;   // partial sums a token has beside h

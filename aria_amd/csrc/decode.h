@@ -8,8 +8,8 @@
 
 // Splits of the keys of one head: a round of eight workgroups a CU over all heads and tokens, one pass of 128 keys at least.  Up to 256 keys one workgroup
 // of 16 waves per head is as fast and needs no merge.  8 sequences of 750 .. 3000 keys, 20 heads of 128: 5 splits 49 + 5 us, 13 splits 42 + 5 (165 MB of keys
-// and values: 3.9 TB/s).  One sequence of 600 keys: 5 splits 5.7 + 4.5 us, unsplit 12.5.
-ARIA_HIDDEN int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len);
+// and values: 3.9 TB/s).  One sequence of 600 keys: 5 splits 5.7 + 4.5 us, unsplit 12.5.  ARIA_DECODE_SPLIT_KV, where it is set, decides as for aria_decode_token.
+ARIA_HIDDEN int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len, int64_t Smax);
 // RoPE, cache write and attention of T tokens of T sequences: qkv [T, 3 H hd], caches [slots, Smax, H hd], part: T H splits (hd + 2) floats, out [T, H hd]
 ARIA_HIDDEN int aria_decode_rows_attn(const ad::bf16_t* qkv, const ad::bf16_t* freqs, const int32_t* slot, const int32_t* pos, ad::bf16_t* kc, ad::bf16_t* vc,
                                       ad::bf16_t* out, float* part, int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, void* stream);

@@ -813,6 +813,7 @@ int launch_decode_attn(void* stream, const bf16_t* qkv, const bf16_t* freqs, con
     return aria_check_launch();
 }
 
+// Splits of aria_decode_token (the steps of serving, with ARIA_DECODE_SPLIT_KV unset, by the keys that there are: aria_decode_rows_splits).
 // ARIA_DECODE_SPLIT_KV: unset / "1" = one split per 1024 cache slots (2..32) for caches beyond 2048 slots; "0" = off (one workgroup
 // per head; contexts > 16 K take the generic flash kernel); N > 1 = exactly N splits.  Measured on MI355X (profiles/r02_decode_split_kv.json):
 // whole decode step 6.04 -> 3.19 ms at S_max 4096, 15.2 -> 3.70 ms at 16 K, 39.3 -> 4.37 ms at 32 K; the attention launch alone
@@ -1007,7 +1008,8 @@ int decode_one(const OneToken& one, const Scratch& s, const int64_t* dims, float
 
 }  // namespace
 
-int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len) {
+int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len, int64_t Smax) {
+    if (std::getenv("ARIA_DECODE_SPLIT_KV")) return decode_splits_for(Smax);
     if (max_len <= 256) return 1;
     const int64_t fill = (2048 + H * T - 1) / (H * T), passes = (max_len + 127) / 128;
     return int(std::max<int64_t>(1, std::min<int64_t>(std::min(fill, passes), DECODE_MAX_SPLITS)));
@@ -1024,7 +1026,7 @@ int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, con
                     float* logits, char* scratch, void* stream) {
     const Scratch s = carve(scratch, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
     const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]), static_cast<const bf16_t*>(x),
-                       ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len)};
+                       ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len, dims[9])};
     return decode_one(one, s, dims, eps, stream);
 }
 

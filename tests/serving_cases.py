@@ -295,6 +295,45 @@ def case_build(dev):
     assert m.step(empty).shape == (0, 264)
 
 
+def case_decode_splits(dev, monkeypatch, run=True):
+    """ARIA_DECODE_SPLIT_KV decides over the splits of serving steps as over the decode engine's (seen in the scratch that they ask for); the logits stay those of
+    the step's own choice (another order of sums: ``case_gptfast_decode_batch``)."""
+    import ctypes
+
+    import numpy as np
+
+    from aria_amd import hip
+    from aria_amd.serving import StepBatch
+
+    def scratch(T, slots):
+        dims = np.array([2, 2560, 20, 128, 64, 6, 1664, 3328, 1000, slots], dtype=np.int64)
+        return int(hip.get_lib().cdll.aria_decode_step_scratch(dims.ctypes.data_as(ctypes.c_void_p), T, slots - 8))
+
+    one = 4 * 8 * 20 * 130       # floats of one split: 8 tokens, 20 heads
+    monkeypatch.setenv("ARIA_DECODE_SPLIT_KV", "0")
+    none = scratch(8, 4096)
+    for value, slots, splits in (("1", 4096, 4), ("7", 4096, 7), ("99", 4096, 32), ("7", 2048, 1)):
+        monkeypatch.setenv("ARIA_DECODE_SPLIT_KV", value)
+        assert scratch(8, slots) - none == (splits - 1) * one, value
+    if not run:
+        return
+    m = gptfast_routed(dev, 128, 64, 128, 2600)
+    m.setup_caches(3, 2600)
+    for b in m.layers:
+        for c in (b.attention.kv_cache.k, b.attention.kv_cache.v):
+            c.copy_(torch.randn(c.shape, generator=L.gen(1)))
+
+    def step(n):
+        return m.step(StepBatch.build([[5], [9], [77]][:n], list(range(n)), [2590, 3, 1500][:n], None, dev))
+
+    monkeypatch.delenv("ARIA_DECODE_SPLIT_KV")
+    want = [step(n).cpu().double() for n in (1, 3)]
+    for value in "0", "1", "5":
+        monkeypatch.setenv("ARIA_DECODE_SPLIT_KV", value)
+        for n, w in zip((1, 3), want):
+            assert L.logit_err(step(n), w) < 4 * 2 ** -8, value
+
+
 def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

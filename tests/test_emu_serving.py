@@ -49,6 +49,10 @@ def test_build():
     C.case_build(DEV)
 
 
+def test_decode_splits(monkeypatch):
+    C.case_decode_splits(DEV, monkeypatch, run=False)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 

@@ -59,6 +59,10 @@ def test_build():
     C.case_build(DEV)
 
 
+def test_decode_splits(monkeypatch):
+    C.case_decode_splits(DEV, monkeypatch)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV)
 
