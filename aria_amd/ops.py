@@ -158,13 +158,18 @@ _WORKSPACES = {}
 GEMM_SPLIT_K = True  # tools flip this off to compare kernels bit for bit (split-K changes the fp32 summation order)
 
 
+WORKSPACE_KEPT = 64 << 20   # bytes kept per (device, stream): one round of 256 slabs
+
+
 def _gemm_workspace(device, stream, nbytes: int) -> torch.Tensor:
-    """Grow-only scratch buffer per (device, stream): launches on one stream are ordered, so they can share it."""
+    """Scratch buffer kept per (device, stream): launches on one stream are ordered, so they can share it.  A larger one is the call's own: the allocator has
+    it back afterwards, and the kept buffer never moves under a captured graph."""
+    if nbytes > WORKSPACE_KEPT:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     key = (str(device), int(stream or 0))
     ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 64 << 20), dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = ws
+    if ws is None:
+        ws = _WORKSPACES[key] = torch.empty(WORKSPACE_KEPT, dtype=torch.uint8, device=device)
     return ws
 
 

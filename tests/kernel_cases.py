@@ -114,6 +114,30 @@ def case_gemm_split_k_slabs(dev, M, N, K, a_oc, b_oc):
     assert torch.equal(acc.cpu(), (ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias.to(dev), out_dtype=torch.float32).cpu() + old.float()).to(bf16))
 
 
+def case_gemm_workspace_kept(dev):
+    """What is kept per stream is one buffer of a fixed size; a larger need is the call's own and leaves nothing behind."""
+    from aria_amd import ops
+
+    kept = ops._gemm_workspace(torch.device(dev), 0, 1 << 20)
+    large = ops._gemm_workspace(torch.device(dev), 0, ops.WORKSPACE_KEPT + 256)
+    assert large.numel() == ops.WORKSPACE_KEPT + 256 and kept.numel() == ops.WORKSPACE_KEPT
+    assert ops._gemm_workspace(torch.device(dev), 0, ops.WORKSPACE_KEPT).data_ptr() == kept.data_ptr()
+    assert all(w.numel() == ops.WORKSPACE_KEPT for w in ops._WORKSPACES.values())
+
+
+def case_gemm_tile_rule(dev, tiles, K, variant):
+    """A dense product on both sides of the fewest 256 x 256 tiles and the shortest reduction that the large tiles take in a partly filled round, with a ragged last
+    row tile: 32-bit sums of K products of bf16 (error at most K 2^-24 of the sum of magnitudes, here 2e-6 of the result's norm)."""
+    from aria_amd import hip, ops
+
+    M, N = 256 * tiles - 3, 256
+    a, w = rnd(M, K, seed=tiles), rnd(N, K, seed=K)
+    got = ops.gemm(a.to(dev), w.to(dev), out_dtype=torch.float32).cpu()
+    assert hip.get_lib().cdll.aria_last_gemm_variant() == variant
+    want = a.double() @ w.double().T
+    assert float((got.double() - want).norm() / want.norm()) < 2e-6
+
+
 def case_unpermute_with_residual(dev, T, D, k, E=8):
     """r05b: the decoder layer's residual add as the last step of the un-permute launch (aria_moe_unpermute_res) == aria_moe_unpermute +
     aria_add_bf16, bit for bit (bf16(h + bf16(combine + shared))), with and without scores / shared rows; widths without a compile-time kernel

@@ -181,6 +181,10 @@ def test_gemm_v3_split_k_skinny_outputs(M, N, a_oc, b_oc):
     assert lib.aria_last_gemm_variant() == 3
 
 
+def test_gemm_workspace_kept():
+    C.case_gemm_workspace_kept(DEV)
+
+
 @pytest.mark.parametrize("counts", [[3, 0, 130, 5, 0, 0, 300, 1], [1, 1, 1]])
 def test_grouped_gemm_v3(force_gemm_v3, counts):
     from aria_amd import hip
