@@ -197,6 +197,27 @@ def test_gemm_v3_split_k(a_oc, b_oc):
     assert torch.allclose(got, ref, rtol=1e-4, atol=1e-2)
 
 
+def test_gemm_workspace_kept():
+    C.case_gemm_workspace_kept(DEV)
+
+
+@pytest.mark.parametrize("a_oc,b_oc", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(200, 300, 16384), (64, 2560, 8192), (2300, 520, 12296)])
+def test_gemm_split_into_many_pieces(M, N, K, a_oc, b_oc):
+    """A few tiles with a long reduction: more than eight pieces."""
+    from aria_amd import hip
+
+    tiles = -(-M // 256) * -(-N // 256)
+    assert hip.get_lib().cdll.aria_gemm_workspace_bytes(M, N, K, int(a_oc), int(b_oc)) > 8 * tiles * 4 * 256 * 256
+    C.case_gemm_split_k_slabs(DEV, M, N, K, a_oc, b_oc)
+    assert hip.get_lib().cdll.aria_last_gemm_variant() == 3
+
+
+@pytest.mark.parametrize("tiles,K,variant", [(79, 512, 1), (80, 512, 3), (80, 504, 1), (191, 504, 1), (191, 512, 3), (192, 504, 3)])
+def test_gemm_tile_rule(tiles, K, variant):
+    C.case_gemm_tile_rule(DEV, tiles, K, variant)
+
+
 @pytest.mark.parametrize("counts,K,I,T", [([300, 0, 70, 5, 0, 0, 260, 1], 128, 128, 300), ([1536] * 8 + [1500, 1580], 2560, 1664, 4096)])
 def test_gemm_swiglu_fused(counts, K, I, T):
     C.case_gemm_swiglu_fused(DEV, counts, K, I, T)
