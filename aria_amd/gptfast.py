@@ -290,7 +290,7 @@ class Transformer(nn.Module):
         self._tables: Optional["_StepTables"] = None
         # bumped by whatever may re-home a weight (module.to / .cuda / casts; load_state_dict, also through a parent module, also assign=True):
         # the decode engine re-checks its whole pointer table only then
-        self._weights_version = 0
+        self._weights_version, self._paired_version = 0, -1
         self.register_load_state_dict_post_hook(lambda module, incompatible: module._bump_weights_version())
 
     def _bump_weights_version(self):
@@ -435,12 +435,17 @@ class Transformer(nn.Module):
             logits = tables.run(embed(), batch.slot, batch.pos, batch.max_len)
             if logits is not None:
                 return logits if batch.every_row else logits[batch.wanted.long()]
-        if together and batch.fresh and batch.longest > 1 and self.freqs_cis.shape[0] >= self.max_seq_length and not tables.watched(self):
-            logits = tables.prompts(batch, embed) if batch.n_wanted <= batch.ids.numel() else None
-            if logits is not None:
-                return logits
-            if self._packs(batch) and embed() is not None:
-                return self._prompts(batch, embed())
+        prompts = together and batch.fresh and batch.longest > 1 and not tables.watched(self)
+        logits = tables.prompts(batch, embed) if prompts and batch.n_wanted <= batch.ids.numel() else None
+        # Every tensor is compared with the tables beside the device's work (20 us a layer of host time in front of it otherwise).  The tables keep what they
+        # point to: where something was exchanged, the step on the old tensors has done no harm and is run again on the new ones.
+        if tables is not None and batch.longest > 1 and not tables.current(self):
+            tables = self._tables = _StepTables(self)
+            logits = tables.prompts(batch, embed) if logits is not None else None
+        if logits is not None:
+            return logits
+        if prompts and self._packs(batch) and embed() is not None:
+            return self._prompts(batch, embed())
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:
@@ -479,6 +484,7 @@ class Transformer(nn.Module):
 
 def _pair_weights(model: "Transformer") -> None:
     """Gate / up pairs into one allocation each before anybody records parameter addresses: the layers, which pair lazily, then find nothing to move."""
+    model._paired_version = model._weights_version
     for b in model.layers:
         ff = b.feed_forward
         _glu_pair_ready(ff.cond_ffn.w1, ff.cond_ffn.w3)
@@ -487,15 +493,18 @@ def _pair_weights(model: "Transformer") -> None:
 
 def _own_layers(model: "Transformer") -> bool:
     """Layers of other classes run as modules: the library knows nothing of what they compute."""
-    return all(type(b) is TransformerBlock and type(b.attention) is Attention and type(b.feed_forward) is MOEFeedForward and
-               type(b.attention_norm) is type(b.ffn_norm) is RMSNorm for b in model.layers)
+    for b in model._modules["layers"]._modules.values():
+        parts = b._modules
+        if not (type(b) is TransformerBlock and type(parts["attention"]) is Attention and type(parts["feed_forward"]) is MOEFeedForward and
+                type(parts["attention_norm"]) is type(parts["ffn_norm"]) is RMSNorm):
+            return False
+    return True
 
 
 class _StepTables:
-    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches.  Every step compares them with the tensors that the model
-    holds then (assigned, moved or replaced weights and modules: about 0.1 us a tensor, beside a device that is busy with the step before), and
-    the tables keep the storage alive that they point to.  The scratch is a step's own: steps of other streams never share it, and the allocator
-    knows whose stream it was used on."""
+    """Pointer and size tables of ``aria_decode_step`` for a model's weights and whole caches, which keep the storage alive that they point to: re-made when
+    weights are loaded or converted or the caches set up, and with a prompt when any tensor was exchanged.  The scratch is a step's own: steps of
+    other streams never share it, and the allocator knows whose stream it was used on."""
 
     def __init__(self, model: "Transformer"):
         import ctypes
@@ -503,52 +512,62 @@ class _StepTables:
         import numpy as np
 
         c = model.config
-        self.modules, self.served = [], False
+        self.served = False
         if not _own_layers(model):
             return
-        _pair_weights(model)
+        if model._paired_version != model._weights_version:     # (loaded or converted since the caches were set up)
+            _pair_weights(model)
         self.key, self.eps = DecodeEngine._cheap_key(model), float(c.norm_eps)
         self.dims = np.array([c.n_layer, c.dim, c.n_head, c.head_dim, c.num_experts, c.router_topk, c.intermediate_size,
                               c.intermediate_size * c.num_shared_experts, c.vocab_size, model.max_seq_length], dtype=np.int64)
         self.dims_p = self.dims.ctypes.data_as(ctypes.c_void_p)
-        tensors = [model.freqs_cis, model.norm.weight, model.output.weight] + _layer_table(model)
+        tensors, device = self._tensors(model), model.device
         self.tensors = [t.detach() for t in tensors]      # (a parameter's storage may be exchanged, a detached tensor's not)
-        D, I, Is, E, cache = c.dim, c.intermediate_size, c.intermediate_size * c.num_shared_experts, c.num_experts, tuple(model.layers[0].attention.kv_cache.k.shape)
+        D, I, Is, E = c.dim, c.intermediate_size, c.intermediate_size * c.num_shared_experts, c.num_experts
+        cache = (tensors[-1].shape[0], model.max_seq_length, D)
         layer = [(D,), (3 * D, D), (D, D), (D,), (E, D), (E, I, D), (E, I, D), (E, D, I), (Is, D), (Is, D), (D, Is), cache, cache]
-        shapes = [(model.freqs_cis.shape[0], c.head_dim // 2, 2), (D,), (c.vocab_size, D)] + layer * c.n_layer
-        self.served = (all(t.is_contiguous() and t.dtype == bf16 and t.device == model.device for t in tensors) and [tuple(t.shape) for t in tensors] == shapes
-                       and cache[1:] == (model.max_seq_length, D) and model.freqs_cis.shape[0] >= model.max_seq_length)
-        self.ptrs = (ctypes.c_void_p * len(tensors))(*(t.data_ptr() for t in tensors))
-        # ways to the weights: (modules of the parent, name, module), (parameters of the module, name); addresses and sizes of these
-        self.ways, seen = [], set()
-        for path in [("norm", "weight"), ("output", "weight")] + [("layers", str(i)) + w for i in range(c.n_layer) for w in _LAYER_WEIGHTS]:
-            at = model
-            for name in path[:-1]:
-                parent, at = at, at._modules[name]
-                if (id(parent), name) not in seen:
-                    seen.add((id(parent), name))
-                    self.modules.append((parent._modules, name, at))
-            self.ways.append((at._parameters, path[-1]))
-        weights = [of.get(name) for of, name in self.ways]
-        self.served = self.served and all(t is not None for t in weights)       # (one that is computed from other parameters has no address of its own)
-        if self.served:
-            self.where, self.sizes = [t.data_ptr() for t in weights], [t.numel() for t in weights]
+        self.shapes = [(tensors[0].shape[0], c.head_dim // 2, 2), (D,), (c.vocab_size, D)] + layer * c.n_layer
+        self.served = (all(t.is_contiguous() and t.dtype == bf16 and t.device == device for t in tensors) and [t.shape for t in tensors] == self.shapes
+                       and self.shapes[0][0] >= model.max_seq_length)
+        self.version, self.where = model._weights_version, [t.data_ptr() for t in tensors]
+        self.ptrs = (ctypes.c_void_p * len(tensors))(*self.where)
+
+    @staticmethod
+    def _tensors(model: "Transformer") -> List[torch.Tensor]:
+        return [model.freqs_cis, model._modules["norm"].weight, model._modules["output"].weight] + _layer_table(model)
 
     def valid_for(self, model: "Transformer") -> bool:
+        """By what moves in the usual ways: weights loaded or converted (the model's version), caches set up anew."""
         if not self.served or DecodeEngine._cheap_key(model) != self.key:      # (tensors that the library does not take: looked at again with every step)
             return False
-        if [None for of, name, module in self.modules if of.get(name) is not module]:
+        if self.version != model._weights_version:
+            if not self.current(model):
+                return False
+            self.version = model._weights_version
+        return True
+
+    def current(self, model: "Transformer") -> bool:
+        """By every tensor that the model holds now: exchanged parameters and modules too."""
+        if not self.served:
+            return True
+        try:
+            tensors = self._tensors(model)
+        except (AttributeError, KeyError):       # (modules of other classes)
             return False
-        weights = [of.get(name) for of, name in self.ways]
-        return (not [None for t in weights if t is None] and list(map(torch.Tensor.data_ptr, weights)) == self.where and list(map(torch.Tensor.numel, weights)) == self.sizes
-                and all(map(torch.Tensor.is_contiguous, weights)))
+        return [t.data_ptr() for t in tensors] == self.where and [t.shape for t in tensors] == self.shapes and all(t.is_contiguous() for t in tensors)
 
     def watched(self, model: "Transformer") -> bool:
         """Somebody looks at or changes what the model's modules do with a prompt (forward hooks, other forwards): it then runs module by module.  (Single
         tokens have never done that on the decode engine.)"""
         everywhere = nn.modules.module
-        return not _own_layers(model) or bool(everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks or
-                                              [None for _, _, m in self.modules if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__])
+        if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks or not _own_layers(model):
+            return True
+        for b in model._modules["layers"]._modules.values():
+            parts = b._modules
+            for m in (b, parts["attention"], parts["feed_forward"], parts["attention_norm"]):
+                if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                    return True
+        return False
 
     def run(self, x, slot, pos, max_len: int) -> Optional[torch.Tensor]:
         """embedding rows x [T, D] -> logits float32 [T, vocab]; None: sizes that the library does not serve in one call"""
@@ -579,22 +598,15 @@ class _StepTables:
         return logits
 
 
-# a layer's weights in the order of the decode engine's pointer tables (the caches behind them)
-_LAYER_WEIGHTS = (("attention_norm", "weight"), ("attention", "wqkv", "weight"), ("attention", "wo", "weight"), ("ffn_norm", "weight"),
-                  ("feed_forward", "gate", "weight"), ("feed_forward", "cond_ffn", "w1"), ("feed_forward", "cond_ffn", "w3"), ("feed_forward", "cond_ffn", "w2"),
-                  ("feed_forward", "shared_ffn", "w1", "weight"), ("feed_forward", "shared_ffn", "w3", "weight"), ("feed_forward", "shared_ffn", "w2", "weight"))
-
-
 def _layer_table(model: "Transformer") -> List[torch.Tensor]:
     """the tensors of every layer in the order of the decode engine's pointer tables"""
     out = []
-    for blk in model.layers:
-        for path in _LAYER_WEIGHTS:
-            t = blk
-            for name in path:
-                t = getattr(t, name)
-            out.append(t)
-        out += [blk.attention.kv_cache.k, blk.attention.kv_cache.v]
+    for blk in model._modules["layers"]._modules.values():
+        at = blk._modules
+        a, f = at["attention"]._modules, at["feed_forward"]._modules
+        cond, shared, cache = f["cond_ffn"], f["shared_ffn"]._modules, at["attention"].kv_cache
+        out += [at["attention_norm"].weight, a["wqkv"].weight, a["wo"].weight, at["ffn_norm"].weight, f["gate"].weight, cond.w1, cond.w3, cond.w2,
+                shared["w1"].weight, shared["w3"].weight, shared["w2"].weight, cache.k, cache.v]
     return out
 
 

@@ -266,7 +266,9 @@ def case_gptfast_hooks(dev, dim=128, inter=128):
             return super().forward(x)
 
     block.feed_forward.__class__ = Other
-    assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2, -3, -2]
+    for again in (1, 2):      # (on tables that were made before, and on new ones)
+        assert L.logit_err(prompt(), want) < 4 * 2 ** -8 and seen == [3, 2] + [-3, -2] * again
+        m._tables = None
 
 
 def case_build(dev):
