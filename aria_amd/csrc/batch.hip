@@ -180,8 +180,7 @@ int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, in
     if (need == 0) return ARIA_ERR_UNSUPPORTED;
     const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8], Smax = dims[9];
     if (scratch_bytes < need || max_len > Smax) return ARIA_ERR_INVALID;
-    for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
-        if (!ptrs[i]) return ARIA_ERR_INVALID;
+    if (const int bad = aria_decode_table_ok(ptrs, L)) return bad;
     if (T == 1) return aria_decode_one(ptrs, dims, eps, x, slot, pos, max_len, logits, static_cast<char*>(scratch), stream);
     const Scratch z = layout(dims, T, max_len, static_cast<char*>(scratch));
     auto weight = [&](int64_t i) { return static_cast<const bf16_t*>(ptrs[i]); };

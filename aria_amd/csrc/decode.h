@@ -16,6 +16,8 @@ ARIA_HIDDEN int aria_decode_rows_attn(const ad::bf16_t* qkv, const ad::bf16_t* f
 ARIA_HIDDEN int aria_route_and_sort(const ad::bf16_t* logits, ad::bf16_t* scores, int32_t* idx, int32_t* counts, int32_t* offsets, int32_t* src, int32_t* inv,
                                     int32_t* rows, int T, int E, int k, void* stream);
 ARIA_HIDDEN int aria_decode_dims_ok(const int64_t* dims);
+// ARIA_OK where every tensor of a step's table is there and starts at 16 bytes
+ARIA_HIDDEN int aria_decode_table_ok(const void* const* ptrs, int64_t layers);
 // One sequence's step by the engine's kernels
 ARIA_HIDDEN int64_t aria_decode_one_scratch(const int64_t* dims);
 ARIA_HIDDEN int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, const void* x, const int32_t* slot, const int32_t* pos,

@@ -1019,6 +1019,14 @@ int aria_decode_rows_attn(const bf16_t* qkv, const bf16_t* freqs, const int32_t*
     return launch_decode_attn(stream, qkv, freqs, pos, kc, vc, out, part, H, hd, H * hd, splits, T, slot, Smax * H * hd);
 }
 int aria_decode_dims_ok(const int64_t* dims) { return dims_ok(dims); }
+int aria_decode_table_ok(const void* const* ptrs, int64_t layers) {
+    uintptr_t low = 0;
+    for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * layers; ++i) {
+        if (!ptrs[i]) return ARIA_ERR_INVALID;
+        low |= reinterpret_cast<uintptr_t>(ptrs[i]);
+    }
+    return low & 15 ? ARIA_ERR_ALIGN : ARIA_OK;
+}
 int64_t aria_decode_one_scratch(const int64_t* dims) {
     return int64_t(carve(nullptr, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]).bytes);
 }

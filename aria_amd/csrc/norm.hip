@@ -622,7 +622,8 @@ int aria_rope_interleaved_inplace(void* x, const void* freqs_cis, const int32_t*
 int aria_rope_cache_rows(void* qkv, const void* freqs_cis, const int32_t* slot, const int32_t* pos, void* k_cache, void* v_cache, int64_t T, int64_t H, int64_t hd,
                          int64_t S_max, void* stream) {
     if (!qkv || !freqs_cis || !slot || !pos || !k_cache || !v_cache || T < 0 || H <= 0 || hd <= 0 || S_max <= 0) return ARIA_ERR_INVALID;
-    if (hd & 7) return ARIA_ERR_ALIGN;
+    if ((hd & 7) || ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(freqs_cis) | reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15))
+        return ARIA_ERR_ALIGN;
     if (T == 0) return ARIA_OK;
     const int64_t nch = H * hd / 8;
     const long long nitems = T * 3 * nch;

@@ -59,8 +59,7 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
     if (need == 0) return ARIA_ERR_UNSUPPORTED;
     const int64_t L = dims[0], D = dims[1], H = dims[2], hd = dims[3], E = dims[4], k = dims[5], I = dims[6], Is = dims[7], V = dims[8], Smax = dims[9];
     if (scratch_bytes < need || longest > Smax || n_wanted > T) return ARIA_ERR_INVALID;
-    for (int64_t i = 0; i < ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * L; ++i)
-        if (!ptrs[i]) return ARIA_ERR_INVALID;
+    if (const int bad = aria_decode_table_ok(ptrs, L)) return bad;
     const Scratch z = layout(dims, T, static_cast<char*>(scratch));
     ARIA_LAUNCH(clear_counts_kernel, dim3(unsigned((L * E + 255) / 256)), dim3(256), 0, stream, z.counts, int(L * E));
     int rc = aria_check_launch();

@@ -530,6 +530,7 @@ class _StepTables:
         self.served = (all(t.is_contiguous() and t.dtype == bf16 and t.device == device for t in tensors) and [t.shape for t in tensors] == self.shapes
                        and self.shapes[0][0] >= model.max_seq_length)
         self.version, self.where = model._weights_version, [t.data_ptr() for t in tensors]
+        self.served = self.served and not any(p % 16 for p in self.where)
         self.ptrs = (ctypes.c_void_p * len(tensors))(*self.where)
 
     @staticmethod

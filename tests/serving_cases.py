@@ -336,6 +336,28 @@ def case_decode_splits(dev, monkeypatch, run=True):
             assert L.logit_err(step(n), w) < 4 * 2 ** -8, value
 
 
+def case_alignment(dev):
+    """Tensors that do not start at 16 bytes are refused in front of every launch, as the tile products refuse them."""
+    from aria_amd import gptfast as G
+    from aria_amd import hip, ops
+    from aria_amd.serving import Scheduler
+
+    def off(t):
+        return torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+
+    T, H, hd, S = 3, 2, 64, 8
+    slot, pos = torch.zeros(T, dtype=torch.int32, device=dev), torch.arange(T, dtype=torch.int32, device=dev)
+    tensors = [L.rnd(T, 3 * H * hd, seed=1).to(dev), G.precompute_freqs_cis(S, hd).to(dev), L.rnd(1, S, H * hd, seed=2).to(dev), L.rnd(1, S, H * hd, seed=3).to(dev)]
+    for bad in range(4):
+        qkv, fc, k, v = (off(t) if i == bad else t for i, t in enumerate(tensors))
+        with pytest.raises(hip.AriaHipError):
+            ops.rope_cache_rows_(qkv, fc, slot, pos, k, v, H, hd)
+    m = gptfast_routed(dev, 128, 64, 128, 32)
+    m.layers[1].attention.wo.weight.data = off(m.layers[1].attention.wo.weight.data)
+    with pytest.raises(hip.AriaHipError):
+        Scheduler(m, 8).step("ab", [[5, 9], [5, 3, 7]])
+
+
 def case_gptfast_portion_order(dev, engine=False):
     """A portion of a prompt: logits in the order in which its places are named."""
     from aria_amd.serving import Scheduler

@@ -53,6 +53,10 @@ def test_decode_splits(monkeypatch):
     C.case_decode_splits(DEV, monkeypatch, run=False)
 
 
+def test_alignment():
+    C.case_alignment(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 

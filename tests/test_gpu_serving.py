@@ -63,6 +63,10 @@ def test_decode_splits(monkeypatch):
     C.case_decode_splits(DEV, monkeypatch)
 
 
+def test_alignment():
+    C.case_alignment(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV)
 
