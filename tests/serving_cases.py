@@ -26,8 +26,9 @@ def gptfast_toy(dev, head_dim=64):
 
 
 def case_gptfast_batch(dev, engine=True):
-    """Unequal requests of one batch give each request's own logits bit for bit (its sequence runs by itself on its slot), with the decode engine and
-    with the tile path; the tile path also equals one prefill of the whole prefix.  Slots are used again by a second batch."""
+    """At sizes that no one-call step serves, unequal requests of one batch give each request's own logits bit for bit (its sequence runs by itself on its slot),
+    with the decode engine and with the tile path; the tile path also equals one prefill of the whole prefix.  Slots are used again by a second
+    batch."""
     from aria_amd.serving import Scheduler
 
     m = gptfast_toy(dev)
@@ -429,6 +430,84 @@ def case_rows_qkv(dev, M, D, hd, S):
         q = ops.rows_qkv_rope_cache(x, w, fc, k, v, hd, **where)
         qkv = ops.rope_cache_rows_(ops.rows_gemm(x, w), fc, slot.to(dev), pos.to(dev), k2, v2, D // hd, hd)
         assert torch.equal(q, qkv[:, :D]) and torch.equal(k, k2) and torch.equal(v, v2)
+
+
+def gptfast_oracle(m, toks, r=lambda t: t):
+    """A whole sequence through a gptfast decoder in float64, in plain torch: (logits [n, vocab], [(rotated keys, values) of a layer, [n, dim] each]).  ``r`` is
+    applied to what the kernels keep in 16 bits."""
+    c, n = m.config, len(toks)
+    w = {name: p.detach().double() for name, p in m.named_parameters()}
+    dev, D, H, hd = m.device, c.dim, c.n_head, c.head_dim
+    angle = torch.arange(n, dtype=torch.float64, device=dev)[:, None] * c.rope_base ** (-torch.arange(0, hd, 2, dtype=torch.float64, device=dev) / hd)
+    cos, sin = r(angle.cos())[:, None], r(angle.sin())[:, None]
+    future = torch.ones(n, n, dtype=torch.bool, device=dev).triu(1)
+
+    def norm(x, name):
+        return r(x * (x.pow(2).mean(-1, keepdim=True) + c.norm_eps).rsqrt() * w[name + ".weight"])
+
+    def rotate(x):
+        a, b = x.view(n, H, hd // 2, 2).unbind(-1)
+        return r(torch.stack([a * cos - b * sin, b * cos + a * sin], -1).view(n, D))
+
+    def glu(h, up, gate, down):      # (w1 goes through silu)
+        return r(r(torch.nn.functional.silu(r(h @ up.T)) * r(h @ gate.T)) @ down.T)
+
+    x, cache = w["tok_embeddings.weight"][torch.as_tensor(toks, device=dev)], []
+    for i in range(c.n_layer):
+        p = f"layers.{i}."
+        q, k, v = r(norm(x, p + "attention_norm") @ w[p + "attention.wqkv.weight"].T).split(D, -1)
+        q, k = rotate(q), rotate(k)
+        cache.append((k, v))
+        heads = [t.view(n, H, hd).transpose(0, 1).contiguous() for t in (q, k, v)]
+        prob = (heads[0] @ heads[1].mT.contiguous() * hd ** -0.5).masked_fill(future, -float("inf")).softmax(-1)
+        x = r(x + r(r((prob @ heads[2]).transpose(0, 1).reshape(n, D)) @ w[p + "attention.wo.weight"].T))
+        h, f = norm(x, p + "ffn_norm"), p + "feed_forward."
+        top, chosen = r(h @ w[f + "gate.weight"].T).topk(c.router_topk, -1)
+        score, routed = r(top.softmax(-1)), torch.zeros_like(x)
+        for e in range(c.num_experts):
+            t, place = (chosen == e).nonzero(as_tuple=True)
+            if len(t):
+                routed[t] += score[t, place, None] * glu(h[t], *(w[f + "cond_ffn." + name][e] for name in ("w1", "w3", "w2")))
+        shared = glu(h, *(w[f + f"shared_ffn.{name}.weight"] for name in ("w1", "w3", "w2")))
+        x = r(x + r(r(routed) + shared))
+    return norm(x, "norm") @ w["output.weight"].T, cache
+
+
+def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2):
+    """Prompts of several requests, tokens of all of them and a token of one against float64: logits and cache rows, each step seen to be one library call.  Bound:
+    three times what 16-bit tensors between exact operations make of the same sequence."""
+    from aria_amd import gptfast as G
+    from aria_amd.serving import Scheduler
+
+    m, served = gptfast_routed(dev, dim, 64, inter, max(lens) + 8), []
+    for name in ("prompts", "run"):
+        def seen(self, *a, plain=getattr(G._StepTables, name), name=name):
+            out = plain(self, *a)
+            served.append((name, out is not None))
+            return out
+        monkeypatch.setattr(G._StepTables, name, seen)
+    toks = [torch.randint(0, 264, (n + steps,), generator=L.gen(n)).tolist() for n in lens]
+    exact = [gptfast_oracle(m, t) for t in toks]
+    rounded = [gptfast_oracle(m, t, lambda x: x.to(bf16).double()) for t in toks]
+    tol = 3 * max(L.logit_err(b[0], a[0].cpu()) for a, b in zip(exact, rounded))
+    # a row of keys or values of one head, the worst one
+    rows = [[t.reshape(-1, 64) for a in one for pair in a[1] for t in pair] for one in (exact, rounded)]
+    cache_tol = 3 * max(L.logit_err(b, a.cpu()) for a, b in zip(*rows))
+    assert tol < 0.06 and cache_tol < 0.12, (tol, cache_tol)      # (far below what a step that leaves something out gives, about 1)
+    sched, ids = Scheduler(m, max(lens) + steps + 1), list(range(len(lens)))
+    got = sched.step(ids, [t[:n] for t, n in zip(toks, lens)], [list(range(n)) for n in lens])
+    assert L.logit_err(got, torch.cat([x[0][:n] for x, n in zip(exact, lens)]).cpu()) < tol
+    for s in range(steps):
+        who = ids[::-1] if s == 0 else ids[:1]
+        got = sched.step(who, [[toks[i][lens[i] + s]] for i in who])
+        assert L.logit_err(got, torch.stack([exact[i][0][lens[i] + s] for i in who]).cpu()) < tol
+    for i in ids:
+        n = lens[i] + (steps if i == 0 else 1)
+        for layer, pair in enumerate(exact[i][1]):
+            kv = m.layers[layer].attention.kv_cache
+            for got, want in zip((kv.k, kv.v), pair):
+                assert L.logit_err(got[sched.live[i][0], :n].reshape(-1, 64), want[:n].reshape(-1, 64).cpu()) < cache_tol
+    assert served == [("prompts", True)] + [("run", True)] * steps
 
 
 def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17), inter=128):

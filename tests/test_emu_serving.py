@@ -74,6 +74,10 @@ def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV, 128, (5, 1, 9))
 
 
+def test_gptfast_steps_oracle(monkeypatch):
+    C.case_gptfast_steps_oracle(DEV, monkeypatch, 512, 512, (3, 1, 5))
+
+
 def test_gptfast_batch():
     C.case_gptfast_batch(DEV, engine=False)   # (the engine's emulated form takes a minute: on hardware only)
 

@@ -86,6 +86,11 @@ def test_gptfast_packed_prompts_in_one_call(dim, inter, lens):
     C.case_gptfast_packed_prompts(DEV, dim, lens, inter)
 
 
+@pytest.mark.parametrize("dim,inter,lens", [(512, 512, (9, 1, 20, 7)), (1024, 1664, (20,)), (2560, 1664, (33, 30, 8)), (2560, 1664, (140, 1))])
+def test_gptfast_steps_oracle(monkeypatch, dim, inter, lens):
+    C.case_gptfast_steps_oracle(DEV, monkeypatch, dim, inter, lens)
+
+
 def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV)
     C.case_gptfast_packed_prompts(DEV, 1024, (300, 64, 65, 2, 129))
