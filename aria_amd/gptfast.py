@@ -294,11 +294,11 @@ class Transformer(nn.Module):
         self.register_load_state_dict_post_hook(lambda module, incompatible: module._bump_weights_version())
 
     def _bump_weights_version(self):
-        self._weights_version += 1
-
-    def _apply(self, fn, *a, **k):
         self._weights_version = getattr(self, "_weights_version", 0) + 1
         self._tables = None      # (they keep the storage that is given up here)
+
+    def _apply(self, fn, *a, **k):
+        self._bump_weights_version()
         return super()._apply(fn, *a, **k)
 
     def _engine_capable(self) -> bool:
@@ -539,13 +539,8 @@ class _StepTables:
 
     def valid_for(self, model: "Transformer") -> bool:
         """By what moves in the usual ways: weights loaded or converted (the model's version), caches set up anew."""
-        if not self.served or DecodeEngine._cheap_key(model) != self.key:      # (tensors that the library does not take: looked at again with every step)
-            return False
-        if self.version != model._weights_version:
-            if not self.current(model):
-                return False
-            self.version = model._weights_version
-        return True
+        # (tensors that the library does not take: looked at again with every step)
+        return self.served and self.version == model._weights_version and DecodeEngine._cheap_key(model) == self.key
 
     def current(self, model: "Transformer") -> bool:
         """By every tensor that the model holds now: exchanged parameters and modules too."""

@@ -161,6 +161,19 @@ def case_gptfast_moved_weights(dev, names=("assign", "parameter", "data", "modul
         sched.step(["a", "b"], prompts)
 
 
+def case_gptfast_weights_given_up(dev):
+    """A step's tables keep no weights alive that a load has replaced."""
+    import weakref
+
+    from aria_amd.serving import Scheduler
+
+    m = gptfast_routed(dev, 128, 64, 128, 32)
+    Scheduler(m, 8).step("ab", [[5], [9]])
+    kept = [weakref.ref(t) for t in m._tables.tensors]
+    m.load_state_dict({k: v.clone() for k, v in m.state_dict().items()}, assign=True)
+    assert kept and not any(r() is not None for r in kept)
+
+
 def toy(design, dev):
     """A small decoder whose steps of several requests are one call."""
     if design == "gptfast":

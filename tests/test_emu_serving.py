@@ -57,6 +57,10 @@ def test_alignment():
     C.case_alignment(DEV)
 
 
+def test_gptfast_weights_given_up():
+    C.case_gptfast_weights_given_up(DEV)
+
+
 def test_gptfast_moved_weights():
     C.case_gptfast_moved_weights(DEV, ("assign", "module"))
 
