@@ -1,6 +1,7 @@
-// A serving step over short prompts of the gptfast (Aria) decoder in one call: packed tokens of one or several sequences, every product by the row-streaming
-// kernels of wide.hip.  At these sizes a layer is fifteen launches of 5 .. 230 us; enqueued one by one from Python they take longer than they run (four
-// layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
+// A serving step over short prompts of the gptfast (Aria) decoder in one call: packed tokens of one or several sequences, the products by the row-streaming kernels
+// of wide.hip (the experts' down-projections by the grouped tiles, beyond four rows an expert).  At these sizes a layer is fifteen launches of 5 .. 230 us;
+// enqueued one by one from Python they take longer than they run (four layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
+// Served: what wide.hip's products take, up to 27 rows an expert on average (6 of 64 experts: 288 tokens).
 #include "decode.h"
 #include <algorithm>
 

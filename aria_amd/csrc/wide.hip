@@ -1,13 +1,15 @@
 // Products of 17 .. a few hundred tokens that are bound by their weights: short prompts, and the experts of somewhat longer ones.
 //
 // A 256 x 256 tile of the matrix product leaves most of the chip idle there: 280 tokens x 7680 outputs are 60 tiles, each with the whole reduction to itself
-// (58 us for 39 MB of weights).  The row-streaming kernels of the decode step (rows.h) split the reduction over a workgroup's waves instead and take
-// up to 64 tokens at a time past the weights; further tokens find the weights in the L2 / MALL.  280 tokens, us as tiles / here: q | k | v 58 / 39
-// (with rotation and cache write in the epilogue 58 / 42), gate and up with SwiGLU (2 x 3328) 56 / 40, 2560 x 2560 34 / 22; 64 tokens: 58 / 17, 56 / 17,
-// 34 / 13; lm_head of one token 140 / 86.  From about 400 tokens on the tiles are ahead.
+// (44 us for 39 MB of weights).  The row-streaming kernels of the decode step (rows.h) split the reduction over a workgroup's waves instead and take
+// up to 64 tokens at a time past the weights; further tokens find the weights in the L2 / MALL.  Weights from HBM, us as tiles / here: 64 tokens: q | k | v
+// 29 / 17, gate and up with SwiGLU (2 x 3328) 48 / 18, 2560 x 2560 27 / 13; 280: 44 / 37, 49 / 39, 30 / 21; 352: 45 / 44, 52 / 40, 30 / 21; 400: 46 / 54,
+// 57 / 48, 31 / 24; lm_head of one token 140 / 86.
 // Routed experts: with n tokens an expert's matrix meets n k / E rows (26 at 280 tokens, 6 of 64 experts); its rows are read once per 64 of them.  Up pairs
-// (64 experts of 2 x 1664 x 2560), tiles / here: 32 tokens 238 / 182, 280 tokens 270 / 234, 350 tokens (92 rows for the most popular expert: read twice)
-// 271 / 373.  Down (2560 x 1664): 32 tokens 103 / 97, from 64 tokens on the tiles are ahead (104 / 134).
+// (64 experts of 2 x 1664 x 2560, several draws of preferred experts), tiles / here: 32 tokens 238 / 182, 128 260 / 225, 280 270 / 232 .. 245, 352 271 /
+// 235 .. 257, 400 272 / 254 .. 264, 480 273 / 276.  Smaller ones: 32 experts of 2 x 1024 x 1536, 4 a token: 64 tokens 47 / 44, 128 48 / 53, 216 49 / 55;
+// 16 of 2 x 768 x 1024, 2 a token: 64 tokens 26 / 14, 216 29 / 17.  Down (2560 x 1664): 32 tokens 103 / 97, from 64 tokens on the tiles are ahead
+// (104 / 134).
 #include "rows.h"
 
 namespace {
@@ -65,50 +67,53 @@ struct ExpertRows {   // rows sorted by expert: X row of place i is rows[i] (row
     long long ldx;
     int E, K, N;
 };
-// The row groups of all experts that have rows are one sequence, cut into equal pieces for the workgroups (experts.h); e(value, up value, place, row)
+// upto[e]: tiles of up to ROWS rows that experts 0 .. e have together; the sum of all
+template <int ROWS>
+__device__ __forceinline__ int count_tiles(const int32_t* offsets, int E, int* upto) {
+    const int l = threadIdx.x & 63;
+    int seen = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int e = min(e0 + l, E - 1), n = e0 + l < E ? offsets[e + 1] - offsets[e] : 0;
+        const int at = seen + wave_incl_scan((n + ROWS - 1) / ROWS);
+        if (int(threadIdx.x) == l && e0 + l < E) upto[e] = at;   // (the first wave; all waves hold the same numbers)
+        seen = read_lane(at, 63);
+    }
+    return seen;
+}
+// The weight row groups of all token tiles of all experts are one sequence, cut into equal pieces for the workgroups (experts.h): an expert with more rows than a
+// tile holds is further work in the sequence.  (As further work of the workgroups that own its weight rows it held up the launch: 64 experts of
+// 2 x 1664 x 2560, 280 tokens, 80 rows for the most popular one: 361 us, now 245; 55 rows 234 in both.)  e(value, up value, place, row)
 template <int KS, int MT, class Ep, bool PAIR>
 __global__ __launch_bounds__(512) void sorted_rows_kernel(ExpertRows in, Ep e) {
     ARIA_SMEM_STATIC RowsRed<8, MT> red;
-    constexpr int OUT = PAIR ? 8 : 16;
+    ARIA_SMEM_STATIC int upto[256];
+    constexpr int OUT = PAIR ? 8 : 16, ROWS = 16 * MT;
     const int t = threadIdx.x, l = t & 63, c16 = t & 15, groups = (in.N + OUT - 1) / OUT;
-    unsigned long long used[4];
-    int n_used = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int x = l + 64 * i;
-        used[i] = ballot(x < in.E && in.offsets[min(x, in.E - 1) + 1] > in.offsets[min(x, in.E - 1)]);
-        n_used += __builtin_popcountll(used[i]);
-    }
-    const int total = n_used * groups, per = (total + int(gridDim.x) - 1) / int(gridDim.x), end = min(total, (int(blockIdx.x) + 1) * per);
+    const int total = count_tiles<ROWS>(in.offsets, in.E, upto) * groups;
+    const int per = (total + int(gridDim.x) - 1) / int(gridDim.x), end = min(total, (int(blockIdx.x) + 1) * per);
     int g = int(blockIdx.x) * per;
+    sync();
     while (g < end) {
-        int a = g / groups, id = 0;
-        const int g0 = g - a * groups, g1 = min(groups, g0 + end - g);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int here = __builtin_popcountll(used[i]);
-            if (a >= 0 && a < here) {
-                unsigned long long m = used[i];
-                for (int j = 0; j < a; ++j) m &= m - 1;
-                id = 64 * i + __builtin_ctzll(m);
-            }
-            a -= here;
+        const int tile = g / groups, g0 = g - tile * groups, g1 = min(groups, g0 + end - g);
+        int id = 0;
+        for (int e0 = 0; e0 < in.E; e0 += 64) {   // the first expert with tiles beyond this one's number
+            const unsigned long long behind = ballot(e0 + l < in.E && upto[min(e0 + l, in.E - 1)] > tile);
+            id = e0 + (behind ? __builtin_ctzll(behind) : 0);
+            if (behind) break;
         }
-        const int first = in.offsets[id], m = in.offsets[id + 1] - first;
+        const int first = in.offsets[id], m = in.offsets[id + 1] - first, t0 = (tile - (id ? upto[id - 1] : 0)) * ROWS;
         const bf16_t* W = (PAIR && c16 >= 8 ? in.W2 : in.W) + (long long)id * in.N * in.K;
-        for (int t0 = 0; t0 < m; t0 += 16 * MT) {
-            sync();   // (the sums of the piece before are read)
-            stream_rows<8, KS, MT>(
-                in.K, [&](int gg) { return W + (long long)min(gg * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * in.K; },
-                [&](int i) {
-                    const int at = first + min(t0 + 16 * i + c16, m - 1);
-                    return in.X + (long long)(in.rows ? in.rows[at] : at) * in.ldx;
-                },
-                g0, g1, red, [&](float v, int tok, int n, int gg) {
-                    const float u = PAIR ? shfl_xor(v, 8) : 0.f;
-                    if (t0 + tok < m && gg * OUT + n < in.N && n < OUT) e(v, u, first + t0 + tok, gg * OUT + n);
-                });
-        }
+        sync();   // (the sums of the piece before are read)
+        stream_rows<8, KS, MT>(
+            in.K, [&](int gg) { return W + (long long)min(gg * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * in.K; },
+            [&](int i) {
+                const int at = first + min(t0 + 16 * i + c16, m - 1);
+                return in.X + (long long)(in.rows ? in.rows[at] : at) * in.ldx;
+            },
+            g0, g1, red, [&](float v, int tok, int n, int gg) {
+                const float u = PAIR ? shfl_xor(v, 8) : 0.f;
+                if (t0 + tok < m && gg * OUT + n < in.N && n < OUT) e(v, u, first + t0 + tok, gg * OUT + n);
+            });
         g += g1 - g0;
     }
 }

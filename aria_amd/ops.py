@@ -45,8 +45,10 @@ ACTIVATIONS = {None: 0, "gelu_tanh": 1, "relu_squared": 2}
 
 
 # Products of few tokens are bound by their weights; up to these sizes the row-streaming kernels (csrc/wide.hip) are ahead of the tiles.
-ROWS_TOKENS = 320      # 280 tokens x 7680 x 2560: 37 us, tiles 58; 400: 54, tiles 58
-ROWS_PER_EXPERT = 27       # on average, gate and up pairs: 280 tokens, 6 of 64 experts of 1664 x 2560: 234 us, tiles 270; 350: 373, tiles 271
+ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44; 352: 44, 45; 400: 54, 46
+# Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token: 27 rows 232 us, tiles 270; 37: 254 .. 264, 272; 45: 276, 273.  32 of
+# 1024 x 1536, whose tiles are one full round: 8 rows 44, tiles 47; 27: 55, 49.  16 of 768 x 1024: 27 rows 17, tiles 29; 50: 21, 29.
+ROWS_PER_EXPERT = 27
 ROWS_PER_EXPERT_DOWN = 4   # down projections: 32 tokens 97 us, tiles 103; 64: 134, tiles 104
 
 

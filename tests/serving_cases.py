@@ -427,6 +427,25 @@ def case_rows_products(dev, M, N, K, E=3):
         assert L.rel(ops.rows_experts(xd, we.to(dev), off, w_up=ue.to(dev), **kw), torch.nn.functional.silu(y) * z) < 2 ** -7
 
 
+def case_rows_experts_uneven(dev, counts, N, K):
+    """Experts of no rows, one row, whole token tiles and a row more, among more than 64 experts too: the bits of each expert's product by itself."""
+    from aria_amd import ops
+
+    E, M = len(counts), sum(counts)
+    x, w, u = (L.rnd(*n, K, seed=i, scale=K ** -0.5 if i else 1.0).to(dev) for i, n in enumerate(((M,), (E, N), (E, N))))
+    cuts = [sum(counts[:e]) for e in range(E + 1)]
+    rows = torch.randperm(M, generator=L.gen(M)).to(torch.int32)
+    xs = x[rows.long().to(dev)]
+    each = [(xs[a:b], w[e], u[e]) for e, (a, b) in enumerate(zip(cuts, cuts[1:])) if b > a]
+    args = x, w, torch.tensor(cuts, dtype=torch.int32, device=dev), rows.to(dev)
+    assert torch.equal(ops.rows_experts(*args), torch.cat([ops.rows_gemm(t, a) for t, a, _ in each]))
+    assert torch.equal(ops.rows_experts(*args, w_up=u), torch.cat([ops.rows_swiglu(t, a, b) for t, a, b in each]))
+
+
+# sixteen, 32 and 64 rows a tile
+UNEVEN = [[0] * 65 + [40, 0, 16, 1, 17], [33, 0, 1, 24, 0, 2, 0, 0, 4], [0, 65, 1, 129, 0, 64, 2]]
+
+
 def case_rows_qkv(dev, M, D, hd, S):
     """Projection, rotation and cache write in one launch against the separate ones on the same product, bit for bit: positions 0 .. and any slots."""
     from aria_amd import gptfast as G

@@ -70,6 +70,11 @@ def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("counts", C.UNEVEN)
+def test_rows_experts_uneven(counts):
+    C.case_rows_experts_uneven(DEV, counts, 20, 136)
+
+
 def test_rows_qkv():
     C.case_rows_qkv(DEV, 37, 128, 64, 40)
 

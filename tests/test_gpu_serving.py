@@ -80,6 +80,12 @@ def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("N,K", [(33, 1024), (1664, 2560), (24, 1672)])
+@pytest.mark.parametrize("counts", C.UNEVEN)
+def test_rows_experts_uneven(counts, N, K):
+    C.case_rows_experts_uneven(DEV, counts, N, K)
+
+
 @pytest.mark.parametrize("M,D,hd,S", [(5, 512, 64, 8), (100, 2560, 128, 104), (37, 768, 64, 40)])
 def test_rows_qkv(M, D, hd, S):
     C.case_rows_qkv(DEV, M, D, hd, S)
