@@ -350,10 +350,10 @@ __global__ __launch_bounds__(256) void mix_up_kernel(const float* logits, const 
     }
     const int n = blockIdx.x * 4 + w;
     if (n >= F) return;
-    float acc[2][1] = {{0.f}, {0.f}};
+    float acc[2] = {0.f, 0.f};
     const long long row = ((long long)e * F + n) * K;
-    two_rows<1>(acc, Wg + row, Wu + row, X + (long long)tok * K, K, 1, K, l);
-    if (l == 0) act[((long long)tok * k + j) * F + n] = f2bf(silu_fast(acc[0][0]) * acc[1][0]);
+    two_rows(acc, Wg + row, Wu + row, X + (long long)tok * K, K, l);
+    if (l == 0) act[((long long)tok * k + j) * F + n] = f2bf(silu_fast(acc[0]) * acc[1]);
 }
 // down-projections of a token's k experts for two stream columns, their weighted sum, residual and norms
 __global__ __launch_bounds__(256) void mix_down_kernel(const bf16_t* Wd, const float* weights, const int32_t* idx, int k, const bf16_t* act, int F, int D,
@@ -364,11 +364,11 @@ __global__ __launch_bounds__(256) void mix_down_kernel(const bf16_t* Wd, const f
     float y0 = 0.f, y1 = 0.f;
     for (int j = 0; j < k; ++j) {
         const bf16_t* base = Wd + (long long)idx[tok * k + j] * D * F;
-        float acc[2][1] = {{0.f}, {0.f}};
-        two_rows<1>(acc, base + (long long)row0 * F, base + (long long)min(row0 + 1, D - 1) * F, act + ((long long)tok * k + j) * F, F, 1, F, l);
+        float acc[2] = {0.f, 0.f};
+        two_rows(acc, base + (long long)row0 * F, base + (long long)min(row0 + 1, D - 1) * F, act + ((long long)tok * k + j) * F, F, l);
         const float wj = weights[tok * k + j];
-        y0 += wj * acc[0][0];
-        y1 += wj * acc[1][0];
+        y0 += wj * acc[0];
+        y1 += wj * acc[1];
     }
     if (l < 2 && row0 + l < D) stream_step(l ? y1 : y0, ro.post, ro.next, ro.x, ro.h, (long long)tok * D + row0 + l, row0 + l);
 }

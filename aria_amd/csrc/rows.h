@@ -16,10 +16,9 @@ __device__ __forceinline__ u32x4 ldw16(const bf16_t* p) {   // a weight stream i
     return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 #endif
 }
-// acc[r][b] += W[row r] . X[token b], a wave over two weight rows and NB token rows: four 16-byte chunks per row and lane requested before the
-// first use, the token rows come from the L1 / L2
-template <int NB>
-__device__ __forceinline__ void two_rows(float (&acc)[2][NB], const bf16_t* w0, const bf16_t* w1, const bf16_t* x, long long ldx, int nb, int K, int l) {
+// acc[r] += W[row r] . x, a wave over two weight rows: four 16-byte chunks per row and lane requested before the first use, the token's row comes from the
+// L1 / L2
+__device__ __forceinline__ void two_rows(float (&acc)[2], const bf16_t* w0, const bf16_t* w1, const bf16_t* x, int K, int l) {
     const int nch = K >> 3;
     for (int c0 = l; c0 < nch; c0 += 256) {
         u32x4 a[2][4];
@@ -30,25 +29,19 @@ __device__ __forceinline__ void two_rows(float (&acc)[2][NB], const bf16_t* w0, 
             a[1][u] = ldw16(w1 + c * 8);
         }
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const bf16_t* xr = x + (long long)min(b, nb - 1) * ldx;
+        for (int u = 0; u < 4; ++u) {
+            u32x4 v = ld16(x + min(c0 + 64 * u, nch - 1) * 8);
+            const bool in = c0 + 64 * u < nch;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                u32x4 v = ld16(xr + min(c0 + 64 * u, nch - 1) * 8);
-                const bool in = c0 + 64 * u < nch;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t xv = in ? v[q] : 0u;
-                    acc[0][b] = dot2bf(a[0][u][q], xv, acc[0][b]);
-                    acc[1][b] = dot2bf(a[1][u][q], xv, acc[1][b]);
-                }
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t xv = in ? v[q] : 0u;
+                acc[0] = dot2bf(a[0][u][q], xv, acc[0]);
+                acc[1] = dot2bf(a[1][u][q], xv, acc[1]);
             }
         }
     }
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[r][b] = wave_sum_bcast(acc[r][b]);
+    acc[0] = wave_sum_bcast(acc[0]);
+    acc[1] = wave_sum_bcast(acc[1]);
 }
 
 struct RowsIn {
@@ -78,9 +71,9 @@ __global__ __launch_bounds__(256) void row_kernel(RowsPair rp, E e) {
     if (in.sq) {
         for (int i = t; i < in.sq_n; i += 256) ss += in.sq[i];
     }
-    float acc[2][1] = {{0.f}, {0.f}};
-    two_rows<1>(acc, in.W + (long long)r0 * in.K, (PAIR ? in.W2 : in.W) + (long long)r1 * in.K, in.X, 0, 1, in.K, l);
-    float v0 = acc[0][0], v1 = acc[1][0];
+    float acc[2] = {0.f, 0.f};
+    two_rows(acc, in.W + (long long)r0 * in.K, (PAIR ? in.W2 : in.W) + (long long)r1 * in.K, in.X, in.K, l);
+    float v0 = acc[0], v1 = acc[1];
     if (in.sq) {
         ss = wave_sum_bcast(ss);
         if (l == 0) red[w] = ss;
