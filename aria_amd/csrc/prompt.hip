@@ -3,6 +3,7 @@
 // enqueued one by one from Python they take longer than they run (four layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
 // Served: what wide.hip's products take, up to 27 rows an expert on average (6 of 64 experts: 288 tokens).
 #include "decode.h"
+#include "rows.h"
 #include <algorithm>
 
 namespace {
@@ -104,7 +105,11 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
     if (n_wanted == 0) return rc;
     ARIA_TRY(aria_rmsnorm_fwd(delta, x, ptrs[1], y, z.h, nullptr, T, D, eps, stream));
     ARIA_TRY(aria_moe_permute(z.h, wanted, z.ao, n_wanted, D, 1, D, stream));
-    ARIA_TRY(aria_rows_gemm(z.ao, ptrs[2], logits, 1, n_wanted, V, D, D, V, stream));
+    if (rows_ahead(n_wanted, V, D) || (V & 1)) {   // (the tiles store pairs of columns)
+        ARIA_TRY(aria_rows_gemm(z.ao, ptrs[2], logits, 1, n_wanted, V, D, D, V, stream));
+    } else {
+        ARIA_TRY(aria_gemm_bf16(z.ao, ptrs[2], logits, nullptr, n_wanted, V, D, 0, 0, D, D, V, 1, 0, stream));
+    }
 #undef ARIA_TRY
     return rc;
 }

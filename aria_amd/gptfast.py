@@ -102,7 +102,7 @@ def _glu_pair_ready(w_gate: nn.Parameter, w_up: nn.Parameter) -> bool:
 
 def _project(x2d: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x w^T: the row-streaming kernel for few tokens, the tile product beyond"""
-    return ops.rows_gemm(x2d, w) if ops.rows_take(*x2d.shape) and w.is_contiguous() and w.shape[0] % 2 == 0 else ops.gemm(x2d, w)
+    return ops.rows_gemm(x2d, w) if ops.rows_take(*x2d.shape, w.shape[0]) and w.is_contiguous() and w.shape[0] % 2 == 0 else ops.gemm(x2d, w)
 
 
 class RMSNorm(nn.Module):
@@ -150,7 +150,7 @@ class Attention(nn.Module):
             # rotation nor the cache row depends on a device tensor nobody validated.  A prompt longer than the cache takes the
             # path below, whose copy raises.
             cache = self.kv_cache
-            if ops.rows_take(S, D) and self.wqkv.weight.is_contiguous():
+            if ops.rows_take(S, D, 3 * D) and self.wqkv.weight.is_contiguous():
                 q = ops.rows_qkv_rope_cache(x2d, self.wqkv.weight, freqs_cis, cache.k[:1], cache.v[:1], hd)
             else:
                 q = ops.gemm_qkv_rope_cache(x2d, self.wqkv.weight, freqs_cis, None, cache.k, cache.v, S, hd)
@@ -213,7 +213,7 @@ class MOEFeedForward(nn.Module):
 
     def forward(self, x2d):
         k = self.config.router_topk
-        few = ops.rows_take(*x2d.shape)   # few tokens: every product is bound by its weights
+        few = ops.rows_take(*x2d.shape, 2 * self.shared_ffn.w1.weight.shape[0])   # few tokens: every product is bound by its weights
         if not few and ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
             logits, scores, idx, counts = ops.moe_router_fused(x2d, self.gate.weight, k)
         else:

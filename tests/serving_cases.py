@@ -57,11 +57,11 @@ def case_gptfast_batch(dev, engine=True):
             sched.finish(r)
 
 
-def gptfast_routed(dev, dim, head_dim, inter, block):
+def gptfast_routed(dev, dim, head_dim, inter, block, vocab=264):
     """Embeddings carry the directions of their experts, so that no choice is a close call."""
     from aria_amd import gptfast as G
 
-    E, k, V = 16, 3, 264
+    E, k, V = 16, 3, vocab
     args = G.ModelArgs(block_size=block, vocab_size=V, n_layer=2, n_head=dim // head_dim, dim=dim, intermediate_size=inter, rope_base=10000.0, norm_eps=1e-5,
                        num_experts=E, router_topk=k, num_shared_experts=2)
     m, g = G.Transformer(args), L.gen(5)
@@ -505,13 +505,13 @@ def gptfast_oracle(m, toks, r=lambda t: t):
     return norm(x, "norm") @ w["output.weight"].T, cache
 
 
-def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2):
+def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2, vocab=264):
     """Prompts of several requests, tokens of all of them and a token of one against float64: logits and cache rows, each step seen to be one library call.  Bound:
     three times what 16-bit tensors between exact operations make of the same sequence."""
     from aria_amd import gptfast as G
     from aria_amd.serving import Scheduler
 
-    m, served = gptfast_routed(dev, dim, 64, inter, max(lens) + 8), []
+    m, served = gptfast_routed(dev, dim, 64, inter, max(lens) + 8, vocab), []
     for name in ("prompts", "run"):
         def seen(self, *a, plain=getattr(G._StepTables, name), name=name):
             out = plain(self, *a)
@@ -540,6 +540,20 @@ def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2):
             for got, want in zip((kv.k, kv.v), pair):
                 assert L.logit_err(got[sched.live[i][0], :n].reshape(-1, 64), want[:n].reshape(-1, 64).cpu()) < cache_tol
     assert served == [("prompts", True)] + [("run", True)] * steps
+
+
+def case_rows_rule():
+    """The line between products by rows and by tiles: its points on both sides as measured, and beyond it nothing comes back."""
+    from aria_amd import ops
+
+    for M, K, N in ((320, 2560, 7680), (128, 2560, 16384), (320, 1536, 8192), (64, 1024, 32000), (16, 2560, 100352), (96, 4096, 7680), (256, 4096, 2560)):
+        assert ops.rows_take(M, K, N), (M, K, N)
+    for M, K, N in ((192, 2560, 16384), (128, 1024, 32000), (64, 2560, 100352), (128, 4096, 7680), (320, 4096, 2560), (321, 2560, 2560), (16, 504, 2560), (0, 2560, 64)):
+        assert not ops.rows_take(M, K, N), (M, K, N)
+    for K in (512, 2560, 4096):
+        for N in (64, 7680, 20000, 50000):
+            taken = [ops.rows_take(M, K, N) for M in range(1, 400)]
+            assert taken == sorted(taken, reverse=True)
 
 
 def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17), inter=128):

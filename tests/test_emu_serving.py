@@ -83,6 +83,10 @@ def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV, 128, (5, 1, 9))
 
 
+def test_rows_rule():
+    C.case_rows_rule()
+
+
 def test_gptfast_steps_oracle(monkeypatch):
     C.case_gptfast_steps_oracle(DEV, monkeypatch, 512, 512, (3, 1, 5))
 

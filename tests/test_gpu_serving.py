@@ -96,9 +96,10 @@ def test_gptfast_packed_prompts_in_one_call(dim, inter, lens):
     C.case_gptfast_packed_prompts(DEV, dim, lens, inter)
 
 
-@pytest.mark.parametrize("dim,inter,lens", [(512, 512, (9, 1, 20, 7)), (1024, 1664, (20,)), (2560, 1664, (33, 30, 8)), (2560, 1664, (140, 1))])
-def test_gptfast_steps_oracle(monkeypatch, dim, inter, lens):
-    C.case_gptfast_steps_oracle(DEV, monkeypatch, dim, inter, lens)
+@pytest.mark.parametrize("dim,inter,lens,vocab", [(512, 512, (9, 1, 20, 7), 264), (1024, 1664, (20,), 264), (2560, 1664, (33, 30, 8), 264), (2560, 1664, (140, 1), 264),
+                                                  (512, 512, (9, 10), 41002), (512, 512, (9, 10), 41003)])   # (heads by tiles; of odd size)
+def test_gptfast_steps_oracle(monkeypatch, dim, inter, lens, vocab):
+    C.case_gptfast_steps_oracle(DEV, monkeypatch, dim, inter, lens, vocab=vocab)
 
 
 def test_gptfast_packed_prompts():
