@@ -156,17 +156,18 @@ class StepBatch:
             for t in ([[t[0] for t in tokens]] if T == n and max(lengths, default=0) == 1 else tokens):
                 put(_numbers(t), len(t))
         each = np.asarray(lengths, dtype=np.int64)
-        ends = np.cumsum(each)
-        put(np.repeat(_numbers(slots), each), T)
-        put(np.arange(T) + np.repeat(_numbers(starts, "iub") - (ends - each), each), T)
-        put(np.repeat(np.arange(n), each), T)
+        ends = each.cumsum()
+        put(_numbers(slots).repeat(each), T)
+        put(np.arange(T) + (_numbers(starts, "iub") - (ends - each)).repeat(each), T)
+        put(np.arange(n).repeat(each), T)
         put(0, 1)
         put(ends, n)
         if wanted is not None:
             put(_numbers(wanted), len(wanted))
-        if fill.min() < -2 ** 31 or fill.max() >= 2 ** 31:     # (the assignment would wrap)
+        narrow = host.numpy()
+        narrow[:] = fill
+        if np.count_nonzero(narrow != fill):     # (the assignment has wrapped)
             raise RuntimeError("value cannot be converted to type int32 without overflow")
-        host.numpy()[:] = fill
         buf = host.to(device, non_blocking=True) if cuda else host
         at = 0
 
