@@ -46,10 +46,11 @@ ACTIVATIONS = {None: 0, "gelu_tanh": 1, "relu_squared": 2}
 
 # Products of few tokens are bound by their weights; up to these sizes the row-streaming kernels (csrc/wide.hip) are ahead of the tiles.
 ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44; 352: 44, 45; 400: 54, 46
-# Weight rows times passes over them (64 tokens each, 32 beyond 2560 columns), and those times columns: 16384 x 2560: 128 tokens 37 us, tiles 43; 192: 52, 47.  13312:
-# 192 tokens 45, 44; 256: 51, 46.  8192 x 1536: 320 tokens 34, 41.  32000 x 1024: 64 tokens 20, 24; 128: 31, 27.  100352 x 2560: 16 tokens 100, 110; 64: 120, 119;
-# 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.
-ROWS_PASSED, ROWS_READ = 41000, 100_000_000
+# Weight rows times passes over them, 64 tokens each up to 2560 columns, 32 beyond.  us, tiles: 16384 x 2560: 128 tokens 37, 43; 192: 52, 47.  13312: 192 tokens 45, 44;
+# 256: 51, 46.  8192 x 1536: 320 tokens 34, 41.  32000 x 1024: 64 tokens 20, 24; 128: 31, 27.  64000 x 1536: 64 tokens 54, 43.  100352 x 2560: 16 tokens 100, 110; 64:
+# 120, 119; 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.  (The line up to 2560 columns lies
+# behind the crossing since a tile product takes about 15 us more of the host's time: 10240 x 2560, 200 .. 300 tokens, four in a prompt of 1.5 ms.)
+ROWS_PASSED, ROWS_PASSED_LONG = 52000, 24000
 # Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token: 27 rows 232 us, tiles 270; 37: 254 .. 264, 272; 45: 276, 273.  32 of
 # 1024 x 1536, whose tiles are one full round: 8 rows 44, tiles 47; 27: 55, 49.  16 of 768 x 1024: 27 rows 17, tiles 29; 50: 21, 29.
 ROWS_PER_EXPERT = 27
@@ -58,8 +59,8 @@ ROWS_PER_EXPERT_DOWN = 4   # down projections: 32 tokens 97 us, tiles 103; 64: 1
 
 def rows_take(M: int, K: int, N: int) -> bool:
     """Whether x [M, K] w^T for a w [N, K] goes by rows.  (Below 512 columns a launch costs more than the weights in either form.)"""
-    passed = N * -(-M // (64 if K <= 2560 else 32))
-    return 0 < M <= ROWS_TOKENS and 512 <= K <= 4096 and K % 8 == 0 and (M <= 16 or (passed <= ROWS_PASSED and passed * K <= ROWS_READ))
+    return (0 < M <= ROWS_TOKENS and 512 <= K <= 4096 and K % 8 == 0
+            and (M <= 16 or (N * -(-M // 64) <= ROWS_PASSED if K <= 2560 else N * -(-M // 32) <= ROWS_PASSED_LONG)))
 
 
 def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> bool:

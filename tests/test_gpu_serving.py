@@ -97,7 +97,7 @@ def test_gptfast_packed_prompts_in_one_call(dim, inter, lens):
 
 
 @pytest.mark.parametrize("dim,inter,lens,vocab", [(512, 512, (9, 1, 20, 7), 264), (1024, 1664, (20,), 264), (2560, 1664, (33, 30, 8), 264), (2560, 1664, (140, 1), 264),
-                                                  (512, 512, (9, 10), 41002), (512, 512, (9, 10), 41003)])   # (heads by tiles; of odd size)
+                                                  (512, 512, (9, 10), 52002), (512, 512, (9, 10), 52003)])   # (heads by tiles; of odd size)
 def test_gptfast_steps_oracle(monkeypatch, dim, inter, lens, vocab):
     C.case_gptfast_steps_oracle(DEV, monkeypatch, dim, inter, lens, vocab=vocab)
 
