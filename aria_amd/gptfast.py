@@ -439,13 +439,20 @@ class Transformer(nn.Module):
         logits = tables.prompts(batch, embed) if prompts and batch.n_wanted <= batch.ids.numel() else None
         # Every tensor is compared with the tables beside the device's work (20 us a layer of host time in front of it otherwise).  The tables keep what they
         # point to: where something was exchanged, the step on the old tensors has done no harm and is run again on the new ones.
-        if tables is not None and batch.longest > 1 and not tables.current(self):
+        looked = logits is not None or not batch.fresh or min(batch.lengths) < 2     # (whole prompts on the modules do not read the tables)
+        if tables is not None and batch.longest > 1 and looked and not tables.current(self):
             tables = self._tables = _StepTables(self)
             logits = tables.prompts(batch, embed) if logits is not None else None
-        if logits is not None:
-            return logits
-        if prompts and self._packs(batch) and embed() is not None:
-            return self._prompts(batch, embed())
+        if logits is None and prompts and self._packs(batch) and embed() is not None:
+            logits = self._prompts(batch, embed())
+        if logits is None:
+            logits = self._one_by_one(batch, tables, embed)
+        if not looked and tables is not None and not tables.current(self):
+            self._tables = None
+        return logits
+
+    def _one_by_one(self, batch, tables, embed) -> torch.Tensor:
+        """The batch's sequences one after the other, each on its own slot."""
         whole = [b.attention.kv_cache for b in self.layers]
         key = tuple(c.k.data_ptr() for c in whole)
         if getattr(self, "_slot_key", None) != key:
