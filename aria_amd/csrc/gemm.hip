@@ -349,7 +349,9 @@ bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB,
 // Fewest 256 x 256 tiles that v3 takes in one partly filled round: its time there is the reduction's (about 1.45 us per 64 columns), the 128 x 128 kernel's
 // grows with the tiles.  us as 128 x 128 / 256 x 256: 4096 x 2560 outputs (160 tiles), K = 2560 86 / 58, K = 1664 57 / 40, K = 512 27 / 19; 2100 x 2560 (90
 // tiles), K = 2560 54 / 54.  Shorter reductions stay with the small tiles.
-constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150;
+// Rows by expert: where they fill a third of a tile and more.  128 x 128 / 256 x 256, 150 .. 191 tiles: 64 experts of 2560 x 1664: 60 rows each on average 132 / 146, 72 134 /
+// 140; 3328 x 2560: 48 rows 248 / 277; 32 experts of 3328 x 2560: 88 rows 173 / 145; 64 of 1536 x 1024: 96 rows 76 / 54; 16 of 2560 x 1664: 240 rows 83 / 47.
+constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150, V3_FEW_ROWS = 84;
 long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
 }  // namespace
@@ -449,7 +451,7 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const char* gforce = std::getenv("ARIA_GEMM_FORCE");
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
     if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
-                      v3_least(K, V3_FEW_TILES_GROUPED)))
+                      v3_least(K, M_total >= V3_FEW_ROWS * E ? V3_FEW_TILES_GROUPED : 192)))
         return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc, int(M_total / 256 + E), stream);
     if (use_v2((M_total / 256 + 1) * ((N + 255) / 256))) return g_last_variant = 2, aria_launch_gemm2(p, 0, b_oc, int(M_total / 256 + E), 1, stream);
     return g_last_variant = 1, launch_gemm(p, 0, b_oc, p.ntn * max_tm, 1, stream);

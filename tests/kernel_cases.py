@@ -138,6 +138,20 @@ def case_gemm_tile_rule(dev, tiles, K, variant):
     assert float((got.double() - want).norm() / want.norm()) < 2e-6
 
 
+def case_grouped_gemm_tile_rule(dev, E, variant):
+    """Rows by expert on both sides of the rows that the large tiles want in a partly filled round, against float64 (bf16 results: half an ulp, 2^-9)."""
+    from aria_amd import hip, ops
+
+    M, N, K = 3840, 2560, 512      # (160 tiles)
+    g = torch.Generator().manual_seed(E)
+    cuts = torch.cat([torch.zeros(2), torch.randint(0, M, (E - 2,), generator=g).sort().values, torch.tensor([M])]).to(torch.int32)
+    a, w = rnd(M, K, seed=1), rnd(E, N, K, seed=2)
+    got = ops.grouped_gemm(a.to(dev), w.to(dev), cuts.to(dev), w_is_kn=False).double().cpu()
+    assert hip.get_lib().cdll.aria_last_gemm_variant() == variant
+    want = torch.cat([a[i:j].double() @ w[e].double().T for e, (i, j) in enumerate(zip(cuts.tolist(), cuts.tolist()[1:]))])
+    assert float((got - want).norm() / want.norm()) < 2 ** -8
+
+
 def case_unpermute_with_residual(dev, T, D, k, E=8):
     """r05b: the decoder layer's residual add as the last step of the un-permute launch (aria_moe_unpermute_res) == aria_moe_unpermute +
     aria_add_bf16, bit for bit (bf16(h + bf16(combine + shared))), with and without scores / shared rows; widths without a compile-time kernel

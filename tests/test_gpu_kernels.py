@@ -213,6 +213,11 @@ def test_gemm_split_into_many_pieces(M, N, K, a_oc, b_oc):
     assert hip.get_lib().cdll.aria_last_gemm_variant() == 3
 
 
+@pytest.mark.parametrize("E,variant", [(45, 3), (46, 1)])
+def test_grouped_gemm_tile_rule(E, variant):
+    C.case_grouped_gemm_tile_rule(DEV, E, variant)
+
+
 @pytest.mark.parametrize("tiles,K,variant", [(79, 512, 1), (80, 512, 3), (80, 504, 1), (191, 504, 1), (191, 512, 3), (192, 504, 3)])
 def test_gemm_tile_rule(tiles, K, variant):
     C.case_gemm_tile_rule(DEV, tiles, K, variant)
