@@ -317,7 +317,7 @@ inline int rows_tiles(int64_t K, int64_t T) {
 // the L2 / MALL (100352 x 2560: 16 tokens 100 us, tiles 110; 64: 120, 119; 320: 405, 212; 13312 x 2560: 192 tokens 45, 44; 256: 51, 46; 7680 x 4096: 96 tokens 35, 36;
 // 128: 44, 37).
 inline bool rows_ahead(int64_t M, int64_t N, int64_t K) {
-    return M <= 16 || (K <= 2560 ? N * ((M + 63) / 64) <= 52000 : N * ((M + 31) / 32) <= 24000);
+    return M <= 16 || (K <= 2560 ? N * ((M + 63) / 64) <= 52000 : N * ((M + 31) / 32) <= 26000);
 }
 template <bool PAIR, class E>
 int launch_rows_wide(const RowsIn& in, int64_t T, const E& e, void* stream) {

@@ -49,8 +49,8 @@ ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44;
 # Weight rows times passes over them, 64 tokens each up to 2560 columns, 32 beyond.  us, tiles: 16384 x 2560: 128 tokens 37, 43; 192: 52, 47.  13312: 192 tokens 45, 44;
 # 256: 51, 46.  8192 x 1536: 320 tokens 34, 41.  32000 x 1024: 64 tokens 20, 24; 128: 31, 27.  64000 x 1536: 64 tokens 54, 43.  100352 x 2560: 16 tokens 100, 110; 64:
 # 120, 119; 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.  Level up to the line: 10240 x 2560: 200
-# tokens 39, 39; 300: 52, 51 -- by rows with 8 us of the host's time, by tiles 15.
-ROWS_PASSED, ROWS_PASSED_LONG = 52000, 24000
+# tokens 39, 39; 300: 52, 51 -- by rows with 8 us of the host's time, by tiles 15; 2560 x 3328: 320 tokens 33, 34, in a model 7 us ahead (300 tokens, four layers, 2540 us against 2569).
+ROWS_PASSED, ROWS_PASSED_LONG = 52000, 26000
 # Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token: 27 rows 232 us, tiles 270; 37: 254 .. 264, 272; 45: 276, 273.  32 of
 # 1024 x 1536, whose tiles are one full round: 8 rows 44, tiles 47; 27: 55, 49.  16 of 768 x 1024: 27 rows 17, tiles 29; 50: 21, 29.
 ROWS_PER_EXPERT = 27

@@ -546,9 +546,9 @@ def case_rows_rule():
     """The line between products by rows and by tiles: its points on both sides as measured, and beyond it nothing comes back."""
     from aria_amd import ops
 
-    for M, K, N in ((320, 2560, 7680), (192, 2560, 13312), (320, 1536, 8192), (64, 1024, 32000), (16, 2560, 100352), (96, 4096, 7680), (256, 4096, 2560)):
+    for M, K, N in ((320, 2560, 7680), (192, 2560, 13312), (320, 1536, 8192), (64, 1024, 32000), (16, 2560, 100352), (96, 4096, 7680), (320, 3328, 2560)):
         assert ops.rows_take(M, K, N), (M, K, N)
-    for M, K, N in ((256, 2560, 13312), (128, 1024, 32000), (64, 2560, 100352), (128, 4096, 7680), (320, 4096, 2560), (321, 2560, 2560), (16, 504, 2560), (0, 2560, 64)):
+    for M, K, N in ((256, 2560, 13312), (128, 1024, 32000), (64, 2560, 100352), (128, 4096, 7680), (320, 4096, 2664), (321, 2560, 2560), (16, 504, 2560), (0, 2560, 64)):
         assert not ops.rows_take(M, K, N), (M, K, N)
     for K in (512, 2560, 4096):
         for N in (64, 7680, 20000, 50000):
