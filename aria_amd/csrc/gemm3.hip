@@ -1088,43 +1088,78 @@ __global__ __launch_bounds__(512) void gemm3_kernel(GemmParams p) {
         store_any3<0>(p, acc, C, m0, m_end, n0, l, w, wm, wn, smem);
 }
 
-// Sums the `split` slabs of every split tile in slab order (deterministic), then bias / accumulate / round exactly like the
-// main epilogue.  grid (split tiles, 16): block (r, part) finishes the part-th sixteenth of split tile r IN THE SLABS' ORDER (the accumulators'
-// order, see the slab store in gemm3_kernel): a thread's four consecutive floats are registers 4 q .. 4 q + 3 of one lane = one row, four
-// consecutive columns (r06: transposed accumulators).
+// Sums the `split` slabs of every split tile in slab order (deterministic), then bias / activation / accumulate / round exactly like the main
+// epilogue.  grid (split tiles, 16): block (r, part) finishes 32 rows x 128 columns of split tile r -- the accumulator tiles (a, i, b) = part's
+// bits of the four waves that share wm -- which the slabs hold as 16 runs of 1 KiB (see the slab store in gemm3_kernel): a thread's 16 bytes are
+// registers 4 q .. 4 q + 3 of one lane = one row, four consecutive columns.
+// Bound by latency and by the form of its stores, not by bytes: with one slab's piece requested at a time (a chain of 4 x split round trips) and four
+// 2-byte stores a piece, 80 tiles of 3 slabs took 22 us, 40 of 4 14.5, 34 of 2 12.9 (sums added to an old tile); now a thread requests its four pieces of three more slabs at once,
+// and the sums cross the LDS so that the result leaves (and an accumulated one arrives) as 16-byte pieces of 256-byte rows: 12.1, 10.3 and 8.1 us.
+constexpr int REDP = 132;   // floats a parked row
 __global__ __launch_bounds__(256) void gemm3_reduce_kernel(GemmParams p) {
+    ARIA_SMEM_STATIC float sums[32 * REDP];
     int tn, tmi;
     if (!aria_tile_from_pos(p, p.split_first + blockIdx.x, tmi, tn)) return;
-    const int t = threadIdx.x;
-    const float* ws = p.ws + (long long)blockIdx.x * p.split * (BM * BN);
+    const int t = threadIdx.x, part = blockIdx.y, wm = part & 1, b = part >> 3, a = (part >> 2) & 1, i = (part >> 1) & 1;
+    const int l = t & 63, q = t >> 6;
+    const float* ws = p.ws + (long long)blockIdx.x * p.split * (BM * BN) + (wm * 4 * 8 + (b * 2 + a) * 2 + i) * 1024 + q * 256 + l * 4;
+    f32x4 sum[4];   // wave wn = 0..3 of the row group
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int j = (blockIdx.y * 4 + it) * 256 + t;   // 16-byte piece of the slab
-        const int l = j & 63, q = (j >> 6) & 3, t8 = (j >> 8) & 7, w = j >> 11;
-        const int b = t8 >> 2, a = (t8 >> 1) & 1, i = t8 & 1, wm = w >> 2, wn = w & 3;
-        // (r06, transposed accumulators: registers 4 q .. 4 q + 3 of a lane = one ROW, four consecutive columns)
-        const int row = a * 128 + wm * 64 + i * 32 + (l & 31), col0 = b * 128 + wn * 32 + 8 * q + 4 * (l >> 5);
-        f32x4 sum = *reinterpret_cast<const f32x4*>(ws + 4 * j);
-        for (int s = 1; s < p.split; ++s) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(ws + (long long)s * (BM * BN) + 4 * j);
+    for (int wn = 0; wn < 4; ++wn) sum[wn] = *reinterpret_cast<const f32x4*>(ws + wn * 8192);
+    int s = 1;
+    for (; s + 3 <= p.split; s += 3) {
+        f32x4 v[3][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sum[e] += v[e];
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int wn = 0; wn < 4; ++wn) v[k][wn] = *reinterpret_cast<const f32x4*>(ws + (long long)(s + k) * (BM * BN) + wn * 8192);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int wn = 0; wn < 4; ++wn)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[wn][e] += v[k][wn][e];
+    }
+    for (; s < p.split; ++s) {
+        f32x4 v[4];
+#pragma unroll
+        for (int wn = 0; wn < 4; ++wn) v[wn] = *reinterpret_cast<const f32x4*>(ws + (long long)s * (BM * BN) + wn * 8192);
+#pragma unroll
+        for (int wn = 0; wn < 4; ++wn)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[wn][e] += v[wn][e];
+    }
+#pragma unroll
+    for (int wn = 0; wn < 4; ++wn) *reinterpret_cast<f32x4*>(sums + (l & 31) * REDP + wn * 32 + 8 * q + 4 * (l >> 5)) = sum[wn];
+    sync();
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int row = it * 16 + (t >> 4), col = (t & 15) * 8;
+        const int m = tmi * BM + a * 128 + wm * 64 + i * 32 + row, n = tn * BN + b * 128 + col;
+        if (m >= p.M || n >= p.N) continue;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            v[e] = aria_epilogue_act(p, sums[row * REDP + col + e] + (p.bias && n + e < p.N ? bf2f(p.bias[n + e]) : 0.f));
+        if (!p.c_f32 && p.wide_store && n + 8 <= p.N) {
+            bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n;
+            if (p.accumulate) {
+                const u32x4 o = ld16(d);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[2 * e] += bflo(o[e]), v[2 * e + 1] += bfhi(o[e]);
+            }
+            st16(d, u32x4{pack2bf(v[0], v[1]), pack2bf(v[2], v[3]), pack2bf(v[4], v[5]), pack2bf(v[6], v[7])});
+            continue;
         }
-        const int m = tmi * BM + row;
-        if (m >= p.M) continue;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int n = tn * BN + col0 + e;
-            if (n >= p.N) continue;
-            const float bv = p.bias ? bf2f(p.bias[n]) : 0.f;
-            float v = aria_epilogue_act(p, sum[e] + bv);
+        for (int e = 0; e < 8; ++e) {
+            if (n + e >= p.N) continue;
             if (p.c_f32) {
-                float* d = static_cast<float*>(p.C) + (long long)m * p.ldc + n;
-                *d = p.accumulate ? *d + v : v;
+                float* d = static_cast<float*>(p.C) + (long long)m * p.ldc + n + e;
+                *d = p.accumulate ? *d + v[e] : v[e];
             } else {
-                bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n;
-                if (p.accumulate) v += bf2f(*d);
-                *d = f2bf(v);
+                bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n + e;
+                *d = f2bf(p.accumulate ? v[e] + bf2f(*d) : v[e]);
             }
         }
     }

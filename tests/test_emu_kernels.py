@@ -318,7 +318,7 @@ def test_gemm_accumulate_into_bf16_is_one_rounding(M, N, K, b_oc, monkeypatch):
     C.case_gemm_accumulate_exact(DEV, M, N, K, b_oc)
 
 
-@pytest.mark.parametrize("M,N,K,a_oc,b_oc", [(512, 512, 2048, False, False), (300, 520, 1536, False, True), (256, 264, 1024, True, True)])
+@pytest.mark.parametrize("M,N,K,a_oc,b_oc", [(512, 512, 2048, False, False), (300, 520, 1536, False, True), (256, 264, 1024, True, True), (40, 264, 3072, False, False)])
 def test_gemm_split_k_slabs_in_accumulator_order(M, N, K, a_oc, b_oc):
     C.case_gemm_split_k_slabs(DEV, M, N, K, a_oc, b_oc)
 
