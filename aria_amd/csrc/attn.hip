@@ -188,11 +188,28 @@ __device__ __forceinline__ void tile2_store(const Chunks2<HD, NW>& r, bf16_t* s,
     }
 }
 
+// Blocks of two heights (no causal mask): a (b, head)'s first `whole` blocks hold QB queries, the others PB.  An XCD runs the whole blocks of all its (b, head)
+// pairs first, then the lower ones: those fill the last round.
+__device__ __forceinline__ bool attn_part_coords(int Sq, int QB, int whole, int PB, int H, int B, int& q0, int& q_end, int& head, int& b) {
+    const int nbh = H * B, pairs = (nbh + 7) >> 3, xcd = blockIdx.x & 7, n = blockIdx.x >> 3;
+    const int parts = max(0, Sq - whole * QB + PB - 1) / PB;
+    const bool first = n < pairs * whole;
+    const int j = first ? n : n - pairs * whole, per = first ? whole : parts;
+    if (!first && j >= pairs * parts) return false;
+    const int bh = (j / per) * 8 + xcd, blk = j % per;
+    if (bh >= nbh) return false;
+    q0 = first ? blk * QB : whole * QB + blk * PB;
+    q_end = min(Sq, q0 + (first ? QB : PB));
+    head = bh % H;
+    b = bh / H;
+    return true;
+}
+
 template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, const bf16_t* K, const bf16_t* V, bf16_t* O, float* LSE,
                                                         const int32_t* kv_len, const uint8_t* key_mask, int Sq, int S, int H,
                                                         long long ldq, long long ldk, long long ldv, long long ldo, float scale,
-                                                        int causal, int nbatch) {
+                                                        int causal, int nbatch, int whole, int part_waves) {
     using C = Cfg2<HD, NW>;
     ARIA_DYN_SMEM(smem);
     bf16_t* sK = reinterpret_cast<bf16_t*>(smem);          // [2][64][KP]
@@ -200,15 +217,21 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, con
     uint8_t* sM = reinterpret_cast<uint8_t*>(sV + 2 * 64 * C::VP);  // [2][64]
     int* sFlag = reinterpret_cast<int*>(sM + 128);         // [2]
     const int t = threadIdx.x, l = t & 63, w = t >> 6, h2 = l >> 5;
-    int qblk, head, b;
-    if (!attn_block_coords((Sq + C::QB - 1) / C::QB, H, nbatch, causal, true, qblk, head, b)) return;
-    const int q0 = qblk * C::QB;
+    int q0, q_end, head, b;
+    if (part_waves) {
+        if (!attn_part_coords(Sq, C::QB, whole, 32 * part_waves, H, nbatch, q0, q_end, head, b)) return;
+    } else {
+        int qblk;
+        if (!attn_block_coords((Sq + C::QB - 1) / C::QB, H, nbatch, causal, true, qblk, head, b)) return;
+        q0 = qblk * C::QB, q_end = min(Sq, q0 + C::QB);
+    }
     const long long tok0 = (long long)b * S, tokq0 = (long long)b * Sq;
     const bf16_t* Qb = Q + tokq0 * ldq + head * HD;
     const bf16_t* Kb = K + tok0 * ldk + head * HD;
     const bf16_t* Vb = V + tok0 * ldv + head * HD;
     const uint8_t* kmb = key_mask ? key_mask + tok0 : nullptr;
     const int q_wmin = q0 + 32 * w, q_abs = q_wmin + (l & 31);
+    const bool working = q_wmin < q_end;   // (wave-uniform: the others only help to stage the tiles)
     const int klen = kv_len ? min(S, kv_len[b]) : S;
     const float scale2 = scale * 1.4426950408889634f;
 
@@ -217,7 +240,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, con
     for (int kk = 0; kk < C::KS; ++kk) {
         u32x4 v = zero16();
         const int col = kk * 16 + h2 * 8;
-        if (q_abs < Sq && col < HD) v = ld16(Qb + (long long)q_abs * ldq + col);
+        if (q_abs < q_end && col < HD) v = ld16(Qb + (long long)q_abs * ldq + col);
         qf[kk] = __builtin_bit_cast(s16x8, v);
     }
 #pragma unroll
@@ -265,7 +288,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, con
         const bf16_t* cV = sV + cur * 64 * C::VP;
         // (a tile without a single valid key -- the padded bottom rows of an image are one contiguous patch range -- contributes exactly
         // nothing: every probability is exp2(-inf) = 0 and the running maximum does not move)
-        if (!(causal && kv0 > q_wmin + 31) && !(kmb && (sFlag[cur] & 2))) {  // wave-uniform: this wave has at least one visible key in the tile
+        if (working && !(causal && kv0 > q_wmin + 31) && !(kmb && (sFlag[cur] & 2))) {  // wave-uniform: this wave has at least one visible key in the tile
             f32x16 st[2];
             st[0] = zero_acc();
             st[1] = zero_acc();
@@ -389,7 +412,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, con
     // ROWSUM_IN_MFMA: feature row HD = 32 (DT-1) + 8 sits in accumulator register 4 of the lanes with h2 == 0
     const float ltot = C::ROWSUM_IN_MFMA ? shfl(o[C::DT - 1][4], l & 31) : lsum + shfl_xor(lsum, 32);
     const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-    if (q_abs < Sq) {
+    if (q_abs < q_end) {
         if (h2 == 0 && LSE)
             LSE[((long long)b * H + head) * Sq + q_abs] = (ltot > 0.f) ? (m + log2f(ltot)) * 0.6931471805599453f : -INFINITY;
         bf16_t* orow = O + (tokq0 + q_abs) * ldo + head * HD;
@@ -1544,6 +1567,36 @@ thread_local int g_last_fwd_variant = 0;  // 2: attn_fwd2 (staged through regist
 thread_local int g_last_bwd_variant = 0;  // 2: the padded-tile pair (hd 64 / 72), 5: role-split dK/dV + dQ v5 (hd 128) -- tests assert which ran
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+struct Plan72 {
+    int whole = 0, part_waves = 0;   // blocks of 12 waves a (b, head), waves of its other blocks (0: only blocks of 12)
+    unsigned grid = 0;
+};
+// One block of 12 waves runs on a CU at a time, so a launch takes whole rounds of 32 blocks an XCD, and a (b, head)'s queries are cut to fill the last one: `whole`
+// blocks of 384 queries for the first rounds, blocks of 256 or 128 (8 or 4 of the 12 waves compute) for the rest.  A round of those costs 0.84 and 0.62 of a
+// whole one (4900 keys, 16 heads: 150, 125 and 93 us; one wave a SIMD waits for its own chain), so the plan is the cheapest sum of rounds.  Measured, microseconds,
+// only whole blocks / planned: 4900 queries of 2, 3, 4 images 303 / 280, 463 / 436, 622 / 571; 1225 queries of 1, 2, 3 images 43.7 / 27.6, 44.8 / 36.8,
+// 47.9 / 40.2; one image of 4900 and four of 1225 fit one round.
+Plan72 plan72(int64_t Sq, int64_t pairs) {
+    Plan72 best;
+    const int64_t tiles = (Sq + 31) / 32, per = (pairs + 7) / 8, rounds = ((tiles + 11) / 12 * per + 31) / 32;
+    double cost = 0.97 * double(rounds);   // (a plan has to be worth 3 %)
+    for (int64_t r = rounds > 5 ? rounds - 5 : 0; r < rounds; ++r) {
+        const int64_t whole = std::min(r * 32 / per, tiles / 12), rest = tiles - 12 * whole;
+        if (rest <= 0) continue;
+        const int64_t used = (whole * per + 31) / 32;
+        for (int waves = 4; waves <= 8; waves += 4) {
+            const int64_t parts = (rest + waves - 1) / waves;
+            const double c = double(used) + (waves == 4 ? 0.62 : 0.84) * double((parts * per + 31) / 32);
+            if (c < cost) {
+                cost = c;
+                best.whole = int(whole), best.part_waves = waves;
+                best.grid = unsigned(8 * per * (whole + parts));
+            }
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1576,19 +1629,21 @@ int aria_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
     else if (hd == 128)
         ARIA_LAUNCH((attn_fwd2_kernel<128, 8>), dim3(attn_grid((Sq + 255) / 256, H, B)), dim3(512), size_t(Cfg2<128>::SMEM), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
-                    (long long)ldv, (long long)ldo, scale, causal, int(B));
+                    (long long)ldv, (long long)ldo, scale, causal, int(B), 0, 0);
     else if (hd == 72 && nw72 && nw72[0] == '8')
         ARIA_LAUNCH((attn_fwd2_kernel<72, 8>), dim3(attn_grid((Sq + 255) / 256, H, B)), dim3(512), size_t(Cfg2<72>::SMEM), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
-                    (long long)ldv, (long long)ldo, scale, causal, int(B));
-    else if (hd == 72)
-        ARIA_LAUNCH((attn_fwd2_kernel<72, 12>), dim3(attn_grid((Sq + 383) / 384, H, B)), dim3(768), size_t(Cfg2<72>::SMEM), stream, Q, K, V,
+                    (long long)ldv, (long long)ldo, scale, causal, int(B), 0, 0);
+    else if (hd == 72) {
+        const Plan72 pl = causal ? Plan72{} : plan72(Sq, H * B);
+        const unsigned grid = pl.part_waves ? pl.grid : attn_grid((Sq + 383) / 384, H, B);
+        ARIA_LAUNCH((attn_fwd2_kernel<72, 12>), dim3(grid), dim3(768), size_t(Cfg2<72>::SMEM), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
-                    (long long)ldv, (long long)ldo, scale, causal, int(B));
-    else
+                    (long long)ldv, (long long)ldo, scale, causal, int(B), pl.whole, pl.part_waves);
+    } else
         ARIA_LAUNCH((attn_fwd2_kernel<64, 8>), dim3(attn_grid((Sq + 255) / 256, H, B)), dim3(512), size_t(Cfg2<64>::SMEM), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
-                    (long long)ldv, (long long)ldo, scale, causal, int(B));
+                    (long long)ldv, (long long)ldo, scale, causal, int(B), 0, 0);
     return aria_check_launch();
 }
 

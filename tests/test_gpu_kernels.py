@@ -96,7 +96,8 @@ def test_attention_with_whole_key_tiles_masked(hd, H, S):
     C.case_attention_masked_tiles(DEV, hd, H, S=S)
 
 
-@pytest.mark.parametrize("B,Sq,Skv,H,masked", [(2, 70, 70, 2, True), (1, 300, 90, 1, False), (2, 4900, 4900, 4, True), (3, 256, 4900, 16, True)])
+@pytest.mark.parametrize("B,Sq,Skv,H,masked", [(2, 70, 70, 2, True), (1, 300, 90, 1, False), (2, 4900, 4900, 4, True), (3, 256, 4900, 16, True),
+                                              (17, 450, 70, 8, True), (5, 1500, 70, 16, True), (1, 1225, 130, 16, False)])   # (blocks of two heights; of 4 waves only)
 def test_attention_hd72_forward(B, Sq, Skv, H, masked):
     C.case_attention_hd72_forward(DEV, B, Sq, Skv, H, masked)
 
