@@ -28,6 +28,7 @@
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "gemm_params.h"
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
@@ -340,8 +341,11 @@ bool use_v2(long long tiles256) {
 
 // v3 (LDS-DMA staged, phase-scheduled 256x256 tile, gemm3.hip): the operand byte offsets must fit 32 bits.
 // ARIA_GEMM_FORCE=3 pins it where eligible.
+bool fits_dma(long long K, long long bytesA, long long bytesB, long long extentA, long long extentB) {
+    return K >= 64 && bytesA < (1ll << 32) && bytesB < (1ll << 32) && extentA >= 8 && extentB >= 8;
+}
 bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB, long long extentA, long long extentB, long long least = 192) {
-    if (K < 64 || bytesA >= (1ll << 32) || bytesB >= (1ll << 32) || extentA < 8 || extentB < 8) return false;
+    if (!fits_dma(K, bytesA, bytesB, extentA, extentB)) return false;
     const char* force = std::getenv("ARIA_GEMM_FORCE");
     if (force) return force[0] == '3';
     return tiles256 >= least;
@@ -352,6 +356,13 @@ bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB,
 // Rows by expert: where they fill a third of a tile and more.  128 x 128 / 256 x 256, 150 .. 191 tiles: 64 experts of 2560 x 1664: 60 rows each on average 132 / 146, 72 134 /
 // 140; 3328 x 2560: 48 rows 248 / 277; 32 experts of 3328 x 2560: 88 rows 173 / 145; 64 of 1536 x 1024: 96 rows 76 / 54; 16 of 2560 x 1664: 240 rows 83 / 47.
 constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150, V3_FEW_ROWS = 84;
+// the LDS-DMA kernels: the four-wave tiles where their plan takes the product, the 256 x 256 ones elsewhere (rows: see aria_plan_gemm4)
+int launch_large(const GemmParams& p, int a_oc, int b_oc, int ntm, void* stream, void* workspace = nullptr, long long workspace_bytes = 0, long long rows = -1) {
+    const int split3 = p.mode == 0 && workspace ? aria_gemm3_split(p.M, p.N, p.K) : 1;
+    const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, rows, split3, workspace ? workspace_bytes : 0);
+    if (plan.form) return aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
+    return aria_launch_gemm3(p, a_oc, b_oc, ntm, stream, workspace, workspace_bytes);
+}
 long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
 }  // namespace
@@ -362,7 +373,7 @@ int aria_last_gemm_variant(void) { return g_last_variant; }
 
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc) {
     if (M <= 0 || N <= 0 || (a_oc && !b_oc)) return 0;
-    return aria_gemm3_workspace_bytes(M, N, K);
+    return std::max(aria_gemm3_workspace_bytes(M, N, K), a_oc ? 0 : aria_gemm4_workspace_bytes(M, N, K));
 }
 
 int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
@@ -414,8 +425,13 @@ int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, 
     // with a workspace the partly filled last round of tiles is split along K (gemm3.hip), so small outputs fill the chip too
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
+    const bool strides = 2 * lda < (1ll << 24) && 2 * ldb < (1ll << 24);
+    if ((!a_oc || b_oc) && strides && fits_dma(K, bytesA, bytesB, M, N)) {
+        const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0);
+        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
+    }
     if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
-        return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
+        return g_last_variant = 3, launch_large(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
 }
@@ -450,9 +466,13 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const int gmask = gsel ? std::atoi(gsel) : GROUPED_V3_DEFAULT;
     const char* gforce = std::getenv("ARIA_GEMM_FORCE");
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
+    if (fits_dma(K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N) && 2 * lda < (1ll << 24) && 2 * ldb < (1ll << 24)) {
+        const Gemm4Plan plan = aria_plan_gemm4(p, 0, b_oc, -1, 1, 0);
+        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 0, b_oc, plan, nullptr, stream);
+    }
     if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
                       v3_least(K, M_total >= V3_FEW_ROWS * E ? V3_FEW_TILES_GROUPED : 192)))
-        return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc, int(M_total / 256 + E), stream);
+        return g_last_variant = 3, launch_large(p, 0, b_oc, int(M_total / 256 + E), stream);
     if (use_v2((M_total / 256 + 1) * ((N + 255) / 256))) return g_last_variant = 2, aria_launch_gemm2(p, 0, b_oc, int(M_total / 256 + E), 1, stream);
     return g_last_variant = 1, launch_gemm(p, 0, b_oc, p.ntn * max_tm, 1, stream);
 }
@@ -489,7 +509,7 @@ int aria_grouped_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* A
     p.E = int(E);
     p.strideB = strideB;
     p.glu = 1;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 1, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb,
@@ -507,7 +527,7 @@ int aria_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* ACT, int6
     p.M = int(M), p.N = int(N2), p.K = int(K);
     p.mode = 0;
     p.glu = 1;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 int aria_gemm_relu_glu_bf16(const void* A, const void* B, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb, int64_t ldact, void* stream) {
@@ -523,7 +543,7 @@ int aria_gemm_relu_glu_bf16(const void* A, const void* B, void* ACT, int64_t M, 
     p.M = int(M), p.N = int(N2), p.K = int(K);
     p.mode = 0;
     p.glu = 2;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // gate / up weights as two [.., I, K] tensors of one allocation (gptfast's w1 / w3): rows of the up tensor as an offset from the gate tensor
@@ -562,7 +582,7 @@ int aria_grouped_gemm_swiglu_split_bf16(const void* A, const void* Bg, const voi
     p.strideB = strideB;
     p.glu = 1;
     p.glu_up_rows = up_rows;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_swiglu_split_bf16(const void* A, const void* Bg, const void* Bu, void* H, void* ACT, int64_t M, int64_t I, int64_t K, int64_t lda,
@@ -586,7 +606,7 @@ int aria_gemm_swiglu_split_bf16(const void* A, const void* Bg, const void* Bu, v
     p.mode = 0;
     p.glu = 1;
     p.glu_up_rows = up_rows;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // Expert parallelism: grouped launches over the SEGMENTS of an all-to-all's output (ordered (source rank, local expert)): segment g uses
@@ -612,7 +632,7 @@ int aria_grouped_gemm_seg_bf16(const void* A, const void* B, void* C, const int3
     p.E = int(n_seg);
     p.strideB = strideB;
     p.expert_mod = int(n_local);
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc, int(M_total / 256 + n_seg), stream);
+    return g_last_variant = 3, launch_large(p, 0, b_oc, int(M_total / 256 + n_seg), stream);
 }
 
 int aria_grouped_gemm_swiglu_seg_bf16(const void* A, const void* B, void* H, void* ACT, const int32_t* offsets, int64_t n_seg, int64_t n_local,
@@ -637,7 +657,7 @@ int aria_grouped_gemm_swiglu_seg_bf16(const void* A, const void* B, void* H, voi
     p.strideB = strideB;
     p.glu = 1;
     p.expert_mod = int(n_local);
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 1, int(M_total / 256 + n_seg), stream);
+    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + n_seg), stream);
 }
 
 // K2: the two fused SwiGLU launches over grouped rows with the dispatcher's gather folded into the A loader.  X is the un-permuted token
@@ -664,7 +684,7 @@ int aria_grouped_gemm_swiglu_gather_bf16(const void* X, const int32_t* rows, int
     p.strideB = strideB;
     p.glu = 1;
     p.gather_rows = rows;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 1, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_swiglu_split_gather_bf16(const void* X, const int32_t* rows, int64_t T, const void* Bg, const void* Bu, void* H, void* ACT,
@@ -693,7 +713,7 @@ int aria_grouped_gemm_swiglu_split_gather_bf16(const void* X, const int32_t* row
     p.glu = 1;
     p.glu_up_rows = up_rows;
     p.gather_rows = rows;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 // K7: wqkv projection + interleaved RoPE + KV-cache write in one launch (gptfast/model.py:413-435, 67-93).
@@ -721,7 +741,7 @@ int aria_gemm_qkv_rope_cache_bf16(const void* X, const void* Wqkv, void* Q, void
     p.rope_hd = int(hd), p.rope_D = int(D), p.rope_S = int(S), p.cache_S = int(S_cache);
     p.kc = Kc, p.vc = Vc;
     p.ld_cache = ld_cache;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // The HF layer's q | k | v projection + half-split RoPE in one launch (LlamaAttention.forward, modeling_llama.py:243-281, 130-160)
@@ -743,7 +763,7 @@ int aria_gemm_qkv_rope_hf_bf16(const void* X, const void* Wqkv, void* QKV, const
     p.rope_fc = static_cast<const bf16_t*>(cos);
     p.rope_sn = static_cast<const bf16_t*>(sin);
     p.rope_hd = int(hd), p.rope_D = int(D), p.rope_S = int(S);
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // shared validation of the fused input-gradient + SwiGLU-backward entries (gemm3_kernel<.., .., 5>)
@@ -775,7 +795,7 @@ int aria_grouped_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H,
     p.E = int(E);
     p.strideB = strideB;
     p.dglu = 1;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* DH, int64_t M, int64_t I, int64_t K, int b_oc, int64_t lda,
@@ -793,7 +813,7 @@ int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* D
     p.M = int(M), p.N = int(I), p.K = int(K);
     p.mode = 0;
     p.dglu = 1;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
 }
 
 // The weight gradient of experts.fc1 WITHOUT the permuted copy of the tokens (moe_lm.py:326-334: permuted = x.index_select(0, sorted // topk)):
@@ -801,6 +821,11 @@ int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* D
 // permuted row; the 64 entries of padding are read, never used).  v3 only.
 int aria_grouped_gemm_wgrad_gather_bf16(const void* X, const int32_t* rows, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t T,
                                         int64_t K, int64_t N, int64_t ldx, int64_t ldy, int c_f32, int accumulate, void* stream) {
+    return aria_grouped_gemm_wgrad_gather_sized_bf16(X, rows, dY, dW, offsets, E, T, K, N, ldx, ldy, c_f32, accumulate, -1, stream);
+}
+
+int aria_grouped_gemm_wgrad_gather_sized_bf16(const void* X, const int32_t* rows, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t T,
+                                              int64_t K, int64_t N, int64_t ldx, int64_t ldy, int c_f32, int accumulate, int64_t M_total, void* stream) {
     // T == 0 (no tokens: every expert's reduction is empty) is a valid call like its sibling aria_grouped_gemm_wgrad_bf16's: dW is
     // zero-filled (or left alone with `accumulate`)
     if (!dW || !offsets || E <= 0 || T < 0 || K < 0 || N < 0) return ARIA_ERR_INVALID;
@@ -816,7 +841,9 @@ int aria_grouped_gemm_wgrad_gather_bf16(const void* X, const int32_t* rows, cons
     }
     if (!X || !rows || !dY) return ARIA_ERR_INVALID;
     if (!aligned16(X) || !aligned16(dY) || (ldx & 7) || (ldy & 7) || (K & 7) || (N & 7) || (reinterpret_cast<uintptr_t>(rows) & 3)) return ARIA_ERR_ALIGN;
-    if (T >= (1ll << 24) || 2 * ldx >= (1ll << 24) || 2 * T * ldx >= (1ll << 32) || !use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, 0, 0, K, N))
+    const char* force4 = std::getenv("ARIA_GEMM_FORCE");
+    if (T >= (1ll << 24) || 2 * ldx >= (1ll << 24) || 2 * T * ldx >= (1ll << 32) ||
+        !(use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, 0, 0, K, N) || (force4 && force4[0] == '4' && K >= 8 && N >= 8)))
         return ARIA_ERR_UNSUPPORTED;
     GemmParams p{};
     p.A = static_cast<const bf16_t*>(X);
@@ -832,7 +859,7 @@ int aria_grouped_gemm_wgrad_gather_bf16(const void* X, const int32_t* rows, cons
     p.accumulate = accumulate;
     p.gather_rows = rows;
     p.ntn = int((N + BN - 1) / BN);
-    return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream, nullptr, 0, 2 * ldy < (1ll << 24) ? M_total : -1);
 }
 
 // ---- LoRA as a K-extension of the base GEMM (GemmParams::ext_k; aria/lora/layers.py:129-139, peft's Linear adapter): v3 only -- shapes the
@@ -864,7 +891,7 @@ int aria_gemm_lora_bf16(const void* A, const void* B, void* C, int64_t M, int64_
     const long long t256 = ((M + 255) / 256) * ((N + 255) / 256);
     if (!use_v3(t256, K, 2 * M * lda, 2 * (b_oc ? K * ldb : N * ldb), M, N) || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24))
         return ARIA_ERR_UNSUPPORTED;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
 }
 
 int aria_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb,
@@ -883,7 +910,7 @@ int aria_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT,
     p.glu = 1;
     rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, 0);
     if (rc != ARIA_OK) return rc;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 int aria_grouped_gemm_lora_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total, int64_t N, int64_t K,
@@ -906,7 +933,7 @@ int aria_grouped_gemm_lora_bf16(const void* A, const void* B, void* C, const int
     if (!use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N) ||
         2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24))
         return ARIA_ERR_UNSUPPORTED;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc ? 1 : 0, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT, const int32_t* offsets, int64_t E, int64_t M_total,
@@ -931,11 +958,16 @@ int aria_grouped_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, vo
     p.glu = 1;
     rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, stride_eb);
     if (rc != ARIA_OK) return rc;
-    return g_last_variant = 3, aria_launch_gemm3(p, 0, 1, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_wgrad_bf16(const void* A, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t K,
                                  int64_t N, int64_t lda, int64_t ldy, int c_f32, int accumulate, void* stream) {
+    return aria_grouped_gemm_wgrad_sized_bf16(A, dY, dW, offsets, E, K, N, lda, ldy, c_f32, accumulate, -1, stream);
+}
+
+int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t K, int64_t N, int64_t lda, int64_t ldy,
+                                       int c_f32, int accumulate, int64_t M_total, void* stream) {
     if (!A || !dY || !dW || !offsets || E <= 0) return ARIA_ERR_INVALID;
     if (K == 0 || N == 0) return ARIA_OK;
     if (!aligned16(A) || !aligned16(dY) || (lda & 7) || (ldy & 7) || (K & 7) || (N & 7)) return ARIA_ERR_ALIGN;
@@ -957,6 +989,10 @@ int aria_grouped_gemm_wgrad_bf16(const void* A, const void* dY, void* dW, const 
     p.accumulate = accumulate;
     p.ntn = int((N + BN - 1) / BN);
     const int ntm = int((K + BM - 1) / BM);
+    if (K >= 8 && N >= 8 && 2 * lda < (1ll << 24) && 2 * ldy < (1ll << 24)) {
+        const Gemm4Plan plan = aria_plan_gemm4(p, 1, 1, M_total, 1, 0);
+        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 1, 1, plan, nullptr, stream);
+    }
     // (the reduction length is per expert and data dependent: 64 stands in for "long enough" in the eligibility test)
     // both operands are token-major (output-contiguous): their per-lane DMA offsets stay inside one 64-token tile, no 4 GiB limit
     // Measured on MI355X (98304 routed rows, 64 experts): v3 749 TF/s vs v2 800-830 on these short (~24 K-tile) reductions with two
@@ -965,7 +1001,7 @@ int aria_grouped_gemm_wgrad_bf16(const void* A, const void* dY, void* dW, const 
     // r02: with the wide epilogue v3 is level with v2 here too (in-bench 710.3 vs 714.6 ms/step); ARIA_GEMM_WGRAD_V3=0 goes back to v2
     const char* wg3 = std::getenv("ARIA_GEMM_WGRAD_V3");
     if (((force3 && force3[0] == '3') || !(wg3 && wg3[0] == '0')) && !(force3 && (force3[0] == '1' || force3[0] == '2')) && use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, 0, 0, K, N))
-        return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
+        return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream);
     if (use_v2(((K + 255) / 256) * ((N + 255) / 256) * E)) return g_last_variant = 2, aria_launch_gemm2(p, 1, 1, int((K + 255) / 256), int(E), stream);
     return g_last_variant = 1, launch_gemm(p, 1, 1, p.ntn * ntm, int(E), stream);
 }

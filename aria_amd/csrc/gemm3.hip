@@ -1135,33 +1135,7 @@ __global__ __launch_bounds__(256) void gemm3_reduce_kernel(GemmParams p) {
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
         const int row = it * 16 + (t >> 4), col = (t & 15) * 8;
-        const int m = tmi * BM + a * 128 + wm * 64 + i * 32 + row, n = tn * BN + b * 128 + col;
-        if (m >= p.M || n >= p.N) continue;
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-            v[e] = aria_epilogue_act(p, sums[row * REDP + col + e] + (p.bias && n + e < p.N ? bf2f(p.bias[n + e]) : 0.f));
-        if (!p.c_f32 && p.wide_store && n + 8 <= p.N) {
-            bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n;
-            if (p.accumulate) {
-                const u32x4 o = ld16(d);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[2 * e] += bflo(o[e]), v[2 * e + 1] += bfhi(o[e]);
-            }
-            st16(d, u32x4{pack2bf(v[0], v[1]), pack2bf(v[2], v[3]), pack2bf(v[4], v[5]), pack2bf(v[6], v[7])});
-            continue;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            if (n + e >= p.N) continue;
-            if (p.c_f32) {
-                float* d = static_cast<float*>(p.C) + (long long)m * p.ldc + n + e;
-                *d = p.accumulate ? *d + v[e] : v[e];
-            } else {
-                bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n + e;
-                *d = f2bf(p.accumulate ? v[e] + bf2f(*d) : v[e]);
-            }
-        }
+        aria_finish_sums(p, sums + row * REDP + col, tmi * BM + a * 128 + wm * 64 + i * 32 + row, tn * BN + b * 128 + col);
     }
 }
 
@@ -1198,6 +1172,12 @@ long long aria_gemm3_workspace_bytes(long long M, long long N, long long K) {
     long long R = 0;
     const int S = plan_split(((M + 255) / 256) * ((N + 255) / 256), (K + 63) / 64, &R);
     return S > 1 ? R * S * (long long)(BM * BN) * 4 : 0;
+}
+
+int aria_gemm3_split(long long M, long long N, long long K) {
+    long long R = 0;
+    const long long tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    return tiles < 256 && aria_gemm3_workspace_bytes(M, N, K) > 0 ? plan_split(tiles, (K + 63) / 64, &R) : 1;
 }
 
 // v3 eligibility is decided by the caller (gemm.hip): K % 64 == 0, K >= 64, mode 0 or 1, operand bytes < 4 GiB

@@ -1,0 +1,640 @@
+// GEMM with four waves, one a SIMD, for the products whose tiles of 256 x 256 leave CUs idle or stand half empty.  Three forms, by what bounds them:
+//
+//   tiles of 128 x 256, stages 64 deep, three of them (144 KiB), one workgroup a CU: outputs of up to one round, and rows by expert of a few dozen
+//   tiles of 256 x 160 ([N, K] weights) or 128 x 320 ([K, N]): outputs of one round whose 256 x 256 tiles would fill only part of it
+//   tiles of 128 x 256, stages 32 deep, two workgroups a CU: weight gradients with short reductions, where a tile's start and its stores are the time and the
+//     other workgroup's work hides them
+//
+// Geometry.  Wave (wm, wn) of WM x WN owns rows {i * 32 WM + 32 wm + [0, 32)} x columns {b * 32 WN + 32 wn + [0, 32)} of the tile, i < MI, b < NI, as
+// v_mfma_f32_32x32x16_bf16 tiles with transposed accumulators (mfma(B fragment, A fragment): a lane owns four consecutive columns of one row a register group).
+// Large wave tiles keep the LDS reads below the matrix work: 128 x 64 a wave reads 24 KiB for 1024 cycles of products (eight waves of 64 x 64: 32 KiB).
+//
+// The reduction goes through S stages in the LDS, KD deep, filled by LDS-DMA, in sixteenths (one MFMA step).  While the products of one sixteenth run, the fragments
+// of the next are read and pieces of stage t + S - 1 requested, one behind each product (in front of the products a wave's issue of the pieces took as long as the
+// products).  Before the last sixteenth every wave holds its fragments, stage t + 1 has landed, and one s_barrier frees stage t's buffer.  A fragment never crosses a
+// branch or the loop's back edge before it has arrived.
+//
+// What bounds the loop is the CU's rate of fetching lines: 777 x 2560 x 5120 on 70 CUs, a step of 32: the products alone 0.21 us, with every fragment read 0.22, with pieces
+// from one fixed place 0.26, with the operands 0.30 .. 0.36.  A row operand ([rows][k]) in stages 32 deep fetches every 128-byte line twice (64 bytes, then the others): 0.355
+// against 0.27 in stages 64 deep; 8192^3 1070 and 913 us.
+//
+// LDS images of a stage: A rows, then B rows.
+//   rc operand ([rows][k]): a row = 2 KD bytes; its 16-byte chunk c lies at c ^ ((r >> 2) & 3) (KD 32) or c ^ ((r >> 1) & 7): the 16 rows of a ds_read_b128 group hit
+//     16 different 16-byte bank groups.  A DMA piece (1 KiB) is 16 or 8 rows.
+//   oc operand ([k][rows]): units of 64 rows, [KD][128 bytes]; 32-byte chunk c of k-row k lies at c ^ 2 ((k >> 1) & 1): the 32 lanes of a transposing read's half
+//     wave (four k-rows, two chunks) hit eight different 32-byte bank groups.  A piece is 8 k-rows of a unit.
+// The order of the products of an output element is that of the 256 x 256 kernel: the same bits where neither splits the reduction.
+#include "aria_hip.h"
+#include "gemm_params.h"
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+#include <utility>
+
+namespace {
+using namespace ad;
+
+__device__ const uint32_t zero_page4[64] = {};   // the source of granules beyond the end of the reduction
+
+template <int OFF>
+__device__ __forceinline__ s16x8 lds_b128(const char* smem, uint32_t at) {   // (the caller waits before the first use)
+#ifdef ARIA_EMU
+    return *reinterpret_cast<const s16x8*>(smem + at + OFF);
+#else
+    s16x8 f;
+    const uint32_t a = uint32_t(reinterpret_cast<uintptr_t>(smem)) + at;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(a), "n"(OFF));
+    return f;
+#endif
+}
+template <int OFF>
+__device__ __forceinline__ s16x8 lds_tr(const char* smem, uint32_t at) {   // eight k-rows of one column; the rows lie 128 bytes apart
+#ifdef ARIA_EMU
+    const s16x4 a0 = ds_read_tr16(reinterpret_cast<const bf16_t*>(smem + at + OFF)), a1 = ds_read_tr16(reinterpret_cast<const bf16_t*>(smem + at + OFF + 512));
+#else
+    s16x4 a0, a1;
+    const uint32_t a = uint32_t(reinterpret_cast<uintptr_t>(smem)) + at;
+    asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4" : "=&v"(a0), "=&v"(a1) : "v"(a), "n"(OFF), "n"(OFF + 512));
+#endif
+    return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// fragment addresses of one operand in stages of KD: W waves side by side, this one at `wi`
+template <bool OC, int W, int KD>
+struct Frag {
+    static constexpr int UNIT = KD * 128;   // bytes of 64 rows
+    uint32_t v[2];
+    __device__ __forceinline__ void init(int wi, int l) {
+        if (!OC) {
+            const int swap = KD == 32 ? (l >> 2) & 3 : (l >> 1) & 7;
+            v[0] = uint32_t((wi * 32 + (l & 31)) * (2 * KD) + (((l >> 5) ^ swap) << 4));
+            v[1] = 0;
+        } else {
+            const int k = 8 * (l >> 5) + ((l & 15) >> 2), f = ((l & 15) >> 3) << 1, first = wi * 32;
+            const uint32_t at = uint32_t((first >> 6) * UNIT + k * 128 + 8 * (l & 3));
+            v[0] = at + uint32_t(((((first & 32) >> 4) + ((l >> 4) & 1)) ^ f) << 5);
+            v[1] = at + uint32_t(((2 + ((l >> 4) & 1)) ^ f) << 5);   // (W == 1: the odd 32-row tiles)
+        }
+    }
+    // rows I * 32 W + 32 wi + (l & 31), k = 16 KK + 8 (l >> 5) + 0..7 of the image at `base`
+    template <int I, int KK>
+    __device__ __forceinline__ s16x8 read(const char* smem, uint32_t base) const {
+        if (!OC) return lds_b128<I * W * 64 * KD>(smem, base + (v[0] ^ uint32_t(KK << 5)));
+        constexpr int OFF = (I * W * 32 / 64) * UNIT + KK * 2048;
+        return lds_tr<OFF>(smem, base + v[W == 1 ? I & 1 : 0]);
+    }
+};
+
+template <class F, size_t... I>
+__device__ __forceinline__ void each(F&& f, std::index_sequence<I...>) {
+    (f(std::integral_constant<int, int(I)>{}), ...);
+}
+
+template <int WM, int WN, int MI, int NI, int KD, int S>
+struct Shape4 {
+    static constexpr int BM = WM * MI * 32, BN = WN * NI * 32, PA = BM * KD / 2048, PB = BN * KD / 2048;   // pieces a wave and stage
+    static constexpr int STAGE = (BM + BN) * KD * 2, ROWP = BN * 2 + 16;                                   // bytes; pitch of the parked tile
+    static constexpr size_t SMEM = std::max(size_t(S) * STAGE, size_t(BM) * ROWP);
+};
+
+// VER: what happens to the tile (the numbers of gemm3_kernel): 3 plain (bias, activation, accumulation, 32-bit results), 5 SwiGLU backward, 6 / 9 fused SwiGLU on two
+// weight tensors (9: gathered rows), 8 on [K, N] weights with gathered rows, 14 on one [gate | up] tensor, 13 relu gate, 7 / 10 rotations,
+// 11 plain, with the reduction's rows of A reached through an index (per-expert weight gradients)
+constexpr bool gathers(int ver) { return ver == 8 || ver == 9; }   // (11: gathered rows of the reduction)
+constexpr bool gated(int ver) { return ver == 6 || ver == 8 || ver == 9 || ver == 13 || ver == 14; }
+
+// one 16-byte piece (8 columns) of the parked tile on its way out
+template <int VER, class P>
+__device__ __forceinline__ void finish_piece(const P& p, char* C, const char* parked, int m, int n0, int cc) {
+    u32x4 v = *reinterpret_cast<const u32x4*>(parked + cc * 2);
+    bf16_t* out = reinterpret_cast<bf16_t*>(C);
+    if (VER == 7) {   // interleaved rotation and the cache's rows (store_tile3_rows_rope of the 256 x 256 kernel)
+        const int region = n0 / p.rope_D, col = n0 - region * p.rope_D + cc;
+        const int seq = m / p.rope_S, ps = p.rope_pos ? p.rope_pos[m] : m - seq * p.rope_S;
+        if (region < 2) {
+            const u32x4 f = ld16(p.rope_fc + (long long)ps * p.rope_hd + col % p.rope_hd);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float x0 = bflo(v[q]), x1 = bfhi(v[q]), cs = bflo(f[q]), sn = bfhi(f[q]);
+                v[q] = pack2bf(x0 * cs - x1 * sn, x1 * cs + x0 * sn);
+            }
+        }
+        if (region == 0)
+            st16(out + (long long)m * p.ldc + col, v);
+        else if (unsigned(ps) < unsigned(p.cache_S))
+            st16(static_cast<bf16_t*>(region == 1 ? p.kc : p.vc) + ((long long)seq * p.cache_S + ps) * p.ld_cache + col, v);
+        return;
+    }
+    if (VER == 10) {   // half-split rotation: the partner columns lie in the same parked row
+        if (n0 < 2 * p.rope_D) {
+            const int half = p.rope_hd >> 1, fcol = (n0 + cc) % p.rope_hd, ps = m % p.rope_S;
+            const bool second = fcol >= half;
+            const u32x4 pv = *reinterpret_cast<const u32x4*>(parked + (second ? cc - half : cc + half) * 2);
+            const u32x4 fc = ld16(p.rope_fc + (long long)ps * p.rope_hd + fcol), fs = ld16(p.rope_sn + (long long)ps * p.rope_hd + fcol);
+            const float sg = second ? 1.f : -1.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                v[q] = pack2bf(rbf(bflo(v[q]) * bflo(fc[q])) + rbf(sg * bflo(pv[q]) * bflo(fs[q])),
+                               rbf(bfhi(v[q]) * bfhi(fc[q])) + rbf(sg * bfhi(pv[q]) * bfhi(fs[q])));
+        }
+        st16(out + (long long)m * p.ldc + n0 + cc, v);
+        return;
+    }
+    if (VER == 5) {   // v = d_act: gate and up of the same elements give their gradients
+        const bf16_t* h = p.H + (long long)m * p.ldh + n0 + cc;
+        const u32x4 g = ld16(h), u = ld16(h + p.N);
+        u32x4 og, ou;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            f32x2 da, db;
+            swiglu_bwd_pair(f32x2{bflo(g[q]), bfhi(g[q])}, f32x2{bflo(u[q]), bfhi(u[q])}, f32x2{bflo(v[q]), bfhi(v[q])}, da, db);
+            og[q] = pack2bf(da.x, da.y), ou[q] = pack2bf(db.x, db.y);
+        }
+        bf16_t* d = out + (long long)m * p.ldc + n0 + cc;
+        st16(d, og);
+        st16(d + p.N, ou);
+        return;
+    }
+    st16(out + (long long)m * p.ldc + n0 + cc, v);
+}
+
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
+    using T = Shape4<WM, WN, MI, NI, KD, S>;
+    constexpr int BM = T::BM, BN = T::BN, PA = T::PA, PB = T::PB, STAGE = T::STAGE, ROWP = T::ROWP, HALVES = KD / 16;
+    constexpr bool GATHER = gathers(VER), GLU = gated(VER), GATHER_K = VER == 11, PLAIN = VER == 3 || VER == 11;
+    ARIA_DYN_SMEM(smem);
+    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), wm = w / WN, wn = w % WN;
+
+    int tn = 0, tmi = 0, slab = -1, ks = 0;
+    if (p.mode == 1) {
+        // aria_grouped_tile below
+    } else if (p.split > 1) {
+        slab = blockIdx.x;
+        ks = slab % p.split;
+        if (!aria_tile_from_pos(p, slab / p.split, tmi, tn)) return;
+    } else if (!aria_tile_coords(p, blockIdx.x, int(gridDim.x), tmi, tn)) {
+        return;
+    }
+    constexpr int STEP = GLU ? BN / 2 : BN;
+    long long b_off = 0, c_off = 0;
+    int m0 = tmi * BM, m_end = p.M, k_begin = 0, k_len = p.K;
+    if (p.mode == 2) {
+        k_begin = p.offsets[blockIdx.y];
+        k_len = p.offsets[blockIdx.y + 1] - k_begin;
+        c_off = (long long)blockIdx.y * p.strideC;
+    } else if (p.mode == 1) {
+        int expert = 0;
+        if (!aria_grouped_tile<BM>(p, blockIdx.x, l, expert, m0, m_end, tn)) return;
+        expert = first_lane(expert), m0 = first_lane(m0), m_end = first_lane(m_end), tn = first_lane(tn);
+        b_off = (long long)(p.expert_mod > 0 ? expert % p.expert_mod : expert) * p.strideB;
+    }
+    const int n0 = tn * STEP;
+    char* C = static_cast<char*>(p.C) + c_off * (p.c_f32 ? 4 : 2);
+
+    // ---- the stages' sources
+    int steps = (k_len + KD - 1) / KD, first_step = 0;
+    const int tail_step = steps - 1, tail_k = k_len - tail_step * KD;
+    if (slab >= 0) {
+        first_step = int((long long)steps * ks / p.split);
+        steps = int((long long)steps * (ks + 1) / p.split);
+    }
+    const uint32_t lda2 = uint32_t(2 * p.lda), ldb2 = uint32_t(2 * p.ldb);
+    const char* gA = reinterpret_cast<const char*>(p.A) + (A_OC ? 2 * k_begin * p.lda : 2 * (long long)k_begin);
+    const char* gB = reinterpret_cast<const char*>(p.B + b_off) + (B_OC ? 2 * k_begin * p.ldb : 2 * (long long)k_begin);
+    const long long stepA = A_OC ? 2 * KD * p.lda : 2 * KD, stepB = B_OC ? 2 * KD * p.ldb : 2 * KD;
+    // rc: a piece of 16 (KD 32) or 8 rows; oc: 8 k-rows of 64 columns -- this lane's row, chunk (bytes) and k-row, column of piece 0
+    constexpr int RC = KD == 32 ? 16 : 8, OCU = KD / 32;   // rows of a piece; a wave's pieces of a 64-column unit
+    const int rc_row = KD == 32 ? 16 * w + (l >> 2) : 8 * w + (l >> 3);
+    const int rc_chunk = KD == 32 ? ((l & 3) ^ ((l >> 4) & 3)) * 16 : ((l & 7) ^ (4 * (w & 1) + (l >> 4))) * 16;
+    const int oc_k = 8 * w + (l >> 3), oc_col = ((((l & 7) >> 1) ^ (((l >> 4) & 1) << 1)) << 4) + (l & 1) * 8;
+    uint32_t offA[PA], offB[PB];
+#pragma unroll
+    for (int s = 0; s < PA; ++s) {
+        if (A_OC) {
+            offA[s] = (GATHER_K ? 0u : mul24(uint32_t(oc_k + 32 * (s % OCU)), lda2)) + 2u * uint32_t(min(m0 + 64 * (s / OCU) + oc_col, p.M - 8));
+        } else {
+            const int row = min(m0 + 4 * RC * s + rc_row, m_end - 1);
+            offA[s] = mul24(uint32_t(GATHER ? p.gather_rows[row] : row), lda2) + uint32_t(rc_chunk);
+        }
+    }
+    constexpr bool UP_ROWS = VER == 6 || VER == 9;   // up rows in a tensor of their own
+#pragma unroll
+    for (int s = 0; s < PB; ++s) {
+        int first = n0 + (B_OC ? 64 * (s / OCU) : 4 * RC * s);
+        if (GLU && s >= PB / 2) first += (UP_ROWS ? p.glu_up_rows : p.N / 2) - BN / 2;
+        if (B_OC)
+            offB[s] = mul24(uint32_t(oc_k + 32 * (s % OCU)), ldb2) + 2u * uint32_t(min(first + oc_col, p.N - 8));
+        else
+            offB[s] = mul24(uint32_t(UP_ROWS ? first + rc_row : min(first + rc_row, p.N - 1)), ldb2) + uint32_t(rc_chunk);
+    }
+    static_assert(!GATHER_K || (A_OC && OCU == 1), "one gathered row a lane and stage");
+    // GATHER_K: the token row of this lane's k-row of a stage (past the end of the reduction: the last one, which meets zeros of B)
+    auto row_of = [&](int step) __attribute__((always_inline)) { return p.gather_rows[k_begin + min(step * KD + oc_k, k_len - 1)]; };
+    const char* A0 = reinterpret_cast<const char*>(p.A);
+    // piece s of a stage (A's pieces first) from the step's operand addresses; the general form ends the reduction with zeros
+    auto piece = [&](auto s, const char* a, const char* b, char* d) __attribute__((always_inline)) {
+        constexpr int I = decltype(s)::value;
+        if constexpr (I < PA)
+            glds16(a + offA[I], d + 4096 * I);
+        else
+            glds16(b + offB[I - PA], d + 4096 * I);
+    };
+    auto dma = [&](int step, uint32_t at) __attribute__((always_inline)) {
+        const char* a = GATHER_K ? A0 + mul24(uint32_t(row_of(step)), lda2) : gA + step * stepA;
+        const char* b = gB + step * stepB;
+        char* d = smem + at + 1024 * w;
+        if (step == tail_step && tail_k < KD) {
+            const char* z = reinterpret_cast<const char*>(zero_page4) + 16 * (l & 15);
+#pragma unroll
+            for (int s = 0; s < PA + PB; ++s) {
+                const int k = (s < PA ? A_OC : B_OC) ? oc_k + 32 * ((s < PA ? s : s - PA) % OCU) : rc_chunk >> 1;
+                const char* src = k < tail_k ? (s < PA ? a + offA[s] : b + offB[s - PA]) : z;
+                hold(src);   // (one piece for the whole wave, not one for each side of the choice)
+                glds16(src, d + 4096 * s);
+            }
+        } else {
+            each([&](auto s) { piece(s, a, b, d); }, std::make_index_sequence<PA + PB>{});
+        }
+    };
+
+    Frag<A_OC, WM, KD> fa;
+    Frag<B_OC, WN, KD> fb;
+    fa.init(wm, l);
+    fb.init(wn, l);
+    f32x16 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int b = 0; b < NI; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][b][r] = 0.f;
+    s16x8 xa[MI], xb[NI], ya[MI], yb[NI];
+
+    // fragment I (B's first: the first product needs one of each) of sixteenth KK
+    auto frag = [&](auto kk, auto f, s16x8 (&ra)[MI], s16x8 (&rb)[NI], uint32_t at) __attribute__((always_inline)) {
+        constexpr int KK = decltype(kk)::value, I = decltype(f)::value;
+        if constexpr (I < NI)
+            rb[I] = fb.template read<I, KK>(smem, at + BM * KD * 2);
+        else
+            ra[I - NI] = fa.template read<I - NI, KK>(smem, at);
+    };
+    constexpr auto FRAGS = std::make_index_sequence<MI + NI>{};
+    constexpr auto PRODUCTS = std::make_index_sequence<MI * NI>{};
+    auto product = [&](auto j, const s16x8 (&ra)[MI], const s16x8 (&rb)[NI]) __attribute__((always_inline)) {
+        constexpr int J = decltype(j)::value;
+        acc[J / NI][J % NI] = mfma32(rb[J % NI], ra[J / NI], acc[J / NI][J % NI]);
+        sched_fence();
+    };
+    auto arrived = [&](s16x8 (&ra)[MI], s16x8 (&rb)[NI]) __attribute__((always_inline)) {
+        wait_lds();
+#pragma unroll
+        for (int i = 0; i < MI; ++i) hold(ra[i]);
+#pragma unroll
+        for (int b = 0; b < NI; ++b) hold(rb[b]);
+    };
+
+    const int count = steps - first_step;
+    if (count > 0) {
+#pragma unroll
+        for (int s = 0; s < S - 1; ++s)
+            if (s < count) dma(first_step + s, uint32_t(s * STAGE));
+        if (count >= S - 1)
+            wait_vm<(S - 2) * (PA + PB)>();
+        else
+            wait_vm<0>();
+        raw_barrier();
+        each([&](auto f) { frag(std::integral_constant<int, 0>{}, f, xa, xb, 0u); }, FRAGS);
+        arrived(xa, xb);
+        int row = GATHER_K ? row_of(S - 1) : 0;
+        uint32_t at = 0, fill = (S - 1) * STAGE;   // the stage in use; the one that was in use before it and is filled now
+        // the products of sixteenth KK of the stage, with the reads of the next and a share of the DMA pieces one by one between them
+        constexpr int QUOTA = (PA + PB + HALVES - 2) / (HALVES - 1);
+        auto sixteenth = [&](auto kk, s16x8 (&ra)[MI], s16x8 (&rb)[NI], s16x8 (&na)[MI], s16x8 (&nb)[NI], uint32_t from, auto whole, const char* a, const char* b, char* d)
+                             __attribute__((always_inline)) {
+            constexpr int KK = decltype(kk)::value, NEXT = (KK + 1) % HALVES;
+            each([&](auto j) {
+                constexpr int J = decltype(j)::value;
+                if constexpr (J < MI + NI) frag(std::integral_constant<int, NEXT>{}, j, na, nb, from);
+                product(j, ra, rb);
+                if constexpr (decltype(whole)::value && KK < HALVES - 1 && J < QUOTA && KK * QUOTA + J < PA + PB) piece(std::integral_constant<int, KK * QUOTA + J>{}, a, b, d);
+            }, PRODUCTS);
+            arrived(na, nb);
+        };
+        auto stage = [&](int step, auto whole) __attribute__((always_inline)) {
+            const uint32_t next = at + STAGE == S * STAGE ? 0u : at + STAGE;
+            const char* a = GATHER_K ? A0 + mul24(uint32_t(row), lda2) : gA + (first_step + step + S - 1) * stepA;
+            const char* b = gB + (first_step + step + S - 1) * stepB;
+            char* d = smem + fill + 1024 * w;
+            if (GATHER_K && decltype(whole)::value) row = row_of(step + S);   // (in front of this stage's pieces: waiting for it waits for none of them)
+            if (!decltype(whole)::value && step + S - 1 < count) dma(first_step + step + S - 1, fill);
+            each([&](auto kk) {
+                constexpr int KK = decltype(kk)::value;
+                if constexpr (KK % 2 == 0)
+                    sixteenth(kk, xa, xb, ya, yb, at, whole, a, b, d);
+                else
+                    sixteenth(kk, ya, yb, xa, xb, at, whole, a, b, d);
+            }, std::make_index_sequence<HALVES - 1>{});
+            if (decltype(whole)::value || step + S - 1 < count)   // behind stage step + 1: stages up to step + S - 1
+                wait_vm<(S - 2) * (PA + PB)>();
+            else
+                wait_vm<0>();
+            raw_barrier();
+            sixteenth(std::integral_constant<int, HALVES - 1>{}, ya, yb, xa, xb, next, whole, a, b, d);   // (behind the last step the reads are never used)
+            fill = at;
+            at = next;
+        };
+        static_assert(QUOTA <= MI * NI && MI + NI <= MI * NI && HALVES % 2 == 0, "a piece and a read behind each product");
+        int step = 0;
+        // steady steps: the stage that is filled exists and is whole
+        const int steady = count - (S - 1) - (first_step + count - 1 == tail_step && tail_k < KD ? 1 : 0);
+        for (; step < steady; ++step) stage(step, std::true_type{});
+        for (; step < count; ++step) stage(step, std::false_type{});
+    }
+
+    const int c = l & 31, h = l >> 5;
+    if (slab >= 0) {   // partial sums in the accumulators' order: 1 KiB contiguous a store
+        float* dst = p.ws + (long long)slab * (BM * BN) + l * 4;
+#pragma unroll
+        for (int b = 0; b < NI; ++b)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4*>(dst + (((b * MI + i) * WM + wm) * WN + wn) * 1024 + q * 256) =
+                        f32x4{acc[i][b][4 * q], acc[i][b][4 * q + 1], acc[i][b][4 * q + 2], acc[i][b][4 * q + 3]};
+        return;
+    }
+    if (PLAIN && (p.c_f32 || !p.wide_store || (p.N & 7))) {   // straight from the registers
+#pragma unroll
+        for (int b = 0; b < NI; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int n = n0 + b * (WN * 32) + wn * 32 + 8 * q + 4 * h;
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const int m = m0 + i * (WM * 32) + wm * 32 + c;
+                    if (m >= m_end) continue;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if (n + j >= p.N) continue;
+                        const float v = aria_epilogue_act(p, acc[i][b][4 * q + j] + (p.bias ? bf2f(p.bias[n + j]) : 0.f));
+                        if (p.c_f32) {
+                            float* d = reinterpret_cast<float*>(C) + (long long)m * p.ldc + n + j;
+                            *d = p.accumulate ? *d + v : v;
+                        } else {
+                            bf16_t* d = reinterpret_cast<bf16_t*>(C) + (long long)m * p.ldc + n + j;
+                            *d = f2bf(p.accumulate ? v + bf2f(*d) : v);
+                        }
+                    }
+                }
+            }
+        return;
+    }
+    // ---- the tile is parked as bf16 rows and leaves in 16-byte pieces of them
+    constexpr int CPR = BN / 8, ITS = BM * CPR / 256;
+    const bool old = PLAIN && p.accumulate;
+    raw_barrier();   // (the last stage's reads)
+    if (old) {       // the old tile waits where the new values will be parked: they are added in 32 bits and rounded once
+#pragma unroll 8
+        for (int it = 0; it < ITS; ++it) {
+            const int idx = it * 256 + t, row = idx / CPR, cc = (idx % CPR) * 8, m = m0 + row;
+            const u32x4 o = m < m_end && n0 + cc < p.N ? ld16(reinterpret_cast<const bf16_t*>(C) + (long long)m * p.ldc + n0 + cc) : zero16();
+            *reinterpret_cast<u32x4*>(smem + row * ROWP + cc * 2) = o;
+        }
+        sync();
+    }
+    auto park = [&](auto act) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act)::value;
+#pragma unroll
+        for (int b = 0; b < NI; ++b)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = b * (WN * 32) + wn * 32 + 8 * q + 4 * h;
+                float bv[4] = {0.f, 0.f, 0.f, 0.f};
+                if (PLAIN && p.bias) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (n0 + col + j < p.N) bv[j] = bf2f(p.bias[n0 + col + j]);
+                }
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    float v[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j += 2) {
+                        const f32x2 pr = aria_epilogue_act2<ACT>(f32x2{acc[i][b][4 * q + j] + bv[j], acc[i][b][4 * q + j + 1] + bv[j + 1]});
+                        v[j] = pr.x, v[j + 1] = pr.y;
+                    }
+                    u32x2* slot = reinterpret_cast<u32x2*>(smem + (i * (WM * 32) + wm * 32 + c) * ROWP + col * 2);
+                    if (old) {
+                        const u32x2 o = *slot;
+                        v[0] += bflo(o[0]), v[1] += bfhi(o[0]), v[2] += bflo(o[1]), v[3] += bfhi(o[1]);
+                    }
+                    *slot = u32x2{pack2bf(v[0], v[1]), pack2bf(v[2], v[3])};
+                }
+            }
+    };
+    if (VER == 3 && p.act == 1)
+        park(std::integral_constant<int, 1>{});
+    else if (VER == 3 && !A_OC && !B_OC && p.act == 2)
+        park(std::integral_constant<int, 2>{});
+    else
+        park(std::integral_constant<int, 0>{});
+    sync();
+    if (GLU) {   // rounding points as the unfused chain has them: h in bf16, silu(gate) in bf16, the product in bf16
+        constexpr int HALF = BN / 2, GP = HALF / 8;
+        const int I = p.N / 2;
+        bf16_t *H = reinterpret_cast<bf16_t*>(C), *ACT = static_cast<bf16_t*>(p.C2);
+#pragma unroll 4
+        for (int it = 0; it < ITS / 2; ++it) {
+            const int idx = it * 256 + t, row = idx / GP, cc = (idx % GP) * 8, m = m0 + row;
+            if (m >= m_end) continue;
+            const u32x4 g = *reinterpret_cast<const u32x4*>(smem + row * ROWP + cc * 2), u = *reinterpret_cast<const u32x4*>(smem + row * ROWP + (HALF + cc) * 2);
+            u32x4 y;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float g0 = bflo(g[q]), g1 = bfhi(g[q]);
+                y[q] = VER == 13 ? pack2bf(fmaxf(g0, 0.f) * bflo(u[q]), fmaxf(g1, 0.f) * bfhi(u[q]))
+                                 : pack2bf(rbf(silu_fast(g0)) * bflo(u[q]), rbf(silu_fast(g1)) * bfhi(u[q]));
+            }
+            st16(ACT + (long long)m * p.ldc2 + n0 + cc, y);
+            if (VER != 13 && H) {
+                st16(H + (long long)m * p.ldc + n0 + cc, g);
+                st16(H + (long long)m * p.ldc + I + n0 + cc, u);
+            }
+        }
+        return;
+    }
+#pragma unroll 4
+    for (int it = 0; it < ITS; ++it) {
+        const int idx = it * 256 + t, row = idx / CPR, cc = (idx % CPR) * 8, m = m0 + row;
+        if (m < m_end && n0 + cc < p.N) finish_piece<VER>(p, C, smem + row * ROWP, m, n0, cc);
+    }
+}
+
+// the sums of the slabs of gemm4_kernel<.., WM, WN, MI, NI, ..>: see gemm3_reduce_kernel; a block finishes 32 rows of 32 WN columns
+template <int WM, int WN, int MI, int NI>
+__global__ __launch_bounds__(256) void gemm4_reduce_kernel(GemmParams p) {
+    constexpr int BM = WM * MI * 32, BN = WN * NI * 32, COLS = WN * 32, PITCH = COLS + 4;
+    ARIA_SMEM_STATIC float sums[32 * PITCH];
+    int tn, tmi;
+    if (!aria_tile_from_pos(p, blockIdx.x, tmi, tn)) return;
+    const int t = threadIdx.x, part = blockIdx.y, wm = part % WM, i = part / WM % MI, b = part / (WM * MI);
+    const int l = t & 63, q = t >> 6;
+    const float* ws = p.ws + (long long)blockIdx.x * p.split * (BM * BN) + part * (WN * 1024) + q * 256 + l * 4;
+    f32x4 sum[WN];
+#pragma unroll
+    for (int k = 0; k < WN; ++k) sum[k] = *reinterpret_cast<const f32x4*>(ws + k * 1024);
+    int s = 1;
+    for (; s + 3 <= p.split; s += 3) {
+        f32x4 v[3][WN];
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int k = 0; k < WN; ++k) v[z][k] = *reinterpret_cast<const f32x4*>(ws + (long long)(s + z) * (BM * BN) + k * 1024);
+#pragma unroll
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int k = 0; k < WN; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[k][e] += v[z][k][e];
+    }
+    for (; s < p.split; ++s) {
+        f32x4 v[WN];
+#pragma unroll
+        for (int k = 0; k < WN; ++k) v[k] = *reinterpret_cast<const f32x4*>(ws + (long long)s * (BM * BN) + k * 1024);
+#pragma unroll
+        for (int k = 0; k < WN; ++k)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[k][e] += v[k][e];
+    }
+#pragma unroll
+    for (int k = 0; k < WN; ++k) *reinterpret_cast<f32x4*>(sums + (l & 31) * PITCH + k * 32 + 8 * q + 4 * (l >> 5)) = sum[k];
+    sync();
+    for (int idx = t; idx < 32 * COLS / 8; idx += 256) {
+        const int row = idx / (COLS / 8), col = (idx % (COLS / 8)) * 8;
+        aria_finish_sums(p, sums + row * PITCH + col, tmi * BM + i * (WM * 32) + wm * 32 + row, tn * BN + b * COLS + col);
+    }
+}
+
+
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
+int launch4(GemmParams q, int split, float* ws, void* stream) {
+    using T = Shape4<WM, WN, MI, NI, KD, S>;
+    constexpr int STEP = gated(VER) ? T::BN / 2 : T::BN;
+    const int cols = gated(VER) ? q.N / 2 : q.N;
+    q.ntn = (cols + STEP - 1) / STEP;
+    q.ntm = q.mode == 1 ? q.M / T::BM + q.E : (q.M + T::BM - 1) / T::BM;
+    q.split = split;
+    q.ws = ws;
+    if (q.ntn * q.ntm <= 0) return ARIA_OK;
+    const unsigned grid = q.mode == 1 ? unsigned(q.ntn * q.ntm + 16) : unsigned(q.ntn * q.ntm * std::max(split, 1));
+    ARIA_LAUNCH((gemm4_kernel<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, PER_CU>), dim3(grid, q.mode == 2 ? unsigned(q.E) : 1u), dim3(256), T::SMEM, stream, q);
+    if (split > 1) ARIA_LAUNCH((gemm4_reduce_kernel<WM, WN, MI, NI>), dim3(unsigned(q.ntn * q.ntm), NI * MI * WM), dim3(256), 0, stream, q);
+    return aria_check_launch();
+}
+
+constexpr long long ROUND = 256;   // CUs
+long long cdiv(long long a, long long b) { return (a + b - 1) / b; }
+
+// Time of a dense product, microseconds, as the kernels were measured on it (n: reduction in units of 64).  A round of the tiles named, whole workgroups a CU:
+//   256 x 256 12 + 1.1 n (4096 x 2560: K 2560 57, 3328 69), split S times + 5 + 0.04 a slab (777 x 2560 x 2560, 40 tiles: 34)
+//   128 x 128 5 + 1.25 n, three a CU
+//   128 x 256 7 + 0.66 n (777 x 2560 x 2560 32.5, 1868 x 2560 x 2560 34, 777 x 7680 x 2560 36.5), split + 5 + 0.02 a slab (777 x 2560 x 2560 twice 27, 280 x 2560 x 2560 four
+//     times 18.8)
+//   256 x 160 9 + 0.85 n (4096 x 2560: K 2560 47.5, 3328 59; 5600 x 1536: K 1536 30.6, 4096 65.6)
+//   128 x 320 9 + n (4096 x 2560: K 2560 51.3, 3328 63.4; K 7680 158 against 153: up to 4096)
+double time_128(long long tiles, double n, int split) { return double(cdiv(tiles * split, ROUND)) * (7.0 + 0.66 * n / split) + (split > 1 ? 5.0 + 0.02 * double(tiles * split) : 0.0); }
+double time_else(long long M, long long N, double n, int split) {
+    const long long t3 = cdiv(M, 256) * cdiv(N, 256), t1 = cdiv(M, 128) * cdiv(N, 128);
+    if (split > 1) return double(cdiv(t3 * split, ROUND)) * (12.0 + 1.1 * n / split) + 5.0 + 0.04 * double(t3 * split);
+    return t3 >= 80 ? double(cdiv(t3, ROUND)) * (12.0 + 1.1 * n) : double(cdiv(t1, 3 * ROUND)) * (5.0 + 1.25 * n);
+}
+
+int split_128(long long M, long long N, long long K) {   // pieces of the reduction that tiles of 128 x 256 would take in one round
+    const long long tiles = cdiv(M, 128) * cdiv(N, 256);
+    const double n = double(K) / 64.0;
+    int best = 1;
+    for (int s = 2; s <= 8 && tiles * s <= ROUND && n / s >= 6.0; ++s)
+        if (time_128(tiles, n, s) < 0.95 * time_128(tiles, n, best)) best = s;
+    return best;
+}
+// outputs of at least four column tiles and reductions of at least 12 stages: what the figures above were taken on
+bool dense_range(long long N, long long K) { return N >= 1024 && (N & 7) == 0 && K >= 768; }
+
+}  // namespace
+
+long long aria_gemm4_workspace_bytes(long long M, long long N, long long K) {
+    if (M <= 0 || !dense_range(N, K)) return 0;
+    const int s = split_128(M, N, K);
+    return s > 1 ? cdiv(M, 128) * cdiv(N, 256) * s * (128 * 256 * 4) : 0;
+}
+
+Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes) {
+    Gemm4Plan none, plan;
+    if (p.ext_k || (a_oc && !b_oc) || p.N < 8 || (a_oc && p.M < 8)) return none;
+    const bool plain = !p.glu && !p.dglu && !p.rope_fc;
+    if (const char* force = std::getenv("ARIA_GEMM_FORCE")) {   // "4": tiles of 128 x 256, "46": the wide ones where there is such a form
+        if (force[0] != '4') return none;
+        plan.form = a_oc ? 3 : force[1] == '6' && plain && p.mode == 0 ? 2 : 1;
+        return plan;
+    }
+    if (p.mode == 2) {   // rows: of all experts together, < 0: not known
+        // Weight gradients by expert, 64 of them, 256 x 256 / 128 x 256 tiles: 2560 x 3328 at 6 rows each on average 283 / 222, 28 rows 301 / 237, 73 332 / 301, 140 405 / 392, 384
+        // 641 / 634, 768 946 / 976; 1664 x 2560 139 / 114, 149 / 125, 171 / 161, 217 / 204, 328 / 328, 507 / 500.
+        if (rows >= 0 && rows < 400ll * p.E) plan.form = 3;
+        return plan;
+    }
+    if (a_oc) {   // 2560 x 2560, 7680 x 2560, 6656 x 2560: K 128 13 / 10, 21 / 18, 21 / 17; 784 24 / 18, 48 / 38, 49 / 39; 1568 39 / 27, 75 / 67, 68 / 66; 2048 45 / 33, 87 / 84, 77 / 82
+        if (p.N >= 1024 && p.M >= 1024 && cdiv(p.M, 128) * cdiv(p.N, 256) <= 8 * ROUND && p.K >= 64 && p.K <= 1600) plan.form = 3;
+        return plan;
+    }
+    if (p.mode == 1) {
+        // Rows by expert.  Up to 100 a expert its tile of 256 rows is mostly empty and the weights' stream counts, of which three stages of 48 KiB keep more in flight.
+        // 64 experts of 2560 x 1664, rows each on average 28 / 73 / 140, before and now: gate and up, gathered, [K, N] 254 -> 213, 276 -> 233, (306 -> 345); two [N, K]
+        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 114, 135 -> 124, (153 -> 155), at 6 rows (109 -> 111); SwiGLU backward 144 -> 121, 160 -> 149,
+        // (185 -> 200); gate and up backward [N, K] 214 -> 207, 245 -> 220.  And where all of it is one round: 16 experts of 1024 x 768, 187 rows each, 32.6 -> 20.2 and 25 -> 16.
+        if (p.K < 768 || p.N < 512) return none;
+        const long long cols = p.glu ? p.N / 2 : p.N, ntn = cdiv(cols, p.glu ? 128 : 256);
+        const bool few = p.M < 100ll * p.E && (!plain || p.M >= 16ll * p.E), one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
+        if (few || one_round) plan.form = 1;
+        return plan;
+    }
+    if (!dense_range(p.N, p.K)) return none;
+    const double n = double(p.K) / 64.0;
+    const long long t2 = cdiv(p.M, 128) * (p.glu ? cdiv(p.N / 2, 128) : cdiv(p.N, 256));
+    if (!plain) {   // (these forms never split)
+        if (t2 <= ROUND) plan.form = 1;
+        return plan;
+    }
+    double best = 0.94 * time_else(p.M, p.N, n, split3);
+    int s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
+    if (t2 * s <= ROUND && time_128(t2, n, s) < best) best = time_128(t2, n, s), plan.form = 1, plan.split = s;
+    const long long t6 = b_oc ? cdiv(p.M, 128) * cdiv(p.N, 320) : cdiv(p.M, 256) * cdiv(p.N, 160);
+    const double time6 = 9.0 + (b_oc ? 1.0 : 0.85) * n;
+    if (t6 <= ROUND && time6 < best && !(b_oc && p.K > 4096)) plan.form = 2, plan.split = 1;
+    return plan;
+}
+
+int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream) {
+    GemmParams q = p;
+    q.wide_store = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0 && (p.strideC & 7) == 0;
+    q.order = 4 | (p.glu && p.mode == 1 ? 512 : 0);
+    const int split = ws && plan.split > 1 ? plan.split : 1;
+    float* slabs = split > 1 ? ws : nullptr;
+    if (plan.form == 3) {
+        if (p.gather_rows) return launch4<true, true, 1, 4, 4, 2, 32, 3, 11, 2>(q, 1, nullptr, stream);
+        return launch4<true, true, 1, 4, 4, 2, 32, 3, 3, 2>(q, 1, nullptr, stream);
+    }
+    if (plan.form == 2)
+        return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
+#define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
+    if (p.rope_fc) return p.rope_sn ? ARIA_G4(false, 10) : ARIA_G4(false, 7);
+    if (p.glu == 2) return ARIA_G4(false, 13);
+    if (p.glu && p.gather_rows) return p.glu_up_rows > 0 ? ARIA_G4(false, 9) : ARIA_G4(true, 8);
+    if (p.glu && p.glu_up_rows > 0) return ARIA_G4(false, 6);
+    if (p.glu) return b_oc ? ARIA_G4(true, 14) : ARIA_G4(false, 14);
+    if (p.dglu) return b_oc ? ARIA_G4(true, 5) : ARIA_G4(false, 5);
+    return b_oc ? ARIA_G4(true, 3) : ARIA_G4(false, 3);
+#undef ARIA_G4
+}

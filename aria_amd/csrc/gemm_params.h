@@ -175,9 +175,10 @@ __device__ __forceinline__ bool aria_grouped_tile_interleaved(const P& p, int bi
     return false;
 }
 
-template <class P>
+// (ROWS: rows of a tile; the interleave is for tiles of 256)
+template <int ROWS = 256, class P>
 __device__ __forceinline__ bool aria_grouped_tile(const P& p, int bid, int l, int& expert, int& m0, int& m_end, int& tn) {
-    if ((p.order >> 12) & 1) return aria_grouped_tile_interleaved(p, bid, l, expert, m0, m_end, tn);
+    if (ROWS == 256 && ((p.order >> 12) & 1)) return aria_grouped_tile_interleaved(p, bid, l, expert, m0, m_end, tn);
     const bool split = (p.order >> 9) & 1;
     int TF = 0, TR = 0;  // tiles in the list of full (or, without the bit, all) row tiles / of ragged row tiles
     for (int e0 = 0; e0 < p.E; e0 += 64) {
@@ -185,8 +186,8 @@ __device__ __forceinline__ bool aria_grouped_tile(const P& p, int bid, int l, in
         int cf = 0, cr = 0;
         if (e < p.E) {
             const int n = p.offsets[e + 1] - p.offsets[e];
-            cf = (split ? n / 256 : (n + 255) / 256) * p.ntn;
-            cr = (split && (n & 255)) ? p.ntn : 0;
+            cf = (split ? n / ROWS : (n + ROWS - 1) / ROWS) * p.ntn;
+            cr = (split && (n & (ROWS - 1))) ? p.ntn : 0;
         }
         TF += ad::wave_bcast(ad::wave_incl_scan(cf), 63);
         if (split) TR += ad::wave_bcast(ad::wave_incl_scan(cr), 63);
@@ -211,8 +212,8 @@ __device__ __forceinline__ bool aria_grouped_tile(const P& p, int bid, int l, in
             o1 = p.offsets[e + 1];
         }
         const int n = o1 - o0;
-        const int nt = split ? n / 256 : (n + 255) / 256;  // row tiles of this expert in the full list
-        const int c = ragged ? ((n & 255) ? p.ntn : 0) : nt * p.ntn;
+        const int nt = split ? n / ROWS : (n + ROWS - 1) / ROWS;  // row tiles of this expert in the full list
+        const int c = ragged ? ((n & (ROWS - 1)) ? p.ntn : 0) : nt * p.ntn;
         const int incl = ad::wave_incl_scan(c);  // (DPP, no LDS round trips: this runs in front of every grouped tile)
         const int excl = base + incl - c;
         const unsigned long long mask = ad::ballot(c > 0 && v >= excl && v < excl + c);
@@ -228,7 +229,7 @@ __device__ __forceinline__ bool aria_grouped_tile(const P& p, int bid, int l, in
                 tn = local / nts;
                 row = local % nts;
             }
-            m0 = ad::wave_bcast(o0, src) + row * 256;
+            m0 = ad::wave_bcast(o0, src) + row * ROWS;
             m_end = ad::wave_bcast(o1, src);
             return true;
         }
@@ -266,6 +267,37 @@ __device__ __forceinline__ ad::f32x2 aria_epilogue_act2(ad::f32x2 v) {
     return ad::f32x2{aria_epilogue_act_c<ACT>(v.x), aria_epilogue_act_c<ACT>(v.y)};
 }
 
+// eight consecutive 32-bit sums of row m, columns n .. n + 7, through the epilogue of a split product: bias, activation, accumulation, rounding
+template <class P>
+__device__ __forceinline__ void aria_finish_sums(const P& p, const float* sums, int m, int n) {
+    using namespace ad;
+    if (m >= p.M || n >= p.N) return;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = aria_epilogue_act(p, sums[e] + (p.bias && n + e < p.N ? bf2f(p.bias[n + e]) : 0.f));
+    if (!p.c_f32 && p.wide_store && n + 8 <= p.N) {
+        bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n;
+        if (p.accumulate) {
+            const u32x4 o = ld16(d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[2 * e] += bflo(o[e]), v[2 * e + 1] += bfhi(o[e]);
+        }
+        st16(d, u32x4{pack2bf(v[0], v[1]), pack2bf(v[2], v[3]), pack2bf(v[4], v[5]), pack2bf(v[6], v[7])});
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if (n + e >= p.N) continue;
+        if (p.c_f32) {
+            float* d = static_cast<float*>(p.C) + (long long)m * p.ldc + n + e;
+            *d = p.accumulate ? *d + v[e] : v[e];
+        } else {
+            bf16_t* d = static_cast<bf16_t*>(p.C) + (long long)m * p.ldc + n + e;
+            *d = f2bf(p.accumulate ? v[e] + bf2f(*d) : v[e]);
+        }
+    }
+}
+
 // (internal to the library: hidden, not part of the C ABI)
 // v2 launcher (gemm2.hip); returns ARIA_* status
 __attribute__((visibility("hidden"))) int aria_launch_gemm2(const GemmParams& p, int a_oc, int b_oc, int ntm_or_max_tm, int grid_y, void* stream);
@@ -274,3 +306,13 @@ __attribute__((visibility("hidden"))) int aria_launch_gemm3(const GemmParams& p,
                       long long workspace_bytes = 0);
 // fp32 workspace bytes the v3 remainder split-K wants for a dense problem (0: it would not split)
 __attribute__((visibility("hidden"))) long long aria_gemm3_workspace_bytes(long long M, long long N, long long K);
+// the four-wave kernels (gemm4.hip).  form 0: not theirs; 1: tiles of 128 x 256; 2: 256 x 160 or 128 x 320; 3: 128 x 256, two workgroups a CU (both operands [k][rows])
+struct Gemm4Plan {
+    int form = 0, split = 1;
+};
+// rows: mode 2's rows of all experts together (< 0: not known); split3: pieces that the 256 x 256 tiles would cut the reduction of a partly filled round into (1: none)
+__attribute__((visibility("hidden"))) Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes);
+__attribute__((visibility("hidden"))) int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream);
+__attribute__((visibility("hidden"))) long long aria_gemm4_workspace_bytes(long long M, long long N, long long K);
+// pieces the v3 remainder split-K would take for a dense problem of at most one round (1: none)
+__attribute__((visibility("hidden"))) int aria_gemm3_split(long long M, long long N, long long K);

@@ -512,12 +512,12 @@ def grouped_gemm_wgrad_gather(x: torch.Tensor, rows: torch.Tensor, dy: torch.Ten
     out = torch.empty((E, K, N), dtype=out_dtype, device=x.device)
     if dy.shape[0] == 0:
         return out.zero_()
-    rc = hip.get_lib().cdll.aria_grouped_gemm_wgrad_gather_bf16(_p(x), _p(rows), _p(dy), _p(out), _p(offsets), E, x.shape[0], K, N, _rowmajor_2d(x, "x"),
-                                                                _rowmajor_2d(dy, "dy"), int(out_dtype == torch.float32), 0, _stream(x))
+    rc = hip.get_lib().cdll.aria_grouped_gemm_wgrad_gather_sized_bf16(_p(x), _p(rows), _p(dy), _p(out), _p(offsets), E, x.shape[0], K, N, _rowmajor_2d(x, "x"),
+                                                                      _rowmajor_2d(dy, "dy"), int(out_dtype == torch.float32), 0, dy.shape[0], _stream(x))
     if rc == 3:
         return None
     if rc != 0:
-        raise hip.AriaHipError(f"aria_grouped_gemm_wgrad_gather_bf16 failed: {hip.ERRORS.get(rc, rc)}")
+        raise hip.AriaHipError(f"aria_grouped_gemm_wgrad_gather_sized_bf16 failed: {hip.ERRORS.get(rc, rc)}")
     return out
 
 
@@ -639,8 +639,8 @@ def grouped_gemm_wgrad(a: torch.Tensor, dy: torch.Tensor, offsets: torch.Tensor,
     c_f32 = {bf16: 0, torch.float32: 1}[out.dtype]
     if a.shape[0] == 0:  # no rows at all: every expert's gradient is zero
         return out if accumulate else out.zero_()
-    hip.get_lib().call("aria_grouped_gemm_wgrad_bf16", _p(a), _p(dy), _p(out), _p(offsets), E, K, N, _rowmajor_2d(a, "a"),
-                       _rowmajor_2d(dy, "dy"), c_f32, int(accumulate), _stream(a))
+    hip.get_lib().call("aria_grouped_gemm_wgrad_sized_bf16", _p(a), _p(dy), _p(out), _p(offsets), E, K, N, _rowmajor_2d(a, "a"),
+                       _rowmajor_2d(dy, "dy"), c_f32, int(accumulate), a.shape[0], _stream(a))
     return out
 
 

@@ -33,7 +33,7 @@ extern "C" {
 #define ARIA_ABI_VERSION 5
 int aria_abi_version(void);
 /* Test/diagnostic aid: which GEMM kernel family the calling thread's last aria_*gemm* call dispatched to
- * (1 = 128x128 tile, 2 = 256x256 register-staged, 3 = 256x256 LDS-DMA phase-scheduled; 0 = none yet). */
+ * (1 = 128x128 tile, 2 = 256x256 register-staged, 3 = LDS-DMA: 256x256 phase-scheduled, or the four-wave tiles; 0 = none yet). */
 int aria_last_gemm_variant(void);
 
 /* ------------------------------------------------------------------------------------------------
@@ -149,6 +149,9 @@ int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t 
  * ARIA_ERR_UNSUPPORTED. */
 int aria_grouped_gemm_wgrad_gather_bf16(const void* X, const int32_t* rows, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t T,
                                         int64_t K, int64_t N, int64_t ldx, int64_t ldy, int c_f32, int accumulate, void* stream);
+/* The same with the number of permuted rows (see aria_grouped_gemm_wgrad_sized_bf16). */
+int aria_grouped_gemm_wgrad_gather_sized_bf16(const void* X, const int32_t* rows, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t T,
+                                              int64_t K, int64_t N, int64_t ldx, int64_t ldy, int c_f32, int accumulate, int64_t M_total, void* stream);
 
 /* K7: gptfast's Attention.forward up to the attention call (gptfast/model.py:413-435) as ONE launch: the fused wqkv projection
  * X [M, K] x Wqkv^T ([3 D, K]: q rows, k rows, v rows), the interleaved-pair RoPE of q and k (apply_rotary_emb :519-531: fp32 arithmetic on
@@ -202,6 +205,9 @@ int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* D
  * Experts with zero rows get zeros (or keep dW when accumulate). */
 int aria_grouped_gemm_wgrad_bf16(const void* A, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t K,
                                  int64_t N, int64_t lda, int64_t ldy, int c_f32, int accumulate, void* stream);
+/* The same with the rows of all experts together (offsets[E], which the host otherwise does not know): the tiles are chosen by it. */
+int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t K, int64_t N, int64_t lda, int64_t ldy,
+                                       int c_f32, int accumulate, int64_t M_total, void* stream);
 
 /* ------------------------------------------------------------------------------------------------
  * MoE routing / dispatch (moe.hip)

@@ -114,6 +114,31 @@ def case_gemm_split_k_slabs(dev, M, N, K, a_oc, b_oc):
     assert torch.equal(acc.cpu(), (ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias.to(dev), out_dtype=torch.float32).cpu() + old.float()).to(bf16))
 
 
+def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
+    """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
+    activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""
+    from aria_amd import ops
+
+    a, b = rnd(*((K, M) if a_oc else (M, K)), seed=M + K).to(dev), rnd(*((K, N) if b_oc else (N, K)), seed=N, scale=0.3).to(dev)
+    bias, old = rnd(N, seed=3).to(dev), rnd(M, N + 10, seed=4).to(dev)
+
+    def results():
+        out = [ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias), ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, out_dtype=torch.float32)]
+        out += [ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias, act=t) for t in ("gelu_tanh", "relu_squared") if t == "gelu_tanh" or not (a_oc or b_oc)]
+        for first in (0, 2):
+            c = old.clone()
+            ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias, out=c[:, first:first + N], accumulate=True)
+            out.append(c)
+        return out
+
+    monkeypatch.setattr(ops, "GEMM_SPLIT_K", False)
+    monkeypatch.setenv("ARIA_GEMM_FORCE", force)
+    got = results()
+    monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
+    for x, y in zip(got, results()):
+        assert torch.equal(x.cpu(), y.cpu())
+
+
 def case_gemm_workspace_kept(dev):
     """What is kept per stream is one buffer of a fixed size; a larger need is the call's own and leaves nothing behind."""
     from aria_amd import ops

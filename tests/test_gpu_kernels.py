@@ -335,3 +335,31 @@ def test_grouped_tile_orders_cover_every_tile_once(monkeypatch):
     monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
     C.case_grouped_tile_orders(DEV)
     C.case_grouped_tile_orders(DEV, T=6000, E=9, k=2, K=256, I=256, seed=78)
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 256, 64), (8, 264, 72), (136, 520, 200), (264, 328, 320), (520, 168, 456)])
+@pytest.mark.parametrize("a_oc,b_oc", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("force", ["4", "46"])
+def test_gemm_four_waves(monkeypatch, force, M, N, K, a_oc, b_oc):
+    C.case_gemm_four_waves(DEV, monkeypatch, force, M, N, K, a_oc, b_oc)
+
+
+def test_gemm_four_waves_fused(monkeypatch):
+    """Every other end of these tiles, with rows by expert that fill no tile, one and several."""
+    monkeypatch.setenv("ARIA_GEMM_FORCE", "4")
+    counts = [130, 0, 70, 5, 0, 257, 1]
+    C.case_grouped_gemm(DEV, counts)
+    C.case_gemm_swiglu_fused(DEV, counts, 128, 128, 130)
+    C.case_gemm_swiglu_split(DEV, counts, 192, 256, 72)
+    C.case_gemm_dswiglu_fused(DEV, counts, 128, 384, 129)
+    C.case_gemm_swiglu_gather(DEV, 150, 8, 2, 128, 128)
+    C.case_gemm_qkv_rope_cache(DEV, 2, 37, 256, 64, 128, 48, True)
+    assert C.case_gemm_qkv_rope_hf(DEV, 1, 140, 256, 64, 64)
+    for T, E, k, K, N in ((150, 8, 2, 264, 136), (700, 8, 1, 128, 256), (40, 4, 3, 64, 72)):
+        C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
+
+
+@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 1536, False), (130, 1024, 1664, True)])
+def test_gemm_four_waves_split(M, N, K, b_oc):
+    """A reduction cut into pieces of whole stages, by the rule itself."""
+    C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)
