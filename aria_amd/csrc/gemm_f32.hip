@@ -12,6 +12,7 @@
 // 1480 us, 64 x 32 x 4 1650).
 #include "aria_device.h"
 #include "aria_hip.h"
+#include "elem.h"
 #include <algorithm>
 
 namespace {
@@ -25,6 +26,12 @@ struct GemmF32 {
     const int* offsets;   // rows grouped by expert, or NULL
     int E;
     long long strideW;
+};
+// a product a head (blockIdx.y) of the latent attention's expansion: the result's row t of head h times its output gate over its softmax sum
+struct Heads {
+    const float *ml, *gate;   // [T, H, 2] (maximum, sum), gate logits [T, ldg]
+    long long ldg;
+    int H, cols;              // columns of a head's result in memory (zeros behind N)
 };
 
 // The (expert, rows) of row tile y where the tiles of all experts are one sequence; every wave finds it for itself.  false: behind the last one.
@@ -47,12 +54,13 @@ __device__ __forceinline__ bool find_rows(const GemmF32& p, int y, int rows, int
     return false;
 }
 
-template <int MT, int NT, int NW>
-__global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
+template <int MT, int NT, int NW, bool HEADS>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p, Heads hd) {
     constexpr int DEPTH = MT + NT > 4 ? 2 : 4, TM = 16 * MT, TN = 16 * NT;
     ARIA_SMEM_STATIC float red[NW][TM][TN + 1];
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15;
-    const unsigned ntn = unsigned(p.N + TN - 1) / TN;
+    if (HEADS) p.A += (long long)blockIdx.y * p.K, p.W += blockIdx.y * p.strideW, p.C += (long long)blockIdx.y * hd.cols;
+    const unsigned ntn = unsigned((HEADS ? hd.cols : p.N) + TN - 1) / TN;
     const int y = int(blockIdx.x / ntn), n0 = int(blockIdx.x % ntn) * TN;
     int m0 = y * TM, m_end = p.M, e = 0;
     if (p.offsets && !find_rows(p, y, TM, e, m0, m_end)) return;
@@ -132,7 +140,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
         float v = 0.f;
 #pragma unroll
         for (int ww = 0; ww < NW; ++ww) v += red[ww][m][n];
-        if (m0 + m < m_end && n0 + n < p.N) p.C[(long long)(m0 + m) * p.ldc + n0 + n] = v;
+        if (HEADS) {
+            if (m0 + m < m_end && n0 + n < hd.cols) {
+                const float sum = hd.ml[((long long)(m0 + m) * hd.H + blockIdx.y) * 2 + 1], z = hd.gate[(m0 + m) * hd.ldg + blockIdx.y];
+                p.C[(long long)(m0 + m) * p.ldc + n0 + n] = n0 + n < p.N ? v / sum * sigmoid_exact(z) : 0.f;
+            }
+        } else if (m0 + m < m_end && n0 + n < p.N) {
+            p.C[(long long)(m0 + m) * p.ldc + n0 + n] = v;
+        }
     }
 }
 
@@ -141,11 +156,19 @@ int launch_f32(const GemmF32& p, void* stream) {
     const int64_t ntm = (int64_t(p.M) + 16 * MT - 1) / (16 * MT) + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
     const int64_t ntn = (int64_t(p.N) + 16 * NT - 1) / (16 * NT);
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
-    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
+    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, false>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p, Heads{});
     return aria_check_launch();
 }
 
 }  // namespace
+
+__attribute__((visibility("hidden"))) int aria_gemm_f32_heads(const float* part_o, const float* uv, float* out, const AriaLatentShape& s, const float* part_ml, const float* proj,
+                                                              int64_t T, void* stream) {
+    const GemmF32 p{part_o, uv, out, int(T), int(s.dv), int(s.R), (long long)(s.H * s.R), (long long)s.rp, (long long)(s.H * s.dvp), nullptr, 1, (long long)(s.dv * s.rp)};
+    const Heads hd{part_ml, proj + s.g_off, (long long)s.ldp, int(s.H), int(s.dvp)};
+    ARIA_LAUNCH((gemm_f32_kernel<4, 2, 4, true>), dim3(unsigned((T + 63) / 64 * ((s.dvp + 31) / 32)), unsigned(s.H)), dim3(256), 0, stream, p, hd);
+    return aria_check_launch();
+}
 
 extern "C" {
 

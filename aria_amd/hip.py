@@ -25,7 +25,8 @@ P, I64, I32, F32 = c_void_p, c_int64, c_int, c_float
 RESTYPES = {"aria_gemm_workspace_bytes": c_int64, "aria_decode_scratch_bytes": c_int64, "aria_decode_step_scratch": c_int64, "aria_prompt_step_scratch": c_int64, "aria_decode_graph_create": c_void_p,
             "aria_decode_graph_destroy": None, "aria_decode_attn_workspace_bytes": c_int64,
             "aria_latent_decode_scratch": c_int64, "aria_latent_splits": c_int64, "aria_linear_chunks_scratch": c_int64, "aria_mix_decode_scratch": c_int64,
-            "aria_chunk_decode_scratch": c_int64}  # everything else returns an int status
+            "aria_chunk_decode_scratch": c_int64,
+            "aria_latent_splits_f32": c_int64}  # everything else returns an int status
 
 # name -> argtypes (all return int).  Kept in one table so tests can check that the shared
 # library exports every symbol the header declares.
@@ -123,6 +124,7 @@ SIGNATURES = {
     "aria_latent_attn": [P, P, P, P, P, P, P, I64, I64, I32, P],
     "aria_latent_expand": [P, P, P, P, P, P, I64, I64, I32, P],
     "aria_latent_splits": [P, I64, I64],
+    "aria_latent_splits_f32": [P, I64, I64],
     "aria_latent_decode_scratch": [P, P, I64, I64],
     "aria_latent_decode": [P, P, I64, P, P, P, I64, P, P, I64, P],
     "aria_gemm_relu_glu_bf16": [P, P, P, I64, I64, I64, I64, I64, I64, P],

@@ -1237,7 +1237,7 @@ def latent_decode_attention(shape, proj, slot, pos, rope, kv_norm, uk, uv, cache
     f32, dev, lib, ref = _f32(proj), proj.device, hip.get_lib(), ctypes.byref(shape)
     qa = torch.empty((T, shape.H, shape.cw), dtype=proj.dtype, device=dev)
     lib.call("aria_latent_absorb", _p(proj), ref, _p(slot), _p(pos), _p(rope), _p(kv_norm), _p(uk), _p(cache), _p(qa), T, f32, _stream(proj))
-    splits = 1 if f32 else int(lib.cdll.aria_latent_splits(ref, T, max_len))
+    splits = int((lib.cdll.aria_latent_splits_f32 if f32 else lib.cdll.aria_latent_splits)(ref, T, max_len))
     part_o = torch.empty((T, splits, shape.H, shape.R), dtype=torch.float32, device=dev)
     part_ml = torch.empty((T, splits, shape.H, 2), dtype=torch.float32, device=dev)
     lib.call("aria_latent_attn", _p(qa), _p(cache), ref, _p(slot), _p(pos), _p(part_o), _p(part_ml), T, splits, f32, _stream(proj))

@@ -575,6 +575,7 @@ int aria_latent_decode(const AriaLatentStack* stack, const AriaLatentLayer* laye
                        int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
 /* how many splits aria_latent_decode / a caller of aria_latent_attn should use */
 int64_t aria_latent_splits(const AriaLatentShape* s, int64_t T, int64_t max_len);
+int64_t aria_latent_splits_f32(const AriaLatentShape* s, int64_t T, int64_t max_len);
 
 /* ------------------------------------------------------------------------------------------------
  * Chunk-local grouped-query attention, linear attention, RMS-normed stream: the mechanisms of the Kozipel design.  `f32` as above.  Residual stream,

@@ -611,3 +611,51 @@ def case_bad_inputs(dev):
     assert [l.source for l in chain.layers] == [2, 2, 2]
     with pytest.raises(ValueError):
         DuguzenConfig.from_dict(dict(cfg, layers=[dict(one, weights_of=1), dict(one, weights_of=0)]))
+
+
+def case_latent_attention_f32(dev, H, R, dr, dv, runs):
+    """32-bit latent attention and its expansion against float64, tokens given as (slot, first position, tokens) runs: several heads and tokens a workgroup, tokens
+    of several sequences, portions, an earlier position behind a later one; splits for few tokens.  32-bit sums of cw products: errors of some 1e-6.  A row
+    that is no number stays with the tokens that see it."""
+    import ctypes
+
+    from aria_amd import hip, ops
+
+    cw, rp, dvp, cap = (R + dr + 63) // 64 * 64, (R + 7) // 8 * 8, (dv + 7) // 8 * 8, 96
+    slot = torch.tensor([s for s, _, n in runs for _ in range(n)], dtype=torch.int32)
+    pos = torch.tensor([p + i for _, p, n in runs for i in range(n)], dtype=torch.int32)
+    T = slot.numel()
+    dq = (8 + dr + 7) // 8 * 8
+    g_off = H * dq + (R + dr + 7) // 8 * 8
+    s = hip.LatentShape(H=H, dn=8, dr=dr, dv=dv, R=R, rot=dr, dq=dq, dvp=dvp, cw=cw, rp=rp, ldp=g_off + (H + 7) // 8 * 8, kv_off=H * dq, g_off=g_off, S_cap=cap,
+                        scale=0.2, eps=1e-6)
+    qa, cache = torch.zeros(T, H, cw), torch.zeros(int(slot.max()) + 1, cap, cw)
+    qa[..., :R + dr], cache[..., :R + dr] = rnd(T, H, R + dr, seed=1, dtype=f32), rnd(cache.shape[0], cap, R + dr, seed=2, dtype=f32)
+    proj, uv = rnd(T, s.ldp, seed=3, dtype=f32), torch.zeros(H * dv, rp)
+    uv[:, :R] = rnd(H * dv, R, seed=4, dtype=f32)
+    lib, ref = hip.get_lib(), ctypes.byref(s)
+
+    def run(cache):
+        splits = int(lib.cdll.aria_latent_splits_f32(ref, T, int(pos.max()) + 1))
+        po, ml = torch.empty(T, splits, H, R, device=dev), torch.empty(T, splits, H, 2, device=dev)
+        out, dq, dc, ds, dp = torch.empty(T, H, dvp, device=dev), qa.to(dev), cache.to(dev), slot.to(dev), pos.to(dev)
+        lib.call("aria_latent_attn", dq.data_ptr(), dc.data_ptr(), ref, ds.data_ptr(), dp.data_ptr(), po.data_ptr(), ml.data_ptr(), T, splits, 1, ops._stream(dq))
+        pr, u = proj.to(dev), uv.to(dev)
+        lib.call("aria_latent_expand", po.data_ptr(), ml.data_ptr(), ref, pr.data_ptr(), u.data_ptr(), out.data_ptr(), T, splits, 1, ops._stream(dq))
+        return out.cpu(), splits
+
+    got, splits = run(cache)
+    assert (splits > 1) == (T <= 16 and int(pos.max()) >= 64)
+    want = torch.zeros(T, H, dvp, dtype=torch.float64)
+    for t in range(T):
+        k = cache[slot[t], :pos[t] + 1].double()
+        p = (qa[t].double() @ k.T * s.scale).softmax(-1)
+        want[t, :, :dv] = torch.einsum("hr,hdr->hd", p @ k[:, :R], uv[:, :R].double().view(H, dv, R)) * torch.sigmoid(proj[t, g_off:g_off + H].double())[:, None]
+    assert rel(got, want) < 3e-6
+    if T > 16:
+        bad = cache.clone()
+        row = int(pos[slot == slot[0]].float().median())
+        bad[slot[0], row] = float("nan")
+        sees = (slot == slot[0]) & (pos >= row)
+        got2 = run(bad)[0]
+        assert bool(got2[sees][..., :dv].isnan().all()) and torch.equal(got2[~sees], got[~sees])
