@@ -26,7 +26,7 @@ RESTYPES = {"aria_gemm_workspace_bytes": c_int64, "aria_decode_scratch_bytes": c
             "aria_decode_graph_destroy": None, "aria_decode_attn_workspace_bytes": c_int64,
             "aria_latent_decode_scratch": c_int64, "aria_latent_splits": c_int64, "aria_linear_chunks_scratch": c_int64, "aria_mix_decode_scratch": c_int64,
             "aria_chunk_decode_scratch": c_int64,
-            "aria_latent_splits_f32": c_int64}  # everything else returns an int status
+            "aria_latent_splits_f32": c_int64, "aria_latent_step_f32_scratch": c_int64, "aria_mix_step_f32_scratch": c_int64}  # everything else returns an int status
 
 # name -> argtypes (all return int).  Kept in one table so tests can check that the shared
 # library exports every symbol the header declares.
@@ -127,6 +127,10 @@ SIGNATURES = {
     "aria_latent_splits_f32": [P, I64, I64],
     "aria_latent_decode_scratch": [P, P, I64, I64],
     "aria_latent_decode": [P, P, I64, P, P, P, I64, P, P, I64, P],
+    "aria_latent_step_f32_scratch": [P, P, I64, I64, I64],
+    "aria_latent_step_f32": [P, P, I64, P, P, P, I64, P, I64, P, P, I64, P],
+    "aria_mix_step_f32_scratch": [P, P, I64, I64],
+    "aria_mix_step_f32": [P, P, I64, P, P, P, P, P, I64, I64, P, I64, P, P, I64, P],
     "aria_gemm_relu_glu_bf16": [P, P, P, I64, I64, I64, I64, I64, I64, P],
     "aria_rms_stream": [P, I64, I64, I32, P],
     "aria_softcap": [P, I64, F32, P],

@@ -5,9 +5,10 @@ embedding output added to the stream before every pass but the first; every pass
 This file reads the design's config.json and tensor names and assembles the mechanisms of ``layers.py`` into the serving protocol of ``serving.py``
 (caches, step function, scheduler, sampling and command line are the framework's).  A step runs in one of two ways:
 
-* prompts, large batches and float32: sublayer by sublayer from here (tile GEMMs, flash attention and linear attention on the matrix pipe, the fused stream
+* prompts and large batches in bf16: sublayer by sublayer from here (tile GEMMs, flash attention and linear attention on the matrix pipe, the fused stream
   pass);
-* up to ``DECODE_ROWS`` single tokens in bf16: one C call (``aria_mix_decode``) that enqueues every kernel of every layer run."""
+* up to ``DECODE_ROWS`` single tokens in bf16: one C call (``aria_mix_decode``) that enqueues every kernel of every layer run;
+* float32: one C call (``aria_mix_step_f32``) that enqueues the launches of the step run sublayer by sublayer, for any batch."""
 from __future__ import annotations
 
 import ctypes
@@ -19,7 +20,7 @@ import torch.nn as nn
 
 from . import hip, ops
 from .checkpoint import load_checkpoint_dir
-from .layers import ChunkAttention, LinearAttention, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, padded, up8
+from .layers import ChunkAttention, Held, LinearAttention, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, padded, shapes_of, table_batch, up8
 from .registry import read_config
 
 bf16, f32 = torch.bfloat16, torch.float32
@@ -120,6 +121,7 @@ class KozipelForCausalLM(nn.Module):
         self.caches: List[list] = []
         self.geometry = None
         self._decode: Optional["_DecodeTables"] = None
+        self._shapes = shapes_of(self)
 
     @classmethod
     def from_tensors(cls, config: dict, tensors: Dict[str, torch.Tensor], device="cuda", dtype=bf16) -> "KozipelForCausalLM":
@@ -171,6 +173,11 @@ class KozipelForCausalLM(nn.Module):
                 self._decode = _DecodeTables(self)
             logits = self._decode.run(batch)
             return logits if batch.every_row else logits[batch.wanted.long()]
+        if self.dtype == f32 and trace is None and batch.seq is not None and table_batch(batch, self.device) and all(L.mixer.table_step and L.mixer.parts[-1].eps == c.eps for L in self.layers):
+            if self._decode is None or not self._decode.held.current():
+                self._decode = _DecodeTables(self)
+            if self._decode.held.plain():
+                return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.rms_stream(x, c.width, c.eps, self.layers[c.runs[0].layer].norm1.weight, ids=batch.ids, table=self.embed, scale=c.embedding_scale)
         for i, run in enumerate(c.runs):
@@ -210,6 +217,18 @@ class _DecodeTables:
         self.stack = hip.MixStack(n, model.width, c.width, model.head.shape[0], c.embedding_scale, c.residual_mult, c.eps, c.logit_softcap,
                                   model.layers[c.runs[0].layer].norm1.weight.data_ptr(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows, self.vocab = model.device, model.head.shape[0], model.vocab
+        flat = [c for run in model.caches for c in run]
+        self.held = Held(model, model._shapes, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
+                         + [(model.caches, i, run) for i, run in enumerate(model.caches)])
+
+    def run_f32(self, batch) -> torch.Tensor:
+        T, W, lib = batch.ids.numel(), batch.wanted.numel() if batch.wanted is not None else -1, hip.get_lib()
+        stack, runs = ctypes.byref(self.stack), ctypes.byref(self.runs)
+        scratch = torch.empty(int(lib.cdll.aria_mix_step_f32_scratch(stack, runs, T, W)), dtype=torch.uint8, device=self.device)
+        logits = torch.empty((batch.n_wanted, self.rows), dtype=f32, device=self.device)
+        lib.call("aria_mix_step_f32", stack, runs, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.seq.data_ptr(), batch.cu.data_ptr(),
+                 len(batch.lengths), batch.max_len, ops._p(batch.wanted), W, logits.data_ptr(), scratch.data_ptr(), scratch.numel(), ops._stream(scratch))
+        return logits[:, :self.vocab]
 
     def run(self, batch) -> torch.Tensor:
         T, lib = batch.ids.numel(), hip.get_lib()

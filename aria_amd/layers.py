@@ -41,6 +41,41 @@ def _frozen(t: torch.Tensor, dtype) -> nn.Parameter:
     return nn.Parameter(t.to(dtype).contiguous(), requires_grad=False)
 
 
+def shapes_of(model: nn.Module) -> dict:
+    return {n: tuple(p.shape) for n, p in model.named_parameters()}
+
+
+class Held:
+    """What a float32 step's table of addresses was made from: every parameter, cache and constant of a model, compared before each step that runs by the table.
+    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks or forwards of
+    its own, or with tensors other than those it was made with (``shapes``), is not ``plain``."""
+
+    def __init__(self, model: nn.Module, shapes: dict, others: Sequence[tuple] = ()):
+        self.modules = list(model.modules())
+        tensors = [(m._parameters, n, t) for m in self.modules for n, t in m._parameters.items()] + [e for e in others if torch.is_tensor(e[2])]
+        self.tensors = [(*e, e[2].data_ptr()) for e in tensors if e[2] is not None]
+        self.values = [(m._modules, n, c) for m in self.modules for n, c in m._modules.items()] + [e for e in others if not torch.is_tensor(e[2])]
+        device = next(model.parameters()).device
+        self.fits = shapes_of(model) == shapes and all(t.dtype == f32 and t.is_contiguous() and t.device == device for _, _, t, _ in self.tensors)
+
+    def current(self) -> bool:
+        try:
+            return all(d[n] is t and t.data_ptr() == p for d, n, t, p in self.tensors) and all(d[n] is v for d, n, v in self.values)
+        except (KeyError, IndexError):
+            return False
+
+    def plain(self) -> bool:
+        return self.fits and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in self.modules)
+
+
+def table_batch(batch, device) -> bool:
+    """the batch's tables as a call by addresses reads them"""
+    T = batch.ids.numel()
+    own = [batch.ids, batch.slot, batch.pos, batch.cu] + [t for t in (batch.seq, batch.wanted) if t is not None]
+    return (T > 0 and all(t.dtype == torch.int32 and t.is_contiguous() and t.device == device for t in own)
+            and batch.slot.numel() == T == batch.pos.numel() and batch.cu.numel() == len(batch.lengths) + 1 and (batch.seq is None or batch.seq.numel() == T))
+
+
 class DynamicTanh(nn.Module):
     """tanh(alpha x) w + b with scalar alpha; parameters in float32 (norms are evaluated in 32-bit)."""
 
@@ -337,6 +372,16 @@ class MixerGroup(nn.Module):
         if len(self.parts) == 1:
             return lin.norm_groups == 1 and not lin.silu_gate
         return isinstance(self.parts[0], ChunkAttention) and self.parts[0].flash and lin.norm.numel() == lin.geometry["dvp"] and lin.silu_gate
+
+    @property
+    def table_step(self) -> bool:
+        """aria_mix_step_f32 takes the group: the same mixers in float32"""
+        lin = self.parts[-1]
+        if self.w_in.dtype != f32 or not isinstance(lin, LinearAttention):
+            return False
+        if len(self.parts) == 1:
+            return lin.norm_groups == 1 and not lin.silu_gate
+        return isinstance(self.parts[0], ChunkAttention) and lin.norm_groups == lin.geometry["H"] and lin.norm.numel() == lin.geometry["dvp"] and lin.silu_gate
 
     def fill_table(self, t: hip.MixLayer, caches: list) -> None:
         lin = self.parts[-1]

@@ -573,6 +573,12 @@ int64_t aria_latent_decode_scratch(const AriaLatentStack* stack, const AriaLaten
  * epilogues: meant for T up to 16. */
 int aria_latent_decode(const AriaLatentStack* stack, const AriaLatentLayer* layers, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
                        int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
+/* One float32 step (every tensor of the stack in 32-bit) of any batch: T packed tokens of any sequences, their keys in the caches by position.  wanted: the W rows
+ * whose logits are asked for, in order (int32 on the device); W < 0: every row.  Enqueues the launches of the step run sublayer by sublayer, on the same operands;
+ * logits fp32 [W or T, V]. */
+int64_t aria_latent_step_f32_scratch(const AriaLatentStack* stack, const AriaLatentLayer* layers, int64_t T, int64_t max_len, int64_t W);
+int aria_latent_step_f32(const AriaLatentStack* stack, const AriaLatentLayer* layers, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
+                         int64_t max_len, const int32_t* wanted, int64_t W, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
 /* how many splits aria_latent_decode / a caller of aria_latent_attn should use */
 int64_t aria_latent_splits(const AriaLatentShape* s, int64_t T, int64_t max_len);
 int64_t aria_latent_splits_f32(const AriaLatentShape* s, int64_t T, int64_t max_len);
@@ -681,6 +687,12 @@ int64_t aria_mix_decode_scratch(const AriaMixStack* stack, const AriaMixLayer* r
  * ARIA_ERR_UNSUPPORTED: widths beyond the matrix-pipe attention. */
 int aria_mix_decode(const AriaMixStack* stack, const AriaMixLayer* runs, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos, int64_t max_len,
                     float* logits, void* scratch, int64_t scratch_bytes, void* stream);
+
+/* One float32 step of any batch, as aria_latent_step_f32; seq: the sequence of every token, cu: first row of every sequence [n_seq + 1]. */
+int64_t aria_mix_step_f32_scratch(const AriaMixStack* stack, const AriaMixLayer* runs, int64_t T, int64_t W);
+int aria_mix_step_f32(const AriaMixStack* stack, const AriaMixLayer* runs, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos, const int32_t* seq,
+                      const int32_t* cu, int64_t n_seq, int64_t max_len, const int32_t* wanted, int64_t W, float* logits, void* scratch, int64_t scratch_bytes,
+                      void* stream);
 
 #ifdef __cplusplus
 }

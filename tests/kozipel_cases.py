@@ -567,3 +567,38 @@ def case_bad_inputs(dev):
     assert [(r.layer, r.again) for r in c.runs] == [(0, False), (1, False), (1, True)] == O.layer_runs(cfg)
     assert [r.layer for r in KozipelConfig.from_dict(dict(cfg, loop=None)).runs] == [0, 1]
     assert (c.eps, c.residual_mult, c.logit_softcap, c.embedding_scale) == (EPS, 0.5, 12.0, 2.0)
+
+
+def case_float32_step_as_one_call(dev, monkeypatch, name):
+    """A float32 step is one call, and its logits and caches are those of the step run sublayer by sublayer (as it is with a trace), bit for bit: whole prompts,
+    portions, single tokens, some rows wanted, none, every one.  Weights put in place of others are seen; hooks are called."""
+    from aria_amd import ops
+    from aria_amd.serving import StepBatch
+
+    cfg = CONFIGS[name]
+    w = checkpoint(cfg, seed=3)
+    one, ref = build(cfg, w, dev, f32), build(cfg, w, dev, f32)
+    toks = [tokens(cfg, 12, seed=s) for s in (1, 2, 3)]
+    for m in (one, ref):
+        m.setup_caches(3, 12)
+
+    def both(seqs, starts, wanted, one_call=True):
+        batch = StepBatch.build(seqs, list(range(len(seqs))), starts, wanted, dev)
+        with monkeypatch.context() as mp:
+            if one_call:
+                mp.setattr(ops, "linear_any", None)
+            got = one.step(batch)
+        assert torch.equal(got.cpu(), ref.step(batch, []).cpu())
+
+    both([t[:n] for t, n in zip(toks, (5, 1, 4))], [0, 0, 0], [4, 5, 9])
+    both([t[a:b] for t, a, b in zip(toks, (5, 1, 4), (8, 2, 5))], [5, 1, 4], [4, 1, 0])
+    both([t[a:a + 1] for t, a in zip(toks, (8, 2, 5))], [8, 2, 5], None)
+    both([t[a:a + 1] for t, a in zip(toks[:2], (9, 3))], [9, 3], [])
+    for m in (one, ref):
+        m.head.data = m.head.data * 0.5
+    both([toks[0][10:11]], [10], None)
+    calls = []
+    hook = one.layers[0].mixer.register_forward_hook(lambda *a: calls.append(1))
+    both([toks[0][11:12]], [11], None, one_call=False)
+    hook.remove()
+    assert calls

@@ -613,6 +613,41 @@ def case_bad_inputs(dev):
         DuguzenConfig.from_dict(dict(cfg, layers=[dict(one, weights_of=1), dict(one, weights_of=0)]))
 
 
+def case_float32_step_as_one_call(dev, monkeypatch, name):
+    """A float32 step is one call, and its logits and caches are those of the step run sublayer by sublayer (as it is with a trace), bit for bit: whole prompts,
+    portions, single tokens, some rows wanted, none, every one.  Weights put in place of others are seen; hooks are called."""
+    from aria_amd import ops
+    from aria_amd.serving import StepBatch
+
+    cfg = CONFIGS[name]
+    w = checkpoint(cfg, seed=3)
+    one, ref = build(cfg, w, dev, f32), build(cfg, w, dev, f32)
+    toks = [tokens(cfg, 12, seed=s) for s in (1, 2, 3)]
+    for m in (one, ref):
+        m.setup_caches(3, 12)
+
+    def both(seqs, starts, wanted, one_call=True):
+        batch = StepBatch.build(seqs, list(range(len(seqs))), starts, wanted, dev)
+        with monkeypatch.context() as mp:
+            if one_call:
+                mp.setattr(ops, "linear_any", None)
+            got = one.step(batch)
+        assert torch.equal(got.cpu(), ref.step(batch, []).cpu())
+
+    both([t[:n] for t, n in zip(toks, (5, 1, 4))], [0, 0, 0], [4, 5, 9])
+    both([t[a:b] for t, a, b in zip(toks, (5, 1, 4), (8, 2, 5))], [5, 1, 4], [4, 1, 0])
+    both([t[a:a + 1] for t, a in zip(toks, (8, 2, 5))], [8, 2, 5], None)
+    both([t[a:a + 1] for t, a in zip(toks[:2], (9, 3))], [9, 3], [])
+    for m in (one, ref):
+        m.head.data = m.head.data * 0.5
+    both([toks[0][10:11]], [10], None)
+    calls = []
+    hook = one.layer(0).mixer.register_forward_hook(lambda *a: calls.append(1))
+    both([toks[0][11:12]], [11], None, one_call=False)
+    hook.remove()
+    assert calls
+
+
 def case_latent_attention_f32(dev, H, R, dr, dv, runs):
     """32-bit latent attention and its expansion against float64, tokens given as (slot, first position, tokens) runs: several heads and tokens a workgroup, tokens
     of several sequences, portions, an earlier position behind a later one; splits for few tokens.  32-bit sums of cw products: errors of some 1e-6.  A row

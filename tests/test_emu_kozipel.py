@@ -100,3 +100,8 @@ def test_greedy_generation(dtype, tmp_path):
 
 def test_bad_inputs():
     C.case_bad_inputs(DEV)
+
+
+@pytest.mark.parametrize("name", ["mixed", "odd"])
+def test_float32_step_as_one_call(monkeypatch, name):
+    C.case_float32_step_as_one_call(DEV, monkeypatch, name)

@@ -142,6 +142,11 @@ def test_bad_inputs():
     C.case_bad_inputs(DEV)
 
 
+@pytest.mark.parametrize("name", ["mixed", "odd"])
+def test_float32_step_as_one_call(monkeypatch, name):
+    C.case_float32_step_as_one_call(DEV, monkeypatch, name)
+
+
 @pytest.mark.parametrize("H,R,dr,dv", [(8, 256, 64, 128), (3, 36, 8, 20), (1, 64, 6, 8), (20, 52, 10, 16), (4, 384, 32, 24), (5, 21, 6, 11)])
 @pytest.mark.parametrize("runs", [[(0, 0, 41), (2, 3, 30)], [(0, 20, 3), (1, 0, 1), (0, 5, 2), (2, 60, 35)], [(1, 70, 1), (0, 4, 1), (2, 0, 1)]])
 def test_latent_attention_f32(H, R, dr, dv, runs):
