@@ -367,6 +367,22 @@ long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
 }  // namespace
 
+int aria_expert_pair_tiles(const void* X, const int32_t* rows, int64_t T, const void* w_gate, const void* w_up, void* act, const int32_t* offsets, int64_t E, int64_t M, int64_t I,
+                           int64_t K, int64_t ldx, void* stream) {
+    if (I % 128 || K % 64 || K < 64 || E <= 0 || M <= 0 || T >= (1ll << 24) || 2 * T * ldx >= (1ll << 32) || 2 * ldx >= (1ll << 24) || 2 * K >= (1ll << 24) || I >= (1ll << 24) ||
+        2 * I * K >= (1ll << 32) || !aligned16(X) || !aligned16(w_gate) || !aligned16(w_up) || !aligned16(act) || (ldx & 7))
+        return ARIA_ERR_UNSUPPORTED;
+    GemmParams p{};
+    p.A = static_cast<const bf16_t*>(X), p.B = static_cast<const bf16_t*>(w_gate), p.B_up = static_cast<const bf16_t*>(w_up), p.C2 = act;
+    p.lda = ldx, p.ldb = K, p.ldc2 = I, p.strideB = I * K;
+    p.M = int(M), p.N = int(2 * I), p.K = int(K);
+    p.mode = 1, p.E = int(E), p.offsets = offsets, p.gather_rows = rows;
+    p.glu = 1, p.glu_up_rows = 1;   // (two tensors; the distance in rows is of the 256 x 256 kernels)
+    Gemm4Plan plan;
+    plan.form = 1;
+    return aria_launch_gemm4(p, 0, 0, plan, nullptr, stream);
+}
+
 extern "C" {
 
 int aria_last_gemm_variant(void) { return g_last_variant; }
@@ -572,6 +588,7 @@ int aria_grouped_gemm_swiglu_split_bf16(const void* A, const void* Bg, const voi
     GemmParams p{};
     p.A = static_cast<const bf16_t*>(A);
     p.B = static_cast<const bf16_t*>(Bg);
+    p.B_up = static_cast<const bf16_t*>(Bu);
     p.C = H;
     p.C2 = ACT;
     p.lda = lda, p.ldb = ldb, p.ldc = ldh, p.ldc2 = ldact;
@@ -599,6 +616,7 @@ int aria_gemm_swiglu_split_bf16(const void* A, const void* Bg, const void* Bu, v
     GemmParams p{};
     p.A = static_cast<const bf16_t*>(A);
     p.B = static_cast<const bf16_t*>(Bg);
+    p.B_up = static_cast<const bf16_t*>(Bu);
     p.C = H;
     p.C2 = ACT;
     p.lda = lda, p.ldb = ldb, p.ldc = ldh, p.ldc2 = ldact;
@@ -702,6 +720,7 @@ int aria_grouped_gemm_swiglu_split_gather_bf16(const void* X, const int32_t* row
     GemmParams p{};
     p.A = static_cast<const bf16_t*>(X);
     p.B = static_cast<const bf16_t*>(Bg);
+    p.B_up = static_cast<const bf16_t*>(Bu);
     p.C = H;
     p.C2 = ACT;
     p.lda = ldx, p.ldb = ldb, p.ldc = ldh, p.ldc2 = ldact;

@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
 #pragma unroll
     for (int s = 0; s < PB; ++s) {
         int first = n0 + (B_OC ? 64 * (s / OCU) : 4 * RC * s);
-        if (GLU && s >= PB / 2) first += (UP_ROWS ? p.glu_up_rows : p.N / 2) - BN / 2;
+        if (GLU && s >= PB / 2) first += (UP_ROWS ? 0 : p.N / 2) - BN / 2;
         if (B_OC)
             offB[s] = mul24(uint32_t(oc_k + 32 * (s % OCU)), ldb2) + 2u * uint32_t(min(first + oc_col, p.N - 8));
         else
@@ -232,13 +232,15 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     // GATHER_K: the token row of this lane's k-row of a stage (past the end of the reduction: the last one, which meets zeros of B)
     auto row_of = [&](int step) __attribute__((always_inline)) { return p.gather_rows[k_begin + min(step * KD + oc_k, k_len - 1)]; };
     const char* A0 = reinterpret_cast<const char*>(p.A);
+    // (up rows of a tensor of their own: as a distance from the gate rows' addresses)
+    const long long up = UP_ROWS ? reinterpret_cast<const char*>(p.B_up) - reinterpret_cast<const char*>(p.B) : 0;
     // piece s of a stage (A's pieces first) from the step's operand addresses; the general form ends the reduction with zeros
     auto piece = [&](auto s, const char* a, const char* b, char* d) __attribute__((always_inline)) {
         constexpr int I = decltype(s)::value;
         if constexpr (I < PA)
             glds16(a + offA[I], d + 4096 * I);
         else
-            glds16(b + offB[I - PA], d + 4096 * I);
+            glds16(b + (I - PA >= PB / 2 ? up : 0) + offB[I - PA], d + 4096 * I);
     };
     auto dma = [&](int step, uint32_t at) __attribute__((always_inline)) {
         const char* a = GATHER_K ? A0 + mul24(uint32_t(row_of(step)), lda2) : gA + step * stepA;
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
 #pragma unroll
             for (int s = 0; s < PA + PB; ++s) {
                 const int k = (s < PA ? A_OC : B_OC) ? oc_k + 32 * ((s < PA ? s : s - PA) % OCU) : rc_chunk >> 1;
-                const char* src = k < tail_k ? (s < PA ? a + offA[s] : b + offB[s - PA]) : z;
+                const char* src = k < tail_k ? (s < PA ? a + offA[s] : b + (s - PA >= PB / 2 ? up : 0) + offB[s - PA]) : z;
                 hold(src);   // (one piece for the whole wave, not one for each side of the choice)
                 glds16(src, d + 4096 * s);
             }
@@ -592,11 +594,11 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     if (p.mode == 1) {
         // Rows by expert.  Up to 100 a expert its tile of 256 rows is mostly empty and the weights' stream counts, of which three stages of 48 KiB keep more in flight.
         // 64 experts of 2560 x 1664, rows each on average 28 / 73 / 140, before and now: gate and up, gathered, [K, N] 254 -> 213, 276 -> 233, (306 -> 345); two [N, K]
-        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 114, 135 -> 124, (153 -> 155), at 6 rows (109 -> 111); SwiGLU backward 144 -> 121, 160 -> 149,
+        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 114, 135 -> 124, (153 -> 155), at 6 rows (109 -> 111), [N, K] at 26 rows in a prompt (109 -> 114); SwiGLU backward 144 -> 121, 160 -> 149,
         // (185 -> 200); gate and up backward [N, K] 214 -> 207, 245 -> 220.  And where all of it is one round: 16 experts of 1024 x 768, 187 rows each, 32.6 -> 20.2 and 25 -> 16.
         if (p.K < 768 || p.N < 512) return none;
         const long long cols = p.glu ? p.N / 2 : p.N, ntn = cdiv(cols, p.glu ? 128 : 256);
-        const bool few = p.M < 100ll * p.E && (!plain || p.M >= 16ll * p.E), one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
+        const bool few = p.M < 100ll * p.E && (!plain || p.M >= 40ll * p.E), one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
         if (few || one_round) plan.form = 1;
         return plan;
     }

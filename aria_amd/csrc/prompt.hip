@@ -1,8 +1,9 @@
 // A serving step over short prompts of the gptfast (Aria) decoder in one call: packed tokens of one or several sequences, the products by the row-streaming kernels
-// of wide.hip (the experts' down-projections by the grouped tiles, beyond four rows an expert).  At these sizes a layer is fifteen launches of 5 .. 230 us;
+// of wide.hip, by the tiles of gemm4.hip from 193 tokens on, the experts' from 8 (down-projections: four) rows an expert on.  At these sizes a layer is fifteen launches of 5 .. 230 us;
 // enqueued one by one from Python they take longer than they run (four layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
 // Served: what wide.hip's products take, up to 27 rows an expert on average (6 of 64 experts: 288 tokens).
 #include "decode.h"
+#include "gemm_params.h"
 #include "rows.h"
 #include <algorithm>
 
@@ -17,8 +18,12 @@ __global__ __launch_bounds__(256) void clear_counts_kernel(int32_t* counts, int 
 struct Scratch {
     bf16_t *x, *y, *h, *qkv, *ao, *d, *logits, *scores, *act, *eo, *sact, *sh;
     int32_t *idx, *counts, *offsets, *src, *inv, *rows;
-    int64_t bytes;
+    char* ws;
+    int64_t ws_bytes, bytes;
 };
+// A dense product x [T, K] w [N, K]^T as tiles (its reduction in pieces).  Weights from HBM, us by rows / tiles: 7680 x 2560: 128 tokens 23.7 / 23.7, 192 29.3 / 28.3, 256 34.8 /
+// 29.7; 2560 x 2560: 192 16.3 / 18.1, 256 19.2 / 18.2, 288 20.9 / 19.5; 2560 x 3328: 192 20.9 / 19.0, 288 31.4 / 21.7.  Narrower: 4096 x 1536: 288 19.3 / 18.9.
+bool tiles_ahead(int64_t T, int64_t N, int64_t K) { return T > 192 && K >= 2048 && N * K >= (6 << 20) && K % 64 == 0 && N % 8 == 0; }
 Scratch layout(const int64_t* dims, int64_t T, char* base) {
     const int64_t L = dims[0], D = dims[1], E = dims[4], k = dims[5], I = dims[6], Is = dims[7];
     Scratch z{};
@@ -33,6 +38,10 @@ Scratch layout(const int64_t* dims, int64_t T, char* base) {
     z.act = rows(k * I), z.eo = rows(k * D), z.sact = rows(Is), z.sh = rows(D);
     auto ints = [&](int64_t n) { return reinterpret_cast<int32_t*>(take(4 * n)); };
     z.idx = ints(T * k), z.counts = ints(L * E), z.offsets = ints(E + 1), z.src = ints(T * k), z.inv = ints(T * k), z.rows = ints(T * k);
+    const int64_t shapes[3][2] = {{3 * D, D}, {D, D}, {D, Is}};
+    for (const auto& nk : shapes)
+        if (tiles_ahead(T, nk[0], nk[1])) z.ws_bytes = std::max(z.ws_bytes, aria_gemm_workspace_bytes(T, nk[0], nk[1], 0, 0));
+    z.ws = take(z.ws_bytes);
     z.bytes = at;
     return z;
 }
@@ -71,6 +80,17 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         x = y;
         std::swap(y, spare);
     };
+    auto product = [&](const bf16_t* a, const void* w, bf16_t* out, int64_t N, int64_t K) {
+        if (tiles_ahead(T, N, K)) return aria_gemm_bf16_ws(a, w, out, nullptr, T, N, K, 0, 0, K, K, N, 0, 0, z.ws_bytes ? z.ws : nullptr, z.ws_bytes, stream);
+        return aria_rows_gemm(a, w, out, 0, T, N, K, K, N, stream);
+    };
+    // gate and up of the experts.  Rows of an expert on average, us by rows / tiles (weights from HBM): 64 experts of 2 x 1664 x 2560: 6 192 / 206, 9 218 / 210, 12 225 / 211, 18 227 /
+    // 211, 24 247 / 215, 27 233 / 215
+    auto expert_pairs = [&](const void* gate, const void* up) {
+        int r = ARIA_ERR_UNSUPPORTED;
+        if (T * k > 8 * E) r = aria_expert_pair_tiles(z.h, z.rows, T, gate, up, z.act, z.offsets, E, T * k, I, D, D, stream);
+        return r != ARIA_ERR_UNSUPPORTED ? r : aria_rows_experts(z.h, z.rows, z.offsets, gate, up, z.act, E, T * k, I, D, D, I, stream);
+    };
 #define ARIA_TRY(call) \
     if (rc == ARIA_OK) rc = (call)
     for (int64_t li = 0; li < L; ++li) {
@@ -82,23 +102,23 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         } else {
             ARIA_TRY(aria_rmsnorm_fwd(x, nullptr, p[0], nullptr, z.h, nullptr, T, D, eps, stream));
         }
-        ARIA_TRY(aria_rows_gemm(z.h, p[1], z.qkv, 0, T, 3 * D, D, D, 3 * D, stream));
+        ARIA_TRY(product(z.h, p[1], z.qkv, 3 * D, D));
         ARIA_TRY(aria_rope_cache_rows(z.qkv, ptrs[0], slot, pos, kc, vc, T, H, hd, Smax, stream));
         ARIA_TRY(aria_attn_varlen_fwd(z.qkv, z.qkv + D, z.qkv + 2 * D, z.ao, cu, nullptr, n_seq, longest, H, H, hd, hd, 3 * D, 3 * D, 3 * D, D, 0,
                                       1.0f / sqrtf(float(hd)), stream));
-        ARIA_TRY(aria_rows_gemm(z.ao, p[2], z.d, 0, T, D, D, D, D, stream));
+        ARIA_TRY(product(z.ao, p[2], z.d, D, D));
         ARIA_TRY(aria_rmsnorm_fwd(z.d, x, p[3], y, z.h, nullptr, T, D, eps, stream));
         summed();
         ARIA_TRY(aria_rows_gemm(z.h, p[4], z.logits, 0, T, E, D, D, E, stream));
         ARIA_TRY(aria_route_and_sort(z.logits, z.scores, z.idx, z.counts + li * E, z.offsets, z.src, z.inv, z.rows, int(T), int(E), int(k), stream));
-        ARIA_TRY(aria_rows_experts(z.h, z.rows, z.offsets, p[5], p[6], z.act, E, T * k, I, D, D, I, stream));
+        ARIA_TRY(expert_pairs(p[5], p[6]));
         if (T * k <= 4 * E) {   // (beyond: the tiles, see wide.hip)
             ARIA_TRY(aria_rows_experts(z.act, nullptr, z.offsets, p[7], nullptr, z.eo, E, T * k, D, I, I, D, stream));
         } else {
             ARIA_TRY(aria_grouped_gemm_bf16(z.act, p[7], z.eo, z.offsets, E, T * k, D, I, 0, I, I, D * I, D, stream));
         }
         ARIA_TRY(aria_rows_swiglu(z.h, p[8], p[9], z.sact, T, Is, D, D, Is, stream));
-        ARIA_TRY(aria_rows_gemm(z.sact, p[10], z.sh, 0, T, D, Is, Is, D, stream));
+        ARIA_TRY(product(z.sact, p[10], z.sh, D, Is));
         ARIA_TRY(aria_moe_unpermute(z.eo, z.inv, z.scores, z.sh, z.d, T, D, k, stream));
         delta = z.d;
     }

@@ -206,7 +206,8 @@ class GroupLimitedMixture(nn.Module):
         weights, idx, counts = ops.moe_route_groups(logits, self.correction, self.groups, self.keep, self.top)
         offsets, sorted_src, inv = ops.moe_sort(idx, counts)
         g, u = self.gate, self.up
-        if h.dtype == bf16 and ops.rows_experts_take(sorted_src.numel(), self.n_experts, h.shape[1], self.ff):
+        if h.dtype == bf16 and ops.rows_experts_take(sorted_src.numel(), self.n_experts, h.shape[1], self.ff) and not (
+                ops.experts_tiles_ahead(sorted_src.numel(), self.n_experts, h.shape[1], self.ff) and ops.gather_fusable(h.shape[1]) and _glu_pair_ready(g, u)):
             act = ops.rows_experts(h, g, offsets, ops.permuted_token_rows(sorted_src, self.top), u)
             if ops.rows_experts_take(sorted_src.numel(), self.n_experts, self.ff, h.shape[1], down=True):
                 return dict(y=ops.rows_experts(act, self.down, offsets), inv=inv, weights=weights)

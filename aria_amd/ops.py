@@ -69,6 +69,13 @@ def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> boo
             and N % 8 == 0)
 
 
+def experts_tiles_ahead(M: int, E: int, K: int, N: int) -> bool:
+    """Whether the gathered tiles of gate and up are ahead of the rows by expert.  us by rows / tiles, rows an expert: 32 of 1024 x 1536: 4 39 / 40, 8 44 / 41, 12 54 / 40, 24 53 / 42, 32
+    57 / 42; 64 of 1664 x 2560: 6 192 / 206, 9 218 / 210, 18 227 / 211, 27 233 / 215; 16 of 768 x 1024: 12 14.2 / 15.6, 24 14.6 / 16.0, 32 18.9 / 16.1 (few weights: a
+    launch's ramp)."""
+    return M > 8 * E and E * K * N >= 1 << 25
+
+
 def rows_gemm(x: torch.Tensor, w: torch.Tensor, out_dtype=bf16) -> torch.Tensor:
     """x [M, K] w^T for a contiguous w [N, K], M of a few hundred at most."""
     _chk(x, name="x"), _chk(w, name="w")

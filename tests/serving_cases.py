@@ -57,11 +57,11 @@ def case_gptfast_batch(dev, engine=True):
             sched.finish(r)
 
 
-def gptfast_routed(dev, dim, head_dim, inter, block, vocab=264):
+def gptfast_routed(dev, dim, head_dim, inter, block, vocab=264, top=3):
     """Embeddings carry the directions of their experts, so that no choice is a close call."""
     from aria_amd import gptfast as G
 
-    E, k, V = 16, 3, vocab
+    E, k, V = 16, top, vocab
     args = G.ModelArgs(block_size=block, vocab_size=V, n_layer=2, n_head=dim // head_dim, dim=dim, intermediate_size=inter, rope_base=10000.0, norm_eps=1e-5,
                        num_experts=E, router_topk=k, num_shared_experts=2)
     m, g = G.Transformer(args), L.gen(5)
@@ -505,13 +505,13 @@ def gptfast_oracle(m, toks, r=lambda t: t):
     return norm(x, "norm") @ w["output.weight"].T, cache
 
 
-def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2, vocab=264):
+def case_gptfast_steps_oracle(dev, monkeypatch, dim, inter, lens, steps=2, vocab=264, top=3):
     """Prompts of several requests, tokens of all of them and a token of one against float64: logits and cache rows, each step seen to be one library call.  Bound:
     three times what 16-bit tensors between exact operations make of the same sequence."""
     from aria_amd import gptfast as G
     from aria_amd.serving import Scheduler
 
-    m, served = gptfast_routed(dev, dim, 64, inter, max(lens) + 8, vocab), []
+    m, served = gptfast_routed(dev, dim, 64, inter, max(lens) + 8, vocab, top), []
     for name in ("prompts", "run"):
         def seen(self, *a, plain=getattr(G._StepTables, name), name=name):
             out = plain(self, *a)

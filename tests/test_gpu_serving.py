@@ -102,6 +102,11 @@ def test_gptfast_steps_oracle(monkeypatch, dim, inter, lens, vocab):
     C.case_gptfast_steps_oracle(DEV, monkeypatch, dim, inter, lens, vocab=vocab)
 
 
+def test_gptfast_steps_oracle_by_tiles(monkeypatch):
+    """more tokens than the projections take by rows"""
+    C.case_gptfast_steps_oracle(DEV, monkeypatch, 2560, 640, (200, 8), top=2)
+
+
 def test_gptfast_packed_prompts():
     C.case_gptfast_packed_prompts(DEV)
     C.case_gptfast_packed_prompts(DEV, 1024, (300, 64, 65, 2, 129))
