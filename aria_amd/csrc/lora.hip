@@ -1,0 +1,303 @@
+// The thin products of a low-rank adapter (rank 8 or 16) of a training step: result = base(x) + lora_B(lora_A(dropout(x))) * scaling
+// (aria/lora/layers.py:129-139; for nn.Linear peft's adapter, the same line).  The base launch carries lora_B (the *_lora_* entries); here are
+//   down:   u = scale * x W^T                      forward with lora_A, backward with lora_B (d_u = scale * dy lora_B)
+//   up:     dx += keep ? (d_u A) / (1 - p) : 0     the adapter's input gradient through its dropout mask, added where the base's gradient lies
+//   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
+// All three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
+// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9; up as a product and a masked add 22, here 10; wgrad as
+// a split product and its sum 24, here 14.  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
+// 21 and 43); an adapted training step of 4 x 1024 tokens 11 260 / 9 870.
+#include "aria_device.h"
+#include "aria_hip.h"
+#include "elem.h"
+#include <algorithm>
+
+namespace {
+using namespace ad;
+
+constexpr int ROWS = 32;                // rows of a block
+constexpr int PAD = 32;                 // a row of the staged factor ends 64 bytes further: rows start on different banks
+constexpr int64_t LDS_MAX = 112 << 10;  // the staged factor: rank 16 up to 3552 columns
+
+// The rows of a block: block bid's tile of 32, or with offsets the bid-th of the tiles of 32 rows that start anew at every expert (collective; false: none left).
+__device__ __forceinline__ bool rows_of(const int32_t* offsets, int E, int M, int bid, int& e, int& m0, int& m1) {
+    if (!offsets) {
+        e = 0, m0 = bid * ROWS, m1 = M;
+        return m0 < M;
+    }
+    const int l = threadIdx.x & 63;
+    int before = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int n = e0 + l < E ? offsets[e0 + l + 1] - offsets[e0 + l] : 0, t = (n + ROWS - 1) / ROWS, incl = wave_incl_scan(t);
+        const unsigned long long hit = ballot(before + incl > bid);
+        if (hit) {
+            const int j = __builtin_ctzll(hit);
+            e = e0 + j;
+            m0 = offsets[e] + (bid - before - wave_bcast(incl - t, j)) * ROWS;
+            m1 = offsets[e + 1];
+            return true;
+        }
+        before += wave_bcast(incl, 63);
+    }
+    return false;
+}
+
+// u[m][n] = scale * sum_k X[m][k] W[n][k], n < r.  W: [r][K], or with w_oc [K][r]; per expert where there are offsets.
+// The factor is staged once a block, k-contiguous whichever way it lies; the eight waves take every eighth 64 columns of the reduction, four such steps of 32 rows
+// in flight each, straight from global memory (16-row fragments of v_mfma_f32_16x16x32_bf16 read 64 bytes of a row, its neighbour the other half of the line).
+// Splitting the reduction over the waves is what puts 4096 rows on 128 CUs with all of a block's bytes in flight at once.
+__global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const bf16_t* W, bf16_t* U, const int32_t* offsets, int E, int M, int K, int r, int w_oc,
+                                                        long long ldx, long long ldu, float scale) {
+    ARIA_DYN_SMEM(lds);
+    bf16_t* wt = reinterpret_cast<bf16_t*>(lds);
+    const int l = threadIdx.x & 63, lr = l & 15, kg = l >> 4, w = first_lane(int(threadIdx.x) >> 6), pitch = K + PAD, nch = K / 64;
+    int e, m0, m1;
+    if (!rows_of(offsets, E, M, blockIdx.x, e, m0, m1)) return;
+    const bf16_t* xr[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) xr[h] = X + (long long)min(m0 + 16 * h + lr, m1 - 1) * ldx + 8 * kg;   // (rows past the end: the last one, never stored)
+    s16x8 x[4][2][2];
+    auto load = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (c0 + 8 * i < nch)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) x[i][h][s] = *reinterpret_cast<const s16x8*>(xr[h] + (c0 + 8 * i) * 64 + 32 * s);
+    };
+    load(w);
+    const bf16_t* we = W + (long long)e * r * K;
+    for (int i = threadIdx.x; i < r * K / 8; i += 512) {
+        const u32x4 v = ld16(we + 8ll * i);
+        if (w_oc) {
+            const int k = i / (r / 8), n = 8 * (i % (r / 8));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                wt[(n + 2 * q) * pitch + k] = bf16_t(v[q] & 0xffffu);
+                wt[(n + 2 * q + 1) * pitch + k] = bf16_t(v[q] >> 16);
+            }
+        } else {
+            const int n = i / (K / 8), k = 8 * (i % (K / 8));
+            st16(wt + n * pitch + k, v);
+        }
+    }
+    sync();
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    const bf16_t* wr = wt + (lr & (r - 1)) * pitch + 8 * kg;   // (rank 8: columns 8 .. 15 repeat the first, never stored)
+    for (int c0 = w; c0 < nch; c0 += 32) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (c0 + 8 * i < nch)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const s16x8 b = *reinterpret_cast<const s16x8*>(wr + (c0 + 8 * i) * 64 + 32 * s);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) acc[h] = mfma16(x[i][h][s], b, acc[h]);
+                }
+        if (c0 + 32 < nch) load(c0 + 32);
+    }
+    sync();
+    float* red = reinterpret_cast<float*>(lds);   // [wave][row][16]
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[(w * ROWS + 16 * h + 4 * kg + i) * 16 + lr] = acc[h][i];
+    sync();
+    for (int i = threadIdx.x; i < ROWS * r; i += 512) {
+        const int row = i / r, n = i % r;
+        float s = 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) s += red[(q * ROWS + row) * 16 + n];
+        if (m0 + row < m1) U[(long long)(m0 + row) * ldu + n] = f2bf(scale * s);
+    }
+}
+
+__device__ __forceinline__ float half_of(const u32x4& v, int i) { return i & 1 ? bfhi(v[i >> 1]) : bflo(v[i >> 1]); }
+
+// DX[m][k] += keep ? scale * sum_j DU[m][j] A[j][k] : 0.  A: [r][K] (a_oc), else [K][r]; per expert where there are offsets.  mask null: every element is kept.
+// A lane holds eight columns of A and runs a wave's eight rows through them: a read and a write of DX, on the vector pipe in 32 bits, rounded once.
+template <int R8, bool A_OC>
+__global__ __launch_bounds__(256) void lora_up_kernel(const bf16_t* DU, const bf16_t* A, const unsigned char* mask, bf16_t* DX, const int32_t* offsets, int E, int M,
+                                                      int K, long long ldu, float scale) {
+    constexpr int r = 8 * R8, NR = ROWS / 4;
+    int e, m0, m1;
+    if (!rows_of(offsets, E, M, blockIdx.x, e, m0, m1)) return;
+    const int c = blockIdx.y * 64 + (threadIdx.x & 63), first = m0 + NR * first_lane(int(threadIdx.x) >> 6);
+    if (c >= K / 8 || first >= m1) return;
+    u32x4 old[NR];
+    unsigned keep[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const long long m = min(first + i, m1 - 1);
+        old[i] = ld16(DX + m * K + 8 * c);
+        keep[i] = mask ? mask[m * (K / 8) + c] : 255u;
+    }
+    float y[NR][8];
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) y[i][q] = 0.f;
+    const bf16_t* ae = A + (long long)e * r * K;
+#pragma unroll
+    for (int jb = 0; jb < R8; ++jb) {
+        u32x4 a[8];   // A_OC: eight columns of factor row 8 jb + i; else factor entries 8 jb .. of column 8 c + i
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] = A_OC ? ld16(ae + (long long)(8 * jb + i) * K + 8 * c) : ld16(ae + (8ll * c + i) * r + 8 * jb);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const u32x4 d = ld16(DU + (long long)min(first + i, m1 - 1) * ldu + 8 * jb);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) y[i][q] = fmaf(half_of(d, j), A_OC ? half_of(a[j], q) : half_of(a[q], j), y[i][q]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        if (first + i >= m1) break;
+        u32x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float lo = keep[i] >> (2 * q) & 1u ? scale * y[i][2 * q] : 0.f, hi = keep[i] >> (2 * q + 1) & 1u ? scale * y[i][2 * q + 1] : 0.f;
+            o[q] = pack2bf(bflo(old[i][q]) + lo, bfhi(old[i][q]) + hi);
+        }
+        st16(DX + (long long)(first + i) * K + 8 * c, o);
+    }
+}
+
+// part[split][j][n] = sum over the split's rows of Y[m][n] U[m][j], j = 8 z .. 8 z + 7.  A lane holds 8 columns x 8 factor entries in 32 bits; the eight waves of a block take
+// every eighth row of it and meet in LDS.
+constexpr int WG_ROWS = 128;
+__global__ __launch_bounds__(512) void lora_wgrad_kernel(const bf16_t* Y, const bf16_t* U, float* part, int M, int N, int r, long long ldy, long long ldu) {
+    ARIA_DYN_SMEM(lds);
+    float* red = reinterpret_cast<float*>(lds);   // [4 waves][64 sums][64 lanes]
+    const int l = threadIdx.x & 63, w = first_lane(int(threadIdx.x) >> 6), c = blockIdx.y * 64 + l, cc = min(c, N / 8 - 1), jb = blockIdx.z;
+    const int m0 = blockIdx.x * WG_ROWS, m1 = min(M, m0 + WG_ROWS);
+    float acc[8][8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc[j][q] = 0.f;
+    for (int m = m0 + w; m < m1; m += 32) {   // four rows in flight
+        u32x4 y[4], u[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = min(m + 8 * i, m1 - 1);
+            y[i] = ld16(Y + (long long)row * ldy + 8 * cc);
+            u[i] = ld16(U + (long long)row * ldu + 8 * jb);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (m + 8 * i >= m1) break;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) acc[j][q] = fmaf(half_of(u[i], j), half_of(y[i], q), acc[j][q]);
+        }
+    }
+#pragma unroll
+    for (int half = 4; half; half >>= 1) {
+        if (w >= half && w < 2 * half)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) red[((w - half) * 64 + 8 * j + q) * 64 + l] = acc[j][q];
+        sync();
+        if (w < half)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) acc[j][q] += red[(w * 64 + 8 * j + q) * 64 + l];
+        sync();
+    }
+    if (w || c >= N / 8) return;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const f32x4 v = {acc[j][4 * h], acc[j][4 * h + 1], acc[j][4 * h + 2], acc[j][4 * h + 3]};
+            *reinterpret_cast<f32x4*>(part + ((long long)blockIdx.x * r + 8 * jb + j) * N + 8ll * c + 4 * h) = v;
+        }
+}
+
+// the splits' sum: out[j][n], or with n_first out[n][j].  Four threads share four columns' splits.
+__global__ __launch_bounds__(256) void lora_wgrad_sum_kernel(const float* part, bf16_t* out, int splits, int N, int r, int n_first) {
+    ARIA_SMEM_STATIC f32x4 red[4][64];
+    const int t = threadIdx.x & 63, q = threadIdx.x >> 6, i = blockIdx.x * 64 + t;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if (i < r * N / 4)
+#pragma unroll 8
+        for (int k = q; k < splits; k += 4) s += *reinterpret_cast<const f32x4*>(part + (long long)k * r * N + 4ll * i);
+    red[q][t] = s;
+    sync();
+    if (q || i >= r * N / 4) return;
+    s = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+    const int j = 4 * i / N, n = 4 * i % N;
+    if (n_first) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) out[(long long)(n + k) * r + j] = f2bf(s[k]);
+    } else {
+        unsigned* dst = reinterpret_cast<unsigned*>(out + (long long)j * N + n);
+        dst[0] = pack2bf(s[0], s[1]);
+        dst[1] = pack2bf(s[2], s[3]);
+    }
+}
+
+bool off16(const void* p) { return reinterpret_cast<uintptr_t>(p) & 15; }
+bool thin(int64_t r) { return r == 8 || r == 16; }
+unsigned row_tiles(int64_t M, const int32_t* offsets, int64_t E) { return unsigned(offsets ? M / ROWS + E : (M + ROWS - 1) / ROWS); }
+
+}  // namespace
+
+extern "C" {
+
+int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
+                        float scale, void* stream) {
+    if (!X || !W || !U || M < 0 || K <= 0 || r <= 0 || (offsets && E <= 0)) return ARIA_ERR_INVALID;
+    const int64_t lds = std::max<int64_t>(r * (K + PAD) * 2, 8 * ROWS * 16 * 4);
+    if (!thin(r) || (K & 63) || lds > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
+    if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
+    if (M == 0) return ARIA_OK;
+    ARIA_LAUNCH(lora_down_kernel, dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
+                static_cast<bf16_t*>(U), offsets, int(E), int(M), int(K), int(r), w_oc, (long long)ldx, (long long)ldu, scale);
+    return aria_check_launch();
+}
+
+int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,
+                      int64_t ldu, float scale, void* stream) {
+    if (!DU || !A || !DX || M < 0 || K <= 0 || r <= 0 || (offsets && E <= 0)) return ARIA_ERR_INVALID;
+    if (!thin(r) || (K & 7) || K >= (1ll << 24) || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
+    if (off16(DU) || off16(A) || off16(DX) || (ldu & 7)) return ARIA_ERR_ALIGN;
+    if (M == 0) return ARIA_OK;
+    const dim3 grid(row_tiles(M, offsets, E), unsigned((K / 8 + 63) / 64)), block(256);
+#define UP(R8, OC)                                                                                                                                    \
+    ARIA_LAUNCH((lora_up_kernel<R8, OC>), grid, block, 0, stream, static_cast<const bf16_t*>(DU), static_cast<const bf16_t*>(A),                      \
+                static_cast<const unsigned char*>(mask), static_cast<bf16_t*>(DX), offsets, int(E), int(M), int(K), (long long)ldu, scale)
+    if (r == 8 && a_oc)
+        UP(1, true);
+    else if (r == 8)
+        UP(1, false);
+    else if (a_oc)
+        UP(2, true);
+    else
+        UP(2, false);
+#undef UP
+    return aria_check_launch();
+}
+
+int aria_lora_wgrad_bf16(const void* Y, const void* U, void* out, int n_first, int64_t M, int64_t N, int64_t r, int64_t ldy, int64_t ldu, float* workspace,
+                         int64_t workspace_floats, void* stream) {
+    if (!Y || !U || !out || !workspace || M <= 0 || N <= 0 || r <= 0) return ARIA_ERR_INVALID;
+    const int64_t splits = (M + WG_ROWS - 1) / WG_ROWS;
+    if (!thin(r) || (N & 7) || M >= (1ll << 30) || N >= (1ll << 24)) return ARIA_ERR_UNSUPPORTED;
+    if (workspace_floats < splits * r * N) return ARIA_ERR_INVALID;
+    if (off16(Y) || off16(U) || off16(out) || off16(workspace) || (ldy & 7) || (ldu & 7)) return ARIA_ERR_ALIGN;
+    ARIA_LAUNCH(lora_wgrad_kernel, dim3(unsigned(splits), unsigned((N / 8 + 63) / 64), unsigned(r / 8)), dim3(512), 65536, stream, static_cast<const bf16_t*>(Y),
+                static_cast<const bf16_t*>(U), workspace, int(M), int(N), int(r), (long long)ldy, (long long)ldu);
+    ARIA_LAUNCH(lora_wgrad_sum_kernel, dim3(unsigned((r * N / 4 + 63) / 64)), dim3(256), 0, stream, workspace, static_cast<bf16_t*>(out), int(splits), int(N), int(r),
+                n_first);
+    return aria_check_launch();
+}
+
+}  // extern "C"

@@ -7,14 +7,14 @@ nn.Linear targets -- the same line):
     result = base(x) + lora_B(lora_A(dropout(x))) * scaling              base weights frozen, A / B trainable
 
 What runs here, per module:
-  * ``u = scaling * lora_A(dropout(x))`` -- a skinny GEMM (N = r) on the dropped input (``ops.dropout``: one pass, one mask byte per 8
-    elements kept for the backward);
+  * ``u = scaling * lora_A(dropout(x))`` -- a thin product (``ops.lora_down``, ranks 8 and 16; a general product and a scaling else) on the dropped
+    input (``ops.dropout``: one pass, one mask byte per 8 elements kept for the backward);
   * the base launch with the adapter's second projection as a K-EXTENSION (``ops.*_lora``: one extra K-tile fed from u and lora_B): no
     output-sized ``base + delta`` pass, and the fused epilogues keep working -- fc1 + SwiGLU, gate|up + SwiGLU, the q|k|v and gate|up wide
     launches (their adapters enter side by side with a block-diagonal B);
   * backward: the base input gradients exactly as the un-adapted layer computes them (weight gradients of the frozen base are skipped);
-    per adapter d_u = scaling * dy lora_B^T (skinny), d lora_B = u^T dy, d lora_A = dropout(x)^T d_u, and the adapter's input gradient
-    ``mask * (d_u lora_A) / (1 - p)`` added into dx (``ops.dropout_bwd_``; without dropout: an accumulating GEMM).
+    per adapter d_u = scaling * dy lora_B^T (thin), d lora_B = u^T dy, d lora_A = dropout(x)^T d_u (``ops.lora_wgrad``), and the adapter's input
+    gradient ``mask * (d_u lora_A) / (1 - p)`` added into dx in one pass (``ops.lora_up_``; other ranks: a product, then ``ops.dropout_bwd_``).
 Everything else of the layer (RMSNorm with the residual folded in, RoPE, flash attention, router, dispatch, un-permute + shared add) is the
 un-adapted layer's code path (aria_amd.functional).  The module-by-module form (aria_amd.lora.GroupedGemmLoraLayer / LinearLoraLayer called
 as modules) stays as the reference arrangement the tests compare against.
@@ -45,6 +45,11 @@ class LoraSite:
 
 def _scaled(u: torch.Tensor, s: float) -> torch.Tensor:
     return u if s == 1.0 else (u.float() * s).to(bf16)   # (u is [rows, r]: a few hundred KB)
+
+
+def _factor(w: torch.Tensor) -> torch.Tensor:
+    """An adapter factor as the thin products read it: dense and on a 16-byte boundary."""
+    return w if w.is_contiguous() and w.data_ptr() % 16 == 0 else w.clone(memory_format=torch.contiguous_format)
 
 
 class _Drop:
@@ -82,7 +87,10 @@ def dense_lora_fwd(x: torch.Tensor, w: torch.Tensor, sites: List[Optional[LoraSi
     for j, s in live:
         r = s.a.shape[0]
         d = _Drop(x, s.p, training, _seed(seeds))
-        U[:, c0:c0 + r] = _scaled(ops.gemm(d.xd, s.a), s.scaling)
+        if ops.lora_thin(r, x.shape[1]):
+            ops.lora_down(d.xd, _factor(s.a), s.scaling, w_oc=False, out=U[:, c0:c0 + r])
+        else:
+            U[:, c0:c0 + r] = _scaled(ops.gemm(d.xd, s.a), s.scaling)
         Bx[starts[j]:starts[j] + rows[j], c0:c0 + r] = s.b
         drops.append(d)
         c0 += r
@@ -95,18 +103,26 @@ def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: L
     grads[key] = (dA, dB)."""
     if ctx is None:
         return
-    dU = ops.gemm(dy, ctx["Bx"], b_oc=True)                       # [T, R] = dy Bx  (block-diagonal: column block j = dy_j lora_B_j)
-    dBx = ops.gemm(dy, ctx["U"], a_oc=True, b_oc=True)            # [N, R] = dy^T U (scaling is inside U)
+    live, starts, rows, U = ctx["live"], ctx["starts"], ctx["rows"], ctx["U"]
+    thin = dx.is_contiguous() and dx.shape[0] > 0 and all(ops.lora_thin(s.a.shape[0], n) and starts[j] % 8 == 0 for j, s in live for n in (rows[j], dx.shape[1]))
+    if not thin:
+        dU = ops.gemm(dy, ctx["Bx"], b_oc=True)                   # [T, R] = dy Bx  (block-diagonal: column block j = dy_j lora_B_j)
+        dBx = ops.gemm(dy, U, a_oc=True, b_oc=True)               # [N, R] = dy^T U (scaling is inside U)
     c0 = 0
-    for (j, s), d in zip(ctx["live"], ctx["drops"]):
-        r = s.a.shape[0]
-        du = _scaled(dU[:, c0:c0 + r].contiguous(), s.scaling)
-        dA = ops.gemm(du, d.xd, a_oc=True, b_oc=True)             # [r, K] = d_u^T dropout(x)
-        dB = dBx[ctx["starts"][j]:ctx["starts"][j] + ctx["rows"][j], c0:c0 + r].contiguous()
-        if d.mask is None:
-            ops.gemm(du, s.a, b_oc=True, out=dx, accumulate=True)
+    for (j, s), d in zip(live, ctx["drops"]):
+        r, r0, r1 = s.a.shape[0], starts[j], starts[j] + rows[j]
+        if thin:
+            du = ops.lora_down(dy[:, r0:r1], _factor(s.b), s.scaling, w_oc=True)
+            dA, dB = ops.lora_wgrad(d.xd, du, n_first=False), ops.lora_wgrad(dy[:, r0:r1], U[:, c0:c0 + r], n_first=True)
+            ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p)
         else:
-            ops.dropout_bwd_(dx, ops.gemm(du, s.a, b_oc=True), d.mask, d.p)
+            du = _scaled(dU[:, c0:c0 + r].contiguous(), s.scaling)
+            dA = ops.gemm(du, d.xd, a_oc=True, b_oc=True)         # [r, K] = d_u^T dropout(x)
+            dB = dBx[r0:r1, c0:c0 + r].contiguous()
+            if d.mask is None:
+                ops.gemm(du, s.a, b_oc=True, out=dx, accumulate=True)
+            else:
+                ops.dropout_bwd_(dx, ops.gemm(du, s.a, b_oc=True), d.mask, d.p)
         grads[keys[j]] = (dA, dB)
         c0 += r
 
@@ -118,7 +134,10 @@ def grouped_lora_fwd(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, si
         out = ops.grouped_gemm_swiglu(x, w, offsets, want_h=want_h) if glu else ops.grouped_gemm(x, w, offsets)
         return out, None
     d = _Drop(x, site.p, training, _seed(seeds))
-    U = _scaled(ops.grouped_gemm(d.xd, site.a, offsets), site.scaling)                      # [M, r]
+    if ops.lora_thin(site.a.shape[2], x.shape[1]):
+        U = ops.lora_down(d.xd, _factor(site.a), site.scaling, w_oc=True, offsets=offsets)           # [M, r]
+    else:
+        U = _scaled(ops.grouped_gemm(d.xd, site.a, offsets), site.scaling)
     out = ops.grouped_gemm_swiglu_lora(x, w, offsets, U, site.b, want_h=want_h) if glu else ops.grouped_gemm_lora(x, w, offsets, U, site.b)
     return out, dict(site=site, drop=d, U=U)
 
@@ -128,14 +147,21 @@ def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Ten
         return
     s, d = ctx["site"], ctx["drop"]
     E = s.a.shape[0]
-    du = _scaled(ops.grouped_gemm(dy, s.b, offsets, w_is_kn=False), s.scaling)              # [M, r] = dy lora_B[e]^T
+    thin = ops.lora_thin(s.a.shape[2], dy.shape[1]) and dx.is_contiguous()
+    if thin:
+        du = ops.lora_down(dy, _factor(s.b), s.scaling, w_oc=False, offsets=offsets)                 # [M, r] = dy lora_B[e]^T
+    else:
+        du = _scaled(ops.grouped_gemm(dy, s.b, offsets, w_is_kn=False), s.scaling)
     dB = ops.grouped_gemm_wgrad(ctx["U"], dy, offsets, E)                                   # [E, r, N]
     dA = ops.grouped_gemm_wgrad(d.xd, du, offsets, E)                                       # [E, K, r]
-    term = ops.grouped_gemm(du, s.a, offsets, w_is_kn=False)                                # [M, K] = d_u lora_A[e]^T
-    if d.mask is None:
-        dx.add_(term)
+    if thin:
+        ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p, offsets=offsets)                             # d_u lora_A[e]^T
     else:
-        ops.dropout_bwd_(dx, term, d.mask, d.p)
+        term = ops.grouped_gemm(du, s.a, offsets, w_is_kn=False)
+        if d.mask is None:
+            dx.add_(term)
+        else:
+            ops.dropout_bwd_(dx, term, d.mask, d.p)
     grads[key] = (dA, dB)
 
 

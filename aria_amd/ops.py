@@ -274,6 +274,54 @@ def dropout_bwd_(dx: torch.Tensor, term: torch.Tensor, mask: torch.Tensor, p: fl
     return dx
 
 
+def lora_thin(r: int, K: int) -> bool:
+    """Adapters whose thin products have kernels of their own: rank 8 or 16 on a reduction of whole 64-column steps whose factor fits on chip.  Above that rank the
+    256-wide tiles are no longer mostly padding."""
+    return r in (8, 16) and K % 64 == 0 and r * (K + 32) <= 57344
+
+
+def lora_down(x: torch.Tensor, w: torch.Tensor, scale: float, w_oc: bool, offsets=None, out=None) -> torch.Tensor:
+    """bf16(scale * x w^T): x [M, K] (unit-stride rows), w [r, K], or [K, r] with ``w_oc``; with ``offsets`` a leading expert dimension.  out: [M, r], strided rows."""
+    _chk(x, name="x"), _chk(w, name="w")
+    M, K = x.shape
+    r = w.shape[-1] if w_oc else w.shape[-2]
+    if not w.is_contiguous() or tuple(w.shape[-2:]) != ((K, r) if w_oc else (r, K)) or (w.dim() == 3) != (offsets is not None):
+        raise ValueError("lora_down: w must be a contiguous factor of x's width")
+    out = torch.empty((M, r), dtype=x.dtype, device=x.device) if out is None else out
+    if tuple(out.shape) != (M, r):
+        raise ValueError("lora_down: out must be [M, r]")
+    hip.get_lib().call("aria_lora_down_bf16", _p(x), _p(w), int(w_oc), _p(out), _p(offsets) if offsets is not None else None, w.shape[0] if offsets is not None else 1, M, K, r,
+                       _rowmajor_2d(x, "x"), _rowmajor_2d(out, "out"), float(scale), _stream(x))
+    return out
+
+
+def lora_up_(dx: torch.Tensor, du: torch.Tensor, a: torch.Tensor, mask, p: float, offsets=None) -> torch.Tensor:
+    """dx += mask * (du a) / (1 - p) in place: a [r, K], with ``offsets`` [E, K, r]; mask None: everything is kept and nothing scaled."""
+    _chk(dx, name="dx"), _chk(du, name="du"), _chk(a, name="a")
+    M, K = dx.shape
+    r = du.shape[1]
+    if not (dx.is_contiguous() and a.is_contiguous()) or du.shape[0] != M or (mask is not None and mask.numel() * 8 != dx.numel()):
+        raise ValueError("lora_up_: contiguous dx and a, one mask byte per 8 elements")
+    if tuple(a.shape) != ((r, K) if offsets is None else (a.shape[0], K, r)):
+        raise ValueError("lora_up_: a must be [r, K], the experts' [E, K, r]")
+    hip.get_lib().call("aria_lora_up_bf16", _p(du), _p(a), int(offsets is None), _p(mask) if mask is not None else None, _p(dx), _p(offsets) if offsets is not None else None,
+                       a.shape[0] if offsets is not None else 1, M, K, r, _rowmajor_2d(du, "du"), 1.0 if mask is None else 1.0 / (1.0 - p), _stream(dx))
+    return dx
+
+
+def lora_wgrad(y: torch.Tensor, u: torch.Tensor, n_first: bool) -> torch.Tensor:
+    """u^T y as [r, N], or with ``n_first`` its transpose [N, r]: y [M, N], u [M, r], unit-stride rows."""
+    _chk(y, name="y"), _chk(u, name="u")
+    M, N = y.shape
+    r = u.shape[1]
+    if u.shape[0] != M:
+        raise ValueError("lora_wgrad: y and u must have the same rows")
+    out = torch.empty((N, r) if n_first else (r, N), dtype=y.dtype, device=y.device)
+    ws = torch.empty(((M + 127) // 128 * r * N,), dtype=torch.float32, device=y.device)
+    hip.get_lib().call("aria_lora_wgrad_bf16", _p(y), _p(u), _p(out), int(n_first), M, N, r, _rowmajor_2d(y, "y"), _rowmajor_2d(u, "u"), _p(ws), ws.numel(), _stream(y))
+    return out
+
+
 # ------------------------------------------------------------------------------------------------ LoRA as a K-extension (SURVEY 8(f)3)
 def _lora_ext_ok(K: int, ext_k: int) -> bool:
     import os

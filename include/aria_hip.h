@@ -141,6 +141,18 @@ int aria_grouped_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, vo
 int aria_dropout_fwd_bf16(const void* x, void* out, void* mask, int64_t n, float p, uint64_t seed, void* stream);
 int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t n, float p, int accumulate, void* stream);
 
+/* The thin products of an adapter of rank r = 8 or 16 (else ARIA_ERR_UNSUPPORTED).  offsets: null, or the experts' row offsets [E + 1] -- the factor is then one per
+ * expert, r K elements apart.
+ * _down: U [M, r] (row stride ldu) = bf16(scale * X W^T), W [r, K] or with w_oc [K, r]; K % 64 == 0, r (K + 32) <= 57344.
+ * _up:   DX [M, K] += keep ? scale * (DU A) : 0, A [r, K] with a_oc, else [K, r]; mask as aria_dropout_fwd_bf16 writes it (null: everything is kept), K % 8 == 0.
+ * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 128 rows begun. */
+int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
+                        float scale, void* stream);
+int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,
+                      int64_t ldu, float scale, void* stream);
+int aria_lora_wgrad_bf16(const void* Y, const void* U, void* out, int n_first, int64_t M, int64_t N, int64_t r, int64_t ldy, int64_t ldu, float* workspace,
+                         int64_t workspace_floats, void* stream);
+
 /* K2 for the TRAINING step (round 5): the weight gradient of experts.fc1 through the dispatcher's index -- dW[e] = sum over the expert's permuted rows r
  * of X[rows[r]]^T dY[r] (autograd of experts_gemm(index_select(x, sorted // topk), fc1), moe_lm.py:326-334, 467-484) -- so that the [6T, D] permuted copy
  * of the tokens is never written: forward = aria_grouped_gemm_swiglu_gather_bf16, weight gradient = this.  The indices of a K-tile reach the loader as one

@@ -1128,6 +1128,50 @@ def case_router_fused(dev, T, D, E, k):
     assert int(counts.sum()) == T * k
 
 
+def case_lora_thin(dev, T, K, N, r, counts=None, p=0.0):
+    """The thin products of an adapter (down, up through the dropout mask, weight gradient) against 64-bit ones of the same bf16 operands: every result is a 32-bit
+    sum rounded once to bf16 -- half a unit of the last place (2^-9 of the result) and the sum's own error (a few 2^-24 of the sum of magnitudes)."""
+    from aria_amd import ops
+
+    f64 = torch.float64
+    T = T if counts is None else sum(counts)
+    x, dy, dx = rnd(T, K, seed=1), rnd(T, N + 16, seed=2)[:, 8:8 + N], rnd(T, K, seed=3)
+    E = 1 if counts is None else len(counts)
+    a, b = rnd(E, r, K, seed=4, scale=0.3), rnd(E, N, r, seed=5, scale=0.3)       # lora_A [r, K], lora_B [N, r]; the experts hold both transposed
+    off = torch.tensor([0] + list(counts or [T])).cumsum(0)
+    of = None if counts is None else off.to(torch.int32).to(dev)
+    x, dy, dx = x.to(dev), rnd(T, N + 16, seed=2).to(dev)[:, 8:8 + N], dx.to(dev)
+    wa, wb = (a[0], b[0]) if counts is None else (a.transpose(1, 2).contiguous(), b.transpose(1, 2).contiguous())
+    wa, wb = wa.to(dev), wb.to(dev)
+
+    def by_expert(y, w):   # [T, n] x [E, n, m] -> [T, m]
+        return torch.cat([y[off[e]:off[e + 1]].to(f64).cpu() @ w[e].to(f64) for e in range(E)])
+
+    def near(got, want, size):
+        got = got.to(f64).cpu()
+        assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size + 1e-30).all()), float((got - want).abs().max())
+
+    U = torch.zeros((T, 2 * r), dtype=bf16, device=dev)
+    ops.lora_down(x, wa, 1.7, w_oc=counts is not None, offsets=of, out=U[:, r:])
+    near(U[:, r:], 1.7 * by_expert(x, a.transpose(1, 2)), 1.7 * by_expert(x.abs(), a.abs().transpose(1, 2)))
+    assert not bool(U[:, :r].any())
+    du = ops.lora_down(dy, wb, 0.6, w_oc=counts is None, offsets=of)
+    near(du, 0.6 * by_expert(dy, b), 0.6 * by_expert(dy.abs(), b.abs()))
+    mask = ops.dropout(x, p, 77)[1] if p else None
+    keep = ((mask.cpu().to(torch.int32)[:, None] >> torch.arange(8)) & 1).reshape(T, K).to(f64) / (1 - p) if p else torch.ones(T, K, dtype=f64)
+    before = dx.to(f64).cpu()
+    ops.lora_up_(dx, du, wa, mask, p, offsets=of)
+    near(dx, before + keep * by_expert(du, a), before.abs() + keep * by_expert(du.abs(), a.abs()))
+    if counts is None:
+        for y, u, first in ((x, du, False), (dy, U[:, r:], True)):
+            w, m = u.to(f64).cpu().t() @ y.to(f64).cpu(), u.abs().to(f64).cpu().t() @ y.abs().to(f64).cpu()
+            near(ops.lora_wgrad(y, u, n_first=first), w.t() if first else w, m.t() if first else m)
+
+
+LORA_THIN = [(1, 64, 64, 8, None, 0.0), (33, 128, 192, 16, None, 0.3), (264, 576, 128, 8, None, 0.05), (0, 128, 64, 8, [70, 0, 33, 5, 0], 0.3),
+             (0, 64, 128, 16, [1, 0, 32] + [3] * 70, 0.0)]
+
+
 def case_gemm_qkv_rope_hf(dev, B, S, D, hd, K):
     """LlamaAttention's q | k | v projection + half-split RoPE in one launch (gemm3_kernel<false, false, 10>) == gemm + rope_ (the stand-alone
     kernel), bit for bit; v columns untouched; the rotation itself against the oracle's apply_rope_half on the bf16-rounded product."""

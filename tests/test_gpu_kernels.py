@@ -241,6 +241,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(B, S, D, hd, K):   # q | k | v proje
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K) == (D >= 2560)
 
 
+@pytest.mark.parametrize("T,K,N,r,counts,p", C.LORA_THIN + [(4096, 2560, 3328, 8, None, 0.05), (1000, 3328, 2560, 16, None, 0.0), (0, 2560, 1664, 8, [300, 0, 1500, 70], 0.05)])
+def test_lora_thin_products(T, K, N, r, counts, p):
+    C.case_lora_thin(DEV, T, K, N, r, counts, p)
+
+
 @pytest.mark.parametrize("T,D,E,k", [(70, 256, 64, 6), (16384, 2560, 64, 6), (4099, 2560, 64, 6), (33, 512, 32, 2)])
 def test_router_fused_is_gemm_plus_route(T, D, E, k):   # K1: gating GEMM + top-k + softmax + histogram in one launch, bit for bit
     C.case_router_fused(DEV, T, D, E, k)
