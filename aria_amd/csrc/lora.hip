@@ -5,8 +5,8 @@
 //   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
 // All three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
 // 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9; up as a product and a masked add 22, here 10; wgrad as
-// a split product and its sum 24, here 14.  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
-// 21 and 43); an adapted training step of 4 x 1024 tokens 11 260 / 9 870.
+// a split product and its sum 24, here 11 (64 rows a block: 12.5 us on cold rows, with 128 and four loads in flight a wave 15.5).  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
+// 21 and 43); an adapted training step of 4 x 1024 tokens 11 470 / 9 780.
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "elem.h"
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void lora_up_kernel(const bf16_t* DU, const bf
 
 // part[split][j][n] = sum over the split's rows of Y[m][n] U[m][j], j = 8 z .. 8 z + 7.  A lane holds 8 columns x 8 factor entries in 32 bits; the eight waves of a block take
 // every eighth row of it and meet in LDS.
-constexpr int WG_ROWS = 128;
+constexpr int WG_ROWS = 64;
 __global__ __launch_bounds__(512) void lora_wgrad_kernel(const bf16_t* Y, const bf16_t* U, float* part, int M, int N, int r, long long ldy, long long ldu) {
     ARIA_DYN_SMEM(lds);
     float* red = reinterpret_cast<float*>(lds);   // [4 waves][64 sums][64 lanes]
@@ -179,22 +179,20 @@ __global__ __launch_bounds__(512) void lora_wgrad_kernel(const bf16_t* Y, const 
     for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int q = 0; q < 8; ++q) acc[j][q] = 0.f;
-    for (int m = m0 + w; m < m1; m += 32) {   // four rows in flight
-        u32x4 y[4], u[4];
+    u32x4 y[WG_ROWS / 8], u[WG_ROWS / 8];   // (every load of the wave in flight at once)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = min(m + 8 * i, m1 - 1);
-            y[i] = ld16(Y + (long long)row * ldy + 8 * cc);
-            u[i] = ld16(U + (long long)row * ldu + 8 * jb);
-        }
+    for (int i = 0; i < WG_ROWS / 8; ++i) {
+        const int row = min(m0 + w + 8 * i, m1 - 1);
+        y[i] = ld16(Y + (long long)row * ldy + 8 * cc);
+        u[i] = ld16(U + (long long)row * ldu + 8 * jb);
+    }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (m + 8 * i >= m1) break;
+    for (int i = 0; i < WG_ROWS / 8; ++i) {
+        if (m0 + w + 8 * i >= m1) break;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-                for (int q = 0; q < 8; ++q) acc[j][q] = fmaf(half_of(u[i], j), half_of(y[i], q), acc[j][q]);
-        }
+            for (int q = 0; q < 8; ++q) acc[j][q] = fmaf(half_of(u[i], j), half_of(y[i], q), acc[j][q]);
     }
 #pragma unroll
     for (int half = 4; half; half >>= 1) {

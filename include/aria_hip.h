@@ -145,7 +145,7 @@ int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t 
  * expert, r K elements apart.
  * _down: U [M, r] (row stride ldu) = bf16(scale * X W^T), W [r, K] or with w_oc [K, r]; K % 64 == 0, r (K + 32) <= 57344.
  * _up:   DX [M, K] += keep ? scale * (DU A) : 0, A [r, K] with a_oc, else [K, r]; mask as aria_dropout_fwd_bf16 writes it (null: everything is kept), K % 8 == 0.
- * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 128 rows begun. */
+ * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 64 rows begun. */
 int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
                         float scale, void* stream);
 int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,
