@@ -1,10 +1,11 @@
 // The thin products of a low-rank adapter (rank 8 or 16) of a training step: result = base(x) + lora_B(lora_A(dropout(x))) * scaling
 // (aria/lora/layers.py:129-139; for nn.Linear peft's adapter, the same line).  The base launch carries lora_B (the *_lora_* entries); here are
-//   down:   u = scale * x W^T                      forward with lora_A, backward with lora_B (d_u = scale * dy lora_B)
+//   scale:  u * scaling                            into the adapter's columns of the launch's extension
+//   down:   d_u = scale * dy W^T                   with lora_B
 //   up:     dx += keep ? (d_u A) / (1 - p) : 0     the adapter's input gradient through its dropout mask, added where the base's gradient lies
 //   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
 // All three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
-// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9; up as a product and a masked add 22, here 10; wgrad as
+// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9 (the scaling alone 16 with its copy, here SC_US); up as a product and a masked add 22, here 10; wgrad as
 // a split product and its sum 24, here 11 (64 rows a block: 12.5 us on cold rows, with 128 and four loads in flight a wave 15.5).  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
 // 21 and 43); an adapted training step of 4 x 1024 tokens 11 470 / 9 780.
 #include "aria_device.h"
@@ -40,6 +41,16 @@ __device__ __forceinline__ bool rows_of(const int32_t* offsets, int E, int M, in
         before += wave_bcast(incl, 63);
     }
     return false;
+}
+
+__global__ __launch_bounds__(256) void lora_scale_kernel(const bf16_t* u, bf16_t* out, long long n, int pieces, long long ldo, float scale) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const u32x4 v = ld16(u + 8 * i);
+    u32x4 o;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) o[q] = pack2bf(bflo(v[q]) * scale, bfhi(v[q]) * scale);
+    st16(out + i / pieces * ldo + 8 * (i % pieces), o);
 }
 
 // u[m][n] = scale * sum_k X[m][k] W[n][k], n < r.  W: [r][K], or with w_oc [K][r]; per expert where there are offsets.
@@ -249,6 +260,17 @@ unsigned row_tiles(int64_t M, const int32_t* offsets, int64_t E) { return unsign
 }  // namespace
 
 extern "C" {
+
+int aria_lora_scale_bf16(const void* U, void* OUT, int64_t M, int64_t r, int64_t ldo, float scale, void* stream) {
+    if (!U || !OUT || M < 0 || r <= 0) return ARIA_ERR_INVALID;
+    if (off16(U) || off16(OUT) || (r & 7) || (ldo & 7)) return ARIA_ERR_ALIGN;
+    if (M == 0) return ARIA_OK;
+    const int64_t n = M * (r / 8);
+    if (n >= (1ll << 38)) return ARIA_ERR_UNSUPPORTED;
+    ARIA_LAUNCH(lora_scale_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, static_cast<const bf16_t*>(U), static_cast<bf16_t*>(OUT), (long long)n,
+                int(r / 8), (long long)ldo, scale);
+    return aria_check_launch();
+}
 
 int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
                         float scale, void* stream) {

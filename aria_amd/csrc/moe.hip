@@ -211,8 +211,6 @@ __global__ __launch_bounds__(256) void route_groups_kernel(const float* logits, 
 }
 
 // ------------------------------------------------------------------------------------------- stable sort (E <= 64)
-constexpr int SORT_CHUNK = 2048;
-
 __device__ __forceinline__ unsigned long long match_mask(int key, const unsigned long long (&bal)[6], unsigned long long valid) {
     unsigned long long m = valid;
 #pragma unroll
@@ -220,77 +218,86 @@ __device__ __forceinline__ unsigned long long match_mask(int key, const unsigned
     return m;
 }
 
+// More than SORT_SMALL entries: two launches, a wave per 1024 entries in both, all of a wave's entries loaded at once.  What bounds them is latency: a count
+// per chunk, then every block adds the chunks in front of its own (coalesced 256-byte rows, four waves) instead of a launch in between.  22 000 entries on 32 experts:
+// a wave's 2048 entries one load after the other, and the sums as a third launch 29 us, with the token rows as two more 40; now SORT_US.
+constexpr int SORT_CHUNK = 1024, SORT_PER = SORT_CHUNK / 64;
+
 // pass 1: per-chunk histogram (lane e = expert e)
-__global__ __launch_bounds__(64) void sort_count_kernel(const int32_t* idx, int32_t* chunk_counts, int M) {
-    const int l = threadIdx.x, c = blockIdx.x;
-    int cnt = 0;
-    const int begin = c * SORT_CHUNK, end = min(M, begin + SORT_CHUNK);
-    for (int i0 = begin; i0 < end; i0 += 64) {
-        const int i = i0 + l;
-        const bool valid = i < end;
-        const int e = valid ? idx[i] : 0;
+__global__ __launch_bounds__(256) void sort_count_kernel(const int32_t* idx, int32_t* chunk_counts, int M, int nchunks) {
+    const int l = threadIdx.x & 63, c = blockIdx.x * 4 + first_lane(int(threadIdx.x) >> 6);
+    if (c >= nchunks) return;
+    int v[SORT_PER], cnt = 0;
+#pragma unroll
+    for (int j = 0; j < SORT_PER; ++j) {
+        const int i = c * SORT_CHUNK + 64 * j + l;
+        v[j] = i < M ? idx[i] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < SORT_PER; ++j) {
         unsigned long long bal[6];
 #pragma unroll
-        for (int b = 0; b < 6; ++b) bal[b] = ballot((e >> b) & 1);
-        const unsigned long long vm = ballot(valid);
-        cnt += __builtin_popcountll(match_mask(l, bal, vm));
+        for (int b = 0; b < 6; ++b) bal[b] = ballot((v[j] >> b) & 1);
+        cnt += __builtin_popcountll(match_mask(l, bal, ballot(c * SORT_CHUNK + 64 * j + l < M)));
     }
     chunk_counts[c * 64 + l] = cnt;
 }
 
-// pass 2: offsets = exclusive scan of counts; chunk_base[c][e] = offsets[e] + sum_{c' < c} chunk_counts[c'][e]
-__global__ __launch_bounds__(64) void sort_scan_kernel(const int32_t* counts, const int32_t* chunk_counts, int32_t* chunk_base,
-                                                       int32_t* offsets, int E, int nchunks) {
-    const int l = threadIdx.x;
-    const int cnt = l < E ? counts[l] : 0;
-    int incl = cnt;
+// pass 2: offsets = exclusive scan of counts; stable positions, and with rows the token of every place and ``pad`` zeros behind them
+__global__ __launch_bounds__(256) void sort_scatter_kernel(const int32_t* idx, const int32_t* counts, const int32_t* chunk_counts, int32_t* offsets, int32_t* sorted_src,
+                                                           int32_t* inv, int32_t* rows, int E, int M, int k, int nchunks, int pad) {
+    ARIA_SMEM_STATIC int part[4][64];
+    const int l = threadIdx.x & 63, w = first_lane(int(threadIdx.x) >> 6), c0 = blockIdx.x * 4, c = c0 + w;
+    int v[SORT_PER];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int v = shfl(incl, (l - d) & 63);
-        if (l >= d) incl += v;
+    for (int j = 0; j < SORT_PER; ++j) {
+        const int i = c * SORT_CHUNK + 64 * j + l;
+        v[j] = i < M ? idx[i] : 0;
     }
-    int running = incl - cnt;
-    if (l < E) offsets[l] = running;
-    if (l == E - 1) offsets[E] = incl;
-    for (int c = 0; c < nchunks; ++c) {
-        chunk_base[c * 64 + l] = running;
-        running += chunk_counts[c * 64 + l];
+    const int cnt = l < E ? counts[l] : 0;
+    int sum = 0;
+#pragma unroll 4
+    for (int q = w; q < c0; q += 4) sum += chunk_counts[q * 64 + l];
+    part[w][l] = sum;
+    int counter = 0;   // lane e: next free position of expert e
+    for (int q = c0; q < c && q < nchunks; ++q) counter += chunk_counts[q * 64 + l];
+    sync();
+    const int incl = wave_incl_scan(cnt);
+    counter += incl - cnt + part[0][l] + part[1][l] + part[2][l] + part[3][l];
+    if (c == 0) {
+        if (l < E) offsets[l] = incl - cnt;
+        if (l == E - 1) offsets[E] = incl;
+        if (rows)
+            for (int i = l; i < pad; i += 64) rows[M + i] = 0;
     }
-}
-
-// pass 3: stable positions
-__global__ __launch_bounds__(64) void sort_scatter_kernel(const int32_t* idx, const int32_t* chunk_base, int32_t* sorted_src,
-                                                          int32_t* inv, int M) {
-    const int l = threadIdx.x, c = blockIdx.x;
-    int counter = chunk_base[c * 64 + l];  // lane e: next free position of expert e
-    const int begin = c * SORT_CHUNK, end = min(M, begin + SORT_CHUNK);
     const unsigned long long below = (1ull << l) - 1ull;
-    for (int i0 = begin; i0 < end; i0 += 64) {
-        const int i = i0 + l;
-        const bool valid = i < end;
-        const int e = valid ? idx[i] : 0;
+#pragma unroll
+    for (int j = 0; j < SORT_PER; ++j) {
+        const int i = c * SORT_CHUNK + 64 * j + l;
+        const bool valid = i < M;
         unsigned long long bal[6];
 #pragma unroll
-        for (int b = 0; b < 6; ++b) bal[b] = ballot((e >> b) & 1);
-        const unsigned long long vm = ballot(valid);
-        const unsigned long long same = match_mask(e, bal, vm);
-        const int base = shfl(counter, e & 63);
+        for (int b = 0; b < 6; ++b) bal[b] = ballot((v[j] >> b) & 1);
+        const unsigned long long vm = ballot(valid), same = match_mask(v[j], bal, vm);
+        const int base = shfl(counter, v[j] & 63);
         if (valid) {
             const int pos = base + __builtin_popcountll(same & below);
             sorted_src[pos] = i;
             inv[i] = pos;
+            if (rows) rows[pos] = i / k;
         }
         counter += __builtin_popcountll(match_mask(l, bal, vm));
     }
 }
 
 // Up to SORT_SMALL entries: the three passes as one launch of one workgroup, its 16 waves on sixteen ranges of the entries (a chunk of 2048 entries per wave and
-// launch took 9 + 4 + 9 us for the 1680 entries of 280 tokens; 5 us here).  counts NULL: taken from the entries; rows: the token of every place.
+// launch took 9 + 4 + 9 us for the 1680 entries of 280 tokens; 5 us here).  counts NULL: taken from the entries; rows: the token of every place, and ``pad`` zeros behind them.
 constexpr int SORT_SMALL = 8192;
 __global__ __launch_bounds__(1024) void sort_small_kernel(const int32_t* idx, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv,
-                                                          int32_t* rows, int E, int M, int k) {
+                                                          int32_t* rows, int E, int M, int k, int pad) {
     ARIA_SMEM_STATIC int base[16][64];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, per = ((M + 1023) / 1024) * 64, begin = w * per, end = min(M, begin + per);
+    for (int i = threadIdx.x; i < pad; i += 1024) rows[M + i] = 0;
     int cnt = 0;
     for (int i0 = begin; i0 < end; i0 += 64) {
         const bool valid = i0 + l < end;
@@ -747,7 +754,7 @@ ARIA_HIDDEN int aria_route_and_sort(const bf16_t* logits, bf16_t* scores, int32_
                                     int T, int E, int k, void* stream) {
     if (E > 64 || k > 8 || k > E || T * k > SORT_SMALL) return ARIA_ERR_UNSUPPORTED;
     ARIA_LAUNCH((route_kernel<false>), dim3(std::min(grid_for_waves(T), 512)), dim3(256), 0, stream, (const void*)logits, (void*)scores, idx, counts, T, E, k);
-    ARIA_LAUNCH(sort_small_kernel, dim3(1), dim3(1024), 0, stream, (const int32_t*)idx, (const int32_t*)nullptr, offsets, src, inv, rows, E, T * k, k);
+    ARIA_LAUNCH(sort_small_kernel, dim3(1), dim3(1024), 0, stream, (const int32_t*)idx, (const int32_t*)nullptr, offsets, src, inv, rows, E, T * k, k, 0);
     return aria_check_launch();
 }
 
@@ -795,29 +802,26 @@ int aria_moe_router_fused(const void* x, const void* w, void* logits, void* scor
 
 int aria_moe_sort(const int32_t* indices, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv,
                   int32_t* workspace, int64_t T, int64_t E, int64_t k, void* stream) {
-    if (!indices || !counts || !offsets || !sorted_src || !inv || !workspace || T < 0 || E <= 0 || k <= 0) return ARIA_ERR_INVALID;
-    if (E > SORT_WIDE_E) return ARIA_ERR_UNSUPPORTED;
+    return aria_moe_sort_rows(indices, counts, offsets, sorted_src, inv, nullptr, 0, workspace, T, E, k, stream);
+}
+
+int aria_moe_sort_rows(const int32_t* indices, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv, int32_t* rows, int64_t pad,
+                       int32_t* workspace, int64_t T, int64_t E, int64_t k, void* stream) {
+    if (!indices || !counts || !offsets || !sorted_src || !inv || !workspace || T < 0 || E <= 0 || k <= 0 || pad < 0 || (pad && !rows)) return ARIA_ERR_INVALID;
+    if (E > SORT_WIDE_E || (rows && E > 64)) return ARIA_ERR_UNSUPPORTED;
     const int M = int(T * k);
     if (E > 64) {
         ARIA_LAUNCH(sort_wide_kernel, dim3(1), dim3(SORT_WIDE_E), 0, stream, indices, counts, offsets, sorted_src, inv, int(E), M);
         return aria_check_launch();
     }
     if (M <= SORT_SMALL) {
-        ARIA_LAUNCH(sort_small_kernel, dim3(1), dim3(1024), 0, stream, indices, counts, offsets, sorted_src, inv, (int32_t*)nullptr, int(E), M, int(k));
+        ARIA_LAUNCH(sort_small_kernel, dim3(1), dim3(1024), 0, stream, indices, counts, offsets, sorted_src, inv, rows, int(E), M, int(k), int(pad));
         return aria_check_launch();
     }
     const int nchunks = (M + SORT_CHUNK - 1) / SORT_CHUNK;
-    int32_t* chunk_counts = workspace;
-    int32_t* chunk_base = workspace + (size_t)nchunks * 64;
-    if (nchunks > 0) {
-        ARIA_LAUNCH(sort_count_kernel, dim3(nchunks), dim3(64), 0, stream, indices, chunk_counts, M);
-    }
-    ARIA_LAUNCH(sort_scan_kernel, dim3(1), dim3(64), 0, stream, counts, (const int32_t*)chunk_counts, chunk_base, offsets, int(E),
-                nchunks);
-    if (nchunks > 0) {
-        ARIA_LAUNCH(sort_scatter_kernel, dim3(nchunks), dim3(64), 0, stream, indices, (const int32_t*)chunk_base, sorted_src,
-                    inv, M);
-    }
+    ARIA_LAUNCH(sort_count_kernel, dim3((nchunks + 3) / 4), dim3(256), 0, stream, indices, workspace, M, nchunks);
+    ARIA_LAUNCH(sort_scatter_kernel, dim3((nchunks + 3) / 4), dim3(256), 0, stream, indices, counts, (const int32_t*)workspace, offsets, sorted_src, inv, rows, int(E),
+                M, int(k), nchunks, int(pad));
     return aria_check_launch();
 }
 

@@ -106,7 +106,7 @@ def moe_fwd(x, router_w, fc1, fc2, gate_w, up_w, down_w, cfg: MoEConfig, save=Tr
     else:
         logits = ops.gemm(x, router_w)                               # TopKRouter.gating  moe_lm.py:190-201
         scores, idx, counts = ops.moe_route(logits, k)               # routing :261-269 (device-side histogram)
-    offsets, sorted_src, inv = ops.moe_sort(idx, counts)             # token_permutation :326-334 (stable)
+    offsets, sorted_src, inv, token_rows = ops.moe_sort_rows(idx, counts)   # token_permutation :326-334 (stable)
     fused = ops.glu_fusable(fc1.shape[1], fc1.shape[2])
     rows = None
     if fused and ops.gather_fusable(fc1.shape[1]) and ((lean or not save) or ops.wgrad_gather_fusable(fc1.shape[1])):
@@ -114,7 +114,7 @@ def moe_fwd(x, router_w, fc1, fc2, gate_w, up_w, down_w, cfg: MoEConfig, save=Tr
         # checkpointed step, and (r05) the plain training step too: fc1's weight gradient reaches the token rows through the same index
         # (ops.grouped_gemm_wgrad_gather), so nothing in the backward wants `perm` as a tensor
         perm = None
-        rows = ops.permuted_token_rows(sorted_src, k)
+        rows = token_rows
         h1, act = ops.grouped_gemm_swiglu_gather(x, rows, fc1, offsets, want_h=bool(save) and not lean)
     else:
         perm = ops.moe_permute(x, sorted_src, k)

@@ -217,18 +217,18 @@ class MOEFeedForward(nn.Module):
         if not few and ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
             logits, scores, idx, counts = ops.moe_router_fused(x2d, self.gate.weight, k)
         else:
-            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 45 us for 280 tokens, 22 in two launches)
+            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 20 us at any such count, 22 in two launches for 280 tokens, less for fewer)
             scores, idx, counts = ops.moe_route(logits, k)             # topk + softmax (model.py:359-363)
-        offsets, sorted_src, inv = ops.moe_sort(idx, counts)           # token_permutation (:243-254)
+        offsets, sorted_src, inv, rows = ops.moe_sort_rows(idx, counts)   # token_permutation (:243-254)
         cf = self.cond_ffn
         E, I, D = cf.w1.shape
         contiguous = all(w.is_contiguous() for w in (cf.w1, cf.w2, cf.w3))
         if contiguous and ops.rows_experts_take(sorted_src.numel(), E, D, I):
-            act = ops.rows_experts(x2d, cf.w1, offsets, ops.permuted_token_rows(sorted_src, k), cf.w3)
+            act = ops.rows_experts(x2d, cf.w1, offsets, rows, cf.w3)
         elif _glu_pair_ready(cf.w1, cf.w3) and ops.gather_fusable(x2d.shape[1]):
             # K2 + K3: the dispatcher's row gather (model.py:243-254) in the A loader of the fused w1 / w3 / SwiGLU launch -- no permuted copy
             # of the tokens ([6T, D]: 1.6 GB written and read per layer of a 53 K-token prefill), no h1 / h3 round trip
-            act = ops.grouped_gemm_swiglu_split_gather(x2d, ops.permuted_token_rows(sorted_src, k), cf.w1, cf.w3, offsets)[1]
+            act = ops.grouped_gemm_swiglu_split_gather(x2d, rows, cf.w1, cf.w3, offsets)[1]
         elif _glu_pair_ready(cf.w1, cf.w3):   # w1 / w3 GEMMs + SwiGLU in ONE launch (no h1 / h3 round trip: 2 x [6T, I] written and read)
             act = ops.grouped_gemm_swiglu_split(ops.moe_permute(x2d, sorted_src, k), cf.w1, cf.w3, offsets)[1]
         else:

@@ -71,6 +71,7 @@ SIGNATURES = {
     "aria_grouped_gemm_swiglu_lora_bf16": [P, P, P, P, P, I64, I64, I64, I64, I64, I64, I64, I64, I64, P, P, I64, I64, I64, I64, P],
     "aria_dropout_fwd_bf16": [P, P, P, I64, F32, ctypes.c_uint64, P],
     "aria_dropout_bwd_bf16": [P, P, P, I64, F32, I32, P],
+    "aria_lora_scale_bf16": [P, P, I64, I64, I64, F32, P],
     "aria_lora_down_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_up_bf16": [P, P, I32, P, P, P, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_wgrad_bf16": [P, P, P, I32, I64, I64, I64, I64, I64, P, I64, P],
@@ -86,6 +87,7 @@ SIGNATURES = {
     "aria_moe_route": [P, I32, P, P, P, I64, I64, I64, P],
     "aria_moe_router_fused": [P, P, P, P, P, P, I64, I64, I64, I64, I64, P],
     "aria_moe_sort": [P, P, P, P, P, P, I64, I64, I64, P],
+    "aria_moe_sort_rows": [P, P, P, P, P, P, I64, P, I64, I64, I64, P],
     "aria_moe_permute": [P, P, P, I64, I64, I64, I64, P],
     "aria_moe_unpermute": [P, P, P, P, P, I64, I64, I64, P],
     "aria_moe_unpermute_res": [P, P, P, P, P, P, I64, I64, I64, P],

@@ -7,13 +7,15 @@ nn.Linear targets -- the same line):
     result = base(x) + lora_B(lora_A(dropout(x))) * scaling              base weights frozen, A / B trainable
 
 What runs here, per module:
-  * ``u = scaling * lora_A(dropout(x))`` -- a thin product (``ops.lora_down``, ranks 8 and 16; a general product and a scaling else) on the dropped
-    input (``ops.dropout``: one pass, one mask byte per 8 elements kept for the backward);
+  * ``u = scaling * lora_A(dropout(x))`` -- a skinny GEMM (N = r) on the dropped input (``ops.dropout``: one pass, one mask byte per 8
+    elements kept for the backward), scaled into its columns.  The forward keeps the general product's sum order although ``ops.lora_down``, the
+    backward's kernel, is three times as fast: with dropout another rounding of u turns near ties of the next layer's router, and a turned tie
+    moves every later expert row under another mask;
   * the base launch with the adapter's second projection as a K-EXTENSION (``ops.*_lora``: one extra K-tile fed from u and lora_B): no
     output-sized ``base + delta`` pass, and the fused epilogues keep working -- fc1 + SwiGLU, gate|up + SwiGLU, the q|k|v and gate|up wide
     launches (their adapters enter side by side with a block-diagonal B);
   * backward: the base input gradients exactly as the un-adapted layer computes them (weight gradients of the frozen base are skipped);
-    per adapter d_u = scaling * dy lora_B^T (thin), d lora_B = u^T dy, d lora_A = dropout(x)^T d_u (``ops.lora_wgrad``), and the adapter's input
+    per adapter d_u = scaling * dy lora_B^T (thin: ``ops.lora_down``, ranks 8 and 16), d lora_B = u^T dy, d lora_A = dropout(x)^T d_u (``ops.lora_wgrad``), and the adapter's input
     gradient ``mask * (d_u lora_A) / (1 - p)`` added into dx in one pass (``ops.lora_up_``; other ranks: a product, then ``ops.dropout_bwd_``).
 Everything else of the layer (RMSNorm with the residual folded in, RoPE, flash attention, router, dispatch, un-permute + shared add) is the
 un-adapted layer's code path (aria_amd.functional).  The module-by-module form (aria_amd.lora.GroupedGemmLoraLayer / LinearLoraLayer called
@@ -43,8 +45,12 @@ class LoraSite:
     p: float = 0.0
 
 
-def _scaled(u: torch.Tensor, s: float) -> torch.Tensor:
-    return u if s == 1.0 else (u.float() * s).to(bf16)   # (u is [rows, r]: a few hundred KB)
+def _scaled(u: torch.Tensor, s: float, out=None) -> torch.Tensor:
+    """bf16(u * s) (u is [rows, r]: a few hundred KB), where ``out`` is given into those columns"""
+    if u.shape[1] % 8 == 0 and (out is None or (out.storage_offset() % 8 == 0 and out.stride(0) % 8 == 0)):
+        return u if s == 1.0 and out is None else ops.lora_scale(u, s, out)
+    u = u if s == 1.0 else (u.float() * s).to(bf16)
+    return u if out is None else out.copy_(u)
 
 
 def _factor(w: torch.Tensor) -> torch.Tensor:
@@ -87,10 +93,7 @@ def dense_lora_fwd(x: torch.Tensor, w: torch.Tensor, sites: List[Optional[LoraSi
     for j, s in live:
         r = s.a.shape[0]
         d = _Drop(x, s.p, training, _seed(seeds))
-        if ops.lora_thin(r, x.shape[1]):
-            ops.lora_down(d.xd, _factor(s.a), s.scaling, w_oc=False, out=U[:, c0:c0 + r])
-        else:
-            U[:, c0:c0 + r] = _scaled(ops.gemm(d.xd, s.a), s.scaling)
+        _scaled(ops.gemm(d.xd, s.a), s.scaling, out=U[:, c0:c0 + r])
         Bx[starts[j]:starts[j] + rows[j], c0:c0 + r] = s.b
         drops.append(d)
         c0 += r
@@ -134,10 +137,7 @@ def grouped_lora_fwd(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, si
         out = ops.grouped_gemm_swiglu(x, w, offsets, want_h=want_h) if glu else ops.grouped_gemm(x, w, offsets)
         return out, None
     d = _Drop(x, site.p, training, _seed(seeds))
-    if ops.lora_thin(site.a.shape[2], x.shape[1]):
-        U = ops.lora_down(d.xd, _factor(site.a), site.scaling, w_oc=True, offsets=offsets)           # [M, r]
-    else:
-        U = _scaled(ops.grouped_gemm(d.xd, site.a, offsets), site.scaling)
+    U = _scaled(ops.grouped_gemm(d.xd, site.a, offsets), site.scaling)                      # [M, r]
     out = ops.grouped_gemm_swiglu_lora(x, w, offsets, U, site.b, want_h=want_h) if glu else ops.grouped_gemm_lora(x, w, offsets, U, site.b)
     return out, dict(site=site, drop=d, U=U)
 

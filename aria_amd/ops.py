@@ -280,6 +280,17 @@ def lora_thin(r: int, K: int) -> bool:
     return r in (8, 16) and K % 64 == 0 and r * (K + 32) <= 57344
 
 
+def lora_scale(u: torch.Tensor, scale: float, out=None) -> torch.Tensor:
+    """bf16(u * scale): u [M, r] contiguous, r % 8 == 0; out: [M, r], strided rows."""
+    _chk(u, name="u")
+    M, r = u.shape
+    out = torch.empty_like(u) if out is None else out
+    if not u.is_contiguous() or out.shape != u.shape:
+        raise ValueError("lora_scale: contiguous u, out of its shape")
+    hip.get_lib().call("aria_lora_scale_bf16", _p(u), _p(out), M, r, _rowmajor_2d(out, "out"), float(scale), _stream(u))
+    return out
+
+
 def lora_down(x: torch.Tensor, w: torch.Tensor, scale: float, w_oc: bool, offsets=None, out=None) -> torch.Tensor:
     """bf16(scale * x w^T): x [M, K] (unit-stride rows), w [r, K], or [K, r] with ``w_oc``; with ``offsets`` a leading expert dimension.  out: [M, r], strided rows."""
     _chk(x, name="x"), _chk(w, name="w")
@@ -739,6 +750,16 @@ def moe_router_fused(x: torch.Tensor, w: torch.Tensor, k: int):
 
 def moe_sort(indices: torch.Tensor, counts: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """-> offsets int32 [E+1], sorted_src int32 [T*k] (== reference sorted_indices), inv int32 [T*k]."""
+    return _sort(indices, counts, 0)[:3]
+
+
+def moe_sort_rows(indices: torch.Tensor, counts: torch.Tensor, pad: int = 64):
+    """moe_sort and ``permuted_token_rows`` of its order, in the same launches: -> offsets, sorted_src, inv, rows."""
+    out = _sort(indices, counts, pad)
+    return out if out[3] is not None else out[:3] + (permuted_token_rows(out[1], indices.shape[1], pad),)
+
+
+def _sort(indices: torch.Tensor, counts: torch.Tensor, pad: int):
     _chk(indices, torch.int32, "indices"), _chk(counts, torch.int32, "counts")
     T, k = indices.shape
     E = counts.shape[0]
@@ -747,11 +768,12 @@ def moe_sort(indices: torch.Tensor, counts: torch.Tensor) -> Tuple[torch.Tensor,
     offsets = torch.empty((E + 1,), dtype=torch.int32, device=dev)
     sorted_src = torch.empty((M,), dtype=torch.int32, device=dev)
     inv = torch.empty((M,), dtype=torch.int32, device=dev)
+    rows = torch.empty((M + pad,), dtype=torch.int32, device=dev) if pad and E <= 64 else None
     nchunks = (M + 2047) // 2048
     ws = torch.empty((max(1, nchunks) * 128 + 64,), dtype=torch.int32, device=dev)
-    hip.get_lib().call("aria_moe_sort", _p(indices), _p(counts), _p(offsets), _p(sorted_src), _p(inv), _p(ws), T, E, k,
-                       _stream(indices))
-    return offsets, sorted_src, inv
+    hip.get_lib().call("aria_moe_sort_rows", _p(indices), _p(counts), _p(offsets), _p(sorted_src), _p(inv), _p(rows) if rows is not None else None,
+                       pad if rows is not None else 0, _p(ws), T, E, k, _stream(indices))
+    return offsets, sorted_src, inv, rows[:M] if rows is not None else None
 
 
 def moe_permute(x: torch.Tensor, sorted_src: torch.Tensor, k: int) -> torch.Tensor:

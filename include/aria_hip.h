@@ -143,9 +143,11 @@ int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t 
 
 /* The thin products of an adapter of rank r = 8 or 16 (else ARIA_ERR_UNSUPPORTED).  offsets: null, or the experts' row offsets [E + 1] -- the factor is then one per
  * expert, r K elements apart.
+ * _scale: OUT [M, r] (row stride ldo, a multiple of 8) = bf16(scale * U), any r % 8 == 0.
  * _down: U [M, r] (row stride ldu) = bf16(scale * X W^T), W [r, K] or with w_oc [K, r]; K % 64 == 0, r (K + 32) <= 57344.
  * _up:   DX [M, K] += keep ? scale * (DU A) : 0, A [r, K] with a_oc, else [K, r]; mask as aria_dropout_fwd_bf16 writes it (null: everything is kept), K % 8 == 0.
  * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 64 rows begun. */
+int aria_lora_scale_bf16(const void* U, void* OUT, int64_t M, int64_t r, int64_t ldo, float scale, void* stream);
 int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
                         float scale, void* stream);
 int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,
@@ -244,6 +246,9 @@ int aria_moe_route(const void* logits, int logits_f32, void* scores, int32_t* in
  * with nchunks = ceil(T*k / 2048). */
 int aria_moe_sort(const int32_t* indices, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv,
                   int32_t* workspace, int64_t T, int64_t E, int64_t k, void* stream);
+/* aria_moe_sort, and the token of every sorted place: rows[p] = sorted_src[p] / k, with ``pad`` zeros behind them (E <= 64). */
+int aria_moe_sort_rows(const int32_t* indices, const int32_t* counts, int32_t* offsets, int32_t* sorted_src, int32_t* inv, int32_t* rows, int64_t pad,
+                       int32_t* workspace, int64_t T, int64_t E, int64_t k, void* stream);
 
 /* permuted[p, :] = x[sorted_src[p] / k, :]   (index_select, moe_lm.py:330). D % 8 == 0. */
 int aria_moe_permute(const void* x, const int32_t* sorted_src, void* permuted, int64_t M, int64_t D, int64_t k,

@@ -1128,6 +1128,27 @@ def case_router_fused(dev, T, D, E, k):
     assert int(counts.sum()) == T * k
 
 
+def case_sort_rows(dev, T, k, E):
+    """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
+    from aria_amd import ops
+
+    g = torch.Generator().manual_seed(T + E)
+    idx = torch.randint(0, E, (T, k), generator=g).to(torch.int32)
+    if T > 100:
+        idx[50:] = torch.where(idx[50:] == 1, 0, idx[50:])   # (an expert nearly without entries)
+    counts = torch.bincount(idx.flatten().long(), minlength=E).to(torch.int32)
+    off, src, inv, rows = ops.moe_sort_rows(idx.to(dev), counts.to(dev))
+    want = torch.argsort(idx.flatten().long(), stable=True)
+    assert torch.equal(src.cpu().long(), want) and torch.equal(inv.cpu().long(), torch.argsort(want))
+    assert torch.equal(off.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), counts.long().cumsum(0)]))
+    assert torch.equal(rows.cpu().long(), want // k)
+    behind = torch.as_strided(rows, (64,), (1,), rows.storage_offset() + rows.numel())   # the weight gradient's loader reads these
+    assert not bool(behind.any())
+
+
+SORT_ROWS = [(5, 2, 16), (1365, 6, 64), (1366, 6, 64), (2049, 4, 32), (4097, 3, 33), (9001, 1, 1), (2100, 4, 100)]
+
+
 def case_lora_thin(dev, T, K, N, r, counts=None, p=0.0):
     """The thin products of an adapter (down, up through the dropout mask, weight gradient) against 64-bit ones of the same bf16 operands: every result is a 32-bit
     sum rounded once to bf16 -- half a unit of the last place (2^-9 of the result) and the sum's own error (a few 2^-24 of the sum of magnitudes)."""
@@ -1155,6 +1176,8 @@ def case_lora_thin(dev, T, K, N, r, counts=None, p=0.0):
     ops.lora_down(x, wa, 1.7, w_oc=counts is not None, offsets=of, out=U[:, r:])
     near(U[:, r:], 1.7 * by_expert(x, a.transpose(1, 2)), 1.7 * by_expert(x.abs(), a.abs().transpose(1, 2)))
     assert not bool(U[:, :r].any())
+    scaled = ops.lora_scale(U[:, r:].contiguous(), 1.3, out=torch.zeros((T, 3 * r), dtype=bf16, device=dev)[:, r:2 * r])
+    assert torch.equal(scaled, (U[:, r:].float() * 1.3).to(bf16))
     du = ops.lora_down(dy, wb, 0.6, w_oc=counts is None, offsets=of)
     near(du, 0.6 * by_expert(dy, b), 0.6 * by_expert(dy.abs(), b.abs()))
     mask = ops.dropout(x, p, 77)[1] if p else None

@@ -247,6 +247,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(force_gemm_v3, B, S, D, hd, K):
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K)
 
 
+@pytest.mark.parametrize("T,k,E", C.SORT_ROWS)
+def test_sort_with_token_rows(T, k, E):
+    C.case_sort_rows(DEV, T, k, E)
+
+
 @pytest.mark.parametrize("T,K,N,r,counts,p", C.LORA_THIN)
 def test_lora_thin_products(T, K, N, r, counts, p):
     C.case_lora_thin(DEV, T, K, N, r, counts, p)

@@ -241,6 +241,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(B, S, D, hd, K):   # q | k | v proje
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K) == (D >= 2560)
 
 
+@pytest.mark.parametrize("T,k,E", C.SORT_ROWS + [(16384, 6, 64), (53001, 6, 64)])
+def test_sort_with_token_rows(T, k, E):
+    C.case_sort_rows(DEV, T, k, E)
+
+
 @pytest.mark.parametrize("T,K,N,r,counts,p", C.LORA_THIN + [(4096, 2560, 3328, 8, None, 0.05), (1000, 3328, 2560, 16, None, 0.0), (0, 2560, 1664, 8, [300, 0, 1500, 70], 0.05)])
 def test_lora_thin_products(T, K, N, r, counts, p):
     C.case_lora_thin(DEV, T, K, N, r, counts, p)
