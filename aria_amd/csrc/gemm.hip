@@ -404,9 +404,9 @@ int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, i
                               workspace_bytes, stream);
 }
 
-int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
+static int dense_product(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                        int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
-                       int64_t workspace_bytes, void* stream) {
+                       int64_t workspace_bytes, void* stream, bool four_waves) {
     if (act != ARIA_ACT_NONE && act != ARIA_ACT_GELU_TANH && act != ARIA_ACT_RELU2) return ARIA_ERR_UNSUPPORTED;
     if (act == ARIA_ACT_RELU2 && (a_oc || b_oc)) return ARIA_ERR_UNSUPPORTED;   // (built for the forward form only)
     if (!A || !B || !C || M < 0 || N < 0 || K < 0) return ARIA_ERR_INVALID;
@@ -442,14 +442,26 @@ int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, 
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
     const bool strides = 2 * lda < (1ll << 24) && 2 * ldb < (1ll << 24);
-    if ((!a_oc || b_oc) && strides && fits_dma(K, bytesA, bytesB, M, N)) {
+    if (four_waves && (!a_oc || b_oc) && strides && fits_dma(K, bytesA, bytesB, M, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0);
         if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
     }
     if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
-        return g_last_variant = 3, launch_large(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
+        return g_last_variant = 3, four_waves ? launch_large(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes)
+                                              : aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
+}
+
+int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
+                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
+    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, act, workspace, workspace_bytes, stream, true);
+}
+
+int aria_gemm_keep_sums_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc, int b_oc, int64_t lda, int64_t ldb,
+                             int64_t ldc, int c_f32, int accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
+    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, ARIA_ACT_NONE, workspace, workspace_bytes, stream, false);
 }
 
 int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total,

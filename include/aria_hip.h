@@ -67,6 +67,11 @@ int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, i
 int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                        int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
                        int64_t workspace_bytes, void* stream);
+/* aria_gemm_bf16_ws without the four-wave tiles: an output of one round then has the partial sums of the 256 x 256 tiles' split, not of theirs.  For the base product
+ * under an adapter that no fused launch takes: its rounding decides near ties of the next layer's router, and with dropout a turned tie moves every later expert row
+ * under another mask. */
+int aria_gemm_keep_sums_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc, int b_oc, int64_t lda, int64_t ldb,
+                             int64_t ldc, int c_f32, int accumulate, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* experts_gemm(input, weight, tokens_per_expert)  -- seam B1, aria/model/moe_lm.py:431-443 (grouped_gemm.ops.gmm
  * or sequential_gemm :398-428), called from GroupedGEMM.forward :467-484.

@@ -1128,6 +1128,16 @@ def case_router_fused(dev, T, D, E, k):
     assert int(counts.sum()) == T * k
 
 
+def case_gemm_keep_sums(dev, M, N, K):
+    """The base product under an adapter (no four-wave tiles) against the product in 64 bits: a 32-bit sum rounded once."""
+    from aria_amd import ops
+
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.1)
+    got = ops.gemm(x.to(dev), w.to(dev), keep_sums=True).double().cpu()
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
+
+
 def case_sort_rows(dev, T, k, E):
     """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
     from aria_amd import ops

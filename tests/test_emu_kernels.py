@@ -247,6 +247,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(force_gemm_v3, B, S, D, hd, K):
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (300, 264, 512)])
+def test_gemm_keep_sums(M, N, K):
+    C.case_gemm_keep_sums(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("T,k,E", C.SORT_ROWS)
 def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)

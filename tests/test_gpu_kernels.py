@@ -241,6 +241,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(B, S, D, hd, K):   # q | k | v proje
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K) == (D >= 2560)
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (3000, 2560, 3328)])
+def test_gemm_keep_sums(M, N, K):
+    C.case_gemm_keep_sums(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("T,k,E", C.SORT_ROWS + [(16384, 6, 64), (53001, 6, 64)])
 def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
