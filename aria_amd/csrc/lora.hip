@@ -5,7 +5,7 @@
 //   up:     dx += keep ? (d_u A) / (1 - p) : 0     the adapter's input gradient through its dropout mask, added where the base's gradient lies
 //   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
 // All three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
-// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9 (the scaling alone 16 with its copy, here SC_US); up as a product and a masked add 22, here 10; wgrad as
+// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9 (the scaling alone 16 with its copy, here 3.5); up as a product and a masked add 22, here 10; wgrad as
 // a split product and its sum 24, here 11 (64 rows a block: 12.5 us on cold rows, with 128 and four loads in flight a wave 15.5).  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
 // 21 and 43); an adapted training step of 4 x 1024 tokens 11 470 / 9 780.
 #include "aria_device.h"
@@ -18,7 +18,7 @@ using namespace ad;
 
 constexpr int ROWS = 32;                // rows of a block
 constexpr int PAD = 32;                 // a row of the staged factor ends 64 bytes further: rows start on different banks
-constexpr int64_t LDS_MAX = 112 << 10;  // the staged factor: rank 16 up to 3552 columns
+constexpr int64_t LDS_MAX = 112 << 10;  // the staged factor: rank 16 up to 3552 columns, 32 columns of 1728
 
 // The rows of a block: block bid's tile of 32, or with offsets the bid-th of the tiles of 32 rows that start anew at every expert (collective; false: none left).
 __device__ __forceinline__ bool rows_of(const int32_t* offsets, int E, int M, int bid, int& e, int& m0, int& m1) {
@@ -53,11 +53,17 @@ __global__ __launch_bounds__(256) void lora_scale_kernel(const bf16_t* u, bf16_t
     st16(out + i / pieces * ldo + 8 * (i % pieces), o);
 }
 
+__device__ __forceinline__ void put(bf16_t* p, float v) { *p = f2bf(v); }
+__device__ __forceinline__ void put(float* p, float v) { *p = v; }
+
 // u[m][n] = scale * sum_k X[m][k] W[n][k], n < r.  W: [r][K], or with w_oc [K][r]; per expert where there are offsets.
 // The factor is staged once a block, k-contiguous whichever way it lies; the eight waves take every eighth 64 columns of the reduction, four such steps of 32 rows
 // in flight each, straight from global memory (16-row fragments of v_mfma_f32_16x16x32_bf16 read 64 bytes of a row, its neighbour the other half of the line).
 // Splitting the reduction over the waves is what puts 4096 rows on 128 CUs with all of a block's bytes in flight at once.
-__global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const bf16_t* W, bf16_t* U, const int32_t* offsets, int E, int M, int K, int r, int w_oc,
+// NG: groups of 16 columns.  Also the router's product of a mixture with up to 32 experts, in 32 bits (T = float): 5580 rows of 1536 on 32 columns as one 128 x 128 tile
+// of the general kernel per 128 rows 32 us, here 12.
+template <int NG, class T>
+__global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const bf16_t* W, T* U, const int32_t* offsets, int E, int M, int K, int r, int w_oc,
                                                         long long ldx, long long ldu, float scale) {
     ARIA_DYN_SMEM(lds);
     bf16_t* wt = reinterpret_cast<bf16_t*>(lds);
@@ -94,33 +100,43 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
         }
     }
     sync();
-    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    const bf16_t* wr = wt + (lr & (r - 1)) * pitch + 8 * kg;   // (rank 8: columns 8 .. 15 repeat the first, never stored)
+    f32x4 acc[2][NG];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) acc[h][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16_t* wr[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) wr[g] = wt + min(16 * g + lr, r - 1) * pitch + 8 * kg;   // (past the last column: the last one again, never stored)
     for (int c0 = w; c0 < nch; c0 += 32) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             if (c0 + 8 * i < nch)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const s16x8 b = *reinterpret_cast<const s16x8*>(wr + (c0 + 8 * i) * 64 + 32 * s);
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) acc[h] = mfma16(x[i][h][s], b, acc[h]);
-                }
+                    for (int g = 0; g < NG; ++g) {
+                        const s16x8 b = *reinterpret_cast<const s16x8*>(wr[g] + (c0 + 8 * i) * 64 + 32 * s);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) acc[h][g] = mfma16(x[i][h][s], b, acc[h][g]);
+                    }
         if (c0 + 32 < nch) load(c0 + 32);
     }
     sync();
-    float* red = reinterpret_cast<float*>(lds);   // [wave][row][16]
+    float* red = reinterpret_cast<float*>(lds);   // [wave][row][16 NG]
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) red[(w * ROWS + 16 * h + 4 * kg + i) * 16 + lr] = acc[h][i];
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) red[(w * ROWS + 16 * h + 4 * kg + i) * 16 * NG + 16 * g + lr] = acc[h][g][i];
     sync();
     for (int i = threadIdx.x; i < ROWS * r; i += 512) {
         const int row = i / r, n = i % r;
         float s = 0.f;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) s += red[(q * ROWS + row) * 16 + n];
-        if (m0 + row < m1) U[(long long)(m0 + row) * ldu + n] = f2bf(scale * s);
+        for (int q = 0; q < 8; ++q) s += red[(q * ROWS + row) * 16 * NG + n];
+        if (m0 + row < m1) put(U + (long long)(m0 + row) * ldu + n, scale * s);
     }
 }
 
@@ -279,8 +295,26 @@ int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const i
     if (!thin(r) || (K & 63) || lds > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
     if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
     if (M == 0) return ARIA_OK;
-    ARIA_LAUNCH(lora_down_kernel, dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
+    ARIA_LAUNCH((lora_down_kernel<1, bf16_t>), dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
                 static_cast<bf16_t*>(U), offsets, int(E), int(M), int(K), int(r), w_oc, (long long)ldx, (long long)ldu, scale);
+    return aria_check_launch();
+}
+
+int aria_thin_product_f32(const void* X, const void* W, float* C, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldc, void* stream) {
+    if (!X || !W || !C || M < 0 || N <= 0 || K <= 0) return ARIA_ERR_INVALID;
+    const int64_t lds = std::max<int64_t>(N * (K + PAD) * 2, 8 * ROWS * 32 * 4);
+    if (N > 32 || (N & 7) || (K & 63) || lds > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
+    if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
+    if (M == 0) return ARIA_OK;
+    const dim3 grid(row_tiles(M, nullptr, 1)), block(512);
+#define THIN(NG)                                                                                                                                                     \
+    ARIA_LAUNCH((lora_down_kernel<NG, float>), grid, block, unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W), C, (const int32_t*)nullptr, \
+                1, int(M), int(K), int(N), 0, (long long)ldx, (long long)ldc, 1.f)
+    if (N <= 16)
+        THIN(1);
+    else
+        THIN(2);
+#undef THIN
     return aria_check_launch();
 }
 

@@ -220,7 +220,7 @@ __device__ __forceinline__ unsigned long long match_mask(int key, const unsigned
 
 // More than SORT_SMALL entries: two launches, a wave per 1024 entries in both, all of a wave's entries loaded at once.  What bounds them is latency: a count
 // per chunk, then every block adds the chunks in front of its own (coalesced 256-byte rows, four waves) instead of a launch in between.  22 000 entries on 32 experts:
-// a wave's 2048 entries one load after the other, and the sums as a third launch 29 us, with the token rows as two more 40; now SORT_US.
+// a wave's 2048 entries one load after the other, and the sums as a third launch 29 us, with the token rows as two more 40; now SO12.
 constexpr int SORT_CHUNK = 1024, SORT_PER = SORT_CHUNK / 64;
 
 // pass 1: per-chunk histogram (lane e = expert e)

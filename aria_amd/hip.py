@@ -72,6 +72,7 @@ SIGNATURES = {
     "aria_grouped_gemm_swiglu_lora_bf16": [P, P, P, P, P, I64, I64, I64, I64, I64, I64, I64, I64, I64, P, P, I64, I64, I64, I64, P],
     "aria_dropout_fwd_bf16": [P, P, P, I64, F32, ctypes.c_uint64, P],
     "aria_dropout_bwd_bf16": [P, P, P, I64, F32, I32, P],
+    "aria_thin_product_f32": [P, P, P, I64, I64, I64, I64, I64, P],
     "aria_lora_scale_bf16": [P, P, I64, I64, I64, F32, P],
     "aria_lora_down_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_up_bf16": [P, P, I32, P, P, P, I64, I64, I64, I64, I64, F32, P],

@@ -1177,12 +1177,25 @@ def _f32(t: torch.Tensor) -> int:
     return int(t.dtype == torch.float32)
 
 
+def thin_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """A router's product, whose 8 .. 32 columns fill a quarter of a tile at most: the thin kernel, factor staged on chip (5580 rows of 1536 on 32 columns as 128 x 128
+    tiles 32 us, there 12).  Results of 16 bits stay with the tiles: the fused router's are theirs, bit for bit."""
+    N, K = w.shape
+    return (N in (8, 16, 24, 32) and K % 64 == 0 and N * (K + 32) <= 57344 and w.dtype == a.dtype == bf16 and w.is_contiguous() and a.dim() == 2 and a.shape[1] == K
+            and a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.shape[0] > 0)
+
+
 def linear_any(a: torch.Tensor, w: torch.Tensor, out_dtype=None, relu_squared: bool = False) -> torch.Tensor:
     """a [M, K] w^T (then max(z, 0)^2) for a weight [N, K] of the same dtype: the MFMA GEMM for bf16 (the activation in its epilogue), the 32-bit
     kernel for float32."""
     if not _f32(a):
         if not relu_squared and rows_take(*a.shape, w.shape[0]) and w.dtype == bf16 and w.is_contiguous() and w.shape[0] % 2 == 0:   # (odd: gemm raises)
             return rows_gemm(a, w, out_dtype or bf16)
+        if out_dtype == torch.float32 and not relu_squared and thin_takes(a, w):
+            _chk(a, name="a"), _chk(w, name="w")
+            out = torch.empty((a.shape[0], w.shape[0]), dtype=torch.float32, device=a.device)
+            hip.get_lib().call("aria_thin_product_f32", _p(a), _p(w), _p(out), *out.shape, a.shape[1], _rowmajor_2d(a, "a"), w.shape[0], _stream(a))
+            return out
         return gemm(a, w, out_dtype=out_dtype or bf16, act="relu_squared" if relu_squared else None)
     _chk(w, torch.float32, "w")
     M, K = a.shape

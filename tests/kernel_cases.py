@@ -1138,6 +1138,22 @@ def case_gemm_keep_sums(dev, M, N, K):
     assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
 
 
+def case_thin_product(dev, M, N, K):
+    """A product of few columns in 32 bits against 64: exact products of bf16, a 32-bit sum of K of them."""
+    from aria_amd import ops
+
+    x, w = rnd(M, K + 8, seed=1), rnd(N, K, seed=2)
+    a, b = x.to(dev)[:, :K], w.to(dev)
+    assert ops.thin_takes(a, b)
+    out = torch.empty((M, N), dtype=torch.float32, device=dev)
+    from aria_amd import hip
+
+    hip.get_lib().call("aria_thin_product_f32", a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, K + 8, N, ops._stream(a))
+    x = x[:, :K].double()
+    want, size = x @ w.double().t(), x.abs() @ w.double().abs().t()
+    assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -20 * size).all())
+
+
 def case_sort_rows(dev, T, k, E):
     """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
     from aria_amd import ops

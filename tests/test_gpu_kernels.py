@@ -246,6 +246,11 @@ def test_gemm_keep_sums(M, N, K):
     C.case_gemm_keep_sums(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (5580, 32, 1536), (1000, 24, 1728), (300, 16, 3328)])
+def test_thin_product(M, N, K):
+    C.case_thin_product(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("T,k,E", C.SORT_ROWS + [(16384, 6, 64), (53001, 6, 64)])
 def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
