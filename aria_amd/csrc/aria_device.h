@@ -338,6 +338,7 @@ __device__ __forceinline__ void glds16_agent(const void* g, void* lds_wave_base)
 // write and puts `s_waitcnt vmcnt(0)` in front of every LDS read that follows a __builtin_amdgcn_global_load_lds -- a complete drain of
 // the prefetch at its first consumer.  Invisible to the compiler's counters, the piece stays in flight until the caller's wait_vm<N>().
 // (Compiler-issued loads stay correct next to it: a counted wait only ever waits longer when more operations are outstanding.)
+// The s_nop: a scalar write of M0 needs one wait state in front of a load to LDS; nothing inserts it inside an asm block.
 __device__ __forceinline__ void glds16_raw(const void* g, void* lds_wave_base) {
 #ifdef ARIA_EMU
     emu::glds(g, static_cast<char*>(lds_wave_base) + 16 * emu::lane());
@@ -345,7 +346,7 @@ __device__ __forceinline__ void glds16_raw(const void* g, void* lds_wave_base) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     const uint32_t lds = __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>(lds_wave_base)));
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
 #pragma clang diagnostic pop
 #endif
 }
@@ -357,7 +358,7 @@ __device__ __forceinline__ void glds4_raw(const void* g, void* lds_wave_base) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
     const uint32_t lds = __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>(lds_wave_base)));
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
 #pragma clang diagnostic pop
 #endif
 }

@@ -181,3 +181,11 @@ def test_router_reduction_loop_keeps_its_dma_pieces_in_flight():
     waits = [s for s in c if s.startswith("s_waitcnt") and "vmcnt" in s]
     assert waits and all("vmcnt(12)" in s for s in waits), waits
     assert not [s for s in c if s.startswith("global_load_dwordx4")], "an operand fragment is read straight from global memory again"
+
+
+@pytest.mark.parametrize("src", ["attn.hip", "gemm3.hip", "gemm4.hip", "moe.hip"])
+def test_m0_has_its_wait_state(src):
+    """A scalar write of M0 and the load to LDS that reads it are not neighbours: gfx9 wants one wait state between them, and inside an asm block only the source can put it there."""
+    c = [s for s, _ in code(isa(src))]
+    loads = [i for i, s in enumerate(c) if s.startswith("global_load_lds")]
+    assert loads and not [i for i in loads if re.match(r"s_\w+ m0,", c[i - 1])]
