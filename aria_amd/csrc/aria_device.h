@@ -371,6 +371,18 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 #endif
 }
+// wait_vm<N>() and sync() where c (wave-uniform) is even, nothing where it is odd: one block of code, so that a loop with two steps a barrier stays one
+template <int N>
+__device__ __forceinline__ void wait_vm_sync_even(int c) {
+#ifdef ARIA_EMU
+    if (!(c & 1)) {
+        wait_vm<N>();
+        sync();
+    }
+#else
+    asm volatile("s_bitcmp1_b32 %0, 0\n\ts_cbranch_scc1 1f\n\ts_waitcnt vmcnt(%1) lgkmcnt(0)\n\ts_barrier\n1:" ::"s"(c), "n"(N) : "memory", "scc");
+#endif
+}
 __device__ __forceinline__ void wait_lds() {  // all of this wave's LDS reads/writes have completed
 #ifndef ARIA_EMU
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -23,60 +23,71 @@ constexpr int kMaxPerLane = 4;  // E <= 256
 // memory that is 32 cache lines per wave-instruction through the vector L1 (102 us per launch with one wave per token block, 74 us with two and
 // three chunks of prefetch, against ~10 us of traffic).  Here a wave-instruction is an LDS-DMA piece of 8 whole 128-byte row chunks
 // (global_load_lds_dwordx4: lane -> row 8 j + (l >> 3), 16-byte piece (l & 7) ^ (row & 7) -- the XOR spreads a fragment read's 8 rows over the
-// banks), three stages of 128 reduction indices with counted waits, and the fragments come back by ds_read_b128.  Every wave brings its eighth
-// of a stage (1 + NB pieces), the first NB waves multiply (one 32-expert block each), all eight route (four tokens each).  What bounds it at up to
-// one block per CU is not bytes but the two serial chains: D / 128 barrier-to-barrier steps, then the top-k of a wave's tokens (~1 us a token).
-// With NB waves a block, stages of 64 and 16 tokens a wave those were 43 - 46 us at ANY token count up to 8192; now, 2560 -> 64 with 6 of 64 chosen
-// (before / now, each with the 5 us clearing launch): 777 tokens 46.6 / 20.8 us, 4096 42.7 / 21.9, 8192 46.3 / 27.2, 16 384 62.5 / 39.5.
-// Every logit is ONE accumulator run over the whole reduction in gemm's order: bit-identical to gemm + route.
+// banks), six stages of 64 reduction indices with counted waits, and the fragments come back by ds_read_b128.  NB waves stage and multiply (one
+// 32-expert block each), all eight route (four tokens each).  What bounds it at up to one block per CU is not bytes but the two serial chains: D / 128
+// barriers (two chunks a barrier), then the top-k of a wave's tokens (~1 us a token).  With NB waves a block, a barrier a chunk and 16 tokens a wave those
+// were 43 - 46 us at ANY token count up to 8192; now, 2560 -> 64 with 6 of 64 chosen (before / now, each with the 5 us clearing launch): 777 tokens
+// 46.6 / 23.8 us, 4096 42.7 / 25.0, 8192 46.3 / 28.7, 16 384 62.5 / 42.4.  Every logit is ONE accumulator run over the whole reduction in gemm's order:
+// bit-identical to gemm + route.
 template <int NB>
 __global__ __launch_bounds__(512) void router_fused_kernel(const bf16_t* x, const bf16_t* w, bf16_t* logits, bf16_t* scores, int32_t* indices,
                                                            int32_t* counts, int T, int D, int k, long long ldx) {
-    constexpr int E = 32 * NB, ST = 3, XT = 4096, WT = 4096, HALF = XT + NB * WT, STAGE = 2 * HALF;
-    constexpr int PER = 1 + NB;             // DMA pieces per wave and chunk
+    constexpr int E = 32 * NB, CH = 4, ST = 6, XT = 4096, WT = 4096, STAGE = XT + NB * WT;
+    constexpr int XP = 4 / NB;              // x pieces per multiplying wave and chunk (the tile's four 8-row pieces dealt to them)
+    constexpr int PER = XP + 4;             // DMA pieces per multiplying wave and chunk
     ARIA_SMEM_STATIC char stage[ST * STAGE];
     ARIA_SMEM_STATIC bf16_t tile[32 * E];
     ARIA_SMEM_STATIC int hist[64];
-    const int l = threadIdx.x & 63, lr = l & 31, kh = l >> 5, b = first_lane(int(threadIdx.x) >> 6), half = b >> 2, q = b & 3;
+    const int l = threadIdx.x & 63, lr = l & 31, kh = l >> 5, b = first_lane(int(threadIdx.x) >> 6);
     const int t0 = blockIdx.x * 32;
     if (b == 0) hist[l] = 0;
-    const int nch = D / 128;
-    // this lane's part of a piece: row (l >> 3) of the piece's 8, source piece (l & 7) ^ (row & 7) (row & 7 == l >> 3).  Wave b brings, of half
-    // b >> 2 of every chunk, rows 8 (b & 3) .. of the x tile and of each weight tile
-    const int prow = 8 * q + (l >> 3), psrc = 64 * half + ((l & 7) ^ (l >> 3)) * 8;
-    const bf16_t* xsrc = x + (long long)min(t0 + prow, T - 1) * ldx + psrc;   // (rows past T: clamped, never stored)
-    const bf16_t* wsrc = w + (long long)prow * D + psrc;
-    auto issue = [&](int c) __attribute__((always_inline)) {   // chunk c -> stage c % ST (past the end: the last chunk again, into a free stage)
-        const int cc = min(c, nch - 1);
-        char* st = stage + (c % ST) * STAGE + half * HALF + q * 1024;
-        glds16_raw(xsrc + cc * 128, st);
-#pragma unroll
-        for (int j = 0; j < NB; ++j) glds16_raw(wsrc + (long long)(32 * j) * D + cc * 128, st + XT + j * WT);
-    };
+    const int nch = D / 64;   // (even: D % 256 == 0)
     f32x16 acc;
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+    if (b < NB) {
+        // this lane's part of a piece: row (l >> 3) of the piece's 8, source piece (l & 7) ^ (row & 7) (row & 7 == l >> 3)
+        const int prow = l >> 3, psrc = ((l & 7) ^ prow) * 8;
+        const bf16_t* xsrc[XP];
 #pragma unroll
-    for (int c = 0; c < ST - 1; ++c) issue(c);
-    const int fo = lr * 128;   // fragment row offset; piece q of row lr sits in slot q ^ (lr & 7)
-    for (int c = 0; c < nch; ++c) {
-        wait_vm<(ST - 2) * PER>();   // this wave's pieces of chunk c have landed (the newer chunk stays in flight)
-        sync();                      // ... and every other wave's; the readers of chunk c - 1 are done with its stage
-        issue(c + ST - 1);           // -> stage (c - 1) % ST
-        if (b < NB) {
-            const char* st = stage + (c % ST) * STAGE + fo;
-            s16x8 xa[8], wb[8];
+        for (int j = 0; j < XP; ++j) xsrc[j] = x + (long long)min(t0 + 8 * (b * XP + j) + prow, T - 1) * ldx + psrc;   // (rows past T: clamped, never stored)
+        const bf16_t* wsrc = w + (long long)(32 * b + prow) * D + psrc;
+        int slot_in = 0;
+        auto issue = [&](int c) __attribute__((always_inline)) {   // chunk c -> the next stage (past the end: the last chunk again, into a free stage)
+            const int cc = min(c, nch - 1);
+            char* st = stage + slot_in;
+            slot_in = slot_in == (ST - 1) * STAGE ? 0 : slot_in + STAGE;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int slot = (i >> 2) * HALF + ((2 * (i & 3) + kh) ^ (lr & 7)) * 16;
-                xa[i] = *reinterpret_cast<const s16x8*>(st + slot);
-                wb[i] = *reinterpret_cast<const s16x8*>(st + XT + b * WT + slot);
+            for (int j = 0; j < XP; ++j) glds16_raw(xsrc[j] + cc * 64, st + (b * XP + j) * 1024);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) glds16_raw(wsrc + (long long)(8 * j) * D + cc * 64, st + XT + b * WT + j * 1024);
+        };
+#pragma unroll
+        for (int c = 0; c < 4; ++c) issue(c);
+        const int fo = lr * 128;   // fragment row offset; piece q of row lr sits in slot q ^ (lr & 7)
+        int slot = 0;
+#pragma nounroll
+        for (int c = 0; c < nch; ++c) {
+            // (even c) this wave's pieces of chunks c and c + 1 have landed, the two newer ones stay in flight; and the other wave's; the readers of
+            // chunks c - 2 and c - 1 are done with their stages
+            wait_vm_sync_even<2 * PER>(c);
+            issue(c + 4);             // -> the stage of chunk c - 2
+            const char* st = stage + slot + fo;
+            slot = slot == (ST - 1) * STAGE ? 0 : slot + STAGE;
+            s16x8 xa[CH], wb[CH];
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+                const int piece = ((2 * i + kh) ^ (lr & 7)) * 16;
+                xa[i] = *reinterpret_cast<const s16x8*>(st + piece);
+                wb[i] = *reinterpret_cast<const s16x8*>(st + XT + b * WT + piece);
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc = mfma32(xa[i], wb[i], acc);
+            for (int i = 0; i < CH; ++i) acc = mfma32(xa[i], wb[i], acc);
         }
+        wait_vm<0>();   // (the duplicate pieces of the last steps: nothing may still be writing the LDS when the block ends)
+    } else {
+        for (int c = 0; c < nch; c += 2) sync();   // (the waves that only route)
     }
-    wait_vm<0>();   // (the duplicate pieces of the last steps: nothing may still be writing the LDS when the block ends)
     // C layout of the 32 x 32 tile: register j of lane l = (token (j & 3) + 8 (j >> 2) + 4 (l >> 5), expert l & 31)
     if (b < NB) {
 #pragma unroll

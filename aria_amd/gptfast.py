@@ -217,7 +217,7 @@ class MOEFeedForward(nn.Module):
         if not few and ops.router_fusable(x2d.shape[1], self.gate.weight.shape[0], k):   # K1: gate GEMM + topk + softmax (model.py:355-363) as one launch
             logits, scores, idx, counts = ops.moe_router_fused(x2d, self.gate.weight, k)
         else:
-            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 20 us at any such count, 22 in two launches for 280 tokens, less for fewer)
+            logits = _project(x2d, self.gate.weight)   # (32 tokens a workgroup of the fused form: 24 us at any such count, 22 in two launches for 280 tokens, less for fewer)
             scores, idx, counts = ops.moe_route(logits, k)             # topk + softmax (model.py:359-363)
         offsets, sorted_src, inv, rows = ops.moe_sort_rows(idx, counts)   # token_permutation (:243-254)
         cf = self.cond_ffn
