@@ -110,7 +110,7 @@ class DuguzenForCausalLM(nn.Module):
         self.caches: List[LatentCache] = []
         self.ropes: List[torch.Tensor] = []
         self._decode: Optional["_DecodeTables"] = None
-        self._shapes = shapes_of(self)
+        self._shapes = shapes_of(self) if dtype == f32 else None
 
     @classmethod
     def from_tensors(cls, config: dict, tensors: Dict[str, torch.Tensor], device="cuda", dtype=bf16) -> "DuguzenForCausalLM":
@@ -210,9 +210,10 @@ class _DecodeTables:
                     t.w_router, t.correction = L.mlp.router.data_ptr(), L.mlp.correction.data_ptr()
         self.stack = hip.LatentStack(n, model.width, model.head.shape[0], model.layer(0).norm1.params(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows = model.device, model.head.shape[0]
-        self.held = Held(model, model._shapes, [(m.__dict__, "alpha", m.alpha) for m in model.modules() if isinstance(m, DynamicTanh)]
-                         + [(c.__dict__, "rows", c.rows) for c in model.caches] + [(model.ropes, i, t) for i, t in enumerate(model.ropes)]
-                         + [(model.caches, i, c) for i, c in enumerate(model.caches)])
+        if model.dtype == f32:
+            self.held = Held(model, model._shapes, [(m.__dict__, "alpha", m.alpha) for m in model.modules() if isinstance(m, DynamicTanh)]
+                             + [(c.__dict__, "rows", c.rows) for c in model.caches] + [(model.ropes, i, t) for i, t in enumerate(model.ropes)]
+                             + [(model.caches, i, c) for i, c in enumerate(model.caches)])
 
     def run_f32(self, batch) -> torch.Tensor:
         T, W, lib = batch.ids.numel(), batch.wanted.numel() if batch.wanted is not None else -1, hip.get_lib()

@@ -121,7 +121,7 @@ class KozipelForCausalLM(nn.Module):
         self.caches: List[list] = []
         self.geometry = None
         self._decode: Optional["_DecodeTables"] = None
-        self._shapes = shapes_of(self)
+        self._shapes = shapes_of(self) if dtype == f32 else None
 
     @classmethod
     def from_tensors(cls, config: dict, tensors: Dict[str, torch.Tensor], device="cuda", dtype=bf16) -> "KozipelForCausalLM":
@@ -217,9 +217,10 @@ class _DecodeTables:
         self.stack = hip.MixStack(n, model.width, c.width, model.head.shape[0], c.embedding_scale, c.residual_mult, c.eps, c.logit_softcap,
                                   model.layers[c.runs[0].layer].norm1.weight.data_ptr(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows, self.vocab = model.device, model.head.shape[0], model.vocab
-        flat = [c for run in model.caches for c in run]
-        self.held = Held(model, model._shapes, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
-                         + [(model.caches, i, run) for i, run in enumerate(model.caches)])
+        if model.dtype == f32:
+            flat = [c for run in model.caches for c in run]
+            self.held = Held(model, model._shapes, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
+                             + [(model.caches, i, run) for i, run in enumerate(model.caches)])
 
     def run_f32(self, batch) -> torch.Tensor:
         T, W, lib = batch.ids.numel(), batch.wanted.numel() if batch.wanted is not None else -1, hip.get_lib()
