@@ -114,7 +114,7 @@ def moe_fwd(x, router_w, fc1, fc2, gate_w, up_w, down_w, cfg: MoEConfig, save=Tr
         # checkpointed step, and (r05) the plain training step too: fc1's weight gradient reaches the token rows through the same index
         # (ops.grouped_gemm_wgrad_gather), so nothing in the backward wants `perm` as a tensor
         perm = None
-        rows = token_rows
+        rows = ops.permuted_token_rows(sorted_src, k, ready=token_rows)
         h1, act = ops.grouped_gemm_swiglu_gather(x, rows, fc1, offsets, want_h=bool(save) and not lean)
     else:
         perm = ops.moe_permute(x, sorted_src, k)

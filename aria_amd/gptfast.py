@@ -224,11 +224,11 @@ class MOEFeedForward(nn.Module):
         E, I, D = cf.w1.shape
         contiguous = all(w.is_contiguous() for w in (cf.w1, cf.w2, cf.w3))
         if contiguous and ops.rows_experts_take(sorted_src.numel(), E, D, I):
-            act = ops.rows_experts(x2d, cf.w1, offsets, rows, cf.w3)
+            act = ops.rows_experts(x2d, cf.w1, offsets, ops.permuted_token_rows(sorted_src, k, ready=rows), cf.w3)
         elif _glu_pair_ready(cf.w1, cf.w3) and ops.gather_fusable(x2d.shape[1]):
             # K2 + K3: the dispatcher's row gather (model.py:243-254) in the A loader of the fused w1 / w3 / SwiGLU launch -- no permuted copy
             # of the tokens ([6T, D]: 1.6 GB written and read per layer of a 53 K-token prefill), no h1 / h3 round trip
-            act = ops.grouped_gemm_swiglu_split_gather(x2d, rows, cf.w1, cf.w3, offsets)[1]
+            act = ops.grouped_gemm_swiglu_split_gather(x2d, ops.permuted_token_rows(sorted_src, k, ready=rows), cf.w1, cf.w3, offsets)[1]
         elif _glu_pair_ready(cf.w1, cf.w3):   # w1 / w3 GEMMs + SwiGLU in ONE launch (no h1 / h3 round trip: 2 x [6T, I] written and read)
             act = ops.grouped_gemm_swiglu_split(ops.moe_permute(x2d, sorted_src, k), cf.w1, cf.w3, offsets)[1]
         else:

@@ -208,11 +208,11 @@ class GroupLimitedMixture(nn.Module):
         g, u = self.gate, self.up
         if h.dtype == bf16 and ops.rows_experts_take(sorted_src.numel(), self.n_experts, h.shape[1], self.ff) and not (
                 ops.experts_tiles_ahead(sorted_src.numel(), self.n_experts, h.shape[1], self.ff) and ops.gather_fusable(h.shape[1]) and _glu_pair_ready(g, u)):
-            act = ops.rows_experts(h, g, offsets, token, u)
+            act = ops.rows_experts(h, g, offsets, ops.permuted_token_rows(sorted_src, self.top, ready=token), u)
             if ops.rows_experts_take(sorted_src.numel(), self.n_experts, self.ff, h.shape[1], down=True):
                 return dict(y=ops.rows_experts(act, self.down, offsets), inv=inv, weights=weights)
         elif h.dtype == bf16 and ops.gather_fusable(h.shape[1]) and _glu_pair_ready(g, u):
-            act = ops.grouped_gemm_swiglu_split_gather(h, token, g, u, offsets)[1]
+            act = ops.grouped_gemm_swiglu_split_gather(h, ops.permuted_token_rows(sorted_src, self.top, ready=token), g, u, offsets)[1]
         else:
             rows = ops.permute_any(h, sorted_src, self.top)
             act = ops.act_rows(ops.grouped_linear_any(rows, u, offsets), gate=ops.grouped_linear_any(rows, g, offsets))

@@ -557,9 +557,11 @@ def gather_fusable(K: int) -> bool:
     return K % 64 == 0 and K >= 64 and os.environ.get("ARIA_FUSE_GATHER", "1") != "0"
 
 
-def permuted_token_rows(sorted_src: torch.Tensor, k: int, pad: int = 64) -> torch.Tensor:
+def permuted_token_rows(sorted_src: torch.Tensor, k: int, pad: int = 64, ready=None) -> torch.Tensor:
     """Token row of every permuted row (``sorted_indices // topk``, moe_lm.py:330): int32 [T * k] -- a view of a buffer with ``pad`` more entries
-    (the weight gradient's gathered loader reads a whole K-tile of indices at the end of the last expert)."""
+    (the weight gradient's gathered loader reads a whole K-tile of indices at the end of the last expert).  ``ready``: what moe_sort_rows returned."""
+    if ready is not None:
+        return ready
     n = sorted_src.numel()
     buf = torch.zeros((n + pad,), dtype=torch.int32, device=sorted_src.device)
     torch.div(sorted_src, k, rounding_mode="floor", out=buf[:n])
@@ -759,9 +761,8 @@ def moe_sort(indices: torch.Tensor, counts: torch.Tensor) -> Tuple[torch.Tensor,
 
 
 def moe_sort_rows(indices: torch.Tensor, counts: torch.Tensor, pad: int = 64):
-    """moe_sort and ``permuted_token_rows`` of its order, in the same launches: -> offsets, sorted_src, inv, rows."""
-    out = _sort(indices, counts, pad)
-    return out if out[3] is not None else out[:3] + (permuted_token_rows(out[1], indices.shape[1], pad),)
+    """moe_sort and ``permuted_token_rows`` of its order, in the same launches: -> offsets, sorted_src, inv, rows (more than 64 experts: None)."""
+    return _sort(indices, counts, pad)
 
 
 def _sort(indices: torch.Tensor, counts: torch.Tensor, pad: int):

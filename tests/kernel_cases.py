@@ -1167,6 +1167,8 @@ def case_sort_rows(dev, T, k, E):
     want = torch.argsort(idx.flatten().long(), stable=True)
     assert torch.equal(src.cpu().long(), want) and torch.equal(inv.cpu().long(), torch.argsort(want))
     assert torch.equal(off.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), counts.long().cumsum(0)]))
+    assert (rows is None) == (E > 64)
+    rows = ops.permuted_token_rows(src, k, ready=rows)
     assert torch.equal(rows.cpu().long(), want // k)
     behind = torch.as_strided(rows, (64,), (1,), rows.storage_offset() + rows.numel())   # the weight gradient's loader reads these
     assert not bool(behind.any())
