@@ -4,10 +4,11 @@
 //   down:   d_u = scale * dy W^T                   with lora_B
 //   up:     dx += keep ? (d_u A) / (1 - p) : 0     the adapter's input gradient through its dropout mask, added where the base's gradient lies
 //   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
-// All three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
-// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9 (the scaling alone 16 with its copy, here 3.5); up as a product and a masked add 22, here 10; wgrad as
-// a split product and its sum 24, here 11 (64 rows a block: 12.5 us on cold rows, with 128 and four loads in flight a wave 15.5).  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take
-// 21 and 43); an adapted training step of 4 x 1024 tokens 11 470 / 9 780.
+// The last three are bound by the bytes of the one wide operand; a 256-wide tile of the general kernels is 97 % padding here.  Rank 8, us a call with the launches:
+// 4096 rows of 2560, down as a split 256 x 256 tile, its sum and three passes for the scaling 37, here 9 (the scaling alone 16 with its copy, here 3.5); up as a
+// product and a masked add 22, here 10; wgrad as a split product and its sum 24, here 11 (64 rows a block: 12.5 us on cold rows, with 128 and four loads in flight a
+// wave 15.5).  24 576 rows of 64 experts, 2560 wide: down 51 and 12 for the scaling, here 26; up 142, here 51 (6.1 TB/s would take 21 and 43).  An adapted training
+// step of 4 x 1024 tokens 11 350 / 10 030.
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "elem.h"
