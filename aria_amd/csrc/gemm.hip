@@ -389,7 +389,7 @@ int aria_last_gemm_variant(void) { return g_last_variant; }
 
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc) {
     if (M <= 0 || N <= 0 || (a_oc && !b_oc)) return 0;
-    return std::max(aria_gemm3_workspace_bytes(M, N, K), a_oc ? 0 : aria_gemm4_workspace_bytes(M, N, K));
+    return std::max(aria_gemm3_workspace_bytes(M, N, K), a_oc || !b_oc ? 0 : aria_gemm4_workspace_bytes(M, N, K));
 }
 
 int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,

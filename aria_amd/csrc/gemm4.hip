@@ -610,11 +610,16 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
         return plan;
     }
     double best = 0.94 * time_else(p.M, p.N, n, split3);
-    int s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
+    // [N, K] weights are a forward pass's: its sums are cut where the 256 x 256 tiles cut them, and so have their bits.  Another cut rounds a few elements otherwise, and
+    // where a router follows, a near tie of a token's last expert turns.  777 x 2560 x 2560 in 3 pieces (27 us) for 4 (33) and 4500 x 1536 x 4096 whole (57) for 2 (68) so moved
+    // single elements of a training step's gradients and of a prompt's latents by 1.5 and 0.45 of their root mean square.  [K, N] weights (input gradients) are cut as it is
+    // fastest.
+    int s = split3;
+    if (b_oc) s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
     if (t2 * s <= ROUND && time_128(t2, n, s) < best) best = time_128(t2, n, s), plan.form = 1, plan.split = s;
     const long long t6 = b_oc ? cdiv(p.M, 128) * cdiv(p.N, 320) : cdiv(p.M, 256) * cdiv(p.N, 160);
     const double time6 = 9.0 + (b_oc ? 1.0 : 0.85) * n;
-    if (t6 <= ROUND && time6 < best && !(b_oc && p.K > 4096)) plan.form = 2, plan.split = 1;
+    if (t6 <= ROUND && time6 < best && (b_oc ? p.K <= 4096 : split3 == 1)) plan.form = 2, plan.split = 1;
     return plan;
 }
 

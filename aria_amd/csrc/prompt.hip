@@ -21,8 +21,8 @@ struct Scratch {
     char* ws;
     int64_t ws_bytes, bytes;
 };
-// A dense product x [T, K] w [N, K]^T as tiles (its reduction in pieces).  Weights from HBM, us by rows / tiles: 7680 x 2560: 128 tokens 23.7 / 23.7, 192 29.3 / 28.3, 256 34.8 /
-// 29.7; 2560 x 2560: 192 16.3 / 18.1, 256 19.2 / 18.2, 288 20.9 / 19.5; 2560 x 3328: 192 20.9 / 19.0, 288 31.4 / 21.7.  Narrower: 4096 x 1536: 288 19.3 / 18.9.
+// A dense product x [T, K] w [N, K]^T as tiles (its reduction in pieces).  Weights from HBM, us by rows / tiles: 7680 x 2560: 128 tokens 23.7 / 23.7, 200 32.0 / 27.7, 256 34.8 /
+// 28.0, 288 38.4 / 37.0; 2560 x 2560: 200 18.9 / 18.7, 288 21.1 / 19.7; 2560 x 3328: 200 23.2 / 19.0, 288 31.1 / 21.6.  Narrower: 4096 x 1536: 288 19.3 / 18.9.
 bool tiles_ahead(int64_t T, int64_t N, int64_t K) { return T > 192 && K >= 2048 && N * K >= (6 << 20) && K % 64 == 0 && N % 8 == 0; }
 Scratch layout(const int64_t* dims, int64_t T, char* base) {
     const int64_t L = dims[0], D = dims[1], E = dims[4], k = dims[5], I = dims[6], Is = dims[7];

@@ -139,6 +139,18 @@ def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
         assert torch.equal(x.cpu(), y.cpu())
 
 
+def case_gemm_forward_sums(dev, monkeypatch, M, N, K):
+    """A product with [N, K] weights has the sums of the 256 x 256 tiles bit for bit, whichever tiles compute it: a forward pass's products lie in front of routers, whose
+    near ties turn with another cut of the reduction."""
+    from aria_amd import ops
+
+    a, b, bias = rnd(M, K, seed=M + K).to(dev), rnd(N, K, seed=N, scale=0.3).to(dev), rnd(N, seed=3).to(dev)
+    got = [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]
+    monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
+    for x, y in zip(got, [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]):
+        assert torch.equal(x.cpu(), y.cpu())
+
+
 def case_gemm_workspace_kept(dev):
     """What is kept per stream is one buffer of a fixed size; a larger need is the call's own and leaves nothing behind."""
     from aria_amd import ops

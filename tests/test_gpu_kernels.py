@@ -379,7 +379,12 @@ def test_gemm_four_waves_fused(monkeypatch):
         C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
 
 
-@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 1536, False), (130, 1024, 1664, True)])
+@pytest.mark.parametrize("M,N,K", [(40, 1032, 1536), (777, 2560, 2560), (777, 2560, 3328), (777, 7680, 2560), (1868, 2560, 2560), (4500, 1536, 4096), (200, 2560, 6656)])
+def test_gemm_forward_sums(monkeypatch, M, N, K):
+    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 1664, True)])
 def test_gemm_four_waves_split(M, N, K, b_oc):
     """A reduction cut into pieces of whole stages, by the rule itself."""
     C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)
