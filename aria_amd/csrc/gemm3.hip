@@ -1174,6 +1174,14 @@ long long aria_gemm3_workspace_bytes(long long M, long long N, long long K) {
     return S > 1 ? R * S * (long long)(BM * BN) * 4 : 0;
 }
 
+int aria_gemm3_cut(long long M, long long N, long long K, long long* first_row) {
+    long long R = 0;
+    const long long tiles = (M + 255) / 256;
+    const int S = aria_gemm3_workspace_bytes(M, N, K) > 0 ? plan_split(tiles, (K + 63) / 64, &R) : 1;
+    *first_row = 256 * (tiles - R);
+    return S;
+}
+
 int aria_gemm3_split(long long M, long long N, long long K) {
     long long R = 0;
     const long long tiles = ((M + 255) / 256) * ((N + 255) / 256);

@@ -317,6 +317,8 @@ __attribute__((visibility("hidden"))) int aria_launch_gemm4(const GemmParams& p,
 __attribute__((visibility("hidden"))) long long aria_gemm4_workspace_bytes(long long M, long long N, long long K);
 // pieces the v3 remainder split-K would take for a dense problem of at most one round (1: none)
 __attribute__((visibility("hidden"))) int aria_gemm3_split(long long M, long long N, long long K);
+// pieces that the v3 remainder split-K (with a workspace) takes for a dense problem of one column tile, for the rows from *first_row on (1: none)
+__attribute__((visibility("hidden"))) int aria_gemm3_cut(long long M, long long N, long long K, long long* first_row);
 // gate and up of rows by expert, gathered, as four-wave tiles: w_gate, w_up [E, I, K] anywhere; act [M, I].  ARIA_ERR_UNSUPPORTED: sizes of other kernels
 __attribute__((visibility("hidden"))) int aria_expert_pair_tiles(const void* X, const int32_t* rows, int64_t T, const void* w_gate, const void* w_up, void* act, const int32_t* offsets,
                                                                  int64_t E, int64_t M, int64_t I, int64_t K, int64_t ldx, void* stream);

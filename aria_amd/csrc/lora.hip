@@ -12,6 +12,7 @@
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "elem.h"
+#include "gemm_params.h"
 #include <algorithm>
 
 namespace {
@@ -54,17 +55,11 @@ __global__ __launch_bounds__(256) void lora_scale_kernel(const bf16_t* u, bf16_t
     st16(out + i / pieces * ldo + 8 * (i % pieces), o);
 }
 
-__device__ __forceinline__ void put(bf16_t* p, float v) { *p = f2bf(v); }
-__device__ __forceinline__ void put(float* p, float v) { *p = v; }
-
 // u[m][n] = scale * sum_k X[m][k] W[n][k], n < r.  W: [r][K], or with w_oc [K][r]; per expert where there are offsets.
 // The factor is staged once a block, k-contiguous whichever way it lies; the eight waves take every eighth 64 columns of the reduction, four such steps of 32 rows
 // in flight each, straight from global memory (16-row fragments of v_mfma_f32_16x16x32_bf16 read 64 bytes of a row, its neighbour the other half of the line).
 // Splitting the reduction over the waves is what puts 4096 rows on 128 CUs with all of a block's bytes in flight at once.
-// NG: groups of 16 columns.  Also the router's product of a mixture with up to 32 experts, in 32 bits (T = float): 5580 rows of 1536 on 32 columns as one 128 x 128 tile
-// of the general kernel per 128 rows 32 us, here 12.
-template <int NG, class T>
-__global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const bf16_t* W, T* U, const int32_t* offsets, int E, int M, int K, int r, int w_oc,
+__global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const bf16_t* W, bf16_t* U, const int32_t* offsets, int E, int M, int K, int r, int w_oc,
                                                         long long ldx, long long ldu, float scale) {
     ARIA_DYN_SMEM(lds);
     bf16_t* wt = reinterpret_cast<bf16_t*>(lds);
@@ -101,44 +96,94 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
         }
     }
     sync();
-    f32x4 acc[2][NG];
+    f32x4 acc[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int g = 0; g < NG; ++g) acc[h][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16_t* wr[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) wr[g] = wt + min(16 * g + lr, r - 1) * pitch + 8 * kg;   // (past the last column: the last one again, never stored)
+    for (int h = 0; h < 2; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16_t* wr = wt + min(lr, r - 1) * pitch + 8 * kg;   // (past the last column: the last one again, never stored)
     for (int c0 = w; c0 < nch; c0 += 32) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             if (c0 + 8 * i < nch)
 #pragma unroll
-                for (int s = 0; s < 2; ++s)
+                for (int s = 0; s < 2; ++s) {
+                    const s16x8 b = *reinterpret_cast<const s16x8*>(wr + (c0 + 8 * i) * 64 + 32 * s);
 #pragma unroll
-                    for (int g = 0; g < NG; ++g) {
-                        const s16x8 b = *reinterpret_cast<const s16x8*>(wr[g] + (c0 + 8 * i) * 64 + 32 * s);
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) acc[h][g] = mfma16(x[i][h][s], b, acc[h][g]);
-                    }
+                    for (int h = 0; h < 2; ++h) acc[h] = mfma16(x[i][h][s], b, acc[h]);
+                }
         if (c0 + 32 < nch) load(c0 + 32);
     }
     sync();
-    float* red = reinterpret_cast<float*>(lds);   // [wave][row][16 NG]
+    float* red = reinterpret_cast<float*>(lds);   // [wave][row][16]
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) red[(w * ROWS + 16 * h + 4 * kg + i) * 16 * NG + 16 * g + lr] = acc[h][g][i];
+        for (int i = 0; i < 4; ++i) red[(w * ROWS + 16 * h + 4 * kg + i) * 16 + lr] = acc[h][i];
     sync();
     for (int i = threadIdx.x; i < ROWS * r; i += 512) {
         const int row = i / r, n = i % r;
         float s = 0.f;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) s += red[(q * ROWS + row) * 16 * NG + n];
-        if (m0 + row < m1) put(U + (long long)(m0 + row) * ldu + n, scale * s);
+        for (int q = 0; q < 8; ++q) s += red[(q * ROWS + row) * 16 + n];
+        if (m0 + row < m1) U[(long long)(m0 + row) * ldu + n] = f2bf(scale * s);
     }
+}
+
+// C[m][n] = sum_k X[m][k] W[n][k] in 32 bits, N <= 32 columns: the router's product of a mixture with up to 32 experts.
+// The choice of experts hangs on its last bits, so they are those of the general tiles: an element is one chain of v_mfma_f32_32x32x16_bf16 over the reduction, in `cut` pieces
+// for the rows from cut_row on, where those tiles would split it.  That chain (K / 16 products of one wave) and a block's own loads are the time; splitting the reduction
+// over the waves adds in another order and is ahead only where a block's own chain is longest (us: 5580 rows of 1536 on 32 columns 9.9, here 9.8; 16 384 rows 16.2, here 18.9;
+// 2000 rows of 3328 on 16 10.1, here 18.3).  The eight waves stage W once a block and X in rounds of 512 columns, the next round in flight in registers; the first wave multiplies.
+// 5580 rows of 1536 on 32 columns as 128 x 128 tiles of the general kernel 25.8 us.
+constexpr int XR = 512, XPITCH = XR + 8;   // (16 bytes: 16 rows' pieces lie on different banks)
+__global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, float* C, int M, int N, int K, long long ldx, long long ldc, int cut_row,
+                                                           int cut) {
+    ARIA_DYN_SMEM(lds);
+    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), pitch = K + 8, nch = K / 64, m0 = blockIdx.x * ROWS, pieces = m0 >= cut_row ? cut : 1;
+    bf16_t* xs = reinterpret_cast<bf16_t*>(lds);   // [32][XPITCH]
+    bf16_t* ws = xs + ROWS * XPITCH;               // [N][pitch]
+    u32x4 x[4];
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        if (k0 + 8 * l < K)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = ld16(X + (long long)min(m0 + w + 8 * i, M - 1) * ldx + k0 + 8 * l);   // (rows past the end: the last one, never stored)
+    };
+    load(0);
+#pragma unroll 6
+    for (int i = t; i < N * K / 8; i += 512) st16(ws + i / (K / 8) * pitch + 8 * (i % (K / 8)), ld16(W + 8ll * i));
+    f32x16 acc, sum;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = sum[j] = 0.f;
+    const bf16_t *xf = xs + (l & 31) * XPITCH + 8 * (l >> 5), *wf = ws + min(l & 31, N - 1) * pitch + 8 * (l >> 5);
+    int piece = 0;
+    for (int c0 = 0; c0 < nch; c0 += XR / 64) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st16(xs + (w + 8 * i) * XPITCH + 8 * l, x[i]);
+        load(64 * c0 + XR);
+        sync();
+        if (w == 0) {
+#pragma unroll
+            for (int cc = 0; cc < XR / 64; ++cc) {
+                const int c = c0 + cc;
+                if (c >= nch) break;
+                if (piece + 1 < pieces && c == int((long long)nch * (piece + 1) / pieces)) {
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) sum[j] = piece ? sum[j] + acc[j] : acc[j], acc[j] = 0.f;
+                    ++piece;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc = mfma32(*reinterpret_cast<const s16x8*>(wf + c * 64 + 16 * i), *reinterpret_cast<const s16x8*>(xf + cc * 64 + 16 * i), acc);
+            }
+        }
+        sync();
+    }
+    if (w || m0 + (l & 31) >= M) return;
+    float* out = C + (long long)(m0 + (l & 31)) * ldc + 4 * (l >> 5);   // (a lane: a row, columns 8 q + 4 (l / 32) .. + 3)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (8 * q < N)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) out[8 * q + j] = piece ? sum[4 * q + j] + acc[4 * q + j] : acc[4 * q + j];
 }
 
 __device__ __forceinline__ float half_of(const u32x4& v, int i) { return i & 1 ? bfhi(v[i >> 1]) : bflo(v[i >> 1]); }
@@ -296,26 +341,21 @@ int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const i
     if (!thin(r) || (K & 63) || lds > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
     if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
     if (M == 0) return ARIA_OK;
-    ARIA_LAUNCH((lora_down_kernel<1, bf16_t>), dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
+    ARIA_LAUNCH(lora_down_kernel, dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
                 static_cast<bf16_t*>(U), offsets, int(E), int(M), int(K), int(r), w_oc, (long long)ldx, (long long)ldu, scale);
     return aria_check_launch();
 }
 
 int aria_thin_product_f32(const void* X, const void* W, float* C, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldc, void* stream) {
     if (!X || !W || !C || M < 0 || N <= 0 || K <= 0) return ARIA_ERR_INVALID;
-    const int64_t lds = std::max<int64_t>(N * (K + PAD) * 2, 8 * ROWS * 32 * 4);
-    if (N > 32 || (N & 7) || (K & 63) || lds > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
+    const int64_t lds = N * (K + 8) * 2 + ROWS * XPITCH * 2;
+    if (N > 32 || (N & 7) || (K & 63) || N * (K + PAD) * 2 > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
     if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
     if (M == 0) return ARIA_OK;
-    const dim3 grid(row_tiles(M, nullptr, 1)), block(512);
-#define THIN(NG)                                                                                                                                                     \
-    ARIA_LAUNCH((lora_down_kernel<NG, float>), grid, block, unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W), C, (const int32_t*)nullptr, \
-                1, int(M), int(K), int(N), 0, (long long)ldx, (long long)ldc, 1.f)
-    if (N <= 16)
-        THIN(1);
-    else
-        THIN(2);
-#undef THIN
+    long long cut_row = 0;
+    const int cut = aria_gemm3_cut(M, N, K, &cut_row);
+    ARIA_LAUNCH(thin_product_kernel, dim3(row_tiles(M, nullptr, 1)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W), C, int(M),
+                int(N), int(K), (long long)ldx, (long long)ldc, int(cut_row), cut);
     return aria_check_launch();
 }
 

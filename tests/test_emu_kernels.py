@@ -252,7 +252,7 @@ def test_gemm_keep_sums(M, N, K):
     C.case_gemm_keep_sums(DEV, M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (70, 24, 128), (64, 16, 192)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (70, 24, 128), (64, 16, 192), (40, 8, 2048)])
 def test_thin_product(M, N, K):
     C.case_thin_product(DEV, M, N, K)
 

@@ -246,7 +246,7 @@ def test_gemm_keep_sums(M, N, K):
     C.case_gemm_keep_sums(DEV, M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (5580, 32, 1536), (1000, 24, 1728), (300, 16, 3328)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (5580, 32, 1536), (1000, 24, 1728), (300, 16, 3328), (66000, 8, 2048)])
 def test_thin_product(M, N, K):
     C.case_thin_product(DEV, M, N, K)
 
