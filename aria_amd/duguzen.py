@@ -19,7 +19,7 @@ import torch.nn as nn
 
 from . import hip, ops
 from .checkpoint import load_checkpoint_dir
-from .layers import (DynamicTanh, GroupLimitedMixture, Held, LatentAttention, LatentCache, SquaredReluFeedForward, _frozen, padded, rotation_table, shapes_of,
+from .layers import (DynamicTanh, GroupLimitedMixture, Held, LatentAttention, LatentCache, SquaredReluFeedForward, _frozen, functions_of, padded, rotation_table, shapes_of,
                      table_batch, up8)
 from .registry import read_config
 
@@ -165,8 +165,8 @@ class DuguzenForCausalLM(nn.Module):
             return logits if batch.every_row else logits[batch.wanted.long()]
         if self.dtype == f32 and trace is None and table_batch(batch, self.device):
             if self._decode is None or not self._decode.held.current():
-                self._decode = _DecodeTables(self)
-            if self._decode.held.plain() and all(c.rows.shape == self.caches[0].rows.shape[:2] + c.rows.shape[2:] for c in self.caches):
+                self._decode = _DecodeTables(self) if Held.made_of(self.modules(), _OWN) else None
+            if self._decode is not None and self._decode.held.plain() and all(c.rows.shape == self.caches[0].rows.shape[:2] + c.rows.shape[2:] for c in self.caches):
                 return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.dyt_stream(x, None, self.layer(0).norm1.params(), ids=batch.ids, table=self.embed)
@@ -211,7 +211,7 @@ class _DecodeTables:
         self.stack = hip.LatentStack(n, model.width, model.head.shape[0], model.layer(0).norm1.params(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows = model.device, model.head.shape[0]
         if model.dtype == f32:
-            self.held = Held(model, model._shapes, [(m.__dict__, "alpha", m.alpha) for m in model.modules() if isinstance(m, DynamicTanh)]
+            self.held = Held(model, model._shapes, _OWN, [(m.__dict__, "alpha", m.alpha) for m in model.modules() if isinstance(m, DynamicTanh)]
                              + [(c.__dict__, "rows", c.rows) for c in model.caches] + [(model.ropes, i, t) for i, t in enumerate(model.ropes)]
                              + [(model.caches, i, c) for i, c in enumerate(model.caches)])
 
@@ -236,3 +236,6 @@ class _DecodeTables:
         lib.call("aria_latent_decode", stack, layers, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.max_len,
                  logits.data_ptr(), self.scratch.data_ptr(), self.scratch.numel(), ops._stream(logits))
         return logits[:, :self.vocab]
+
+
+_OWN = functions_of(DuguzenForCausalLM, DuguzenLayer, LatentAttention, SquaredReluFeedForward, GroupLimitedMixture, DynamicTanh)

@@ -20,7 +20,7 @@ import torch.nn as nn
 
 from . import hip, ops
 from .checkpoint import load_checkpoint_dir
-from .layers import ChunkAttention, Held, LinearAttention, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, padded, shapes_of, table_batch, up8
+from .layers import ChunkAttention, Held, LinearAttention, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, functions_of, padded, shapes_of, table_batch, up8
 from .registry import read_config
 
 bf16, f32 = torch.bfloat16, torch.float32
@@ -173,10 +173,10 @@ class KozipelForCausalLM(nn.Module):
                 self._decode = _DecodeTables(self)
             logits = self._decode.run(batch)
             return logits if batch.every_row else logits[batch.wanted.long()]
-        if self.dtype == f32 and trace is None and batch.seq is not None and table_batch(batch, self.device) and all(L.mixer.table_step and L.mixer.parts[-1].eps == c.eps for L in self.layers):
+        if self.dtype == f32 and trace is None and batch.seq is not None and table_batch(batch, self.device):
             if self._decode is None or not self._decode.held.current():
-                self._decode = _DecodeTables(self)
-            if self._decode.held.plain():
+                self._decode = _DecodeTables(self) if Held.made_of(self.modules(), _OWN) and all(L.mixer.table_step for L in self.layers) else None
+            if self._decode is not None and self._decode.held.plain() and all(L.mixer.table_step and L.mixer.parts[-1].eps == c.eps for L in self.layers):
                 return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.rms_stream(x, c.width, c.eps, self.layers[c.runs[0].layer].norm1.weight, ids=batch.ids, table=self.embed, scale=c.embedding_scale)
@@ -219,7 +219,7 @@ class _DecodeTables:
         self.device, self.rows, self.vocab = model.device, model.head.shape[0], model.vocab
         if model.dtype == f32:
             flat = [c for run in model.caches for c in run]
-            self.held = Held(model, model._shapes, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
+            self.held = Held(model, model._shapes, _OWN, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
                              + [(model.caches, i, run) for i, run in enumerate(model.caches)])
 
     def run_f32(self, batch) -> torch.Tensor:
@@ -243,3 +243,6 @@ class _DecodeTables:
         lib.call("aria_mix_decode", stack, runs, T, batch.ids.data_ptr(), batch.slot.data_ptr(), batch.pos.data_ptr(), batch.max_len,
                  logits.data_ptr(), self.scratch.data_ptr(), self.scratch.numel(), ops._stream(logits))
         return logits[:, :self.vocab]
+
+
+_OWN = functions_of(KozipelForCausalLM, KozipelLayer, MixerGroup, LinearAttention, ChunkAttention, ReluGatedFeedForward, RmsNorm)

@@ -15,7 +15,7 @@ bf16 and in float32 (``dtype``); the float32 form runs the 32-bit kernels throug
 from __future__ import annotations
 
 import math
-from typing import List, Optional, Sequence
+from typing import Iterable, List, Optional, Sequence
 
 import torch
 import torch.nn as nn
@@ -45,18 +45,29 @@ def shapes_of(model: nn.Module) -> dict:
     return {n: tuple(p.shape) for n, p in model.named_parameters()}
 
 
+def functions_of(*classes: type) -> List[tuple]:
+    """(class, name, what it defines) of classes whose modules a table of addresses stands in for, as they are now"""
+    return [(c, n, f) for c in classes for n, f in vars(c).items() if callable(f) or isinstance(f, property)]
+
+
 class Held:
     """What a float32 step's table of addresses was made from: every parameter, cache and constant of a model, compared before each step that runs by the table.
-    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks or forwards of
-    its own, or with tensors other than those it was made with (``shapes``), is not ``plain``."""
+    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks, with modules or
+    functions that are not ``own`` (of other classes, or put in place of what these define) or with tensors other than those it was made with (``shapes``) is not
+    ``plain``."""
 
-    def __init__(self, model: nn.Module, shapes: dict, others: Sequence[tuple] = ()):
-        self.modules = list(model.modules())
+    def __init__(self, model: nn.Module, shapes: dict, own: Sequence[tuple], others: Sequence[tuple] = ()):
+        self.modules, self.own = list(model.modules()), own
         tensors = [(m._parameters, n, t) for m in self.modules for n, t in m._parameters.items()] + [e for e in others if torch.is_tensor(e[2])]
         self.tensors = [(*e, e[2].data_ptr()) for e in tensors if e[2] is not None]
         self.values = [(m._modules, n, c) for m in self.modules for n, c in m._modules.items()] + [e for e in others if not torch.is_tensor(e[2])]
         device = next(model.parameters()).device
         self.fits = shapes_of(model) == shapes and all(t.dtype == f32 and t.is_contiguous() and t.device == device for _, _, t, _ in self.tensors)
+
+    @staticmethod
+    def made_of(modules: Iterable[nn.Module], own: Sequence[tuple]) -> bool:
+        classes, names = {c for c, _, _ in own} | {nn.ModuleList, nn.ModuleDict}, {n for _, n, _ in own}
+        return all(type(m) in classes and names.isdisjoint(m.__dict__) for m in modules) and all(vars(c).get(n) is f for c, n, f in own)
 
     def current(self) -> bool:
         try:
@@ -65,7 +76,7 @@ class Held:
             return False
 
     def plain(self) -> bool:
-        return self.fits and not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in self.modules)
+        return self.fits and self.made_of(self.modules, self.own) and not any(m._forward_hooks or m._forward_pre_hooks for m in self.modules)
 
 
 def table_batch(batch, device) -> bool:

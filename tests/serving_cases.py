@@ -656,3 +656,59 @@ def case_registry():
     assert registry.resolve({"architecture": "Kozipel"})[1].__name__ == "KozipelForCausalLM"
     with pytest.raises(ValueError):
         registry.architecture({"architecture": "nothing"})
+
+
+# what is done to a float32 model whose steps run by a table of addresses
+MODULES_CHANGED = ["subclass", "class", "instance", "wrapped"]
+
+
+def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
+    """A float32 step's table of addresses stands in for modules: whatever is done to them, the step's logits are those of the step run sublayer by sublayer (as it is
+    with a trace).  ``cases``: the model family's cases."""
+    from aria_amd.serving import StepBatch
+
+    cfg = cases.CONFIGS["mixed"]
+    w, toks = cases.checkpoint(cfg, seed=3), cases.tokens(cfg, 12, seed=1)
+    models = [cases.build(cfg, w, dev, torch.float32) for _ in range(2)]
+
+    def layers(m):
+        return list(m.weights.values()) if hasattr(m, "weights") else list(m.layers)
+
+    plain = type(layers(models[0])[0].mixer).forward
+
+    def twice(self, *a):
+        y = plain(self, *a)
+        return dict(y, y=2.0 * y["y"]) if isinstance(y, dict) else 2.0 * y
+
+    class Wrap(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, h):
+            return {k: 2.0 * v if k == "y" else v for k, v in self.inner(h).items()}
+
+    def change(m):
+        mixer = layers(m)[0].mixer
+        if what == "subclass":
+            mixer.__class__ = type("Twice", (type(mixer),), dict(forward=twice))
+        elif what == "class":
+            monkeypatch.setattr(type(mixer), "forward", twice)
+        elif what == "instance":
+            mixer.forward = lambda *a: twice(mixer, *a)
+        elif what == "wrapped":
+            owner = next(L for L in layers(m) if L.mlp is not None)
+            owner.mlp = Wrap(owner.mlp)
+
+    def both(a, b):
+        got, want = (m.step(StepBatch.build([toks[a:b]], [0], [a], None, dev), t) for m, t in zip(models, (None, [])))
+        assert torch.equal(got.cpu(), want.cpu())
+        return got.cpu()
+
+    for m in models:
+        m.setup_caches(1, 12)
+    before = both(0, 5)
+    for m in models:
+        change(m)
+    assert not torch.equal(both(0, 5), before)
+    both(5, 8), both(8, 9)

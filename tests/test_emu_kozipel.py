@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from tests import kozipel_cases as C
+from tests import serving_cases as S
 
 bf16, f32 = torch.bfloat16, torch.float32
 DEV = "cpu"
@@ -105,3 +106,8 @@ def test_bad_inputs():
 @pytest.mark.parametrize("name", ["mixed", "odd"])
 def test_float32_step_as_one_call(monkeypatch, name):
     C.case_float32_step_as_one_call(DEV, monkeypatch, name)
+
+
+@pytest.mark.parametrize("what", S.MODULES_CHANGED)
+def test_float32_step_asks_the_modules(monkeypatch, what):
+    S.case_float32_step_asks_the_modules(DEV, monkeypatch, C, what)

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from tests import kozipel_cases as C
+from tests import serving_cases as S
 
 bf16, f32 = torch.bfloat16, torch.float32
 pytestmark = pytest.mark.gpu
@@ -163,3 +164,8 @@ def test_bad_inputs():
 @pytest.mark.parametrize("name", ["mixed", "odd"])
 def test_float32_step_as_one_call(monkeypatch, name):
     C.case_float32_step_as_one_call(DEV, monkeypatch, name)
+
+
+@pytest.mark.parametrize("what", S.MODULES_CHANGED)
+def test_float32_step_asks_the_modules(monkeypatch, what):
+    S.case_float32_step_asks_the_modules(DEV, monkeypatch, C, what)

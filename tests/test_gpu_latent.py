@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from tests import latent_cases as C
+from tests import serving_cases as S
 
 bf16, f32 = torch.bfloat16, torch.float32
 pytestmark = pytest.mark.gpu
@@ -151,3 +152,8 @@ def test_float32_step_as_one_call(monkeypatch, name):
 @pytest.mark.parametrize("runs", [[(0, 0, 41), (2, 3, 30)], [(0, 20, 3), (1, 0, 1), (0, 5, 2), (2, 60, 35)], [(1, 70, 1), (0, 4, 1), (2, 0, 1)]])
 def test_latent_attention_f32(H, R, dr, dv, runs):
     C.case_latent_attention_f32(DEV, H, R, dr, dv, runs)
+
+
+@pytest.mark.parametrize("what", S.MODULES_CHANGED)
+def test_float32_step_asks_the_modules(monkeypatch, what):
+    S.case_float32_step_asks_the_modules(DEV, monkeypatch, C, what)
