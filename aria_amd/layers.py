@@ -52,7 +52,7 @@ def functions_of(*classes: type) -> List[tuple]:
 
 class Held:
     """What a float32 step's table of addresses was made from: every parameter, cache and constant of a model, compared before each step that runs by the table.
-    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks, with modules or
+    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks (its own or those of all modules), with modules or
     functions that are not ``own`` (of other classes, or put in place of what these define) or with tensors other than those it was made with (``shapes``) is not
     ``plain``."""
 
@@ -76,6 +76,9 @@ class Held:
             return False
 
     def plain(self) -> bool:
+        everywhere = nn.modules.module
+        if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks:
+            return False
         return self.fits and self.made_of(self.modules, self.own) and not any(m._forward_hooks or m._forward_pre_hooks for m in self.modules)
 
 

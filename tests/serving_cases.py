@@ -659,7 +659,7 @@ def case_registry():
 
 
 # what is done to a float32 model whose steps run by a table of addresses
-MODULES_CHANGED = ["subclass", "class", "instance", "wrapped"]
+MODULES_CHANGED = ["subclass", "class", "instance", "wrapped", "global hook", "global pre hook"]
 
 
 def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
@@ -676,9 +676,11 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
 
     plain = type(layers(models[0])[0].mixer).forward
 
-    def twice(self, *a):
-        y = plain(self, *a)
+    def twice_of(y):
         return dict(y, y=2.0 * y["y"]) if isinstance(y, dict) else 2.0 * y
+
+    def twice(self, *a):
+        return twice_of(plain(self, *a))
 
     class Wrap(torch.nn.Module):
         def __init__(self, inner):
@@ -686,7 +688,7 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
             self.inner = inner
 
         def forward(self, h):
-            return {k: 2.0 * v if k == "y" else v for k, v in self.inner(h).items()}
+            return twice_of(self.inner(h))
 
     def change(m):
         mixer = layers(m)[0].mixer
@@ -700,6 +702,10 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
             owner = next(L for L in layers(m) if L.mlp is not None)
             owner.mlp = Wrap(owner.mlp)
 
+    def hook(mod, args, out=None):   # (everything that a first mixer returns, or is given, doubled)
+        if any(mod is layers(m)[0].mixer for m in models):
+            return twice_of(out) if out is not None else (2.0 * args[0],) + tuple(args[1:])
+
     def both(a, b):
         got, want = (m.step(StepBatch.build([toks[a:b]], [0], [a], None, dev), t) for m, t in zip(models, (None, [])))
         assert torch.equal(got.cpu(), want.cpu())
@@ -710,5 +716,14 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
     before = both(0, 5)
     for m in models:
         change(m)
-    assert not torch.equal(both(0, 5), before)
-    both(5, 8), both(8, 9)
+    everywhere, handle = torch.nn.modules.module, None
+    if what == "global hook":
+        handle = everywhere.register_module_forward_hook(hook)
+    elif what == "global pre hook":
+        handle = everywhere.register_module_forward_pre_hook(hook)
+    try:
+        assert not torch.equal(both(0, 5), before)
+        both(5, 8), both(8, 9)
+    finally:
+        if handle is not None:
+            handle.remove()
