@@ -150,6 +150,12 @@ class DuguzenForCausalLM(nn.Module):
         """the norm that reads the stream after layer run i"""
         return self.layer(i + 1).norm1 if i + 1 < len(self.config.layers) else self.final
 
+    def _table_step(self) -> bool:
+        """aria_latent_step_f32 takes the model as it is"""
+        own = [self.layer(i) for i in range(len(self.config.layers))] if Held.made_of(self.modules(), _OWN) else []
+        return (bool(own) and all(L.mixer.table_step and (L.mlp is None or L.mlp.table_step) for L in own)
+                and all(c.rows.shape == self.caches[0].rows.shape[:2] + c.rows.shape[2:] for c in self.caches))
+
     @torch.no_grad()
     def step(self, batch, trace: Optional[list] = None) -> torch.Tensor:
         """Run a ``serving.StepBatch``; -> float32 logits [wanted rows, vocab].  ``trace``: receives the residual stream after every layer run."""
@@ -165,8 +171,8 @@ class DuguzenForCausalLM(nn.Module):
             return logits if batch.every_row else logits[batch.wanted.long()]
         if self.dtype == f32 and trace is None and table_batch(batch, self.device):
             if self._decode is None or not self._decode.held.current():
-                self._decode = _DecodeTables(self) if Held.made_of(self.modules(), _OWN) else None
-            if self._decode is not None and self._decode.held.plain() and all(c.rows.shape == self.caches[0].rows.shape[:2] + c.rows.shape[2:] for c in self.caches):
+                self._decode = _DecodeTables(self) if self._table_step() else None
+            if self._decode is not None and self._decode.held.plain():
                 return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.dyt_stream(x, None, self.layer(0).norm1.params(), ids=batch.ids, table=self.embed)
@@ -211,9 +217,7 @@ class _DecodeTables:
         self.stack = hip.LatentStack(n, model.width, model.head.shape[0], model.layer(0).norm1.params(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows = model.device, model.head.shape[0]
         if model.dtype == f32:
-            self.held = Held(model, model._shapes, _OWN, [(m.__dict__, "alpha", m.alpha) for m in model.modules() if isinstance(m, DynamicTanh)]
-                             + [(c.__dict__, "rows", c.rows) for c in model.caches] + [(model.ropes, i, t) for i, t in enumerate(model.ropes)]
-                             + [(model.caches, i, c) for i, c in enumerate(model.caches)])
+            self.held = Held(model, model._shapes, _OWN)
 
     def run_f32(self, batch) -> torch.Tensor:
         T, W, lib = batch.ids.numel(), batch.wanted.numel() if batch.wanted is not None else -1, hip.get_lib()

@@ -159,6 +159,11 @@ class KozipelForCausalLM(nn.Module):
         runs = self.config.runs
         return self.layers[runs[i + 1].layer].norm1 if i + 1 < len(runs) else self.final
 
+    def _table_step(self) -> bool:
+        """aria_mix_step_f32 takes the model as it is"""
+        return Held.made_of(self.modules(), _OWN) and all(L.mixer.table_step and L.mixer.parts[-1].eps == self.config.eps and (L.mlp is None or L.mlp.table_step)
+                                                          for L in self.layers)
+
     @torch.no_grad()
     def step(self, batch, trace: Optional[list] = None) -> torch.Tensor:
         """Run a ``serving.StepBatch``; -> float32 logits [wanted rows, vocab].  ``trace``: receives the residual stream after every layer run."""
@@ -175,8 +180,8 @@ class KozipelForCausalLM(nn.Module):
             return logits if batch.every_row else logits[batch.wanted.long()]
         if self.dtype == f32 and trace is None and batch.seq is not None and table_batch(batch, self.device):
             if self._decode is None or not self._decode.held.current():
-                self._decode = _DecodeTables(self) if Held.made_of(self.modules(), _OWN) and all(L.mixer.table_step for L in self.layers) else None
-            if self._decode is not None and self._decode.held.plain() and all(L.mixer.table_step and L.mixer.parts[-1].eps == c.eps for L in self.layers):
+                self._decode = _DecodeTables(self) if self._table_step() else None
+            if self._decode is not None and self._decode.held.plain():
                 return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.rms_stream(x, c.width, c.eps, self.layers[c.runs[0].layer].norm1.weight, ids=batch.ids, table=self.embed, scale=c.embedding_scale)
@@ -218,9 +223,7 @@ class _DecodeTables:
                                   model.layers[c.runs[0].layer].norm1.weight.data_ptr(), model.embed.data_ptr(), model.head.data_ptr())
         self.device, self.rows, self.vocab = model.device, model.head.shape[0], model.vocab
         if model.dtype == f32:
-            flat = [c for run in model.caches for c in run]
-            self.held = Held(model, model._shapes, _OWN, [(c.__dict__, "rows", c.rows) for c in flat] + [(run, i, c) for run in model.caches for i, c in enumerate(run)]
-                             + [(model.caches, i, run) for i, run in enumerate(model.caches)])
+            self.held = Held(model, model._shapes, _OWN)
 
     def run_f32(self, batch) -> torch.Tensor:
         T, W, lib = batch.ids.numel(), batch.wanted.numel() if batch.wanted is not None else -1, hip.get_lib()

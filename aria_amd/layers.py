@@ -51,35 +51,58 @@ def functions_of(*classes: type) -> List[tuple]:
 
 
 class Held:
-    """What a float32 step's table of addresses was made from: every parameter, cache and constant of a model, compared before each step that runs by the table.
-    ``others``: (container, key, value) of what is no parameter.  The table's step runs no module and checks no shape: a model with hooks (its own or those of all modules), with modules or
-    functions that are not ``own`` (of other classes, or put in place of what these define) or with tensors other than those it was made with (``shapes``) is not
-    ``plain``."""
+    """What a float32 step's table of addresses was made from, compared before each step that runs by the table: every tensor, constant and module of a model, what its
+    config and caches hold included.  The table's step runs no module and checks no shape: a model with hooks (its own or those of all modules), with modules
+    or functions that are not ``own`` (of other classes, or put in place of what these define) or with tensors other than those it was made with (``shapes``)
+    is not ``plain``."""
 
-    def __init__(self, model: nn.Module, shapes: dict, own: Sequence[tuple], others: Sequence[tuple] = ()):
-        self.modules, self.own = list(model.modules()), own
-        tensors = [(m._parameters, n, t) for m in self.modules for n, t in m._parameters.items()] + [e for e in others if torch.is_tensor(e[2])]
-        self.tensors = [(*e, e[2].data_ptr()) for e in tensors if e[2] is not None]
-        self.values = [(m._modules, n, c) for m in self.modules for n, c in m._modules.items()] + [e for e in others if not torch.is_tensor(e[2])]
+    def __init__(self, model: nn.Module, shapes: dict, own: Sequence[tuple]):
+        self.modules, self.own, self.values, self.sizes, tensors, seen = [(m, type(m)) for m in model.modules()], own, [], [], [], set()
+
+        def look(container, items, of_module):
+            if id(container) in seen:
+                return
+            seen.add(id(container))
+            self.sizes.append((container, len(container)))
+            for k, v in items:
+                if torch.is_tensor(v):
+                    tensors.append((container, k, v))
+                    continue
+                self.values.append((container, k, v))
+                if isinstance(v, list):
+                    look(v, enumerate(v), False)
+                elif isinstance(v, dict) and of_module:          # (a module's sizes and offsets; what a config's entries were read from is not read again)
+                    look(v, v.items(), False)
+                elif type(v).__module__.startswith(__package__ + ".") and not isinstance(v, nn.Module):   # configs and caches
+                    look(v.__dict__, v.__dict__.items(), False)
+
+        for m, _ in self.modules:
+            look(m.__dict__, [(k, v) for k, v in m.__dict__.items() if k[0] != "_" and k != "training"], True)
+            look(m._parameters, m._parameters.items(), False)
+            look(m._modules, m._modules.items(), False)
+        self.tensors = [(*e, e[2].data_ptr(), e[2].shape) for e in tensors]
         device = next(model.parameters()).device
-        self.fits = shapes_of(model) == shapes and all(t.dtype == f32 and t.is_contiguous() and t.device == device for _, _, t, _ in self.tensors)
+        self.fits = shapes_of(model) == shapes and all(t.dtype == f32 and t.is_contiguous() and t.device == device for _, _, t in tensors)
 
     @staticmethod
     def made_of(modules: Iterable[nn.Module], own: Sequence[tuple]) -> bool:
         classes, names = {c for c, _, _ in own} | {nn.ModuleList, nn.ModuleDict}, {n for _, n, _ in own}
-        return all(type(m) in classes and names.isdisjoint(m.__dict__) for m in modules) and all(vars(c).get(n) is f for c, n, f in own)
+        return all(type(m) in classes and names.isdisjoint(m.__dict__) for m in modules) and all(c.__dict__.get(n) is f for c, n, f in own)
 
     def current(self) -> bool:
         try:
-            return all(d[n] is t and t.data_ptr() == p for d, n, t, p in self.tensors) and all(d[n] is v for d, n, v in self.values)
+            return (all(len(d) == n for d, n in self.sizes) and all(d[n] is v for d, n, v in self.values)
+                    and all(d[n] is t and t.data_ptr() == p and t.shape == s and t.is_contiguous() for d, n, t, p, s in self.tensors))
         except (KeyError, IndexError):
             return False
 
     def plain(self) -> bool:
+        """(a function put on a module itself is one entry more: not ``current``, and then not ``made_of`` its own)"""
         everywhere = nn.modules.module
         if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks:
             return False
-        return self.fits and self.made_of(self.modules, self.own) and not any(m._forward_hooks or m._forward_pre_hooks for m in self.modules)
+        return (self.fits and all(type(m) is c and not m._forward_hooks and not m._forward_pre_hooks for m, c in self.modules)
+                and all(c.__dict__.get(n) is f for c, n, f in self.own))
 
 
 def table_batch(batch, device) -> bool:
@@ -158,6 +181,11 @@ class LatentAttention(nn.Module):
     def shape(self, S_cap: int) -> hip.LatentShape:
         return hip.LatentShape(S_cap=S_cap, **self.geometry)
 
+    @property
+    def table_step(self) -> bool:
+        """aria_latent_step_f32 takes the mixer"""
+        return self.dtype == f32 and not self.flash
+
     def new_cache(self, slots: int, max_len: int, device) -> LatentCache:
         return LatentCache(slots, max_len, self.geometry["cw"], self.dtype, device)
 
@@ -184,6 +212,11 @@ class SquaredReluFeedForward(nn.Module):
         super().__init__()
         self.ff = up8(up.shape[0])
         self.up, self.down = _frozen(padded(up, self.ff, width), dtype), _frozen(padded(down, width, self.ff), dtype)
+
+    @property
+    def table_step(self) -> bool:
+        """a table's sizes are the weights' own"""
+        return self.up.shape[0] == self.ff == self.down.shape[1]
 
     def forward(self, h: torch.Tensor):
         return dict(y=ops.linear_any(ops.linear_any(h, self.up, relu_squared=True), self.down))
@@ -214,6 +247,11 @@ class GroupLimitedMixture(nn.Module):
     @property
     def up(self):
         return self.gate_up[1]
+
+    @property
+    def table_step(self) -> bool:
+        """a table's sizes are the weights' own"""
+        return self.gate_up.shape[1:3] == (self.n_experts, self.ff) and self.correction.numel() == self.n_experts
 
     def forward(self, h: torch.Tensor):
         logits = ops.linear_any(h, self.router, out_dtype=f32)
@@ -392,11 +430,13 @@ class MixerGroup(nn.Module):
     def table_step(self) -> bool:
         """aria_mix_step_f32 takes the group: the same mixers in float32"""
         lin = self.parts[-1]
-        if self.w_in.dtype != f32 or not isinstance(lin, LinearAttention):
+        if self.w_in.dtype != f32 or not isinstance(lin, LinearAttention) or lin.chunked:
             return False
+        H, dv = lin.geometry["H"], lin.geometry["dv"]
         if len(self.parts) == 1:
-            return lin.norm_groups == 1 and not lin.silu_gate
-        return isinstance(self.parts[0], ChunkAttention) and lin.norm_groups == lin.geometry["H"] and lin.norm.numel() == lin.geometry["dvp"] and lin.silu_gate
+            return lin.norm_groups == 1 and lin.norm_n == H * dv and not lin.silu_gate
+        return (isinstance(self.parts[0], ChunkAttention) and not self.parts[0].flash and lin.norm_groups == H and lin.norm_n == dv
+                and lin.norm.numel() == lin.geometry["dvp"] and lin.silu_gate)
 
     def fill_table(self, t: hip.MixLayer, caches: list) -> None:
         lin = self.parts[-1]
@@ -422,6 +462,11 @@ class ReluGatedFeedForward(nn.Module):
         self.ff = up8(up.shape[0])
         self.gate_up = _frozen(torch.cat([padded(t, self.ff, width) for t in (gate, up)]), dtype)
         self.down = _frozen(padded(down, width, self.ff), dtype)
+
+    @property
+    def table_step(self) -> bool:
+        """a table's sizes are the weights' own"""
+        return self.gate_up.shape[0] == 2 * self.ff and self.down.shape[1] == self.ff
 
     def forward(self, h: torch.Tensor) -> dict:
         return dict(y=ops.linear_any(ops.relu_glu(h, self.gate_up), self.down))

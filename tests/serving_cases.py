@@ -659,7 +659,7 @@ def case_registry():
 
 
 # what is done to a float32 model whose steps run by a table of addresses
-MODULES_CHANGED = ["subclass", "class", "instance", "wrapped", "global hook", "global pre hook"]
+MODULES_CHANGED = ["subclass", "class", "instance", "wrapped", "global hook", "global pre hook", "config", "runs", "geometry", "attribute", "weight view"]
 
 
 def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
@@ -701,6 +701,30 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
         elif what == "wrapped":
             owner = next(L for L in layers(m) if L.mlp is not None)
             owner.mlp = Wrap(owner.mlp)
+        elif what == "config":
+            for name in ("residual_mult", "embedding_scale", "logit_softcap"):   # (Duguzen's has none of them: a layer run less)
+                if hasattr(m.config, name):
+                    setattr(m.config, name, 0.25 * getattr(m.config, name))
+            if hasattr(m, "weights"):
+                m.config.layers.pop()
+        elif what == "runs":
+            if hasattr(m, "weights"):
+                m.caches[0], m.caches[1] = type(m.caches[0])(*m.caches[0].rows.shape, f32, dev), type(m.caches[0])(*m.caches[1].rows.shape, f32, dev)
+                m.ropes[0] = m.ropes[0].flip(1).contiguous()
+            else:
+                m.config.runs[3].again = not m.config.runs[3].again
+        elif what == "geometry":
+            for part in getattr(mixer, "parts", [mixer]):
+                for name in ("scale", "q_scale"):
+                    if name in part.geometry:
+                        part.geometry[name] = 0.25 * part.geometry[name]
+        elif what == "attribute":
+            for part in m.modules():
+                for name, new in (("top", lambda k: 1), ("norm_n", lambda n: n - 1), ("eps", lambda e: 0.5), ("ff", lambda n: n + 8)):
+                    if name in part.__dict__:
+                        setattr(part, name, new(getattr(part, name)))
+        elif what == "weight view":
+            m.head.data = m.head.data.flip(0)
 
     def hook(mod, args, out=None):   # (everything that a first mixer returns, or is given, doubled)
         if any(mod is layers(m)[0].mixer for m in models):
