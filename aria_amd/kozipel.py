@@ -135,6 +135,9 @@ class KozipelForCausalLM(nn.Module):
         self._decode = None
         return super()._apply(fn, *a, **k)
 
+    def __getstate__(self):              # (nor are they a copy's)
+        return dict(self.__dict__, _decode=None)
+
     @property
     def device(self):
         return self.head.device

@@ -751,3 +751,28 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
     finally:
         if handle is not None:
             handle.remove()
+
+
+def case_stepped_model_copied(dev, cases, dtype):
+    """A model that has made a step's tables is copied and pickled like any other; the copy's steps read its own weights and caches."""
+    import copy
+    import pickle
+
+    from aria_amd.serving import StepBatch
+
+    cfg = cases.CONFIGS["mixed"]
+    m = cases.build(cfg, cases.checkpoint(cfg, seed=3), dev, dtype)
+    toks = cases.tokens(cfg, 12, seed=1)
+    m.setup_caches(1, 12)
+
+    def steps(m):
+        return [m.step(StepBatch.build([toks[a:b]], [0], [a], None, dev)).cpu() for a, b in ((0, 5), (5, 6))]
+
+    want = steps(m)
+    copies = copy.deepcopy(m), pickle.loads(pickle.dumps(m))
+    with torch.no_grad():
+        for t in m.parameters():
+            t.zero_()
+    assert not torch.equal(steps(m)[1], want[1])
+    for c in copies:
+        assert all(torch.equal(x, y) for x, y in zip(steps(c), want))

@@ -111,3 +111,8 @@ def test_float32_step_as_one_call(monkeypatch, name):
 @pytest.mark.parametrize("what", S.MODULES_CHANGED)
 def test_float32_step_asks_the_modules(monkeypatch, what):
     S.case_float32_step_asks_the_modules(DEV, monkeypatch, C, what)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_stepped_model_copied(dtype):
+    S.case_stepped_model_copied(DEV, C, dtype)
