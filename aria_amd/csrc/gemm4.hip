@@ -98,7 +98,7 @@ struct Shape4 {
 };
 
 // VER: what happens to the tile (the numbers of gemm3_kernel): 3 plain (bias, activation, accumulation, 32-bit results), 5 SwiGLU backward, 6 / 9 fused SwiGLU on two
-// weight tensors (9: gathered rows), 8 on [K, N] weights with gathered rows, 14 on one [gate | up] tensor, 13 relu gate, 7 / 10 rotations,
+// weight tensors (9: gathered rows), 8 on [K, N] weights with gathered rows, 14 on one [gate | up] tensor, 13 relu gate, 7 the interleaved rotation,
 // 11 plain, with the reduction's rows of A reached through an index (per-expert weight gradients)
 constexpr bool gathers(int ver) { return ver == 8 || ver == 9; }   // (11: gathered rows of the reduction)
 constexpr bool gated(int ver) { return ver == 6 || ver == 8 || ver == 9 || ver == 13 || ver == 14; }
@@ -123,21 +123,6 @@ __device__ __forceinline__ void finish_piece(const P& p, char* C, const char* pa
             st16(out + (long long)m * p.ldc + col, v);
         else if (unsigned(ps) < unsigned(p.cache_S))
             st16(static_cast<bf16_t*>(region == 1 ? p.kc : p.vc) + ((long long)seq * p.cache_S + ps) * p.ld_cache + col, v);
-        return;
-    }
-    if (VER == 10) {   // half-split rotation: the partner columns lie in the same parked row
-        if (n0 < 2 * p.rope_D) {
-            const int half = p.rope_hd >> 1, fcol = (n0 + cc) % p.rope_hd, ps = m % p.rope_S;
-            const bool second = fcol >= half;
-            const u32x4 pv = *reinterpret_cast<const u32x4*>(parked + (second ? cc - half : cc + half) * 2);
-            const u32x4 fc = ld16(p.rope_fc + (long long)ps * p.rope_hd + fcol), fs = ld16(p.rope_sn + (long long)ps * p.rope_hd + fcol);
-            const float sg = second ? 1.f : -1.f;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                v[q] = pack2bf(rbf(bflo(v[q]) * bflo(fc[q])) + rbf(sg * bflo(pv[q]) * bflo(fs[q])),
-                               rbf(bfhi(v[q]) * bfhi(fc[q])) + rbf(sg * bfhi(pv[q]) * bfhi(fs[q])));
-        }
-        st16(out + (long long)m * p.ldc + n0 + cc, v);
         return;
     }
     if (VER == 5) {   // v = d_act: gate and up of the same elements give their gradients
@@ -574,7 +559,7 @@ long long aria_gemm4_workspace_bytes(long long M, long long N, long long K) {
 
 Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes) {
     Gemm4Plan none, plan;
-    if (p.ext_k || (a_oc && !b_oc) || p.N < 8 || (a_oc && p.M < 8)) return none;
+    if (p.ext_k || p.rope_sn || (a_oc && !b_oc) || p.N < 8 || (a_oc && p.M < 8)) return none;   // (p.rope_sn: the entry takes whole rounds of 256 x 256 tiles only)
     const bool plain = !p.glu && !p.dglu && !p.rope_fc;
     if (const char* force = std::getenv("ARIA_GEMM_FORCE")) {   // "4": tiles of 128 x 256, "46": the wide ones where there is such a form
         if (force[0] != '4') return none;
@@ -636,7 +621,7 @@ int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, f
     if (plan.form == 2)
         return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
 #define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
-    if (p.rope_fc) return p.rope_sn ? ARIA_G4(false, 10) : ARIA_G4(false, 7);
+    if (p.rope_fc) return ARIA_G4(false, 7);
     if (p.glu == 2) return ARIA_G4(false, 13);
     if (p.glu && p.gather_rows) return p.glu_up_rows > 0 ? ARIA_G4(false, 9) : ARIA_G4(true, 8);
     if (p.glu && p.glu_up_rows > 0) return ARIA_G4(false, 6);
