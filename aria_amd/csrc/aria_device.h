@@ -295,7 +295,7 @@ __device__ __forceinline__ f32x4 mfma16(s16x8 a, s16x8 b, f32x4 c) {
 // low 32 bits of the product of two values below 2^24 (v_mul_u32_u24: full rate; v_mul_lo_u32 is quarter rate)
 __device__ __forceinline__ uint32_t mul24(uint32_t a, uint32_t b) {
 #ifdef ARIA_EMU
-    return a * b;
+    return (a & 0xffffffu) * (b & 0xffffffu);
 #else
     return __umul24(a, b);
 #endif

@@ -339,13 +339,14 @@ bool use_v2(long long tiles256) {
     return tiles256 >= 192;
 }
 
-// v3 (LDS-DMA staged, phase-scheduled 256x256 tile, gemm3.hip): the operand byte offsets must fit 32 bits.
-// ARIA_GEMM_FORCE=3 pins it where eligible.
-bool fits_dma(long long K, long long bytesA, long long bytesB, long long extentA, long long extentB) {
-    return K >= 64 && bytesA < (1ll << 32) && bytesB < (1ll << 32) && extentA >= 8 && extentB >= 8;
+// The LDS-DMA kernels (gemm3.hip, gemm4.hip): operand byte offsets in 32 bits, made by 24-bit multiplies of a row's number and its bytes.
+// ARIA_GEMM_FORCE=3 pins v3 (the phase-scheduled 256x256 tile) where eligible.
+bool fits_dma(long long K, long long lda, long long ldb, long long bytesA, long long bytesB, long long extentA, long long extentB) {
+    constexpr long long B24 = 1ll << 24, B32 = 1ll << 32;
+    return K >= 64 && 2 * lda < B24 && 2 * ldb < B24 && bytesA < B32 && bytesB < B32 && extentA >= 8 && extentB >= 8 && extentA < B24 && extentB < B24;
 }
-bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB, long long extentA, long long extentB, long long least = 192) {
-    if (!fits_dma(K, bytesA, bytesB, extentA, extentB)) return false;
+bool use_v3(long long tiles256, long long K, long long lda, long long ldb, long long bytesA, long long bytesB, long long extentA, long long extentB, long long least = 192) {
+    if (!fits_dma(K, lda, ldb, bytesA, bytesB, extentA, extentB)) return false;
     const char* force = std::getenv("ARIA_GEMM_FORCE");
     if (force) return force[0] == '3';
     return tiles256 >= least;
@@ -356,12 +357,11 @@ bool use_v3(long long tiles256, long long K, long long bytesA, long long bytesB,
 // Rows by expert: where they fill a third of a tile and more.  128 x 128 / 256 x 256, 150 .. 191 tiles: 64 experts of 2560 x 1664: 60 rows each on average 132 / 146, 72 134 /
 // 140; 3328 x 2560: 48 rows 248 / 277; 32 experts of 3328 x 2560: 88 rows 173 / 145; 64 of 1536 x 1024: 96 rows 76 / 54; 16 of 2560 x 1664: 240 rows 83 / 47.
 constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150, V3_FEW_ROWS = 84;
-// the LDS-DMA kernels: the four-wave tiles where their plan takes the product, the 256 x 256 ones elsewhere (rows: see aria_plan_gemm4)
-int launch_large(const GemmParams& p, int a_oc, int b_oc, int ntm, void* stream, void* workspace = nullptr, long long workspace_bytes = 0, long long rows = -1) {
-    const int split3 = p.mode == 0 && workspace ? aria_gemm3_split(p.M, p.N, p.K) : 1;
-    const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, rows, split3, workspace ? workspace_bytes : 0);
-    if (plan.form) return aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
-    return aria_launch_gemm3(p, a_oc, b_oc, ntm, stream, workspace, workspace_bytes);
+// the fused launches (none splits its reduction): the four-wave tiles where their plan takes the product, the 256 x 256 ones elsewhere (rows: see aria_plan_gemm4)
+int launch_large(const GemmParams& p, int a_oc, int b_oc, int ntm, void* stream, long long rows = -1) {
+    const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, rows, 1, 0);
+    if (plan.form) return aria_launch_gemm4(p, a_oc, b_oc, plan, nullptr, stream);
+    return aria_launch_gemm3(p, a_oc, b_oc, ntm, stream);
 }
 long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
@@ -441,14 +441,12 @@ static int dense_product(const void* A, const void* B, void* C, const void* bias
     // with a workspace the partly filled last round of tiles is split along K (gemm3.hip), so small outputs fill the chip too
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
-    const bool strides = 2 * lda < (1ll << 24) && 2 * ldb < (1ll << 24);
-    if (four_waves && (!a_oc || b_oc) && strides && fits_dma(K, bytesA, bytesB, M, N)) {
+    if (four_waves && (!a_oc || b_oc) && fits_dma(K, lda, ldb, bytesA, bytesB, M, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0);
         if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
     }
-    if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
-        return g_last_variant = 3, four_waves ? launch_large(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes)
-                                              : aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
+    if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, lda, ldb, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
+        return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
 }
@@ -494,13 +492,13 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const int gmask = gsel ? std::atoi(gsel) : GROUPED_V3_DEFAULT;
     const char* gforce = std::getenv("ARIA_GEMM_FORCE");
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
-    if (fits_dma(K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N) && 2 * lda < (1ll << 24) && 2 * ldb < (1ll << 24)) {
+    if (fits_dma(K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, 0, b_oc, -1, 1, 0);
         if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 0, b_oc, plan, nullptr, stream);
     }
-    if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
+    if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
                       v3_least(K, M_total >= V3_FEW_ROWS * E ? V3_FEW_TILES_GROUPED : 192)))
-        return g_last_variant = 3, launch_large(p, 0, b_oc, int(M_total / 256 + E), stream);
+        return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc, int(M_total / 256 + E), stream);
     if (use_v2((M_total / 256 + 1) * ((N + 255) / 256))) return g_last_variant = 2, aria_launch_gemm2(p, 0, b_oc, int(M_total / 256 + E), 1, stream);
     return g_last_variant = 1, launch_gemm(p, 0, b_oc, p.ntn * max_tm, 1, stream);
 }
@@ -512,7 +510,7 @@ static int glu_check(const void* A, const void* B, const void* H, const void* AC
     if (!aligned16(A) || !aligned16(B) || !aligned16(ACT) || (H && !aligned16(H)) || (lda & 7) || (ldb & 7) || (K & 7) || (ldact & 7) ||
         (H && (ldh & 7)))
         return ARIA_ERR_ALIGN;
-    if ((N2 & 1) || ((N2 / 2) % 128) || K < 64 || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24)) return ARIA_ERR_UNSUPPORTED;
+    if ((N2 & 1) || ((N2 / 2) % 128) || K < 64 || M >= (1ll << 24) || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24)) return ARIA_ERR_UNSUPPORTED;
     return ARIA_OK;
 }
 
@@ -781,7 +779,7 @@ int aria_gemm_qkv_rope_hf_bf16(const void* X, const void* Wqkv, void* QKV, const
     if (!X || !Wqkv || !QKV || !cos || !sin || M < 0 || D <= 0 || K <= 0 || hd <= 0 || S <= 0) return ARIA_ERR_INVALID;
     if (!aligned16(X) || !aligned16(Wqkv) || !aligned16(QKV) || !aligned16(cos) || !aligned16(sin) || (ldx & 7) || (ldw & 7) || (ldc & 7)) return ARIA_ERR_ALIGN;
     if ((D % 256) || (256 % hd) || (hd & 15) || (K % 64) || K < 64 || 2 * M * ldx >= (1ll << 32) || 2 * 3 * D * ldw >= (1ll << 32) || 2 * ldx >= (1ll << 24) ||
-        2 * ldw >= (1ll << 24) || !use_v3(((M + 255) / 256) * (3 * D / 256), K, 2 * M * ldx, 2 * 3 * D * ldw, M, 3 * D))
+        2 * ldw >= (1ll << 24) || !use_v3(((M + 255) / 256) * (3 * D / 256), K, ldx, ldw, 2 * M * ldx, 2 * 3 * D * ldw, M, 3 * D))
         return ARIA_ERR_UNSUPPORTED;
     if (M == 0) return ARIA_OK;
     GemmParams p{};
@@ -794,7 +792,7 @@ int aria_gemm_qkv_rope_hf_bf16(const void* X, const void* Wqkv, void* QKV, const
     p.rope_fc = static_cast<const bf16_t*>(cos);
     p.rope_sn = static_cast<const bf16_t*>(sin);
     p.rope_hd = int(hd), p.rope_D = int(D), p.rope_S = int(S);
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // shared validation of the fused input-gradient + SwiGLU-backward entries (gemm3_kernel<.., .., 5>)
@@ -802,7 +800,7 @@ static int dglu_check(const void* A, const void* B, const void* H, const void* D
                       int64_t ldh, int64_t lddh) {
     if (!A || !B || !H || !DH || M < 0 || I <= 0 || K <= 0) return ARIA_ERR_INVALID;
     if (!aligned16(A) || !aligned16(B) || !aligned16(H) || !aligned16(DH) || (lda & 7) || (ldb & 7) || (ldh & 7) || (lddh & 7)) return ARIA_ERR_ALIGN;
-    if ((I % 128) || (K % 64) || K < 64 || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24)) return ARIA_ERR_UNSUPPORTED;
+    if ((I % 128) || (K % 64) || K < 64 || M >= (1ll << 24) || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24)) return ARIA_ERR_UNSUPPORTED;
     return ARIA_OK;
 }
 
@@ -873,8 +871,8 @@ int aria_grouped_gemm_wgrad_gather_sized_bf16(const void* X, const int32_t* rows
     if (!X || !rows || !dY) return ARIA_ERR_INVALID;
     if (!aligned16(X) || !aligned16(dY) || (ldx & 7) || (ldy & 7) || (K & 7) || (N & 7) || (reinterpret_cast<uintptr_t>(rows) & 3)) return ARIA_ERR_ALIGN;
     const char* force4 = std::getenv("ARIA_GEMM_FORCE");
-    if (T >= (1ll << 24) || 2 * ldx >= (1ll << 24) || 2 * T * ldx >= (1ll << 32) ||
-        !(use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, 0, 0, K, N) || (force4 && force4[0] == '4' && K >= 8 && N >= 8)))
+    if (T >= (1ll << 24) || 2 * ldx >= (1ll << 24) || 2 * ldy >= (1ll << 24) || 2 * T * ldx >= (1ll << 32) ||
+        !(use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, ldx, ldy, 0, 0, K, N) || (force4 && force4[0] == '4' && K >= 8 && N >= 8)))
         return ARIA_ERR_UNSUPPORTED;
     GemmParams p{};
     p.A = static_cast<const bf16_t*>(X);
@@ -890,7 +888,7 @@ int aria_grouped_gemm_wgrad_gather_sized_bf16(const void* X, const int32_t* rows
     p.accumulate = accumulate;
     p.gather_rows = rows;
     p.ntn = int((N + BN - 1) / BN);
-    return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream, nullptr, 0, 2 * ldy < (1ll << 24) ? M_total : -1);
+    return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream, M_total);
 }
 
 // ---- LoRA as a K-extension of the base GEMM (GemmParams::ext_k; aria/lora/layers.py:129-139, peft's Linear adapter): v3 only -- shapes the
@@ -920,9 +918,9 @@ int aria_gemm_lora_bf16(const void* A, const void* B, void* C, int64_t M, int64_
     const int rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, 0);
     if (rc != ARIA_OK) return rc;
     const long long t256 = ((M + 255) / 256) * ((N + 255) / 256);
-    if (!use_v3(t256, K, 2 * M * lda, 2 * (b_oc ? K * ldb : N * ldb), M, N) || 2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24))
+    if (!use_v3(t256, K, lda, ldb, 2 * M * lda, 2 * (b_oc ? K * ldb : N * ldb), M, N))
         return ARIA_ERR_UNSUPPORTED;
-    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
 }
 
 int aria_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb,
@@ -941,7 +939,7 @@ int aria_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT,
     p.glu = 1;
     rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, 0);
     if (rc != ARIA_OK) return rc;
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 int aria_grouped_gemm_lora_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total, int64_t N, int64_t K,
@@ -961,10 +959,9 @@ int aria_grouped_gemm_lora_bf16(const void* A, const void* B, void* C, const int
     p.ntn = int((N + BN - 1) / BN);
     const int rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, stride_eb);
     if (rc != ARIA_OK) return rc;
-    if (!use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N) ||
-        2 * lda >= (1ll << 24) || 2 * ldb >= (1ll << 24))
+    if (!use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N))
         return ARIA_ERR_UNSUPPORTED;
-    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, 0, b_oc ? 1 : 0, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, void* ACT, const int32_t* offsets, int64_t E, int64_t M_total,
@@ -989,7 +986,7 @@ int aria_grouped_gemm_swiglu_lora_bf16(const void* A, const void* B, void* H, vo
     p.glu = 1;
     rc = lora_ext(p, EA, EB, ext_k, ld_ea, ld_eb, stride_eb);
     if (rc != ARIA_OK) return rc;
-    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_wgrad_bf16(const void* A, const void* dY, void* dW, const int32_t* offsets, int64_t E, int64_t K,
@@ -1020,7 +1017,7 @@ int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, 
     p.accumulate = accumulate;
     p.ntn = int((N + BN - 1) / BN);
     const int ntm = int((K + BM - 1) / BM);
-    if (K >= 8 && N >= 8 && 2 * lda < (1ll << 24) && 2 * ldy < (1ll << 24)) {
+    if (fits_dma(64, lda, ldy, 0, 0, K, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, 1, 1, M_total, 1, 0);
         if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 1, 1, plan, nullptr, stream);
     }
@@ -1031,8 +1028,8 @@ int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, 
     const char* force3 = std::getenv("ARIA_GEMM_FORCE");
     // r02: with the wide epilogue v3 is level with v2 here too (in-bench 710.3 vs 714.6 ms/step); ARIA_GEMM_WGRAD_V3=0 goes back to v2
     const char* wg3 = std::getenv("ARIA_GEMM_WGRAD_V3");
-    if (((force3 && force3[0] == '3') || !(wg3 && wg3[0] == '0')) && !(force3 && (force3[0] == '1' || force3[0] == '2')) && use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, 0, 0, K, N))
-        return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream);
+    if (((force3 && force3[0] == '3') || !(wg3 && wg3[0] == '0')) && !(force3 && (force3[0] == '1' || force3[0] == '2')) && use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, lda, ldy, 0, 0, K, N))
+        return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
     if (use_v2(((K + 255) / 256) * ((N + 255) / 256) * E)) return g_last_variant = 2, aria_launch_gemm2(p, 1, 1, int((K + 255) / 256), int(E), stream);
     return g_last_variant = 1, launch_gemm(p, 1, 1, p.ntn * ntm, int(E), stream);
 }

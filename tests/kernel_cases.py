@@ -151,6 +151,27 @@ def case_gemm_forward_sums(dev, monkeypatch, M, N, K):
         assert torch.equal(x.cpu(), y.cpu())
 
 
+def case_gemm_long_rows(dev, monkeypatch, force):
+    """Rows 2^24 bytes and more apart are beyond the 24-bit multiplies of the LDS-DMA kernels' addresses: such products take others (weight gradients, by expert
+    too, whose rows are the reduction's).  The values between the rows are never touched."""
+    from aria_amd import ops
+
+    K, M, N, ld = 64, 72, 264, (1 << 23) + 8
+    a, b = rnd(K, M, seed=1), rnd(K, N, seed=2)
+    far = torch.empty(K * ld, dtype=bf16, device=dev)
+    monkeypatch.setenv("ARIA_GEMM_FORCE", force)
+    off = torch.tensor([0, 40, 64], dtype=torch.int32, device=dev)
+    for first in (True, False):
+        x, y = (torch.as_strided(far, (K, n), (ld, 1)) if (t is a) == first else torch.empty((K, n), dtype=bf16, device=dev) for t, n in ((a, M), (b, N)))
+        x.copy_(a), y.copy_(b)
+        close(ops.gemm(x, y, a_oc=True, b_oc=True, out_dtype=torch.float32), a.float().t() @ b.float(), 1e-4, 1e-3)
+        got = ops.grouped_gemm_wgrad(x, y, off, 2, out_dtype=torch.float32)
+        close(got, torch.stack([a[:40].float().t() @ b[:40].float(), a[40:].float().t() @ b[40:].float()]), 1e-4, 1e-3)
+        rows = torch.arange(K + 64, dtype=torch.int32, device=dev) % K
+        got = ops.grouped_gemm_wgrad_gather(x, rows[:K], y, off, 2, out_dtype=torch.float32)
+        assert got is None   # (the caller permutes)
+
+
 def case_gemm_workspace_kept(dev):
     """What is kept per stream is one buffer of a fixed size; a larger need is the call's own and leaves nothing behind."""
     from aria_amd import ops

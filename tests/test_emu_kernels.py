@@ -388,6 +388,11 @@ def test_gemm_four_waves_fused(dma_order, monkeypatch):
         C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
 
 
+@pytest.mark.parametrize("force", ["3", "4"])
+def test_gemm_long_rows(monkeypatch, force):
+    C.case_gemm_long_rows(DEV, monkeypatch, force)
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 1032, 1536), (40, 1032, 2048), (200, 1024, 2304)])
 def test_gemm_forward_sums(monkeypatch, M, N, K):
     C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K)

@@ -378,6 +378,11 @@ def test_gemm_four_waves_fused(monkeypatch):
         C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
 
 
+@pytest.mark.parametrize("force", ["3", "4"])
+def test_gemm_long_rows(monkeypatch, force):
+    C.case_gemm_long_rows(DEV, monkeypatch, force)
+
+
 @pytest.mark.parametrize("M,N,K", [(40, 1032, 1536), (777, 2560, 2560), (777, 2560, 3328), (777, 7680, 2560), (1868, 2560, 2560), (4500, 1536, 4096), (200, 2560, 6656)])
 def test_gemm_forward_sums(monkeypatch, M, N, K):
     C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K)
