@@ -492,7 +492,7 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const int gmask = gsel ? std::atoi(gsel) : GROUPED_V3_DEFAULT;
     const char* gforce = std::getenv("ARIA_GEMM_FORCE");
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
-    if (fits_dma(K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N)) {
+    if (gv3 && fits_dma(K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, 0, b_oc, -1, 1, 0);
         if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 0, b_oc, plan, nullptr, stream);
     }
@@ -1017,19 +1017,16 @@ int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, 
     p.accumulate = accumulate;
     p.ntn = int((N + BN - 1) / BN);
     const int ntm = int((K + BM - 1) / BM);
-    if (fits_dma(64, lda, ldy, 0, 0, K, N)) {
-        const Gemm4Plan plan = aria_plan_gemm4(p, 1, 1, M_total, 1, 0);
-        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 1, 1, plan, nullptr, stream);
-    }
     // (the reduction length is per expert and data dependent: 64 stands in for "long enough" in the eligibility test)
     // both operands are token-major (output-contiguous): their per-lane DMA offsets stay inside one 64-token tile, no 4 GiB limit
-    // Measured on MI355X (98304 routed rows, 64 experts): v3 749 TF/s vs v2 800-830 on these short (~24 K-tile) reductions with two
-    // transposed operands -- v3's longer prologue and its 24-read first phase do not pay here, so v2 stays the default.
-    const char* force3 = std::getenv("ARIA_GEMM_FORCE");
-    // r02: with the wide epilogue v3 is level with v2 here too (in-bench 710.3 vs 714.6 ms/step); ARIA_GEMM_WGRAD_V3=0 goes back to v2
+    // With the wide epilogue v3 is level with v2 here (in-bench 710.3 vs 714.6 ms/step).  ARIA_GEMM_WGRAD_V3=0 goes back to v2, whichever LDS-DMA kernel would run.
+    const char* force = std::getenv("ARIA_GEMM_FORCE");
     const char* wg3 = std::getenv("ARIA_GEMM_WGRAD_V3");
-    if (((force3 && force3[0] == '3') || !(wg3 && wg3[0] == '0')) && !(force3 && (force3[0] == '1' || force3[0] == '2')) && use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, lda, ldy, 0, 0, K, N))
-        return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
+    if (force || !(wg3 && wg3[0] == '0')) {
+        const Gemm4Plan plan = fits_dma(64, lda, ldy, 0, 0, K, N) ? aria_plan_gemm4(p, 1, 1, M_total, 1, 0) : Gemm4Plan{};
+        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 1, 1, plan, nullptr, stream);
+        if (use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, lda, ldy, 0, 0, K, N)) return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
+    }
     if (use_v2(((K + 255) / 256) * ((N + 255) / 256) * E)) return g_last_variant = 2, aria_launch_gemm2(p, 1, 1, int((K + 255) / 256), int(E), stream);
     return g_last_variant = 1, launch_gemm(p, 1, 1, p.ntn * ntm, int(E), stream);
 }

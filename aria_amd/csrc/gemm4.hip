@@ -610,7 +610,8 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
 
 int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream) {
     GemmParams q = p;
-    q.wide_store = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0 && (p.strideC & 7) == 0;
+    const char* wsd = std::getenv("ARIA_GEMM_WIDE_STORE");
+    q.wide_store = !(wsd && wsd[0] == '0') && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0 && (p.strideC & 7) == 0;
     q.order = 4 | (p.glu && p.mode == 1 ? 512 : 0);
     const int split = ws && plan.split > 1 ? plan.split : 1;
     float* slabs = split > 1 ? ws : nullptr;

@@ -172,6 +172,24 @@ def case_gemm_long_rows(dev, monkeypatch, force):
         assert got is None   # (the caller permutes)
 
 
+def case_grouped_gemm_switches(dev, monkeypatch):
+    """ARIA_GEMM_GROUPED_V3 (bit 0: [N, K] weights, bit 1: [K, N]) and ARIA_GEMM_WGRAD_V3=0 take a form off the LDS-DMA kernels, the four-wave tiles among them."""
+    from aria_amd import hip, ops
+
+    M, N, K, lib = 100, 512, 768, hip.get_lib().cdll
+    x, dy, off = rnd(M, K, seed=1).to(dev), rnd(M, N, seed=2).to(dev), torch.tensor([0, 44, M], dtype=torch.int32, device=dev)
+    forms = [lambda w=rnd(2, N, K, seed=3, scale=0.1).to(dev): ops.grouped_gemm(x, w, off, w_is_kn=False),
+             lambda w=rnd(2, K, N, seed=4, scale=0.1).to(dev): ops.grouped_gemm(x, w, off, w_is_kn=True), lambda: ops.grouped_gemm_wgrad(x, dy, off, 2)]
+    want = [f() for f in forms]
+    for name, value, on in ((None, None, (1, 1, 1)), ("ARIA_GEMM_GROUPED_V3", "2", (0, 1, 1)), ("ARIA_GEMM_GROUPED_V3", "1", (1, 0, 1)), ("ARIA_GEMM_WGRAD_V3", "0", (1, 1, 0))):
+        with monkeypatch.context() as mp:
+            if name:
+                mp.setenv(name, value)
+            for f, w, v3 in zip(forms, want, on):
+                close(f(), w, 1e-2, 1e-2)
+                assert (lib.aria_last_gemm_variant() == 3) == bool(v3), (name, value)
+
+
 def case_gemm_workspace_kept(dev):
     """What is kept per stream is one buffer of a fixed size; a larger need is the call's own and leaves nothing behind."""
     from aria_amd import ops

@@ -388,6 +388,10 @@ def test_gemm_four_waves_fused(dma_order, monkeypatch):
         C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
 
 
+def test_grouped_gemm_switches(monkeypatch):
+    C.case_grouped_gemm_switches(DEV, monkeypatch)
+
+
 @pytest.mark.parametrize("force", ["3", "4"])
 def test_gemm_long_rows(monkeypatch, force):
     C.case_gemm_long_rows(DEV, monkeypatch, force)
