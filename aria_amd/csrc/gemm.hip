@@ -357,11 +357,15 @@ bool use_v3(long long tiles256, long long K, long long lda, long long ldb, long 
 // Rows by expert: where they fill a third of a tile and more.  128 x 128 / 256 x 256, 150 .. 191 tiles: 64 experts of 2560 x 1664: 60 rows each on average 132 / 146, 72 134 /
 // 140; 3328 x 2560: 48 rows 248 / 277; 32 experts of 3328 x 2560: 88 rows 173 / 145; 64 of 1536 x 1024: 96 rows 76 / 54; 16 of 2560 x 1664: 240 rows 83 / 47.
 constexpr long long V3_FEW_TILES = 80, V3_FEW_TILES_GROUPED = 150, V3_FEW_ROWS = 84;
+int launch4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, void* workspace, void* stream) {
+    g_last_variant = 3 | plan.form << 8 | plan.split << 12;
+    return aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
+}
 // the fused launches (none splits its reduction): the four-wave tiles where their plan takes the product, the 256 x 256 ones elsewhere (rows: see aria_plan_gemm4)
 int launch_large(const GemmParams& p, int a_oc, int b_oc, int ntm, void* stream, long long rows = -1) {
     const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, rows, 1, 0);
-    if (plan.form) return aria_launch_gemm4(p, a_oc, b_oc, plan, nullptr, stream);
-    return aria_launch_gemm3(p, a_oc, b_oc, ntm, stream);
+    if (plan.form) return launch4(p, a_oc, b_oc, plan, nullptr, stream);
+    return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, ntm, stream);
 }
 long long v3_least(long long K, long long few) { return K >= 512 ? few : 192; }
 
@@ -385,7 +389,9 @@ int aria_expert_pair_tiles(const void* X, const int32_t* rows, int64_t T, const 
 
 extern "C" {
 
-int aria_last_gemm_variant(void) { return g_last_variant; }
+int aria_last_gemm_variant(void) { return g_last_variant & 255; }
+
+int aria_last_gemm_tiles(void) { return g_last_variant >> 8; }
 
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc) {
     if (M <= 0 || N <= 0 || (a_oc && !b_oc)) return 0;
@@ -404,9 +410,9 @@ int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, i
                               workspace_bytes, stream);
 }
 
-static int dense_product(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
+int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                        int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
-                       int64_t workspace_bytes, void* stream, bool four_waves) {
+                       int64_t workspace_bytes, void* stream) {
     if (act != ARIA_ACT_NONE && act != ARIA_ACT_GELU_TANH && act != ARIA_ACT_RELU2) return ARIA_ERR_UNSUPPORTED;
     if (act == ARIA_ACT_RELU2 && (a_oc || b_oc)) return ARIA_ERR_UNSUPPORTED;   // (built for the forward form only)
     if (!A || !B || !C || M < 0 || N < 0 || K < 0) return ARIA_ERR_INVALID;
@@ -441,25 +447,14 @@ static int dense_product(const void* A, const void* B, void* C, const void* bias
     // with a workspace the partly filled last round of tiles is split along K (gemm3.hip), so small outputs fill the chip too
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
-    if (four_waves && (!a_oc || b_oc) && fits_dma(K, lda, ldb, bytesA, bytesB, M, N)) {
+    if ((!a_oc || b_oc) && fits_dma(K, lda, ldb, bytesA, bytesB, M, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0);
-        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, a_oc, b_oc, plan, static_cast<float*>(workspace), stream);
+        if (plan.form) return launch4(p, a_oc, b_oc, plan, workspace, stream);
     }
     if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, lda, ldb, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
         return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
-}
-
-int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
-                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
-                       int64_t workspace_bytes, void* stream) {
-    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, act, workspace, workspace_bytes, stream, true);
-}
-
-int aria_gemm_keep_sums_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc, int b_oc, int64_t lda, int64_t ldb,
-                             int64_t ldc, int c_f32, int accumulate, void* workspace, int64_t workspace_bytes, void* stream) {
-    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, ARIA_ACT_NONE, workspace, workspace_bytes, stream, false);
 }
 
 int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total,
@@ -494,7 +489,7 @@ int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t*
     const bool gv3 = (gforce && gforce[0] == '3') || ((gmask >> (b_oc ? 1 : 0)) & 1);
     if (gv3 && fits_dma(K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, 0, b_oc, -1, 1, 0);
-        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 0, b_oc, plan, nullptr, stream);
+        if (plan.form) return launch4(p, 0, b_oc, plan, nullptr, stream);
     }
     if (gv3 && use_v3((M_total / 256 + 1) * ((N + 255) / 256), K, lda, ldb, 2 * M_total * lda, 2 * (b_oc ? K * ldb : N * ldb), M_total, N,
                       v3_least(K, M_total >= V3_FEW_ROWS * E ? V3_FEW_TILES_GROUPED : 192)))
@@ -535,7 +530,7 @@ int aria_grouped_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* A
     p.E = int(E);
     p.strideB = strideB;
     p.glu = 1;
-    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
+    return launch_large(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb,
@@ -553,7 +548,7 @@ int aria_gemm_swiglu_bf16(const void* A, const void* B, void* H, void* ACT, int6
     p.M = int(M), p.N = int(N2), p.K = int(K);
     p.mode = 0;
     p.glu = 1;
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 int aria_gemm_relu_glu_bf16(const void* A, const void* B, void* ACT, int64_t M, int64_t N2, int64_t K, int64_t lda, int64_t ldb, int64_t ldact, void* stream) {
@@ -569,7 +564,7 @@ int aria_gemm_relu_glu_bf16(const void* A, const void* B, void* ACT, int64_t M, 
     p.M = int(M), p.N = int(N2), p.K = int(K);
     p.mode = 0;
     p.glu = 2;
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // gate / up weights as two [.., I, K] tensors of one allocation (gptfast's w1 / w3): rows of the up tensor as an offset from the gate tensor
@@ -609,7 +604,7 @@ int aria_grouped_gemm_swiglu_split_bf16(const void* A, const void* Bg, const voi
     p.strideB = strideB;
     p.glu = 1;
     p.glu_up_rows = up_rows;
-    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
+    return launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_swiglu_split_bf16(const void* A, const void* Bg, const void* Bu, void* H, void* ACT, int64_t M, int64_t I, int64_t K, int64_t lda,
@@ -634,7 +629,7 @@ int aria_gemm_swiglu_split_bf16(const void* A, const void* Bg, const void* Bu, v
     p.mode = 0;
     p.glu = 1;
     p.glu_up_rows = up_rows;
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // Expert parallelism: grouped launches over the SEGMENTS of an all-to-all's output (ordered (source rank, local expert)): segment g uses
@@ -660,7 +655,7 @@ int aria_grouped_gemm_seg_bf16(const void* A, const void* B, void* C, const int3
     p.E = int(n_seg);
     p.strideB = strideB;
     p.expert_mod = int(n_local);
-    return g_last_variant = 3, launch_large(p, 0, b_oc, int(M_total / 256 + n_seg), stream);
+    return launch_large(p, 0, b_oc, int(M_total / 256 + n_seg), stream);
 }
 
 int aria_grouped_gemm_swiglu_seg_bf16(const void* A, const void* B, void* H, void* ACT, const int32_t* offsets, int64_t n_seg, int64_t n_local,
@@ -685,7 +680,7 @@ int aria_grouped_gemm_swiglu_seg_bf16(const void* A, const void* B, void* H, voi
     p.strideB = strideB;
     p.glu = 1;
     p.expert_mod = int(n_local);
-    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + n_seg), stream);
+    return launch_large(p, 0, 1, int(M_total / 256 + n_seg), stream);
 }
 
 // K2: the two fused SwiGLU launches over grouped rows with the dispatcher's gather folded into the A loader.  X is the un-permuted token
@@ -712,7 +707,7 @@ int aria_grouped_gemm_swiglu_gather_bf16(const void* X, const int32_t* rows, int
     p.strideB = strideB;
     p.glu = 1;
     p.gather_rows = rows;
-    return g_last_variant = 3, launch_large(p, 0, 1, int(M_total / 256 + E), stream);
+    return launch_large(p, 0, 1, int(M_total / 256 + E), stream);
 }
 
 int aria_grouped_gemm_swiglu_split_gather_bf16(const void* X, const int32_t* rows, int64_t T, const void* Bg, const void* Bu, void* H, void* ACT,
@@ -742,7 +737,7 @@ int aria_grouped_gemm_swiglu_split_gather_bf16(const void* X, const int32_t* row
     p.glu = 1;
     p.glu_up_rows = up_rows;
     p.gather_rows = rows;
-    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
+    return launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 // K7: wqkv projection + interleaved RoPE + KV-cache write in one launch (gptfast/model.py:413-435, 67-93).
@@ -770,7 +765,7 @@ int aria_gemm_qkv_rope_cache_bf16(const void* X, const void* Wqkv, void* Q, void
     p.rope_hd = int(hd), p.rope_D = int(D), p.rope_S = int(S), p.cache_S = int(S_cache);
     p.kc = Kc, p.vc = Vc;
     p.ld_cache = ld_cache;
-    return g_last_variant = 3, launch_large(p, 0, 0, int((M + 255) / 256), stream);
+    return launch_large(p, 0, 0, int((M + 255) / 256), stream);
 }
 
 // The HF layer's q | k | v projection + half-split RoPE in one launch (LlamaAttention.forward, modeling_llama.py:243-281, 130-160)
@@ -824,7 +819,7 @@ int aria_grouped_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H,
     p.E = int(E);
     p.strideB = strideB;
     p.dglu = 1;
-    return g_last_variant = 3, launch_large(p, 0, 0, int(M_total / 256 + E), stream);
+    return launch_large(p, 0, 0, int(M_total / 256 + E), stream);
 }
 
 int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* DH, int64_t M, int64_t I, int64_t K, int b_oc, int64_t lda,
@@ -842,7 +837,7 @@ int aria_gemm_dswiglu_bf16(const void* dY, const void* B, const void* H, void* D
     p.M = int(M), p.N = int(I), p.K = int(K);
     p.mode = 0;
     p.dglu = 1;
-    return g_last_variant = 3, launch_large(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
+    return launch_large(p, 0, b_oc ? 1 : 0, int((M + 255) / 256), stream);
 }
 
 // The weight gradient of experts.fc1 WITHOUT the permuted copy of the tokens (moe_lm.py:326-334: permuted = x.index_select(0, sorted // topk)):
@@ -888,7 +883,7 @@ int aria_grouped_gemm_wgrad_gather_sized_bf16(const void* X, const int32_t* rows
     p.accumulate = accumulate;
     p.gather_rows = rows;
     p.ntn = int((N + BN - 1) / BN);
-    return g_last_variant = 3, launch_large(p, 1, 1, int((K + 255) / 256), stream, M_total);
+    return launch_large(p, 1, 1, int((K + 255) / 256), stream, M_total);
 }
 
 // ---- LoRA as a K-extension of the base GEMM (GemmParams::ext_k; aria/lora/layers.py:129-139, peft's Linear adapter): v3 only -- shapes the
@@ -1024,7 +1019,7 @@ int aria_grouped_gemm_wgrad_sized_bf16(const void* A, const void* dY, void* dW, 
     const char* wg3 = std::getenv("ARIA_GEMM_WGRAD_V3");
     if (force || !(wg3 && wg3[0] == '0')) {
         const Gemm4Plan plan = fits_dma(64, lda, ldy, 0, 0, K, N) ? aria_plan_gemm4(p, 1, 1, M_total, 1, 0) : Gemm4Plan{};
-        if (plan.form) return g_last_variant = 3, aria_launch_gemm4(p, 1, 1, plan, nullptr, stream);
+        if (plan.form) return launch4(p, 1, 1, plan, nullptr, stream);
         if (use_v3(((K + 255) / 256) * ((N + 255) / 256) * E, 64, lda, ldy, 0, 0, K, N)) return g_last_variant = 3, aria_launch_gemm3(p, 1, 1, int((K + 255) / 256), stream);
     }
     if (use_v2(((K + 255) / 256) * ((N + 255) / 256) * E)) return g_last_variant = 2, aria_launch_gemm2(p, 1, 1, int((K + 255) / 256), int(E), stream);

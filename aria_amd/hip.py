@@ -33,6 +33,7 @@ RESTYPES = {"aria_gemm_workspace_bytes": c_int64, "aria_decode_scratch_bytes": c
 SIGNATURES = {
     "aria_abi_version": [],
     "aria_last_gemm_variant": [],
+    "aria_last_gemm_tiles": [],
     "aria_last_attn_bwd_variant": [],
     "aria_last_attn_fwd_variant": [],
     "aria_decode_scratch_bytes": [P],
@@ -55,7 +56,6 @@ SIGNATURES = {
     "aria_decode_graph_destroy": [P],
     "aria_gemm_bf16": [P, P, P, P, I64, I64, I64, I32, I32, I64, I64, I64, I32, I32, P],
     "aria_gemm_bf16_ws": [P, P, P, P, I64, I64, I64, I32, I32, I64, I64, I64, I32, I32, P, I64, P],
-    "aria_gemm_keep_sums_bf16": [P, P, P, P, I64, I64, I64, I32, I32, I64, I64, I64, I32, I32, P, I64, P],
     "aria_gemm_workspace_bytes": [I64, I64, I64, I32, I32],
     "aria_gemm_act_bf16": [P, P, P, P, I64, I64, I64, I32, I32, I64, I64, I64, I32, I32, I32, P, I64, P],
     "aria_grouped_gemm_bf16": [P, P, P, P, I64, I64, I64, I64, I32, I64, I64, I64, I64, P],

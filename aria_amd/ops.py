@@ -134,10 +134,9 @@ def rows_experts(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, rows: 
 
 
 def gemm(a: torch.Tensor, b: torch.Tensor, *, a_oc: bool = False, b_oc: bool = False, bias: Optional[torch.Tensor] = None,
-         out: Optional[torch.Tensor] = None, out_dtype=bf16, accumulate: bool = False, act: Optional[str] = None,
-         keep_sums: bool = False) -> torch.Tensor:
+         out: Optional[torch.Tensor] = None, out_dtype=bf16, accumulate: bool = False, act: Optional[str] = None) -> torch.Tensor:
     """C[M,N] = op(A) op(B) (+bias) (+C).  a: [M,K] (a_oc=False) or [K,M] (a_oc=True);
-    b: [N,K] (b_oc=False, i.e. nn.Linear weight) or [K,N] (b_oc=True).  keep_sums: the 256 x 256 tiles' order of sums (aria_gemm_keep_sums_bf16)."""
+    b: [N,K] (b_oc=False, i.e. nn.Linear weight) or [K,N] (b_oc=True)."""
     _chk(a, name="a"), _chk(b, name="b")
     lda, ldb = _rowmajor_2d(a, "a"), _rowmajor_2d(b, "b")
     M, K = (a.shape[1], a.shape[0]) if a_oc else (a.shape[0], a.shape[1])
@@ -160,10 +159,6 @@ def gemm(a: torch.Tensor, b: torch.Tensor, *, a_oc: bool = False, b_oc: bool = F
         ws = _gemm_workspace(a.device, _stream(a), need) if need > 0 else None
         lib.call("aria_gemm_act_bf16", _p(a), _p(b), _p(out), _p(bias), M, N, K, int(a_oc), int(b_oc), lda, ldb, ldc, c_f32,
                  int(accumulate), ACTIVATIONS[act], _p(ws), ws.numel() if ws is not None else 0, _stream(a))
-    elif keep_sums:
-        ws = _gemm_workspace(a.device, _stream(a), need) if need > 0 else None
-        lib.call("aria_gemm_keep_sums_bf16", _p(a), _p(b), _p(out), _p(bias), M, N, K, int(a_oc), int(b_oc), lda, ldb, ldc, c_f32, int(accumulate), _p(ws),
-                 ws.numel() if ws is not None else 0, _stream(a))
     elif need > 0:  # small outputs: let the library split the last round of tiles along K (fp32 slabs in a scratch buffer)
         ws = _gemm_workspace(a.device, _stream(a), need)
         lib.call("aria_gemm_bf16_ws", _p(a), _p(b), _p(out), _p(bias), M, N, K, int(a_oc), int(b_oc), lda, ldb, ldc,
@@ -371,7 +366,7 @@ def gemm_lora(a: torch.Tensor, b: torch.Tensor, ea: torch.Tensor, eb: torch.Tens
     if _lora_ext_ok(K, r) and _try_lora("aria_gemm_lora_bf16", _p(a), _p(b), _p(out), M, N, K, int(b_oc), lda, ldb, N, _p(ea), _p(eb), r,
                                         _rowmajor_2d(ea, "ea"), _rowmajor_2d(eb, "eb"), _stream(a)):
         return out
-    gemm(a, b, b_oc=b_oc, out=out, keep_sums=True)
+    gemm(a, b, b_oc=b_oc, out=out)
     return gemm(ea, eb, b_oc=b_oc, out=out, accumulate=True)
 
 
@@ -386,7 +381,7 @@ def gemm_swiglu_lora(x: torch.Tensor, w: torch.Tensor, ea: torch.Tensor, eb: tor
         if _try_lora("aria_gemm_swiglu_lora_bf16", _p(x), _p(w), _p(h) if want_h else None, _p(act), M, N2, K, _rowmajor_2d(x, "x"),
                      _rowmajor_2d(w, "w"), N2, N2 // 2, _p(ea), _p(eb), r, _rowmajor_2d(ea, "ea"), _rowmajor_2d(eb, "eb"), _stream(x)):
             return h, act
-    h = gemm(x, w, keep_sums=True)
+    h = gemm(x, w)
     gemm(ea, eb, out=h, accumulate=True)
     return (h if want_h else None), swiglu(h)
 

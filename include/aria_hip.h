@@ -35,6 +35,8 @@ int aria_abi_version(void);
 /* Test/diagnostic aid: which GEMM kernel family the calling thread's last aria_*gemm* call dispatched to
  * (1 = 128x128 tile, 2 = 256x256 register-staged, 3 = LDS-DMA: 256x256 phase-scheduled, or the four-wave tiles; 0 = none yet). */
 int aria_last_gemm_variant(void);
+/* The same of the four-wave tiles: their form (1: 128 x 256, 2: 256 x 160 or 128 x 320, 3: 128 x 256 twice a CU) + 16 times the pieces of the reduction; 0: other tiles. */
+int aria_last_gemm_tiles(void);
 
 /* ------------------------------------------------------------------------------------------------
  * GEMM family (gemm.hip) -- v_mfma_f32_32x32x16_bf16, fp32 accumulate.
@@ -53,7 +55,8 @@ int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias /* bf
 /* Same GEMM with a caller-owned scratch buffer.  When the 256x256 tile list ends in a partly filled round (e.g. a
  * [2560,2560] weight gradient = 100 tiles on 256 CUs) those tiles are computed by several workgroups over disjoint K ranges
  * into fp32 slabs in `workspace` and summed in a fixed order by a second kernel (deterministic).  aria_gemm_workspace_bytes
- * returns the size that enables it for a problem (0: no split would be used); a NULL / too small workspace just disables it. */
+ * returns the size that enables it for a problem (0: no split would be used); a NULL / too small workspace just disables it.
+ * A product with [N, K] weights (0, 0) has the sums of the 256 x 256 tiles, in these pieces, bit for bit, whichever tiles compute it. */
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc);
 int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, void* workspace,
@@ -67,12 +70,6 @@ int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, i
 int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                        int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
                        int64_t workspace_bytes, void* stream);
-/* aria_gemm_bf16_ws without the four-wave tiles: an output of one round then has the partial sums of the 256 x 256 tiles' split, not of theirs.  For the base product
- * under an adapter that no fused launch takes: its rounding decides near ties of the next layer's router, and with dropout a turned tie moves every later expert row
- * under another mask. */
-int aria_gemm_keep_sums_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc, int b_oc, int64_t lda, int64_t ldb,
-                             int64_t ldc, int c_f32, int accumulate, void* workspace, int64_t workspace_bytes, void* stream);
-
 /* experts_gemm(input, weight, tokens_per_expert)  -- seam B1, aria/model/moe_lm.py:431-443 (grouped_gemm.ops.gmm
  * or sequential_gemm :398-428), called from GroupedGEMM.forward :467-484.
  *   C[s_e : s_e+n_e, :] = A[s_e : s_e+n_e, :] * B_e       offsets[e] = s_e (device int32[E+1], offsets[E] = M_total)

@@ -114,6 +114,12 @@ def case_gemm_split_k_slabs(dev, M, N, K, a_oc, b_oc):
     assert torch.equal(acc.cpu(), (ops.gemm(a, b, a_oc=a_oc, b_oc=b_oc, bias=bias.to(dev), out_dtype=torch.float32).cpu() + old.float()).to(bf16))
 
 
+def last_gemm_tiles():
+    from aria_amd import hip
+
+    return hip.get_lib().cdll.aria_last_gemm_tiles()
+
+
 def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
     activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""
@@ -134,21 +140,24 @@ def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     monkeypatch.setattr(ops, "GEMM_SPLIT_K", False)
     monkeypatch.setenv("ARIA_GEMM_FORCE", force)
     got = results()
+    assert last_gemm_tiles() == (3 if a_oc else 2 if force == "46" else 1) + 16
     monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
     for x, y in zip(got, results()):
         assert torch.equal(x.cpu(), y.cpu())
 
 
-def case_gemm_forward_sums(dev, monkeypatch, M, N, K):
+def case_gemm_forward_sums(dev, monkeypatch, M, N, K, tiles):
     """A product with [N, K] weights has the sums of the 256 x 256 tiles bit for bit, whichever tiles compute it: a forward pass's products lie in front of routers, whose
-    near ties turn with another cut of the reduction."""
+    near ties turn with another cut of the reduction.  tiles: what the rule takes (aria_last_gemm_tiles)."""
     from aria_amd import ops
 
     a, b, bias = rnd(M, K, seed=M + K).to(dev), rnd(N, K, seed=N, scale=0.3).to(dev), rnd(N, seed=3).to(dev)
     got = [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]
+    assert last_gemm_tiles() == tiles
     monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
     for x, y in zip(got, [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]):
         assert torch.equal(x.cpu(), y.cpu())
+    assert last_gemm_tiles() == 0
 
 
 def case_gemm_long_rows(dev, monkeypatch, force):
@@ -1179,14 +1188,19 @@ def case_router_fused(dev, T, D, E, k):
     assert int(counts.sum()) == T * k
 
 
-def case_gemm_keep_sums(dev, M, N, K):
-    """The base product under an adapter (no four-wave tiles) against the product in 64 bits: a 32-bit sum rounded once."""
+def case_gemm_keep_sums(dev, monkeypatch, M, N, K):
+    """The base product under an adapter that no fused launch takes: the 256 x 256 tiles' sums bit for bit (its rounding decides near ties of the next layer's router, and
+    with dropout a turned tie moves every later expert row under another mask), each a 32-bit sum rounded once against the product in 64 bits."""
     from aria_amd import ops
 
-    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.1)
-    got = ops.gemm(x.to(dev), w.to(dev), keep_sums=True).double().cpu()
+    x, w, ea, eb = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.1), rnd(M, 8, seed=3).to(dev), rnd(N, 8, seed=4).to(dev)
+    got = ops.gemm_lora(x.to(dev), w.to(dev), ea, eb)
+    with monkeypatch.context() as mp:
+        mp.setenv("ARIA_GEMM_FORCE", "3")
+        base = ops.gemm(x.to(dev), w.to(dev))
     want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
-    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
+    assert bool(((base.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
+    assert torch.equal(got, ops.gemm(ea, eb, out=base, accumulate=True))
 
 
 def case_thin_product(dev, M, N, K):

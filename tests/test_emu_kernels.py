@@ -247,9 +247,9 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(force_gemm_v3, B, S, D, hd, K):
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (300, 264, 512)])
-def test_gemm_keep_sums(M, N, K):
-    C.case_gemm_keep_sums(DEV, M, N, K)
+@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (300, 264, 512), (40, 1032, 1536)])
+def test_gemm_keep_sums(monkeypatch, M, N, K):
+    C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (70, 24, 128), (64, 16, 192), (40, 8, 2048)])
@@ -397,12 +397,13 @@ def test_gemm_long_rows(monkeypatch, force):
     C.case_gemm_long_rows(DEV, monkeypatch, force)
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 1032, 1536), (40, 1032, 2048), (200, 1024, 2304)])
-def test_gemm_forward_sums(monkeypatch, M, N, K):
-    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K)
+@pytest.mark.parametrize("M,N,K,tiles", [(40, 1032, 1536, 17), (40, 1032, 2048, 65), (200, 1024, 2304, 65)])
+def test_gemm_forward_sums(monkeypatch, M, N, K, tiles):
+    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K, tiles)
 
 
 @pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 1664, True)])
 def test_gemm_four_waves_split(M, N, K, b_oc):
     """A reduction cut into pieces of whole stages, by the rule itself."""
     C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)
+    assert C.last_gemm_tiles() > 32 and C.last_gemm_tiles() % 16 == 1   # (128 x 256, at least two pieces)

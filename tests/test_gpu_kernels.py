@@ -241,9 +241,9 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(B, S, D, hd, K):   # q | k | v proje
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K) == (D >= 2560)
 
 
-@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (3000, 2560, 3328)])
-def test_gemm_keep_sums(M, N, K):
-    C.case_gemm_keep_sums(DEV, M, N, K)
+@pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (777, 2560, 2560), (3000, 2560, 3328)])
+def test_gemm_keep_sums(monkeypatch, M, N, K):
+    C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 32, 576), (5580, 32, 1536), (1000, 24, 1728), (300, 16, 3328), (66000, 8, 2048)])
@@ -387,12 +387,14 @@ def test_gemm_long_rows(monkeypatch, force):
     C.case_gemm_long_rows(DEV, monkeypatch, force)
 
 
-@pytest.mark.parametrize("M,N,K", [(40, 1032, 1536), (777, 2560, 2560), (777, 2560, 3328), (777, 7680, 2560), (1868, 2560, 2560), (4500, 1536, 4096), (200, 2560, 6656)])
-def test_gemm_forward_sums(monkeypatch, M, N, K):
-    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K)
+@pytest.mark.parametrize("M,N,K,tiles", [(40, 1032, 1536, 17), (777, 2560, 2560, 0), (777, 2560, 3328, 0), (777, 7680, 2560, 17), (1868, 2560, 2560, 0),
+                                         (4500, 1536, 4096, 0), (200, 2560, 6656, 193), (4096, 2560, 2560, 18)])
+def test_gemm_forward_sums(monkeypatch, M, N, K, tiles):
+    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K, tiles)
 
 
 @pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 1664, True)])
 def test_gemm_four_waves_split(M, N, K, b_oc):
     """A reduction cut into pieces of whole stages, by the rule itself."""
     C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)
+    assert C.last_gemm_tiles() > 32 and C.last_gemm_tiles() % 16 == 1   # (128 x 256, at least two pieces)
