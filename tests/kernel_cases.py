@@ -120,6 +120,36 @@ def last_gemm_tiles():
     return hip.get_lib().cdll.aria_last_gemm_tiles()
 
 
+FUSED_FOUR_WAVES = ["grouped_gemm", "grouped_gemm_wgrad", "grouped_gemm_wgrad_gather", "grouped_gemm_swiglu", "gemm_swiglu", "grouped_gemm_swiglu_split", "gemm_swiglu_split",
+                    "grouped_gemm_swiglu_gather", "grouped_gemm_swiglu_split_gather", "grouped_gemm_dswiglu", "gemm_dswiglu", "gemm_qkv_rope_cache"]
+
+
+def case_gemm_four_waves_fused(dev, monkeypatch):
+    """Every other end of these tiles, with rows by expert that fill no tile, one and several; each operation is seen to run on them."""
+    from aria_amd import ops
+
+    seen = {}
+    for name in FUSED_FOUR_WAVES:
+        def run(*a, plain=getattr(ops, name), name=name, **k):
+            out = plain(*a, **k)
+            seen.setdefault(name, set()).add(last_gemm_tiles())
+            return out
+
+        monkeypatch.setattr(ops, name, run)
+    monkeypatch.setenv("ARIA_GEMM_FORCE", "4")
+    counts = [130, 0, 70, 5, 0, 257, 1]
+    case_grouped_gemm(dev, counts)
+    case_gemm_swiglu_fused(dev, counts, 128, 128, 130)
+    case_gemm_swiglu_split(dev, counts, 192, 256, 72)
+    case_gemm_dswiglu_fused(dev, counts, 128, 384, 129)
+    case_gemm_swiglu_gather(dev, 150, 8, 2, 128, 128)
+    case_gemm_qkv_rope_cache(dev, 2, 37, 256, 64, 128, 48, True)
+    for T, E, k, K, N in ((150, 8, 2, 264, 136), (700, 8, 1, 128, 256), (40, 4, 3, 64, 72)):
+        case_grouped_gemm_wgrad_gather(dev, T, E, k, K, N)
+    form = {n: 3 if "wgrad" in n else 1 for n in FUSED_FOUR_WAVES}
+    assert all(form[n] + 16 in seen.get(n, ()) for n in FUSED_FOUR_WAVES), seen
+
+
 def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
     activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""

@@ -375,17 +375,7 @@ def test_gemm_four_waves(dma_order, monkeypatch, force, M, N, K, a_oc, b_oc):
 
 
 def test_gemm_four_waves_fused(dma_order, monkeypatch):
-    """Every other end of these tiles, with rows by expert that fill no tile, one and several."""
-    monkeypatch.setenv("ARIA_GEMM_FORCE", "4")
-    counts = [130, 0, 70, 5, 0, 257, 1]
-    C.case_grouped_gemm(DEV, counts)
-    C.case_gemm_swiglu_fused(DEV, counts, 128, 128, 130)
-    C.case_gemm_swiglu_split(DEV, counts, 192, 256, 72)
-    C.case_gemm_dswiglu_fused(DEV, counts, 128, 384, 129)
-    C.case_gemm_swiglu_gather(DEV, 150, 8, 2, 128, 128)
-    C.case_gemm_qkv_rope_cache(DEV, 2, 37, 256, 64, 128, 48, True)
-    for T, E, k, K, N in ((150, 8, 2, 264, 136), (700, 8, 1, 128, 256), (40, 4, 3, 64, 72)):
-        C.case_grouped_gemm_wgrad_gather(DEV, T, E, k, K, N)
+    C.case_gemm_four_waves_fused(DEV, monkeypatch)
 
 
 def test_grouped_gemm_switches(monkeypatch):
