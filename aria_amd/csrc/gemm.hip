@@ -387,6 +387,13 @@ int aria_expert_pair_tiles(const void* X, const int32_t* rows, int64_t T, const 
     return aria_launch_gemm4(p, 0, 0, plan, nullptr, stream);
 }
 
+static int dense_product(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc, int b_oc, int64_t lda, int64_t ldb, int64_t ldc,
+                         int c_f32, int accumulate, int act, void* workspace, int64_t workspace_bytes, void* stream, bool own_cut);
+int aria_gemm_own_cut(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+    return dense_product(A, B, C, nullptr, M, N, K, 0, 0, K, K, N, 0, 0, ARIA_ACT_NONE, workspace, workspace_bytes, stream, true);
+}
+int64_t aria_gemm_own_cut_bytes(int64_t M, int64_t N, int64_t K) { return std::max(aria_gemm3_workspace_bytes(M, N, K), aria_gemm4_workspace_bytes(M, N, K)); }
+
 extern "C" {
 
 int aria_last_gemm_variant(void) { return g_last_variant & 255; }
@@ -395,7 +402,7 @@ int aria_last_gemm_tiles(void) { return g_last_variant >> 8; }
 
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc) {
     if (M <= 0 || N <= 0 || (a_oc && !b_oc)) return 0;
-    return std::max(aria_gemm3_workspace_bytes(M, N, K), a_oc || !b_oc ? 0 : aria_gemm4_workspace_bytes(M, N, K));
+    return a_oc || !b_oc ? aria_gemm3_workspace_bytes(M, N, K) : aria_gemm_own_cut_bytes(M, N, K);
 }
 
 int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
@@ -410,9 +417,10 @@ int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, i
                               workspace_bytes, stream);
 }
 
-int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
-                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
-                       int64_t workspace_bytes, void* stream) {
+// own_cut: whether the four-wave tiles may cut the reduction as it is fastest for them (see aria_plan_gemm4)
+static int dense_product(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
+                         int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
+                         int64_t workspace_bytes, void* stream, bool own_cut) {
     if (act != ARIA_ACT_NONE && act != ARIA_ACT_GELU_TANH && act != ARIA_ACT_RELU2) return ARIA_ERR_UNSUPPORTED;
     if (act == ARIA_ACT_RELU2 && (a_oc || b_oc)) return ARIA_ERR_UNSUPPORTED;   // (built for the forward form only)
     if (!A || !B || !C || M < 0 || N < 0 || K < 0) return ARIA_ERR_INVALID;
@@ -448,13 +456,19 @@ int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, 
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
     if ((!a_oc || b_oc) && fits_dma(K, lda, ldb, bytesA, bytesB, M, N)) {
-        const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0);
+        const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0, own_cut);
         if (plan.form) return launch4(p, a_oc, b_oc, plan, workspace, stream);
     }
     if ((!a_oc || b_oc) && use_v3(splits ? (t256 < 192 ? 192 : t256) : t256, K, lda, ldb, bytesA, bytesB, M, N, v3_least(K, V3_FEW_TILES)))
         return g_last_variant = 3, aria_launch_gemm3(p, a_oc, b_oc, int((M + 255) / 256), stream, workspace, workspace_bytes);
     if (use_v2(t256)) return g_last_variant = 2, aria_launch_gemm2(p, a_oc, b_oc, int((M + 255) / 256), 1, stream);
     return g_last_variant = 1, launch_gemm(p, a_oc, b_oc, p.ntn * ntm, 1, stream);
+}
+
+int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
+                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
+                       int64_t workspace_bytes, void* stream) {
+    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, act, workspace, workspace_bytes, stream, b_oc != 0);
 }
 
 int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total,

@@ -557,7 +557,7 @@ long long aria_gemm4_workspace_bytes(long long M, long long N, long long K) {
     return s > 1 ? cdiv(M, 128) * cdiv(N, 256) * s * (128 * 256 * 4) : 0;
 }
 
-Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes) {
+Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes, bool own_cut) {
     Gemm4Plan none, plan;
     if (p.ext_k || p.rope_sn || (a_oc && !b_oc) || p.N < 8 || (a_oc && p.M < 8)) return none;   // (p.rope_sn: the entry takes whole rounds of 256 x 256 tiles only)
     const bool plain = !p.glu && !p.dglu && !p.rope_fc;
@@ -598,13 +598,14 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     // [N, K] weights are a forward pass's: its sums are cut where the 256 x 256 tiles cut them, and so have their bits.  Another cut rounds a few elements otherwise, and
     // where a router follows, a near tie of a token's last expert turns.  777 x 2560 x 2560 in 3 pieces (27 us) for 4 (33) and 4500 x 1536 x 4096 whole (57) for 2 (68) so moved
     // single elements of a training step's gradients and of a prompt's latents by 1.5 and 0.45 of their root mean square.  [K, N] weights (input gradients) are cut as it is
-    // fastest.
+    // fastest, and so are Aria's prompts of up to 288 tokens, which other kernels than the 256 x 256 tiles served before (280 tokens, four layers: 1.014 times as
+    // fast as those with the 256 x 256 tiles' cut, 1.039 times with these tiles' own).
     int s = split3;
-    if (b_oc) s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
+    if (own_cut) s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
     if (t2 * s <= ROUND && time_128(t2, n, s) < best) best = time_128(t2, n, s), plan.form = 1, plan.split = s;
     const long long t6 = b_oc ? cdiv(p.M, 128) * cdiv(p.N, 320) : cdiv(p.M, 256) * cdiv(p.N, 160);
     const double time6 = 9.0 + (b_oc ? 1.0 : 0.85) * n;
-    if (t6 <= ROUND && time6 < best && (b_oc ? p.K <= 4096 : split3 == 1)) plan.form = 2, plan.split = 1;
+    if (t6 <= ROUND && time6 < best && (own_cut || split3 == 1) && !(b_oc && p.K > 4096)) plan.form = 2, plan.split = 1;
     return plan;
 }
 

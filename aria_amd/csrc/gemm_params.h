@@ -311,10 +311,15 @@ __attribute__((visibility("hidden"))) long long aria_gemm3_workspace_bytes(long 
 struct Gemm4Plan {
     int form = 0, split = 1;
 };
-// rows: mode 2's rows of all experts together (< 0: not known); split3: pieces that the 256 x 256 tiles would cut the reduction of a partly filled round into (1: none)
-__attribute__((visibility("hidden"))) Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes);
+// rows: mode 2's rows of all experts together (< 0: not known); split3: pieces that the 256 x 256 tiles would cut the reduction of a partly filled round into (1:
+// none), which are these tiles' too unless own_cut
+__attribute__((visibility("hidden"))) Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes, bool own_cut = false);
 __attribute__((visibility("hidden"))) int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream);
 __attribute__((visibility("hidden"))) long long aria_gemm4_workspace_bytes(long long M, long long N, long long K);
+// X W^T for a dense x [M, K] and w [N, K] whose sums need not be the 256 x 256 tiles' (prompts, whose shorter ones are summed by other kernels anyway)
+__attribute__((visibility("hidden"))) int aria_gemm_own_cut(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes,
+                                                            void* stream);
+__attribute__((visibility("hidden"))) int64_t aria_gemm_own_cut_bytes(int64_t M, int64_t N, int64_t K);
 // pieces the v3 remainder split-K would take for a dense problem of at most one round (1: none)
 __attribute__((visibility("hidden"))) int aria_gemm3_split(long long M, long long N, long long K);
 // pieces that the v3 remainder split-K (with a workspace) takes for a dense problem of one column tile, for the rows from *first_row on (1: none)

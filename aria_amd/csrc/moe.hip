@@ -230,8 +230,9 @@ __device__ __forceinline__ unsigned long long match_mask(int key, const unsigned
 }
 
 // More than SORT_SMALL entries: two launches, a wave per 1024 entries in both, all of a wave's entries loaded at once.  What bounds them is latency: a count
-// per chunk, then every block adds the chunks in front of its own (coalesced 256-byte rows, four waves) instead of a launch in between.  22 000 entries on 32 experts:
-// a wave's 2048 entries one load after the other, and the sums as a third launch 29 us, with the token rows as two more 40; now SO12.
+// per chunk, then every block adds the chunks in front of its own (coalesced 256-byte rows, four waves) instead of a launch in between.  Us a call, with a wave's 2048
+// entries one load after the other and the sums as a third launch / here: 22 000 entries on 32 experts 23.3 / 17.0, with the token rows (two launches more / none) 31.0 / 19.6;
+// 393 216 on 64 63 / 17; 1.6 million 196 / 40, 6.3 million 782 / 124 (the sums of the chunks in front grow with the square, and are still the smaller part).
 constexpr int SORT_CHUNK = 1024, SORT_PER = SORT_CHUNK / 64;
 
 // pass 1: per-chunk histogram (lane e = expert e)

@@ -21,8 +21,8 @@ struct Scratch {
     char* ws;
     int64_t ws_bytes, bytes;
 };
-// A dense product x [T, K] w [N, K]^T as tiles (its reduction in pieces).  Weights from HBM, us by rows / tiles: 7680 x 2560: 128 tokens 23.7 / 23.7, 200 32.0 / 27.7, 256 34.8 /
-// 28.0, 288 38.4 / 37.0; 2560 x 2560: 200 18.9 / 18.7, 288 21.1 / 19.7; 2560 x 3328: 200 23.2 / 19.0, 288 31.1 / 21.6.  Narrower: 4096 x 1536: 288 19.3 / 18.9.
+// A dense product x [T, K] w [N, K]^T as tiles (its reduction in pieces).  Weights from HBM, us by rows / tiles: 7680 x 2560: 128 tokens 23.7 / 23.7, 200 32.0 / 28.1, 256 34.6 /
+// 30.2, 288 38.0 / 34.8; 2560 x 2560: 200 19.0 / 19.0, 288 21.1 / 20.0; 2560 x 3328: 200 23.2 / 18.9, 288 31.2 / 21.6.  Narrower: 4096 x 1536: 288 19.3 / 18.9.
 bool tiles_ahead(int64_t T, int64_t N, int64_t K) { return T > 192 && K >= 2048 && N * K >= (6 << 20) && K % 64 == 0 && N % 8 == 0; }
 Scratch layout(const int64_t* dims, int64_t T, char* base) {
     const int64_t L = dims[0], D = dims[1], E = dims[4], k = dims[5], I = dims[6], Is = dims[7];
@@ -40,7 +40,7 @@ Scratch layout(const int64_t* dims, int64_t T, char* base) {
     z.idx = ints(T * k), z.counts = ints(L * E), z.offsets = ints(E + 1), z.src = ints(T * k), z.inv = ints(T * k), z.rows = ints(T * k);
     const int64_t shapes[3][2] = {{3 * D, D}, {D, D}, {D, Is}};
     for (const auto& nk : shapes)
-        if (tiles_ahead(T, nk[0], nk[1])) z.ws_bytes = std::max(z.ws_bytes, aria_gemm_workspace_bytes(T, nk[0], nk[1], 0, 0));
+        if (tiles_ahead(T, nk[0], nk[1])) z.ws_bytes = std::max(z.ws_bytes, aria_gemm_own_cut_bytes(T, nk[0], nk[1]));
     z.ws = take(z.ws_bytes);
     z.bytes = at;
     return z;
@@ -81,7 +81,7 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         std::swap(y, spare);
     };
     auto product = [&](const bf16_t* a, const void* w, bf16_t* out, int64_t N, int64_t K) {
-        if (tiles_ahead(T, N, K)) return aria_gemm_bf16_ws(a, w, out, nullptr, T, N, K, 0, 0, K, K, N, 0, 0, z.ws_bytes ? z.ws : nullptr, z.ws_bytes, stream);
+        if (tiles_ahead(T, N, K)) return aria_gemm_own_cut(a, w, out, T, N, K, z.ws_bytes ? z.ws : nullptr, z.ws_bytes, stream);
         return aria_rows_gemm(a, w, out, 0, T, N, K, K, N, stream);
     };
     // gate and up of the experts.  Rows of an expert on average, us by rows / tiles (weights from HBM): 64 experts of 2 x 1664 x 2560: 6 192 / 206, 9 218 / 210, 12 225 / 211, 18 227 /
