@@ -2,7 +2,7 @@
 // gemm_f32.hip), enqueued in order from here.  The kernels, their operands and so the results are those of the step run sublayer by sublayer.
 //
 // Why: the host bounded these steps.  Three layers 1024 wide: 46 launches that keep the device busy for 0.32 ms took 1.2 ms, most of it the operations' own checks
-// and allocations around each launch.  A session of four prompts of up to 250 tokens and four decoded tokens took the host 3.1 ms (6 on a slower one), now 1.1.
+// and allocations around each launch.  A session of four prompts of up to 250 tokens and four decoded tokens took the host 3.1 ms (6 on a slower one), now 1.2.
 #include "aria_device.h"
 #include "aria_hip.h"
 #include <algorithm>

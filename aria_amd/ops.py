@@ -328,7 +328,7 @@ def lora_wgrad(y: torch.Tensor, u: torch.Tensor, n_first: bool) -> torch.Tensor:
     if u.shape[0] != M:
         raise ValueError("lora_wgrad: y and u must have the same rows")
     out = torch.empty((N, r) if n_first else (r, N), dtype=y.dtype, device=y.device)
-    ws = torch.empty(((M + 63) // 64 * r * N,), dtype=torch.float32, device=y.device)
+    ws = torch.empty((min(256, (M + 63) // 64) * r * N,), dtype=torch.float32, device=y.device)
     hip.get_lib().call("aria_lora_wgrad_bf16", _p(y), _p(u), _p(out), int(n_first), M, N, r, _rowmajor_2d(y, "y"), _rowmajor_2d(u, "u"), _p(ws), ws.numel(), _stream(y))
     return out
 

@@ -148,7 +148,7 @@ int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t 
  * _scale: OUT [M, r] (row stride ldo, a multiple of 8) = bf16(scale * U), any r % 8 == 0.
  * _down: U [M, r] (row stride ldu) = bf16(scale * X W^T), W [r, K] or with w_oc [K, r]; K % 64 == 0, r (K + 32) <= 57344.
  * _up:   DX [M, K] += keep ? scale * (DU A) : 0, A [r, K] with a_oc, else [K, r]; mask as aria_dropout_fwd_bf16 writes it (null: everything is kept), K % 8 == 0.
- * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 64 rows begun. */
+ * _wgrad: out [r, N], or [N, r] with n_first, = U^T Y; workspace: r N floats for every 64 rows begun, 256 times r N at most. */
 /* C [M, N] fp32 = X W^T for N = 8, 16, 24 or 32 columns, K % 64 == 0, N (K + 32) <= 57344: X, W [N, K] bf16 (the shapes and strides of the adapters' _down).  The bits
  * are those of aria_gemm_bf16_ws with a workspace: a router's choice hangs on them. */
 int aria_thin_product_f32(const void* X, const void* W, float* C, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldc, void* stream);

@@ -1315,6 +1315,18 @@ def case_lora_thin(dev, T, K, N, r, counts=None, p=0.0):
             near(ops.lora_wgrad(y, u, n_first=first), w.t() if first else w, m.t() if first else m)
 
 
+def case_lora_wgrad_many_rows(dev, M, N, r):
+    """More than 16 384 rows: 256 partial sums are workspace enough, and the sums are those of the product in 64 bits (rounded once)."""
+    from aria_amd import hip, ops
+
+    y, u = rnd(M, N, seed=1), rnd(M, r, seed=2)
+    a, b, ws, out = y.to(dev), u.to(dev), torch.empty(256 * r * N, dtype=torch.float32, device=dev), torch.empty((r, N), dtype=bf16, device=dev)
+    hip.get_lib().call("aria_lora_wgrad_bf16", a.data_ptr(), b.data_ptr(), out.data_ptr(), 0, M, N, r, N, r, ws.data_ptr(), ws.numel(), ops._stream(a))
+    want, size = u.double().t() @ y.double(), u.double().abs().t() @ y.double().abs()
+    assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
+    assert torch.equal(ops.lora_wgrad(a, b, n_first=False).cpu(), out.cpu())
+
+
 LORA_THIN = [(1, 64, 64, 8, None, 0.0), (33, 128, 192, 16, None, 0.3), (264, 576, 128, 8, None, 0.05), (0, 128, 64, 8, [70, 0, 33, 5, 0], 0.3),
              (0, 64, 128, 16, [1, 0, 32] + [3] * 70, 0.0)]
 

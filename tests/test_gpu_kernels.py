@@ -256,6 +256,11 @@ def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
 
 
+@pytest.mark.parametrize("M,N,r", [(16385, 8, 8), (50000, 2560, 16)])
+def test_lora_wgrad_of_many_rows(M, N, r):
+    C.case_lora_wgrad_many_rows(DEV, M, N, r)
+
+
 @pytest.mark.parametrize("T,K,N,r,counts,p", C.LORA_THIN + [(4096, 2560, 3328, 8, None, 0.05), (1000, 3328, 2560, 16, None, 0.0), (0, 2560, 1664, 8, [300, 0, 1500, 70], 0.05)])
 def test_lora_thin_products(T, K, N, r, counts, p):
     C.case_lora_thin(DEV, T, K, N, r, counts, p)
