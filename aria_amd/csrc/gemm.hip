@@ -402,7 +402,7 @@ int aria_last_gemm_tiles(void) { return g_last_variant >> 8; }
 
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc) {
     if (M <= 0 || N <= 0 || (a_oc && !b_oc)) return 0;
-    return a_oc || !b_oc ? aria_gemm3_workspace_bytes(M, N, K) : aria_gemm_own_cut_bytes(M, N, K);
+    return aria_gemm3_workspace_bytes(M, N, K);
 }
 
 int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
@@ -468,7 +468,7 @@ static int dense_product(const void* A, const void* B, void* C, const void* bias
 int aria_gemm_act_bf16(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                        int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, int act, void* workspace,
                        int64_t workspace_bytes, void* stream) {
-    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, act, workspace, workspace_bytes, stream, b_oc != 0);
+    return dense_product(A, B, C, bias, M, N, K, a_oc, b_oc, lda, ldb, ldc, c_f32, accumulate, act, workspace, workspace_bytes, stream, false);
 }
 
 int aria_grouped_gemm_bf16(const void* A, const void* B, void* C, const int32_t* offsets, int64_t E, int64_t M_total,

@@ -595,11 +595,11 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
         return plan;
     }
     double best = 0.94 * time_else(p.M, p.N, n, split3);
-    // [N, K] weights are a forward pass's: its sums are cut where the 256 x 256 tiles cut them, and so have their bits.  Another cut rounds a few elements otherwise, and
-    // where a router follows, a near tie of a token's last expert turns.  777 x 2560 x 2560 in 3 pieces (27 us) for 4 (33) and 4500 x 1536 x 4096 whole (57) for 2 (68) so moved
-    // single elements of a training step's gradients and of a prompt's latents by 1.5 and 0.45 of their root mean square.  [K, N] weights (input gradients) are cut as it is
-    // fastest, and so are Aria's prompts of up to 288 tokens, which other kernels than the 256 x 256 tiles served before (280 tokens, four layers: 1.014 times as
-    // fast as those with the 256 x 256 tiles' cut, 1.039 times with these tiles' own).
+    // A product's sums are cut where the 256 x 256 tiles cut them, and so have their bits.  Another cut rounds a few elements otherwise; in front of a router a near tie of a
+    // token's last expert can turn, and in a short sample's gradient of the embedding, most of whose rows are zeros, single elements moved by 1.1 .. 1.9 of its root mean
+    // square (64 .. 130 tokens; 0 with this cut, 777 tokens 5.15 -> 5.20 ms).  Given up for it, us: 777 x 2560 x 2560 in 3 pieces 27, in those tiles' 4 33; 4500 x 1536 x 4096
+    // whole 57, in 2 68.  Aria's prompts of up to 288 tokens, which other kernels than the 256 x 256 tiles served before, are cut as it is fastest (own_cut; 280 tokens, four
+    // layers: 1.014 times as fast as those with the 256 x 256 tiles' cut, 1.039 times with these tiles' own).
     int s = split3;
     if (own_cut) s = workspace_bytes >= aria_gemm4_workspace_bytes(p.M, p.N, p.K) ? split_128(p.M, p.N, p.K) : 1;
     if (t2 * s <= ROUND && time_128(t2, n, s) < best) best = time_128(t2, n, s), plan.form = 1, plan.split = s;

@@ -56,7 +56,7 @@ int aria_gemm_bf16(const void* A, const void* B, void* C, const void* bias /* bf
  * [2560,2560] weight gradient = 100 tiles on 256 CUs) those tiles are computed by several workgroups over disjoint K ranges
  * into fp32 slabs in `workspace` and summed in a fixed order by a second kernel (deterministic).  aria_gemm_workspace_bytes
  * returns the size that enables it for a problem (0: no split would be used); a NULL / too small workspace just disables it.
- * A product with [N, K] weights (0, 0) has the sums of the 256 x 256 tiles, in these pieces, bit for bit, whichever tiles compute it. */
+ * A forward product or an input gradient has the sums of the 256 x 256 tiles, in these pieces, bit for bit, whichever tiles compute it. */
 int64_t aria_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int a_oc, int b_oc);
 int aria_gemm_bf16_ws(const void* A, const void* B, void* C, const void* bias, int64_t M, int64_t N, int64_t K, int a_oc,
                       int b_oc, int64_t lda, int64_t ldb, int64_t ldc, int c_f32, int accumulate, void* workspace,

@@ -176,16 +176,20 @@ def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
         assert torch.equal(x.cpu(), y.cpu())
 
 
-def case_gemm_forward_sums(dev, monkeypatch, M, N, K, tiles):
-    """A product with [N, K] weights has the sums of the 256 x 256 tiles bit for bit, whichever tiles compute it: a forward pass's products lie in front of routers, whose
-    near ties turn with another cut of the reduction.  tiles: what the rule takes (aria_last_gemm_tiles)."""
+def case_gemm_same_sums(dev, monkeypatch, M, N, K, b_oc, tiles):
+    """A product has the sums of the 256 x 256 tiles bit for bit, whichever tiles compute it: a forward pass's products lie in front of routers, whose near ties turn with
+    another cut of the reduction, and gradients of short samples move in single elements.  tiles: what the rule takes (aria_last_gemm_tiles)."""
     from aria_amd import ops
 
-    a, b, bias = rnd(M, K, seed=M + K).to(dev), rnd(N, K, seed=N, scale=0.3).to(dev), rnd(N, seed=3).to(dev)
-    got = [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]
+    a, b, bias = rnd(M, K, seed=M + K).to(dev), rnd(*((K, N) if b_oc else (N, K)), seed=N, scale=0.3).to(dev), rnd(N, seed=3).to(dev)
+
+    def results():
+        return [ops.gemm(a, b, b_oc=b_oc, bias=bias), ops.gemm(a, b, b_oc=b_oc, out_dtype=torch.float32)]
+
+    got = results()
     assert last_gemm_tiles() == tiles
     monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
-    for x, y in zip(got, [ops.gemm(a, b, bias=bias), ops.gemm(a, b, out_dtype=torch.float32)]):
+    for x, y in zip(got, results()):
         assert torch.equal(x.cpu(), y.cpu())
     assert last_gemm_tiles() == 0
 

@@ -392,12 +392,13 @@ def test_gemm_long_rows(monkeypatch, force):
     C.case_gemm_long_rows(DEV, monkeypatch, force)
 
 
-@pytest.mark.parametrize("M,N,K,tiles", [(40, 1032, 1536, 17), (40, 1032, 2048, 65), (200, 1024, 2304, 65)])
-def test_gemm_forward_sums(monkeypatch, M, N, K, tiles):
-    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K, tiles)
+@pytest.mark.parametrize("M,N,K,b_oc,tiles", [(40, 1032, 1536, False, 17), (40, 1032, 2048, False, 65), (200, 1024, 2304, False, 65), (40, 1032, 1536, True, 17),
+                                              (40, 1032, 2048, True, 65)])
+def test_gemm_same_sums(monkeypatch, M, N, K, b_oc, tiles):
+    C.case_gemm_same_sums(DEV, monkeypatch, M, N, K, b_oc, tiles)
 
 
-@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 1664, True)])
+@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 2048, True)])
 def test_gemm_four_waves_split(M, N, K, b_oc):
     """A reduction cut into pieces of whole stages, by the rule itself."""
     C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)

@@ -382,13 +382,15 @@ def test_gemm_long_rows(monkeypatch, force):
     C.case_gemm_long_rows(DEV, monkeypatch, force)
 
 
-@pytest.mark.parametrize("M,N,K,tiles", [(40, 1032, 1536, 17), (777, 2560, 2560, 0), (777, 2560, 3328, 0), (777, 7680, 2560, 17), (1868, 2560, 2560, 0),
-                                         (4500, 1536, 4096, 0), (200, 2560, 6656, 193), (4096, 2560, 2560, 18)])
-def test_gemm_forward_sums(monkeypatch, M, N, K, tiles):
-    C.case_gemm_forward_sums(DEV, monkeypatch, M, N, K, tiles)
+@pytest.mark.parametrize("M,N,K,b_oc,tiles", [(40, 1032, 1536, False, 17), (777, 2560, 2560, False, 0), (777, 2560, 3328, False, 0), (777, 7680, 2560, False, 17),
+                                              (1868, 2560, 2560, False, 0), (4500, 1536, 4096, False, 0), (200, 2560, 6656, False, 193), (4096, 2560, 2560, False, 18),
+                                              (777, 2560, 2560, True, 0), (777, 2560, 7680, True, 0), (777, 2560, 6656, True, 0), (64, 2560, 7680, True, 209),
+                                              (4096, 2560, 2560, True, 18)])
+def test_gemm_same_sums(monkeypatch, M, N, K, b_oc, tiles):
+    C.case_gemm_same_sums(DEV, monkeypatch, M, N, K, b_oc, tiles)
 
 
-@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 1664, True)])
+@pytest.mark.parametrize("M,N,K,b_oc", [(40, 1032, 2048, False), (130, 1024, 2048, True)])
 def test_gemm_four_waves_split(M, N, K, b_oc):
     """A reduction cut into pieces of whole stages, by the rule itself."""
     C.case_gemm_split_k_slabs(DEV, M, N, K, False, b_oc)
