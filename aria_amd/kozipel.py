@@ -182,9 +182,9 @@ class KozipelForCausalLM(nn.Module):
             logits = self._decode.run(batch)
             return logits if batch.every_row else logits[batch.wanted.long()]
         if self.dtype == f32 and trace is None and batch.seq is not None and table_batch(batch, self.device):
-            if self._decode is None or not self._decode.held.current():
+            if self._decode is None or not self._decode.held.current(self):
                 self._decode = _DecodeTables(self) if self._table_step() else None
-            if self._decode is not None and self._decode.held.plain():
+            if self._decode is not None and self._decode.held.plain(self):
                 return self._decode.run_f32(batch)
         x = torch.empty((T, self.width), dtype=f32, device=self.device)
         h = ops.rms_stream(x, c.width, c.eps, self.layers[c.runs[0].layer].norm1.weight, ids=batch.ids, table=self.embed, scale=c.embedding_scale)

@@ -57,18 +57,21 @@ class Held:
     is not ``plain``."""
 
     def __init__(self, model: nn.Module, shapes: dict, own: Sequence[tuple]):
-        self.modules, self.own, self.values, self.sizes, tensors, seen = [(m, type(m)) for m in model.modules()], own, [], [], [], set()
+        # (the model itself is not kept: it holds its table, and would live until cycles are collected)
+        self.modules, self.own, self.values, self.sizes, tensors, seen = [(m, type(m)) for m in model.modules() if m is not model], own, [], [], [], set()
+        self.model = type(model)
 
-        def look(container, items, of_module):
+        def look(container, items, of_module, name=None):
+            """name: the model's own container, by the attribute that it is"""
             if id(container) in seen:
                 return
             seen.add(id(container))
-            self.sizes.append((container, len(container)))
+            self.sizes.append((name or container, len(container)))
             for k, v in items:
                 if torch.is_tensor(v):
-                    tensors.append((container, k, v))
+                    tensors.append((name or container, k, v))
                     continue
-                self.values.append((container, k, v))
+                self.values.append((name or container, k, v))
                 if isinstance(v, list):
                     look(v, enumerate(v), False)
                 elif isinstance(v, dict) and of_module:          # (a module's sizes and offsets; what a config's entries were read from is not read again)
@@ -76,10 +79,11 @@ class Held:
                 elif type(v).__module__.startswith(__package__ + ".") and not isinstance(v, nn.Module):   # configs and caches
                     look(v.__dict__, v.__dict__.items(), False)
 
-        for m, _ in self.modules:
-            look(m.__dict__, [(k, v) for k, v in m.__dict__.items() if k[0] != "_" and k != "training"], True)
-            look(m._parameters, m._parameters.items(), False)
-            look(m._modules, m._modules.items(), False)
+        for m in model.modules():
+            for name in ("__dict__", "_parameters", "_modules"):
+                d = getattr(m, name)
+                items = [(k, v) for k, v in d.items() if k[0] != "_" and k != "training"] if name == "__dict__" else d.items()
+                look(d, items, name == "__dict__", name if m is model else None)
         self.tensors = [(*e, e[2].data_ptr(), e[2].shape) for e in tensors]
         device = next(model.parameters()).device
         self.fits = shapes_of(model) == shapes and all(t.dtype == f32 and t.is_contiguous() and t.device == device for _, _, t in tensors)
@@ -89,17 +93,19 @@ class Held:
         classes, names = {c for c, _, _ in own} | {nn.ModuleList, nn.ModuleDict}, {n for _, n, _ in own}
         return all(type(m) in classes and names.isdisjoint(m.__dict__) for m in modules) and all(c.__dict__.get(n) is f for c, n, f in own)
 
-    def current(self) -> bool:
+    def current(self, model: nn.Module) -> bool:
+        its = {name: getattr(model, name) for name in ("__dict__", "_parameters", "_modules")}
         try:
-            return (all(len(d) == n for d, n in self.sizes) and all(d[n] is v for d, n, v in self.values)
-                    and all(d[n] is t and t.data_ptr() == p and t.shape == s and t.is_contiguous() for d, n, t, p, s in self.tensors))
+            return (all(len(its[d] if type(d) is str else d) == n for d, n in self.sizes)
+                    and all((its[d] if type(d) is str else d)[n] is v for d, n, v in self.values)
+                    and all((its[d] if type(d) is str else d)[n] is t and t.data_ptr() == p and t.shape == s and t.is_contiguous() for d, n, t, p, s in self.tensors))
         except (KeyError, IndexError):
             return False
 
-    def plain(self) -> bool:
+    def plain(self, model: nn.Module) -> bool:
         """(a function put on a module itself is one entry more: not ``current``, and then not ``made_of`` its own)"""
         everywhere = nn.modules.module
-        if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks:
+        if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks or model._forward_hooks or model._forward_pre_hooks or type(model) is not self.model:
             return False
         return (self.fits and all(type(m) is c and not m._forward_hooks and not m._forward_pre_hooks for m, c in self.modules)
                 and all(c.__dict__.get(n) is f for c, n, f in self.own))

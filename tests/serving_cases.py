@@ -776,3 +776,26 @@ def case_stepped_model_copied(dev, cases, dtype):
     assert not torch.equal(steps(m)[1], want[1])
     for c in copies:
         assert all(torch.equal(x, y) for x, y in zip(steps(c), want))
+
+
+def case_stepped_model_released(dev, cases, dtype):
+    """A model that has made a step's tables is given back with its last reference, its memory with it, not when cycles are next collected."""
+    import gc
+    import weakref
+
+    from aria_amd.serving import StepBatch
+
+    cfg = cases.CONFIGS["mixed"]
+    m = cases.build(cfg, cases.checkpoint(cfg, seed=3), dev, dtype)
+    toks = cases.tokens(cfg, 12, seed=1)
+    m.setup_caches(1, 12)
+    for a, b in ((0, 5), (5, 6)):
+        m.step(StepBatch.build([toks[a:b]], [0], [a], None, dev))
+    held = [weakref.ref(t) for t in (m, *m.parameters())]
+    gc.collect()
+    gc.disable()
+    try:
+        del m
+        assert not any(r() is not None for r in held)
+    finally:
+        gc.enable()

@@ -174,3 +174,8 @@ def test_float32_step_asks_the_modules(monkeypatch, what):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_stepped_model_copied(dtype):
     S.case_stepped_model_copied(DEV, C, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_stepped_model_released(dtype):
+    S.case_stepped_model_released(DEV, C, dtype)
