@@ -131,8 +131,8 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
 // C[m][n] = sum_k X[m][k] W[n][k] in 32 bits, N <= 32 columns: the router's product of a mixture with up to 32 experts.
 // The choice of experts hangs on its last bits, so they are those of the general tiles: an element is one chain of v_mfma_f32_32x32x16_bf16 over the reduction, in `cut` pieces
 // for the rows from cut_row on, where those tiles would split it.  That chain (K / 16 products of one wave) and a block's own loads are the time; splitting the reduction
-// over the waves adds in another order and is ahead only where a block's own chain is longest (us: 5580 rows of 1536 on 32 columns 9.9, here 9.8, in a prompt's step 11.6 and 15.3; 16 384 rows 16.2, here 18.9;
-// 2000 rows of 3328 on 16 10.1, here 18.3).  The eight waves stage W once a block and X in rounds of 512 columns, the next round in flight in registers; the first wave multiplies.
+// over the waves adds in another order, at most twice as fast (us: 5580 rows of 1536 on 32 columns 9.9, here 9.8, in a prompt's step 11.6, here 15.3; 16 384 rows 16.2, here
+// 18.9; 2000 rows of 3328 on 16 columns 10.1, here 18.3).  The eight waves stage W once a block and X in rounds of 512 columns, the next round in flight in registers; the first wave multiplies.
 // 5580 rows of 1536 on 32 columns as 128 x 128 tiles of the general kernel 25.8 us.
 constexpr int XR = 512, XPITCH = XR + 8;   // (16 bytes: 16 rows' pieces lie on different banks)
 __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, float* C, int M, int N, int K, long long ldx, long long ldc, int cut_row,

@@ -156,7 +156,9 @@ class DuguzenForCausalLM(nn.Module):
 
     def _table_step(self) -> bool:
         """aria_latent_step_f32 takes the model as it is"""
-        own = [self.layer(i) for i in range(len(self.config.layers))] if Held.made_of(self.modules(), _OWN) else []
+        c, plain = self.config, Held.made_of(self.modules(), _OWN)
+        plain = plain and type(c) is DuguzenConfig and all(type(l) is DuguzenLayerConfig for l in c.layers) and all(type(k) is LatentCache for k in self.caches)
+        own = [self.layer(i) for i in range(len(c.layers))] if plain else []
         return (bool(own) and all(L.mixer.table_step and (L.mlp is None or L.mlp.table_step) for L in own)
                 and all(c.rows.shape == self.caches[0].rows.shape[:2] + c.rows.shape[2:] for c in self.caches))
 

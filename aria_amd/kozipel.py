@@ -20,7 +20,7 @@ import torch.nn as nn
 
 from . import hip, ops
 from .checkpoint import load_checkpoint_dir
-from .layers import ChunkAttention, Held, LinearAttention, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, functions_of, padded, shapes_of, table_batch, up8
+from .layers import ChunkAttention, ChunkCache, Held, LinearAttention, LinearState, MixerGroup, ReluGatedFeedForward, RmsNorm, _frozen, functions_of, padded, shapes_of, table_batch, up8
 from .registry import read_config
 
 bf16, f32 = torch.bfloat16, torch.float32
@@ -164,8 +164,9 @@ class KozipelForCausalLM(nn.Module):
 
     def _table_step(self) -> bool:
         """aria_mix_step_f32 takes the model as it is"""
-        return Held.made_of(self.modules(), _OWN) and all(L.mixer.table_step and L.mixer.parts[-1].eps == self.config.eps and (L.mlp is None or L.mlp.table_step)
-                                                          for L in self.layers)
+        c, plain = self.config, Held.made_of(self.modules(), _OWN)
+        plain = plain and type(c) is KozipelConfig and all(type(r) is KozipelRun for r in c.runs) and all(type(k) in (ChunkCache, LinearState) for run in self.caches for k in run)
+        return plain and all(L.mixer.table_step and L.mixer.parts[-1].eps == c.eps and (L.mlp is None or L.mlp.table_step) for L in self.layers)
 
     @torch.no_grad()
     def step(self, batch, trace: Optional[list] = None) -> torch.Tensor:

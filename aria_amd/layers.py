@@ -50,6 +50,9 @@ def functions_of(*classes: type) -> List[tuple]:
     return [(c, n, f) for c in classes for n, f in vars(c).items() if callable(f) or isinstance(f, property)]
 
 
+_CALL = nn.Module.__call__
+
+
 class Held:
     """What a float32 step's table of addresses was made from, compared before each step that runs by the table: every tensor, constant and module of a model, what its
     config and caches hold included.  The table's step runs no module and checks no shape: a model with hooks (its own or those of all modules), with modules
@@ -59,7 +62,7 @@ class Held:
     def __init__(self, model: nn.Module, shapes: dict, own: Sequence[tuple]):
         # (the model itself is not kept: it holds its table, and would live until cycles are collected)
         self.modules, self.own, self.values, self.sizes, tensors, seen = [(m, type(m)) for m in model.modules() if m is not model], own, [], [], [], set()
-        self.model = type(model)
+        self.model, self.plain_objects = type(model), []
 
         def look(container, items, of_module, name=None):
             """name: the model's own container, by the attribute that it is"""
@@ -77,6 +80,7 @@ class Held:
                 elif isinstance(v, dict) and of_module:          # (a module's sizes and offsets; what a config's entries were read from is not read again)
                     look(v, v.items(), False)
                 elif type(v).__module__.startswith(__package__ + ".") and not isinstance(v, nn.Module):   # configs and caches
+                    self.plain_objects.append((v, type(v)))
                     look(v.__dict__, v.__dict__.items(), False)
 
         for m in model.modules():
@@ -105,10 +109,12 @@ class Held:
     def plain(self, model: nn.Module) -> bool:
         """(a function put on a module itself is one entry more: not ``current``, and then not ``made_of`` its own)"""
         everywhere = nn.modules.module
-        if everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks or model._forward_hooks or model._forward_pre_hooks or type(model) is not self.model:
+        if nn.Module.__call__ is not _CALL or everywhere._global_forward_hooks or everywhere._global_forward_pre_hooks:
+            return False
+        if type(model) is not self.model or model._forward_hooks or model._forward_pre_hooks:
             return False
         return (self.fits and all(type(m) is c and not m._forward_hooks and not m._forward_pre_hooks for m, c in self.modules)
-                and all(c.__dict__.get(n) is f for c, n, f in self.own))
+                and all(type(v) is c for v, c in self.plain_objects) and all(c.__dict__.get(n) is f for c, n, f in self.own))
 
 
 def table_batch(batch, device) -> bool:

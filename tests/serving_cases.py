@@ -659,7 +659,7 @@ def case_registry():
 
 
 # what is done to a float32 model whose steps run by a table of addresses
-MODULES_CHANGED = ["subclass", "class", "instance", "wrapped", "global hook", "global pre hook", "config", "runs", "geometry", "attribute", "weight view"]
+MODULES_CHANGED = ["subclass", "class", "instance", "wrapped", "global hook", "global pre hook", "config", "runs", "geometry", "attribute", "weight view", "call", "config class"]
 
 
 def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
@@ -690,9 +690,13 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
         def forward(self, h):
             return twice_of(self.inner(h))
 
+    later, call = [], torch.nn.Module.__call__
+
     def change(m):
         mixer = layers(m)[0].mixer
-        if what == "subclass":
+        if what == "call":
+            monkeypatch.setattr(torch.nn.Module, "__call__", lambda mod, *a: twice_of(call(mod, *a)) if any(mod is layers(m)[0].mixer for m in models) else call(mod, *a))
+        elif what == "subclass":
             mixer.__class__ = type("Twice", (type(mixer),), dict(forward=twice))
         elif what == "class":
             monkeypatch.setattr(type(mixer), "forward", twice)
@@ -725,6 +729,12 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
                         setattr(part, name, new(getattr(part, name)))
         elif what == "weight view":
             m.head.data = m.head.data.flip(0)
+        elif what == "config class":   # (a constant that no entry of the object holds)
+            name = "residual_mult" if hasattr(m.config, "residual_mult") else "layers"
+            now, was = [2], getattr(m.config, name)
+            whole = property(lambda c: was[:now[0]] if name == "layers" else was * now[0], lambda c, v: None)
+            m.config.__class__ = type("Config", (type(m.config),), {name: whole})
+            later.append(lambda: now.__setitem__(0, 3))
 
     def hook(mod, args, out=None):   # (everything that a first mixer returns, or is given, doubled)
         if any(mod is layers(m)[0].mixer for m in models):
@@ -746,7 +756,11 @@ def case_float32_step_asks_the_modules(dev, monkeypatch, cases, what):
     elif what == "global pre hook":
         handle = everywhere.register_module_forward_pre_hook(hook)
     try:
-        assert not torch.equal(both(0, 5), before)
+        first = both(0, 5)
+        assert not torch.equal(first, before)
+        for f in later:
+            f()
+        assert not later or not torch.equal(both(0, 5), first)
         both(5, 8), both(8, 9)
     finally:
         if handle is not None:
