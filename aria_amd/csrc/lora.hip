@@ -131,8 +131,9 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
 // C[m][n] = sum_k X[m][k] W[n][k] in 32 bits, N <= 32 columns: the router's product of a mixture with up to 32 experts.
 // The choice of experts hangs on its last bits, so they are those of the general tiles: an element is one chain of v_mfma_f32_32x32x16_bf16 over the reduction, in `cut` pieces
 // for the rows from cut_row on, where those tiles would split it.  That chain (K / 16 products of one wave) and a block's own loads are the time; splitting the reduction
-// over the waves adds in another order, at most twice as fast (us: 5580 rows of 1536 on 32 columns 9.9, here 9.8, in a prompt's step 11.6, here 15.3; 16 384 rows 16.2, here
-// 18.9; 2000 rows of 3328 on 16 columns 10.1, here 18.3).  The eight waves stage W once a block and X in rounds of 512 columns, the next round in flight in registers; the first wave multiplies.
+// over the waves adds in another order and is hardly ahead (us: 5580 rows of 1536 on 32 columns 9.9, here 9.6, in a prompt's step 11.6, here 12.3; 16 384 rows 16.2, here 16.1;
+// 2000 rows of 3328 on 16 columns 10.1, here 15.2).  The eight waves stage W once a block and X in rounds of 512 columns, the next two in flight in registers (one: 15.3 in the
+// step); the first wave multiplies.
 // 5580 rows of 1536 on 32 columns as 128 x 128 tiles of the general kernel 25.8 us.
 constexpr int XR = 512, XPITCH = XR + 8;   // (16 bytes: 16 rows' pieces lie on different banks)
 __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, float* C, int M, int N, int K, long long ldx, long long ldc, int cut_row,
@@ -141,13 +142,14 @@ __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, cons
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), pitch = K + 8, nch = K / 64, m0 = blockIdx.x * ROWS, pieces = m0 >= cut_row ? cut : 1;
     bf16_t* xs = reinterpret_cast<bf16_t*>(lds);   // [32][XPITCH]
     bf16_t* ws = xs + ROWS * XPITCH;               // [N][pitch]
-    u32x4 x[4];
-    auto load = [&](int k0) __attribute__((always_inline)) {
+    u32x4 xa[4], xb[4];
+    auto load = [&](u32x4 (&x)[4], int k0) __attribute__((always_inline)) {
         if (k0 + 8 * l < K)
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[i] = ld16(X + (long long)min(m0 + w + 8 * i, M - 1) * ldx + k0 + 8 * l);   // (rows past the end: the last one, never stored)
     };
-    load(0);
+    load(xa, 0);
+    load(xb, XR);
 #pragma unroll 6
     for (int i = t; i < N * K / 8; i += 512) st16(ws + i / (K / 8) * pitch + 8 * (i % (K / 8)), ld16(W + 8ll * i));
     f32x16 acc, sum;
@@ -155,10 +157,10 @@ __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, cons
     for (int j = 0; j < 16; ++j) acc[j] = sum[j] = 0.f;
     const bf16_t *xf = xs + (l & 31) * XPITCH + 8 * (l >> 5), *wf = ws + min(l & 31, N - 1) * pitch + 8 * (l >> 5);
     int piece = 0;
-    for (int c0 = 0; c0 < nch; c0 += XR / 64) {
+    auto round = [&](u32x4 (&x)[4], int c0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) st16(xs + (w + 8 * i) * XPITCH + 8 * l, x[i]);
-        load(64 * c0 + XR);
+        load(x, 64 * c0 + 2 * XR);
         sync();
         if (w == 0) {
 #pragma unroll
@@ -176,6 +178,10 @@ __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, cons
             }
         }
         sync();
+    };
+    for (int c0 = 0; c0 < nch; c0 += 2 * XR / 64) {
+        round(xa, c0);
+        if (c0 + XR / 64 < nch) round(xb, c0 + XR / 64);
     }
     if (w || m0 + (l & 31) >= M) return;
     float* out = C + (long long)(m0 + (l & 31)) * ldc + 4 * (l >> 5);   // (a lane: a row, columns 8 q + 4 (l / 32) .. + 3)

@@ -1175,7 +1175,7 @@ def _f32(t: torch.Tensor) -> int:
 
 def thin_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
     """A router's product, whose 8 .. 32 columns fill a quarter of a tile at most: the thin kernel, factor staged on chip (5580 rows of 1536 on 32 columns as 128 x 128
-    tiles 25.8 us, there 9.8), with the tiles' bits.  Results of 16 bits stay with the tiles: the fused router's are theirs, bit for bit."""
+    tiles 25.8 us, there 9.6), with the tiles' bits.  Results of 16 bits stay with the tiles: the fused router's are theirs, bit for bit."""
     N, K = w.shape
     return (N in (8, 16, 24, 32) and K % 64 == 0 and N * (K + 32) <= 57344 and w.dtype == a.dtype == bf16 and w.is_contiguous() and a.dim() == 2 and a.shape[1] == K
             and a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and a.shape[0] > 0)
