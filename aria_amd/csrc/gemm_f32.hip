@@ -1,15 +1,17 @@
 // C = A W^T in true 32-bit (v_mfma_f32_16x16x4_f32: 32-bit products, 32-bit sums, 256 multiply-adds a cycle and CU -- twice the vector pipe's unpacked rate).
 //
-// Both operands are k-contiguous, so fragments come straight from global memory: a lane loads 16 bytes of a row, four multiply steps whose reduction
-// indices are whatever the four lanes of a row hold -- the same for both operands.  A workgroup computes a tile of 16 MT x 16 NT outputs, its NW waves on
-// interleaved 16-column steps of the reduction, DEPTH steps in flight; the partial tiles meet in LDS once.  Splitting the REDUCTION over the waves is what
-// fills the chip where a serving step has a few rows only (1 .. 16 rows of a 1024-wide layer are 16 tiles of 64 columns: 100 us a launch as one 64 x 64
-// tile per workgroup with its waves side by side), and costs one pass over the tile in LDS.
-// M x N x K, us as one 64 x 64 tile a workgroup on the vector pipe / now (relative error against 64 bits 5.7e-7 / 2.1e-7 at K = 1024): 4 x 2112 x 1024 57 / 10,
-// 4 x 32000 x 1024 73 / 28, 16 x 1024 x 2816 152 / 12, 300 x 1024 x 1024 59 / 15, 883 x 1024 x 2816 176 / 76, 4096^3 1786 / 1480; 16 experts of 768 x 1024: 8
-// rows 58 / 10, 1240 rows 136 / 43.  Tiles (rows x columns, waves): 16 x 16 x 8 up to 16 rows, where the weights' stream bounds it; 32 x 32 x 4 up to 64 rows, and
-// for experts up to 128; 64 x 32 x 4 (620 x 2112 x 1024: 47 us, 32 x 32 x 4 49, 64 x 64 x 4 54); 64 x 64 x 4 from 512 tiles, where the L2's rate counts (4096^3:
-// 1480 us, 64 x 32 x 4 1650).
+// Both operands are k-contiguous: a lane loads 16 bytes of a row, four multiply steps whose reduction indices are whatever the four lanes of a row hold -- the same for
+// both operands.
+//
+// Few outputs (gemm_f32_kernel): fragments straight from global memory.  A workgroup computes a tile of 16 MT x 16 NT outputs, its NW waves on interleaved 16-column
+// steps of the reduction, DEPTH steps in flight; the partial tiles meet in LDS once.  Splitting the REDUCTION over the waves is what fills the chip where a
+// serving step has a few rows only (1 .. 16 rows of a 1024-wide layer are 16 tiles of 64 columns: 100 us a launch as one 64 x 64 tile per workgroup with its
+// waves side by side), and costs one pass over the tile in LDS.  16 x 16 x 8 waves up to 16 rows, where the weights' stream bounds it; 32 x 32 x 4 up to a round of tiles.
+//
+// More (gemm_f32_tiles_kernel): stages in the LDS.  Read from global memory, the half lines of a 16-column step are fetched from the L2 twice, which bound those tiles.
+// M x N x K, us with the reduction over the waves (64 x 32 a workgroup) / by stages: 883 x 2112 x 1024 61 / 44, 883 x 2816 x 1024 77 / 53, 883 x 1024 x 2816 74 / 59,
+// 1200 x 5632 x 1024 169 / 133, 2048^3 191 / 150; 16 experts of 768 x 1024, 1766 rows 50 / 36, 600 rows 26 / 20.  What is left: a tile of 64 x 64 alone takes 24 us for a
+// reduction of 1024, 18 of them products (one wave a SIMD multiplies 94 .. 115 TFLOP/s with 16x16x4, two 113 .. 131), and whole rounds of tiles.
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "elem.h"
@@ -54,13 +56,12 @@ __device__ __forceinline__ bool find_rows(const GemmF32& p, int y, int rows, int
     return false;
 }
 
-template <int MT, int NT, int NW, bool HEADS>
-__global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p, Heads hd) {
-    constexpr int DEPTH = MT + NT > 4 ? 2 : 4, TM = 16 * MT, TN = 16 * NT;
+template <int MT, int NT, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
+    constexpr int DEPTH = 4, TM = 16 * MT, TN = 16 * NT;
     ARIA_SMEM_STATIC float red[NW][TM][TN + 1];
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15;
-    if (HEADS) p.A += (long long)blockIdx.y * p.K, p.W += blockIdx.y * p.strideW, p.C += (long long)blockIdx.y * hd.cols;
-    const unsigned ntn = unsigned((HEADS ? hd.cols : p.N) + TN - 1) / TN;
+    const unsigned ntn = unsigned(p.N + TN - 1) / TN;
     const int y = int(blockIdx.x / ntn), n0 = int(blockIdx.x % ntn) * TN;
     int m0 = y * TM, m_end = p.M, e = 0;
     if (p.offsets && !find_rows(p, y, TM, e, m0, m_end)) return;
@@ -140,13 +141,153 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p, Heads hd) 
         float v = 0.f;
 #pragma unroll
         for (int ww = 0; ww < NW; ++ww) v += red[ww][m][n];
-        if (HEADS) {
-            if (m0 + m < m_end && n0 + n < hd.cols) {
-                const float sum = hd.ml[((long long)(m0 + m) * hd.H + blockIdx.y) * 2 + 1], z = hd.gate[(m0 + m) * hd.ldg + blockIdx.y];
-                p.C[(long long)(m0 + m) * p.ldc + n0 + n] = n0 + n < p.N ? v / sum * sigmoid_exact(z) : 0.f;
+        if (m0 + m < m_end && n0 + n < p.N) p.C[(long long)(m0 + m) * p.ldc + n0 + n] = v;
+    }
+}
+
+// Tiles of 32 MI x 32 NI outputs, 2 x 2 waves of 16 MI x 16 NI, both operands through the LDS: stages of 32 columns (whole lines of 128 bytes), four of them, filled
+// by LDS-DMA.  The sums are gemm_f32_kernel's with four waves, bit for bit: a wave keeps four accumulators an output, for the 16-column steps 0, 4, 8 .., 1, 5, .. and
+// so on, and adds them up in that order.
+// A piece of 16 bytes of row r lies at slot (piece ^ (r >> 1 & 7)) of the row's 128 bytes: 16 lanes that read one piece of 16 rows touch every bank once.
+template <int MI, int NI, bool HEADS>
+__global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd, int vec) {
+    constexpr int BM = 32 * MI, BN = 32 * NI, STAGE = (BM + BN) * 128, P = MI + NI;   // P: pieces of a wave a stage
+    ARIA_DYN_SMEM(smem);
+    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15, wm = w >> 1, wn = w & 1;
+    if (HEADS) p.A += (long long)blockIdx.y * p.K, p.W += blockIdx.y * p.strideW, p.C += (long long)blockIdx.y * hd.cols;
+    const int cols = HEADS ? hd.cols : p.N;
+    const unsigned ntn = unsigned(cols + BN - 1) / BN;
+    const int y = int(blockIdx.x / ntn), n0 = int(blockIdx.x % ntn) * BN;
+    int m0 = y * BM, m_end = p.M, e = 0;
+    if (p.offsets && !find_rows(p, y, BM, e, m0, m_end)) return;
+    // this lane's pieces of a stage: rows 8 (w + 4 i) + l / 8 of [A's rows, W's rows], rows behind the end the last one again
+    const float* src[P];
+    int at[P];   // its column
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int r = 8 * (w + 4 * i) + (l >> 3);
+        at[i] = ((l & 7) ^ (r >> 1 & 7)) * 4;
+        src[i] = r < BM ? p.A + (long long)min(m0 + r, m_end - 1) * p.lda : p.W + e * p.strideW + (long long)min(n0 + r - BM, p.N - 1) * p.ldw;
+    }
+    auto piece = [&](int s, int i) __attribute__((always_inline)) {   // of stage s (columns behind the row's end: its first ones; never used)
+        const int k = 32 * s + at[i];
+        glds16_raw(src[i] + (k < p.K ? k : 0), smem + (s & 3) * STAGE + (w + 4 * i) * 1024);
+    };
+    f32x4 acc[4][MI][NI];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int n = (p.K + 31) / 32, turn = c16 >> 1 & 7;
+    const char *arow = smem + (wm * 16 * MI + c16) * 128, *brow = smem + (BM + wn * 16 * NI + c16) * 128;
+    struct Half {   // 16 columns of a wave's rows
+        f32x4 a[MI], b[NI];
+    };
+    auto load = [&](Half& f, int s, int half) __attribute__((always_inline)) {
+        const int o = (s & 3) * STAGE + ((4 * half + q4) ^ turn) * 16;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) f.a[i] = *reinterpret_cast<const f32x4*>(arow + o + i * 2048);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) f.b[j] = *reinterpret_cast<const f32x4*>(brow + o + j * 2048);
+        sched_fence();   // (left alone the compiler moves the reads down to their use)
+    };
+    // the products of 16 columns, and between them the requests of stage s (none behind the last one)
+    auto use = [&](const Half& f, f32x4(&sum)[MI][NI], int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j) sum[i][j] = mfma16_f32(f.b[j][c], f.a[i][c], sum[i][j]);   // (a lane: row c16, columns 4 q4 .. + 3)
+            if (c < P && s < n) piece(s, c);
+        }
+        sched_fence();
+    };
+    auto arrive = [&](int s) __attribute__((always_inline)) {   // stage s is there for all waves, stage s - 1 is free
+        if (s == 0 && n > 3)
+            wait_vm<3 * P>();
+        else if (s + 2 < n)
+            wait_vm<2 * P>();
+        else if (s + 1 < n)
+            wait_vm<P>();
+        else
+            wait_vm<0>();
+        wait_lds();
+        raw_barrier();
+    };
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < P; ++i)
+            if (s < n) piece(s, i);
+    arrive(0);
+    int s = 0;
+    const int whole = p.K / 64 * 2;
+    if (whole) {
+        Half f0, f1;
+        load(f0, 0, 0);
+        for (; s < whole; s += 2) {   // (every read one set of products ahead of its use; behind the last stage it finds an old one's, which nothing uses)
+            load(f1, s, 1);
+            use(f0, acc[0], n);
+            arrive(s + 1);
+            load(f0, s + 1, 0);
+            use(f1, acc[1], s + 4);
+            load(f1, s + 1, 1);
+            use(f0, acc[2], n);
+            arrive(s + 2);
+            load(f0, s + 2, 0);
+            use(f1, acc[3], s + 5);
+        }
+    }
+    if (s < n) {   // the rest of the rows: at most 60 columns
+        const int rest = p.K - 32 * s;
+        auto step = [&](int s, int half, f32x4(&sum)[MI][NI], int left) __attribute__((always_inline)) {   // left: columns that the rows have from here
+            if (left <= 0) return;
+            Half f;
+            load(f, s, half);
+            if (4 * q4 >= left) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) f.a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < NI; ++j) f.b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
-        } else if (m0 + m < m_end && n0 + n < p.N) {
-            p.C[(long long)(m0 + m) * p.ldc + n0 + n] = v;
+            use(f, sum, n);
+        };
+        step(s, 0, acc[0], rest);
+        step(s, 1, acc[1], rest - 16);
+        if (rest > 32) {
+            arrive(s + 1);
+            step(s + 1, 0, acc[2], rest - 32);
+            step(s + 1, 1, acc[3], rest - 48);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int m = m0 + 16 * (wm * MI + i) + c16;
+        if (m >= m_end) continue;
+        float sum = 1.f, z = 0.f;
+        if (HEADS) sum = hd.ml[((long long)m * hd.H + blockIdx.y) * 2 + 1], z = sigmoid_exact(hd.gate[m * hd.ldg + blockIdx.y]);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int c0 = n0 + 16 * (wn * NI + j) + 4 * q4;
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[r] += acc[c][i][j][r];
+                if (HEADS) v[r] = c0 + r < p.N ? v[r] / sum * z : 0.f;
+            }
+            float* to = p.C + (long long)m * p.ldc + c0;
+            if (vec && c0 + 3 < cols) {
+                *reinterpret_cast<f32x4*>(to) = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (c0 + r < cols) to[r] = v[r];
+            }
         }
     }
 }
@@ -156,7 +297,18 @@ int launch_f32(const GemmF32& p, void* stream) {
     const int64_t ntm = (int64_t(p.M) + 16 * MT - 1) / (16 * MT) + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
     const int64_t ntn = (int64_t(p.N) + 16 * NT - 1) / (16 * NT);
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
-    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, false>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p, Heads{});
+    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
+    return aria_check_launch();
+}
+
+template <int MI, int NI, bool HEADS>
+int launch_f32_tiles(const GemmF32& p, const Heads& hd, void* stream) {
+    constexpr int BM = 32 * MI, BN = 32 * NI;
+    const int64_t ntm = (int64_t(p.M) + BM - 1) / BM + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
+    const int64_t ntn = ((HEADS ? hd.cols : p.N) + BN - 1) / BN;
+    if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
+    const int vec = !(p.ldc & 3) && !(reinterpret_cast<uintptr_t>(p.C) & 15) && !(HEADS && (hd.cols & 3));
+    ARIA_LAUNCH((gemm_f32_tiles_kernel<MI, NI, HEADS>), dim3(unsigned(ntm * ntn), unsigned(HEADS ? hd.H : 1)), dim3(256), 4 * (BM + BN) * 128, stream, p, hd, vec);
     return aria_check_launch();
 }
 
@@ -166,8 +318,8 @@ __attribute__((visibility("hidden"))) int aria_gemm_f32_heads(const float* part_
                                                               int64_t T, void* stream) {
     const GemmF32 p{part_o, uv, out, int(T), int(s.dv), int(s.R), (long long)(s.H * s.R), (long long)s.rp, (long long)(s.H * s.dvp), nullptr, 1, (long long)(s.dv * s.rp)};
     const Heads hd{part_ml, proj + s.g_off, (long long)s.ldp, int(s.H), int(s.dvp)};
-    ARIA_LAUNCH((gemm_f32_kernel<4, 2, 4, true>), dim3(unsigned((T + 63) / 64 * ((s.dvp + 31) / 32)), unsigned(s.H)), dim3(256), 0, stream, p, hd);
-    return aria_check_launch();
+    // (883 tokens, 8 heads of 128 x 256, us: 64 x 32 with the reduction over the waves 13.3, tiles of 32 x 32 10.9, 32 x 64 10.4, 64 x 64 11.6)
+    return launch_f32_tiles<1, 2, true>(p, hd, stream);
 }
 
 extern "C" {
@@ -179,11 +331,16 @@ int aria_gemm_f32(const float* A, const float* W, float* C, int64_t M, int64_t N
     if (M == 0 || N == 0) return ARIA_OK;
     if ((M + 63) / 64 > 65535 || E > 65535) return ARIA_ERR_UNSUPPORTED;
     const GemmF32 p{A, W, C, int(M), int(N), int(K), (long long)lda, (long long)ldw, (long long)ldc, (const int*)offsets, int(offsets ? E : 1), (long long)strideW};
-    const int64_t rows = offsets ? (M + E - 1) / E : M;   // of an expert on average
-    const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64);
-    if (rows <= 16) return launch_f32<1, 1, 8>(p, stream);
-    if (rows <= (offsets ? 128 : 64)) return launch_f32<2, 2, 4>(p, stream);
-    return tiles < 512 ? launch_f32<4, 2, 4>(p, stream) : launch_f32<4, 4, 4>(p, stream);
+    if (offsets ? M <= 16 * E : M <= 16) return launch_f32<1, 1, 8>(p, stream);
+    // Up to a round of 32 x 32 tiles the reduction over the waves is the shorter chain (48 x 1024 x 2816: 22 us, 24 with stages).  Beyond it the rounds of the chip
+    // decide, and of equal ones the larger tile (883 x 2112 x 1024, us as 64 x 64 / 32 x 64 / 32 x 32: 44 / 47 / 48; 883 x 2816 x 1024 61 / 53 / 55; 300 x 2112 x 1024
+    // 24 / 25 / 20).  An expert's last tile stands half empty on average.
+    auto tiles = [&](int mi, int ni) { return ((M + 32 * mi - 1) / (32 * mi) + (offsets ? E / 2 : 0)) * ((N + 32 * ni - 1) / (32 * ni)); };
+    if (tiles(1, 1) <= 256) return launch_f32<2, 2, 4>(p, stream);
+    auto cost = [&](int mi, int ni, int more) { return (tiles(mi, ni) + 255) / 256 * mi * ni * (100 + more); };
+    const int64_t c22 = cost(2, 2, 0), c12 = cost(1, 2, 5), c11 = cost(1, 1, 10);
+    if (c22 <= c12 && c22 <= c11) return launch_f32_tiles<2, 2, false>(p, {}, stream);
+    return c12 <= c11 ? launch_f32_tiles<1, 2, false>(p, {}, stream) : launch_f32_tiles<1, 1, false>(p, {}, stream);
 }
 
 }  // extern "C"

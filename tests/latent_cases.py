@@ -235,6 +235,24 @@ def case_gemm_f32(dev, M, N, K):
     assert rel(ops.grouped_linear_any(a.to(dev), we.to(dev), off), want) < 2e-6
 
 
+def case_gemm_f32_tiles(dev, M, N, K):
+    """More than a round of 32 x 32 outputs: the stages' kernel.  Its sums are those of the kernel for few outputs, bit for bit, whichever tiles hold them."""
+    from aria_amd import ops
+
+    a, w = rnd(M, K, seed=1, dtype=f32).to(dev), rnd(3, N, K, seed=2, dtype=f32).to(dev)
+    assert (M + 31) // 32 * ((N + 31) // 32) > 256
+    got = ops.linear_any(a, w[1])
+    assert rel(got, a.double().cpu() @ w[1].double().cpu().T) < 2e-6
+    first = M // 3
+    off = torch.tensor([0, first, first, M], dtype=torch.int32, device=dev)
+    by_expert = ops.grouped_linear_any(a, w, off)
+    few = min(256 // ((N + 31) // 32) * 32, M // 3)
+    assert few > 16
+    for rows, expert in ((slice(0, few), 0), (slice(first, first + few), 2), (slice(M - few, M), 2)):
+        assert torch.equal(got[rows], ops.linear_any(a[rows], w[1])), rows
+        assert torch.equal(by_expert[rows], ops.linear_any(a[rows], w[expert])), rows
+
+
 def case_route_groups(dev, T, E, groups, keep, k):
     from aria_amd import ops
 

@@ -44,6 +44,11 @@ def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(560, 481, 20), (1030, 260, 100)])
+def test_gemm_f32_tiles(M, N, K):
+    C.case_gemm_f32_tiles(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("E,groups,keep,k", [(8, 2, 1, 2), (12, 4, 2, 3), (6, 1, 1, 1), (8, 8, 3, 3), (100, 10, 4, 12)])
 def test_route_groups(E, groups, keep, k):
     C.case_route_groups(DEV, 9, E, groups, keep, k)

@@ -48,6 +48,11 @@ def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(560, 481, 4), (600, 484, 36), (1030, 322, 64), (883, 319, 1020), (1500, 190, 2816), (2500, 128, 128), (40000, 96, 52)])   # the last stage's remainders
+def test_gemm_f32_tiles(M, N, K):
+    C.case_gemm_f32_tiles(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("E,groups,keep,k", [(8, 2, 1, 2), (12, 4, 2, 3), (6, 1, 1, 1), (8, 8, 3, 3), (64, 8, 3, 6), (100, 10, 4, 12), (256, 8, 4, 8)])
 def test_route_groups(E, groups, keep, k):
     C.case_route_groups(DEV, 200, E, groups, keep, k)
