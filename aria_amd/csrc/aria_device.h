@@ -254,11 +254,21 @@ __device__ __forceinline__ f32x16 mfma32(s16x8 a, s16x8 b, f32x16 c) {
 // v_mfma_f32_16x16x4_f32, true 32-bit: a = A[l & 15][l >> 4], b = B[l >> 4][l & 15]; the result lies as mfma16's
 __device__ __forceinline__ f32x4 mfma16_f32(float a, float b, f32x4 c) {
 #ifdef ARIA_EMU
+    struct AB { float a, b; };
+    AB mine{a, b};
+    emu::WaveBuf& w = emu::wbuf();
     const int l = emu::lane();
+    std::memcpy(w.slot[l], &mine, sizeof(AB));
+    emu::wave_sync();
     for (int k = 0; k < 4; ++k) {
-        const float bk = emu::shfl(b, 16 * k + (l & 15));
-        for (int r = 0; r < 4; ++r) c[r] = std::fma(emu::shfl(a, 16 * k + 4 * (l >> 4) + r), bk, c[r]);
+        AB rb, ra;
+        std::memcpy(&rb, w.slot[16 * k + (l & 15)], sizeof(AB));
+        for (int r = 0; r < 4; ++r) {
+            std::memcpy(&ra, w.slot[16 * k + 4 * (l >> 4) + r], sizeof(AB));
+            c[r] = std::fma(ra.a, rb.b, c[r]);
+        }
     }
+    emu::wave_sync();
     return c;
 #else
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
