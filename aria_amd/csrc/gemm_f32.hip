@@ -15,20 +15,14 @@
 #include "aria_device.h"
 #include "aria_hip.h"
 #include "elem.h"
+#include "gemm_f32.h"
 #include <algorithm>
 
 namespace {
 using namespace ad;
 
-struct GemmF32 {
-    const float *A, *W;
-    float* C;
-    int M, N, K;
-    long long lda, ldw, ldc;
-    const int* offsets;   // rows grouped by expert, or NULL
-    int E;
-    long long strideW;
-};
+typedef AriaGemmF32 GemmF32;
+constexpr int FIN_HEADS = 4;   // beside gemm_f32.h's
 // a product a head (blockIdx.y) of the latent attention's expansion: the result's row t of head h times its output gate over its softmax sum
 struct Heads {
     const float *ml, *gate;   // [T, H, 2] (maximum, sum), gate logits [T, ldg]
@@ -56,102 +50,141 @@ __device__ __forceinline__ bool find_rows(const GemmF32& p, int y, int rows, int
     return false;
 }
 
-template <int MT, int NT, int NW>
+// the row of A that row m of the result comes from
+__device__ __forceinline__ long long row_of(const GemmF32& p, int m) { return p.rows ? p.rows[m] / p.per : m; }
+
+// What becomes of a sum (v2: the second weight's): as the launches of their own would have it, act_rows_kernel and dyt_stream_kernel
+template <int FIN>
+__device__ __forceinline__ float finished(const GemmF32& p, float v, float v2) {
+    if (FIN == ARIA_F32_RELU2) return relu_squared(v);
+    if (FIN == ARIA_F32_PAIR) return (p.relu_gate ? fmaxf(v, 0.f) : v * sigmoid_exact(v)) * v2;
+    return v;
+}
+__device__ __forceinline__ void stream_step(const GemmF32& p, float v, float& x, float& h, int n) {
+    x += dyt<float>(p.post, v, n);
+    if (p.next.w) h = dyt<float>(p.next, x, n);
+}
+
+template <int MT, int NT, int NW, int FIN>
 __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
+    constexpr bool PAIR = FIN == ARIA_F32_PAIR;
+    constexpr int WS = PAIR ? 2 : 1;
     constexpr int DEPTH = 4, TM = 16 * MT, TN = 16 * NT;
-    ARIA_SMEM_STATIC float red[NW][TM][TN + 1];
+    ARIA_SMEM_STATIC float red[WS][NW][TM][TN + 1];
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15;
     const unsigned ntn = unsigned(p.N + TN - 1) / TN;
     const int y = int(blockIdx.x / ntn), n0 = int(blockIdx.x % ntn) * TN;
     int m0 = y * TM, m_end = p.M, e = 0;
     if (p.offsets && !find_rows(p, y, TM, e, m0, m_end)) return;
-    const float *ap[MT], *wp[NT];
+    const float *ap[MT], *wp[WS][NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) ap[i] = p.A + (long long)min(m0 + 16 * i + c16, m_end - 1) * p.lda;
+    for (int i = 0; i < MT; ++i) ap[i] = p.A + row_of(p, min(m0 + 16 * i + c16, m_end - 1)) * p.lda + w * 16 + q4 * 4;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wp[j] = p.W + e * p.strideW + (long long)min(n0 + 16 * j + c16, p.N - 1) * p.ldw;
-    f32x4 acc[MT][NT];
+    for (int z = 0; z < WS; ++z)
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+        for (int j = 0; j < NT; ++j) wp[z][j] = (z ? p.W2 : p.W) + e * p.strideW + (long long)min(n0 + 16 * j + c16, p.N - 1) * p.ldw + w * 16 + q4 * 4;
+    f32x4 acc[WS][MT][NT];
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < WS; ++z)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[z][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int steps = p.K / 16, mine = (steps - w + NW - 1) / NW;   // whole steps; this wave's: w, w + NW, ...
-#pragma unroll
-    for (int i = 0; i < MT; ++i) ap[i] += w * 16 + q4 * 4;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) wp[j] += w * 16 + q4 * 4;
-    f32x4 a[DEPTH][MT], b[DEPTH][NT];
-    auto load = [&](int s, f32x4(&av)[MT], f32x4(&bv)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) av[i] = *reinterpret_cast<const f32x4*>(ap[i] + s * NW * 16);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) bv[j] = *reinterpret_cast<const f32x4*>(wp[j] + s * NW * 16);
+    struct Step {
+        f32x4 a[MT], b[WS][NT];
     };
-    auto use = [&](const f32x4(&av)[MT], const f32x4(&bv)[NT]) __attribute__((always_inline)) {
+    Step x[DEPTH];
+    auto load = [&](long long k, Step& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) f.a[i] = *reinterpret_cast<const f32x4*>(ap[i] + k);
+#pragma unroll
+        for (int z = 0; z < WS; ++z)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) f.b[z][j] = *reinterpret_cast<const f32x4*>(wp[z][j] + k);
+    };
+    auto use = [&](const Step& f) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+            for (int z = 0; z < WS; ++z)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = mfma16_f32(av[i][c], bv[j][c], acc[i][j]);
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[z][i][j] = mfma16_f32(f.a[i][c], f.b[z][j][c], acc[z][i][j]);
     };
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u)
-        if (u < mine) load(u, a[u], b[u]);
+        if (u < mine) load(u * NW * 16, x[u]);
     int s = 0;
     for (; s + 2 * DEPTH <= mine; s += DEPTH) {
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
-            use(a[u], b[u]);
-            load(s + u + DEPTH, a[u], b[u]);
+            use(x[u]);
+            load((s + u + DEPTH) * NW * 16, x[u]);
         }
     }
     for (; s < mine; s += DEPTH) {   // the last DEPTH .. 2 DEPTH - 1 steps (or fewer altogether)
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
             if (s + u >= mine) break;
-            use(a[u], b[u]);
-            if (s + u + DEPTH < mine) load(s + u + DEPTH, a[u], b[u]);
+            use(x[u]);
+            if (s + u + DEPTH < mine) load((s + u + DEPTH) * NW * 16, x[u]);
         }
     }
     if ((p.K & 15) && w == steps % NW) {   // the rest of the row, K % 16 = 4, 8 or 12 columns: lanes behind it hold zeros in both operands
         const bool in = q4 * 4 < (p.K & 15);
-        const int back = in ? mine * NW * 16 : -(w * 16 + q4 * 4);   // (a column of the same row)
+        load(in ? mine * NW * 16 : -(w * 16 + q4 * 4), x[0]);   // (not in: a column of the same row)
+        if (!in) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            a[0][i] = *reinterpret_cast<const f32x4*>(ap[i] + back);
-            if (!in) a[0][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+            for (int i = 0; i < MT; ++i) x[0].a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            b[0][j] = *reinterpret_cast<const f32x4*>(wp[j] + back);
-            if (!in) b[0][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int z = 0; z < WS; ++z)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) x[0].b[z][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        use(a[0], b[0]);
+        use(x[0]);
     }
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int z = 0; z < WS; ++z)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red[w][16 * i + 4 * q4 + r][16 * j + c16] = acc[i][j][r];
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) red[z][w][16 * i + 4 * q4 + r][16 * j + c16] = acc[z][i][j][r];
     sync();
     for (int i = t; i < TM * TN; i += NW * 64) {
         const int m = i / TN, n = i % TN;
-        float v = 0.f;
+        float v[2] = {0.f, 0.f};
 #pragma unroll
-        for (int ww = 0; ww < NW; ++ww) v += red[ww][m][n];
-        if (m0 + m < m_end && n0 + n < p.N) p.C[(long long)(m0 + m) * p.ldc + n0 + n] = v;
+        for (int z = 0; z < WS; ++z)
+#pragma unroll
+            for (int ww = 0; ww < NW; ++ww) v[z] += red[z][ww][m][n];
+        if (m0 + m >= m_end || n0 + n >= p.N) continue;
+        const long long to = (long long)(m0 + m) * p.ldc + n0 + n;
+        if (FIN == ARIA_F32_STREAM) {
+            float xv = p.x[to], h = 0.f;
+            stream_step(p, v[0], xv, h, n0 + n);
+            p.x[to] = xv;
+            if (p.next.w) p.C[to] = h;
+        } else {
+            p.C[to] = finished<FIN>(p, v[0], v[1]);
+        }
     }
 }
 
 // Tiles of 32 MI x 32 NI outputs, 2 x 2 waves of 16 MI x 16 NI, both operands through the LDS: stages of 32 columns (whole lines of 128 bytes), four of them, filled
 // by LDS-DMA.  The sums are gemm_f32_kernel's with four waves, bit for bit: a wave keeps four accumulators an output, for the 16-column steps 0, 4, 8 .., 1, 5, .. and
 // so on, and adds them up in that order.
+// PAIR: two weights, BN rows of each in a stage.
 // A piece of 16 bytes of row r lies at slot (piece ^ (r >> 1 & 7)) of the row's 128 bytes: 16 lanes that read one piece of 16 rows touch every bank once.
-template <int MI, int NI, bool HEADS>
+template <int MI, int NI, int FIN>
 __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd, int vec) {
-    constexpr int BM = 32 * MI, BN = 32 * NI, STAGE = (BM + BN) * 128, P = MI + NI;   // P: pieces of a wave a stage
+    constexpr bool HEADS = FIN == FIN_HEADS;
+    constexpr int WS = FIN == ARIA_F32_PAIR ? 2 : 1, NB = WS * NI;   // NB: blocks of 16 weight rows of a wave, the second weight's behind the first's
+    constexpr int BM = 32 * MI, BN = 32 * NI, STAGE = (BM + WS * BN) * 128, P = MI + NB;   // P: pieces of a wave a stage
+    static_assert(P <= 8, "requested between the four sets of products");
     ARIA_DYN_SMEM(smem);
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15, wm = w >> 1, wn = w & 1;
     if (HEADS) p.A += (long long)blockIdx.y * p.K, p.W += blockIdx.y * p.strideW, p.C += (long long)blockIdx.y * hd.cols;
@@ -167,41 +200,43 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd
     for (int i = 0; i < P; ++i) {
         const int r = 8 * (w + 4 * i) + (l >> 3);
         at[i] = ((l & 7) ^ (r >> 1 & 7)) * 4;
-        src[i] = r < BM ? p.A + (long long)min(m0 + r, m_end - 1) * p.lda : p.W + e * p.strideW + (long long)min(n0 + r - BM, p.N - 1) * p.ldw;
+        const int rw = r < BM + BN ? r - BM : r - BM - BN;
+        src[i] = r < BM ? p.A + row_of(p, min(m0 + r, m_end - 1)) * p.lda : (r < BM + BN ? p.W : p.W2) + e * p.strideW + (long long)min(n0 + rw, p.N - 1) * p.ldw;
     }
     auto piece = [&](int s, int i) __attribute__((always_inline)) {   // of stage s (columns behind the row's end: its first ones; never used)
         const int k = 32 * s + at[i];
         glds16_raw(src[i] + (k < p.K ? k : 0), smem + (s & 3) * STAGE + (w + 4 * i) * 1024);
     };
-    f32x4 acc[4][MI][NI];
+    f32x4 acc[4][MI][NB];
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NI; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NB; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int n = (p.K + 31) / 32, turn = c16 >> 1 & 7;
     const char *arow = smem + (wm * 16 * MI + c16) * 128, *brow = smem + (BM + wn * 16 * NI + c16) * 128;
     struct Half {   // 16 columns of a wave's rows
-        f32x4 a[MI], b[NI];
+        f32x4 a[MI], b[NB];
     };
     auto load = [&](Half& f, int s, int half) __attribute__((always_inline)) {
         const int o = (s & 3) * STAGE + ((4 * half + q4) ^ turn) * 16;
 #pragma unroll
         for (int i = 0; i < MI; ++i) f.a[i] = *reinterpret_cast<const f32x4*>(arow + o + i * 2048);
 #pragma unroll
-        for (int j = 0; j < NI; ++j) f.b[j] = *reinterpret_cast<const f32x4*>(brow + o + j * 2048);
+        for (int j = 0; j < NB; ++j) f.b[j] = *reinterpret_cast<const f32x4*>(brow + o + j / NI * (BN * 128) + j % NI * 2048);
         sched_fence();   // (left alone the compiler moves the reads down to their use)
     };
     // the products of 16 columns, and between them the requests of stage s (none behind the last one)
-    auto use = [&](const Half& f, f32x4(&sum)[MI][NI], int s) __attribute__((always_inline)) {
+    auto use = [&](const Half& f, f32x4(&sum)[MI][NB], int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < NI; ++j) sum[i][j] = mfma16_f32(f.b[j][c], f.a[i][c], sum[i][j]);   // (a lane: row c16, columns 4 q4 .. + 3)
+                for (int j = 0; j < NB; ++j) sum[i][j] = mfma16_f32(f.b[j][c], f.a[i][c], sum[i][j]);   // (a lane: row c16, columns 4 q4 .. + 3)
             if (c < P && s < n) piece(s, c);
+            if (c + 4 < P && s < n) piece(s, c + 4);
         }
         sched_fence();
     };
@@ -243,7 +278,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd
     }
     if (s < n) {   // the rest of the rows: at most 60 columns
         const int rest = p.K - 32 * s;
-        auto step = [&](int s, int half, f32x4(&sum)[MI][NI], int left) __attribute__((always_inline)) {   // left: columns that the rows have from here
+        auto step = [&](int s, int half, f32x4(&sum)[MI][NB], int left) __attribute__((always_inline)) {   // left: columns that the rows have from here
             if (left <= 0) return;
             Half f;
             load(f, s, half);
@@ -251,7 +286,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd
 #pragma unroll
                 for (int i = 0; i < MI; ++i) f.a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j = 0; j < NI; ++j) f.b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < NB; ++j) f.b[j] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
             use(f, sum, n);
         };
@@ -272,54 +307,116 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
             const int c0 = n0 + 16 * (wn * NI + j) + 4 * q4;
-            f32x4 v;
+            f32x4 v, v2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 v[r] = 0.f;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) v[r] += acc[c][i][j][r];
-                if (HEADS) v[r] = c0 + r < p.N ? v[r] / sum * z : 0.f;
+                for (int c = 0; c < 4; ++c) {
+                    v[r] += acc[c][i][j][r];
+                    if (WS == 2) v2[r] += acc[c][i][(WS - 1) * NI + j][r];
+                }
+                if (HEADS)
+                    v[r] = c0 + r < p.N ? v[r] / sum * z : 0.f;
+                else
+                    v[r] = finished<FIN>(p, v[r], v2[r]);
             }
-            float* to = p.C + (long long)m * p.ldc + c0;
+            const long long to = (long long)m * p.ldc + c0;
             if (vec && c0 + 3 < cols) {
-                *reinterpret_cast<f32x4*>(to) = v;
+                if (FIN == ARIA_F32_STREAM) {
+                    f32x4 x = *reinterpret_cast<const f32x4*>(p.x + to), h = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float xr = x[r], hr = 0.f;
+                        stream_step(p, v[r], xr, hr, c0 + r);
+                        x[r] = xr, h[r] = hr;
+                    }
+                    *reinterpret_cast<f32x4*>(p.x + to) = x;
+                    v = h;
+                    if (!p.next.w) continue;
+                }
+                *reinterpret_cast<f32x4*>(p.C + to) = v;
             } else {
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (c0 + r < cols) to[r] = v[r];
+                for (int r = 0; r < 4; ++r) {
+                    if (c0 + r >= cols) continue;
+                    if (FIN == ARIA_F32_STREAM) {
+                        float x = p.x[to + r], h = 0.f;
+                        stream_step(p, v[r], x, h, c0 + r);
+                        p.x[to + r] = x;
+                        if (p.next.w) p.C[to + r] = h;
+                    } else {
+                        p.C[to + r] = v[r];
+                    }
+                }
             }
         }
     }
 }
 
-template <int MT, int NT, int NW>
+template <int MT, int NT, int NW, int FIN>
 int launch_f32(const GemmF32& p, void* stream) {
     const int64_t ntm = (int64_t(p.M) + 16 * MT - 1) / (16 * MT) + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
     const int64_t ntn = (int64_t(p.N) + 16 * NT - 1) / (16 * NT);
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
-    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
+    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, FIN>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
     return aria_check_launch();
 }
 
-template <int MI, int NI, bool HEADS>
+template <int MI, int NI, int FIN>
 int launch_f32_tiles(const GemmF32& p, const Heads& hd, void* stream) {
+    constexpr bool HEADS = FIN == FIN_HEADS;
     constexpr int BM = 32 * MI, BN = 32 * NI;
     const int64_t ntm = (int64_t(p.M) + BM - 1) / BM + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
     const int64_t ntn = ((HEADS ? hd.cols : p.N) + BN - 1) / BN;
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
-    const int vec = !(p.ldc & 3) && !(reinterpret_cast<uintptr_t>(p.C) & 15) && !(HEADS && (hd.cols & 3));
-    ARIA_LAUNCH((gemm_f32_tiles_kernel<MI, NI, HEADS>), dim3(unsigned(ntm * ntn), unsigned(HEADS ? hd.H : 1)), dim3(256), 4 * (BM + BN) * 128, stream, p, hd, vec);
+    const int vec = !(p.ldc & 3) && !((reinterpret_cast<uintptr_t>(p.C) | reinterpret_cast<uintptr_t>(p.x)) & 15) && !(HEADS && (hd.cols & 3));
+    ARIA_LAUNCH((gemm_f32_tiles_kernel<MI, NI, FIN>), dim3(unsigned(ntm * ntn), unsigned(HEADS ? hd.H : 1)), dim3(256), 4 * (BM + (FIN == ARIA_F32_PAIR ? 2 : 1) * BN) * 128, stream, p, hd, vec);
     return aria_check_launch();
+}
+
+// (an expert's last tile stands half empty on average)
+template <int FIN>
+int product_f32(const GemmF32& p, void* stream) {
+    if (p.offsets ? p.M <= 16 * p.E : p.M <= 16) return launch_f32<1, 1, 8, FIN>(p, stream);
+    // Up to a round of 32 x 32 tiles the reduction over the waves is the shorter chain (48 x 1024 x 2816: 22 us, 24 with stages).  Beyond it the rounds of the chip
+    // decide, and of equal ones the larger tile (883 x 2112 x 1024, us as 64 x 64 / 32 x 64 / 32 x 32: 44 / 47 / 48; 883 x 2816 x 1024 61 / 53 / 55; 300 x 2112 x 1024
+    // 24 / 25 / 20).
+    const int64_t M = p.M, N = p.N;
+    auto tiles = [&](int mi, int ni) { return ((M + 32 * mi - 1) / (32 * mi) + (p.offsets ? p.E / 2 : 0)) * ((N + 32 * ni - 1) / (32 * ni)); };
+    if (tiles(1, 1) <= 256) return launch_f32<2, 2, 4, FIN>(p, stream);
+    auto cost = [&](int mi, int ni, int more) { return (tiles(mi, ni) + 255) / 256 * mi * ni * (100 + more); };
+    const int64_t c22 = cost(2, 2, 0), c12 = cost(1, 2, 5), c11 = cost(1, 1, 10);
+    if (c22 <= c12 && c22 <= c11) return launch_f32_tiles<2, 2, FIN>(p, {}, stream);
+    return c12 <= c11 ? launch_f32_tiles<1, 2, FIN>(p, {}, stream) : launch_f32_tiles<1, 1, FIN>(p, {}, stream);
 }
 
 }  // namespace
 
 __attribute__((visibility("hidden"))) int aria_gemm_f32_heads(const float* part_o, const float* uv, float* out, const AriaLatentShape& s, const float* part_ml, const float* proj,
                                                               int64_t T, void* stream) {
-    const GemmF32 p{part_o, uv, out, int(T), int(s.dv), int(s.R), (long long)(s.H * s.R), (long long)s.rp, (long long)(s.H * s.dvp), nullptr, 1, (long long)(s.dv * s.rp)};
+    GemmF32 p{};
+    p.A = part_o, p.W = uv, p.C = out, p.M = int(T), p.N = int(s.dv), p.K = int(s.R);
+    p.lda = s.H * s.R, p.ldw = s.rp, p.ldc = s.H * s.dvp, p.E = 1, p.strideW = s.dv * s.rp;
     const Heads hd{part_ml, proj + s.g_off, (long long)s.ldp, int(s.H), int(s.dvp)};
     // (883 tokens, 8 heads of 128 x 256, us: 64 x 32 with the reduction over the waves 13.3, tiles of 32 x 32 10.9, 32 x 64 10.4, 64 x 64 11.6)
-    return launch_f32_tiles<1, 2, true>(p, hd, stream);
+    return launch_f32_tiles<1, 2, FIN_HEADS>(p, hd, stream);
+}
+
+int aria_gemm_f32_finished(const AriaGemmF32& p, int finish, void* stream) {
+    if (!p.A || !p.W || !p.C || p.M < 0 || p.N < 0 || p.K <= 0 || (p.offsets && p.E <= 0) || (p.rows && p.per <= 0) || (finish == ARIA_F32_PAIR && !p.W2) ||
+        (finish == ARIA_F32_STREAM && (!p.x || !p.post.w || p.offsets)))
+        return ARIA_ERR_INVALID;
+    if (((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W) | reinterpret_cast<uintptr_t>(p.W2)) & 15) || (p.lda & 3) || (p.ldw & 3) || (p.K & 3) || (p.strideW & 3))
+        return ARIA_ERR_ALIGN;
+    if (p.M == 0 || p.N == 0) return ARIA_OK;
+    if ((p.M + 63) / 64 > 65535 || p.E > 65535) return ARIA_ERR_UNSUPPORTED;
+    switch (finish) {
+        case ARIA_F32_RELU2: return product_f32<ARIA_F32_RELU2>(p, stream);
+        case ARIA_F32_PAIR: return product_f32<ARIA_F32_PAIR>(p, stream);
+        case ARIA_F32_STREAM: return product_f32<ARIA_F32_STREAM>(p, stream);
+        default: return product_f32<ARIA_F32_PLAIN>(p, stream);
+    }
 }
 
 extern "C" {
@@ -330,17 +427,9 @@ int aria_gemm_f32(const float* A, const float* W, float* C, int64_t M, int64_t N
     if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) || (lda & 3) || (ldw & 3) || (K & 3) || (strideW & 3)) return ARIA_ERR_ALIGN;
     if (M == 0 || N == 0) return ARIA_OK;
     if ((M + 63) / 64 > 65535 || E > 65535) return ARIA_ERR_UNSUPPORTED;
-    const GemmF32 p{A, W, C, int(M), int(N), int(K), (long long)lda, (long long)ldw, (long long)ldc, (const int*)offsets, int(offsets ? E : 1), (long long)strideW};
-    if (offsets ? M <= 16 * E : M <= 16) return launch_f32<1, 1, 8>(p, stream);
-    // Up to a round of 32 x 32 tiles the reduction over the waves is the shorter chain (48 x 1024 x 2816: 22 us, 24 with stages).  Beyond it the rounds of the chip
-    // decide, and of equal ones the larger tile (883 x 2112 x 1024, us as 64 x 64 / 32 x 64 / 32 x 32: 44 / 47 / 48; 883 x 2816 x 1024 61 / 53 / 55; 300 x 2112 x 1024
-    // 24 / 25 / 20).  An expert's last tile stands half empty on average.
-    auto tiles = [&](int mi, int ni) { return ((M + 32 * mi - 1) / (32 * mi) + (offsets ? E / 2 : 0)) * ((N + 32 * ni - 1) / (32 * ni)); };
-    if (tiles(1, 1) <= 256) return launch_f32<2, 2, 4>(p, stream);
-    auto cost = [&](int mi, int ni, int more) { return (tiles(mi, ni) + 255) / 256 * mi * ni * (100 + more); };
-    const int64_t c22 = cost(2, 2, 0), c12 = cost(1, 2, 5), c11 = cost(1, 1, 10);
-    if (c22 <= c12 && c22 <= c11) return launch_f32_tiles<2, 2, false>(p, {}, stream);
-    return c12 <= c11 ? launch_f32_tiles<1, 2, false>(p, {}, stream) : launch_f32_tiles<1, 1, false>(p, {}, stream);
+    AriaGemmF32 p{};
+    p.A = A, p.W = W, p.C = C, p.M = int(M), p.N = int(N), p.K = int(K), p.lda = lda, p.ldw = ldw, p.ldc = ldc, p.offsets = offsets, p.E = int(offsets ? E : 1), p.strideW = strideW;
+    return product_f32<ARIA_F32_PLAIN>(p, stream);
 }
 
 }  // extern "C"

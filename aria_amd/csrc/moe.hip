@@ -358,6 +358,54 @@ __global__ __launch_bounds__(1024) void sort_small_kernel(const int32_t* idx, co
     }
 }
 
+// Group-limited routing and sort of a few tokens as one launch of one workgroup (a wave per token in turn): what route_groups_kernel and sort_small_kernel do, whose launches
+// are most of their time -- 4 tokens of 2 from 16 experts: 4.7 (cleared counts) + 4.6 + 4.6 us, 5.0 here.
+constexpr int ROUTE_SORT_T = 64, ROUTE_SORT_M = 1024;
+__global__ __launch_bounds__(1024) void route_sort_kernel(const float* logits, const float* correction, float* weights, int32_t* indices, int32_t* offsets, int32_t* sorted_src,
+                                                          int32_t* inv, int T, int E, int ldl, int groups, int keep, int k) {
+    ARIA_SMEM_STATIC float lds[16][768];
+    ARIA_SMEM_STATIC int chosen[ROUTE_SORT_M], base[16][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, M = T * k;
+    for (int t = w; t < T; t += 16) {
+        float my_w;
+        int my_e;
+        route_group_limited(logits + (long long)t * ldl, correction, E, groups, keep, k, lds[w], l, 0, my_w, my_e);
+        if (l < k) {
+            weights[t * k + l] = my_w;
+            indices[t * k + l] = chosen[t * k + l] = my_e;
+        }
+    }
+    sync();
+    const int i = w * 64 + l;   // (one entry a thread)
+    const bool valid = i < M;
+    const int e = valid ? chosen[i] : 0;
+    unsigned long long bal[6];
+#pragma unroll
+    for (int b = 0; b < 6; ++b) bal[b] = ballot((e >> b) & 1);
+    const unsigned long long vm = ballot(valid);
+    base[w][l] = __builtin_popcountll(match_mask(l, bal, vm));
+    sync();
+    if (w == 0) {
+        int total = 0;
+        for (int j = 0; j < 16; ++j) total += base[j][l];
+        const int upto = wave_incl_scan(total);
+        int at = upto - total;
+        if (l < E) offsets[l] = at;
+        if (l == E - 1) offsets[E] = upto;
+        for (int j = 0; j < 16; ++j) {
+            const int c = base[j][l];
+            base[j][l] = at;
+            at += c;
+        }
+    }
+    sync();
+    if (valid) {
+        const int place = base[w][e] + __builtin_popcountll(match_mask(e, bal, vm) & ((1ull << l) - 1ull));
+        sorted_src[place] = i;
+        inv[i] = place;
+    }
+}
+
 // more than 64 experts: one workgroup, thread e owns expert e and walks the indices (staged through LDS, read as broadcasts) in order
 constexpr int SORT_WIDE_E = 256;
 __global__ __launch_bounds__(SORT_WIDE_E) void sort_wide_kernel(const int32_t* idx, const int32_t* counts, int32_t* offsets, int32_t* sorted_src,
@@ -960,6 +1008,18 @@ int aria_moe_route_groups(const float* logits, const float* correction, float* w
                 int(E), int(ldl), int(groups), int(keep), int(k));
     return aria_check_launch();
 }
+
+}  // extern "C"
+
+__attribute__((visibility("hidden"))) int aria_route_groups_sorted(const float* logits, const float* correction, float* weights, int32_t* indices, int32_t* offsets, int32_t* src,
+                                                                   int32_t* inv, int64_t T, int64_t E, int64_t ldl, int64_t groups, int64_t keep, int64_t k, void* stream) {
+    if (!logits || !correction || !weights || !indices || !offsets || !src || !inv || T <= 0 || E <= 0 || k <= 0 || groups <= 0 || keep <= 0 || ldl < E) return ARIA_ERR_INVALID;
+    if (T > ROUTE_SORT_T || T * k > ROUTE_SORT_M || E > 64 || E % groups || keep > groups || k > keep * (E / groups)) return ARIA_ERR_UNSUPPORTED;
+    ARIA_LAUNCH(route_sort_kernel, dim3(1), dim3(1024), 0, stream, logits, correction, weights, indices, offsets, src, inv, int(T), int(E), int(ldl), int(groups), int(keep), int(k));
+    return aria_check_launch();
+}
+
+extern "C" {
 
 int aria_act_rows(const void* gate, const void* u, void* act, int64_t M, int64_t n_cols, int64_t ld_in, int64_t ld_act, int relu_gate, int f32,
                   void* stream) {
