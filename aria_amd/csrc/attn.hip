@@ -20,6 +20,7 @@
 #include "aria_hip.h"
 #include "tile.h"
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 using namespace ad;
@@ -1419,10 +1420,12 @@ __device__ __forceinline__ void fwd3_step(f32x16 (&st)[2], f32x16 (&sn)[2], f32x
 // 145 VGPRs, THREE waves per SIMD).  Measured for the ViT's shape (profiles/r04_attn_fwd3_ab.json): the third wave is worth more than the
 // in-wave overlap, and with it LDS-DMA staging into the conflict-free images (SQ_LDS_BANK_CONFLICT 0, was 8 % of the LDS cycles) is level
 // with v2's register staging -- so hd 72 stays on v2 by default and both v3 forms are kept selectable (ARIA_ATTN_FWD) as measurements.
+// NW = 8 (blocks of 256 queries) or 4 (128, two workgroups a CU: the images of two fit its LDS exactly, so the ragged form, which has no key mask, asks for no more).  A
+// wave does the same work in both, bit for bit; half blocks stage the keys twice as often and halve the longest block (half_blocks: which where).
 // RAGGED: the sequences of the batch are rows cu[b] .. cu[b + 1] of the token axis (Sq = S = the longest), and every head's output is multiplied
 // by sigmoid(gate[token * ldg + head]) in the epilogue (gate may be NULL); `group` neighbouring query heads share a key / value head.
 template <class F, int NW, bool PIPE, bool RAGGED>
-__global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(const bf16_t* Q, const bf16_t* K, const bf16_t* V, bf16_t* O, float* LSE,
+__global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd3_kernel(const bf16_t* Q, const bf16_t* K, const bf16_t* V, bf16_t* O, float* LSE,
                                                         const int32_t* kv_len, const uint8_t* key_mask, int Sq, int S, int H,
                                                         long long ldq, long long ldk, long long ldv, long long ldo, float scale,
                                                         int causal, int nbatch, const int32_t* cu, const bf16_t* gate, long long ldg, int group) {
@@ -1436,7 +1439,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(const bf16_t* Q, con
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), h2 = l >> 5;
     int qblk, head, b;
     constexpr int QB = NW * 32, KA = PIPE ? 1 : 0;  // queries per workgroup; how many tiles K runs ahead of V in LDS
-    static_assert(NW == 8, "the tile images are dealt to 8 waves");
+    static_assert(NW == 8 || NW == 4, "the tile images are dealt to 8 waves, or two shares to each of 4");
     if (!attn_block_coords((Sq + QB - 1) / QB, H, nbatch, causal, true, qblk, head, b)) return;
     const int q0 = qblk * QB;
     if (RAGGED) {
@@ -1454,6 +1457,29 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(const bf16_t* Q, con
     const float scale2 = scale * 1.4426950408889634f;
     F fmt;
     fmt.init(w, l);
+    // the second share of a wave of four: its places in the image are found anew for every tile (in registers they made the 192-column form spill)
+    auto dma_k = [&](int tile) __attribute__((always_inline)) {
+        char* to = sK + (tile & 1) * F::KTILE;
+        fmt.dma_k(Kb, ldk, tile * 64, S - 1, to, w, l);
+        if (NW == 4) {
+            int lane = l;
+            hold(lane);
+            F other;
+            other.init(w + 4, lane);
+            other.dma_k(Kb, ldk, tile * 64, S - 1, to, w + 4, lane);
+        }
+    };
+    auto dma_v = [&](int tile) __attribute__((always_inline)) {
+        char* to = sV + (tile & 1) * F::VTILE;
+        fmt.dma_v(Vb, ldv, tile * 64, S - 1, to, w, l);
+        if (NW == 4) {
+            int lane = l;
+            hold(lane);
+            F other;
+            other.init(w + 4, lane);
+            other.dma_v(Vb, ldv, tile * 64, S - 1, to, w + 4, lane);
+        }
+    };
 
     s16x8 qf[KS];
 #pragma unroll
@@ -1479,9 +1505,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(const bf16_t* Q, con
         if (t == 0) sFlag[tile % 3] = int(all == ~0ull) | (int(all == 0ull) << 1);
     };
     if (ntiles > 0) {
-        fmt.dma_k(Kb, ldk, 0, S - 1, sK, w, l);
-        fmt.dma_v(Vb, ldv, 0, S - 1, sV, w, l);
-        if (PIPE && ntiles > 1) fmt.dma_k(Kb, ldk, 64, S - 1, sK + F::KTILE, w, l);
+        dma_k(0);
+        dma_v(0);
+        if (PIPE && ntiles > 1) dma_k(1);
         if (kmb && t < 64) {
             mask_park(0, mask_fetch(0));
             if (ntiles > 1) mask_park(1, mask_fetch(1));
@@ -1501,8 +1527,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(const bf16_t* Q, con
     auto duties = [&](int it) __attribute__((always_inline)) {
         wait_vm<0>();  // this wave's pieces of K(it + KA) and V(it) have landed
         sync();        // ... everybody's; every wave is done with K(it + KA - 1) and V(it - 1)
-        if (it + KA + 1 < ntiles) fmt.dma_k(Kb, ldk, (it + KA + 1) * 64, S - 1, sK + ((it + KA + 1) & 1) * F::KTILE, w, l);
-        if (it + 1 < ntiles) fmt.dma_v(Vb, ldv, (it + 1) * 64, S - 1, sV + ((it + 1) & 1) * F::VTILE, w, l);
+        if (it + KA + 1 < ntiles) dma_k(it + KA + 1);
+        if (it + 1 < ntiles) dma_v(it + 1);
         if (kmb && t < 64 && it + 2 < ntiles) mv = mask_fetch(it + 2);
     };
     auto park = [&](int it) __attribute__((always_inline)) {
@@ -1567,6 +1593,11 @@ thread_local int g_last_fwd_variant = 0;  // 2: attn_fwd2 (staged through regist
 thread_local int g_last_bwd_variant = 0;  // 2: the padded-tile pair (hd 64 / 72), 5: role-split dK/dV + dQ v5 (hd 128) -- tests assert which ran
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Blocks of 128 queries rather than 256 where their shorter last blocks are worth more than the keys staged twice as often.  Us, 256 / 128 queries a block, causal, 20 heads of 128:
+// 280 tokens 19.9 / 14.7, 777 34 / 26, 2048 71 / 57, 4096 132 / 121, 8192 405 / 389, 12000 798 / 820, 32768 5536 / 6052; 8 x 2048 257 / 246, 32 x 100 38 / 27; not causal 4096 254 / 231.
+// 12 heads of 192 / 128: six prompts of 500 .. 1200 56 / 52, 4000 150 / 134, 8000 319 / 301, (20 heads) 16384 1842 / 2005.  64 columns gain at every length (33000 2764 / 2661).
+bool half_blocks(int64_t Sq, int causal, int64_t qd) { return qd == 64 || Sq <= (causal ? 8192 : 4096); }
+
 struct Plan72 {
     int whole = 0, part_waves = 0;   // blocks of 12 waves a (b, head), waves of its other blocks (0: only blocks of 12)
     unsigned grid = 0;
@@ -1621,11 +1652,17 @@ int aria_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
     // (r05: the two hd-72 forms of v3 -- measured slower than v2's 12 waves -- left the library: tools/probes/src/attn_fwd3_hd72.patch)
     const bool v3 = !(fwdv && fwdv[0] == '2') && hd == 128 && Skv > 0;
     g_last_fwd_variant = v3 ? 3 : 2;
-    if (v3)
-        ARIA_LAUNCH((attn_fwd3_kernel<Fmt128, 8, true, false>), dim3(attn_grid((Sq + 255) / 256, H, B)), dim3(512), size_t(Fwd3Smem<Fmt128>::BYTES), stream, Q, K, V,
+    auto launch3 = [&](auto nw) {
+        constexpr int NW = decltype(nw)::value;
+        ARIA_LAUNCH((attn_fwd3_kernel<Fmt128, NW, true, false>), dim3(attn_grid((Sq + 32 * NW - 1) / (32 * NW), H, B)), dim3(64 * NW), size_t(Fwd3Smem<Fmt128>::BYTES), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
                     (long long)ldv, (long long)ldo, scale, causal_arg, int(B), static_cast<const int32_t*>(nullptr),
                     static_cast<const bf16_t*>(nullptr), 0ll, 1);
+    };
+    if (v3 && half_blocks(Sq, causal, hd))
+        launch3(std::integral_constant<int, 4>{});
+    else if (v3)
+        launch3(std::integral_constant<int, 8>{});
     else if (hd == 128)
         ARIA_LAUNCH((attn_fwd2_kernel<128, 8>), dim3(attn_grid((Sq + 255) / 256, H, B)), dim3(512), size_t(Cfg2<128>::SMEM), stream, Q, K, V,
                     static_cast<bf16_t*>(o), lse, kv_len, key_mask, int(Sq), int(Skv), int(H), (long long)ldq, (long long)ldk,
@@ -1657,24 +1694,33 @@ int aria_attn_varlen_fwd(const void* q, const void* k, const void* v, void* o, c
     if (!known) return ARIA_ERR_UNSUPPORTED;
     if (B == 0 || S_max == 0) return ARIA_OK;
     const int causal = S_max >= 32768 ? 2 : 1;   // (2: attn_block_coords' grouped order)
-#define ARIA_VARLEN(F, PIPE)                                                                                                                  \
-    ARIA_LAUNCH((attn_fwd3_kernel<F, 8, PIPE, true>), dim3(attn_grid((S_max + 255) / 256, H, B)), dim3(512), size_t(Fwd3Smem<F>::BYTES), stream, \
-                static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), static_cast<bf16_t*>(o),           \
-                static_cast<float*>(nullptr), static_cast<const int32_t*>(nullptr), static_cast<const uint8_t*>(nullptr), int(S_max),           \
-                int(S_max), int(H), (long long)ldq, (long long)ldk, (long long)ldv, (long long)ldo, scale, causal, int(B), cu,                  \
-                static_cast<const bf16_t*>(gate), (long long)ldg, int(H / G))
+    const bool half = half_blocks(S_max, 1, qd);
+    auto launch = [&](auto fmt, auto pipe) {
+        using F = decltype(fmt);
+        auto of = [&](auto nw) {
+            constexpr int NW = decltype(nw)::value;
+            constexpr bool PIPE = decltype(pipe)::value;
+            ARIA_LAUNCH((attn_fwd3_kernel<F, NW, PIPE, true>), dim3(attn_grid((S_max + 32 * NW - 1) / (32 * NW), H, B)), dim3(64 * NW), size_t(Fwd3Smem<F>::M0), stream,
+                        static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), static_cast<bf16_t*>(o), static_cast<float*>(nullptr),
+                        static_cast<const int32_t*>(nullptr), static_cast<const uint8_t*>(nullptr), int(S_max), int(S_max), int(H), (long long)ldq, (long long)ldk,
+                        (long long)ldv, (long long)ldo, scale, causal, int(B), cu, static_cast<const bf16_t*>(gate), (long long)ldg, int(H / G));
+        };
+        if constexpr (2 * Fwd3Smem<F>::M0 <= 160 * 1024) {
+            if (half) return of(std::integral_constant<int, 4>{});
+        }
+        of(std::integral_constant<int, 8>{});
+    };
     using F64 = FmtQV<64, 64>;
     using F192 = FmtQV<192, 128>;
     using F256 = FmtQV<256, 256>;
     if (qd == 64)
-        ARIA_VARLEN(F64, true);
+        launch(F64{}, std::true_type{});
     else if (qd == 128)
-        ARIA_VARLEN(Fmt128, true);
+        launch(Fmt128{}, std::true_type{});
     else if (qd == 192)
-        ARIA_VARLEN(F192, false);   // (the pipelined form holds 18 registers too many and spills: 643 against 736 TF/s, 8192 tokens x 20 heads)
+        launch(F192{}, std::false_type{});   // (the pipelined form holds 18 registers too many and spills: 643 against 736 TF/s, 8192 tokens x 20 heads)
     else
-        ARIA_VARLEN(F256, false);
-#undef ARIA_VARLEN
+        launch(F256{}, std::false_type{});
     return aria_check_launch();
 }
 

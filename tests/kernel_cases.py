@@ -1105,6 +1105,29 @@ def case_attention_forward_variants(dev, B, Sq, Skv, H, hd, causal, masked, use_
     close(got["3"][0], want.transpose(1, 2).reshape(B * Sq, D), 2e-2, 2e-2)
 
 
+def case_attention_varlen_blocks(dev, lens, H=2):
+    """Packed sequences in blocks of 128 queries (the longest up to 8192) or 256: the bits of each sequence alone in the oldest kernel, which has blocks of 256."""
+    import os
+
+    from aria_amd import ops
+
+    T, D = sum(lens), H * 128
+    g = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(T, D, generator=g).to(bf16).to(dev) for _ in range(3))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=dev)
+    got = ops.attention_varlen(q, k, v, cu, max(lens), H, 128, 128, 128 ** -0.5)
+    prev = os.environ.get("ARIA_ATTN_FWD")
+    os.environ["ARIA_ATTN_FWD"] = "2"
+    try:
+        for a, n in zip(cu.tolist(), lens):
+            want = ops.attention_fwd(q[a:a + n], k[a:a + n], v[a:a + n], 1, n, H, 128, 128 ** -0.5, True)[0]
+            assert torch.equal(got[a:a + n], want.view(n, D)), n
+    finally:
+        os.environ.pop("ARIA_ATTN_FWD")
+        if prev is not None:
+            os.environ["ARIA_ATTN_FWD"] = prev
+
+
 def case_attention_bwd_rope(dev, B, S, H, causal, use_len, s_rope=None):
     """r05: ``aria_attn_bwd_rope`` -- the inverse half-split RoPE of dq / dk (the chain rule through apply_rotary_pos_emb,
     modeling_llama.py:130-160) in the attention backward's register epilogues -- gives the bits of ``aria_attn_bwd`` followed by the in-place

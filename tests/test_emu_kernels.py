@@ -114,6 +114,11 @@ def test_attention_forward_variants_give_the_same_bits(B, Sq, Skv, H, hd, causal
     C.case_attention_forward_variants(DEV, B, Sq, Skv, H, hd, causal, masked, use_len)
 
 
+@pytest.mark.parametrize("lens", [(1, 127, 130), (257, 64)])
+def test_attention_varlen_blocks(lens):
+    C.case_attention_varlen_blocks(DEV, lens)
+
+
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
 @pytest.mark.parametrize("M,N,K", [(40, 72, 64), (264, 136, 192), (72, 520, 128)])
 def test_gemm_fused_gelu(monkeypatch, force, M, N, K):
