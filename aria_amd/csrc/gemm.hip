@@ -455,6 +455,13 @@ static int dense_product(const void* A, const void* B, void* C, const void* bias
     // with a workspace the partly filled last round of tiles is split along K (gemm3.hip), so small outputs fill the chip too
     const long long ws_need = workspace ? aria_gemm3_workspace_bytes(M, N, K) : 0;
     const bool splits = ws_need > 0 && workspace_bytes >= ws_need;
+    // (weight gradients of fewer than 64 rows: of the LDS-DMA kernels only strips take them)
+    const char* forced = std::getenv("ARIA_GEMM_FORCE");
+    if (a_oc && b_oc && K > 0 && K < 64 && (!forced || (forced[0] == '4' && forced[1] == '7')) && fits_dma(64, lda, ldb, bytesA, bytesB, M, N) && aria_wgrad_strips_take(p, -1, forced != nullptr)) {
+        Gemm4Plan plan;
+        plan.form = 4;
+        return launch4(p, a_oc, b_oc, plan, nullptr, stream);
+    }
     if ((!a_oc || b_oc) && fits_dma(K, lda, ldb, bytesA, bytesB, M, N)) {
         const Gemm4Plan plan = aria_plan_gemm4(p, a_oc, b_oc, -1, splits ? aria_gemm3_split(M, N, K) : 1, workspace ? workspace_bytes : 0, own_cut);
         if (plan.form) return launch4(p, a_oc, b_oc, plan, workspace, stream);

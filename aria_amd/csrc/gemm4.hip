@@ -561,9 +561,13 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     Gemm4Plan none, plan;
     if (p.ext_k || p.rope_sn || (a_oc && !b_oc) || p.N < 8 || (a_oc && p.M < 8)) return none;   // (p.rope_sn: the entry takes whole rounds of 256 x 256 tiles only)
     const bool plain = !p.glu && !p.dglu && !p.rope_fc;
-    if (const char* force = std::getenv("ARIA_GEMM_FORCE")) {   // "4": tiles of 128 x 256, "46": the wide ones where there is such a form
+    if (const char* force = std::getenv("ARIA_GEMM_FORCE")) {   // "4": tiles of 128 x 256, "46": the wide ones, "47": strips, where there is such a form
         if (force[0] != '4') return none;
-        plan.form = a_oc ? 3 : force[1] == '6' && plain && p.mode == 0 ? 2 : 1;
+        plan.form = a_oc ? (force[1] == '7' && aria_wgrad_strips_take(p, rows, true) ? 4 : 3) : force[1] == '6' && plain && p.mode == 0 ? 2 : 1;
+        return plan;
+    }
+    if (a_oc && aria_wgrad_strips_take(p, rows)) {
+        plan.form = 4;
         return plan;
     }
     if (p.mode == 2) {   // rows: of all experts together, < 0: not known
@@ -610,6 +614,7 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
 }
 
 int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream) {
+    if (plan.form == 4) return aria_launch_wgrad_strips(p, stream);
     GemmParams q = p;
     const char* wsd = std::getenv("ARIA_GEMM_WIDE_STORE");
     q.wide_store = !(wsd && wsd[0] == '0') && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0 && (p.strideC & 7) == 0;

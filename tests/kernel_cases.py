@@ -150,6 +150,30 @@ def case_gemm_four_waves_fused(dev, monkeypatch):
     assert all(form[n] + 16 in seen.get(n, ()) for n in FUSED_FOUR_WAVES), seen
 
 
+def case_wgrad_strips(dev, monkeypatch, counts, M, N):
+    """Weight gradients in strips of 256 columns (the reduction's fragments of dY stay in registers): the bits of the 128 x 256 tiles for experts of any number of rows -- none, partial
+    steps of sixteen, the 256 that are held, more -- plain, gathered and dense, and within the bound of a rounded 32-bit sum of exact products."""
+    from aria_amd import ops
+
+    T, E = sum(counts), len(counts)
+    x, dy = rnd(T, M, seed=T).to(dev), rnd(T, N, seed=N).to(dev)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=dev)
+    rows = torch.cat([torch.randperm(T, generator=torch.Generator().manual_seed(3)).to(torch.int32), torch.zeros(64, dtype=torch.int32)]).to(dev)[:T]
+    jobs = [(lambda: ops.grouped_gemm_wgrad(x, dy, off, E), 4), (lambda: ops.grouped_gemm_wgrad_gather(x, rows, dy, off, E), 4)]
+    jobs += [(lambda n=n: ops.gemm(x[:n], dy[:n], a_oc=True, b_oc=True), 4 if n <= 256 else 3) for n in (1, 63, 64, 200, 256, 257) if n <= T]
+    for f, form in jobs:
+        got = {}
+        for force in ("4", "47"):
+            monkeypatch.setenv("ARIA_GEMM_FORCE", force)
+            got[force] = f()
+            assert last_gemm_tiles() & 15 in ((form,) if force == "47" else (3, 0))   # (0: fewer than 64 rows, the kernels of any size)
+        assert torch.equal(got["4"], got["47"])
+    want = torch.stack([x[a:b].double().t() @ dy[a:b].double() for a, b in zip(off.tolist(), off.tolist()[1:])]) if T else torch.zeros(E, M, N)
+    got = jobs[0][0]()
+    size = torch.stack([x[a:b].double().abs().t() @ dy[a:b].double().abs() for a, b in zip(off.tolist(), off.tolist()[1:])])
+    assert bool(((got.double() - want).abs() <= 2 ** -8 * want.abs() + max(max(counts), 1) * 2 ** -24 * size).all())   # rounding to bf16, a rounding a product
+
+
 def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
     activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""

@@ -252,6 +252,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(force_gemm_v3, B, S, D, hd, K):
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K)
 
 
+@pytest.mark.parametrize("counts,M,N", [([17, 0, 1, 70, 258], 128, 256), ([256, 0, 16], 704, 512)])
+def test_wgrad_strips(monkeypatch, counts, M, N):
+    C.case_wgrad_strips(DEV, monkeypatch, counts, M, N)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 136, 128), (300, 264, 512), (40, 1032, 1536)])
 def test_gemm_keep_sums(monkeypatch, M, N, K):
     C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)

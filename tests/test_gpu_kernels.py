@@ -246,6 +246,11 @@ def test_gemm_qkv_rope_hf_is_gemm_plus_rope(B, S, D, hd, K):   # q | k | v proje
     assert C.case_gemm_qkv_rope_hf(DEV, B, S, D, hd, K) == (D >= 2560)
 
 
+@pytest.mark.parametrize("counts,M,N", [([17, 0, 1, 70, 258], 128, 256), ([256, 0, 16], 704, 512), ([3, 73, 128, 129, 600, 0, 255, 257, 0, 0, 0, 0], 2560, 3328)])
+def test_wgrad_strips(monkeypatch, counts, M, N):
+    C.case_wgrad_strips(DEV, monkeypatch, counts, M, N)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (777, 2560, 2560), (3000, 2560, 3328)])
 def test_gemm_keep_sums(monkeypatch, M, N, K):
     C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)
