@@ -128,14 +128,26 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* dy, cons
         dw_partial[(long long)blockIdx.x * D + d] = red[d] + red[D + d] + red[2 * D + d] + red[3 * D + d];
 }
 
-// 32 columns x 8 row-groups per block: 128-byte row segments, 8x the parallelism of one-thread-per-column
+// 32 columns x 8 row-groups per block: 128-byte row segments, 8x the parallelism of one-thread-per-column.  The rows' latencies are the time: a thread's next eight are in flight
+// together and added in order.  With the norm's
+// backward in front, cold rows of 2560, one / eight in flight, us: 777 tokens (195 rows here) 21.7 / 15.8, 4096 (512) 48 / 32, 16 384 108 / 92.
+constexpr int COLSUM_AHEAD = 8;
 __global__ __launch_bounds__(256) void colsum_kernel(const float* partial, bf16_t* out, int nrows, int D, int accumulate) {
     ARIA_SMEM_STATIC float red[8][32];
     const int c = threadIdx.x & 31, rg = threadIdx.x >> 5;
     const int d = blockIdx.x * 32 + c;
     float s = 0.f;
-    if (d < D)
-        for (int r = rg; r < nrows; r += 8) s += partial[(long long)r * D + d];
+    if (d < D) {
+        int r = rg;
+        for (; r + 8 * (COLSUM_AHEAD - 1) < nrows; r += 8 * COLSUM_AHEAD) {
+            float v[COLSUM_AHEAD];
+#pragma unroll
+            for (int i = 0; i < COLSUM_AHEAD; ++i) v[i] = partial[(long long)(r + 8 * i) * D + d];
+#pragma unroll
+            for (int i = 0; i < COLSUM_AHEAD; ++i) s += v[i];
+        }
+        for (; r < nrows; r += 8) s += partial[(long long)r * D + d];
+    }
     red[rg][c] = s;
     sync();
     if (rg == 0 && d < D) {

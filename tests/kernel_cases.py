@@ -874,6 +874,21 @@ def case_swiglu(dev, exact):
 
 
 # ------------------------------------------------------------------------------------------ norm / rope
+def case_colsum_rows(dev, n, D):
+    """Column sums of 32-bit rows: eight groups, every eighth row in order, then the groups in order; rounded once.  The same bits whatever is in flight together."""
+    from aria_amd import hip, ops
+
+    x, out = rnd(n, D, seed=n).float().div(3).to(dev), torch.empty(D, dtype=bf16, device=dev)
+    hip.get_lib().call("aria_colsum_f32", x.data_ptr(), out.data_ptr(), n, D, 0, ops._stream(x))
+    total, h = torch.zeros(D), x.cpu()
+    for g in range(8):
+        s = torch.zeros(D)
+        for r in range(g, n, 8):
+            s = s + h[r]
+        total = total + s
+    assert torch.equal(out.cpu(), total.to(bf16))
+
+
 def case_rmsnorm(dev, T, D, exact):
     from aria_amd import ops
 

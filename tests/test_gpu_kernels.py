@@ -60,6 +60,11 @@ def test_swiglu():
     C.case_swiglu(DEV, exact=False)
 
 
+@pytest.mark.parametrize("n", [1, 56, 57, 64, 71, 201])
+def test_colsum_rows(n):
+    C.case_colsum_rows(DEV, n, 40)
+
+
 @pytest.mark.parametrize("T,D", [(9, 64), (130, 2560), (3, 1152), (4099, 2560)])
 def test_rmsnorm(T, D):
     C.case_rmsnorm(DEV, T, D, exact=False)
