@@ -1,6 +1,7 @@
 // The thin products of a low-rank adapter (rank 8 or 16) of a training step: result = base(x) + lora_B(lora_A(dropout(x))) * scaling
 // (aria/lora/layers.py:129-139; for nn.Linear peft's adapter, the same line).  The base launch carries lora_B (the *_lora_* entries); here are
-//   scale:  u * scaling                            into the adapter's columns of the launch's extension
+//   u:      scale * dropout(x) lora_A              (thin_product_kernel: the general tiles' bits) into the adapter's columns of the launch's extension
+//   scale:  u * scaling                            where the general product computes u
 //   down:   d_u = scale * dy W^T                   with lora_B
 //   up:     dx += keep ? (d_u A) / (1 - p) : 0     the adapter's input gradient through its dropout mask, added where the base's gradient lies
 //   wgrad:  dW = y^T u                             dense adapters' weight gradients (the experts' run as grouped products)
@@ -14,6 +15,7 @@
 #include "elem.h"
 #include "gemm_params.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 using namespace ad;
@@ -136,10 +138,15 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
 // step); the first wave multiplies.
 // 5580 rows of 1536 on 32 columns as 128 x 128 tiles of the general kernel 25.8 us.
 constexpr int XR = 512, XPITCH = XR + 8;   // (16 bytes: 16 rows' pieces lie on different banks)
-__global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, float* C, int M, int N, int K, long long ldx, long long ldc, int cut_row,
-                                                           int cut) {
+// An adapter's u = bf16(scale * bf16(x W)) too (T = bf16_t; per expert where there are offsets, W_OC: W [K][N]): the forward's, in front of routers like the base products.  With the launches it takes
+// the place of, us: cold rows, rank 8: 777 of 2560 27.6, here 21.5, 4096 32 / 19, 16 384 56 / 40; rows by expert, 4662 of 2560 58 / 19, 24 576 74 / 56, 98 304 174 / 151.
+template <bool W_OC, class T>
+__global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, T* C, const int32_t* offsets, int E, int M, int N, int K, long long ldx, long long ldc,
+                                                           int cut_row, int cut, float scale) {
     ARIA_DYN_SMEM(lds);
-    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), pitch = K + 8, nch = K / 64, m0 = blockIdx.x * ROWS, pieces = m0 >= cut_row ? cut : 1;
+    int e, m0;
+    if (!rows_of(offsets, E, M, blockIdx.x, e, m0, M)) return;
+    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), pitch = K + 8, nch = K / 64, pieces = m0 >= cut_row ? cut : 1;
     bf16_t* xs = reinterpret_cast<bf16_t*>(lds);   // [32][XPITCH]
     bf16_t* ws = xs + ROWS * XPITCH;               // [N][pitch]
     u32x4 xa[4], xb[4];
@@ -151,7 +158,16 @@ __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, cons
     load(xa, 0);
     load(xb, XR);
 #pragma unroll 6
-    for (int i = t; i < N * K / 8; i += 512) st16(ws + i / (K / 8) * pitch + 8 * (i % (K / 8)), ld16(W + 8ll * i));
+    for (int i = t; i < N * K / 8; i += 512) {
+        const u32x4 v = ld16(W + (long long)e * N * K + 8ll * i);
+        if (W_OC) {
+            const int k = i / (N / 8), n = 8 * (i % (N / 8));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ws[(n + 2 * q) * pitch + k] = bf16_t(v[q] & 0xffffu), ws[(n + 2 * q + 1) * pitch + k] = bf16_t(v[q] >> 16);
+        } else {
+            st16(ws + i / (K / 8) * pitch + 8 * (i % (K / 8)), v);
+        }
+    }
     f32x16 acc, sum;
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[j] = sum[j] = 0.f;
@@ -184,12 +200,18 @@ __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, cons
         if (c0 + XR / 64 < nch) round(xb, c0 + XR / 64);
     }
     if (w || m0 + (l & 31) >= M) return;
-    float* out = C + (long long)(m0 + (l & 31)) * ldc + 4 * (l >> 5);   // (a lane: a row, columns 8 q + 4 (l / 32) .. + 3)
+    T* out = C + (long long)(m0 + (l & 31)) * ldc + 4 * (l >> 5);   // (a lane: a row, columns 8 q + 4 (l / 32) .. + 3)
 #pragma unroll
     for (int q = 0; q < 4; ++q)
         if (8 * q < N)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) out[8 * q + j] = piece ? sum[4 * q + j] + acc[4 * q + j] : acc[4 * q + j];
+            for (int j = 0; j < 4; ++j) {
+                const float v = piece ? sum[4 * q + j] + acc[4 * q + j] : acc[4 * q + j];
+                if constexpr (sizeof(T) == 4)
+                    out[8 * q + j] = v;
+                else
+                    out[8 * q + j] = f2bf(rbf(v) * scale);
+            }
 }
 
 __device__ __forceinline__ float half_of(const u32x4& v, int i) { return i & 1 ? bfhi(v[i >> 1]) : bflo(v[i >> 1]); }
@@ -364,8 +386,28 @@ int aria_thin_product_f32(const void* X, const void* W, float* C, int64_t M, int
     if (M == 0) return ARIA_OK;
     long long cut_row = 0;
     const int cut = aria_gemm3_cut(M, N, K, &cut_row);
-    ARIA_LAUNCH(thin_product_kernel, dim3(row_tiles(M, nullptr, 1)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W), C, int(M),
-                int(N), int(K), (long long)ldx, (long long)ldc, int(cut_row), cut);
+    ARIA_LAUNCH((thin_product_kernel<false, float>), dim3(row_tiles(M, nullptr, 1)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X), static_cast<const bf16_t*>(W),
+                C, static_cast<const int32_t*>(nullptr), 1, int(M), int(N), int(K), (long long)ldx, (long long)ldc, int(cut_row), cut, 1.f);
+    return aria_check_launch();
+}
+
+int aria_lora_u_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu, float scale,
+                     void* stream) {
+    if (!X || !W || !U || M < 0 || K <= 0 || r <= 0 || (offsets && E <= 0)) return ARIA_ERR_INVALID;
+    const int64_t lds = r * (K + 8) * 2 + ROWS * XPITCH * 2;
+    if (!thin(r) || (K & 63) || r * (K + PAD) * 2 > LDS_MAX || M >= (1ll << 30)) return ARIA_ERR_UNSUPPORTED;
+    if (off16(X) || off16(W) || (ldx & 7)) return ARIA_ERR_ALIGN;
+    if (M == 0) return ARIA_OK;
+    long long cut_row = 0;
+    const int cut = offsets ? 1 : aria_gemm3_cut(M, r, K, &cut_row);   // (rows by expert are never cut)
+    auto launch = [&](auto oc) {
+        ARIA_LAUNCH((thin_product_kernel<decltype(oc)::value, bf16_t>), dim3(row_tiles(M, offsets, E)), dim3(512), unsigned(lds), stream, static_cast<const bf16_t*>(X),
+                    static_cast<const bf16_t*>(W), static_cast<bf16_t*>(U), offsets, int(E), int(M), int(r), int(K), (long long)ldx, (long long)ldu, int(cut_row), cut, scale);
+    };
+    if (w_oc)
+        launch(std::true_type{});
+    else
+        launch(std::false_type{});
     return aria_check_launch();
 }
 

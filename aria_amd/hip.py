@@ -74,6 +74,7 @@ SIGNATURES = {
     "aria_dropout_bwd_bf16": [P, P, P, I64, F32, I32, P],
     "aria_thin_product_f32": [P, P, P, I64, I64, I64, I64, I64, P],
     "aria_lora_scale_bf16": [P, P, I64, I64, I64, F32, P],
+    "aria_lora_u_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_down_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_up_bf16": [P, P, I32, P, P, P, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_wgrad_bf16": [P, P, P, I32, I64, I64, I64, I64, I64, P, I64, P],

@@ -8,8 +8,8 @@ nn.Linear targets -- the same line):
 
 What runs here, per module:
   * ``u = scaling * lora_A(dropout(x))`` -- a skinny GEMM (N = r) on the dropped input (``ops.dropout``: one pass, one mask byte per 8
-    elements kept for the backward), scaled into its columns.  The forward keeps the general product's sum order although ``ops.lora_down``, the
-    backward's kernel, is three times as fast: with dropout another rounding of u turns near ties of the next layer's router, and a turned tie
+    elements kept for the backward), scaled into its columns (``ops.lora_u``).  The forward keeps the general product's sum order although ``ops.lora_down``, the
+    backward's kernel, is faster still: with dropout another rounding of u turns near ties of the next layer's router, and a turned tie
     moves every later expert row under another mask;
   * the base launch with the adapter's second projection as a K-EXTENSION (``ops.*_lora``: one extra K-tile fed from u and lora_B): no
     output-sized ``base + delta`` pass, and the fused epilogues keep working -- fc1 + SwiGLU, gate|up + SwiGLU, the q|k|v and gate|up wide
@@ -53,6 +53,13 @@ def _scaled(u: torch.Tensor, s: float, out=None) -> torch.Tensor:
     return u if out is None else out.copy_(u)
 
 
+def _u(x: torch.Tensor, a: torch.Tensor, s: float, offsets=None, out=None) -> torch.Tensor:
+    """scale * lora_A(x) with the general product's bits: by the thin product where it takes the shapes"""
+    if ops.lora_u_takes(x, a, offsets is not None):
+        return ops.lora_u(x, a, s, offsets=offsets, out=out)
+    return _scaled(ops.gemm(x, a) if offsets is None else ops.grouped_gemm(x, a, offsets), s, out=out)
+
+
 def _factor(w: torch.Tensor) -> torch.Tensor:
     """An adapter factor as the thin products read it: dense and on a 16-byte boundary."""
     return w if w.is_contiguous() and w.data_ptr() % 16 == 0 else w.clone(memory_format=torch.contiguous_format)
@@ -93,7 +100,7 @@ def dense_lora_fwd(x: torch.Tensor, w: torch.Tensor, sites: List[Optional[LoraSi
     for j, s in live:
         r = s.a.shape[0]
         d = _Drop(x, s.p, training, _seed(seeds))
-        _scaled(ops.gemm(d.xd, s.a), s.scaling, out=U[:, c0:c0 + r])
+        _u(d.xd, s.a, s.scaling, out=U[:, c0:c0 + r])
         Bx[starts[j]:starts[j] + rows[j], c0:c0 + r] = s.b
         drops.append(d)
         c0 += r
@@ -137,7 +144,7 @@ def grouped_lora_fwd(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, si
         out = ops.grouped_gemm_swiglu(x, w, offsets, want_h=want_h) if glu else ops.grouped_gemm(x, w, offsets)
         return out, None
     d = _Drop(x, site.p, training, _seed(seeds))
-    U = _scaled(ops.grouped_gemm(d.xd, site.a, offsets), site.scaling)                      # [M, r]
+    U = _u(d.xd, site.a, site.scaling, offsets)                      # [M, r]
     out = ops.grouped_gemm_swiglu_lora(x, w, offsets, U, site.b, want_h=want_h) if glu else ops.grouped_gemm_lora(x, w, offsets, U, site.b)
     return out, dict(site=site, drop=d, U=U)
 
@@ -301,7 +308,7 @@ def lm_head_lora_loss_fwd_bwd(hn, lm_w, labels_shifted, site: LoraSite, training
         labels_v[n:] = -100
     hv = ops.moe_permute(hn, rows, 1)
     d = _Drop(hv, site.p, training, _seed([int(seed)]))
-    U = _scaled(ops.gemm(d.xd, site.a), site.scaling)
+    U = _u(d.xd, site.a, site.scaling)
     logits = ops.gemm_lora(hv, lm_w, U, site.b)
     count_in = torch.full((1,), n, dtype=torch.int32, device=hn.device)
     loss_sum, _, _ = ops.cross_entropy(logits, labels_v, grad_scale=1.0, dlogits=logits, count_in=count_in)

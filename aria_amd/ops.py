@@ -291,6 +291,28 @@ def lora_scale(u: torch.Tensor, scale: float, out=None) -> torch.Tensor:
     return out
 
 
+def lora_u_takes(x: torch.Tensor, w: torch.Tensor, w_oc: bool) -> bool:
+    """whether ``lora_u`` takes the product; others are the general product's, then a scaling"""
+    K, r = (w.shape[-2], w.shape[-1]) if w_oc else (w.shape[-1], w.shape[-2])
+    return (GEMM_SPLIT_K and lora_thin(r, K) and x.dtype == w.dtype == bf16 and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.dim() == 2 and x.shape[1] == K
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and 0 < x.shape[0] < 1 << 30)
+
+
+def lora_u(x: torch.Tensor, w: torch.Tensor, scale: float, offsets=None, out=None) -> torch.Tensor:
+    """bf16(bf16(x w^T) * scale): x [M, K], w [r, K]; with ``offsets`` x w per expert, w [E, K, r].  The bits of the general product and ``lora_scale``.  out: [M, r], strided rows."""
+    _chk(x, name="x"), _chk(w, name="w")
+    M, K = x.shape
+    r = w.shape[0] if offsets is None else w.shape[2]
+    if w.dim() != (2 if offsets is None else 3) or (offsets is not None and offsets.numel() != w.shape[0] + 1):
+        raise ValueError("lora_u: a factor [r, K], the experts' [E, K, r]")
+    out = torch.empty((M, r), dtype=bf16, device=x.device) if out is None else out
+    if tuple(out.shape) != (M, r):
+        raise ValueError("lora_u: out must be [M, r]")
+    hip.get_lib().call("aria_lora_u_bf16", _p(x), _p(w), int(offsets is not None), _p(out), _p(offsets) if offsets is not None else None,
+                       w.shape[0] if offsets is not None else 1, M, K, r, _rowmajor_2d(x, "x"), _rowmajor_2d(out, "out"), float(scale), _stream(x))
+    return out
+
+
 def lora_down(x: torch.Tensor, w: torch.Tensor, scale: float, w_oc: bool, offsets=None, out=None) -> torch.Tensor:
     """bf16(scale * x w^T): x [M, K] (unit-stride rows), w [r, K], or [K, r] with ``w_oc``; with ``offsets`` a leading expert dimension.  out: [M, r], strided rows."""
     _chk(x, name="x"), _chk(w, name="w")

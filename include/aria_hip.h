@@ -153,6 +153,11 @@ int aria_dropout_bwd_bf16(const void* term, const void* mask, void* dx, int64_t 
  * are those of aria_gemm_bf16_ws with a workspace: a router's choice hangs on them. */
 int aria_thin_product_f32(const void* X, const void* W, float* C, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldc, void* stream);
 int aria_lora_scale_bf16(const void* U, void* OUT, int64_t M, int64_t r, int64_t ldo, float scale, void* stream);
+/* U = bf16(bf16(X W) * scale), the forward's first projection of an adapter with its scaling: X [M, K], W [r, K] (w_oc 0) or [K, r], with offsets int32 [E + 1] rows by expert and W
+ * [E, ., .]; r 8 or 16, K % 64 == 0.  Bit for bit aria_gemm_bf16_ws with a workspace (by expert aria_grouped_gemm_bf16) and aria_lora_scale_bf16: near ties of following routers hang on
+ * them. */
+int aria_lora_u_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu, float scale,
+                     void* stream);
 int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r, int64_t ldx, int64_t ldu,
                         float scale, void* stream);
 int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,

@@ -1316,6 +1316,25 @@ def case_thin_product(dev, M, N, K):
     assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -20 * size).all())
 
 
+def case_lora_u(dev, M, K, r, counts=None):
+    """An adapter's forward projection with its scaling: the bits of the general product (whole and cut reductions; rows by expert) and of its scaling, into columns of a wider tensor."""
+    from aria_amd import ops
+
+    x = rnd(M, K + 8, seed=M).to(dev)[:, :K]
+    if counts is None:
+        w, off = rnd(r, K, seed=2).to(dev), None
+        want = ops.gemm(x, w)
+    else:
+        off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=dev)
+        w = rnd(len(counts), K, r, seed=2).to(dev)
+        want = ops.grouped_gemm(x, w, off)
+    assert ops.lora_u_takes(x, w, off is not None)
+    out = torch.full((M, r + 3), 7.0, dtype=bf16, device=dev)
+    for scale in (4.0, 0.3):
+        assert torch.equal(ops.lora_u(x, w, scale, offsets=off, out=out[:, 2:2 + r]), ops.lora_scale(want, scale))
+    assert bool((out[:, :2] == 7).all() and (out[:, 2 + r:] == 7).all())
+
+
 def case_sort_rows(dev, T, k, E):
     """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
     from aria_amd import ops
