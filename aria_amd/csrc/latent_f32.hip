@@ -7,6 +7,7 @@
 //
 // Bound by the matrix pipe's 32-bit rate at (cw + R) / 4 multiply steps a tile, and by the tiles a wave walks.  As one (token, head) a workgroup on the vector
 // pipe the latents were read once for every head: 883 tokens of four prompts, 8 heads, 320-column rows 185 us, now 55; 4 single tokens of 250 keys 22 us, now 15 (four splits).
+// The first keys requested before the queries are staged, and columns dealt to threads without divisions: those 4 tokens 15.3 -> 12.6, 614 tokens of four prompts 40 -> 32.
 #include "aria_device.h"
 #include "aria_hip.h"
 #include <algorithm>
@@ -21,22 +22,20 @@ constexpr size_t lds_bytes(int64_t cw) { return size_t(16 + 16 * NW) * size_t(cw
 // NB: blocks of 16 value columns held; PF: 16-byte pieces of a key tile a lane holds in flight (cw <= 16 PF); tpb: tokens of a workgroup, hp: columns each
 template <int NB, int PF, int NW>
 __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* qa, const float* cache, Shape s, const int32_t* slot, const int32_t* pos, float* part_o,
-                                                                  float* part_ml, int T, int tpb, int hp, int splits) {
+                                                                  float* part_ml, int T, int tpb, int hs, int splits) {
     ARIA_DYN_SMEM(smem);
-    const int cw = int(s.cw), P = cw + 4, R = int(s.R), H = int(s.H), vecs = cw / 4;
+    const int cw = int(s.cw), P = cw + 4, R = int(s.R), H = int(s.H);
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c = l & 15;
     float* sQ = reinterpret_cast<float*>(smem);            // [16 columns][P]
     float* sK = sQ + 16 * P + w * 16 * P;                  // this wave's keys [16][P]
     float* state = sQ + (16 + 16 * NW) * P;                // [NW][16] maxima, [NW][16] sums
-    const int t0 = blockIdx.y * tpb, h0 = blockIdx.x * hp, z = blockIdx.z;
-    const int tok = t0 + c / hp, head = h0 + c % hp;
+    const int t0 = blockIdx.y * tpb, h0 = blockIdx.x << hs, hp = 1 << hs, z = blockIdx.z;
+    const int tok = t0 + (c >> hs), head = h0 + (c & (hp - 1));
     const bool real = tok < T && head < H && c < tpb * hp;
-    for (int i = t; i < 16 * vecs; i += NW * 64) {
-        const int col = i / vecs, at = (i % vecs) * 4, tk = t0 + col / hp, hd = h0 + col % hp;
-        const bool in = tk < T && hd < H && col < tpb * hp;
-        *reinterpret_cast<f32x4*>(sQ + col * P + at) = in ? *reinterpret_cast<const f32x4*>(qa + ((long long)tk * H + hd) * cw + at) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    sync();
+    // a column of 16 to a thread where the columns are gone through one by one, LANES threads each
+    constexpr int LANES = NW * 4;
+    const int col = t / LANES, lane = t % LANES, col_tok = t0 + (col >> hs), col_head = h0 + (col & (hp - 1));
+    const bool col_real = col_tok < T && col_head < H && col < tpb * hp;
     const float scale2 = s.scale * 1.4426950408889634f;
     float m = -INFINITY, lsum = 0.f;
     f32x4 o[NB];
@@ -53,11 +52,11 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* q
     };
     // keys [first, end) of the rows at `base`, all of them seen by the columns with `mine` and by no other; tiles counted on from `tiles`
     int tiles = 0;
-    auto walk = [&](const float* base, int first, int end, bool mine, bool everyone) __attribute__((always_inline)) {
+    auto walk = [&](const float* base, int first, int end, bool mine, bool everyone, bool requested) __attribute__((always_inline)) {
         const int n = (end - first + 15) / 16, turns = NW * splits, me = z * NW + w;
         int u = (me - tiles % turns + turns) % turns;
         tiles += n;
-        if (u < n) request(base, first + 16 * u, end);
+        if (u < n && !requested) request(base, first + 16 * u, end);
         for (; u < n; u += turns) {
             const int k0 = first + 16 * u;
             wave_barrier();
@@ -110,15 +109,26 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* q
             }
         }
     };
-    for (int i = 0; i < tpb && t0 + i < T;) {   // neighbouring tokens of one sequence together: what all of them see, then what is one's alone
+    // neighbouring tokens of one sequence together: what all of them see, then what is one's alone
+    int j = 0, common = 0;
+    auto group_from = [&](int i) __attribute__((always_inline)) {
         const int sl = slot[t0 + i];
-        int j = i + 1, common = pos[t0 + i] + 1;
+        j = i + 1, common = pos[t0 + i] + 1;
         for (; j < tpb && t0 + j < T && slot[t0 + j] == sl; ++j) common = min(common, pos[t0 + j] + 1);
-        const float* base = cache + (long long)sl * s.S_cap * cw;
+        return cache + (long long)sl * s.S_cap * cw;
+    };
+    const float* base = group_from(0);
+    if (16 * (z * NW + w) < common) request(base, 16 * (z * NW + w), common);   // (the first keys come while the queries are staged)
+    for (int at = 4 * lane; at < cw; at += 4 * LANES)
+        *reinterpret_cast<f32x4*>(sQ + col * P + at) =
+            col_real ? *reinterpret_cast<const f32x4*>(qa + ((long long)col_tok * H + col_head) * cw + at) : f32x4{0.f, 0.f, 0.f, 0.f};
+    sync();
+    for (int i = 0; i < tpb && t0 + i < T;) {
+        if (i) base = group_from(i);
         const bool group = real && tok >= t0 + i && tok < t0 + j;
-        walk(base, 0, common, group, i == 0 && j == min(tpb, T - t0));
+        walk(base, 0, common, group, i == 0 && j == min(tpb, T - t0), i == 0);
         for (int b = i; b < j; ++b)
-            if (pos[t0 + b] + 1 > common) walk(base, common, pos[t0 + b] + 1, real && tok == t0 + b, false);
+            if (pos[t0 + b] + 1 > common) walk(base, common, pos[t0 + b] + 1, real && tok == t0 + b, false, false);
         i = j;
     }
     // ---- the waves' states meet
@@ -136,13 +146,19 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* q
                                                                                                      : f32x4{o[n16][0] * f, o[n16][1] * f, o[n16][2] * f, o[n16][3] * f};
     sync();
     const float* all = sQ + 16 * P;
-    for (int i = t; i < 16 * R; i += NW * 64) {
-        const int col = i / R, d = i % R, tk = t0 + col / hp, hd = h0 + col % hp;
-        if (tk >= T || hd >= H || col >= tpb * hp) continue;
-        float v = 0.f;
+    if (col_real) {
+        float* out = part_o + (((long long)col_tok * splits + z) * H + col_head) * R;
+        auto sums = [&](auto v, int d) __attribute__((always_inline)) {
+            using V = decltype(v);
+            v = *reinterpret_cast<const V*>(all + col * P + d);
 #pragma unroll
-        for (int k = 0; k < NW; ++k) v += all[k * 16 * P + col * P + d];
-        part_o[(((long long)tk * splits + z) * H + hd) * R + d] = v;
+            for (int k = 1; k < NW; ++k) v += *reinterpret_cast<const V*>(all + k * 16 * P + col * P + d);
+            *reinterpret_cast<V*>(out + d) = v;
+        };
+        if (R & 3)
+            for (int d = lane; d < R; d += LANES) sums(0.f, d);
+        else
+            for (int d = 4 * lane; d < R; d += 4 * LANES) sums(f32x4{}, d);
     }
     if (w == 0 && q4 == 0 && real) {
         float sum = 0.f;
@@ -162,12 +178,12 @@ __attribute__((visibility("hidden"))) bool aria_latent_f32_takes(const AriaLaten
 // Tokens a workgroup shares latents between only where many follow one another (prompts): single tokens belong to different sequences.
 __attribute__((visibility("hidden"))) int aria_latent_f32_attn(const float* qa, const float* cache, const AriaLatentShape& s, const int32_t* slot, const int32_t* pos, float* part_o, float* part_ml, int64_t T,
                          int64_t splits, void* stream) {
-    int hp = 16;
-    while (hp > 1 && hp / 2 >= s.H) hp /= 2;
-    const int tpb = T > 64 ? 16 / hp : 1;
+    int hs = 4;   // 2^hs columns a token
+    while (hs > 0 && (1 << hs >> 1) >= s.H) --hs;
+    const int hp = 1 << hs, tpb = T > 64 ? 16 / hp : 1;
     const dim3 grid(unsigned((s.H + hp - 1) / hp), unsigned((T + tpb - 1) / tpb), unsigned(splits));
 #define ARIA_LATENT32(NB, PF, NW)                                                                                                                                   \
-    ARIA_LAUNCH((latent_attn_f32_kernel<NB, PF, NW>), grid, dim3(NW * 64), lds_bytes<NW>(s.cw), stream, qa, cache, s, slot, pos, part_o, part_ml, int(T), tpb, hp, \
+    ARIA_LAUNCH((latent_attn_f32_kernel<NB, PF, NW>), grid, dim3(NW * 64), lds_bytes<NW>(s.cw), stream, qa, cache, s, slot, pos, part_o, part_ml, int(T), tpb, hs, \
                 int(splits))
     if (s.R <= 256 && s.cw <= 384)
         ARIA_LATENT32(16, 24, 4);
