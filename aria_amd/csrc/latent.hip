@@ -92,22 +92,24 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const T* proj, Shape
     const int t = threadIdx.x, l = t & 63, w = t >> 6;
     const int RB = int(s.R + 127) / 128, unit = blockIdx.x, t0 = blockIdx.y * NB;
     const int nb = min(NB, n_tok - t0), half = int(s.rot) >> 1;
-    if (unit == s.H * RB) {   // cache rows: the whole workgroup on one token at a time
-        for (int b = 0; b < nb; ++b) {
+    // cache rows: a wave a token, the sums of squares added as four waves on one token add them.  Four waves on each token in turn: 4 float32 tokens 7.1 us, now 6.8, 614 23.0, now 20.8; a
+    // step of 16 bf16 tokens, three layers, 795 -> 786
+    if (unit == s.H * RB) {
+        for (int b = w; b < nb; b += 4) {
             const int tok = t0 + b, ps = pos[tok];
             const T* src = proj + (long long)tok * s.ldp + s.kv_off;
-            float ss = 0.f;
-            for (int i = t; i < s.R; i += 256) {
-                const float v = ldf(src + i);
-                ss += v * v;
-            }
-            ss = wave_sum_bcast(ss);
-            sync();
-            if (l == 0) red[w] = ss;
-            sync();
-            const float r = 1.f / sqrtf((red[0] + red[1] + red[2] + red[3]) / float(s.R) + s.eps);
             T* row = cache + ((long long)slot[tok] * s.S_cap + ps) * s.cw;
-            for (int i = t; i < s.cw; i += 256) stf(row + i, latent_column<T>(src, s, rope + (long long)ps * s.rot, wn, r, i));
+            float ss[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int i = l; i < s.R; i += 256)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const float v = ldf(src + min(i + 64 * p, int(s.R) - 1));
+                    if (i + 64 * p < s.R) ss[p] += v * v;
+                }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) ss[p] = wave_sum_bcast(ss[p]);
+            const float r = 1.f / sqrtf((ss[0] + ss[1] + ss[2] + ss[3]) / float(s.R) + s.eps);
+            for (int i = l; i < s.cw; i += 64) stf(row + i, latent_column<T>(src, s, rope + (long long)ps * s.rot, wn, r, i));
         }
         return;
     }
