@@ -874,6 +874,21 @@ def case_swiglu(dev, exact):
 
 
 # ------------------------------------------------------------------------------------------ norm / rope
+def case_vit_positions(dev, R, patch, side, cut):
+    """Patch masks and position ids of a whole image and of one whose right ``cut[1]`` columns and lower ``cut[0]`` rows are padding, against the oracle's."""
+    from aria_amd import ops
+    from oracle import aria_oracle as O
+
+    pm = torch.ones((2, R, R), dtype=torch.bool)
+    pm[1, R - cut[0]:], pm[1, :, R - cut[1]:] = False, False
+    pm[1, -1, 0] = True   # (one pixel makes its patch)
+    mask = ops.vit_patch_mask(pm.to(dev), patch)
+    want = O.vit_patch_mask(pm, patch)
+    assert torch.equal(mask.cpu().bool(), want.bool().view(mask.shape))
+    bounds = torch.arange(1 / side, 1.0, 1 / side, dtype=torch.float32).to(dev)
+    assert torch.equal(ops.vit_pos_ids(mask, bounds, side).cpu().long(), O.vit_position_ids(want, side))
+
+
 def case_colsum_rows(dev, n, D):
     """Column sums of 32-bit rows: eight groups, every eighth row in order, then the groups in order; rounded once.  The same bits whatever is in flight together."""
     from aria_amd import hip, ops

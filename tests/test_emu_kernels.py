@@ -53,6 +53,11 @@ def test_swiglu():
     C.case_swiglu(DEV, exact=True)
 
 
+@pytest.mark.parametrize("R,patch,side,cut", [(28, 14, 4, (0, 14)), (294, 14, 21, (100, 17)), (100, 20, 5, (40, 20))])
+def test_vit_positions(R, patch, side, cut):
+    C.case_vit_positions(DEV, R, patch, side, cut)
+
+
 @pytest.mark.parametrize("n", [1, 56, 57, 64, 71, 201])
 def test_colsum_rows(n):
     C.case_colsum_rows(DEV, n, 40)
