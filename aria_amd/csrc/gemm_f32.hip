@@ -69,6 +69,9 @@ template <int MT, int NT, int NW, int FIN>
 __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     constexpr bool PAIR = FIN == ARIA_F32_PAIR;
     constexpr int WS = PAIR ? 2 : 1;
+    // 16 x 16 outputs: a wave takes two neighbouring steps, whole lines of both operands (us, one / two: 4 x 64000 x 1536 84 / 78, 16 x 32000 x 1024 43.6 / 42.0, 4 x 12288 x 2048
+    // 26.4 / 25.7, 2 x 8192 x 1024 13.1 / 13.0)
+    constexpr int PER = MT * NT == 1 ? 2 : 1, LINE = 16 * PER;
     constexpr int DEPTH = 4, TM = 16 * MT, TN = 16 * NT;
     ARIA_SMEM_STATIC float red[WS][NW][TM][TN + 1];
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15;
@@ -78,11 +81,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     if (p.offsets && !find_rows(p, y, TM, e, m0, m_end)) return;
     const float *ap[MT], *wp[WS][NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) ap[i] = p.A + row_of(p, min(m0 + 16 * i + c16, m_end - 1)) * p.lda + w * 16 + q4 * 4;
+    for (int i = 0; i < MT; ++i) ap[i] = p.A + row_of(p, min(m0 + 16 * i + c16, m_end - 1)) * p.lda + w * LINE + q4 * 4;
 #pragma unroll
     for (int z = 0; z < WS; ++z)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) wp[z][j] = (z ? p.W2 : p.W) + e * p.strideW + (long long)min(n0 + 16 * j + c16, p.N - 1) * p.ldw + w * 16 + q4 * 4;
+        for (int j = 0; j < NT; ++j) wp[z][j] = (z ? p.W2 : p.W) + e * p.strideW + (long long)min(n0 + 16 * j + c16, p.N - 1) * p.ldw + w * LINE + q4 * 4;
     f32x4 acc[WS][MT][NT];
 #pragma unroll
     for (int z = 0; z < WS; ++z)
@@ -90,7 +93,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[z][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int steps = p.K / 16, mine = (steps - w + NW - 1) / NW;   // whole steps; this wave's: w, w + NW, ...
+    // whole steps; this wave's are groups w, w + NW, .. of PER, the last of which may be short
+    const int steps = p.K / 16, groups = (steps + PER - 1) / PER, own = (groups - w + NW - 1) / NW;
+    const int mine = own * PER - (own > 0 && w + (own - 1) * NW == groups - 1 ? groups * PER - steps : 0);
+    auto at = [](int s) __attribute__((always_inline)) { return (long long)((s / PER) * NW * LINE + (s % PER) * 16); };
     struct Step {
         f32x4 a[MT], b[WS][NT];
     };
@@ -115,13 +121,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     };
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u)
-        if (u < mine) load(u * NW * 16, x[u]);
+        if (u < mine) load(at(u), x[u]);
     int s = 0;
     for (; s + 2 * DEPTH <= mine; s += DEPTH) {
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
             use(x[u]);
-            load((s + u + DEPTH) * NW * 16, x[u]);
+            load(at(s + u + DEPTH), x[u]);
         }
     }
     for (; s < mine; s += DEPTH) {   // the last DEPTH .. 2 DEPTH - 1 steps (or fewer altogether)
@@ -129,12 +135,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
         for (int u = 0; u < DEPTH; ++u) {
             if (s + u >= mine) break;
             use(x[u]);
-            if (s + u + DEPTH < mine) load((s + u + DEPTH) * NW * 16, x[u]);
+            if (s + u + DEPTH < mine) load(at(s + u + DEPTH), x[u]);
         }
     }
     if ((p.K & 15) && w == steps % NW) {   // the rest of the row, K % 16 = 4, 8 or 12 columns: lanes behind it hold zeros in both operands
         const bool in = q4 * 4 < (p.K & 15);
-        load(in ? mine * NW * 16 : -(w * 16 + q4 * 4), x[0]);   // (not in: a column of the same row)
+        load(in ? steps * 16 - w * LINE : -(w * LINE + q4 * 4), x[0]);   // (not in: a column of the same row)
         if (!in) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) x[0].a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
