@@ -77,6 +77,7 @@ SIGNATURES = {
     "aria_lora_u_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_down_bf16": [P, P, I32, P, P, I64, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_up_bf16": [P, P, I32, P, P, P, I64, I64, I64, I64, I64, F32, P],
+    "aria_lora_up_swiglu_bf16": [P, P, I32, P, P, P, P, P, I64, I64, I64, I64, I64, F32, P],
     "aria_lora_wgrad_bf16": [P, P, P, I32, I64, I64, I64, I64, I64, P, I64, P],
     "aria_grouped_gemm_wgrad_gather_bf16": [P, P, P, P, P, I64, I64, I64, I64, I64, I64, I32, I32, P],
     "aria_grouped_gemm_wgrad_gather_sized_bf16": [P, P, P, P, P, I64, I64, I64, I64, I64, I64, I32, I32, I64, P],

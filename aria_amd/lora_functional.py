@@ -16,7 +16,7 @@ What runs here, per module:
     launches (their adapters enter side by side with a block-diagonal B);
   * backward: the base input gradients exactly as the un-adapted layer computes them (weight gradients of the frozen base are skipped);
     per adapter d_u = scaling * dy lora_B^T (thin: ``ops.lora_down``, ranks 8 and 16), d lora_B = u^T dy, d lora_A = dropout(x)^T d_u (``ops.lora_wgrad``), and the adapter's input
-    gradient ``mask * (d_u lora_A) / (1 - p)`` added into dx in one pass (``ops.lora_up_``; other ranks: a product, then ``ops.dropout_bwd_``).
+    gradient ``mask * (d_u lora_A) / (1 - p)`` added into dx in one pass (``ops.lora_up_``, or ``ops.lora_up_swiglu`` through the backward of silu(gate) * up in front of it; other ranks: a product, then ``ops.dropout_bwd_``).
 Everything else of the layer (RMSNorm with the residual folded in, RoPE, flash attention, router, dispatch, un-permute + shared add) is the
 un-adapted layer's code path (aria_amd.functional).  The module-by-module form (aria_amd.lora.GroupedGemmLoraLayer / LinearLoraLayer called
 as modules) stays as the reference arrangement the tests compare against.
@@ -108,11 +108,11 @@ def dense_lora_fwd(x: torch.Tensor, w: torch.Tensor, sites: List[Optional[LoraSi
     return out, dict(live=live, drops=drops, U=U, Bx=Bx, starts=starts, rows=rows)
 
 
-def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: List[str]) -> None:
+def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: List[str], h: Optional[torch.Tensor] = None):
     """Adds the adapters' input gradients into dx (which already holds the base input gradient) and writes d lora_A / d lora_B into
-    grads[key] = (dA, dB)."""
+    grads[key] = (dA, dB).  ``h``: dx is the gradient of silu(gate) * up of h = [gate | up] and not wanted itself; -> h's gradient."""
     if ctx is None:
-        return
+        return ops.swiglu_bwd(h, dx) if h is not None else None
     live, starts, rows, U = ctx["live"], ctx["starts"], ctx["rows"], ctx["U"]
     thin = dx.is_contiguous() and dx.shape[0] > 0 and all(ops.lora_thin(s.a.shape[0], n) and starts[j] % 8 == 0 for j, s in live for n in (rows[j], dx.shape[1]))
     if not thin:
@@ -124,7 +124,10 @@ def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: L
         if thin:
             du = ops.lora_down(dy[:, r0:r1], _factor(s.b), s.scaling, w_oc=True)
             dA, dB = ops.lora_wgrad(d.xd, du, n_first=False), ops.lora_wgrad(dy[:, r0:r1], U[:, c0:c0 + r], n_first=True)
-            ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p)
+            if h is not None and len(live) == 1 and h.is_contiguous():
+                dx, h = ops.lora_up_swiglu(dx, du, _factor(s.a), d.mask, d.p, h), None
+            else:
+                ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p)
         else:
             du = _scaled(dU[:, c0:c0 + r].contiguous(), s.scaling)
             dA = ops.gemm(du, d.xd, a_oc=True, b_oc=True)         # [r, K] = d_u^T dropout(x)
@@ -135,6 +138,7 @@ def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: L
                 ops.dropout_bwd_(dx, ops.gemm(du, s.a, b_oc=True), d.mask, d.p)
         grads[keys[j]] = (dA, dB)
         c0 += r
+    return dx if h is None else ops.swiglu_bwd(h, dx)
 
 
 # ------------------------------------------------------------------------------------------------------------------ grouped (expert) sites
@@ -149,9 +153,10 @@ def grouped_lora_fwd(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, si
     return out, dict(site=site, drop=d, U=U)
 
 
-def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Tensor, grads: dict, key: str) -> None:
+def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Tensor, grads: dict, key: str, h: Optional[torch.Tensor] = None):
+    """``dense_lora_bwd`` of the experts' adapter"""
     if ctx is None:
-        return
+        return ops.swiglu_bwd(h, dx) if h is not None else None
     s, d = ctx["site"], ctx["drop"]
     E = s.a.shape[0]
     thin = ops.lora_thin(s.a.shape[2], dy.shape[1]) and dx.is_contiguous()
@@ -161,6 +166,9 @@ def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Ten
         du = _scaled(ops.grouped_gemm(dy, s.b, offsets, w_is_kn=False), s.scaling)
     dB = ops.grouped_gemm_wgrad(ctx["U"], dy, offsets, E)                                   # [E, r, N]
     dA = ops.grouped_gemm_wgrad(d.xd, du, offsets, E)                                       # [E, K, r]
+    grads[key] = (dA, dB)
+    if thin and h is not None and h.is_contiguous():
+        return ops.lora_up_swiglu(dx, du, _factor(s.a), d.mask, d.p, h, offsets=offsets)
     if thin:
         ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p, offsets=offsets)                             # d_u lora_A[e]^T
     else:
@@ -169,7 +177,7 @@ def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Ten
             dx.add_(term)
         else:
             ops.dropout_bwd_(dx, term, d.mask, d.p)
-    grads[key] = (dA, dB)
+    return dx if h is None else ops.swiglu_bwd(h, dx)
 
 
 # ------------------------------------------------------------------------------------------------------------------ the layer
@@ -239,8 +247,7 @@ def decoder_layer_lora_bwd(dout, c, p: dict, cos, sin, need_base=None) -> Tuple[
         d_h1 = ops.grouped_gemm_dswiglu(d_eo, p["fc2"], offsets, c["h1"])
     else:   # the adapter's input gradient belongs to d_act, in front of the SwiGLU backward
         d_act = ops.grouped_gemm(d_eo, p["fc2"], offsets, w_is_kn=False)
-        grouped_lora_bwd(d_eo, c["c_fc2"], offsets, d_act, g, "fc2")
-        d_h1 = ops.swiglu_bwd(c["h1"], d_act)
+        d_h1 = grouped_lora_bwd(d_eo, c["c_fc2"], offsets, d_act, g, "fc2", h=c["h1"])
     if "fc2" in need:
         gb["fc2"] = ops.grouped_gemm_wgrad(c["act"], d_eo, offsets, E)
     d_perm = ops.grouped_gemm(d_h1, p["fc1"], offsets, w_is_kn=False)
@@ -253,8 +260,7 @@ def decoder_layer_lora_bwd(dout, c, p: dict, cos, sin, need_base=None) -> Tuple[
         d_gu = ops.gemm_dswiglu(dout, p["down"], c["gu"], b_oc=True)
     else:
         d_sact = ops.gemm(dout, p["down"], b_oc=True)
-        dense_lora_bwd(dout, c["c_down"], d_sact, g, ["down"])
-        d_gu = ops.swiglu_bwd(c["gu"], d_sact)
+        d_gu = dense_lora_bwd(dout, c["c_down"], d_sact, g, ["down"], h=c["gu"])
     if "down" in need:
         gb["down"] = ops.gemm(dout, c["sact"], a_oc=True, b_oc=True)
     ops.gemm(d_gu, c["wgu"], b_oc=True, out=dhn, accumulate=True)

@@ -342,6 +342,22 @@ def lora_up_(dx: torch.Tensor, du: torch.Tensor, a: torch.Tensor, mask, p: float
     return dx
 
 
+def lora_up_swiglu(d: torch.Tensor, du: torch.Tensor, a: torch.Tensor, mask, p: float, h: torch.Tensor, offsets=None) -> torch.Tensor:
+    """``swiglu_bwd(h, lora_up_(d, du, a, mask, p, offsets))`` in one launch: d [M, K] is only read, h [M, 2 K] = [gate | up] -> its gradient."""
+    _chk(d, name="d"), _chk(du, name="du"), _chk(a, name="a"), _chk(h, name="h")
+    M, K = d.shape
+    r = du.shape[1]
+    if not (d.is_contiguous() and a.is_contiguous() and h.is_contiguous()) or du.shape[0] != M or tuple(h.shape) != (M, 2 * K) or (mask is not None and mask.numel() * 8 != d.numel()):
+        raise ValueError("lora_up_swiglu: contiguous d, a and h [M, 2 K], one mask byte per 8 elements")
+    if tuple(a.shape) != ((r, K) if offsets is None else (a.shape[0], K, r)):
+        raise ValueError("lora_up_swiglu: a must be [r, K], the experts' [E, K, r]")
+    dh = torch.empty_like(h)
+    hip.get_lib().call("aria_lora_up_swiglu_bf16", _p(du), _p(a), int(offsets is None), _p(mask) if mask is not None else None, _p(d), _p(h), _p(dh),
+                       _p(offsets) if offsets is not None else None, a.shape[0] if offsets is not None else 1, M, K, r, _rowmajor_2d(du, "du"),
+                       1.0 if mask is None else 1.0 / (1.0 - p), _stream(d))
+    return dh
+
+
 def lora_wgrad(y: torch.Tensor, u: torch.Tensor, n_first: bool) -> torch.Tensor:
     """u^T y as [r, N], or with ``n_first`` its transpose [N, r]: y [M, N], u [M, r], unit-stride rows."""
     _chk(y, name="y"), _chk(u, name="u")

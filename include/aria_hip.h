@@ -162,6 +162,10 @@ int aria_lora_down_bf16(const void* X, const void* W, int w_oc, void* U, const i
                         float scale, void* stream);
 int aria_lora_up_bf16(const void* DU, const void* A, int a_oc, const void* mask, void* DX, const int32_t* offsets, int64_t E, int64_t M, int64_t K, int64_t r,
                       int64_t ldu, float scale, void* stream);
+/* _up on D [M, K], the gradient of silu(gate) up, straight through the backward of that (aria_swiglu_bwd on H [M, 2 K] = [gate | up], dense): DH [M, 2 K]; D is only read.  Bit for bit
+ * the two launches. */
+int aria_lora_up_swiglu_bf16(const void* DU, const void* A, int a_oc, const void* mask, const void* D, const void* H, void* DH, const int32_t* offsets, int64_t E, int64_t M, int64_t K,
+                             int64_t r, int64_t ldu, float scale, void* stream);
 int aria_lora_wgrad_bf16(const void* Y, const void* U, void* out, int n_first, int64_t M, int64_t N, int64_t r, int64_t ldy, int64_t ldu, float* workspace,
                          int64_t workspace_floats, void* stream);
 

@@ -1350,6 +1350,20 @@ def case_lora_u(dev, M, K, r, counts=None):
     assert bool((out[:, :2] == 7).all() and (out[:, 2 + r:] == 7).all())
 
 
+def case_lora_up_swiglu(dev, M, K, r, counts=None):
+    """An adapter's masked input gradient through the backward of silu(gate) * up in one launch: the bits of the two, the gradient that it starts from untouched."""
+    from aria_amd import ops
+
+    d, h, du, x = rnd(M, K, seed=1).to(dev), rnd(M, 2 * K, seed=2).to(dev), rnd(M, r, seed=3).to(dev), rnd(M, K, seed=4).to(dev)
+    off = None if counts is None else torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=dev)
+    a = (rnd(r, K, seed=5) if counts is None else rnd(len(counts), K, r, seed=5)).to(dev)
+    for p, mask in ((0.0, None), (0.3, ops.dropout(x, 0.3, 9)[1])):
+        before = d.clone()
+        got = ops.lora_up_swiglu(d, du, a, mask, p, h, offsets=off)
+        assert torch.equal(d, before)
+        assert torch.equal(got, ops.swiglu_bwd(h, ops.lora_up_(before, du, a, mask, p, offsets=off)))
+
+
 def case_sort_rows(dev, T, k, E):
     """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
     from aria_amd import ops

@@ -282,6 +282,11 @@ def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
 
 
+@pytest.mark.parametrize("M,K,r,counts", [(37, 72, 8, None), (33, 520, 16, [1, 0, 32])])
+def test_lora_up_swiglu(M, K, r, counts):
+    C.case_lora_up_swiglu(DEV, M, K, r, counts)
+
+
 @pytest.mark.parametrize("M,K,r,counts", [(37, 128, 8, None), (300, 1024, 16, None), (75, 192, 8, [40, 0, 1, 34])])
 def test_lora_u(M, K, r, counts):
     C.case_lora_u(DEV, M, K, r, counts)

@@ -276,6 +276,11 @@ def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
 
 
+@pytest.mark.parametrize("M,K,r,counts", [(1, 8, 8, None), (37, 72, 8, None), (33, 520, 16, [1, 0, 32]), (4096, 3328, 8, None), (4662, 1664, 8, [73] * 63 + [63])])
+def test_lora_up_swiglu(M, K, r, counts):
+    C.case_lora_up_swiglu(DEV, M, K, r, counts)
+
+
 @pytest.mark.parametrize("M,K,r,counts", [(1, 64, 16, None), (37, 128, 8, None), (300, 1024, 16, None), (777, 2560, 8, None), (4096, 2560, 8, None), (4096, 3328, 16, None), (75, 192, 8, [40, 0, 1, 34]),
                                            (4662, 2560, 8, [73] * 63 + [63]), (24576, 1664, 16, [384] * 64)])
 def test_lora_u(M, K, r, counts):
