@@ -571,7 +571,7 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
         return plan;
     }
     if (p.mode == 2) {   // rows: of all experts together, < 0: not known
-        // Weight gradients by expert, 64 of them, 256 x 256 / 128 x 256 tiles: 2560 x 3328 at 6 rows each on average 283 / 222, 28 rows 301 / 237, 73 332 / 301, 140 405 / 392, 384
+        // Weight gradients by expert that strips do not take, 64 of them, 256 x 256 / 128 x 256 tiles: 2560 x 3328 at 6 rows each on average 283 / 222, 28 rows 301 / 237, 73 332 / 301, 140 405 / 392, 384
         // 641 / 634, 768 946 / 976; 1664 x 2560 139 / 114, 149 / 125, 171 / 161, 217 / 204, 328 / 328, 507 / 500.
         if (rows >= 0 && rows < 400ll * p.E) plan.form = 3;
         return plan;
