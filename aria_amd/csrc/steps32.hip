@@ -139,13 +139,12 @@ int aria_latent_step_f32(const AriaLatentStack* st, const AriaLatentLayer* L, in
         const Mixture m = mixture(z, y, T, D);
         const int64_t ldl = (y.E + 7) & ~int64_t(7), M = T * y.k;
         rc = product(c.h, y.w_router, m.logits, T, ldl, D, stream);
-        int sorted = rc;
-        if (rc == ARIA_OK) sorted = aria_route_groups_sorted(m.logits, y.correction, m.weights, m.idx, m.offsets, m.src, m.inv, T, y.E, ldl, y.groups, y.keep, y.k, stream);
-        if (sorted == ARIA_ERR_UNSUPPORTED) {   // more tokens, more experts
-            rc = aria_moe_route_groups(m.logits, y.correction, m.weights, m.idx, m.counts, T, y.E, ldl, y.groups, y.keep, y.k, stream);
-            if (rc == ARIA_OK) rc = aria_moe_sort(m.idx, m.counts, m.offsets, m.src, m.inv, m.ws, T, y.E, y.k, stream);
-        } else {
-            rc = sorted;
+        if (rc == ARIA_OK) {
+            rc = aria_route_groups_sorted(m.logits, y.correction, m.weights, m.idx, m.offsets, m.src, m.inv, T, y.E, ldl, y.groups, y.keep, y.k, stream);
+            if (rc == ARIA_ERR_UNSUPPORTED) {   // more tokens, more experts
+                rc = aria_moe_route_groups(m.logits, y.correction, m.weights, m.idx, m.counts, T, y.E, ldl, y.groups, y.keep, y.k, stream);
+                if (rc == ARIA_OK) rc = aria_moe_sort(m.idx, m.counts, m.offsets, m.src, m.inv, m.ws, T, y.E, y.k, stream);
+            }
         }
         AriaGemmF32 up = dense(c.h, y.w_gate, m.act, M, y.ff, D), down = dense(m.act, y.w_down, m.eo, M, D, y.ff);
         up.W2 = static_cast<const float*>(y.w_up), up.rows = m.src, up.per = int(y.k), up.offsets = down.offsets = m.offsets, up.E = down.E = int(y.E);
