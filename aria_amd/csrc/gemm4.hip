@@ -26,6 +26,7 @@
 // The order of the products of an output element is that of the 256 x 256 kernel: the same bits where neither splits the reduction.
 #include "aria_hip.h"
 #include "gemm_params.h"
+#include "wgrad.h"
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -143,37 +144,22 @@ __device__ __forceinline__ void finish_piece(const P& p, char* C, const char* pa
     st16(out + (long long)m * p.ldc + n0 + cc, v);
 }
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
-__global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
+// Where a workgroup's tile lies: row tile from m0 (rows end at m_end), column tile tn, its reduction, its expert's operand and result; slab >= 0: piece ks of a split reduction
+struct Tile4 {
+    int tn, m0, m_end, k_begin, k_len;
+    long long b_off, c_off;
+    int slab, ks;
+};
+
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER>
+__device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& place, char* smem) {
     using T = Shape4<WM, WN, MI, NI, KD, S>;
     constexpr int BM = T::BM, BN = T::BN, PA = T::PA, PB = T::PB, STAGE = T::STAGE, ROWP = T::ROWP, HALVES = KD / 16;
     constexpr bool GATHER = gathers(VER), GLU = gated(VER), GATHER_K = VER == 11, PLAIN = VER == 3 || VER == 11;
-    ARIA_DYN_SMEM(smem);
-    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), wm = w / WN, wn = w % WN;
-
-    int tn = 0, tmi = 0, slab = -1, ks = 0;
-    if (p.mode == 1) {
-        // aria_grouped_tile below
-    } else if (p.split > 1) {
-        slab = blockIdx.x;
-        ks = slab % p.split;
-        if (!aria_tile_from_pos(p, slab / p.split, tmi, tn)) return;
-    } else if (!aria_tile_coords(p, blockIdx.x, int(gridDim.x), tmi, tn)) {
-        return;
-    }
     constexpr int STEP = GLU ? BN / 2 : BN;
-    long long b_off = 0, c_off = 0;
-    int m0 = tmi * BM, m_end = p.M, k_begin = 0, k_len = p.K;
-    if (p.mode == 2) {
-        k_begin = p.offsets[blockIdx.y];
-        k_len = p.offsets[blockIdx.y + 1] - k_begin;
-        c_off = (long long)blockIdx.y * p.strideC;
-    } else if (p.mode == 1) {
-        int expert = 0;
-        if (!aria_grouped_tile<BM>(p, blockIdx.x, l, expert, m0, m_end, tn)) return;
-        expert = first_lane(expert), m0 = first_lane(m0), m_end = first_lane(m_end), tn = first_lane(tn);
-        b_off = (long long)(p.expert_mod > 0 ? expert % p.expert_mod : expert) * p.strideB;
-    }
+    const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), wm = w / WN, wn = w % WN;
+    const int tn = place.tn, m0 = place.m0, m_end = place.m_end, k_begin = place.k_begin, k_len = place.k_len, slab = place.slab, ks = place.ks;
+    const long long b_off = place.b_off, c_off = place.c_off;
     const int n0 = tn * STEP;
     char* C = static_cast<char*>(p.C) + c_off * (p.c_f32 ? 4 : 2);
 
@@ -459,6 +445,35 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     }
 }
 
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
+    constexpr int BM = Shape4<WM, WN, MI, NI, KD, S>::BM;
+    ARIA_DYN_SMEM(smem);
+    int tn = 0, tmi = 0, slab = -1, ks = 0;
+    if (p.mode == 1) {
+        // aria_grouped_tile below
+    } else if (p.split > 1) {
+        slab = blockIdx.x;
+        ks = slab % p.split;
+        if (!aria_tile_from_pos(p, slab / p.split, tmi, tn)) return;
+    } else if (!aria_tile_coords(p, blockIdx.x, int(gridDim.x), tmi, tn)) {
+        return;
+    }
+    long long b_off = 0, c_off = 0;
+    int m0 = tmi * BM, m_end = p.M, k_begin = 0, k_len = p.K;
+    if (p.mode == 2) {
+        k_begin = p.offsets[blockIdx.y];
+        k_len = p.offsets[blockIdx.y + 1] - k_begin;
+        c_off = (long long)blockIdx.y * p.strideC;
+    } else if (p.mode == 1) {
+        int expert = 0;
+        if (!aria_grouped_tile<BM>(p, blockIdx.x, int(threadIdx.x) & 63, expert, m0, m_end, tn)) return;
+        expert = first_lane(expert), m0 = first_lane(m0), m_end = first_lane(m_end), tn = first_lane(tn);
+        b_off = (long long)(p.expert_mod > 0 ? expert % p.expert_mod : expert) * p.strideB;
+    }
+    gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER>(p, Tile4{tn, m0, m_end, k_begin, k_len, b_off, c_off, slab, ks}, smem);
+}
+
 // the sums of the slabs of gemm4_kernel<.., WM, WN, MI, NI, ..>: see gemm3_reduce_kernel; a block finishes 32 rows of 32 WN columns
 template <int WM, int WN, int MI, int NI>
 __global__ __launch_bounds__(256) void gemm4_reduce_kernel(GemmParams p) {
@@ -504,6 +519,43 @@ __global__ __launch_bounds__(256) void gemm4_reduce_kernel(GemmParams p) {
     }
 }
 
+
+// the h-th expert of more than `rows` rows and its part of the reduction; false: there are fewer
+__device__ __forceinline__ bool long_expert(const int* offsets, int E, int rows, int h, int l, int& e, int& k_begin, int& k_len) {
+    for (int e0 = 0; e0 < E; e0 += 64) {
+        const int begin = offsets[min(e0 + l, E)], n = offsets[min(e0 + l + 1, E)] - begin;
+        unsigned long long m = ballot(n > rows);
+        const int here = __builtin_popcountll(m);
+        if (h >= here) {
+            h -= here;
+            continue;
+        }
+        for (; h > 0; --h) m &= m - 1;
+        const int at = __builtin_ctzll(m);
+        e = e0 + at, k_begin = first_lane(shfl(begin, at)), k_len = first_lane(shfl(n, at));
+        return true;
+    }
+    return false;
+}
+
+// Weight gradients by strips (wgrad.h), and in front of them `tiling` workgroups that go through the tiles of the experts too long for strips; both kinds run side by side.
+template <bool GATHER>
+__global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(GemmParams p, int tiling, int parts, int per) {
+    ARIA_DYN_SMEM(smem);
+    const int bid = blockIdx.x;
+    if (bid >= tiling) {
+        wgrad_strip<GATHER>(p, bid - tiling, int(gridDim.x) - tiling, parts, per, smem);
+        return;
+    }
+    const int tiles = p.ntn * p.ntm, padded = (tiles + 7) & ~7;   // (an expert starts with XCD 0)
+    for (int i = bid;; i += tiling) {
+        int e = 0, k_begin = 0, k_len = 0, tmi = 0, tn = 0;
+        if (!long_expert(p.offsets, p.E, KC, i / padded, int(threadIdx.x) & 63, e, k_begin, k_len)) return;
+        if (i % padded >= tiles || !aria_tile_coords(p, i % padded, tiles, tmi, tn)) continue;
+        sync();   // the rows that the tile before parked have left
+        gemm4_tile<true, true, 1, 4, 4, 2, 32, 3, GATHER ? 11 : 3>(p, Tile4{tn, tmi * 128, p.M, k_begin, k_len, 0, (long long)e * p.strideC, -1, 0}, smem);
+    }
+}
 
 template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
 int launch4(GemmParams q, int split, float* ws, void* stream) {
@@ -564,10 +616,11 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     if (const char* force = std::getenv("ARIA_GEMM_FORCE")) {   // "4": tiles of 128 x 256, "46": the wide ones, "47": strips, where there is such a form
         if (force[0] != '4') return none;
         plan.form = a_oc ? (force[1] == '7' && aria_wgrad_strips_take(p, rows, true) ? 4 : 3) : force[1] == '6' && plain && p.mode == 0 ? 2 : 1;
+        plan.rows = rows;
         return plan;
     }
     if (a_oc && aria_wgrad_strips_take(p, rows)) {
-        plan.form = 4;
+        plan.form = 4, plan.rows = rows;
         return plan;
     }
     if (p.mode == 2) {   // rows: of all experts together, < 0: not known
@@ -613,8 +666,41 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     return plan;
 }
 
+// Where strips are the faster ones, us, 128 x 256 or 256 x 256 tiles / strips.  By expert, 64 of 2560 x 3328 (gathered) and 1664 x 2560, rows each on average, spread evenly, as a router
+// does (the most wanted one four times the average) and with half of all rows on one expert: 6 254 / 200, 238 / 204, 238 / 198 and 124 / 109, 120 / 108, 122 / 108; 73 361 / 220, 336 / 225,
+// 339 / 269 and 174 / 124, 166 / 126, 181 / 157; 144 471 / 292, 456 / 337, 446 / 344 and 225 / 160, 220 / 194, 244 / 207; beyond the line 192 456 / 322, 448 / 419 and 235 / 170, 237 / 218, 384 612 / 606,
+// 624 / 615 and (a quarter on one) 628 / 749.  (Experts beyond 256 rows as strips too, 128 rows at a time: 73 rows, half on one, 339 / 794, 144 446 / 1386.)  All rows on six experts: 6
+// 197 / 193 and 100 / 105, the rest zeros.  Dense: 100352 x 2560, 16 rows 266 / 106, 64 145 / 116, 200 209 / 163, 256 221 / 180; 64000 x 1536, 128
+// rows 69 / 62, 256 91 / 82.  Outputs of a few rounds have too few strips: 7680 x 2560, 64 rows 18 / 22, 256 rows 25 / 34.  Dense ones of fewer than 64 rows are the others' slower
+// kernels': 32000 x 1024, 8 rows 46 / 24, 2560 x 3328 15 / 20.
+bool aria_wgrad_strips_take(const GemmParams& p, long long rows, bool any_size) {
+    if (p.c_f32 || p.accumulate || p.bias || p.act || p.M % FT || p.N % STRIP || (reinterpret_cast<uintptr_t>(p.C) & 15) || (p.ldc & 7) || (p.strideC & 7)) return false;
+    const long long experts = p.mode == 2 ? p.E : 1, outputs = experts * p.M * p.N;
+    if (outputs <= (p.mode == 0 && p.K < 64 ? 16ll << 20 : 64ll << 20) && !any_size) return false;
+    return p.mode == 2 ? rows >= 0 && rows <= 144 * experts : p.K <= KC;
+}
+
+static int launch_wgrad_strips(GemmParams p, long long rows, void* stream) {
+    const int tiles = p.M / FT, experts = p.mode == 2 ? p.E : 1;
+    // (ten tiles of 3.5 us to a start of 4; five or twenty 257 and 235 us for 240 at 73 rows, 207 and 219 for 206 at 26)
+    const int parts = (tiles + 9) / 10, per = (tiles + parts - 1) / parts;
+    using T = Shape4<1, 4, 4, 2, 32, 3>;
+    p.ntm = (p.M + T::BM - 1) / T::BM, p.ntn = p.N / T::BN, p.order = 4, p.wide_store = 1, p.split = 1;
+    // Experts of more than KC rows: at most rows / (KC + 1), whose tiles are a round of the chip's two workgroups a CU at a time.  (One at least: `rows` decides how many
+    // workgroups look for them, never whether they are found.)
+    const long long most = p.mode == 2 ? std::max<long long>(1, rows / (KC + 1)) : 0;
+    const int tiling = int(std::min<long long>(2 * ROUND, most * ((p.ntm * p.ntn + 7) & ~7)));
+    const dim3 grid(unsigned(tiling) + unsigned(experts) * unsigned(parts) * unsigned(p.N / STRIP));
+    constexpr size_t SMEM = std::max(size_t(WGRAD_SMEM), T::SMEM);
+    if (p.gather_rows)
+        ARIA_LAUNCH((wgrad_strip_kernel<true>), grid, dim3(256), SMEM, stream, p, tiling, parts, per);
+    else
+        ARIA_LAUNCH((wgrad_strip_kernel<false>), grid, dim3(256), SMEM, stream, p, tiling, parts, per);
+    return aria_check_launch();
+}
+
 int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream) {
-    if (plan.form == 4) return aria_launch_wgrad_strips(p, stream);
+    if (plan.form == 4) return launch_wgrad_strips(p, plan.rows, stream);
     GemmParams q = p;
     const char* wsd = std::getenv("ARIA_GEMM_WIDE_STORE");
     q.wide_store = !(wsd && wsd[0] == '0') && (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (p.ldc & 7) == 0 && (p.strideC & 7) == 0;

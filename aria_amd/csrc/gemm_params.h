@@ -308,16 +308,16 @@ __attribute__((visibility("hidden"))) int aria_launch_gemm3(const GemmParams& p,
 // fp32 workspace bytes the v3 remainder split-K wants for a dense problem (0: it would not split)
 __attribute__((visibility("hidden"))) long long aria_gemm3_workspace_bytes(long long M, long long N, long long K);
 // the four-wave kernels (gemm4.hip).  form 0: not theirs; 1: tiles of 128 x 256; 2: 256 x 160 or 128 x 320; 3: 128 x 256, two workgroups a CU (both operands [k][rows]); 4: strips of
-// 256 columns (wgrad.hip)
+// 256 columns (wgrad.h)
 struct Gemm4Plan {
     int form = 0, split = 1;
+    long long rows = 0;   // form 4 by expert: of all experts together
 };
 // rows: mode 2's rows of all experts together (< 0: not known); split3: pieces that the 256 x 256 tiles would cut the reduction of a partly filled round into (1:
 // none), which are these tiles' too unless own_cut
 __attribute__((visibility("hidden"))) Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long rows, int split3, long long workspace_bytes, bool own_cut = false);
-// weight gradients whose reductions are short (wgrad.hip); rows: as for aria_plan_gemm4; any_size: of outputs that other tiles are faster for too
+// weight gradients whose reductions are short (wgrad.h); rows: as for aria_plan_gemm4; any_size: of outputs that other tiles are faster for too
 __attribute__((visibility("hidden"))) bool aria_wgrad_strips_take(const GemmParams& p, long long rows, bool any_size = false);
-__attribute__((visibility("hidden"))) int aria_launch_wgrad_strips(const GemmParams& p, void* stream);
 __attribute__((visibility("hidden"))) int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, float* ws, void* stream);
 __attribute__((visibility("hidden"))) long long aria_gemm4_workspace_bytes(long long M, long long N, long long K);
 // X W^T for a dense x [M, K] and w [N, K] whose sums need not be the 256 x 256 tiles' (prompts, whose shorter ones are summed by other kernels anyway)

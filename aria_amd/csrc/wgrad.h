@@ -4,16 +4,17 @@
 // A workgroup of four waves owns a strip of 256 columns and runs over tiles of 64 features; wave w owns columns [64 w, 64 w + 64) of the strip and holds dY's fragments of them
 // for the whole reduction in registers (128 for 256 rows).  Only A moves: a tile's rows [up to 256][64] arrive by LDS-DMA in one of two buffers while the tile before is computed
 // and stored, one barrier a tile, and every output line is written whole, eight lines a store instruction.  Two workgroups a CU (80 KiB each: the buffers, 4 KiB a wave in which
-// 32 x 64 results are turned into rows).  Reductions beyond 256 rows (an expert that most tokens want) reload dY's fragments for every tile and 128 rows.
+// 32 x 64 results are turned into rows).
+//
+// Longer reductions (an expert that most tokens want) are the 128 x 256 tiles', in the same launch (wgrad_strip_kernel, gemm4.hip).
 //
 // What bounds it is the stores: 64 experts of 2560 x 3328 outputs (1.09 GB) 196 us at 6 rows each and 206 at 26, where stores alone take 200 (5.5 TB/s; tiles of 128 x 256 took
-// 240 and 265); 240 (318) at 73 rows, where two waves a SIMD leave a third of a tile's reads and products uncovered.
+// 240 and 265); 220 (361) at 73 rows each, where two waves a SIMD leave a part of a tile's reads and products uncovered.
 //
 // LDS images: [k][64 features or columns], 128 bytes a k-row; the 32-byte chunk c of k-row k lies at c ^ 2 ((k >> 1) & 1), so that the 32 lanes of a transposing read's half wave hit
 // eight different 32-byte bank groups.  The products of an element come in the order of the other kernels' (sixteen rows a step, rows in order): the same bits.
-#include "aria_hip.h"
+#pragma once
 #include "gemm_params.h"
-#include <type_traits>
 
 namespace {
 using namespace ad;
@@ -44,21 +45,30 @@ __device__ __forceinline__ void frags4(s16x8 (&f)[4], const char* smem, uint32_t
 #endif
 }
 
-// parts: pieces of a strip's feature tiles, per: tiles of one
+// Strip `wg` of `nwg`.  parts: pieces of a strip's feature tiles, per: tiles of one
 template <bool GATHER>
-__global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(const bf16_t* A, const bf16_t* B, bf16_t* C, const int32_t* offsets, const int32_t* gather_rows, int M, int N, int K,
-                                                             long long lda, long long ldb, long long ldc, long long strideC, int parts, int per) {
-    ARIA_DYN_SMEM(smem);
+__device__ __forceinline__ void wgrad_strip(const GemmParams& p, int wg, int nwg, int parts, int per, char* smem) {
+    const bf16_t *A = p.A, *B = p.B;
+    bf16_t* C = static_cast<bf16_t*>(p.C);
+    const int32_t *offsets = p.offsets, *gather_rows = p.gather_rows;
+    const int M = p.M, N = p.N, K = p.K;
+    const long long lda = p.lda, ldb = p.ldb, ldc = p.ldc, strideC = p.strideC;
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6);
     // an XCD runs the strips of one expert after the other's: its rows are read into one L2
-    const int nwg = gridDim.x, q8 = nwg >> 3, r8 = nwg & 7, xcd = blockIdx.x & 7, strips = N / STRIP;
-    int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (int(blockIdx.x) >> 3);
+    const int q8 = nwg >> 3, r8 = nwg & 7, xcd = wg & 7, strips = N / STRIP;
+    int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (wg >> 3);
     const int n0 = (id % strips) * STRIP;
     id /= strips;
     const int first = (id % parts) * per, last = min(first + per, M / FT), e = id / parts;
     int k_begin = 0, k_len = K;
     if (offsets) k_begin = first_lane(offsets[e]), k_len = first_lane(offsets[e + 1]) - k_begin;
+    if (k_len > KC) return;   // (the tiles')
     C += e * strideC;
+    if (k_len <= 0) {   // nothing but stores: two rows of the strip a wave's store
+        bf16_t* out = C + (long long)(first * FT + (t >> 5)) * ldc + n0 + (t & 31) * 8;
+        for (int row = first * FT; row < last * FT; row += 8, out += 8 * ldc) st16(out, zero16());
+        return;
+    }
     const uint32_t lda2 = uint32_t(2 * lda), ldb2 = uint32_t(2 * ldb);
     // this lane's k-row of a DMA piece of eight, its column (LDS images: the chunks' places swapped at the source)
     const int krow = l >> 3, col = ((((l & 7) >> 1) ^ (((l >> 4) & 1) << 1)) << 4) + (l & 1) * 8;
@@ -72,18 +82,18 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(const bf16_t* A, co
     s16x8 held[KC / 16][2];   // dY's fragments
     uint32_t rows[KC / 32];   // byte offsets of this lane's rows of A
 
-    // rows [k0, k0 + kc) of the reduction: dY's fragments through the buffers (16 KiB of them a wave), A's row offsets
-    auto load_held = [&](auto halves, int k0, int kc) __attribute__((always_inline)) {
-        const char* b = reinterpret_cast<const char*>(B) + ((long long)(k_begin + k0) * ldb + n0 + 64 * w + col) * 2;
+    // the kc rows of the reduction: dY's fragments through the buffers (16 KiB of them a wave), A's row offsets
+    auto load_held = [&](int kc) __attribute__((always_inline)) {
+        const char* b = reinterpret_cast<const char*>(B) + ((long long)k_begin * ldb + n0 + 64 * w + col) * 2;
         char* mine = smem + 16384 * w;
 #pragma unroll
-        for (int i = 0; i < 4 * decltype(halves)::value; ++i)
+        for (int i = 0; i < KC / 32; ++i)
             if (32 * i < kc) {
                 const int k = 32 * i + 8 * w + krow;
-                rows[i] = GATHER ? mul24(uint32_t(gather_rows[k_begin + k0 + min(k, kc - 1)]), lda2) : mul24(uint32_t(k), lda2);
+                rows[i] = GATHER ? mul24(uint32_t(gather_rows[k_begin + min(k, kc - 1)]), lda2) : mul24(uint32_t(k), lda2);
             }
 #pragma unroll
-        for (int half = 0; half < decltype(halves)::value; ++half) {
+        for (int half = 0; half < 2; ++half) {
             const int left = kc - 128 * half;
             if (left <= 0) break;
             for (int j = 0; j < min(2 * ((left + 15) / 16), 16); ++j) {
@@ -108,11 +118,11 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(const bf16_t* A, co
         }
         raw_barrier();   // (A's pieces land in the other waves' places too)
     };
-    auto fetch = [&](auto halves, int tile, int k0, int kc, int buf) __attribute__((always_inline)) {
-        const char* a = reinterpret_cast<const char*>(A) + (GATHER ? 0ll : 2 * (long long)(k_begin + k0) * lda) + (tile * FT + col) * 2ll;
+    auto fetch = [&](int tile, int kc, int buf) __attribute__((always_inline)) {
+        const char* a = reinterpret_cast<const char*>(A) + (GATHER ? 0ll : 2 * (long long)k_begin * lda) + (tile * FT + col) * 2ll;
         char* d = smem + buf * STAGE + 1024 * w;
 #pragma unroll
-        for (int i = 0; i < 4 * decltype(halves)::value; ++i)
+        for (int i = 0; i < KC / 32; ++i)
             if (32 * i < kc) {
                 const char* src = 32 * i + 8 * w + krow < kc ? a + rows[i] : zeros;
                 hold(src);
@@ -120,9 +130,9 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(const bf16_t* A, co
             }
     };
     // features 32 g .. of a buffer's tile times the held columns
-    auto products = [&](auto halves, f32x16 (&acc)[2], int g, int buf, int steps) __attribute__((always_inline)) {
+    auto products = [&](f32x16 (&acc)[2], int g, int buf, int steps) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k4 = 0; k4 < 2 * decltype(halves)::value; ++k4)
+        for (int k4 = 0; k4 < KC / 64; ++k4)
             if (4 * k4 < steps) {
                 s16x8 f[4];
                 frags4(f, smem, fv[g] + uint32_t(buf * STAGE + k4 * 8192));
@@ -160,77 +170,24 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(const bf16_t* A, co
             for (int i = 0; i < 16; ++i) acc[n][i] = 0.f;
     };
 
-    constexpr std::integral_constant<int, 2> whole{};
-    constexpr std::integral_constant<int, 1> half{};
-    if (k_len <= KC) {
-        const int steps = (k_len + 15) / 16;
-        if (k_len > 0) {
-            load_held(whole, 0, k_len);
-            fetch(whole, first, 0, k_len, 0);
-        }
-        for (int tile = first; tile < last; ++tile) {
-            const int buf = (tile - first) & 1;
-            if (tile == first)
-                wait_vm<0>();
-            else
-                wait_vm<8>();   // this wave's pieces of the tile; the eight stores of the tile before may be under way
-            raw_barrier();      // everybody's, and the other buffer is free
-            if (tile + 1 < last) fetch(whole, tile + 1, 0, k_len, buf ^ 1);
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                f32x16 acc[2];
-                clear(acc);
-                products(whole, acc, g, buf, steps);
-                store(acc, tile, g);
-            }
-        }
-        return;
-    }
+    const int steps = (k_len + 15) / 16;
+    load_held(k_len);
+    fetch(first, k_len, 0);
     for (int tile = first; tile < last; ++tile) {
-        f32x16 lo[2], hi[2];
-        clear(lo);
-        clear(hi);
-        for (int k0 = 0; k0 < k_len; k0 += KC / 2) {
-            const int kc = min(KC / 2, k_len - k0), steps = (kc + 15) / 16;
-            raw_barrier();   // the buffers are free
-            load_held(half, k0, kc);
-            fetch(half, tile, k0, kc, 0);
+        const int buf = (tile - first) & 1;
+        if (tile == first)
             wait_vm<0>();
-            raw_barrier();
-            products(half, lo, 0, 0, steps);
-            products(half, hi, 1, 0, steps);
+        else
+            wait_vm<8>();   // this wave's pieces of the tile; the eight stores of the tile before may be under way
+        raw_barrier();      // everybody's, and the other buffer is free
+        if (tile + 1 < last) fetch(tile + 1, k_len, buf ^ 1);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            f32x16 acc[2];
+            clear(acc);
+            products(acc, g, buf, steps);
+            store(acc, tile, g);
         }
-        store(lo, tile, 0);
-        store(hi, tile, 1);
     }
 }
 }  // namespace
-
-// Where strips are the faster ones, us, 128 x 256 or 256 x 256 tiles / strips.  By expert, 64 of 2560 x 3328 and 1664 x 2560, rows each on average (the most wanted one 2.5 times as many):
-// 6 240 / 196 and 120 / 109, 26 265 / 206 and 128 / 114, 73 318 / 240 and 165 / 128, 94 363 / 255 and 186 / 141, 128 394 / 309 and 202 / 163, 159 436 / 401 and 219 / 206, 192 478 / 488
-// and 236 / 275 (a tenth of the experts beyond the 256 rows that are held).  Dense: 100352 x 2560, 16 rows 266 / 106, 64 145 / 116, 200 209 / 163, 256 221 / 180; 64000 x 1536, 128
-// rows 69 / 62, 256 91 / 82.  Outputs of a few rounds have too few strips: 7680 x 2560, 64 rows 18 / 22, 256 rows 25 / 34.  Dense ones of fewer than 64 rows are the others' slower
-// kernels': 32000 x 1024, 8 rows 46 / 24, 2560 x 3328 15 / 20.
-bool aria_wgrad_strips_take(const GemmParams& p, long long rows, bool any_size) {
-    if (p.c_f32 || p.accumulate || p.bias || p.act || p.M % FT || p.N % STRIP || (reinterpret_cast<uintptr_t>(p.C) & 15) || (p.ldc & 7) || (p.strideC & 7)) return false;
-    const long long experts = p.mode == 2 ? p.E : 1, outputs = experts * p.M * p.N;
-    if (outputs <= (p.mode == 0 && p.K < 64 ? 16ll << 20 : 64ll << 20) && !any_size) return false;
-    return p.mode == 2 ? rows >= 0 && rows <= 144 * experts : p.K <= KC;
-}
-
-int aria_launch_wgrad_strips(const GemmParams& p, void* stream) {
-    const int tiles = p.M / FT, experts = p.mode == 2 ? p.E : 1;
-    // (ten tiles of 3.5 us to a start of 4; five or twenty 257 and 235 us for 240 at 73 rows, 207 and 219 for 206 at 26)
-    const int parts = (tiles + 9) / 10, per = (tiles + parts - 1) / parts;
-    const dim3 grid(unsigned(experts) * unsigned(parts) * unsigned(p.N / STRIP));
-    const int32_t* offsets = p.mode == 2 ? p.offsets : nullptr;
-    auto launch = [&](auto gather) {
-        ARIA_LAUNCH((wgrad_strip_kernel<decltype(gather)::value>), grid, dim3(256), size_t(WGRAD_SMEM), stream, p.A, p.B, static_cast<bf16_t*>(p.C), offsets, p.gather_rows, p.M, p.N,
-                    p.K, p.lda, p.ldb, p.ldc, p.strideC, parts, per);
-    };
-    if (p.gather_rows)
-        launch(std::true_type{});
-    else
-        launch(std::false_type{});
-    return aria_check_launch();
-}

@@ -174,6 +174,30 @@ def case_wgrad_strips(dev, monkeypatch, counts, M, N):
     assert bool(((got.double() - want).abs() <= 2 ** -8 * want.abs() + max(max(counts), 1) * 2 ** -24 * size).all())   # rounding to bf16, a rounding a product
 
 
+def case_wgrad_strips_long(dev, monkeypatch, counts, M, N):
+    """Experts beyond the 256 rows that a strip holds are tiles of 128 x 256 of the same launch, however many there are and wherever they stand, gathered or not: the tiles' bits.  The
+    count of all rows that the caller gives sizes the launch and decides nothing else."""
+    from aria_amd import hip, ops
+
+    T, E = sum(counts), len(counts)
+    x, dy = rnd(T, M, seed=T).to(dev), rnd(T, N, seed=N).to(dev)
+    off = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32, device=dev)
+    rows = torch.cat([torch.randperm(T, generator=torch.Generator().manual_seed(3)).to(torch.int32), torch.zeros(64, dtype=torch.int32)]).to(dev)[:T]
+
+    def told(n):
+        out = torch.full((E, M, N), 7.0, dtype=bf16, device=dev)
+        hip.get_lib().call("aria_grouped_gemm_wgrad_sized_bf16", x.data_ptr(), dy.data_ptr(), out.data_ptr(), off.data_ptr(), E, M, N, M, N, 0, 0, n, ops._stream(x))
+        return out
+
+    got = {}
+    for force in ("4", "47"):
+        monkeypatch.setenv("ARIA_GEMM_FORCE", force)
+        got[force] = [told(n) for n in (T, 0, 257)] + [ops.grouped_gemm_wgrad_gather(x, rows, dy, off, E)]
+        assert last_gemm_tiles() & 15 == (4 if force == "47" else 3)
+    for a, b in zip(got["4"], got["47"]):
+        assert torch.equal(a, b)
+
+
 def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
     activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""

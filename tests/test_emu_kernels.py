@@ -267,6 +267,11 @@ def test_wgrad_strips(monkeypatch, counts, M, N):
     C.case_wgrad_strips(DEV, monkeypatch, counts, M, N)
 
 
+@pytest.mark.parametrize("counts,M,N", [([300, 0, 257, 5], 192, 256), ([0] * 63 + [258, 1, 0, 290], 64, 256)])
+def test_wgrad_strips_long(monkeypatch, counts, M, N):
+    C.case_wgrad_strips_long(DEV, monkeypatch, counts, M, N)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 136, 128), (300, 264, 512), (40, 1032, 1536)])
 def test_gemm_keep_sums(monkeypatch, M, N, K):
     C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)

@@ -261,6 +261,11 @@ def test_wgrad_strips(monkeypatch, counts, M, N):
     C.case_wgrad_strips(DEV, monkeypatch, counts, M, N)
 
 
+@pytest.mark.parametrize("counts,M,N", [([300, 0, 257, 5], 192, 256), ([0] * 63 + [258, 1, 0, 290], 64, 256), ([3000] + [0, 1200] * 2 + [37] * 59, 2560, 3328), ([257] * 16 + [0] * 54, 1664, 2560)])
+def test_wgrad_strips_long(monkeypatch, counts, M, N):
+    C.case_wgrad_strips_long(DEV, monkeypatch, counts, M, N)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (777, 2560, 2560), (3000, 2560, 3328)])
 def test_gemm_keep_sums(monkeypatch, M, N, K):
     C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)
