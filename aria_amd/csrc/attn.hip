@@ -1421,7 +1421,7 @@ __device__ __forceinline__ void fwd3_step(f32x16 (&st)[2], f32x16 (&sn)[2], f32x
 // in-wave overlap, and with it LDS-DMA staging into the conflict-free images (SQ_LDS_BANK_CONFLICT 0, was 8 % of the LDS cycles) is level
 // with v2's register staging -- so hd 72 stays on v2 by default and both v3 forms are kept selectable (ARIA_ATTN_FWD) as measurements.
 // NW = 8 (blocks of 256 queries) or 4 (128, two workgroups a CU: the images of two fit its LDS exactly, so the ragged form, which has no key mask, asks for no more).  A
-// wave does the same work in both, bit for bit; half blocks stage the keys twice as often and halve the longest block (half_blocks: which where).
+// wave does the same work in both, bit for bit; half blocks stage the keys twice as often and halve the longest block (half_blocks_causal, half_blocks_full: which where).
 // RAGGED: the sequences of the batch are rows cu[b] .. cu[b + 1] of the token axis (Sq = S = the longest), and every head's output is multiplied
 // by sigmoid(gate[token * ldg + head]) in the epilogue (gate may be NULL); `group` neighbouring query heads share a key / value head.
 template <class F, int NW, bool PIPE, bool RAGGED>
@@ -1589,14 +1589,41 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_fwd3_kernel(const bf16_t
 }
 
 
+thread_local int g_last_fwd_waves = 0;    // of attn_fwd3: a workgroup's
 thread_local int g_last_fwd_variant = 0;  // 2: attn_fwd2 (staged through registers), 3: attn_fwd3 (software-pipelined, LDS-DMA)
 thread_local int g_last_bwd_variant = 0;  // 2: the padded-tile pair (hd 64 / 72), 5: role-split dK/dV + dQ v5 (hd 128) -- tests assert which ran
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// Blocks of 128 queries rather than 256 where their shorter last blocks are worth more than the keys staged twice as often.  Us, 256 / 128 queries a block, causal, 20 heads of 128:
-// 280 tokens 19.9 / 14.7, 777 34 / 26, 2048 71 / 57, 4096 132 / 121, 8192 405 / 389, 12000 798 / 820, 32768 5536 / 6052; 8 x 2048 257 / 246, 32 x 100 38 / 27; not causal 4096 254 / 231.
-// 12 heads of 192 / 128: six prompts of 500 .. 1200 56 / 52, 4000 150 / 134, 8000 319 / 301, (20 heads) 16384 1842 / 2005.  64 columns gain at every length (33000 2764 / 2661).
-bool half_blocks(int64_t Sq, int causal, int64_t qd) { return qd == 64 || Sq <= (causal ? 8192 : 4096); }
+// Blocks of 128 queries rather than 256, four waves and two workgroups a CU rather than eight and one.  They halve what a launch's longest blocks and its last round cost and stage the keys
+// twice as often.  Us, 256 / 128 queries a block:
+//
+// Causal, the longest blocks first.  128 columns, 20 heads: 280 tokens 19.9 / 14.7, 777 36 / 28, 4096 135 / 124, 8192 442 / 402, 12000 857 / 852, 32768 5536 / 6052.  The blocks of all heads run
+// side by side, so keys and values come from the Infinity Cache (256 MB) as long as it holds most of them, then from memory; MB of them in all: 1024 tokens, 325 376 / 351, 398 460 / 453, 514
+// 586 / 627; 2048, 315 541 / 498, 398 694 / 669, 503 861 / 931, 650 1105 / 1270; 4096, 336 943 / 903, 419 1196 / 1216, 629 1782 / 2038; 8192, 252 1245 / 1217, 336 1622 / 1625, 671 3421 / 3695.  Up
+// to 256 tokens half of a block of 256 is empty or masked at any size (256, 640 MB 457 / 428).
+// 192 / 128 columns: six of 1000 59 / 53, 1 x 8000 331 / 311, 8 x 4000 (246 MB) 666 / 656, (410 MB) 1152 / 1181, 12000 636 / 678; where two rounds are full, blocks of 256 pair long and short
+// ones exactly: 8 heads, 2 x 8000 383 / 424, 8 x 2000 131 / 138 (128 columns 333 / 332, 109 / 108).
+// 64 columns gain at every length and size (30 000 3172 / 2783; 1.3 GB 9146 / 9309 the worst).
+bool half_blocks_causal(int64_t S, double blocks, double kv_bytes, int64_t qd) {
+    if (qd == 64 || S <= 256) return true;
+    return S <= 8192 && kv_bytes <= 384.0 * (1 << 20) && !(qd == 192 && blocks > 448 && blocks <= 512);
+}
+
+// Not causal every block is as long as the keys, so the rounds decide: 256 blocks of 256 or 512 of 128, which take 4 % longer, at a time, and a last round of one block of 128 a CU 0.7 of a whole
+// one.  16 heads of 128 columns, 2048 keys: 128 blocks (of 256) 74 / 61, 256 86 / 90, 512 165 / 182; 20 heads: 160 81 / 85, 320 153 / 134, 1280 of 4096 keys 778 / 802; 256 queries of 4900
+// keys: 64 blocks 154 / 123, 320 362 / 332; 128 queries, 320 blocks 309 / 200.  Beyond a round of short sequences a block's start and end count: 256 keys, 512 blocks 48 / 44, 1024 90 / 77.
+bool half_blocks_full(int64_t Sq, int64_t Skv, int64_t pairs) {
+    if (Sq > 4096) return false;
+    const int64_t whole = pairs * ((Sq + 255) / 256), half = pairs * ((Sq + 127) / 128), rest = half % 512;
+    const double round = Skv <= 512 && whole > 256 ? 0.99 : 1.04;
+    return round * double(half / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 0.7 : round) < double((whole + 255) / 256);
+}
+
+// 4 or 8 waves that the environment asks for (ARIA_ATTN_FWD=34, 38: tests and measurements), or 0
+int forced_waves() {
+    const char* f = std::getenv("ARIA_ATTN_FWD");
+    return f && f[0] == '3' && (f[1] == '4' || f[1] == '8') ? f[1] - '0' : 0;
+}
 
 struct Plan72 {
     int whole = 0, part_waves = 0;   // blocks of 12 waves a (b, head), waves of its other blocks (0: only blocks of 12)
@@ -1643,7 +1670,7 @@ int aria_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
     if (B == 0 || Sq == 0) return ARIA_OK;
     const bf16_t *Q = static_cast<const bf16_t*>(q), *K = static_cast<const bf16_t*>(k), *V = static_cast<const bf16_t*>(v);
     const char* nw72 = std::getenv("ARIA_ATTN_HD72_WAVES");  // "8": the two-waves-per-SIMD variant (A/B measurements)
-    const char* fwdv = std::getenv("ARIA_ATTN_FWD");          // "2": the round-1..3 kernels (A/B measurements, bit-identity tests)
+    const char* fwdv = std::getenv("ARIA_ATTN_FWD");          // "2": the older kernels; "34", "38": blocks of four or eight waves (A/B measurements, bit-identity tests)
     const char* grp = std::getenv("ARIA_ATTN_CAUSAL_GROUPED");   // "1" / "0": force the XCD-grouped causal block order on / off (tests, A/B)
     const int causal_arg = causal ? ((grp ? grp[0] == '1' : Sq >= 32768) ? 2 : 1) : 0;   // (2: attn_block_coords' grouped order; default: the forward from 32 K tokens up)
     // default: hd 128 -> v3 pipelined (+4..8 % over v2 from 2K to 64K tokens); hd 72 -> v2 with 12 waves (measured, same box: v2 2.23-2.46 ms,
@@ -1659,7 +1686,10 @@ int aria_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
                     (long long)ldv, (long long)ldo, scale, causal_arg, int(B), static_cast<const int32_t*>(nullptr),
                     static_cast<const bf16_t*>(nullptr), 0ll, 1);
     };
-    if (v3 && half_blocks(Sq, causal, hd))
+    const int waves = !v3 ? 0 : forced_waves() ? forced_waves() : (causal ? half_blocks_causal(Sq, double(H * B) * double((Sq + 255) / 256), 512.0 * double(B * H) * double(Skv), hd)
+                                                                         : half_blocks_full(Sq, Skv, H * B)) ? 4 : 8;
+    g_last_fwd_waves = waves;
+    if (waves == 4)
         launch3(std::integral_constant<int, 4>{});
     else if (v3)
         launch3(std::integral_constant<int, 8>{});
@@ -1687,6 +1717,12 @@ int aria_attn_fwd(const void* q, const void* k, const void* v, void* o, float* l
 int aria_attn_varlen_fwd(const void* q, const void* k, const void* v, void* o, const int32_t* cu, const void* gate, int64_t B, int64_t S_max,
                          int64_t H, int64_t G, int64_t qd, int64_t vd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t ldg,
                          float scale, void* stream) {
+    return aria_attn_varlen_sized_fwd(q, k, v, o, cu, gate, B, S_max, H, G, qd, vd, ldq, ldk, ldv, ldo, ldg, scale, -1, stream);
+}
+
+int aria_attn_varlen_sized_fwd(const void* q, const void* k, const void* v, void* o, const int32_t* cu, const void* gate, int64_t B, int64_t S_max,
+                               int64_t H, int64_t G, int64_t qd, int64_t vd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t ldg,
+                               float scale, int64_t T, void* stream) {
     if (!q || !k || !v || !o || !cu || B < 0 || S_max < 0 || H <= 0 || G <= 0 || H % G) return ARIA_ERR_INVALID;
     if (!al16(q) || !al16(k) || !al16(v) || (ldq & 7) || (ldk & 7) || (ldv & 7) || (ldo & 3) || (reinterpret_cast<uintptr_t>(o) & 7))
         return ARIA_ERR_ALIGN;
@@ -1694,21 +1730,27 @@ int aria_attn_varlen_fwd(const void* q, const void* k, const void* v, void* o, c
     if (!known) return ARIA_ERR_UNSUPPORTED;
     if (B == 0 || S_max == 0) return ARIA_OK;
     const int causal = S_max >= 32768 ? 2 : 1;   // (2: attn_block_coords' grouped order)
-    const bool half = half_blocks(S_max, 1, qd);
+    const double tokens = T >= 0 ? double(T) : double(B) * double(S_max);
+    const int forced = forced_waves();
+    const bool half = forced ? forced == 4 : half_blocks_causal(S_max, double(H) * tokens / 256, 2.0 * double(G * (qd + vd)) * tokens, qd);
     auto launch = [&](auto fmt, auto pipe) {
         using F = decltype(fmt);
         auto of = [&](auto nw) {
             constexpr int NW = decltype(nw)::value;
             constexpr bool PIPE = decltype(pipe)::value;
+            g_last_fwd_waves = NW;
             ARIA_LAUNCH((attn_fwd3_kernel<F, NW, PIPE, true>), dim3(attn_grid((S_max + 32 * NW - 1) / (32 * NW), H, B)), dim3(64 * NW), size_t(Fwd3Smem<F>::M0), stream,
                         static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(k), static_cast<const bf16_t*>(v), static_cast<bf16_t*>(o), static_cast<float*>(nullptr),
                         static_cast<const int32_t*>(nullptr), static_cast<const uint8_t*>(nullptr), int(S_max), int(S_max), int(H), (long long)ldq, (long long)ldk,
                         (long long)ldv, (long long)ldo, scale, causal, int(B), cu, static_cast<const bf16_t*>(gate), (long long)ldg, int(H / G));
         };
-        if constexpr (2 * Fwd3Smem<F>::M0 <= 160 * 1024) {
-            if (half) return of(std::integral_constant<int, 4>{});
-        }
-        of(std::integral_constant<int, 8>{});
+        constexpr bool two = 2 * Fwd3Smem<F>::M0 <= 160 * 1024;   // (256 columns: one workgroup fills the LDS)
+        if constexpr (F::QD == 64)
+            of(std::integral_constant<int, 4>{});
+        else if (two && half)
+            of(std::integral_constant<int, two ? 4 : 8>{});
+        else
+            of(std::integral_constant<int, 8>{});
     };
     using F64 = FmtQV<64, 64>;
     using F192 = FmtQV<192, 128>;
@@ -1726,6 +1768,7 @@ int aria_attn_varlen_fwd(const void* q, const void* k, const void* v, void* o, c
 
 int aria_last_attn_bwd_variant(void) { return g_last_bwd_variant; }
 int aria_last_attn_fwd_variant(void) { return g_last_fwd_variant; }
+int aria_last_attn_fwd_waves(void) { return g_last_fwd_waves; }
 
 int aria_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* delta,
                   void* dq, void* dk, void* dv, const int32_t* kv_len, const uint8_t* key_mask, int64_t B, int64_t Sq, int64_t Skv,

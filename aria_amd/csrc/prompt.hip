@@ -104,8 +104,8 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         }
         ARIA_TRY(product(z.h, p[1], z.qkv, 3 * D, D));
         ARIA_TRY(aria_rope_cache_rows(z.qkv, ptrs[0], slot, pos, kc, vc, T, H, hd, Smax, stream));
-        ARIA_TRY(aria_attn_varlen_fwd(z.qkv, z.qkv + D, z.qkv + 2 * D, z.ao, cu, nullptr, n_seq, longest, H, H, hd, hd, 3 * D, 3 * D, 3 * D, D, 0,
-                                      1.0f / sqrtf(float(hd)), stream));
+        ARIA_TRY(aria_attn_varlen_sized_fwd(z.qkv, z.qkv + D, z.qkv + 2 * D, z.ao, cu, nullptr, n_seq, longest, H, H, hd, hd, 3 * D, 3 * D, 3 * D, D, 0,
+                                            1.0f / sqrtf(float(hd)), T, stream));
         ARIA_TRY(product(z.ao, p[2], z.d, D, D));
         ARIA_TRY(aria_rmsnorm_fwd(z.d, x, p[3], y, z.h, nullptr, T, D, eps, stream));
         summed();

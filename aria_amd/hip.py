@@ -36,6 +36,7 @@ SIGNATURES = {
     "aria_last_gemm_tiles": [],
     "aria_last_attn_bwd_variant": [],
     "aria_last_attn_fwd_variant": [],
+    "aria_last_attn_fwd_waves": [],
     "aria_decode_scratch_bytes": [P],
     "aria_decode_trace_layout": [P, P],
     "aria_decode_token": [P, P, F32, P],
@@ -124,6 +125,7 @@ SIGNATURES = {
     "aria_colsum_bf16": [P, P, I64, I64, I64, I64, P],
     "aria_cross_entropy": [P, P, P, P, P, F32, P, I64, I64, I64, P],
     "aria_attn_varlen_fwd": [P, P, P, P, P, P, I64, I64, I64, I64, I64, I64, I64, I64, I64, I64, I64, F32, P],
+    "aria_attn_varlen_sized_fwd": [P, P, P, P, P, P, I64, I64, I64, I64, I64, I64, I64, I64, I64, I64, I64, F32, I64, P],
     "aria_dyt_stream": [P, P, P, P, P, I64, P, P, P, P, I64, I64, I64, I32, P],
     "aria_act_rows": [P, P, P, I64, I64, I64, I64, I32, I32, P],
     "aria_gemm_f32": [P, P, P, I64, I64, I64, I64, I64, I64, P, I64, I64, P],

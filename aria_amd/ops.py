@@ -1329,8 +1329,9 @@ def attention_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cu: torc
         _chk(t, name=n)
     _chk(cu, torch.int32, "cu")
     out = torch.empty((q.shape[0], H * vd), dtype=bf16, device=q.device)
-    hip.get_lib().call("aria_attn_varlen_fwd", _p(q), _p(k), _p(v), _p(out), _p(cu), _p(gate), cu.numel() - 1, S_max, H, kv_heads or H, qd, vd, _rowmajor_2d(q, "q"),
-                       _rowmajor_2d(k, "k"), _rowmajor_2d(v, "v"), H * vd, _rowmajor_2d(gate, "gate") if gate is not None else 0, float(scale), _stream(q))
+    hip.get_lib().call("aria_attn_varlen_sized_fwd", _p(q), _p(k), _p(v), _p(out), _p(cu), _p(gate), cu.numel() - 1, S_max, H, kv_heads or H, qd, vd, _rowmajor_2d(q, "q"),
+                       _rowmajor_2d(k, "k"), _rowmajor_2d(v, "v"), H * vd, _rowmajor_2d(gate, "gate") if gate is not None else 0, float(scale), q.shape[0],
+                       _stream(q))
     return out
 
 

@@ -390,12 +390,18 @@ int aria_attn_bwd_rope(const void* q, const void* k, const void* v, const void* 
 int aria_attn_varlen_fwd(const void* q, const void* k, const void* v, void* o, const int32_t* cu, const void* gate, int64_t B, int64_t S_max,
                          int64_t H, int64_t G, int64_t qd, int64_t vd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t ldg, float scale,
                          void* stream);
+/* ... with the number of tokens T = cu[B], which the host may know: it decides over block sizes only, the bits are the same (T < 0: not known) */
+int aria_attn_varlen_sized_fwd(const void* q, const void* k, const void* v, void* o, const int32_t* cu, const void* gate, int64_t B, int64_t S_max,
+                               int64_t H, int64_t G, int64_t qd, int64_t vd, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t ldg, float scale,
+                               int64_t T, void* stream);
 
 /* which backward the calling thread's last aria_attn_bwd ran: 2 = padded-tile pair (hd 64 / 72), 5 = role-split dK/dV + dQ v5 (hd 128) */
 int aria_last_attn_bwd_variant(void);
 /* which forward the calling thread's last aria_attn_fwd launched: 3 = attn_fwd3 (hd 128 / 72: software-pipelined score tiles, K / V by
  * LDS-DMA), 2 = attn_fwd2 (hd 64; or ARIA_ATTN_FWD=2: the round-3 kernels for A/B runs and the bit-identity tests) */
 int aria_last_attn_fwd_variant(void);
+/* waves of a workgroup (32 queries each) of the calling thread's last attn_fwd3 launch: 4 or 8, 0 where aria_attn_fwd ran attn_fwd2.  ARIA_ATTN_FWD=34 or 38 forces them. */
+int aria_last_attn_fwd_waves(void);
 
 /* ------------------------------------------------------------------------------------------------
  * ViT / projector support (vit.hip)

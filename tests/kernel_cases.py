@@ -1206,6 +1206,15 @@ def case_attention_varlen_blocks(dev, lens, H=2):
             os.environ["ARIA_ATTN_FWD"] = prev
 
 
+def case_attention_block_rule(dev, causal, B, S, Skv, H, waves):
+    """which blocks a call takes, on both sides of the rule's lines"""
+    from aria_amd import hip, ops
+
+    q, kv = rnd(B * S, H * 128, seed=1).to(dev), rnd(B * Skv, H * 128, seed=2).to(dev)
+    ops.attention_fwd(q, kv, kv, B, S, H, 128, 128 ** -0.5, causal, Skv=Skv)
+    assert hip.get_lib().cdll.aria_last_attn_fwd_waves() == waves
+
+
 def case_attention_bwd_rope(dev, B, S, H, causal, use_len, s_rope=None):
     """r05: ``aria_attn_bwd_rope`` -- the inverse half-split RoPE of dq / dk (the chain rule through apply_rotary_pos_emb,
     modeling_llama.py:130-160) in the attention backward's register epilogues -- gives the bits of ``aria_attn_bwd`` followed by the in-place

@@ -129,6 +129,11 @@ def test_attention_varlen_blocks(lens):
     C.case_attention_varlen_blocks(DEV, lens)
 
 
+@pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 1, 130, 130, 1, 4), (False, 1, 130, 70, 1, 4), (False, 1, 16, 70, 1, 4)])
+def test_attention_block_rule(causal, B, S, Skv, H, waves):
+    C.case_attention_block_rule(DEV, causal, B, S, Skv, H, waves)
+
+
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
 @pytest.mark.parametrize("M,N,K", [(40, 72, 64), (264, 136, 192), (72, 520, 128)])
 def test_gemm_fused_gelu(monkeypatch, force, M, N, K):

@@ -129,6 +129,13 @@ def test_attention_varlen_blocks(lens):
     C.case_attention_varlen_blocks(DEV, lens)
 
 
+@pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 8, 2048, 2048, 20, 4), (True, 24, 2048, 2048, 20, 8), (True, 200, 256, 256, 20, 4), (True, 1, 8192, 8192, 4, 4), (True, 1, 8193, 8193, 4, 8),
+                                                      (False, 1, 2048, 2048, 16, 4), (False, 1, 2048, 2048, 20, 8), (False, 2, 2048, 2048, 20, 4), (False, 1, 4096, 4096, 16, 8), (False, 16, 128, 4900, 20, 4),
+                                                      (False, 1, 4097, 600, 2, 8), (False, 16, 256, 256, 32, 4)])
+def test_attention_block_rule(causal, B, S, Skv, H, waves):
+    C.case_attention_block_rule(DEV, causal, B, S, Skv, H, waves)
+
+
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
 @pytest.mark.parametrize("M,N,K", [(40, 72, 64), (264, 136, 192), (2048, 4304, 1152), (2560, 2560, 4096)])
 def test_gemm_fused_gelu(monkeypatch, force, M, N, K):
