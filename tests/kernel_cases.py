@@ -1206,6 +1206,47 @@ def case_attention_varlen_blocks(dev, lens, H=2):
             os.environ["ARIA_ATTN_FWD"] = prev
 
 
+def case_attention_waves(dev, monkeypatch, B, Sq, Skv, H, causal, masked, use_len):
+    """Blocks of 128 queries (four waves) and of 256 (eight) give the bits of the oldest kernel, with key masks, lengths, queries and keys of different counts."""
+    from aria_amd import hip, ops
+
+    D, g = H * 128, torch.Generator().manual_seed(Sq + Skv)
+    q, kv = torch.randn(B * Sq, D, generator=g).to(bf16).to(dev), torch.randn(B * Skv, 2 * D, generator=g).to(bf16).to(dev)
+    km = kl = None
+    if masked:
+        km = (torch.rand(B, Skv, generator=g) > 0.3).to(torch.uint8)
+        km[:, 0], km[0, 64:128], km[0, Skv - Skv // 4:] = 1, 0, 0
+        km = km.to(dev)
+    if use_len:
+        kl = torch.randint(1, Skv + 1, (B,), generator=g).to(torch.int32).to(dev)
+    got = {}
+    for force in ("2", "34", "38"):
+        monkeypatch.setenv("ARIA_ATTN_FWD", force)
+        got[force] = ops.attention_fwd(q, kv[:, :D], kv[:, D:], B, Sq, H, 128, 128 ** -0.5, causal, kv_len=kl, key_mask=km, Skv=Skv)
+        assert hip.get_lib().cdll.aria_last_attn_fwd_waves() == {"2": 0, "34": 4, "38": 8}[force]
+    for force in ("34", "38"):
+        assert torch.equal(got[force][0], got["2"][0]) and torch.equal(got[force][1], got["2"][1]), force
+
+
+def case_attention_varlen_waves(dev, monkeypatch, lens, qd, vd, H=4, G=2):
+    """Packed sequences, gated, with shared key / value heads: the same bits in blocks of 128 and 256 queries; the count of all tokens that the caller gives changes no bit."""
+    from aria_amd import hip, ops
+
+    T, g = sum(lens), torch.Generator().manual_seed(sum(lens) + qd)
+    q, k, v, gate = (torch.randn(T, n, generator=g).to(bf16).to(dev) for n in (H * qd, G * qd, G * vd, H))
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=dev)
+    got = []
+    for force, waves in (("38", 8), ("34", 4)):
+        monkeypatch.setenv("ARIA_ATTN_FWD", force)
+        got.append(ops.attention_varlen(q, k, v, cu, max(lens), H, qd, vd, qd ** -0.5, gate=gate, kv_heads=G))
+        assert hip.get_lib().cdll.aria_last_attn_fwd_waves() == (4 if qd == 64 else 8 if qd == 256 else waves)
+    monkeypatch.delenv("ARIA_ATTN_FWD")
+    got.append(torch.empty_like(got[0]))
+    hip.get_lib().call("aria_attn_varlen_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), got[2].data_ptr(), cu.data_ptr(), gate.data_ptr(), len(lens), max(lens), H, G, qd, vd, H * qd, G * qd,
+                       G * vd, H * vd, H, qd ** -0.5, ops._stream(q))
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
 def case_attention_block_rule(dev, causal, B, S, Skv, H, waves):
     """which blocks a call takes, on both sides of the rule's lines"""
     from aria_amd import hip, ops

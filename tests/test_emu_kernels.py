@@ -129,6 +129,20 @@ def test_attention_varlen_blocks(lens):
     C.case_attention_varlen_blocks(DEV, lens)
 
 
+@pytest.mark.parametrize("defer", ["0", "1"])
+@pytest.mark.parametrize("B,Sq,Skv,H,causal,masked,use_len", [(1, 330, 330, 1, False, True, False), (1, 513, 513, 1, True, False, True), (1, 300, 200, 1, False, False, False)])
+def test_attention_waves(monkeypatch, defer, B, Sq, Skv, H, causal, masked, use_len):
+    monkeypatch.setenv("ARIA_EMU_GLDS_DEFER", defer)   # pieces landing at once, or at the counted wait only
+    C.case_attention_waves(DEV, monkeypatch, B, Sq, Skv, H, causal, masked, use_len)
+
+
+@pytest.mark.parametrize("defer", ["0", "1"])
+@pytest.mark.parametrize("lens,qd,vd", [((257, 64, 3), 128, 128), ((300,), 192, 128), ((130, 5), 64, 64), ((70,), 256, 256)])
+def test_attention_varlen_waves(monkeypatch, defer, lens, qd, vd):
+    monkeypatch.setenv("ARIA_EMU_GLDS_DEFER", defer)   # pieces landing at once, or at the counted wait only
+    C.case_attention_varlen_waves(DEV, monkeypatch, lens, qd, vd)
+
+
 @pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 1, 130, 130, 1, 4), (False, 1, 130, 70, 1, 4), (False, 1, 16, 70, 1, 4)])
 def test_attention_block_rule(causal, B, S, Skv, H, waves):
     C.case_attention_block_rule(DEV, causal, B, S, Skv, H, waves)

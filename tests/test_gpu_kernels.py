@@ -129,6 +129,16 @@ def test_attention_varlen_blocks(lens):
     C.case_attention_varlen_blocks(DEV, lens)
 
 
+@pytest.mark.parametrize("B,Sq,Skv,H,causal,masked,use_len", [(1, 330, 330, 1, False, True, False), (2, 513, 513, 2, True, False, True), (3, 300, 4900, 2, False, True, False), (2, 2048, 2048, 4, False, False, True), (1, 4097, 4097, 2, True, False, False)])
+def test_attention_waves(monkeypatch, B, Sq, Skv, H, causal, masked, use_len):
+    C.case_attention_waves(DEV, monkeypatch, B, Sq, Skv, H, causal, masked, use_len)
+
+
+@pytest.mark.parametrize("lens,qd,vd", [((257, 64, 1000, 31, 32), 128, 128), ((8200, 300), 192, 128), ((8200, 129), 128, 128), ((1300, 5), 64, 64), ((700, 1), 256, 256)])
+def test_attention_varlen_waves(monkeypatch, lens, qd, vd):
+    C.case_attention_varlen_waves(DEV, monkeypatch, lens, qd, vd)
+
+
 @pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 8, 2048, 2048, 20, 4), (True, 24, 2048, 2048, 20, 8), (True, 200, 256, 256, 20, 4), (True, 1, 8192, 8192, 4, 4), (True, 1, 8193, 8193, 4, 8),
                                                       (False, 1, 2048, 2048, 16, 4), (False, 1, 2048, 2048, 20, 8), (False, 2, 2048, 2048, 20, 4), (False, 1, 4096, 4096, 16, 8), (False, 16, 128, 4900, 20, 4),
                                                       (False, 1, 4097, 600, 2, 8), (False, 16, 256, 256, 32, 4)])
