@@ -6,7 +6,7 @@
 // Few outputs (gemm_f32_kernel): fragments straight from global memory.  A workgroup computes a tile of 16 MT x 16 NT outputs, its NW waves on interleaved 16-column
 // steps of the reduction, DEPTH steps in flight; the partial tiles meet in LDS once.  Splitting the REDUCTION over the waves is what fills the chip where a
 // serving step has a few rows only (1 .. 16 rows of a 1024-wide layer are 16 tiles of 64 columns: 100 us a launch as one 64 x 64 tile per workgroup with its
-// waves side by side), and costs one pass over the tile in LDS.  16 x 16 x 8 waves up to 16 rows, where the weights' stream bounds it; 32 x 32 x 4 up to a round of tiles.
+// waves side by side), and costs one pass over the tile in LDS.  16 x 16 x 8 waves up to 16 rows, where the weights' stream bounds it; 32 x 32 x 4 and 64 x 32 x 4 up to a round of tiles.
 //
 // More (gemm_f32_tiles_kernel): stages in the LDS.  Read from global memory, the half lines of a 16-column step are fetched from the L2 twice, which bound those tiles.
 // M x N x K, us with the reduction over the waves (64 x 32 a workgroup) / by stages: 883 x 2112 x 1024 61 / 44, 883 x 2816 x 1024 77 / 53, 883 x 1024 x 2816 74 / 59,
@@ -22,7 +22,7 @@ namespace {
 using namespace ad;
 
 typedef AriaGemmF32 GemmF32;
-constexpr int FIN_HEADS = 4;   // beside gemm_f32.h's
+constexpr int FIN_HEADS = 4, FIN_ROWS = 5;   // beside gemm_f32.h's: PLAIN with rows of A by index
 // a product a head (blockIdx.y) of the latent attention's expansion: the result's row t of head h times its output gate over its softmax sum
 struct Heads {
     const float *ml, *gate;   // [T, H, 2] (maximum, sum), gate logits [T, ldg]
@@ -50,8 +50,11 @@ __device__ __forceinline__ bool find_rows(const GemmF32& p, int y, int rows, int
     return false;
 }
 
-// the row of A that row m of the result comes from
-__device__ __forceinline__ long long row_of(const GemmF32& p, int m) { return p.rows ? p.rows[m] / p.per : m; }
+// the row of A that row m of the result comes from (the others do not ask: a dependent load and a division in front of the first fetch, 0.5 us of the 10 of 17 x 1024 x 1024)
+template <int FIN>
+__device__ __forceinline__ long long row_of(const GemmF32& p, int m) {
+    return FIN == FIN_ROWS || (FIN == ARIA_F32_PAIR && p.rows) ? p.rows[m] / p.per : m;
+}
 
 // What becomes of a sum (v2: the second weight's): as the launches of their own would have it, act_rows_kernel and dyt_stream_kernel
 template <int FIN>
@@ -72,7 +75,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     // 16 x 16 outputs: a wave takes two neighbouring steps, whole lines of both operands (us, one / two: 4 x 64000 x 1536 84 / 78, 16 x 32000 x 1024 43.6 / 42.0, 4 x 12288 x 2048
     // 26.4 / 25.7, 2 x 8192 x 1024 13.1 / 13.0)
     constexpr int PER = MT * NT == 1 ? 2 : 1, LINE = 16 * PER;
-    constexpr int DEPTH = 4, TM = 16 * MT, TN = 16 * NT;
+    constexpr int DEPTH = MT + NT > 4 ? 2 : 4, TM = 16 * MT, TN = 16 * NT;
     ARIA_SMEM_STATIC float red[WS][NW][TM][TN + 1];
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), q4 = l >> 4, c16 = l & 15;
     const unsigned ntn = unsigned(p.N + TN - 1) / TN;
@@ -81,7 +84,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     if (p.offsets && !find_rows(p, y, TM, e, m0, m_end)) return;
     const float *ap[MT], *wp[WS][NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) ap[i] = p.A + row_of(p, min(m0 + 16 * i + c16, m_end - 1)) * p.lda + w * LINE + q4 * 4;
+    for (int i = 0; i < MT; ++i) ap[i] = p.A + row_of<FIN>(p, min(m0 + 16 * i + c16, m_end - 1)) * p.lda + w * LINE + q4 * 4;
 #pragma unroll
     for (int z = 0; z < WS; ++z)
 #pragma unroll
@@ -128,6 +131,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
         for (int u = 0; u < DEPTH; ++u) {
             use(x[u]);
             load(at(s + u + DEPTH), x[u]);
+            sched_fence();   // (left alone the compiler asks for all of them behind the last product)
         }
     }
     for (; s < mine; s += DEPTH) {   // the last DEPTH .. 2 DEPTH - 1 steps (or fewer altogether)
@@ -207,7 +211,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiles_kernel(GemmF32 p, Heads hd
         const int r = 8 * (w + 4 * i) + (l >> 3);
         at[i] = ((l & 7) ^ (r >> 1 & 7)) * 4;
         const int rw = r < BM + BN ? r - BM : r - BM - BN;
-        src[i] = r < BM ? p.A + row_of(p, min(m0 + r, m_end - 1)) * p.lda : (r < BM + BN ? p.W : p.W2) + e * p.strideW + (long long)min(n0 + rw, p.N - 1) * p.ldw;
+        src[i] = r < BM ? p.A + row_of<FIN>(p, min(m0 + r, m_end - 1)) * p.lda : (r < BM + BN ? p.W : p.W2) + e * p.strideW + (long long)min(n0 + rw, p.N - 1) * p.ldw;
     }
     auto piece = [&](int s, int i) __attribute__((always_inline)) {   // of stage s (columns behind the row's end: its first ones; never used)
         const int k = 32 * s + at[i];
@@ -381,17 +385,21 @@ int launch_f32_tiles(const GemmF32& p, const Heads& hd, void* stream) {
     return aria_check_launch();
 }
 
-// (an expert's last tile stands half empty on average)
 template <int FIN>
 int product_f32(const GemmF32& p, void* stream) {
     if (p.offsets ? p.M <= 16 * p.E : p.M <= 16) return launch_f32<1, 1, 8, FIN>(p, stream);
-    // Up to a round of 32 x 32 tiles the reduction over the waves is the shorter chain (48 x 1024 x 2816: 22 us, 24 with stages).  Beyond it the rounds of the chip
-    // decide, and of equal ones the larger tile (883 x 2112 x 1024, us as 64 x 64 / 32 x 64 / 32 x 32: 44 / 47 / 48; 883 x 2816 x 1024 61 / 53 / 55; 300 x 2112 x 1024
-    // 24 / 25 / 20).
-    const int64_t M = p.M, N = p.N;
-    auto tiles = [&](int mi, int ni) { return ((M + 32 * mi - 1) / (32 * mi) + (p.offsets ? p.E / 2 : 0)) * ((N + 32 * ni - 1) / (32 * ni)); };
-    if (tiles(1, 1) <= 256) return launch_f32<2, 2, 4, FIN>(p, stream);
-    auto cost = [&](int mi, int ni, int more) { return (tiles(mi, ni) + 255) / 256 * mi * ni * (100 + more); };
+    // Up to a round of 32 x 32 tiles, and of 64 x 32 ones, the reduction over the waves is the shorter chain (us, here / by stages: 48 x 1024 x 2816 22 / 24; 64 x 32: 300 x 1024 x 2816
+    // 35 / 40, 500 x 768 x 2048 27 / 30, 100 x 2816 x 1024 15 / 17).  Beyond them the rounds of the chip decide, and of equal ones the larger tile (883 x 2112 x 1024, us as 64 x 64 / 32 x 64 / 32 x 32: 44 / 47 / 48; 883 x 2816 x 1024 61 / 53 / 55; 300 x 2112 x 1024
+    // 24 / 25 / 20).  An expert's last tile stands half empty on average; for the first question every expert counts as one tile at least, which is what evenly spread rows come to (8 experts of
+    // 768 x 1024, 200 rows: even 12 / 17, as a router spreads them 16 / 17).
+    const int64_t M = p.M, N = p.N, round = 256;
+    auto cols = [&](int ni) { return (N + 32 * ni - 1) / (32 * ni); };
+    auto tiles = [&](int mi, int ni) { return ((M + 32 * mi - 1) / (32 * mi) + (p.offsets ? p.E / 2 : 0)) * cols(ni); };
+    if ((p.offsets ? std::max<int64_t>((M + 31) / 32, p.E) * cols(1) : tiles(1, 1)) <= round) return launch_f32<2, 2, 4, FIN>(p, stream);
+    if constexpr (FIN != ARIA_F32_PAIR) {   // (two weights' sums of 64 x 32 do not fit the static LDS)
+        if (!p.offsets && tiles(2, 1) <= round) return launch_f32<4, 2, 4, FIN>(p, stream);
+    }
+    auto cost = [&](int mi, int ni, int more) { return (tiles(mi, ni) + round - 1) / round * mi * ni * (100 + more); };
     const int64_t c22 = cost(2, 2, 0), c12 = cost(1, 2, 5), c11 = cost(1, 1, 10);
     if (c22 <= c12 && c22 <= c11) return launch_f32_tiles<2, 2, FIN>(p, {}, stream);
     return c12 <= c11 ? launch_f32_tiles<1, 2, FIN>(p, {}, stream) : launch_f32_tiles<1, 1, FIN>(p, {}, stream);
@@ -411,7 +419,7 @@ __attribute__((visibility("hidden"))) int aria_gemm_f32_heads(const float* part_
 
 int aria_gemm_f32_finished(const AriaGemmF32& p, int finish, void* stream) {
     if (!p.A || !p.W || !p.C || p.M < 0 || p.N < 0 || p.K <= 0 || (p.offsets && p.E <= 0) || (p.rows && p.per <= 0) || (finish == ARIA_F32_PAIR && !p.W2) ||
-        (finish == ARIA_F32_STREAM && (!p.x || !p.post.w || p.offsets)))
+        (finish == ARIA_F32_STREAM && (!p.x || !p.post.w || p.offsets)) || (p.rows && (finish == ARIA_F32_RELU2 || finish == ARIA_F32_STREAM)))
         return ARIA_ERR_INVALID;
     if (((reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W) | reinterpret_cast<uintptr_t>(p.W2)) & 15) || (p.lda & 3) || (p.ldw & 3) || (p.K & 3) || (p.strideW & 3))
         return ARIA_ERR_ALIGN;
@@ -421,7 +429,7 @@ int aria_gemm_f32_finished(const AriaGemmF32& p, int finish, void* stream) {
         case ARIA_F32_RELU2: return product_f32<ARIA_F32_RELU2>(p, stream);
         case ARIA_F32_PAIR: return product_f32<ARIA_F32_PAIR>(p, stream);
         case ARIA_F32_STREAM: return product_f32<ARIA_F32_STREAM>(p, stream);
-        default: return product_f32<ARIA_F32_PLAIN>(p, stream);
+        default: return p.rows ? product_f32<FIN_ROWS>(p, stream) : product_f32<ARIA_F32_PLAIN>(p, stream);
     }
 }
 
