@@ -602,3 +602,11 @@ def case_float32_step_as_one_call(dev, monkeypatch, name):
     both([toks[0][11:12]], [11], None, one_call=False)
     hook.remove()
     assert calls
+
+
+# float32 steps whose products take more than a round of 64 x 32 tiles (latent_cases.WIDE_STEPS)
+WIDE_STEPS = {
+    "layers": (config([parallel(left(heads=8, kv_heads=2, dim=128, vdim=128, size=500), right(heads=4, dim=128, vdim=120, tau=16.0), ff=2824),
+                       lightning(heads=8, dim=128, vdim=128, decay=[0.9 + 0.01 * i for i in range(8)], ff=768)], width=1024, vocab=8197), (50, 300, 620, 883, 1088, 1300)),
+    "ends": (config([lightning(heads=1, dim=8, vdim=8, decay=(0.8,), ff=2077)], width=24, vocab=4105), (260,)),
+}

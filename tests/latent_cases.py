@@ -666,6 +666,45 @@ def case_float32_step_as_one_call(dev, monkeypatch, name):
     assert calls
 
 
+# float32 steps whose products take more than a round of 64 x 32 tiles, so that the staged 32-bit tiles compute them: widths whose reductions and last tiles end anywhere
+WIDE_STEPS = {
+    # squared relu, gate times up gathered by expert, the stream's step; on every tile shape between 300 and 1632 tokens
+    "layers": (config([(mixer(heads=8, dim=64, rot_dim=32, vdim=128, kv_rank=250), dense(ff=2824)), (mixer(heads=8, dim=64, rot_dim=32, vdim=120, kv_rank=256), moe(ff=768, experts=16, top=2)),
+                       (mixer(heads=4, dim=64, rot_dim=32, vdim=128, kv_rank=256), moe(ff=776, experts=16, top=2))], width=1024, vocab=8197), (50, 300, 620, 883, 1088, 1300, 1632)),
+    # the same at sizes for the emulator
+    "ends": (config([(mixer(heads=2, dim=16, rot_dim=8, vdim=16, kv_rank=32), dense(ff=2077)), (mixer(heads=1, dim=8, rot_dim=2, vdim=24, kv_rank=20), moe(ff=1037, experts=4, top=2, count=2,
+                                                                                                                                                     keep=1))], width=24, vocab=4105), (260,)),
+    "stream": (config([(mixer(heads=1, dim=8, rot_dim=2, vdim=12, kv_rank=20), dense(ff=20))], width=1032, vocab=40), (450,)),
+}
+
+
+def case_float32_step_beyond_a_round(dev, monkeypatch, build, cfg, w, counts):
+    """Prompts of `counts` tokens as one call and sublayer by sublayer: the same bits of the logits of every row, of a hundred rows in any order, and of the tokens that follow them."""
+    from aria_amd import ops
+    from aria_amd.serving import StepBatch
+
+    one, ref = build(cfg, w, dev, f32), build(cfg, w, dev, f32)
+    for n in counts:
+        toks = tokens(cfg, n + 3, seed=n)
+        lens = [n // 2 - 1, n // 3, n - (n // 2 - 1) - n // 3]
+        cuts = [0, lens[0], lens[0] + lens[1], n]
+        for m in (one, ref):
+            m.setup_caches(3, max(lens) + 1)
+
+        def both(seqs, starts, wanted):
+            batch = StepBatch.build(seqs, [0, 1, 2], starts, wanted, dev)
+            with monkeypatch.context() as mp:
+                mp.setattr(ops, "linear_any", None)
+                got = one.step(batch)
+            assert torch.isfinite(got).all()
+            assert torch.equal(got.cpu(), ref.step(batch, []).cpu()), n
+
+        prompts = [toks[a:b] for a, b in zip(cuts, cuts[1:])]
+        both(prompts, [0, 0, 0], None)
+        both(prompts, [0, 0, 0], torch.randperm(n, generator=gen(n))[:100].tolist())
+        both([[t] for t in toks[n:]], lens, None)
+
+
 def case_latent_attention_f32(dev, H, R, dr, dv, runs):
     """32-bit latent attention and its expansion against float64, tokens given as (slot, first position, tokens) runs: several heads and tokens a workgroup, tokens
     of several sequences, portions, an earlier position behind a later one; splits for few tokens.  32-bit sums of cw products: errors of some 1e-6.  A row

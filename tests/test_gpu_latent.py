@@ -148,6 +148,12 @@ def test_bad_inputs():
     C.case_bad_inputs(DEV)
 
 
+@pytest.mark.parametrize("name", ["layers", "ends", "stream"])
+def test_float32_step_beyond_a_round(monkeypatch, name):
+    cfg, counts = C.WIDE_STEPS[name]
+    C.case_float32_step_beyond_a_round(DEV, monkeypatch, C.build, cfg, C.checkpoint(cfg, seed=3), counts)
+
+
 @pytest.mark.parametrize("name", ["mixed", "odd"])
 def test_float32_step_as_one_call(monkeypatch, name):
     C.case_float32_step_as_one_call(DEV, monkeypatch, name)
