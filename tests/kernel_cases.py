@@ -198,6 +198,42 @@ def case_wgrad_strips_long(dev, monkeypatch, counts, M, N):
         assert torch.equal(a, b)
 
 
+def case_wgrad_rule(dev, monkeypatch):
+    """Which weight gradients are strips, on both sides of the rule's lines: 144 rows an expert on more than 64 million outputs, dense ones of up to 256 rows on as many or, under 64 rows, on
+    more than 16 million; not into 32 bits, not added to what is there."""
+    from aria_amd import ops
+
+    monkeypatch.delenv("ARIA_GEMM_FORCE", raising=False)
+    E, K, N = 64, 1024, 1280
+
+    def grouped(rows, e=E, **kw):
+        x, dy = torch.zeros((rows, K), dtype=bf16, device=dev), torch.zeros((rows, N), dtype=bf16, device=dev)
+        off = torch.full((e + 1,), rows, dtype=torch.int32, device=dev)
+        off[0] = 0
+        ops.grouped_gemm_wgrad(x, dy, off, e, **kw)
+        plain = last_gemm_tiles() & 15
+        if not kw:
+            ops.grouped_gemm_wgrad_gather(x, torch.zeros(rows + 64, dtype=torch.int32, device=dev)[:rows], dy, off, e)
+            assert last_gemm_tiles() & 15 == plain
+        return plain
+
+    assert grouped(144 * E) == 4 and grouped(144 * E + 1) == 3 and grouped(1) == 4
+    assert grouped(144, e=1) == 3
+    assert grouped(E, out_dtype=torch.float32) == 3
+    assert grouped(E, out=torch.zeros((E, K, N), dtype=bf16, device=dev), accumulate=True) == 3
+
+    def dense(rows, M, n, **kw):
+        a, b = torch.zeros((rows, M), dtype=bf16, device=dev), torch.zeros((rows, n), dtype=bf16, device=dev)
+        ops.gemm(a, b, a_oc=True, b_oc=True, **kw)
+        return last_gemm_tiles() & 15
+
+    for rows in (1, 16, 63, 64, 256):
+        assert dense(rows, 65600, 1024) == 4, rows
+    assert dense(257, 65600, 1024) != 4 and dense(64, 64, 1024) != 4
+    assert dense(63, 16448, 1024) == 4 and dense(63, 16384, 1024) != 4 and dense(64, 16448, 1024) != 4
+    assert dense(16, 65600, 1024, out_dtype=torch.float32) != 4
+
+
 def case_gemm_four_waves(dev, monkeypatch, force, M, N, K, a_oc, b_oc):
     """The four-wave tiles add the products of an output element in the order of the 256 x 256 ones: the same bits, with every end of a plain product (bias,
     activations, accumulation, 32-bit results, an output whose rows are no whole 16-byte pieces)."""

@@ -283,6 +283,10 @@ def test_wgrad_strips_long(monkeypatch, counts, M, N):
     C.case_wgrad_strips_long(DEV, monkeypatch, counts, M, N)
 
 
+def test_wgrad_rule(monkeypatch):
+    C.case_wgrad_rule(DEV, monkeypatch)
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 136, 128), (350, 7680, 2560), (777, 2560, 2560), (3000, 2560, 3328)])
 def test_gemm_keep_sums(monkeypatch, M, N, K):
     C.case_gemm_keep_sums(DEV, monkeypatch, M, N, K)
