@@ -139,7 +139,8 @@ __global__ __launch_bounds__(512) void lora_down_kernel(const bf16_t* X, const b
 // 5580 rows of 1536 on 32 columns as 128 x 128 tiles of the general kernel 25.8 us.
 constexpr int XR = 512, XPITCH = XR + 8;   // (16 bytes: 16 rows' pieces lie on different banks)
 // An adapter's u = bf16(scale * bf16(x W)) too (T = bf16_t; per expert where there are offsets, W_OC: W [K][N]): the forward's, in front of routers like the base products.  With the launches it takes
-// the place of, us: cold rows, rank 8: 777 of 2560 27.6, here 21.5, 4096 32 / 19, 16 384 56 / 40; rows by expert, 4662 of 2560 58 / 19, 24 576 74 / 56, 98 304 174 / 151.
+// the place of, us: cold rows, rank 8: 777 of 2560 27.6, here 21.5, 4096 32 / 19, 16 384 56 / 40; rows by expert, 4662 of 2560 58 / 19, 24 576 74 / 56, 98 304 174 / 151; where it
+// is the slower one: lora_u_takes of ops.py.
 template <bool W_OC, class T>
 __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, T* C, const int32_t* offsets, int E, int M, int N, int K, long long ldx, long long ldc,
                                                            int cut_row, int cut, float scale) {

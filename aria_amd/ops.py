@@ -292,10 +292,13 @@ def lora_scale(u: torch.Tensor, scale: float, out=None) -> torch.Tensor:
 
 
 def lora_u_takes(x: torch.Tensor, w: torch.Tensor, w_oc: bool) -> bool:
-    """whether ``lora_u`` takes the product; others are the general product's, then a scaling"""
+    """Whether ``lora_u`` takes the product; others are the general product's, then a scaling.  Those are the faster ones on many rows, whose 16 columns or long reductions one wave of a
+    block multiplies: us, general / here, 64 experts, rank 16, 512 rows each of 2560 66 / 57, 768 52 / 79, 1536 121 / 147; of 1664 47 / 42, 37 / 58, 77 / 105; dense 32 768 of 2560 49 / 45, 65 536
+    65 / 87; rank 8 of 3328, 512 each 80 / 61, 768 71 / 86.  Rank 8 by expert of up to 2560 gains at any size (384 each 54 / 30, 768 50 / 50, 1536 119 / 100)."""
     K, r = (w.shape[-2], w.shape[-1]) if w_oc else (w.shape[-1], w.shape[-2])
     return (GEMM_SPLIT_K and lora_thin(r, K) and x.dtype == w.dtype == bf16 and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.dim() == 2 and x.shape[1] == K
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and 0 < x.shape[0] < 1 << 30)
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and 0 < x.shape[0] < 1 << 30
+            and (x.shape[0] <= 32768 or (r == 8 and w_oc and K <= 2560)))
 
 
 def lora_u(x: torch.Tensor, w: torch.Tensor, scale: float, offsets=None, out=None) -> torch.Tensor:

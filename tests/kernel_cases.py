@@ -1460,6 +1460,17 @@ def case_lora_u(dev, M, K, r, counts=None):
     assert bool((out[:, :2] == 7).all() and (out[:, 2 + r:] == 7).all())
 
 
+def case_lora_u_rule(dev):
+    """the thin product takes an adapter's forward projection up to 32 768 rows, at rank 8 by expert of up to 2560 columns any number"""
+    from aria_amd import ops
+
+    for rows, r, K, by_expert, takes in ((32768, 16, 2560, True, True), (32769, 16, 2560, True, False), (32769, 16, 1664, False, False), (32769, 8, 2560, False, False),
+                                         (100000, 8, 2560, True, True), (32769, 8, 2624, True, False), (32768, 8, 3328, True, True), (0, 8, 2560, True, False)):
+        x = torch.zeros(K, dtype=bf16, device=dev).expand(rows, K)
+        w = torch.zeros((64, K, r) if by_expert else (r, K), dtype=bf16, device=dev)
+        assert ops.lora_u_takes(x, w, by_expert) == takes, (rows, r, K, by_expert)
+
+
 def case_lora_up_swiglu(dev, M, K, r, counts=None):
     """An adapter's masked input gradient through the backward of silu(gate) * up in one launch: the bits of the two, the gradient that it starts from untouched."""
     from aria_amd import ops

@@ -306,6 +306,10 @@ def test_sort_with_token_rows(T, k, E):
     C.case_sort_rows(DEV, T, k, E)
 
 
+def test_lora_u_rule():
+    C.case_lora_u_rule(DEV)
+
+
 @pytest.mark.parametrize("M,K,r,counts", [(37, 72, 8, None), (33, 520, 16, [1, 0, 32])])
 def test_lora_up_swiglu(M, K, r, counts):
     C.case_lora_up_swiglu(DEV, M, K, r, counts)
