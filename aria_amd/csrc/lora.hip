@@ -219,74 +219,79 @@ __device__ __forceinline__ float half_of(const u32x4& v, int i) { return i & 1 ?
 
 // DX[m][k] += keep ? scale * sum_j DU[m][j] A[j][k] : 0.  A: [r][K] (a_oc), else [K][r]; per expert where there are offsets.  mask null: every element is kept.
 // A lane holds eight columns of A and runs a wave's eight rows through them: a read and a write of DX, on the vector pipe in 32 bits, rounded once.
-// GLU: DX is the gradient of silu(gate) up and stays as it is; its sum goes through the backward of that, H [M, 2 K] = [gate | up], DH its gradient (the bits of the two launches; us,
-// two / one: 4096 rows of 3328 52.5 / 48.5, by expert 24 576 of 1664 133 / 129, 98 304 507 / 396).
+// GLU: DX is the gradient of silu(gate) up and stays as it is; its sum goes through the backward of that, H [M, 2 K] = [gate | up], DH its gradient (the bits of the two launches, which
+// are the faster ones on few rows: lora_up_swiglu_pays of ops.py).
 template <int R8, bool A_OC, bool GLU>
 __global__ __launch_bounds__(256) void lora_up_kernel(const bf16_t* DU, const bf16_t* A, const unsigned char* mask, bf16_t* DX, const int32_t* offsets, int E, int M,
                                                       int K, long long ldu, float scale, const bf16_t* H, bf16_t* DH) {
-    constexpr int r = 8 * R8, NR = ROWS / 4;
+    // rows at a time (by expert at rank 16 with GLU four: eight with their gate and up take 320 registers, one wave a SIMD; 4096 rows of 1664 34.8 / 30.6 us, 24 576 151 / 128, 98 304 562 /
+    // 472; dense ones lose, the factor's rows being held for both halves: 2048 rows of 1664 13.6 / 14.8)
+    constexpr int r = 8 * R8, NR = GLU && R8 == 2 && !A_OC ? ROWS / 8 : ROWS / 4;
     int e, m0, m1;
     if (!rows_of(offsets, E, M, blockIdx.x, e, m0, m1)) return;
-    const int c = blockIdx.y * 64 + (threadIdx.x & 63), first = m0 + NR * first_lane(int(threadIdx.x) >> 6);
-    if (c >= K / 8 || first >= m1) return;
-    u32x4 old[NR];
-    unsigned keep[NR];
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        const long long m = min(first + i, m1 - 1);
-        old[i] = ld16(DX + m * K + 8 * c);
-        keep[i] = mask ? mask[m * (K / 8) + c] : 255u;
-    }
-    float y[NR][8];
-#pragma unroll
-    for (int i = 0; i < NR; ++i)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) y[i][q] = 0.f;
+    const int c = blockIdx.y * 64 + (threadIdx.x & 63), begin = m0 + ROWS / 4 * first_lane(int(threadIdx.x) >> 6);
+    if (c >= K / 8) return;
     const bf16_t* ae = A + (long long)e * r * K;
-#pragma unroll
-    for (int jb = 0; jb < R8; ++jb) {
-        u32x4 a[8];   // A_OC: eight columns of factor row 8 jb + i; else factor entries 8 jb .. of column 8 c + i
-#pragma unroll
-        for (int i = 0; i < 8; ++i) a[i] = A_OC ? ld16(ae + (long long)(8 * jb + i) * K + 8 * c) : ld16(ae + (8ll * c + i) * r + 8 * jb);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            const u32x4 d = ld16(DU + (long long)min(first + i, m1 - 1) * ldu + 8 * jb);
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-#pragma unroll
-                for (int q = 0; q < 8; ++q) y[i][q] = fmaf(half_of(d, j), A_OC ? half_of(a[j], q) : half_of(a[q], j), y[i][q]);
-        }
-    }
-    u32x4 gate[GLU ? NR : 1], up[GLU ? NR : 1];
-    if (GLU)
+#pragma unroll 1
+    for (int first = begin; first < min(begin + ROWS / 4, m1); first += NR) {
+        u32x4 old[NR];
+        unsigned keep[NR];
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-            const bf16_t* h = H + (long long)min(first + i, m1 - 1) * 2 * K + 8 * c;
-            gate[GLU ? i : 0] = ld16(h), up[GLU ? i : 0] = ld16(h + K);
+            const long long m = min(first + i, m1 - 1);
+            old[i] = ld16(DX + m * K + 8 * c);
+            keep[i] = mask ? mask[m * (K / 8) + c] : 255u;
         }
+        float y[NR][8];
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-        if (first + i >= m1) break;
-        u32x4 o;
+        for (int i = 0; i < NR; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float lo = keep[i] >> (2 * q) & 1u ? scale * y[i][2 * q] : 0.f, hi = keep[i] >> (2 * q + 1) & 1u ? scale * y[i][2 * q + 1] : 0.f;
-            o[q] = pack2bf(bflo(old[i][q]) + lo, bfhi(old[i][q]) + hi);
+            for (int q = 0; q < 8; ++q) y[i][q] = 0.f;
+#pragma unroll
+        for (int jb = 0; jb < R8; ++jb) {
+            u32x4 a[8];   // A_OC: eight columns of factor row 8 jb + i; else factor entries 8 jb .. of column 8 c + i
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[i] = A_OC ? ld16(ae + (long long)(8 * jb + i) * K + 8 * c) : ld16(ae + (8ll * c + i) * r + 8 * jb);
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const u32x4 d = ld16(DU + (long long)min(first + i, m1 - 1) * ldu + 8 * jb);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) y[i][q] = fmaf(half_of(d, j), A_OC ? half_of(a[j], q) : half_of(a[q], j), y[i][q]);
+            }
         }
-        if (GLU) {
-            u32x4 dg, du;
+        u32x4 gate[GLU ? NR : 1], up[GLU ? NR : 1];
+        if (GLU)
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                const bf16_t* h = H + (long long)min(first + i, m1 - 1) * 2 * K + 8 * c;
+                gate[GLU ? i : 0] = ld16(h), up[GLU ? i : 0] = ld16(h + K);
+            }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            if (first + i >= m1) break;
+            u32x4 o;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const u32x4 &g = gate[GLU ? i : 0], &u = up[GLU ? i : 0];
-                f32x2 da, db;
-                swiglu_bwd_pair(f32x2{bflo(g[q]), bfhi(g[q])}, f32x2{bflo(u[q]), bfhi(u[q])}, f32x2{bflo(o[q]), bfhi(o[q])}, da, db);
-                dg[q] = pack2bf(da.x, da.y), du[q] = pack2bf(db.x, db.y);
+                const float lo = keep[i] >> (2 * q) & 1u ? scale * y[i][2 * q] : 0.f, hi = keep[i] >> (2 * q + 1) & 1u ? scale * y[i][2 * q + 1] : 0.f;
+                o[q] = pack2bf(bflo(old[i][q]) + lo, bfhi(old[i][q]) + hi);
             }
-            bf16_t* d = DH + (long long)(first + i) * 2 * K + 8 * c;
-            st16(d, dg);
-            st16(d + K, du);
-        } else {
-            st16(DX + (long long)(first + i) * K + 8 * c, o);
+            if (GLU) {
+                u32x4 dg, du;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const u32x4 &g = gate[GLU ? i : 0], &u = up[GLU ? i : 0];
+                    f32x2 da, db;
+                    swiglu_bwd_pair(f32x2{bflo(g[q]), bfhi(g[q])}, f32x2{bflo(u[q]), bfhi(u[q])}, f32x2{bflo(o[q]), bfhi(o[q])}, da, db);
+                    dg[q] = pack2bf(da.x, da.y), du[q] = pack2bf(db.x, db.y);
+                }
+                bf16_t* d = DH + (long long)(first + i) * 2 * K + 8 * c;
+                st16(d, dg);
+                st16(d + K, du);
+            } else {
+                st16(DX + (long long)(first + i) * K + 8 * c, o);
+            }
         }
     }
 }

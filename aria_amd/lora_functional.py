@@ -124,7 +124,7 @@ def dense_lora_bwd(dy: torch.Tensor, ctx, dx: torch.Tensor, grads: dict, keys: L
         if thin:
             du = ops.lora_down(dy[:, r0:r1], _factor(s.b), s.scaling, w_oc=True)
             dA, dB = ops.lora_wgrad(d.xd, du, n_first=False), ops.lora_wgrad(dy[:, r0:r1], U[:, c0:c0 + r], n_first=True)
-            if h is not None and len(live) == 1 and h.is_contiguous():
+            if h is not None and len(live) == 1 and h.is_contiguous() and ops.lora_up_swiglu_pays(dx.shape[0], r):
                 dx, h = ops.lora_up_swiglu(dx, du, _factor(s.a), d.mask, d.p, h), None
             else:
                 ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p)
@@ -167,7 +167,7 @@ def grouped_lora_bwd(dy: torch.Tensor, ctx, offsets: torch.Tensor, dx: torch.Ten
     dB = ops.grouped_gemm_wgrad(ctx["U"], dy, offsets, E)                                   # [E, r, N]
     dA = ops.grouped_gemm_wgrad(d.xd, du, offsets, E)                                       # [E, K, r]
     grads[key] = (dA, dB)
-    if thin and h is not None and h.is_contiguous():
+    if thin and h is not None and h.is_contiguous() and ops.lora_up_swiglu_pays(dx.shape[0], s.a.shape[2], E):
         return ops.lora_up_swiglu(dx, du, _factor(s.a), d.mask, d.p, h, offsets=offsets)
     if thin:
         ops.lora_up_(dx, du, _factor(s.a), d.mask, d.p, offsets=offsets)                             # d_u lora_A[e]^T

@@ -345,6 +345,15 @@ def lora_up_(dx: torch.Tensor, du: torch.Tensor, a: torch.Tensor, mask, p: float
     return dx
 
 
+def lora_up_swiglu_pays(rows: int, r: int, experts: Optional[int] = None) -> bool:
+    """Where ``lora_up_swiglu`` is faster than its two launches.  Us, two / one, 3328 columns (dense), 1664 (64 experts): rank 8, 200 rows 8.8 / 8.7, 384 10.1 / 9.2, 4096 36.7 / 29.4, 16 384
+    141 / 117; by expert 1024 13.7 / 16.2 (a few rows of a block's 32 are an expert's), 2048 18.2 / 16.3, 24 576 110 / 93.  Rank 16, 64 rows 9.4 / 10.0, 700 14.0 / 12.3, 2048 25.2 / 24.7, 4096
+    42.2 / 44.2 (gate and up beside 16 factor rows leave one wave a SIMD), 16 384 155 / 166; by expert 1024 19.2 / 20.6, 2048 23.6 / 22.1, 24 576 158 / 128."""
+    if experts is not None:
+        return rows >= 32 * experts
+    return rows >= 256 if r == 8 else 512 <= rows <= 2048
+
+
 def lora_up_swiglu(d: torch.Tensor, du: torch.Tensor, a: torch.Tensor, mask, p: float, h: torch.Tensor, offsets=None) -> torch.Tensor:
     """``swiglu_bwd(h, lora_up_(d, du, a, mask, p, offsets))`` in one launch: d [M, K] is only read, h [M, 2 K] = [gate | up] -> its gradient."""
     _chk(d, name="d"), _chk(du, name="du"), _chk(a, name="a"), _chk(h, name="h")

@@ -1485,6 +1485,37 @@ def case_lora_up_swiglu(dev, M, K, r, counts=None):
         assert torch.equal(got, ops.swiglu_bwd(h, ops.lora_up_(before, du, a, mask, p, offsets=off)))
 
 
+def case_lora_up_swiglu_rule(dev):
+    """one launch or two: by expert from 32 rows each, dense from 256 at rank 8 and between 512 and 2048 at rank 16; the adapter's backward asks"""
+    from aria_amd import lora_functional as LF
+    from aria_amd import ops
+
+    for rows, r, experts, pays in ((255, 8, None, False), (256, 8, None, True), (511, 16, None, False), (512, 16, None, True), (2048, 16, None, True), (2049, 16, None, False),
+                                   (2047, 8, 64, False), (2048, 8, 64, True), (128, 16, 4, True), (127, 16, 4, False)):
+        assert ops.lora_up_swiglu_pays(rows, r, experts) == pays, (rows, r, experts)
+    calls = []
+    real = ops.lora_up_swiglu
+
+    def seen(*a, **kw):
+        calls.append(a[0].shape[0])
+        return real(*a, **kw)
+
+    ops.lora_up_swiglu = seen
+    try:
+        for M in (40, 264):
+            x, dy, h = rnd(M, 64, seed=1).to(dev), rnd(M, 128, seed=2).to(dev), rnd(M, 128, seed=3).to(dev)
+            site = LF.LoraSite(rnd(8, 64, seed=4).to(dev), rnd(128, 8, seed=5).to(dev), 2.0, 0.3)
+            _, ctx = LF.dense_lora_fwd(x, rnd(128, 64, seed=6).to(dev), [site], [128], True, seeds=[7])
+            dx, grads = rnd(M, 64, seed=8).to(dev), {}
+            got = LF.dense_lora_bwd(dy, ctx, dx.clone(), grads, ["down"], h=h)
+            want = dx.clone()
+            LF.dense_lora_bwd(dy, ctx, want, grads, ["down"])
+            assert torch.equal(got, ops.swiglu_bwd(h, want))
+    finally:
+        ops.lora_up_swiglu = real
+    assert calls == [264]
+
+
 def case_sort_rows(dev, T, k, E):
     """The dispatcher's stable sort and the token of every place == a stable argsort, on both sides of the one-launch form's 8192 entries and of a block's four chunks."""
     from aria_amd import ops

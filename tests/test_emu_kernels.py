@@ -310,6 +310,15 @@ def test_lora_u_rule():
     C.case_lora_u_rule(DEV)
 
 
+@pytest.mark.parametrize("M,K,r,counts", [(72, 520, 16, [5, 4, 9, 3, 31, 0, 20])])   # four rows of a wave's eight at a time
+def test_lora_up_swiglu_halves(M, K, r, counts):
+    C.case_lora_up_swiglu(DEV, M, K, r, counts)
+
+
+def test_lora_up_swiglu_rule():
+    C.case_lora_up_swiglu_rule(DEV)
+
+
 @pytest.mark.parametrize("M,K,r,counts", [(37, 72, 8, None), (33, 520, 16, [1, 0, 32])])
 def test_lora_up_swiglu(M, K, r, counts):
     C.case_lora_up_swiglu(DEV, M, K, r, counts)

@@ -306,6 +306,15 @@ def test_lora_u_rule():
     C.case_lora_u_rule(DEV)
 
 
+@pytest.mark.parametrize("M,K,r,counts", [(72, 520, 16, [5, 4, 9, 3, 31, 0, 20]), (24576, 1664, 16, [384] * 64)])   # four rows of a wave's eight at a time
+def test_lora_up_swiglu_halves(M, K, r, counts):
+    C.case_lora_up_swiglu(DEV, M, K, r, counts)
+
+
+def test_lora_up_swiglu_rule():
+    C.case_lora_up_swiglu_rule(DEV)
+
+
 @pytest.mark.parametrize("M,K,r,counts", [(1, 8, 8, None), (37, 72, 8, None), (33, 520, 16, [1, 0, 32]), (4096, 3328, 8, None), (4662, 1664, 8, [73] * 63 + [63])])
 def test_lora_up_swiglu(M, K, r, counts):
     C.case_lora_up_swiglu(DEV, M, K, r, counts)
