@@ -145,8 +145,8 @@ template <bool W_OC, class T>
 __global__ __launch_bounds__(512) void thin_product_kernel(const bf16_t* X, const bf16_t* W, T* C, const int32_t* offsets, int E, int M, int N, int K, long long ldx, long long ldc,
                                                            int cut_row, int cut, float scale) {
     ARIA_DYN_SMEM(lds);
-    int e, m0;
-    if (!rows_of(offsets, E, M, blockIdx.x, e, m0, M)) return;
+    int e = 0, m0 = blockIdx.x * ROWS;
+    if (sizeof(T) == 2 && !rows_of(offsets, E, M, blockIdx.x, e, m0, M)) return;   // (routers have no experts to ask for: 0.3 us of 7)
     const int t = threadIdx.x, l = t & 63, w = first_lane(t >> 6), pitch = K + 8, nch = K / 64, pieces = m0 >= cut_row ? cut : 1;
     bf16_t* xs = reinterpret_cast<bf16_t*>(lds);   // [32][XPITCH]
     bf16_t* ws = xs + ROWS * XPITCH;               // [N][pitch]
