@@ -666,6 +666,41 @@ def case_float32_step_as_one_call(dev, monkeypatch, name):
     assert calls
 
 
+def case_latent_cache_rows(dev, dtype, H, R, dr):
+    """The cache rows that a step of 1 .. 9 single tokens writes: the bits that do not depend on how many waves share a row, and the normed latent and rotated key within 32-bit rounding (bf16:
+    one more) of float64."""
+    import ctypes
+
+    from aria_amd import hip, ops
+
+    cw, dq, cap = (R + dr + 63) // 64 * 64, (8 + dr + 7) // 8 * 8, 40
+    s = hip.LatentShape(H=H, dn=8, dr=dr, dv=8, R=R, rot=dr, dq=dq, dvp=8, cw=cw, rp=(R + 7) // 8 * 8, kv_off=H * dq, g_off=H * dq + R + dr, S_cap=cap, scale=0.2, eps=1e-5)
+    s.ldp = (s.g_off + H + 7) // 8 * 8
+    n = 9
+    proj, rope, wn = rnd(n, s.ldp, seed=1, dtype=dtype).to(dev), rnd(cap, dr, seed=2, dtype=f32).to(dev), rnd(R, seed=3, dtype=f32).to(dev)
+    uk = rnd(H * 8, s.rp, seed=4, dtype=dtype).to(dev)
+    pos = torch.randint(0, cap, (n,), generator=gen(5)).to(torch.int32).to(dev)
+
+    def rows(first, count):
+        slot = torch.arange(first, first + count, dtype=torch.int32, device=dev)
+        cache, qa = torch.full((n, cap, cw), 7.0, dtype=dtype, device=dev), torch.empty(count, H, cw, dtype=dtype, device=dev)
+        p, at = proj[first:first + count].contiguous(), pos[first:first + count].contiguous()
+        hip.get_lib().call("aria_latent_absorb", p.data_ptr(), ctypes.byref(s), slot.data_ptr(), at.data_ptr(), rope.data_ptr(), wn.data_ptr(), uk.data_ptr(), cache.data_ptr(), qa.data_ptr(),
+                           count, int(dtype == f32), ops._stream(p))
+        return torch.stack([cache[first + i, int(at[i])] for i in range(count)])
+
+    alone = torch.cat([rows(i, 1) for i in range(n)])
+    for count in range(2, n + 1):
+        assert torch.equal(rows(0, count), alone[:count]), count
+    x = proj.cpu().double()[:, s.kv_off:s.kv_off + R + dr]
+    want = torch.zeros(n, cw, dtype=torch.float64)
+    want[:, :R] = x[:, :R] / (x[:, :R].pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * wn.cpu().double()
+    cs = rope.cpu().double()[pos.cpu().long()].view(n, dr // 2, 2)
+    a, b = x[:, R:R + dr // 2], x[:, R + dr // 2:]
+    want[:, R:R + dr // 2], want[:, R + dr // 2:R + dr] = a * cs[..., 0] - b * cs[..., 1], b * cs[..., 0] + a * cs[..., 1]
+    assert rel(alone, want) < (1e-6 if dtype == f32 else 3e-3)
+
+
 # float32 steps whose products take more than a round of 64 x 32 tiles, so that the staged 32-bit tiles compute them: widths whose reductions and last tiles end anywhere
 WIDE_STEPS = {
     # squared relu, gate times up gathered by expert, the stream's step; on every tile shape between 300 and 1632 tokens

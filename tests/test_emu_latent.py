@@ -112,6 +112,12 @@ def test_bad_inputs():
     C.case_bad_inputs(DEV)
 
 
+@both
+@pytest.mark.parametrize("H,R,dr", [(3, 40, 6), (2, 300, 64), (16, 512, 64)])
+def test_latent_cache_rows(dtype, H, R, dr):
+    C.case_latent_cache_rows(DEV, dtype, H, R, dr)
+
+
 @pytest.mark.parametrize("name", ["ends", "stream"])
 def test_float32_step_beyond_a_round(monkeypatch, name):
     cfg, counts = C.WIDE_STEPS[name]
