@@ -155,7 +155,7 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* q
             for (int k = 1; k < NW; ++k) v += *reinterpret_cast<const V*>(all + k * 16 * P + col * P + d);
             *reinterpret_cast<V*>(out + d) = v;
         };
-        if (R & 3)
+        if ((R & 3) || (reinterpret_cast<uintptr_t>(part_o) & 15))   // (a caller's buffer may start at any float)
             for (int d = lane; d < R; d += LANES) sums(0.f, d);
         else
             for (int d = 4 * lane; d < R; d += 4 * LANES) sums(f32x4{}, d);

@@ -666,6 +666,29 @@ def case_float32_step_as_one_call(dev, monkeypatch, name):
     assert calls
 
 
+def case_latent_partials_anywhere(dev, T, n):
+    """32-bit latent attention into partial sums at any multiple of four bytes: the bits of an aligned buffer."""
+    import ctypes
+
+    from aria_amd import hip, ops
+
+    H, R, dr, cw = 5, 48, 8, 64
+    s = hip.LatentShape(H=H, dn=8, dr=dr, dv=8, R=R, rot=dr, dq=16, dvp=8, cw=cw, rp=48, ldp=160, kv_off=80, g_off=136, S_cap=n, scale=0.2, eps=1e-5)
+    qa, cache = rnd(T, H, cw, seed=1, dtype=f32).to(dev), rnd(1, n, cw, seed=2, dtype=f32).to(dev)
+    slot, pos = torch.zeros(T, dtype=torch.int32, device=dev), torch.arange(n - T, n, dtype=torch.int32, device=dev)
+    lib, ref = hip.get_lib(), ctypes.byref(s)
+    splits = int(lib.cdll.aria_latent_splits_f32(ref, T, n))
+    got = []
+    for shift in (0, 1, 2, 3):
+        flat, ml = torch.zeros(T * splits * H * R + 4, device=dev), torch.zeros(T, splits, H, 2, device=dev)
+        po = flat[shift:shift + T * splits * H * R]
+        lib.call("aria_latent_attn", qa.data_ptr(), cache.data_ptr(), ref, slot.data_ptr(), pos.data_ptr(), po.data_ptr(), ml.data_ptr(), T, splits, 1, ops._stream(qa))
+        got.append((po.clone(), ml))
+        assert not flat[:shift].any() and not flat[shift + po.numel():].any()
+    for po, ml in got[1:]:
+        assert torch.equal(po, got[0][0]) and torch.equal(ml, got[0][1])
+
+
 def case_latent_cache_rows(dev, dtype, H, R, dr):
     """The cache rows that a step of 1 .. 9 single tokens writes: the bits that do not depend on how many waves share a row, and the normed latent and rotated key within 32-bit rounding (bf16:
     one more) of float64."""

@@ -112,6 +112,11 @@ def test_bad_inputs():
     C.case_bad_inputs(DEV)
 
 
+@pytest.mark.parametrize("T,n", [(1, 200), (70, 80)])
+def test_latent_partials_anywhere(T, n):
+    C.case_latent_partials_anywhere(DEV, T, n)
+
+
 @both
 @pytest.mark.parametrize("H,R,dr", [(3, 40, 6), (2, 300, 64), (16, 512, 64)])
 def test_latent_cache_rows(dtype, H, R, dr):
