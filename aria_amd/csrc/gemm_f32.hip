@@ -1,4 +1,4 @@
-// C = A W^T in true 32-bit (v_mfma_f32_16x16x4_f32: 32-bit products, 32-bit sums, 256 multiply-adds a cycle and CU -- twice the vector pipe's unpacked rate).
+// C = A W^T in true 32-bit (v_mfma_f32_16x16x4_f32: 32-bit products, 32-bit sums, 128 multiply-adds a cycle and CU -- twice the vector pipe's unpacked rate).
 //
 // Both operands are k-contiguous: a lane loads 16 bytes of a row, four multiply steps whose reduction indices are whatever the four lanes of a row hold -- the same for
 // both operands.

@@ -492,42 +492,40 @@ __global__ __launch_bounds__(256) void unpermute_rows_kernel(const bf16_t* eo, c
             rows[j] = inv[(long long)t * K + j];
             sc[j] = scores ? bf2f(scores[(long long)t * K + j]) : 1.f;
         }
-        {
-            const int c = l + 64 * i;
-            u32x4 v[K], a = zero16();
+        const int c = l + 64 * i;
+        u32x4 v[K], a = zero16();
 #pragma unroll
-            for (int j = 0; j < K; ++j) v[j] = ld16(eo + (long long)rows[j] * D + c * 8);
-            if (add) a = ld16(add + (long long)t * D + c * 8);
-            float acc[8];
+        for (int j = 0; j < K; ++j) v[j] = ld16(eo + (long long)rows[j] * D + c * 8);
+        if (add) a = ld16(add + (long long)t * D + c * 8);
+        float acc[8];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] = 0.f;
+        for (int q = 0; q < 8; ++q) acc[q] = 0.f;
 #pragma unroll
-            for (int j = 0; j < K; ++j)
+        for (int j = 0; j < K; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (scores) {  // product materialised in bf16 by the reference (moe_lm.py:362)
-                        acc[2 * q] += rbf(bflo(v[j][q]) * sc[j]);
-                        acc[2 * q + 1] += rbf(bfhi(v[j][q]) * sc[j]);
-                    } else {
-                        acc[2 * q] += bflo(v[j][q]);
-                        acc[2 * q + 1] += bfhi(v[j][q]);
-                    }
+            for (int q = 0; q < 4; ++q) {
+                if (scores) {  // product materialised in bf16 by the reference (moe_lm.py:362)
+                    acc[2 * q] += rbf(bflo(v[j][q]) * sc[j]);
+                    acc[2 * q + 1] += rbf(bfhi(v[j][q]) * sc[j]);
+                } else {
+                    acc[2 * q] += bflo(v[j][q]);
+                    acc[2 * q + 1] += bfhi(v[j][q]);
                 }
-            u32x4 o;
-            if (add) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) o[q] = pack2bf(rbf(acc[2 * q]) + bflo(a[q]), rbf(acc[2 * q + 1]) + bfhi(a[q]));
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) o[q] = pack2bf(acc[2 * q], acc[2 * q + 1]);
             }
-            if (res) {   // r05b: the decoder layer's residual add `h + moe(h)` (moe_lm.py:617-627 through LlamaDecoderLayer) as a second rounding step
-                const u32x4 rv = ld16(res + (long long)t * D + c * 8);   // here instead of a launch of its own: bf16(h + bf16(moe)), as add_kernel gives
+        u32x4 o;
+        if (add) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) o[q] = pack2bf(bflo(rv[q]) + bflo(o[q]), bfhi(rv[q]) + bfhi(o[q]));
-            }
-            st16(out + (long long)t * D + c * 8, o);
+            for (int q = 0; q < 4; ++q) o[q] = pack2bf(rbf(acc[2 * q]) + bflo(a[q]), rbf(acc[2 * q + 1]) + bfhi(a[q]));
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q] = pack2bf(acc[2 * q], acc[2 * q + 1]);
         }
+        if (res) {   // the decoder layer's residual add `h + moe(h)` (moe_lm.py:617-627 through LlamaDecoderLayer) as a second rounding step
+            const u32x4 rv = ld16(res + (long long)t * D + c * 8);   // here instead of a launch of its own: bf16(h + bf16(moe)), as add_kernel gives
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q] = pack2bf(bflo(rv[q]) + bflo(o[q]), bfhi(rv[q]) + bfhi(o[q]));
+        }
+        st16(out + (long long)t * D + c * 8, o);
     }
 }
 

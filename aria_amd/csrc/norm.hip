@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* dy, cons
 }
 
 // 32 columns x 8 row-groups per block: 128-byte row segments, 8x the parallelism of one-thread-per-column.  The rows' latencies are the time: a thread's next eight are in flight
-// together and added in order.  With the norm's
-// backward in front, cold rows of 2560, one / eight in flight, us: 777 tokens (195 rows here) 21.7 / 15.8, 4096 (512) 48 / 32, 16 384 108 / 92.
+// together and added in order.  With the norm's backward in front, cold rows of 2560, one / eight in flight, us: 777 tokens (195 rows here) 21.7 / 15.8, 4096 (512) 48 / 32,
+// 16 384 108 / 92.
 constexpr int COLSUM_AHEAD = 8;
 __global__ __launch_bounds__(256) void colsum_kernel(const float* partial, bf16_t* out, int nrows, int D, int accumulate) {
     ARIA_SMEM_STATIC float red[8][32];

@@ -2,13 +2,13 @@
 group-limited mixture feed-forwards, and layers that run with another layer's weights on a cache of their own.
 
 This file reads the design's config.json and tensor names and assembles the mechanisms of ``layers.py`` into the serving protocol of ``serving.py``
-(caches, step function, scheduler, sampling and command line are the framework's).  A step runs in one of two ways:
+(caches, step function, scheduler, sampling and command line are the framework's).  A step runs in one of three ways:
 
 * prompts and large batches in bf16: sublayer by sublayer from here (tile GEMMs, flash attention, the fused stream passes);
 * up to ``DECODE_ROWS`` single tokens in bf16: one C call (``aria_latent_decode``) that enqueues every kernel of every layer;
-* float32: one C call (``aria_latent_step_f32``) that enqueues the launches of the step run sublayer by sublayer, for any batch.  The host bounded that step: three
-  layers 1024 wide, four prompts of up to 250 tokens and four decoded tokens, took it 3.1 ms (6 on a slower host), 1.2 ms as calls, the look
-  at every tensor, constant and module before each included."""
+* float32: one C call (``aria_latent_step_f32``) with the results of the step run sublayer by sublayer, bit for bit, in fewer launches (activations and the stream's steps in the
+  products' epilogues), for any batch.  The host bounded that step: three layers 1024 wide, four prompts of up to 250 tokens and four decoded tokens, took it 3.1 ms (6 on a slower
+  host), 1.2 ms as calls, the look at every tensor, constant and module before each included."""
 from __future__ import annotations
 
 import ctypes

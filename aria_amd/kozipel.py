@@ -3,12 +3,13 @@ by two mixers side by side, chunk-local softmax attention and gated linear atten
 embedding output added to the stream before every pass but the first; every pass has a cache and states of its own.
 
 This file reads the design's config.json and tensor names and assembles the mechanisms of ``layers.py`` into the serving protocol of ``serving.py``
-(caches, step function, scheduler, sampling and command line are the framework's).  A step runs in one of two ways:
+(caches, step function, scheduler, sampling and command line are the framework's).  A step runs in one of three ways:
 
 * prompts and large batches in bf16: sublayer by sublayer from here (tile GEMMs, flash attention and linear attention on the matrix pipe, the fused stream
   pass);
 * up to ``DECODE_ROWS`` single tokens in bf16: one C call (``aria_mix_decode``) that enqueues every kernel of every layer run;
-* float32: one C call (``aria_mix_step_f32``) that enqueues the launches of the step run sublayer by sublayer, for any batch."""
+* float32: one C call (``aria_mix_step_f32``) with the results of the step run sublayer by sublayer, bit for bit, in fewer launches (gate times up in one product's epilogue), for any
+  batch."""
 from __future__ import annotations
 
 import ctypes
