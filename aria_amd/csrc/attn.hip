@@ -1597,16 +1597,24 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // Blocks of 128 queries rather than 256, four waves and two workgroups a CU rather than eight and one.  They halve what a launch's longest blocks and its last round cost and stage the keys
 // twice as often.  Us, 256 / 128 queries a block:
 //
-// Causal, the longest blocks first.  128 columns, 20 heads: 280 tokens 19.9 / 14.7, 777 36 / 28, 4096 135 / 124, 8192 442 / 402, 12000 857 / 852, 32768 5536 / 6052.  The blocks of all heads run
-// side by side, so keys and values come from the Infinity Cache (256 MB) as long as it holds most of them, then from memory; MB of them in all: 1024 tokens, 325 376 / 351, 398 460 / 453, 514
-// 586 / 627; 2048, 315 541 / 498, 398 694 / 669, 503 861 / 931, 650 1105 / 1270; 4096, 336 943 / 903, 419 1196 / 1216, 629 1782 / 2038; 8192, 252 1245 / 1217, 336 1622 / 1625, 671 3421 / 3695.  Up
-// to 256 tokens half of a block of 256 is empty or masked at any size (256, 640 MB 457 / 428).
-// 192 / 128 columns: six of 1000 59 / 53, 1 x 8000 331 / 311, 8 x 4000 (246 MB) 666 / 656, (410 MB) 1152 / 1181, 12000 636 / 678; where two rounds are full, blocks of 256 pair long and short
-// ones exactly: 8 heads, 2 x 8000 383 / 424, 8 x 2000 131 / 138 (128 columns 333 / 332, 109 / 108).
+// Causal, the longest blocks first.  128 columns, 20 heads: 280 tokens 19.9 / 14.7, 777 36 / 28, 4096 134 / 124, 8192 412 / 396, 12000 857 / 852, 32768 5536 / 6052.
+// Keys and values of all heads come from the Infinity Cache (256 MB) as long as it holds most of them, then from memory; MiB of them in all: 1024 tokens, 220 247 / 237, 280 312 / 316, 320 356 / 369;
+// 2048, 240 423 / 389, 280 473 / 458, 320 546 / 544, 400 690 / 720; 4096, 240 685 / 656, 280 800 / 792, 320 894 / 910; 8192, 160 772 / 761, 240 1217 / 1237, 320 1576 / 1621.  (Another card
+// gained up to 30 % more of them: 1024, 310 MiB 376 / 351; 2048, 380 694 / 669.)  192 / 128 columns, 2048 tokens, 250 MiB 429 / 391, 300 514 / 498, 350 595 / 591, but 8192, 100 523 / 514, 120
+// 596 / 603, 180 924 / 938, 240 1179 / 1218, 300 1530 / 1617.
+// Up to 256 tokens half of a block of 256 is empty or masked at any size (256, 640 MB 457 / 428).
+// About two rounds of blocks of 256 pair long and short ones nearly exactly.  Blocks of 256, 192 / 128 columns: 384 328 / 316 (8192 tokens), 98 / 98 (2048), 400 204 / 219 (5000), 420 225 / 244 (5376),
+// 480 280 / 315 (6144), 120 / 127 (2048), 100 / 104 (1536), 81 / 81 (1024), 512 377 / 428 (8192), 125 / 133 (2048), 560 381 / 400 (7000), 600 476 / 464 (7500), 136 / 128 (1536).  128 columns:
+// 400 164 / 165 (5000), 420 180 / 184 (5376), 440 194 / 204 (5632), 448 97 / 93 (2048), 480 228 / 241 (6144), 98 / 99 (2048), 512 304 / 327 (8192), 164 / 177 (4096), 99 / 94 (1900), 528
+// 234 / 242 (5632), 544 119 / 109 (2048), 560 309 / 306 (7000).
 // 64 columns gain at every length and size (30 000 3172 / 2783; 1.3 GB 9146 / 9309 the worst).
 bool half_blocks_causal(int64_t S, double blocks, double kv_bytes, int64_t qd) {
     if (qd == 64 || S <= 256) return true;
-    return S <= 8192 && kv_bytes <= 384.0 * (1 << 20) && !(qd == 192 && blocks > 448 && blocks <= 512);
+    const bool long_blocks = S > 4096, wide = qd == 192;
+    const bool two_rounds = wide         ? S >= 1536 && blocks > 392 && blocks <= 576
+                            : long_blocks ? blocks > 408 && blocks <= 536
+                                          : S >= 2048 && blocks > 448 && blocks <= 512;
+    return S <= 8192 && kv_bytes <= (wide && long_blocks ? 112.0 : 288.0) * (1 << 20) && !two_rounds;
 }
 
 // Not causal every block is as long as the keys, so the rounds decide: 256 blocks of 256 or 512 of 128, which take 4 % longer, at a time, and a last round of one block of 128 a CU 0.7 of a whole

@@ -1292,6 +1292,15 @@ def case_attention_block_rule(dev, causal, B, S, Skv, H, waves):
     assert hip.get_lib().cdll.aria_last_attn_fwd_waves() == waves
 
 
+def case_attention_varlen_block_rule(dev, n, S, H, qd, waves):
+    """... and what packed sequences of 128 value columns take"""
+    from aria_amd import hip, ops
+
+    x, cu = rnd(n * S, H * qd, seed=3).to(dev), (torch.arange(n + 1, dtype=torch.int32) * S).to(dev)
+    ops.attention_varlen(x, x, x, cu, S, H, qd, 128, qd ** -0.5)
+    assert hip.get_lib().cdll.aria_last_attn_fwd_waves() == waves
+
+
 def case_attention_bwd_rope(dev, B, S, H, causal, use_len, s_rope=None):
     """r05: ``aria_attn_bwd_rope`` -- the inverse half-split RoPE of dq / dk (the chain rule through apply_rotary_pos_emb,
     modeling_llama.py:130-160) in the attention backward's register epilogues -- gives the bits of ``aria_attn_bwd`` followed by the in-place

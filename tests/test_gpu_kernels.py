@@ -139,11 +139,16 @@ def test_attention_varlen_waves(monkeypatch, lens, qd, vd):
     C.case_attention_varlen_waves(DEV, monkeypatch, lens, qd, vd)
 
 
-@pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 8, 2048, 2048, 20, 4), (True, 24, 2048, 2048, 20, 8), (True, 200, 256, 256, 20, 4), (True, 1, 8192, 8192, 4, 4), (True, 1, 8193, 8193, 4, 8),
+@pytest.mark.parametrize("causal,B,S,Skv,H,waves", [(True, 8, 2048, 2048, 20, 4), (True, 24, 2048, 2048, 20, 8), (True, 200, 256, 256, 20, 4), (True, 1, 8192, 8192, 4, 4), (True, 1, 8193, 8193, 4, 8), (True, 1, 6144, 6144, 20, 8), (True, 1, 4096, 4096, 20, 4),
                                                       (False, 1, 2048, 2048, 16, 4), (False, 1, 2048, 2048, 20, 8), (False, 2, 2048, 2048, 20, 4), (False, 1, 4096, 4096, 16, 8), (False, 16, 128, 4900, 20, 4),
                                                       (False, 1, 4097, 600, 2, 8), (False, 16, 256, 256, 32, 4)])
 def test_attention_block_rule(causal, B, S, Skv, H, waves):
     C.case_attention_block_rule(DEV, causal, B, S, Skv, H, waves)
+
+
+@pytest.mark.parametrize("n,S,H,qd,waves", [(1, 5376, 20, 192, 8), (1, 4096, 20, 192, 4), (3, 2048, 20, 192, 8), (2, 2048, 20, 192, 4), (1, 8192, 12, 192, 4), (2, 8192, 12, 192, 8), (3, 2048, 20, 128, 8), (3, 1900, 20, 128, 4)])
+def test_attention_varlen_block_rule(n, S, H, qd, waves):
+    C.case_attention_varlen_block_rule(DEV, n, S, H, qd, waves)
 
 
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
