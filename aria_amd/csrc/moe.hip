@@ -359,8 +359,9 @@ __global__ __launch_bounds__(1024) void sort_small_kernel(const int32_t* idx, co
 }
 
 // Group-limited routing and sort of a few tokens as one launch of one workgroup (a wave per token in turn): what route_groups_kernel and sort_small_kernel do, whose launches
-// are most of their time -- 4 tokens of 2 from 16 experts: 4.7 (cleared counts) + 4.6 + 4.6 us, 5.0 here.
-constexpr int ROUTE_SORT_T = 64, ROUTE_SORT_M = 1024;
+// are most of their time -- 4 tokens of 2 from 16 experts: 4.7 (cleared counts) + 4.6 + 4.6 us, 5.0 here.  The sixteen waves take more tokens in turns; three launches / one, us, 2 of 16, 4 of 32
+// and 6 of 64 experts: 32 tokens 10.0 / 7.1, 14.7 / 10.1, 15.5 / 12.1; 48 9.8 / 9.6, 14.4 / 13.6, 15.6 / 16.2; 64 10.2 / 11.9, 14.6 / 16.6, 15.5 / 20.4.
+constexpr int ROUTE_SORT_T = 48, ROUTE_SORT_M = 1024;
 __global__ __launch_bounds__(1024) void route_sort_kernel(const float* logits, const float* correction, float* weights, int32_t* indices, int32_t* offsets, int32_t* sorted_src,
                                                           int32_t* inv, int T, int E, int ldl, int groups, int keep, int k) {
     ARIA_SMEM_STATIC float lds[16][768];

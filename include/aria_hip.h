@@ -612,7 +612,7 @@ int aria_latent_decode(const AriaLatentStack* stack, const AriaLatentLayer* laye
                        int64_t max_len, float* logits, void* scratch, int64_t scratch_bytes, void* stream);
 /* One float32 step (every tensor of the stack in 32-bit) of any batch: T packed tokens of any sequences, their keys in the caches by position.  wanted: the W rows
  * whose logits are asked for, in order (int32 on the device); W < 0: every row.  The results are those of the step run sublayer by sublayer, bit for bit; the launches are fewer:
- * activations and the stream's steps are the products' epilogues, rows are gathered where they are read, up to 64 tokens are routed and sorted in one.  logits fp32 [W or T, V]. */
+ * activations and the stream's steps are the products' epilogues, rows are gathered where they are read, up to 48 tokens are routed and sorted in one.  logits fp32 [W or T, V]. */
 int64_t aria_latent_step_f32_scratch(const AriaLatentStack* stack, const AriaLatentLayer* layers, int64_t T, int64_t max_len, int64_t W);
 int aria_latent_step_f32(const AriaLatentStack* stack, const AriaLatentLayer* layers, int64_t T, const int32_t* ids, const int32_t* slot, const int32_t* pos,
                          int64_t max_len, const int32_t* wanted, int64_t W, float* logits, void* scratch, int64_t scratch_bytes, void* stream);

@@ -728,7 +728,7 @@ def case_latent_cache_rows(dev, dtype, H, R, dr):
 WIDE_STEPS = {
     # squared relu, gate times up gathered by expert, the stream's step; on every tile shape between 300 and 1632 tokens
     "layers": (config([(mixer(heads=8, dim=64, rot_dim=32, vdim=128, kv_rank=250), dense(ff=2824)), (mixer(heads=8, dim=64, rot_dim=32, vdim=120, kv_rank=256), moe(ff=768, experts=16, top=2)),
-                       (mixer(heads=4, dim=64, rot_dim=32, vdim=128, kv_rank=256), moe(ff=776, experts=16, top=2))], width=1024, vocab=8197), (50, 300, 620, 883, 1088, 1300, 1632)),
+                       (mixer(heads=4, dim=64, rot_dim=32, vdim=128, kv_rank=256), moe(ff=776, experts=16, top=2))], width=1024, vocab=8197), (48, 49, 300, 620, 883, 1088, 1300, 1632)),
     # the same at sizes for the emulator
     "ends": (config([(mixer(heads=2, dim=16, rot_dim=8, vdim=16, kv_rank=32), dense(ff=2077)), (mixer(heads=1, dim=8, rot_dim=2, vdim=24, kv_rank=20), moe(ff=1037, experts=4, top=2, count=2,
                                                                                                                                                      keep=1))], width=24, vocab=4105), (260,)),
