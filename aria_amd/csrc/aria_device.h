@@ -116,6 +116,14 @@ __device__ __forceinline__ float wave_sum_bcast(float v) {  // (the hardware for
     for (int m = 32; m >= 1; m >>= 1) v += emu::shfl(v, emu::lane() ^ m);
     return v;
 }
+__device__ __forceinline__ uint32_t upper_half_from(uint32_t own, uint32_t other) {
+    const uint32_t v = emu::shfl(other, emu::lane() ^ 8);
+    return emu::lane() & 8 ? v : own;
+}
+__device__ __forceinline__ uint32_t lower_half_from(uint32_t own, uint32_t other) {
+    const uint32_t v = emu::shfl(other, emu::lane() ^ 8);
+    return emu::lane() & 8 ? own : v;
+}
 __device__ __forceinline__ unsigned long long ballot(bool p) { return emu::ballot(p); }
 __device__ __forceinline__ int lane_id() { return emu::lane(); }
 __device__ __forceinline__ int first_lane(int v) { return emu::shfl(v, __builtin_ctzll(emu::ballot(true))); }
@@ -133,6 +141,13 @@ __device__ __forceinline__ T shfl_xor(T v, int mask) { return __shfl_xor(v, mask
 // (profiles/r02_gemm_tile_timeline.md)
 __device__ __forceinline__ float xor1(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
+}
+// `own`, but the upper (lower) eight lanes of every row of sixteen hold `other` of the lane eight below (above): one DPP move (row_ror:8, two of the row's four banks)
+__device__ __forceinline__ uint32_t upper_half_from(uint32_t own, uint32_t other) {
+    return uint32_t(__builtin_amdgcn_update_dpp(int(own), int(other), 0x128, 0xF, 0xC, false));
+}
+__device__ __forceinline__ uint32_t lower_half_from(uint32_t own, uint32_t other) {
+    return uint32_t(__builtin_amdgcn_update_dpp(int(own), int(other), 0x128, 0xF, 0x3, false));
 }
 // inclusive prefix sum over the wave's 64 lanes on the vector ALU: four DPP row shifts (scan inside each row of 16) and the two row
 // broadcasts of gfx9 (lane 15 -> next row, lane 31 -> rows 2, 3) -- 6 adds instead of 6 ds_bpermute round trips through the LDS

@@ -81,7 +81,7 @@ namespace {
 // e(value, up value, entry, row).  The row groups of all experts in use are one sequence, cut into equal pieces for the workgroups: how many experts are in
 // use is known on the device only, and a grid over (expert, rows) left the last round of workgroups nearly empty (29 experts x 18 pieces = 522 on
 // 512 places: 110 us; as one sequence 93).
-template <int NW, int KS, class Ep, bool PAIR>
+template <int NW, int KS, class Ep, bool PAIR, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void expert_rows_kernel(ExpertIn in, ExpertLists lists, Ep e) {
     ARIA_SMEM_STATIC RowsRed<NW, 1> red;
     ARIA_SMEM_STATIC int entries[16];
@@ -95,13 +95,13 @@ __global__ __launch_bounds__(NW * 64) void expert_rows_kernel(ExpertIn in, Exper
         const int id = lists.table[1 + a];
         const bool all = id >= in.E;
         const long long at = all ? (id - in.E) * in.s_step : (long long)id * in.N * in.K, ldw = all ? in.s_ld : (long long)in.K;
-        const bf16_t* W = (PAIR && c16 >= 8 ? (all ? in.S2 : in.W2) : (all ? in.S : in.W)) + at;
+        const bf16_t *W = (all ? in.S : in.W) + at, *W2 = PAIR ? (all ? in.S2 : in.W2) + at : W;
         for (int t0 = 0; t0 < m; t0 += 16) {   // (more than 16 only where tokens chose an expert several times: NaN logits)
             sync();                            // (red and entries of the piece before are read)
             const int mine = lists.list[first + min(t0 + c16, m - 1)];
             if (t < 16) entries[t] = mine;     // (published by the first group's barrier)
-            stream_rows<NW, KS, 1>(
-                in.K, [&](int gg) { return W + (long long)min(gg * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * ldw; },
+            stream_rows<NW, KS, 1, ONCE>(
+                in.K, [&](int gg, int r) { return (PAIR && r >= 8 ? W2 : W) + (long long)min(gg * OUT + (PAIR ? r & 7 : r), in.N - 1) * ldw; },
                 [&](int) { return in.X + (long long)(mine / in.div) * in.ldx; }, g0, g1, red, [&](float v, int tok, int n, int gg) {
                     const float u = PAIR ? shfl_xor(v, 8) : 0.f;
                     if (t0 + tok < m && gg * OUT + n < in.N && n < OUT) e(v, u, entries[tok], gg * OUT + n);
@@ -129,7 +129,14 @@ template <bool PAIR, class Ep>
 int launch_expert_rows(const ExpertIn& in, const ExpertLists& lists, int64_t k, int64_t T, const Ep& e, void* stream) {
     const int64_t most = (in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16) * std::min<int64_t>(lists.E, T * k);
     const dim3 grid(unsigned(std::min<int64_t>(512, most)));   // two workgroups a CU are resident
-#define ARIA_ROWS(NW, KS) ARIA_LAUNCH((expert_rows_kernel<NW, KS, Ep, PAIR>), grid, dim3(NW * 64), 0, stream, in, lists, e);
+    const bool once = in.K % 64 == 0 && in.s_ld % 64 == 0;   // (lines that do not straddle rows: rows_once)
+#define ARIA_ROWS(NW, KS)                                                                                                 \
+    {                                                                                                                     \
+        if (once)                                                                                                         \
+            ARIA_LAUNCH((expert_rows_kernel<NW, KS, Ep, PAIR, true>), grid, dim3(NW * 64), 0, stream, in, lists, e);      \
+        else                                                                                                              \
+            ARIA_LAUNCH((expert_rows_kernel<NW, KS, Ep, PAIR, false>), grid, dim3(NW * 64), 0, stream, in, lists, e);     \
+    }
     ARIA_ROWS_SHAPE(in.K, ARIA_ROWS, return ARIA_ERR_UNSUPPORTED;)
 #undef ARIA_ROWS
     return aria_check_launch();

@@ -6,6 +6,7 @@
 #pragma once
 #include "elem.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace ad {
 
@@ -100,56 +101,105 @@ __global__ __launch_bounds__(256) void row_kernel(RowsPair rp, E e) {
 // at the price of one.  Wave w owns the KS 32-column steps of the reduction that start at column 32 KS w: its part of the tokens is loaded ONCE and stays
 // in registers, and a weight fragment's register is refilled with the next group's as soon as it is used, so up to 16 kilobytes a wave are in flight
 // without a break between the groups.  The NW partial results meet in LDS (two images in turn: one barrier a group), where whole waves sum them and call
-// out(value, token, column of the group, group).  wrow(g): this lane's weight row of group g, xrow(i): its token row of tile i; both from column 0.
-// (Plain loads: a fragment touches half a cache line of 16 rows and the next one the other half, which a non-temporal hint fetches twice.)
+// out(value, token, column of the group, group).  wrow(g, r): row r of group g, xrow(i): this lane's token row of tile i; both from column 0.
+//
+// A load takes eight rows' whole cache lines (64 columns), the next one the other eight rows'; the two fragments of 16 rows and 32 columns are these with their halves
+// exchanged between the lanes of a row (whole_lines).  So the weights, which are read once, can be non-temporal: a fragment loaded as it is wanted touches half a line of 16 rows,
+// and the hint then fetches every line twice.  Reading 500 MB: half lines 87 us, non-temporal 104, whole lines 86, non-temporal 77 (6.8 TB/s); 34 MB 8.3, 10.4, 7.9, 7.4.
+// A step left over (KS odd) is a half line that another wave shares: a plain load.  !ONCE: half lines, plain (rows_once).
 template <int NW, int MT>
 struct RowsRed {
     float v[2][NW][16 * MT][17];
 };
-template <int NW, int KS, int MT, class WRow, class XRow, class Out>
+// rows 0 .. 7 and 8 .. 15 of 64 columns, lane (c, q) with row c & 7, chunk q + 4 (c >> 3) -> the fragments of columns 0 .. 31 and 32 .. 63, lane (c, q) with row c, chunk q
+__device__ __forceinline__ void whole_lines(const u32x4& a, const u32x4& b, s16x8& lo, s16x8& hi) {
+    u32x4 x, y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = upper_half_from(a[i], b[i]), y[i] = lower_half_from(b[i], a[i]);
+    lo = __builtin_bit_cast(s16x8, x);
+    hi = __builtin_bit_cast(s16x8, y);
+}
+template <int NW, int KS, int MT, bool ONCE, class WRow, class XRow, class Out>
 __device__ __forceinline__ void stream_rows(int K, const WRow& wrow, const XRow& xrow, int g0, int g1, RowsRed<NW, MT>& red, const Out& out) {
-    constexpr int DEPTH = KS <= 16 ? KS : KS / 2;   // fragments in flight
+    constexpr int P = KS / 2;                                          // ONCE: pairs of steps, and a left-over one where KS is odd
+    constexpr int SLOTS = ONCE ? KS <= 16 ? P : (P + 1) / 2 : 1;       // pairs in flight: pair p in slot p % SLOTS, in two turns at most
+    constexpr int DEPTH = ONCE ? 1 : KS <= 16 ? KS : KS / 2;           // else: fragments in flight
+    static_assert(2 * SLOTS >= P || !ONCE, "two turns");
     static_assert(KS % DEPTH == 0, "a step keeps its register");
     const int t = threadIdx.x, l = t & 63, w = t >> 6, q4 = l >> 4, c16 = l & 15;
     // the last waves' windows are moved down into the row, the columns that another wave owns zeroed in the tokens: every address is base + constant
-    const int own = w * KS * 32, k0 = min(own, K - KS * 32) + q4 * 8;
-    u32x4 x[MT][KS], b[DEPTH];
-    const bf16_t* wp = wrow(g0) + k0;
+    const int own = w * KS * 32, start = min(own, K - KS * 32);
+    // the column of x[][u]: in order, but the left-over step last, which is the window's first where that begins in the middle of a line
+    const int odd = ONCE && KS % 2 ? first_lane(start >> 5 & 1) : 0;
+    auto column = [&](int u) __attribute__((always_inline)) { return start + 32 * (ONCE && KS % 2 && u == KS - 1 ? odd ? 0 : KS - 1 : u + odd); };
+    const int row = c16 & 7, line = column(0) + (q4 + 4 * (c16 >> 3)) * 8;
+    u32x4 x[MT][KS], a[SLOTS], b[SLOTS], f[DEPTH];   // f[0] of ONCE: the left-over step
+    const bf16_t *wa = wrow(g0, ONCE ? row : c16), *wb = ONCE ? wrow(g0, row + 8) : wa, *wf = wrow(g0, c16);
+    if constexpr (ONCE) {
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) b[u] = ld16(wp + 32 * u);
+        for (int p = 0; p < SLOTS; ++p) a[p] = ldw16(wa + line + 64 * p), b[p] = ldw16(wb + line + 64 * p);
+        if (KS % 2) f[0] = ld16(wf + column(KS - 1) + q4 * 8);
+    } else {
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) f[u] = ld16(wf + column(u) + q4 * 8);
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-        const bf16_t* xp = xrow(i) + k0;
+        const bf16_t* xp = xrow(i) + q4 * 8;
 #pragma unroll
-        for (int u = 0; u < KS; ++u) x[i][u] = ld16(xp + 32 * u);
+        for (int u = 0; u < KS; ++u) x[i][u] = ld16(xp + column(u));
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int u = 0; u < KS; ++u)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) x[i][u][q] = k0 + 32 * u >= own ? x[i][u][q] : 0u;
+            for (int q = 0; q < 4; ++q) x[i][u][q] = column(u) + q4 * 8 >= own ? x[i][u][q] : 0u;
     for (int g = g0; g < g1; ++g) {
         const int ph = (g - g0) & 1;
         f32x4 acc[MT];   // (one chain a tile whatever MT is: a token's sums do not depend on how many tokens there are)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const bf16_t* cur = wp;
+        auto step = [&](int u, const s16x8& v) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i] = mfma16(__builtin_bit_cast(s16x8, x[i][u]), v, acc[i]);
+        };
+        // the group's steps; its registers are refilled with its own later steps and (`on`) the next group's
+        auto steps = [&](auto on_, const bf16_t* na, const bf16_t* nb, const bf16_t* nf) __attribute__((always_inline)) {
+            constexpr bool on = decltype(on_)::value;
+            if constexpr (ONCE) {   // (the steps in the row's order in either form: the same bits)
+                if (KS % 2 && odd) step(KS - 1, __builtin_bit_cast(s16x8, f[0]));
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    const int s = p % SLOTS;
+                    s16x8 lo, hi;
+                    whole_lines(a[s], b[s], lo, hi);
+                    step(2 * p, lo);
+                    step(2 * p + 1, hi);
+                    if (p + SLOTS < P)
+                        a[s] = ldw16(wa + line + 64 * (p + SLOTS)), b[s] = ldw16(wb + line + 64 * (p + SLOTS));
+                    else if (on)
+                        a[s] = ldw16(na + line + 64 * s), b[s] = ldw16(nb + line + 64 * s);
+                }
+                if (KS % 2 && !odd) step(KS - 1, __builtin_bit_cast(s16x8, f[0]));
+                if (KS % 2 && on) f[0] = ld16(nf + column(KS - 1) + q4 * 8);
+            } else {
+#pragma unroll
+                for (int u = 0; u < KS; ++u) {
+                    step(u, __builtin_bit_cast(s16x8, f[u % DEPTH]));
+                    if (u + DEPTH < KS)
+                        f[u % DEPTH] = ld16(wf + column(u + DEPTH) + q4 * 8);
+                    else if (on)
+                        f[u % DEPTH] = ld16(nf + column(u + DEPTH - KS) + q4 * 8);
+                }
+            }
+        };
         if (g + 1 < g1) {
-            wp = wrow(g + 1) + k0;
-#pragma unroll
-            for (int u = 0; u < KS; ++u) {
-#pragma unroll
-                for (int i = 0; i < MT; ++i) acc[i] = mfma16(__builtin_bit_cast(s16x8, x[i][u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[i]);
-                b[u % DEPTH] = ld16(u + DEPTH < KS ? cur + 32 * (u + DEPTH) : wp + 32 * (u + DEPTH - KS));
-            }
+            const bf16_t *na = wrow(g + 1, ONCE ? row : c16), *nb = ONCE ? wrow(g + 1, row + 8) : na, *nf = wrow(g + 1, c16);
+            steps(std::true_type{}, na, nb, nf);
+            wa = na, wb = nb, wf = nf;
         } else {
-#pragma unroll
-            for (int u = 0; u < KS; ++u) {
-#pragma unroll
-                for (int i = 0; i < MT; ++i) acc[i] = mfma16(__builtin_bit_cast(s16x8, x[i][u]), __builtin_bit_cast(s16x8, b[u % DEPTH]), acc[i]);
-                if (u + DEPTH < KS) b[u % DEPTH] = ld16(cur + 32 * (u + DEPTH));
-            }
+            steps(std::false_type{}, wa, wb, wf);
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -177,7 +227,7 @@ __device__ __forceinline__ void token_rms(float* rms, const RowsIn& in, int t0, 
     }
 }
 // PAIR: a group is 8 gate rows and the 8 up rows of the same outputs
-template <int NW, int KS, int MT, class E, bool PAIR>
+template <int NW, int KS, int MT, class E, bool PAIR, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, int per, E e) {
     ARIA_SMEM_STATIC RowsRed<NW, MT> red;
     ARIA_SMEM_STATIC float rms[16];
@@ -186,9 +236,8 @@ __global__ __launch_bounds__(NW * 64) void rows_kernel(RowsPair rp, int n_tok, i
     const int c16 = threadIdx.x & 15, t0 = blockIdx.y * 16 * MT, groups = (in.N + OUT - 1) / OUT, g0 = blockIdx.x * per;
     if (g0 >= groups) return;
     if (MT == 1 && in.sq) token_rms(rms, in, t0, n_tok, NW);   // (published by the first group's barrier)
-    const bf16_t* W = PAIR && c16 >= 8 ? in.W2 : in.W;
-    stream_rows<NW, KS, MT>(
-        in.K, [&](int g) { return W + (long long)min(g * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * in.K; },
+    stream_rows<NW, KS, MT, ONCE>(
+        in.K, [&](int g, int r) { return (PAIR && r >= 8 ? in.W2 : in.W) + (long long)min(g * OUT + (PAIR ? r & 7 : r), in.N - 1) * in.K; },
         [&](int i) { return in.X + (long long)min(t0 + 16 * i + c16, n_tok - 1) * in.ldx; }, g0, min(groups, g0 + per), red,
         [&](float v, int tok, int n, int g) {
             const float u = PAIR ? shfl_xor(v, 8) : 0.f;
@@ -280,6 +329,11 @@ __global__ __launch_bounds__(512) void rows_long_kernel(RowsPair rp, int n_tok, 
 // workgroups of one problem, i.e. the partial sums per token that an epilogue with SUMSQ leaves
 inline int rows_parts(int64_t T, int64_t N) { return int(T == 1 ? (N + 7) / 8 : (N + 15) / 16); }
 
+// Whether weights [N, K] that `passes` rows of workgroups go through come by whole lines, non-temporal (stream_rows): read once, lines that do not straddle rows, and enough of them.
+// Us, half lines / whole: 100352 x 2560 at 2, 16, 64 tokens 93 / 82, 103 / 85, 123 / 117; 32000 x 1024 14.0 / 12.9 (2 tokens); 2560 x 2560 5.7 / 5.5; gate and up of 3328 x 2560 at 40 tokens
+// 15.8 / 14.9.  In several passes (found in the L2): 7680 x 2560, 280 tokens, 37.4 / 38.8.  1024 x 1024, 64 x 2560: 3.15 / 3.26, 4.8 / 4.9; 1000 x 1000 2.7 / 3.4.
+inline bool rows_once(int64_t passes, int64_t N, int64_t K) { return passes == 1 && K % 64 == 0 && N * K >= (3 << 20); }
+
 // Row groups per workgroup: one round of the 256 CUs.  More workgroups read the tokens more often (7680 x 2560, 16 tokens: 240 workgroups 10.4 us, 480
 // 13.1), fewer leave CUs idle (4448 rows: two groups each on 139 workgroups 9.5 us, one each on 278 -- a second, nearly empty round -- 12.1).
 inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std::max<int64_t>(1, (groups * problems + 255) / 256)); }
@@ -294,6 +348,8 @@ inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std
         OTHER                           \
     else if ((K) <= 1024)               \
         CALL(8, 4)                      \
+    else if ((K) <= 1536)               \
+        CALL(8, 6)                      \
     else if ((K) <= 1792)               \
         CALL(8, 7)                      \
     else if ((K) <= 2560)               \
@@ -330,26 +386,35 @@ int launch_rows_wide(const RowsIn& in, int64_t T, const E& e, void* stream) {
     const int per = int((groups + most - 1) / most);
     const int64_t tx = (groups + per - 1) / per;
     const dim3 grid(unsigned(ty == 1 ? tx : (tx + 7) / 8 * 8), unsigned(ty));
-#define ARIA_WIDE(KS, MT) ARIA_LAUNCH((rows_kernel<8, KS, MT, E, PAIR>), grid, dim3(512), 0, stream, rp, int(T), per, e)
+#define ARIA_WIDE(KS, MT)                                                                                            \
+    if (once)                                                                                                        \
+        ARIA_LAUNCH((rows_kernel<8, KS, MT, E, PAIR, true>), grid, dim3(512), 0, stream, rp, int(T), per, e);        \
+    else                                                                                                             \
+        ARIA_LAUNCH((rows_kernel<8, KS, MT, E, PAIR, false>), grid, dim3(512), 0, stream, rp, int(T), per, e)
 #define ARIA_WIDE_TILES(KS)  \
-    if (mt == 1)             \
+    if (mt == 1) {           \
         ARIA_WIDE(KS, 1);    \
-    else if (mt == 2)        \
+    } else if (mt == 2) {    \
         ARIA_WIDE(KS, 2);    \
-    else                     \
-        ARIA_WIDE(KS, 4)
+    } else {                 \
+        ARIA_WIDE(KS, 4);    \
+    }
     if (in.K < 128 || in.K > 4096) return ARIA_ERR_UNSUPPORTED;
+    const bool once = rows_once(ty, in.N * (PAIR ? 2 : 1), in.K);
     if (in.K <= 1024) {
         ARIA_WIDE_TILES(4);
+    } else if (in.K <= 1536) {
+        ARIA_WIDE_TILES(6);
     } else if (in.K <= 1792) {
         ARIA_WIDE_TILES(7);
     } else if (in.K <= 2560) {
         ARIA_WIDE_TILES(10);
     } else if (in.K <= 3328) {
-        if (mt == 1)
+        if (mt == 1) {
             ARIA_WIDE(13, 1);
-        else
+        } else {
             ARIA_WIDE(13, 2);
+        }
     } else if (mt == 1) {
         ARIA_WIDE(16, 1);
     } else {
@@ -366,13 +431,16 @@ int launch_rows_of(const RowsPair& rp, int problems, int64_t T, const E& e, void
     const int per = rows_per_workgroup(groups, problems), other = rp.in[problems - 1].K;
     const int K = std::max(rp.in[0].K, other), least = std::min(rp.in[0].K, other);
     const dim3 grid(unsigned((groups + per - 1) / per), unsigned((T + 15) / 16), unsigned(problems));
+    const bool once = rows_once(grid.y, rp.in[0].N * problems, rp.in[0].K) && other % 64 == 0;
 #define ARIA_ROWS_LONG ARIA_LAUNCH((rows_long_kernel<E, PAIR>), dim3(unsigned(long_groups), grid.y, grid.z), dim3(512), 0, stream, rp, int(T), e);
 #define ARIA_ROWS(NW, KS)                                                                                                     \
     {                                                                                                                         \
-        if (least >= KS * 32) /* (a wave's window lies inside the shorter reduction too) */                                   \
-            ARIA_LAUNCH((rows_kernel<NW, KS, 1, E, PAIR>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);                  \
-        else                                                                                                                  \
+        if (least < KS * 32) /* (a wave's window would end beyond the shorter reduction) */                                   \
             ARIA_ROWS_LONG                                                                                                    \
+        else if (once)                                                                                                        \
+            ARIA_LAUNCH((rows_kernel<NW, KS, 1, E, PAIR, true>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);         \
+        else                                                                                                                  \
+            ARIA_LAUNCH((rows_kernel<NW, KS, 1, E, PAIR, false>), grid, dim3(NW * 64), 0, stream, rp, int(T), per, e);        \
     }
     ARIA_ROWS_SHAPE(K, ARIA_ROWS, ARIA_ROWS_LONG)
 #undef ARIA_ROWS

@@ -5,11 +5,9 @@
 // up to 64 tokens at a time past the weights; further tokens find the weights in the L2 / MALL.  Weights from HBM, us as tiles / here: 64 tokens: q | k | v
 // 29 / 17, gate and up with SwiGLU (2 x 3328) 48 / 18, 2560 x 2560 27 / 13; 280: 44 / 37, 49 / 39, 30 / 21; 352: 45 / 44, 52 / 40, 30 / 21; 400: 46 / 54,
 // 57 / 48, 31 / 24; lm_head of one token 140 / 86.
-// Routed experts: with n tokens an expert's matrix meets n k / E rows (26 at 280 tokens, 6 of 64 experts); its rows are read once per 64 of them.  Up pairs
-// (64 experts of 2 x 1664 x 2560, several draws of preferred experts), tiles / here: 32 tokens 238 / 182, 128 260 / 225, 280 270 / 232 .. 245, 352 271 /
-// 235 .. 257, 400 272 / 254 .. 264, 480 273 / 276.  Smaller ones: 32 experts of 2 x 1024 x 1536, 4 a token: 64 tokens 47 / 44, 128 48 / 53, 216 49 / 55;
-// 16 of 2 x 768 x 1024, 2 a token: 64 tokens 26 / 14, 216 29 / 17.  Down (2560 x 1664): 32 tokens 103 / 97, from 64 tokens on the tiles are ahead
-// (104 / 134).
+// Routed experts: with n tokens an expert's matrix meets n k / E rows (26 at 280 tokens, 6 of 64 experts); its rows are read once per 64 of them, by whole lines that are non-temporal
+// (rows.h).  Up pairs (64 experts of 2 x 1664 x 2560), half lines / whole: 24 tokens 174 / 151, 64 204 / 172, 128 220 / 180, 280 238 / 193 (5.6 TB/s of weights); 32 of 2 x 1024 x 1536, 4 a
+// token: 64 tokens 43 / 34, 280 58 / 52.  Down (2560 x 1664): 24 tokens 93 / 77, 64 109 / 89, 280 130 / 116.  Which is ahead of the tiles where: ops.py.
 #include "rows.h"
 
 namespace {
@@ -83,7 +81,7 @@ __device__ __forceinline__ int count_tiles(const int32_t* offsets, int E, int* u
 // The weight row groups of all token tiles of all experts are one sequence, cut into equal pieces for the workgroups (experts.h): an expert with more rows than a
 // tile holds is further work in the sequence.  (As further work of the workgroups that own its weight rows it held up the launch: 64 experts of
 // 2 x 1664 x 2560, 280 tokens, 80 rows for the most popular one: 361 us, now 245; 55 rows 234 in both.)  e(value, up value, place, row)
-template <int KS, int MT, class Ep, bool PAIR>
+template <int KS, int MT, class Ep, bool PAIR, bool ONCE>
 __global__ __launch_bounds__(512) void sorted_rows_kernel(ExpertRows in, Ep e) {
     ARIA_SMEM_STATIC RowsRed<8, MT> red;
     ARIA_SMEM_STATIC int upto[256];
@@ -102,10 +100,10 @@ __global__ __launch_bounds__(512) void sorted_rows_kernel(ExpertRows in, Ep e) {
             if (behind) break;
         }
         const int first = in.offsets[id], m = in.offsets[id + 1] - first, t0 = (tile - (id ? upto[id - 1] : 0)) * ROWS;
-        const bf16_t* W = (PAIR && c16 >= 8 ? in.W2 : in.W) + (long long)id * in.N * in.K;
+        const long long at = (long long)id * in.N * in.K;
         sync();   // (the sums of the piece before are read)
-        stream_rows<8, KS, MT>(
-            in.K, [&](int gg) { return W + (long long)min(gg * OUT + (PAIR ? c16 & 7 : c16), in.N - 1) * in.K; },
+        stream_rows<8, KS, MT, ONCE>(
+            in.K, [&](int gg, int r) { return (PAIR && r >= 8 ? in.W2 : in.W) + at + (long long)min(gg * OUT + (PAIR ? r & 7 : r), in.N - 1) * in.K; },
             [&](int i) {
                 const int at = first + min(t0 + 16 * i + c16, m - 1);
                 return in.X + (long long)(in.rows ? in.rows[at] : at) * in.ldx;
@@ -132,16 +130,24 @@ int launch_sorted_rows(const ExpertRows& in, int64_t M, const Ep& e, void* strea
     const int64_t rows = (M + in.E - 1) / in.E, most = int64_t((in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16)) * std::min<int64_t>(in.E, M);
     const int mt = rows_tiles(in.K, 4 * rows);   // (loads differ: tiles for four times the average -- 280 tokens, 26 rows an expert on average, 63 at most)
     const dim3 grid(unsigned(std::min<int64_t>(mt > 2 ? 256 : 512, most)));
-#define ARIA_SORTED(KS, MT) ARIA_LAUNCH((sorted_rows_kernel<KS, MT, Ep, PAIR>), grid, dim3(512), 0, stream, in, e)
+    const bool once = in.K % 64 == 0;   // (lines that do not straddle rows: rows_once)
+#define ARIA_SORTED(KS, MT)                                                                                  \
+    if (once)                                                                                                \
+        ARIA_LAUNCH((sorted_rows_kernel<KS, MT, Ep, PAIR, true>), grid, dim3(512), 0, stream, in, e);        \
+    else                                                                                                     \
+        ARIA_LAUNCH((sorted_rows_kernel<KS, MT, Ep, PAIR, false>), grid, dim3(512), 0, stream, in, e)
 #define ARIA_SORTED_TILES(KS) \
-    if (mt == 1)              \
+    if (mt == 1) {            \
         ARIA_SORTED(KS, 1);   \
-    else if (mt == 2)         \
+    } else if (mt == 2) {     \
         ARIA_SORTED(KS, 2);   \
-    else                      \
-        ARIA_SORTED(KS, 4)
+    } else {                  \
+        ARIA_SORTED(KS, 4);   \
+    }
     if (in.K <= 1024) {
         ARIA_SORTED_TILES(4);
+    } else if (in.K <= 1536) {
+        ARIA_SORTED_TILES(6);
     } else if (in.K <= 1792) {
         ARIA_SORTED_TILES(7);
     } else {

@@ -108,6 +108,8 @@ CONFIGS = {
     # a head of more than 16384 rows, and a reduction of several rounds of the decode kernels' waves
     "vocabulary": config([lightning(heads=1, dim=8, vdim=8, decay=(0.9,), ff=24)], width=24, vocab=16411),
     "broad": config([parallel(ff=24)], width=2061, vocab=45),
+    # weights that arrive by whole lines in a decode step, the longest windows among them
+    "deep": config([lightning(heads=1, dim=8, vdim=8, decay=(0.9,), ff=4992)], width=768, vocab=40),
 }
 
 

@@ -442,6 +442,19 @@ def case_rows_experts_uneven(dev, counts, N, K):
     assert torch.equal(ops.rows_experts(*args, w_up=u), torch.cat([ops.rows_swiglu(t, a, b) for t, a, b in each]))
 
 
+def case_rows_whole_lines(dev, M, N, K):
+    """Weights that come by whole lines against their first rows by half lines (too few for whole ones): the same bits, and float64."""
+    from aria_amd import ops
+
+    x, w = (L.rnd(n, K, seed=i, scale=K ** -0.5 if i else 1.0) for i, n in enumerate((M, N)))
+    xd, wd = x.to(dev), w.to(dev)
+    assert N * K >= 3 << 20 > 48 * K and K % 64 == 0
+    got = ops.rows_gemm(xd, wd, f32)
+    assert L.rel(got, x.double() @ w.double().T) < 2e-6
+    for at in (0, N // 2, N - 48):
+        assert torch.equal(got[:, at:at + 48], ops.rows_gemm(xd, wd[at:at + 48].contiguous(), f32))
+
+
 # sixteen, 32 and 64 rows a tile
 UNEVEN = [[0] * 65 + [40, 0, 16, 1, 17], [33, 0, 1, 24, 0, 2, 0, 0, 4], [0, 65, 1, 129, 0, 64, 2]]
 

@@ -67,7 +67,7 @@ def test_linear_chunks_agree(kind, m, steep, defer, monkeypatch):
     C.case_linear_chunks_agree(DEV, kind, m, (150, 3), [0, 9], 1, steep)
 
 
-@pytest.mark.parametrize("dtype,name", [(bf16, "odd"), (f32, "odd"), (f32, "mixed"), (bf16, "ones"), (bf16, "steep"), (bf16, "huge"), (bf16, "vocabulary")])
+@pytest.mark.parametrize("dtype,name", [(bf16, "odd"), (f32, "odd"), (f32, "mixed"), (bf16, "ones"), (bf16, "steep"), (bf16, "huge"), (bf16, "vocabulary"), (bf16, "deep")])
 def test_model(dtype, name):
     C.case_model(DEV, dtype, name, lens=(4, 1, 2), tail=2)
 

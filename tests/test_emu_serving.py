@@ -70,6 +70,10 @@ def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)
 
 
+def test_rows_whole_lines():
+    C.case_rows_whole_lines(DEV, 2, 1894, 1664)
+
+
 @pytest.mark.parametrize("counts", C.UNEVEN)
 def test_rows_experts_uneven(counts):
     C.case_rows_experts_uneven(DEV, counts, 20, 136)

@@ -80,6 +80,12 @@ def test_rows_products(M, N, K):
     C.case_rows_products(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 3072, 1024), (16, 2050, 1536), (64, 2049, 1536), (33, 1900, 1664), (17, 1777, 1792), (16, 2000, 1728), (64, 1300, 2496), (9, 100352, 2560), (20, 1000, 3328),
+                                   (16, 990, 3264), (30, 800, 4096)])
+def test_rows_whole_lines(M, N, K):
+    C.case_rows_whole_lines(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("N,K", [(33, 1024), (1664, 2560), (24, 1672)])
 @pytest.mark.parametrize("counts", C.UNEVEN)
 def test_rows_experts_uneven(counts, N, K):
