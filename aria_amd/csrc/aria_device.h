@@ -350,6 +350,15 @@ __device__ __forceinline__ void glds16(const void* g, void* lds_wave_base) {
                                      (__attribute__((address_space(3))) void*)(lds_wave_base), 16, 0, 0);
 #endif
 }
+// glds16 of bytes that nobody reads again: non-temporal
+__device__ __forceinline__ void glds16_once(const void* g, void* lds_wave_base) {
+#ifdef ARIA_EMU
+    emu::glds(g, static_cast<char*>(lds_wave_base) + 16 * emu::lane());
+#else
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(g),
+                                     (__attribute__((address_space(3))) void*)(lds_wave_base), 16, 0, 2 /* nt */);
+#endif
+}
 // glds16 at agent scope (sc1): the source was written by another workgroup of the same launch, possibly on another XCD
 __device__ __forceinline__ void glds16_agent(const void* g, void* lds_wave_base) {
 #ifdef ARIA_EMU

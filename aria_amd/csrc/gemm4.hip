@@ -98,6 +98,7 @@ struct Shape4 {
     static constexpr size_t SMEM = std::max(size_t(S) * STAGE, size_t(BM) * ROWP);
 };
 
+// ONCE: B's pieces are non-temporal (which: aria_launch_gemm4)
 // VER: what happens to the tile (the numbers of gemm3_kernel): 3 plain (bias, activation, accumulation, 32-bit results), 5 SwiGLU backward, 6 / 9 fused SwiGLU on two
 // weight tensors (9: gathered rows), 8 on [K, N] weights with gathered rows, 14 on one [gate | up] tensor, 13 relu gate, 7 the interleaved rotation,
 // 11 plain, with the reduction's rows of A reached through an index (per-expert weight gradients)
@@ -151,7 +152,7 @@ struct Tile4 {
     int slab, ks;
 };
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER>
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, bool ONCE = false>
 __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& place, char* smem) {
     using T = Shape4<WM, WN, MI, NI, KD, S>;
     constexpr int BM = T::BM, BN = T::BN, PA = T::PA, PB = T::PB, STAGE = T::STAGE, ROWP = T::ROWP, HALVES = KD / 16;
@@ -210,6 +211,8 @@ __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& pla
         constexpr int I = decltype(s)::value;
         if constexpr (I < PA)
             glds16(a + offA[I], d + 4096 * I);
+        else if constexpr (ONCE)
+            glds16_once(b + (I - PA >= PB / 2 ? up : 0) + offB[I - PA], d + 4096 * I);
         else
             glds16(b + (I - PA >= PB / 2 ? up : 0) + offB[I - PA], d + 4096 * I);
     };
@@ -445,7 +448,7 @@ __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& pla
     }
 }
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false>
 __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     constexpr int BM = Shape4<WM, WN, MI, NI, KD, S>::BM;
     ARIA_DYN_SMEM(smem);
@@ -471,7 +474,7 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
         expert = first_lane(expert), m0 = first_lane(m0), m_end = first_lane(m_end), tn = first_lane(tn);
         b_off = (long long)(p.expert_mod > 0 ? expert % p.expert_mod : expert) * p.strideB;
     }
-    gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER>(p, Tile4{tn, m0, m_end, k_begin, k_len, b_off, c_off, slab, ks}, smem);
+    gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, ONCE>(p, Tile4{tn, m0, m_end, k_begin, k_len, b_off, c_off, slab, ks}, smem);
 }
 
 // the sums of the slabs of gemm4_kernel<.., WM, WN, MI, NI, ..>: see gemm3_reduce_kernel; a block finishes 32 rows of 32 WN columns
@@ -557,7 +560,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(GemmParams p, int t
     }
 }
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU>
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false>
 int launch4(GemmParams q, int split, float* ws, void* stream) {
     using T = Shape4<WM, WN, MI, NI, KD, S>;
     constexpr int STEP = gated(VER) ? T::BN / 2 : T::BN;
@@ -568,7 +571,7 @@ int launch4(GemmParams q, int split, float* ws, void* stream) {
     q.ws = ws;
     if (q.ntn * q.ntm <= 0) return ARIA_OK;
     const unsigned grid = q.mode == 1 ? unsigned(q.ntn * q.ntm + 16) : unsigned(q.ntn * q.ntm * std::max(split, 1));
-    ARIA_LAUNCH((gemm4_kernel<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, PER_CU>), dim3(grid, q.mode == 2 ? unsigned(q.E) : 1u), dim3(256), T::SMEM, stream, q);
+    ARIA_LAUNCH((gemm4_kernel<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, PER_CU, ONCE>), dim3(grid, q.mode == 2 ? unsigned(q.E) : 1u), dim3(256), T::SMEM, stream, q);
     if (split > 1) ARIA_LAUNCH((gemm4_reduce_kernel<WM, WN, MI, NI>), dim3(unsigned(q.ntn * q.ntm), NI * MI * WM), dim3(256), 0, stream, q);
     return aria_check_launch();
 }
@@ -636,11 +639,12 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     if (p.mode == 1) {
         // Rows by expert.  Up to 100 a expert its tile of 256 rows is mostly empty and the weights' stream counts, of which three stages of 48 KiB keep more in flight.
         // 64 experts of 2560 x 1664, rows each on average 28 / 73 / 140, before and now: gate and up, gathered, [K, N] 254 -> 213, 276 -> 233, (306 -> 345); two [N, K]
-        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 114, 135 -> 124, (153 -> 155), at 6 rows (109 -> 111), [N, K] at 26 rows in a prompt (109 -> 114); SwiGLU backward 144 -> 121, 160 -> 149,
+        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 110, 135 -> 124, (153 -> 155), at 6 rows 111 -> 104,
+        // [N, K] at 2, 6, 15, 26 rows 101 -> 74, 107 -> 103, 112 -> 103, 119 -> 107; SwiGLU backward 144 -> 121, 160 -> 149,
         // (185 -> 200); gate and up backward [N, K] 214 -> 207, 245 -> 220.  And where all of it is one round: 16 experts of 1024 x 768, 187 rows each, 32.6 -> 20.2 and 25 -> 16.
         if (p.K < 768 || p.N < 512) return none;
         const long long cols = p.glu ? p.N / 2 : p.N, ntn = cdiv(cols, p.glu ? 128 : 256);
-        const bool few = p.M < 100ll * p.E && (!plain || p.M >= 40ll * p.E), one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
+        const bool few = p.M < 100ll * p.E, one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
         if (few || one_round) plan.form = 1;
         return plan;
     }
@@ -713,13 +717,20 @@ int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, f
     }
     if (plan.form == 2)
         return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
+    // Weights by expert that nearly all meet one tile of rows are read once, without a place in the caches (pieces that are non-temporal): a stream of 500 MB at 6.9 TB/s for 6.2.  64 experts of
+    // 2560 x 1664, us before and now, rows each on average 6, 26, 47, 73: gate and up, gathered, [K, N] 209 190, 215 204, 222 218, 239 233; SwiGLU backward 108 97, 121 114, 135 123, 147 134; down and gate
+    // and up backward level up to 26, 119 114 and 216 208, 129 123 and 225 219; in a prompt of 280 tokens gate and up 226 201.  32 of 1024 x 1536 at 97 rows, whose second tiles read again, 67 and 70.
+    // Tensors that the Infinity Cache keeps from one use to the next lose by it: 16 of 1024 x 768 (25 MB) 13.8 and 16.7.
+    const bool once = p.mode == 1 && p.expert_mod <= 0 && p.M <= 80ll * p.E && (long long)p.E * p.N * p.K >= 32 << 20;
 #define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
+#define ARIA_G4E(BOC, VER) (once ? launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1, true>(q, split, slabs, stream) : ARIA_G4(BOC, VER))
     if (p.rope_fc) return ARIA_G4(false, 7);
     if (p.glu == 2) return ARIA_G4(false, 13);
-    if (p.glu && p.gather_rows) return p.glu_up_rows > 0 ? ARIA_G4(false, 9) : ARIA_G4(true, 8);
-    if (p.glu && p.glu_up_rows > 0) return ARIA_G4(false, 6);
-    if (p.glu) return b_oc ? ARIA_G4(true, 14) : ARIA_G4(false, 14);
-    if (p.dglu) return b_oc ? ARIA_G4(true, 5) : ARIA_G4(false, 5);
-    return b_oc ? ARIA_G4(true, 3) : ARIA_G4(false, 3);
+    if (p.glu && p.gather_rows) return p.glu_up_rows > 0 ? ARIA_G4E(false, 9) : ARIA_G4E(true, 8);
+    if (p.glu && p.glu_up_rows > 0) return ARIA_G4E(false, 6);
+    if (p.glu) return b_oc ? ARIA_G4E(true, 14) : ARIA_G4(false, 14);
+    if (p.dglu) return b_oc ? ARIA_G4(true, 5) : ARIA_G4E(false, 5);
+    return b_oc ? ARIA_G4E(true, 3) : ARIA_G4E(false, 3);
+#undef ARIA_G4E
 #undef ARIA_G4
 }

@@ -51,10 +51,10 @@ ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44;
 # 120, 119; 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.  Level up to the line: 10240 x 2560: 200
 # tokens 39, 39; 300: 52, 51 -- by rows with 8 us of the host's time, by tiles 15; 2560 x 3328: 320 tokens 33, 34, in a model 7 us ahead (300 tokens, four layers, 2540 us against 2569).
 ROWS_PASSED, ROWS_PASSED_LONG = 52000, 26000
-# Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token: 27 rows 232 us, tiles 270; 37: 254 .. 264, 272; 45: 276, 273.  32 of
-# 1024 x 1536, whose tiles are one full round: 8 rows 44, tiles 47; 27: 55, 49.  16 of 768 x 1024: 27 rows 17, tiles 29; 50: 21, 29.
+# Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token, us by rows / tiles: 9 rows 181 .. 194, 193; 15 185 .. 193, 196; 26 190 .. 200, 201 .. 206; 33 217, 208;
+# 47: 243, 216.  16 of 768 x 1024: 20 rows 16, 22; 44: 22, 22.
 ROWS_PER_EXPERT = 27
-ROWS_PER_EXPERT_DOWN = 4   # down projections: 32 tokens 97 us, tiles 103; 64: 134, tiles 104
+ROWS_PER_EXPERT_DOWN = 10   # down projections of 64 experts: 6 rows 87 .. 91, 103; 12: 94, 100; 15: 98 .. 110, 102; 26: 116, 107; of 32: 8 20.7, 22.8; 12 25.8, 23.3; of 16: 20 12.5, 13.7
 
 
 def rows_take(M: int, K: int, N: int) -> bool:
@@ -70,10 +70,10 @@ def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> boo
 
 
 def experts_tiles_ahead(M: int, E: int, K: int, N: int) -> bool:
-    """Whether the gathered tiles of gate and up are ahead of the rows by expert.  us by rows / tiles, rows an expert: 32 of 1024 x 1536: 4 39 / 40, 8 44 / 41, 12 54 / 40, 24 53 / 42, 32
-    57 / 42; 64 of 1664 x 2560: 6 192 / 206, 9 218 / 210, 18 227 / 211, 27 233 / 215; 16 of 768 x 1024: 12 14.2 / 15.6, 24 14.6 / 16.0, 32 18.9 / 16.1 (few weights: a
-    launch's ramp)."""
-    return M > 8 * E and E * K * N >= 1 << 25
+    """Whether the gathered tiles of gate and up are ahead of the rows by expert up to ROWS_PER_EXPERT: where all of them are one round, and the weights more than a launch's ramp.
+    us by rows / tiles, rows an expert: 32 of 1024 x 1536: 8 36 / 38, 12 45 / 40, 20 46 / 40, 35 51 / 41; 64 of 1664 x 2560: 6 171 / 192, 15 193 / 196, 26 195 / 206; 16 of 768 x 1024:
+    12 15.3 / 21.5, 35 21.8 / 21.7."""
+    return M > 8 * E and E * K * N >= 1 << 25 and E * -(-N // 128) <= 256
 
 
 def rows_gemm(x: torch.Tensor, w: torch.Tensor, out_dtype=bf16) -> torch.Tensor:
