@@ -386,43 +386,115 @@ int grid1d(long long n, int per_block, int cap = 4096) {
     return int(g);
 }
 
+// C consecutive elements, aligned to their size together
+template <int C>
+__device__ __forceinline__ void ldc(const bf16_t* p, float (&v)[C]) {
+    if constexpr (C == 8) {
+        ld8(p, v);
+    } else {
+        const uint32_t a = *reinterpret_cast<const uint32_t*>(p);
+        v[0] = bflo(a), v[1] = bfhi(a);
+    }
+}
+template <int C>
+__device__ __forceinline__ void ldc(const float* p, float (&v)[C]) {
+    if constexpr (C == 8) {
+        ld8(p, v);
+    } else {
+        const f32x2 a = *reinterpret_cast<const f32x2*>(p);
+        v[0] = a[0], v[1] = a[1];
+    }
+}
+template <int C>
+__device__ __forceinline__ void stc(bf16_t* p, const float (&v)[C]) {
+    if constexpr (C == 8)
+        st8(p, v);
+    else
+        *reinterpret_cast<uint32_t*>(p) = pack2bf(v[0], v[1]);
+}
+template <int C>
+__device__ __forceinline__ void stc(float* p, const float (&v)[C]) {
+    if constexpr (C == 8)
+        st8(p, v);
+    else
+        *reinterpret_cast<f32x2*>(p) = f32x2{v[0], v[1]};
+}
+
 // One pass over the fp32 residual stream with the dynamic-tanh norms around it: source (embedding row | sublayer output | weighted sum of a token's
-// expert rows) -> x (+)= post(source) -> h = next(x).  Elementwise in the columns (these norms have no statistics): a thread owns 8 of them.
-template <class T>
+// expert rows) -> x (+)= post(source) -> h = next(x).  Elementwise in the columns (these norms have no statistics): a wave owns 64 C of them, C a lane, whose norms' vectors it
+// keeps in registers, and takes every `step`-th token, the next one's loads in front of this one's arithmetic.
+template <class T, int C>
 __global__ __launch_bounds__(256) void dyt_stream_kernel(const int32_t* ids, const T* table, const T* y, const int32_t* inv, const float* weights, int k,
-                                                         AriaDyT post, float* x, AriaDyT next, T* h, long long nitems, int nch, long long ldy) {
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nitems; i += (long long)gridDim.x * blockDim.x) {
-        const long long t = i / nch;
-        const int n0 = int(i % nch) * 8;
-        float v[8], xv[8];
-        float* xr = x + (t * nch) * 8 + n0;
-        if (ids) {
-            ld8(table + (long long)ids[t] * nch * 8 + n0, xv);
+                                                         AriaDyT post, float* x, AriaDyT next, T* h, long long n_tok, int D, int parts, long long ldy) {
+    const int wave = int(blockIdx.x) * 4 + first_lane(int(threadIdx.x) >> 6), n0 = (wave % parts * 64 + lane_id()) * C, step = int(gridDim.x) * 4 / parts;
+    if (n0 >= D || wave / parts >= step) return;   // (the last workgroup's odd waves)
+    auto norm = [](float alpha, float w, float b, float v) __attribute__((always_inline)) { return tanh_for<T>(alpha * v) * w + b; };
+    struct Columns {
+        float v[C];
+    };
+    auto column = [&](const float* p) __attribute__((always_inline)) {   // of a norm's vector, which may lie at any multiple of four bytes
+        Columns c = {};
+        if (!p) return c;
+        if ((reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+            ldc<C>(p + n0, c.v);
         } else {
-            if (inv) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = 0.f;
-                for (int j = 0; j < k; ++j) {
-                    float r[8];
-                    ld8(y + (long long)inv[t * k + j] * ldy + n0, r);
-                    const float w = weights[t * k + j];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] += w * r[e];
-                }
-            } else {
-                ld8(y + t * ldy + n0, v);
-            }
-            ld8(xr, xv);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) xv[e] += dyt<T>(post, v[e], n0 + e);
+            for (int e = 0; e < C; ++e) c.v[e] = p[n0 + e];
         }
-        st8(xr, xv);
+        return c;
+    };
+    auto stream = [&](long long t) __attribute__((always_inline)) {   // the old x, or the embedding
+        Columns c;
+        if (ids)
+            ldc<C>(table + (long long)ids[t] * D + n0, c.v);
+        else
+            ldc<C>(x + t * D + n0, c.v);
+        return c;
+    };
+    auto output = [&](long long t) __attribute__((always_inline)) {   // the sublayer's
+        Columns c = {};
+        if (!ids && !inv) ldc<C>(y + t * ldy + n0, c.v);
+        return c;
+    };
+    long long t = wave / parts;
+    if (t >= n_tok) return;
+    Columns xv = stream(t), v = output(t);
+    const Columns pw = column(ids ? nullptr : post.w), pb = column(ids ? nullptr : post.b), nw = column(next.w), nb = column(next.w ? next.b : nullptr);
+    auto finish = [&](long long t, Columns xv, Columns v) __attribute__((always_inline)) {
+        if (inv) {
+            Columns r0, r1, r2, r3;
+            auto row = [&](int j) __attribute__((always_inline)) {
+                Columns c;
+                ldc<C>(y + inv[t * k + min(j, k - 1)] * ldy + n0, c.v);
+                return c;
+            };
+            auto add = [&](int j, const Columns& r) __attribute__((always_inline)) {
+                const float w = weights[t * k + min(j, k - 1)];
+#pragma unroll
+                for (int e = 0; e < C; ++e) v.v[e] = j < k ? v.v[e] + w * r.v[e] : v.v[e];
+            };
+            for (int j = 0; j < k; j += 4) {   // four rows in flight
+                r0 = row(j), r1 = row(j + 1), r2 = row(j + 2), r3 = row(j + 3);
+                add(j, r0), add(j + 1, r1), add(j + 2, r2), add(j + 3, r3);
+            }
+        }
+        if (!ids) {
+#pragma unroll
+            for (int e = 0; e < C; ++e) xv.v[e] += norm(post.alpha, pw.v[e], pb.v[e], v.v[e]);
+        }
+        stc<C>(x + t * D + n0, xv.v);
         if (next.w) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = dyt<T>(next, xv[e], n0 + e);
-            st8(h + (t * nch) * 8 + n0, v);
+            for (int e = 0; e < C; ++e) v.v[e] = norm(next.alpha, nw.v[e], nb.v[e], xv.v[e]);
+            stc<C>(h + t * D + n0, v.v);
         }
+    };
+    for (; t + step < n_tok; t += step) {
+        const Columns x1 = stream(t + step), v1 = output(t + step);
+        finish(t, xv, v);
+        xv = x1, v = v1;
     }
+    finish(t, xv, v);
 }
 
 // One pass over the fp32 residual stream with the RMS norms around it, a workgroup per token: x (+)= mult (y, or the half-sum of two normed rows) and
@@ -662,14 +734,30 @@ int aria_dyt_stream(const int32_t* ids, const void* table, const void* y, const 
         return ARIA_ERR_INVALID;
     if ((D & 7) || (!ids && (ldy & 7))) return ARIA_ERR_ALIGN;
     if (T == 0) return ARIA_OK;
-    const long long nitems = T * (D / 8);
-    const dim3 grid(unsigned(std::min<long long>((nitems + 255) / 256, 256 * 16))), block(256);
-    if (f32)
-        ARIA_LAUNCH((dyt_stream_kernel<float>), grid, block, 0, stream, ids, static_cast<const float*>(table), static_cast<const float*>(y), inv, weights,
-                    int(k), *post, x, *next, static_cast<float*>(h), nitems, int(D / 8), (long long)ldy);
-    else
-        ARIA_LAUNCH((dyt_stream_kernel<bf16_t>), grid, block, 0, stream, ids, static_cast<const bf16_t*>(table), static_cast<const bf16_t*>(y), inv,
-                    weights, int(k), *post, x, *next, static_cast<bf16_t*>(h), nitems, int(D / 8), (long long)ldy);
+    // Us, a thread an item with the norms' vectors read for each / here.  32 bits (tanhf is the time): two columns a lane while that fills the chip no more than once, 1024 x 4 5.7 / 2.7, 614 10.3 / 4.3,
+    // by experts 6.4 / 3.0, 12.5 / 5.9 (eight columns 5.1, 6.6); 1868 21 / 9.3, 2560 x 4692 102 / 38.  bf16: 1536 x 4 2.5 / 2.4, 200 2.8 / 3.0, 4692 15.8 / 15.5, by experts 3.3 / 2.6, 3.6 / 3.4, 26.5 / 23.4;
+    // 2560 x 16384 122 / 94 (5.4 TB/s), 168 / 148.
+    const bool few = T * D <= (f32 ? 700000 : 270000);
+    const int cols = few ? 2 : 8;
+    const int64_t parts = (D + 64 * cols - 1) / (64 * cols);   // column parts of a token, a wave each
+    // up to sixteen waves a CU take one item each; beyond, eight (16384 x 1536, 4 / 8 / 16 of them 67 / 53 / 56 us)
+    const int64_t waves = T * parts <= 4096 ? T * parts : std::max<int64_t>(1, 2048 / parts) * parts;
+    const dim3 grid(unsigned((waves + 3) / 4)), block(256);
+#define ARIA_DYT_STREAM(TYPE, C)                                                                                                                                   \
+    ARIA_LAUNCH((dyt_stream_kernel<TYPE, C>), grid, block, 0, stream, ids, static_cast<const TYPE*>(table), static_cast<const TYPE*>(y), inv, weights, int(k), *post, x, *next, \
+                static_cast<TYPE*>(h), (long long)T, int(D), int(parts), (long long)ldy)
+    if (f32) {
+        if (few)
+            ARIA_DYT_STREAM(float, 2);
+        else
+            ARIA_DYT_STREAM(float, 8);
+    } else {
+        if (few)
+            ARIA_DYT_STREAM(bf16_t, 2);
+        else
+            ARIA_DYT_STREAM(bf16_t, 8);
+    }
+#undef ARIA_DYT_STREAM
     return aria_check_launch();
 }
 

@@ -191,6 +191,25 @@ def case_dyt_stream(dev, dtype, T=7, D=40):
     assert bool(torch.isfinite(x).all())
 
 
+def case_dyt_stream_parts(dev, dtype, T, D, k, offset=0):
+    """Lanes of two and of eight columns, column parts that end inside a wave, waves with several tokens, more expert rows than are in flight at a time, norms' vectors `offset`
+    floats behind a multiple of 16 bytes."""
+    from aria_amd import hip, ops
+
+    flat = rnd(4 * (D + 4), seed=3, dtype=f32).to(dev)
+    vec = [flat[i * (D + 4) + offset:][:D] for i in range(4)]
+    post, nxt = (hip.DyTParams(a, vec[i].data_ptr(), vec[i + 1].data_ptr()) for a, i in ((0.7, 0), (0.4, 2)))
+    w = [t.cpu().double() for t in vec]
+    x0, y, inv, wts = rnd(T, D, seed=4, dtype=f32), rnd(T * k, D + 8, seed=5, dtype=dtype), torch.randperm(T * k, generator=gen(9)).to(torch.int32), torch.rand(T, k, generator=gen(8))
+    for experts in (False, True):
+        src = (y.double()[inv.long(), :D].view(T, k, D) * wts.double()[..., None]).sum(1) if experts else y.double()[:T, :D]
+        x1 = x0.double() + torch.tanh(0.7 * src) * w[0] + w[1]
+        x = x0.to(dev, copy=True)
+        rows = y.to(dev)[:, :D]
+        h = ops.dyt_stream(x, post, nxt, **(dict(y=rows, inv=inv.to(dev), weights=wts.to(dev)) if experts else dict(y=rows[:T])))
+        assert rel(x, x1) < 2e-6 and rel(h, torch.tanh(0.4 * x1) * w[2] + w[3]) < (2e-6 if dtype == f32 else 3e-3)
+
+
 def case_activations(dev, dtype):
     from aria_amd import ops
 

@@ -25,6 +25,11 @@ def test_dyt_stream(dtype):
 
 
 @both
+def test_dyt_stream_parts(dtype):
+    C.case_dyt_stream_parts(DEV, dtype, 5, 136, 5, 1)
+
+
+@both
 def test_activations(dtype):
     C.case_activations(DEV, dtype)
 

@@ -29,6 +29,12 @@ def test_dyt_stream(dtype):
 
 
 @both
+@pytest.mark.parametrize("T,D,k,offset", [(3, 136, 1, 1), (201, 1024, 2, 0), (262, 1032, 5, 3), (700, 1000, 4, 0), (701, 1544, 6, 0), (5000, 520, 1, 2)])
+def test_dyt_stream_parts(dtype, T, D, k, offset):
+    C.case_dyt_stream_parts(DEV, dtype, T, D, k, offset)
+
+
+@both
 def test_activations(dtype):
     C.case_activations(DEV, dtype)
 
