@@ -330,6 +330,19 @@ __device__ __forceinline__ uint32_t mul24(uint32_t a, uint32_t b) {
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ void st16(void* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }
 __device__ __forceinline__ u32x4 zero16() { return u32x4{0u, 0u, 0u, 0u}; }
+__device__ __forceinline__ u32x4 ld16_once(const void* p) {   // of bytes that nobody reads again: non-temporal
+#ifdef ARIA_EMU
+    return ld16(p);
+#else
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+#endif
+}
+// Sixteen rows' lines of eight 16-byte chunks: a holds rows 0 .. 7 and b rows 8 .. 15, lane (c, q) with row c & 7, chunk q + 4 (c >> 3) -> lo and hi, lane (c, q) with row c, chunks q and q + 4:
+// what a matrix step's lanes want of such lines
+__device__ __forceinline__ void whole_lines(const u32x4& a, const u32x4& b, u32x4& lo, u32x4& hi) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lo[i] = upper_half_from(a[i], b[i]), hi[i] = lower_half_from(b[i], a[i]);
+}
 // streaming 16-byte store (non-temporal: the line is not kept in the L2 for a reader that will not come from this XCD)
 __device__ __forceinline__ void st16_stream(void* p, u32x4 v) {
 #ifdef ARIA_EMU

@@ -68,7 +68,8 @@ __device__ __forceinline__ void stream_step(const GemmF32& p, float v, float& x,
     if (p.next.w) h = dyt<float>(p.next, x, n);
 }
 
-template <int MT, int NT, int NW, int FIN>
+// ONCE: a step's weights come as the rows 0 .. 7 of a line, the next one's as the rows 8 .. 15 (the same bits)
+template <int MT, int NT, int NW, int FIN, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     constexpr bool PAIR = FIN == ARIA_F32_PAIR;
     constexpr int WS = PAIR ? 2 : 1;
@@ -88,7 +89,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
 #pragma unroll
     for (int z = 0; z < WS; ++z)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) wp[z][j] = (z ? p.W2 : p.W) + e * p.strideW + (long long)min(n0 + 16 * j + c16, p.N - 1) * p.ldw + w * LINE + q4 * 4;
+        for (int j = 0; j < NT; ++j)   // ONCE: of the first of a line's two loads, rows 0 .. 7; the second's are those eight rows on
+            wp[z][j] = (z ? p.W2 : p.W) + e * p.strideW + (long long)min(n0 + 16 * j + (ONCE ? c16 & 7 : c16), p.N - 1) * p.ldw + w * LINE + (ONCE ? q4 + 4 * (c16 >> 3) : q4) * 4;
+    const long long eight = ONCE ? (long long)(min(n0 + (c16 & 7) + 8, p.N - 1) - min(n0 + (c16 & 7), p.N - 1)) * p.ldw - 16 : 0;   // (behind the step's own 16 columns)
     f32x4 acc[WS][MT][NT];
 #pragma unroll
     for (int z = 0; z < WS; ++z)
@@ -104,13 +107,29 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
         f32x4 a[MT], b[WS][NT];
     };
     Step x[DEPTH];
-    auto load = [&](long long k, Step& f) __attribute__((always_inline)) {
+    auto load = [&](long long k, Step& f, bool second) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) f.a[i] = *reinterpret_cast<const f32x4*>(ap[i] + k);
 #pragma unroll
         for (int z = 0; z < WS; ++z)
 #pragma unroll
-            for (int j = 0; j < NT; ++j) f.b[z][j] = *reinterpret_cast<const f32x4*>(wp[z][j] + k);
+            for (int j = 0; j < NT; ++j) {
+                if constexpr (ONCE)
+                    f.b[z][j] = __builtin_bit_cast(f32x4, ld16_once(wp[z][j] + k + (second ? eight : 0)));
+                else
+                    f.b[z][j] = *reinterpret_cast<const f32x4*>(wp[z][j] + k);
+            }
+    };
+    // ONCE: the two loads of a line become the fragments of its two steps
+    auto exchange = [&](Step& f, Step& g) __attribute__((always_inline)) {
+        if constexpr (ONCE) {
+#pragma unroll
+            for (int z = 0; z < WS; ++z) {
+                u32x4 lo, hi;
+                whole_lines(__builtin_bit_cast(u32x4, f.b[z][0]), __builtin_bit_cast(u32x4, g.b[z][0]), lo, hi);
+                f.b[z][0] = __builtin_bit_cast(f32x4, lo), g.b[z][0] = __builtin_bit_cast(f32x4, hi);
+            }
+        }
     };
     auto use = [&](const Step& f) __attribute__((always_inline)) {
 #pragma unroll
@@ -124,13 +143,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
     };
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u)
-        if (u < mine) load(at(u), x[u]);
+        if (u < mine) load(at(u), x[u], u & 1);
     int s = 0;
     for (; s + 2 * DEPTH <= mine; s += DEPTH) {
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
+            if (u % 2 == 0) exchange(x[u], x[(u + 1) % DEPTH]);
             use(x[u]);
-            load(at(s + u + DEPTH), x[u]);
+            load(at(s + u + DEPTH), x[u], u & 1);
             sched_fence();   // (left alone the compiler asks for all of them behind the last product)
         }
     }
@@ -138,13 +158,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_kernel(GemmF32 p) {
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
             if (s + u >= mine) break;
+            if (u % 2 == 0) exchange(x[u], x[(u + 1) % DEPTH]);
             use(x[u]);
-            if (s + u + DEPTH < mine) load(at(s + u + DEPTH), x[u]);
+            if (s + u + DEPTH < mine) load(at(s + u + DEPTH), x[u], u & 1);
         }
     }
-    if ((p.K & 15) && w == steps % NW) {   // the rest of the row, K % 16 = 4, 8 or 12 columns: lanes behind it hold zeros in both operands
+    if (!ONCE && (p.K & 15) && w == steps % NW) {   // the rest of the row, K % 16 = 4, 8 or 12 columns: lanes behind it hold zeros in both operands
         const bool in = q4 * 4 < (p.K & 15);
-        load(in ? steps * 16 - w * LINE : -(w * LINE + q4 * 4), x[0]);   // (not in: a column of the same row)
+        load(in ? steps * 16 - w * LINE : -(w * LINE + q4 * 4), x[0], false);   // (not in: a column of the same row)
         if (!in) {
 #pragma unroll
             for (int i = 0; i < MT; ++i) x[0].a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -369,7 +390,16 @@ int launch_f32(const GemmF32& p, void* stream) {
     const int64_t ntm = (int64_t(p.M) + 16 * MT - 1) / (16 * MT) + (p.offsets ? p.E : 0);   // (an expert's last tile may be ragged)
     const int64_t ntn = (int64_t(p.N) + 16 * NT - 1) / (16 * NT);
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
-    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, FIN>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
+    if constexpr (MT * NT == 1) {
+        // Weights by whole lines, non-temporal (whole_lines): read once, and enough of them or experts'.  Us, half lines / whole: 4 x 32000 x 1024 29.9 / 26.9, 16 40.3 / 35.5, 16 x 64000 x 1536 120 / 99,
+        // 4 x 2816 x 1024 5.7 / 5.4, 4 x 6656 x 2560 19.7 / 17.5; 4 x 1024 x 1024 5.0 / 5.0, 4 x 512 x 256 2.6 / 3.0; 64 experts of 1664 x 2560, 32 rows 86 / 76, 16 of 768 x 1024, 8 rows, that the
+        // Infinity Cache held 8.4 / 8.8 -- in a model's step it does not (four sequences, three layers: 1629 / 1602 with theirs whole too).
+        if (p.K % 32 == 0 && p.ldw % 32 == 0 && p.strideW % 32 == 0 && (p.offsets || (long long)p.N * p.K >= 3 << 19)) {
+            ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, FIN, true>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
+            return aria_check_launch();
+        }
+    }
+    ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, FIN, false>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
     return aria_check_launch();
 }
 

@@ -10,13 +10,7 @@
 
 namespace ad {
 
-__device__ __forceinline__ u32x4 ldw16(const bf16_t* p) {   // a weight stream is read once: non-temporal
-#ifdef ARIA_EMU
-    return ld16(p);
-#else
-    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-#endif
-}
+__device__ __forceinline__ u32x4 ldw16(const bf16_t* p) { return ld16_once(p); }   // a weight stream is read once
 // acc[r] += W[row r] . x, a wave over two weight rows: four 16-byte chunks per row and lane requested before the first use, the token's row comes from the
 // L1 / L2
 __device__ __forceinline__ void two_rows(float (&acc)[2], const bf16_t* w0, const bf16_t* w1, const bf16_t* x, int K, int l) {
@@ -111,14 +105,6 @@ template <int NW, int MT>
 struct RowsRed {
     float v[2][NW][16 * MT][17];
 };
-// rows 0 .. 7 and 8 .. 15 of 64 columns, lane (c, q) with row c & 7, chunk q + 4 (c >> 3) -> the fragments of columns 0 .. 31 and 32 .. 63, lane (c, q) with row c, chunk q
-__device__ __forceinline__ void whole_lines(const u32x4& a, const u32x4& b, s16x8& lo, s16x8& hi) {
-    u32x4 x, y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = upper_half_from(a[i], b[i]), y[i] = lower_half_from(b[i], a[i]);
-    lo = __builtin_bit_cast(s16x8, x);
-    hi = __builtin_bit_cast(s16x8, y);
-}
 template <int NW, int KS, int MT, bool ONCE, class WRow, class XRow, class Out>
 __device__ __forceinline__ void stream_rows(int K, const WRow& wrow, const XRow& xrow, int g0, int g1, RowsRed<NW, MT>& red, const Out& out) {
     constexpr int P = KS / 2;                                          // ONCE: pairs of steps, and a left-over one where KS is odd
@@ -172,10 +158,10 @@ __device__ __forceinline__ void stream_rows(int K, const WRow& wrow, const XRow&
 #pragma unroll
                 for (int p = 0; p < P; ++p) {
                     const int s = p % SLOTS;
-                    s16x8 lo, hi;
+                    u32x4 lo, hi;
                     whole_lines(a[s], b[s], lo, hi);
-                    step(2 * p, lo);
-                    step(2 * p + 1, hi);
+                    step(2 * p, __builtin_bit_cast(s16x8, lo));
+                    step(2 * p + 1, __builtin_bit_cast(s16x8, hi));
                     if (p + SLOTS < P)
                         a[s] = ldw16(wa + line + 64 * (p + SLOTS)), b[s] = ldw16(wb + line + 64 * (p + SLOTS));
                     else if (on)

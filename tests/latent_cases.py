@@ -272,6 +272,23 @@ def case_gemm_f32_tiles(dev, M, N, K):
         assert torch.equal(by_expert[rows], ops.linear_any(a[rows], w[expert])), rows
 
 
+def case_gemm_f32_whole_lines(dev, M, N, K, E=5):
+    """Up to 16 rows whose weights come by whole lines, dense and by expert, against the same by half lines (too few weights for whole ones): the same bits, and float64."""
+    from aria_amd import ops
+
+    a, w = rnd(M, K, seed=1, dtype=f32).to(dev), rnd(N, K, seed=2, dtype=f32).to(dev)
+    assert N * K >= 3 << 19 > 40 * K and K % 32 == 0
+    got = ops.linear_any(a, w)
+    assert rel(got, a.double().cpu() @ w.double().cpu().T) < 2e-6
+    for at in (0, N // 2, N - 40):
+        assert torch.equal(got[:, at:at + 40], ops.linear_any(a, w[at:at + 40].contiguous()))
+    we = w[:37 * E].view(E, 37, K).contiguous()
+    off = torch.tensor([0, 0, M // 2, M // 2, M, M], dtype=torch.int32, device=dev)
+    by_expert = ops.grouped_linear_any(a, we, off)
+    each = [ops.linear_any(a[p:q], we[e]) for p, q, e in ((0, M // 2, 1), (M // 2, M, 3)) if q > p]
+    assert torch.equal(by_expert, torch.cat(each))
+
+
 def case_route_groups(dev, T, E, groups, keep, k):
     from aria_amd import ops
 

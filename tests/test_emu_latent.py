@@ -49,6 +49,10 @@ def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)
 
 
+def test_gemm_f32_whole_lines():
+    C.case_gemm_f32_whole_lines(DEV, 3, 400, 3936)
+
+
 @pytest.mark.parametrize("M,N,K", [(560, 481, 20), (560, 484, 100)])
 def test_gemm_f32_tiles(M, N, K):
     C.case_gemm_f32_tiles(DEV, M, N, K)

@@ -54,6 +54,11 @@ def test_gemm_f32(M, N, K):
     C.case_gemm_f32(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1536, 1024), (4, 32000, 1024), (16, 761, 2080), (7, 397, 4000), (3, 6200, 256), (16, 49200, 32)])
+def test_gemm_f32_whole_lines(M, N, K):
+    C.case_gemm_f32_whole_lines(DEV, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(560, 481, 4), (600, 484, 36), (1030, 322, 64), (883, 319, 1020), (1500, 190, 2816), (2500, 128, 128), (40000, 96, 52)])   # the last stage's remainders
 def test_gemm_f32_tiles(M, N, K):
     C.case_gemm_f32_tiles(DEV, M, N, K)
