@@ -199,7 +199,7 @@ int aria_decode_step(const void* const* ptrs, const int64_t* dims, float eps, in
         const int64_t p = ARIA_DECODE_STEP_PTRS + ARIA_DECODE_LAYER_PTRS * li;
         bf16_t *kc = const_cast<bf16_t*>(weight(p + 11)), *vc = const_cast<bf16_t*>(weight(p + 12));
         rc = rows(input(weight(p + 1), 3 * D), StoreBf16{z.qkv, 3 * D});
-        if (rc == ARIA_OK) rc = aria_decode_rows_attn(z.qkv, weight(0), slot, pos, kc, vc, z.ao, z.part, H, hd, Smax, T, splits, stream);
+        if (rc == ARIA_OK) rc = aria_decode_rows_attn(z.qkv, weight(0), slot, pos, kc, vc, z.ao, z.part, H, hd, Smax, T, splits, max_len, stream);
         RowsIn wo{weight(p + 2), nullptr, z.ao, (long long)D, int(D), int(D)};
         if (rc == ARIA_OK) rc = rows(wo, Residual{z.x, z.h, weight(p + 3), (long long)D, z.sums});
         sq_n = rows_parts(T, D);

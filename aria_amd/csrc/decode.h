@@ -12,7 +12,7 @@
 ARIA_HIDDEN int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len, int64_t Smax);
 // RoPE, cache write and attention of T tokens of T sequences: qkv [T, 3 H hd], caches [slots, Smax, H hd], part: T H splits (hd + 2) floats, out [T, H hd]
 ARIA_HIDDEN int aria_decode_rows_attn(const ad::bf16_t* qkv, const ad::bf16_t* freqs, const int32_t* slot, const int32_t* pos, ad::bf16_t* kc, ad::bf16_t* vc,
-                                      ad::bf16_t* out, float* part, int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, void* stream);
+                                      ad::bf16_t* out, float* part, int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, int64_t max_len, void* stream);
 ARIA_HIDDEN int aria_route_and_sort(const ad::bf16_t* logits, ad::bf16_t* scores, int32_t* idx, int32_t* counts, int32_t* offsets, int32_t* src, int32_t* inv,
                                     int32_t* rows, int T, int E, int k, void* stream);
 ARIA_HIDDEN int aria_decode_dims_ok(const int64_t* dims);

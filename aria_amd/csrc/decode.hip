@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(bf16_t* qkv, const bf16
 // DecodeAttn<HD>::run is the body shared by the two kernels below: keys [kbeg, kend) of one head, `writes_new` (block-uniform) = this
 // workgroup owns the new position and puts the rotated key / value into the cache before reading it back.  On return the lanes with
 // w == 0 && grp == 0 hold the UNNORMALISED state (m, lsum, o[8] for features sub*8 ..) of the whole range.
-template <int HD, int NWV = 4>
+template <int HD, int NWV = 4, bool ONCE = false>
 struct DecodeAttn {
     // NWV waves per workgroup, U keys per lane group and pass: NWV x KPW x U keys per pass over the range, all K / V rows of a pass in
     // flight before the first use.  Round 3: the one-workgroup-per-head kernel went from 4 waves x U 4 (64 keys per pass at hd 128) to
@@ -457,8 +457,8 @@ struct DecodeAttn {
             for (int u = 0; u < U; ++u) {
                 key[u] = j0 + (w * U + u) * KPW + grp;
                 const long long row = (long long)min(key[u], kend - 1) * D + col;
-                kx[u] = ld16(k_cache + row);
-                vx[u] = ld16(v_cache + row);
+                kx[u] = ONCE ? ld16_once(k_cache + row) : ld16(k_cache + row);
+                vx[u] = ONCE ? ld16_once(v_cache + row) : ld16(v_cache + row);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -576,11 +576,11 @@ __global__ __launch_bounds__(DECODE_ATTN_WAVES * 64) void decode_attn_kernel(con
 // decode_attn_kernel; only the order in which partial states are merged differs.
 constexpr int DECODE_MAX_SPLITS = 32;
 
-template <int HD>
+template <int HD, bool ONCE>
 __global__ __launch_bounds__(256) void decode_attn_split_kernel(const bf16_t* qkv, const bf16_t* fc, const int32_t* pos, const int32_t* slot,
                                                                 long long slot_stride, bf16_t* k_cache, bf16_t* v_cache, float* part, int D,
                                                                 float scale) {
-    using A = DecodeAttn<HD>;
+    using A = DecodeAttn<HD, 4, ONCE>;
     ARIA_SMEM_STATIC float red[4][A::LPK][10];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, sub = l % A::LPK, grp = l / A::LPK, head = blockIdx.x, split = blockIdx.y, tok = blockIdx.z;
     const int NS = gridDim.y;
@@ -787,10 +787,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_topk_kernel(const bf16_
 }
 
 // splits == 1: the one-workgroup-per-head kernel; otherwise the split form + merge (part: T * H * splits * (hd + 2) floats).  T tokens of T sequences, each on
-// its own slot of the caches (slot NULL: one sequence)
+// its own slot of the caches (slot NULL: one sequence).  keys: of all tokens together, at most (0: not known)
 int launch_decode_attn(void* stream, const bf16_t* qkv, const bf16_t* freqs, const int32_t* pos, bf16_t* kc, bf16_t* vc, bf16_t* out,
                        float* part, int64_t H, int64_t hd, int64_t D, int splits, int64_t T = 1, const int32_t* slot = nullptr,
-                       int64_t slot_stride = 0) {
+                       int64_t slot_stride = 0, long long keys = 0) {
     const float sc = 1.0f / sqrtf(float(hd));
     const unsigned h = unsigned(H), t = unsigned(T);
     const long long ss = slot_stride;
@@ -803,10 +803,19 @@ int launch_decode_attn(void* stream, const bf16_t* qkv, const bf16_t* freqs, con
         return aria_check_launch();
     }
     const dim3 grid(h, unsigned(splits), t);
-    if (hd == 128)
-        ARIA_LAUNCH((decode_attn_split_kernel<128>), grid, dim3(256), 0, stream, qkv, freqs, pos, slot, ss, kc, vc, part, int(D), sc);
+    // Keys and values that the Infinity Cache will not hold until the next token pass it by (non-temporal; a layer's, bytes).  Aria's steps of four layers, us, without / with: 8 sequences of 750 ..
+    // 3000 keys (150 MB a layer) 1019 / 992, 16 of up to 8000 1844 / 1773, 16 of 300 (49 MB at most) 1234 / 1220, one of 8000 442 / 437; 4 of 500 (20 MB) 703 / 705, one of 600 380 / 382.
+    const bool once = keys * D * 4 >= 40 << 20;
+#define ARIA_SPLIT(HD, ONCE) ARIA_LAUNCH((decode_attn_split_kernel<HD, ONCE>), grid, dim3(256), 0, stream, qkv, freqs, pos, slot, ss, kc, vc, part, int(D), sc)
+    if (hd == 128 && once)
+        ARIA_SPLIT(128, true);
+    else if (hd == 128)
+        ARIA_SPLIT(128, false);
+    else if (once)
+        ARIA_SPLIT(64, true);
     else
-        ARIA_LAUNCH((decode_attn_split_kernel<64>), grid, dim3(256), 0, stream, qkv, freqs, pos, slot, ss, kc, vc, part, int(D), sc);
+        ARIA_SPLIT(64, false);
+#undef ARIA_SPLIT
     int rc = aria_check_launch();
     if (rc != ARIA_OK) return rc;
     ARIA_LAUNCH(decode_attn_merge_kernel, dim3(h, t), dim3(unsigned(hd)), 0, stream, (const float*)part, out, splits, int(hd));
@@ -896,6 +905,7 @@ struct OneToken {
     bf16_t* logits;
     float* logits32;             // instead of logits
     int splits;
+    long long keys;              // at most (0: not known)
 };
 int dims_ok(const int64_t* d) {
     const int64_t L = d[0], D = d[1], H = d[2], hd = d[3], E = d[4], k = d[5], I = d[6], Is = d[7];
@@ -932,7 +942,7 @@ int decode_one(const OneToken& one, const Scratch& s, const int64_t* dims, float
         // attention block: h = x + wo( attn( rope(wqkv(norm(x))) ) )
         ARIA_TRY(launch_gemv(int(3 * D), stream, wqkv, (long long)D, x, attn_norm, eps, int(D), nullptr, s.qkv));
         if (one.slot || Smax <= 16384 || splits > 1) {  // one workgroup per head walks the whole context, or (opt-in) heads x splits workgroups
-            ARIA_TRY(launch_decode_attn(stream, (const bf16_t*)s.qkv, one.freqs, pos, kc, vc, s.ao, s.part, H, hd, D, splits, 1, one.slot, Smax * D));
+            ARIA_TRY(launch_decode_attn(stream, (const bf16_t*)s.qkv, one.freqs, pos, kc, vc, s.ao, s.part, H, hd, D, splits, 1, one.slot, Smax * D, one.keys));
         } else {
             ARIA_LAUNCH(rope_cache_kernel, dim3(unsigned((3 * D / 8 + 255) / 256)), dim3(256), 0, stream, s.qkv, one.freqs, pos, kc, vc, int(D),
                         int(hd), s.kv_len);
@@ -1015,8 +1025,8 @@ int aria_decode_rows_splits(int64_t H, int64_t T, int64_t max_len, int64_t Smax)
     return int(std::max<int64_t>(1, std::min<int64_t>(std::min(fill, passes), DECODE_MAX_SPLITS)));
 }
 int aria_decode_rows_attn(const bf16_t* qkv, const bf16_t* freqs, const int32_t* slot, const int32_t* pos, bf16_t* kc, bf16_t* vc, bf16_t* out, float* part,
-                          int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, void* stream) {
-    return launch_decode_attn(stream, qkv, freqs, pos, kc, vc, out, part, H, hd, H * hd, splits, T, slot, Smax * H * hd);
+                          int64_t H, int64_t hd, int64_t Smax, int64_t T, int splits, int64_t max_len, void* stream) {
+    return launch_decode_attn(stream, qkv, freqs, pos, kc, vc, out, part, H, hd, H * hd, splits, T, slot, Smax * H * hd, T * max_len);
 }
 int aria_decode_dims_ok(const int64_t* dims) { return dims_ok(dims); }
 int aria_decode_table_ok(const void* const* ptrs, int64_t layers) {
@@ -1034,7 +1044,7 @@ int aria_decode_one(const void* const* ptrs, const int64_t* dims, float eps, con
                     float* logits, char* scratch, void* stream) {
     const Scratch s = carve(scratch, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6], dims[7]);
     const OneToken one{static_cast<const bf16_t*>(ptrs[0]), static_cast<const bf16_t*>(ptrs[1]), static_cast<const bf16_t*>(ptrs[2]), static_cast<const bf16_t*>(x),
-                       ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len, dims[9])};
+                       ptrs + ARIA_DECODE_STEP_PTRS, pos, slot, nullptr, logits, aria_decode_rows_splits(dims[2], 1, max_len, dims[9]), max_len};
     return decode_one(one, s, dims, eps, stream);
 }
 

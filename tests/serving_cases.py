@@ -350,6 +350,25 @@ def case_decode_splits(dev, monkeypatch, run=True):
             assert L.logit_err(step(n), w) < 4 * 2 ** -8, value
 
 
+def case_decode_keys_once(dev, monkeypatch, head_dim):
+    """Keys and values read non-temporally (told of more keys than the Infinity Cache holds) and plainly: the same splits, the same bits."""
+    from aria_amd.serving import StepBatch
+
+    m = gptfast_routed(dev, 2560, head_dim, 64, 4104)
+    m.setup_caches(3, 4104)
+    for b in m.layers:
+        for c in (b.attention.kv_cache.k, b.attention.kv_cache.v):
+            c.copy_(torch.randn(c.shape, generator=L.gen(1)))
+    monkeypatch.setenv("ARIA_DECODE_SPLIT_KV", "5")
+    for n in (1, 3):
+        got = []
+        for most in (1300, 4100):
+            assert (n * most * 2560 * 4 >= 40 << 20) == (most == 4100)
+            monkeypatch.setattr(StepBatch, "max_len", property(lambda self, most=most: most))
+            got.append(m.step(StepBatch.build([[5], [9], [77]][:n], list(range(n)), [1290, 3, 700][:n], None, dev)).clone())
+        assert torch.equal(*got)
+
+
 def case_alignment(dev):
     """Tensors that do not start at 16 bytes are refused in front of every launch, as the tile products refuse them."""
     from aria_amd import gptfast as G

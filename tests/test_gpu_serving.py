@@ -63,6 +63,11 @@ def test_decode_splits(monkeypatch):
     C.case_decode_splits(DEV, monkeypatch)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_decode_keys_once(monkeypatch, head_dim):
+    C.case_decode_keys_once(DEV, monkeypatch, head_dim)
+
+
 def test_alignment():
     C.case_alignment(DEV)
 
