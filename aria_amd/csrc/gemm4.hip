@@ -98,7 +98,7 @@ struct Shape4 {
     static constexpr size_t SMEM = std::max(size_t(S) * STAGE, size_t(BM) * ROWP);
 };
 
-// ONCE: B's pieces are non-temporal (which: aria_launch_gemm4)
+// ONCE: B's pieces are non-temporal
 // VER: what happens to the tile (the numbers of gemm3_kernel): 3 plain (bias, activation, accumulation, 32-bit results), 5 SwiGLU backward, 6 / 9 fused SwiGLU on two
 // weight tensors (9: gathered rows), 8 on [K, N] weights with gathered rows, 14 on one [gate | up] tensor, 13 relu gate, 7 the interleaved rotation,
 // 11 plain, with the reduction's rows of A reached through an index (per-expert weight gradients)
@@ -286,14 +286,21 @@ __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& pla
         uint32_t at = 0, fill = (S - 1) * STAGE;   // the stage in use; the one that was in use before it and is filled now
         // the products of sixteenth KK of the stage, with the reads of the next and a share of the DMA pieces one by one between them
         constexpr int QUOTA = (PA + PB + HALVES - 2) / (HALVES - 1);
+        constexpr int READS = (MI + NI + MI * NI - 1) / (MI * NI), PIECES = (QUOTA + MI * NI - 1) / (MI * NI);   // behind one product (one each but in tiles of 32 rows)
         auto sixteenth = [&](auto kk, s16x8 (&ra)[MI], s16x8 (&rb)[NI], s16x8 (&na)[MI], s16x8 (&nb)[NI], uint32_t from, auto whole, const char* a, const char* b, char* d)
                              __attribute__((always_inline)) {
             constexpr int KK = decltype(kk)::value, NEXT = (KK + 1) % HALVES;
             each([&](auto j) {
                 constexpr int J = decltype(j)::value;
-                if constexpr (J < MI + NI) frag(std::integral_constant<int, NEXT>{}, j, na, nb, from);
+                each([&](auto z) {
+                    constexpr int F = J * READS + decltype(z)::value;
+                    if constexpr (F < MI + NI) frag(std::integral_constant<int, NEXT>{}, std::integral_constant<int, F>{}, na, nb, from);
+                }, std::make_index_sequence<READS>{});
                 product(j, ra, rb);
-                if constexpr (decltype(whole)::value && KK < HALVES - 1 && J < QUOTA && KK * QUOTA + J < PA + PB) piece(std::integral_constant<int, KK * QUOTA + J>{}, a, b, d);
+                each([&](auto z) {
+                    constexpr int Q = J * PIECES + decltype(z)::value;
+                    if constexpr (decltype(whole)::value && KK < HALVES - 1 && Q < QUOTA && KK * QUOTA + Q < PA + PB) piece(std::integral_constant<int, KK * QUOTA + Q>{}, a, b, d);
+                }, std::make_index_sequence<PIECES>{});
             }, PRODUCTS);
             arrived(na, nb);
         };
@@ -320,7 +327,7 @@ __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& pla
             fill = at;
             at = next;
         };
-        static_assert(QUOTA <= MI * NI && MI + NI <= MI * NI && HALVES % 2 == 0, "a piece and a read behind each product");
+        static_assert(HALVES % 2 == 0, "a stage ends with the fragments that it began with");
         int step = 0;
         // steady steps: the stage that is filled exists and is whole
         const int steady = count - (S - 1) - (first_step + count - 1 == tail_step && tail_k < KD ? 1 : 0);
@@ -448,7 +455,11 @@ __device__ __forceinline__ void gemm4_tile(const GemmParams& p, const Tile4& pla
     }
 }
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false>
+// LOW: rows by expert, of which most experts have fewer than a tile.  A tile that is its expert's only one holds as many blocks of 32 rows as there are rows, and its weights are non-temporal with
+// ONCE: they are bound by the weights' stream, beside which the pieces of rows that are not there are up to a third of what a CU fetches and their products up to three quarters of the matrix
+// work.  64 experts of 2560 x 1664, us with tiles of 128 rows / of what there is, rows an expert 8, 28, 73 evenly and 73, 100 as a router gives them: gate and up, gathered 190 181, 209 195, 235
+// 219, 235 218, 252 244; down 105 97, 112 103, 125 117, 128 116, 129 118; SwiGLU backward 98 92, 115 107, 139 122, 140 131, 179 165; gate and up backward 202 180, 210 190, 222 210, 220 208, 229 216.
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false, bool LOW = false>
 __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     constexpr int BM = Shape4<WM, WN, MI, NI, KD, S>::BM;
     ARIA_DYN_SMEM(smem);
@@ -464,6 +475,7 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     }
     long long b_off = 0, c_off = 0;
     int m0 = tmi * BM, m_end = p.M, k_begin = 0, k_len = p.K;
+    bool alone = false;   // the only tile of its expert's rows
     if (p.mode == 2) {
         k_begin = p.offsets[blockIdx.y];
         k_len = p.offsets[blockIdx.y + 1] - k_begin;
@@ -473,8 +485,18 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
         if (!aria_grouped_tile<BM>(p, blockIdx.x, int(threadIdx.x) & 63, expert, m0, m_end, tn)) return;
         expert = first_lane(expert), m0 = first_lane(m0), m_end = first_lane(m_end), tn = first_lane(tn);
         b_off = (long long)(p.expert_mod > 0 ? expert % p.expert_mod : expert) * p.strideB;
+        alone = m_end - m0 <= BM && m0 == p.offsets[expert];
     }
-    gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, ONCE>(p, Tile4{tn, m0, m_end, k_begin, k_len, b_off, c_off, slab, ks}, smem);
+    const Tile4 place{tn, m0, m_end, k_begin, k_len, b_off, c_off, slab, ks};
+    if constexpr (LOW) {
+        static_assert(MI == 4 && WM == 1, "heights of 32 .. 128 rows");
+        const int rows = m_end - m0;
+        if (ONCE && !alone) return gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER>(p, place, smem);
+        if (rows <= 32) return gemm4_tile<A_OC, B_OC, WM, WN, 1, NI, KD, S + 1, VER, ONCE>(p, place, smem);
+        if (rows <= 64) return gemm4_tile<A_OC, B_OC, WM, WN, 2, NI, KD, S, VER, ONCE>(p, place, smem);
+        if (rows <= 96) return gemm4_tile<A_OC, B_OC, WM, WN, 3, NI, KD, S, VER, ONCE>(p, place, smem);
+    }
+    gemm4_tile<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, ONCE>(p, place, smem);
 }
 
 // the sums of the slabs of gemm4_kernel<.., WM, WN, MI, NI, ..>: see gemm3_reduce_kernel; a block finishes 32 rows of 32 WN columns
@@ -560,7 +582,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_strip_kernel(GemmParams p, int t
     }
 }
 
-template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false>
+template <bool A_OC, bool B_OC, int WM, int WN, int MI, int NI, int KD, int S, int VER, int PER_CU, bool ONCE = false, bool LOW = false>
 int launch4(GemmParams q, int split, float* ws, void* stream) {
     using T = Shape4<WM, WN, MI, NI, KD, S>;
     constexpr int STEP = gated(VER) ? T::BN / 2 : T::BN;
@@ -571,7 +593,8 @@ int launch4(GemmParams q, int split, float* ws, void* stream) {
     q.ws = ws;
     if (q.ntn * q.ntm <= 0) return ARIA_OK;
     const unsigned grid = q.mode == 1 ? unsigned(q.ntn * q.ntm + 16) : unsigned(q.ntn * q.ntm * std::max(split, 1));
-    ARIA_LAUNCH((gemm4_kernel<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, PER_CU, ONCE>), dim3(grid, q.mode == 2 ? unsigned(q.E) : 1u), dim3(256), T::SMEM, stream, q);
+    static_assert(!LOW || Shape4<WM, WN, 1, NI, KD, S + 1>::SMEM <= T::SMEM, "the lowest tiles' stages");
+    ARIA_LAUNCH((gemm4_kernel<A_OC, B_OC, WM, WN, MI, NI, KD, S, VER, PER_CU, ONCE, LOW>), dim3(grid, q.mode == 2 ? unsigned(q.E) : 1u), dim3(256), T::SMEM, stream, q);
     if (split > 1) ARIA_LAUNCH((gemm4_reduce_kernel<WM, WN, MI, NI>), dim3(unsigned(q.ntn * q.ntm), NI * MI * WM), dim3(256), 0, stream, q);
     return aria_check_launch();
 }
@@ -637,11 +660,10 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
         return plan;
     }
     if (p.mode == 1) {
-        // Rows by expert.  Up to 100 a expert its tile of 256 rows is mostly empty and the weights' stream counts, of which three stages of 48 KiB keep more in flight.
-        // 64 experts of 2560 x 1664, rows each on average 28 / 73 / 140, before and now: gate and up, gathered, [K, N] 254 -> 213, 276 -> 233, (306 -> 345); two [N, K]
-        // tensors 26, 66, 192 rows 271 -> 216, 276 -> 228, (325 -> 418); down [K, N] 119 -> 110, 135 -> 124, (153 -> 155), at 6 rows 111 -> 104,
-        // [N, K] at 2, 6, 15, 26 rows 101 -> 74, 107 -> 103, 112 -> 103, 119 -> 107; SwiGLU backward 144 -> 121, 160 -> 149,
-        // (185 -> 200); gate and up backward [N, K] 214 -> 207, 245 -> 220.  And where all of it is one round: 16 experts of 1024 x 768, 187 rows each, 32.6 -> 20.2 and 25 -> 16.
+        // Rows by expert.  Up to 100 an expert its tile of 256 rows is mostly empty and the weights' stream counts, of which three stages of 48 KiB keep more in flight.
+        // 64 experts of 2560 x 1664, as a router gives the rows, 256 x 256 / these tiles, rows each on average 100, 120, 140: gate and up, gathered, [K, N] 287 / 244, 294 / 295, 298 / 338; down
+        // [K, N] 144 / 118, 146 / 145, 151 / 154; SwiGLU backward 169 / 165, 176 / 188, 180 / 201; gate and up backward [N, K] 266 / 216, 271 / 253, 274 / 269.  And where all of it is one round:
+        // 16 experts of 1024 x 768, 187 rows each, 32.6 / 20.2 and 25 / 16.
         if (p.K < 768 || p.N < 512) return none;
         const long long cols = p.glu ? p.N / 2 : p.N, ntn = cdiv(cols, p.glu ? 128 : 256);
         const bool few = p.M < 100ll * p.E, one_round = (p.M / 128 + p.E / 2) * ntn <= ROUND && p.M >= 16ll * p.E;
@@ -717,13 +739,13 @@ int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, f
     }
     if (plan.form == 2)
         return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
-    // Weights by expert that nearly all meet one tile of rows are read once, without a place in the caches (pieces that are non-temporal): a stream of 500 MB at 6.9 TB/s for 6.2.  64 experts of
-    // 2560 x 1664, us before and now, rows each on average 6, 26, 47, 73: gate and up, gathered, [K, N] 209 190, 215 204, 222 218, 239 233; SwiGLU backward 108 97, 121 114, 135 123, 147 134; down and gate
-    // and up backward level up to 26, 119 114 and 216 208, 129 123 and 225 219; in a prompt of 280 tokens gate and up 226 201.  32 of 1024 x 1536 at 97 rows, whose second tiles read again, 67 and 70.
-    // Tensors that the Infinity Cache keeps from one use to the next lose by it: 16 of 1024 x 768 (25 MB) 13.8 and 16.7.
-    const bool once = p.mode == 1 && p.expert_mod <= 0 && p.M <= 80ll * p.E && (long long)p.E * p.N * p.K >= 32 << 20;
+    // Weights by expert pass the caches where a tile is the only one of its expert's rows (gemm4_kernel): a stream of 500 MB at 6.9 TB/s for 6.2.  Tensors that the Infinity Cache keeps from one use to
+    // the next lose by it: 16 experts of 1024 x 768 (25 MB) 13.8 us and 16.7.
+    const bool once = p.mode == 1 && p.expert_mod <= 0 && (long long)p.E * p.N * p.K >= 32 << 20;
 #define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
-#define ARIA_G4E(BOC, VER) (once ? launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1, true>(q, split, slabs, stream) : ARIA_G4(BOC, VER))
+#define ARIA_G4E(BOC, VER) \
+    (once ? launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1, true, true>(q, split, slabs, stream) \
+          : p.mode == 1 ? launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1, false, true>(q, split, slabs, stream) : ARIA_G4(BOC, VER))
     if (p.rope_fc) return ARIA_G4(false, 7);
     if (p.glu == 2) return ARIA_G4(false, 13);
     if (p.glu && p.gather_rows) return p.glu_up_rows > 0 ? ARIA_G4E(false, 9) : ARIA_G4E(true, 8);

@@ -51,10 +51,10 @@ ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44;
 # 120, 119; 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.  Level up to the line: 10240 x 2560: 200
 # tokens 39, 39; 300: 52, 51 -- by rows with 8 us of the host's time, by tiles 15; 2560 x 3328: 320 tokens 33, 34, in a model 7 us ahead (300 tokens, four layers, 2540 us against 2569).
 ROWS_PASSED, ROWS_PASSED_LONG = 52000, 26000
-# Rows of an expert on average, gate and up pairs.  64 experts of 1664 x 2560, 6 a token, us by rows / tiles: 9 rows 181 .. 194, 193; 15 185 .. 193, 196; 26 190 .. 200, 201 .. 206; 33 217, 208;
-# 47: 243, 216.  16 of 768 x 1024: 20 rows 16, 22; 44: 22, 22.
+# Rows of an expert on average, gate and up pairs.  Launches of one kind in turn, us by rows / tiles: 64 experts of 1664 x 2560: 6 rows 162, 182; 12 180, 184; 16 180, 186; 20 200, 187; 28 205, 192; 40
+# 230, 199.  16 of 768 x 1024: 16 rows 15.6, 16.5; 40 16.4, 18.3.  In a prompt of 280 tokens (26 rows) they take 184 us by rows; by tiles its four layers are 1998 us for 1945.
 ROWS_PER_EXPERT = 27
-ROWS_PER_EXPERT_DOWN = 10   # down projections of 64 experts: 6 rows 87 .. 91, 103; 12: 94, 100; 15: 98 .. 110, 102; 26: 116, 107; of 32: 8 20.7, 22.8; 12 25.8, 23.3; of 16: 20 12.5, 13.7
+ROWS_PER_EXPERT_DOWN = 10   # down projections of 64 experts: 6 rows 88.0, 89.5; 10: 89.3, 90.6; 12: 93.8, 90.7; 16: 114, 92; of 32: 8 19.5, 19.0; 12 23.4, 19.5; of 16: 10 10.5, 11.4; 16 13.1, 11.7
 
 
 def rows_take(M: int, K: int, N: int) -> bool:
@@ -71,8 +71,7 @@ def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> boo
 
 def experts_tiles_ahead(M: int, E: int, K: int, N: int) -> bool:
     """Whether the gathered tiles of gate and up are ahead of the rows by expert up to ROWS_PER_EXPERT: where all of them are one round, and the weights more than a launch's ramp.
-    us by rows / tiles, rows an expert: 32 of 1024 x 1536: 8 36 / 38, 12 45 / 40, 20 46 / 40, 35 51 / 41; 64 of 1664 x 2560: 6 171 / 192, 15 193 / 196, 26 195 / 206; 16 of 768 x 1024:
-    12 15.3 / 21.5, 35 21.8 / 21.7."""
+    us by rows / tiles, rows an expert: 32 of 1024 x 1536: 8 33.1 / 34.3, 10 39.2 / 35.0, 20 42.6 / 35.8, 40 48.8 / 36.9; 16 of 768 x 1024: 12 14.1 / 16.0, 28 15.9 / 17.2."""
     return M > 8 * E and E * K * N >= 1 << 25 and E * -(-N // 128) <= 256
 
 

@@ -150,6 +150,35 @@ def case_gemm_four_waves_fused(dev, monkeypatch):
     assert all(form[n] + 16 in seen.get(n, ()) for n in FUSED_FOUR_WAVES), seen
 
 
+def case_gemm_four_waves_low(dev, monkeypatch, K, I, E):
+    """Tiles by expert as high as the expert's rows, at both sides of every height, and of experts with several: the bits of the 256 x 256 tiles.  E x K x I at 32 Mi and beyond: weights that are
+    read past the caches where a tile is the expert's only one."""
+    from aria_amd import ops
+
+    counts = torch.zeros(E, dtype=torch.int64)
+    counts[torch.arange(12) * (E // 12)] = torch.tensor([1, 32, 0, 33, 64, 65, 96, 97, 128, 129, 200, 31])
+    off = torch.zeros(E + 1, dtype=torch.int32)
+    off[1:] = counts.cumsum(0)
+    M, off = int(off[-1]), off.to(dev)
+    x, tokens, dy = rnd(M, K, seed=1).to(dev), rnd(70, K, seed=2).to(dev), rnd(M, K, seed=3).to(dev)
+    rows = (torch.arange(M, dtype=torch.int32, device=dev) * 13) % 70
+    w, h = rnd(E, 2 * I, K, seed=4, scale=0.1).to(dev), rnd(M, 2 * I, seed=5).to(dev)
+    half, kn = w.view(E, 2, I, K).transpose(0, 1).contiguous(), w.view(E, K, 2 * I)
+    forms = [lambda: ops.grouped_gemm(x, w, off, w_is_kn=False), lambda: ops.grouped_gemm(x, kn, off)]
+    if K % 64 == 0:
+        forms += [lambda: ops.grouped_gemm_swiglu(x, kn, off), lambda: ops.grouped_gemm_swiglu_gather(tokens, rows, kn, off, True), lambda: ops.grouped_gemm_dswiglu(dy, half[0], off, h),
+                  lambda: ops.grouped_gemm_swiglu_split(x, half[0], half[1], off), lambda: ops.grouped_gemm_swiglu_split_gather(tokens, rows, half[0], half[1], off)]
+    got = {}
+    for force in ("4", "3"):
+        monkeypatch.setenv("ARIA_GEMM_FORCE", force)
+        for i, f in enumerate(forms):
+            out = f()
+            got.setdefault(i, []).append([t.cpu() for t in (out if isinstance(out, tuple) else (out,)) if t is not None])
+            assert (last_gemm_tiles() == 17) == (force == "4"), i
+    for i, (a, b) in got.items():
+        assert len(a) == len(b) and all(torch.equal(p, q) for p, q in zip(a, b)), i
+
+
 def case_wgrad_strips(dev, monkeypatch, counts, M, N):
     """Weight gradients in strips of 256 columns (the reduction's fragments of dY stay in registers): the bits of the 128 x 256 tiles for experts of any number of rows -- none, partial
     steps of sixteen, the 256 that are held, more -- plain, gathered and dense, and within the bound of a rounded 32-bit sum of exact products."""

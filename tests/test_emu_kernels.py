@@ -148,6 +148,11 @@ def test_attention_block_rule(causal, B, S, Skv, H, waves):
     C.case_attention_block_rule(DEV, causal, B, S, Skv, H, waves)
 
 
+@pytest.mark.parametrize("K,I,E", [(72, 128, 12), (64, 128, 12), (320, 128, 12), (256, 256, 256)])
+def test_gemm_four_waves_low(monkeypatch, K, I, E):
+    C.case_gemm_four_waves_low(DEV, monkeypatch, K, I, E)
+
+
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
 @pytest.mark.parametrize("M,N,K", [(40, 72, 64), (264, 136, 192), (72, 520, 128)])
 def test_gemm_fused_gelu(monkeypatch, force, M, N, K):

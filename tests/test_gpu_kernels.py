@@ -151,6 +151,11 @@ def test_attention_varlen_block_rule(n, S, H, qd, waves):
     C.case_attention_varlen_block_rule(DEV, n, S, H, qd, waves)
 
 
+@pytest.mark.parametrize("K,I,E", [(72, 128, 12), (64, 128, 12), (320, 128, 12), (256, 256, 256), (1536, 1664, 16)])
+def test_gemm_four_waves_low(monkeypatch, K, I, E):
+    C.case_gemm_four_waves_low(DEV, monkeypatch, K, I, E)
+
+
 @pytest.mark.parametrize("force", ["1", "2", "3", None])
 @pytest.mark.parametrize("M,N,K", [(40, 72, 64), (264, 136, 192), (2048, 4304, 1152), (2560, 2560, 4096)])
 def test_gemm_fused_gelu(monkeypatch, force, M, N, K):
