@@ -124,6 +124,7 @@ __device__ __forceinline__ uint32_t lower_half_from(uint32_t own, uint32_t other
     const uint32_t v = emu::shfl(other, emu::lane() ^ 8);
     return emu::lane() & 8 ? own : v;
 }
+__device__ __forceinline__ float max_halves(float v) { return fmaxf(v, emu::shfl(v, emu::lane() ^ 32)); }
 __device__ __forceinline__ unsigned long long ballot(bool p) { return emu::ballot(p); }
 __device__ __forceinline__ int lane_id() { return emu::lane(); }
 __device__ __forceinline__ int first_lane(int v) { return emu::shfl(v, __builtin_ctzll(emu::ballot(true))); }
@@ -148,6 +149,13 @@ __device__ __forceinline__ uint32_t upper_half_from(uint32_t own, uint32_t other
 }
 __device__ __forceinline__ uint32_t lower_half_from(uint32_t own, uint32_t other) {
     return uint32_t(__builtin_amdgcn_update_dpp(int(own), int(other), 0x128, 0xF, 0x3, false));
+}
+// The larger of a lane's value and of the lane's in the wave's other half, on the vector ALU (a ds_bpermute waits behind the LDS reads in flight).  As assembly: of the builtin's two results the
+// compiler kept one here.
+__device__ __forceinline__ float max_halves(float v) {
+    float lo = v, hi = v;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(lo), "+v"(hi));
+    return fmaxf(lo, hi);
 }
 // inclusive prefix sum over the wave's 64 lanes on the vector ALU: four DPP row shifts (scan inside each row of 16) and the two row
 // broadcasts of gfx9 (lane 15 -> next row, lane 31 -> rows 2, 3) -- 6 adds instead of 6 ds_bpermute round trips through the LDS

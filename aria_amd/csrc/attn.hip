@@ -340,7 +340,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(const bf16_t* Q, con
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[i][r]);
-                mx = fmaxf(mx, shfl_xor(mx, 32));
+                mx = max_halves(mx);
             } else {
                 mx = 8.f;
             }
@@ -1369,7 +1369,7 @@ __device__ __forceinline__ void fwd3_step(f32x16 (&st)[2], f32x16 (&sn)[2], f32x
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[i][r]);
-    mx = fmaxf(mx, shfl_xor(mx, 32));
+    mx = max_halves(mx);
     const float m_new = fmaxf(m, mx * scale2);
     const float m_safe = m_new == -INFINITY ? 0.f : m_new;
     if (ballot(m_new > m) != 0ull) {  // wave-uniform lazy rescale: exact (alpha == 1 whenever it is skipped)

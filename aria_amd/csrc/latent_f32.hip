@@ -83,7 +83,7 @@ __global__ __launch_bounds__(NW * 64) void latent_attn_f32_kernel(const float* q
                 mx = fmaxf(mx, x[r]);
             }
             mx = fmaxf(mx, shfl_xor(mx, 16));
-            mx = fmaxf(mx, shfl_xor(mx, 32));
+            mx = max_halves(mx);
             const float mn = fmaxf(m, mx), safe = mn == -INFINITY ? 0.f : mn, alpha = exp2f(m - safe);
             float sum = 0.f;
 #pragma unroll
