@@ -475,7 +475,7 @@ __global__ __launch_bounds__(256, PER_CU) void gemm4_kernel(GemmParams p) {
     }
     long long b_off = 0, c_off = 0;
     int m0 = tmi * BM, m_end = p.M, k_begin = 0, k_len = p.K;
-    bool alone = false;   // the only tile of its expert's rows
+    bool alone = p.mode == 0 && p.M <= BM;   // the only tile of the rows, or of its expert's
     if (p.mode == 2) {
         k_begin = p.offsets[blockIdx.y];
         k_len = p.offsets[blockIdx.y + 1] - k_begin;
@@ -626,6 +626,11 @@ int split_128(long long M, long long N, long long K) {   // pieces of the reduct
 }
 // outputs of at least four column tiles and reductions of at least 12 stages: what the figures above were taken on
 bool dense_range(long long N, long long K) { return N >= 1024 && (N & 7) == 0 && K >= 768; }
+// A dense product of one tile of rows with weights beyond the Infinity Cache (256 MB) is a stream of weights like an expert's.  100352 x 2560, us by the other tiles / by
+// these: 17 rows 111 / 93, 32 118 / 98, 48 124 / 103, 64 125 / 108, 96 129 / 109, 112 135 / 116, 128 136 / 115 (two tiles of rows, 195, 154 / 193).  64000 x 1536, which the cache keeps, is level.
+bool one_pass(const GemmParams& p, int a_oc, int b_oc) {
+    return p.mode == 0 && !a_oc && !b_oc && p.M <= 128 && dense_range(p.N, p.K) && (long long)p.N * p.K >= 128 << 20 && aria_gemm3_workspace_bytes(p.M, p.N, p.K) == 0;
+}
 
 }  // namespace
 
@@ -675,6 +680,10 @@ Gemm4Plan aria_plan_gemm4(const GemmParams& p, int a_oc, int b_oc, long long row
     const long long t2 = cdiv(p.M, 128) * (p.glu ? cdiv(p.N / 2, 128) : cdiv(p.N, 256));
     if (!plain) {   // (these forms never split)
         if (t2 <= ROUND) plan.form = 1;
+        return plan;
+    }
+    if (one_pass(p, a_oc, b_oc)) {
+        plan.form = 1;
         return plan;
     }
     double best = 0.94 * time_else(p.M, p.N, n, split3);
@@ -741,7 +750,7 @@ int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, f
         return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
     // Weights by expert pass the caches where a tile is the only one of its expert's rows (gemm4_kernel): a stream of 500 MB at 6.9 TB/s for 6.2.  Tensors that the Infinity Cache keeps from one use to
     // the next lose by it: 16 experts of 1024 x 768 (25 MB) 13.8 us and 16.7.
-    const bool once = p.mode == 1 && p.expert_mod <= 0 && (long long)p.E * p.N * p.K >= 32 << 20;
+    const bool once = p.mode == 1 ? p.expert_mod <= 0 && (long long)p.E * p.N * p.K >= 32 << 20 : one_pass(p, 0, b_oc);
 #define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
 #define ARIA_G4E(BOC, VER) \
     (once ? launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1, true, true>(q, split, slabs, stream) \

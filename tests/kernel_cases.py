@@ -179,6 +179,19 @@ def case_gemm_four_waves_low(dev, monkeypatch, K, I, E):
         assert len(a) == len(b) and all(torch.equal(p, q) for p, q in zip(a, b)), i
 
 
+def case_gemm_one_pass(dev, monkeypatch, M, tiles):
+    """A product of few rows with weights beyond the Infinity Cache, on both sides of its tile's rows: the bits of the 256 x 256 tiles, in bf16 and in 32 bits, with a bias."""
+    from aria_amd import ops
+
+    N, K = 100352, 2560
+    x, w, bias = rnd(M, K, seed=M).to(dev), torch.empty(N, K, dtype=bf16, device=dev).normal_(0.0, 0.02, generator=torch.Generator(dev).manual_seed(M)), rnd(N, seed=3).to(dev)
+    got = [ops.gemm(x, w), ops.gemm(x, w, out_dtype=torch.float32), ops.gemm(x, w, bias=bias)]
+    assert (last_gemm_tiles() == 17) == tiles
+    monkeypatch.setenv("ARIA_GEMM_FORCE", "3")
+    for a, b in zip(got, [ops.gemm(x, w), ops.gemm(x, w, out_dtype=torch.float32), ops.gemm(x, w, bias=bias)]):
+        assert torch.equal(a, b)
+
+
 def case_wgrad_strips(dev, monkeypatch, counts, M, N):
     """Weight gradients in strips of 256 columns (the reduction's fragments of dY stay in registers): the bits of the 128 x 256 tiles for experts of any number of rows -- none, partial
     steps of sixteen, the 256 that are held, more -- plain, gathered and dense, and within the bound of a rounded 32-bit sum of exact products."""

@@ -151,6 +151,11 @@ def test_attention_varlen_block_rule(n, S, H, qd, waves):
     C.case_attention_varlen_block_rule(DEV, n, S, H, qd, waves)
 
 
+@pytest.mark.parametrize("M,tiles", [(9, True), (32, True), (33, True), (96, True), (128, True), (129, False)])
+def test_gemm_one_pass(monkeypatch, M, tiles):
+    C.case_gemm_one_pass(DEV, monkeypatch, M, tiles)
+
+
 @pytest.mark.parametrize("K,I,E", [(72, 128, 12), (64, 128, 12), (320, 128, 12), (256, 256, 256), (1536, 1664, 16)])
 def test_gemm_four_waves_low(monkeypatch, K, I, E):
     C.case_gemm_four_waves_low(DEV, monkeypatch, K, I, E)
