@@ -477,7 +477,8 @@ __global__ __launch_bounds__(256) void permute_rows_kernel(const bf16_t* x, cons
 // (compile-time row width, see permute_rows_kernel: the k rows of a token and the shared expert's are in flight together;
 // same arithmetic in the same order as unpermute_kernel -- bit-identical.  A wave takes 512 columns of a token: as one wave a token its five chunks' latencies followed one another.
 // Cold rows, a wave a token / a chunk, us: 1 token 14.8 / 6.8, 280 18.4 / 10.9, 777 21.2 / 18.2, 4096 74 / 70, 16 384 200 / 197)
-template <int NC, int K>
+// ONCE: rows beyond the Infinity Cache are non-temporal (rows_once)
+template <int NC, int K, bool ONCE>
 __global__ __launch_bounds__(256) void unpermute_rows_kernel(const bf16_t* eo, const int32_t* inv, const bf16_t* scores, const bf16_t* add,
                                                              const bf16_t* res, bf16_t* out, int T) {
     const int l = threadIdx.x & 63;
@@ -496,7 +497,7 @@ __global__ __launch_bounds__(256) void unpermute_rows_kernel(const bf16_t* eo, c
         const int c = l + 64 * i;
         u32x4 v[K], a = zero16();
 #pragma unroll
-        for (int j = 0; j < K; ++j) v[j] = ld16(eo + (long long)rows[j] * D + c * 8);
+        for (int j = 0; j < K; ++j) v[j] = ONCE ? ld16_once(eo + (long long)rows[j] * D + c * 8) : ld16(eo + (long long)rows[j] * D + c * 8);
         if (add) a = ld16(add + (long long)t * D + c * 8);
         float acc[8];
 #pragma unroll
@@ -533,7 +534,8 @@ __global__ __launch_bounds__(256) void unpermute_rows_kernel(const bf16_t* eo, c
 // backward of unpermute with a compile-time row width: dout's chunks are fetched ONCE per token (the generic kernel re-reads them for each of
 // the k rows), a row's NC chunks are in flight together, and the dot product's wave sum runs on the DPP ladder instead of six ds_bpermute
 // round trips per row.  d_eo is bit-identical to the generic kernel's; dscores differs from it in the order of the 64-lane sum only (the
-// per-lane partial sums are formed in the same order), within the rounding of the bf16 it is stored in.
+// per-lane partial sums are formed in the same order), within the rounding of the bf16 it is stored in.  The forward's rows, which lie in memory since then, are read non-temporally:
+// 777 tokens 18 -> 15 us, 4096 81 -> 58, 16 384 245 -> 223.
 template <int NC, int K>
 __global__ __launch_bounds__(256) void unpermute_bwd_rows_kernel(const bf16_t* dout, const bf16_t* eo, const int32_t* inv, const bf16_t* scores,
                                                                  bf16_t* d_eo, bf16_t* dscores, int T) {
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(256) void unpermute_bwd_rows_kernel(const bf16_t* d
         for (int j = 0; j < K; ++j) {
             u32x4 v[NC];
 #pragma unroll
-            for (int i = 0; i < NC; ++i) v[i] = ld16(eo + (long long)rows[j] * D + (l + 64 * i) * 8);
+            for (int i = 0; i < NC; ++i) v[i] = ld16_once(eo + (long long)rows[j] * D + (l + 64 * i) * 8);
             float dot = 0.f;
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
@@ -807,6 +809,10 @@ int grid_for_waves(long long n_items, int waves_per_block = 4) {
     return int(g);
 }
 
+// Whether so many rows of D that the launch before wrote are read non-temporally: more than the Infinity Cache still holds most of.  Experts' rows of 2560 back to tokens, us, plain / non-temporal:
+// 3000 tokens (92 MB) 23 / 28, 4096 29 / 34, 6144 (189 MB) 42 / 42.5, 7168 50.7 / 48.7, 8192 59 / 55, 16 384 144 / 107.
+bool rows_once(int64_t rows, int64_t D) { return 2 * rows * D >= 192ll << 20; }
+
 }  // namespace
 
 // Routing of T tokens and the sorted order of their choices, for the prompt step (prompt.hip): bf16 logits, E <= 64, T k <= 8192, counts zeroed by the caller
@@ -917,10 +923,13 @@ int aria_moe_unpermute_res(const void* expert_out, const int32_t* inv, const voi
     if (T == 0) return ARIA_OK;
     const bf16_t *eo = static_cast<const bf16_t*>(expert_out), *sc = static_cast<const bf16_t*>(scores), *ad = static_cast<const bf16_t*>(add);
     const bf16_t* rs = static_cast<const bf16_t*>(residual);
-    if (D == 2560 && k == 6 && !generic_dispatch_kernels())   // Aria's width and top-k: compile-time row width, everything in flight together
-        ARIA_LAUNCH((unpermute_rows_kernel<5, 6>), dim3(grid_for_waves(5 * T)), dim3(256), 0, stream, eo, inv, sc, ad, rs, static_cast<bf16_t*>(out), int(T));
-    else if (D == 512 && k == 2 && !generic_dispatch_kernels())   // (the same template at a width the CPU suite runs)
-        ARIA_LAUNCH((unpermute_rows_kernel<1, 2>), dim3(grid_for_waves(T)), dim3(256), 0, stream, eo, inv, sc, ad, rs, static_cast<bf16_t*>(out), int(T));
+    if (D == 2560 && k == 6 && !generic_dispatch_kernels()) {   // Aria's width and top-k: compile-time row width, everything in flight together
+        if (rows_once(T * k, D))
+            ARIA_LAUNCH((unpermute_rows_kernel<5, 6, true>), dim3(grid_for_waves(5 * T)), dim3(256), 0, stream, eo, inv, sc, ad, rs, static_cast<bf16_t*>(out), int(T));
+        else
+            ARIA_LAUNCH((unpermute_rows_kernel<5, 6, false>), dim3(grid_for_waves(5 * T)), dim3(256), 0, stream, eo, inv, sc, ad, rs, static_cast<bf16_t*>(out), int(T));
+    } else if (D == 512 && k == 2 && !generic_dispatch_kernels())   // (the same template at a width the CPU suite runs)
+        ARIA_LAUNCH((unpermute_rows_kernel<1, 2, false>), dim3(grid_for_waves(T)), dim3(256), 0, stream, eo, inv, sc, ad, rs, static_cast<bf16_t*>(out), int(T));
     else
         ARIA_LAUNCH((unpermute_kernel<8>), dim3(grid_for_waves(T)), dim3(256), 0, stream, eo, inv, sc, ad, static_cast<bf16_t*>(out), int(T), int(D),
                     int(k));

@@ -416,6 +416,23 @@ def case_unpermute_with_residual(dev, T, D, k, E=8):
         assert torch.equal(got.cpu(), want.cpu()), float((got.float() - want.float()).abs().max())
 
 
+def case_unpermute_rows_form(dev, monkeypatch, T):
+    """Experts' rows of 2560 back to tokens and their gradients on both sides of the rows that are read past the caches: the generic kernels' bits (dscores: another order of a 64-lane sum of 2560
+    products, at most 2560 2^-24 of the sum of magnitudes before its rounding to bf16, 2^-9)."""
+    from aria_amd import ops
+
+    g, D, k = torch.Generator().manual_seed(T), 2560, 6
+    inv = torch.randperm(T * k, generator=g).to(torch.int32).to(dev)
+    eo, sh, dout = rnd(T * k, D, seed=1).to(dev), rnd(T, D, seed=2).to(dev), rnd(T, D, seed=3).to(dev)
+    scores = torch.rand(T, k, generator=g).to(bf16).to(dev)
+    run = lambda: (ops.moe_unpermute(eo, inv, scores, k, add=sh), *ops.moe_unpermute_bwd(dout, eo, inv, scores, k))
+    got = run()
+    monkeypatch.setenv("ARIA_MOE_GENERIC_DISPATCH", "1")
+    want = run()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert float((got[2].double() - want[2].double()).norm() / want[2].double().norm()) < 2.0 ** -8
+
+
 def case_layernorm_two_rows_in_flight(dev, T, D):
     """r05b: ``layernorm_fwd2_kernel`` (two rows in flight per wave, compile-time row width; the frozen ViT's LayerNorms) gives the bits of the
     one-row-at-a-time kernel (ARIA_LAYERNORM_V1=1): y, mean, rstd -- odd row counts and rows past the grid's last pair included."""

@@ -427,6 +427,11 @@ def test_gemm_split_k_slabs_in_accumulator_order(M, N, K, a_oc, b_oc):
     C.case_gemm_split_k_slabs(DEV, M, N, K, a_oc, b_oc)
 
 
+@pytest.mark.parametrize("T", [1, 777, 6553, 6554])
+def test_unpermute_rows_form(monkeypatch, T):
+    C.case_unpermute_rows_form(DEV, monkeypatch, T)
+
+
 @pytest.mark.parametrize("T,D,k", [(16384, 2560, 6), (70, 512, 2), (33, 128, 3)])
 def test_unpermute_with_the_residual_add_as_its_last_step(T, D, k):
     C.case_unpermute_with_residual(DEV, T, D, k, E=8 if k < 6 else 64)
