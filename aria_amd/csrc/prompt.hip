@@ -1,5 +1,5 @@
 // A serving step over short prompts of the gptfast (Aria) decoder in one call: packed tokens of one or several sequences, the products by the row-streaming kernels
-// of wide.hip, by the tiles of gemm4.hip from 193 tokens on, the experts' by what is ahead.  At these sizes a layer is fifteen launches of 5 .. 230 us;
+// of wide.hip, by the tiles of gemm4.hip from 193 tokens on, the experts' from 9 (down-projections: five) rows an expert on.  At these sizes a layer is fifteen launches of 5 .. 230 us;
 // enqueued one by one from Python they take longer than they run (four layers, 280 tokens: 3.2 ms of host time for 2.5 ms of kernels).
 // Served: what wide.hip's products take, up to 27 rows an expert on average (6 of 64 experts: 288 tokens).
 #include "decode.h"
@@ -47,7 +47,7 @@ Scratch layout(const int64_t* dims, int64_t T, char* base) {
 }
 bool prompt_ok(const int64_t* d, int64_t T) {
     const int64_t D = d[1], E = d[4], k = d[5], I = d[6], Is = d[7];
-    return aria_decode_dims_ok(d) == ARIA_OK && E <= 64 && k >= 1 && k <= E && T * k <= std::min<int64_t>(8192, 27 * E) && D >= 512 && D <= 2560 && I >= 512 && I <= 2560 && Is <= 4096 &&
+    return aria_decode_dims_ok(d) == ARIA_OK && E <= 64 && k >= 1 && k <= E && T * k <= std::min<int64_t>(8192, aria_rows_experts_most(E, I, D, ARIA_ROWS_PAIR_ONLY)) && D >= 512 && D <= 2560 && I >= 512 && I <= 2560 && Is <= 4096 &&
            D % 16 == 0;
 }
 
@@ -84,10 +84,10 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         if (tiles_ahead(T, N, K)) return aria_gemm_own_cut(a, w, out, T, N, K, z.ws_bytes ? z.ws : nullptr, z.ws_bytes, stream);
         return aria_rows_gemm(a, w, out, 0, T, N, K, K, N, stream);
     };
-    // gate and up of the experts (ops.experts_tiles_ahead): tiles where all of theirs are one round
+    // (the line between rows and tiles by expert: wide.hip)
     auto expert_pairs = [&](const void* gate, const void* up) {
         int r = ARIA_ERR_UNSUPPORTED;
-        if (T * k > 8 * E && E * I * D >= 1 << 25 && E * ((I + 127) / 128) <= 256) r = aria_expert_pair_tiles(z.h, z.rows, T, gate, up, z.act, z.offsets, E, T * k, I, D, D, stream);
+        if (T * k > aria_rows_experts_most(E, I, D, ARIA_ROWS_PAIR)) r = aria_expert_pair_tiles(z.h, z.rows, T, gate, up, z.act, z.offsets, E, T * k, I, D, D, stream);
         return r != ARIA_ERR_UNSUPPORTED ? r : aria_rows_experts(z.h, z.rows, z.offsets, gate, up, z.act, E, T * k, I, D, D, I, stream);
     };
 #define ARIA_TRY(call) \
@@ -111,7 +111,7 @@ int aria_prompt_step(const void* const* ptrs, const int64_t* dims, float eps, in
         ARIA_TRY(aria_rows_gemm(z.h, p[4], z.logits, 0, T, E, D, D, E, stream));
         ARIA_TRY(aria_route_and_sort(z.logits, z.scores, z.idx, z.counts + li * E, z.offsets, z.src, z.inv, z.rows, int(T), int(E), int(k), stream));
         ARIA_TRY(expert_pairs(p[5], p[6]));
-        if (T * k <= 10 * E) {   // (beyond: the tiles, ops.ROWS_PER_EXPERT_DOWN)
+        if (T * k <= aria_rows_experts_most(E, D, I, ARIA_ROWS_DOWN)) {
             ARIA_TRY(aria_rows_experts(z.act, nullptr, z.offsets, p[7], nullptr, z.eo, E, T * k, D, I, I, D, stream));
         } else {
             ARIA_TRY(aria_grouped_gemm_bf16(z.act, p[7], z.eo, z.offsets, E, T * k, D, I, 0, I, I, D * I, D, stream));

@@ -7,7 +7,7 @@
 // 57 / 48, 31 / 24; lm_head of one token 140 / 86.
 // Routed experts: with n tokens an expert's matrix meets n k / E rows (26 at 280 tokens, 6 of 64 experts); its rows are read once per 64 of them, by whole lines that are non-temporal
 // (rows.h).  Up pairs (64 experts of 2 x 1664 x 2560), half lines / whole: 24 tokens 174 / 151, 64 204 / 172, 128 220 / 180, 280 238 / 193 (5.6 TB/s of weights); 32 of 2 x 1024 x 1536, 4 a
-// token: 64 tokens 43 / 34, 280 58 / 52.  Down (2560 x 1664): 24 tokens 93 / 77, 64 109 / 89, 280 130 / 116.  Which is ahead of the tiles where: ops.py.
+// token: 64 tokens 43 / 34, 280 58 / 52.  Down (2560 x 1664): 24 tokens 93 / 77, 64 109 / 89, 280 130 / 116.  The line to the tiles: aria_rows_experts_most.
 #include "rows.h"
 
 namespace {
@@ -191,6 +191,16 @@ int aria_rows_qkv_rope_cache(const void* X, const void* Wqkv, void* Q, void* Kc,
     const RowsIn in{static_cast<const bf16_t*>(Wqkv), nullptr, static_cast<const bf16_t*>(X), (long long)ldx, int(K), int(3 * D)};
     return launch_rows_wide<false>(in, M, QkvCache{static_cast<bf16_t*>(Q), static_cast<bf16_t*>(Kc), static_cast<bf16_t*>(Vc),
                                                    static_cast<const bf16_t*>(freqs_cis), slot, pos, (long long)S_cache, int(D), int(hd)}, stream);
+}
+
+// The line between rows by expert and tiles.  Gate and up, launches of one kind in turn, us by rows / tiles: 64 experts of 1664 x 2560: 6 rows an expert 162 / 182, 12 180 / 184, 16 180 / 186, 20
+// 200 / 187, 28 205 / 192, 40 230 / 199; 32 of 1024 x 1536: 8 33.1 / 34.3, 10 39.2 / 35.0, 20 42.6 / 35.8, 40 48.8 / 36.9.  Fewer weights are a launch's ramp: 16 of 768 x 1024: 12 14.1 / 16.0, 28
+// 15.9 / 17.2, 40 16.4 / 18.3.  Down: 64 experts 6 88.0 / 89.5, 10 89.3 / 90.6, 12 93.8 / 90.7, 16 114 / 92; 32: 8 19.5 / 19.0, 12 23.4 / 19.5; 16: 10 10.5 / 11.4, 16 13.1 / 11.7.
+// A prompt's outputs hold to where the line lay when the tiles were slower, 8 and 4 rows: rows add in another order, which moves an Aria prompt's logits by 0.7 % at the same error against 64 bits.
+// Its four layers by rows up to 27 and 10 rows / by this line: 86 tokens 1706 / 1768, 130 1833 / 1858, 200 1890 / 1932, 240 1926 / 1973, 280 2060 / 2038.
+int64_t aria_rows_experts_most(int64_t E, int64_t N, int64_t K, int which) {
+    if (which == ARIA_ROWS_DOWN) return 4 * E;
+    return which == ARIA_ROWS_PAIR && E * N * K >= 1 << 25 ? 8 * E : 27 * E;
 }
 
 int aria_rows_experts(const void* X, const int32_t* rows, const int32_t* offsets, const void* W, const void* Wu, void* out, int64_t E, int64_t M, int64_t N,

@@ -25,7 +25,7 @@ P, I64, I32, F32 = c_void_p, c_int64, c_int, c_float
 RESTYPES = {"aria_gemm_workspace_bytes": c_int64, "aria_decode_scratch_bytes": c_int64, "aria_decode_step_scratch": c_int64, "aria_prompt_step_scratch": c_int64, "aria_decode_graph_create": c_void_p,
             "aria_decode_graph_destroy": None, "aria_decode_attn_workspace_bytes": c_int64,
             "aria_latent_decode_scratch": c_int64, "aria_latent_splits": c_int64, "aria_linear_chunks_scratch": c_int64, "aria_mix_decode_scratch": c_int64,
-            "aria_chunk_decode_scratch": c_int64,
+            "aria_chunk_decode_scratch": c_int64, "aria_rows_experts_most": c_int64,
             "aria_latent_splits_f32": c_int64, "aria_latent_step_f32_scratch": c_int64, "aria_mix_step_f32_scratch": c_int64}  # everything else returns an int status
 
 # name -> argtypes (all return int).  Kept in one table so tests can check that the shared
@@ -43,6 +43,7 @@ SIGNATURES = {
     "aria_rows_gemm": [P, P, P, I32, I64, I64, I64, I64, I64, P],
     "aria_rows_swiglu": [P, P, P, P, I64, I64, I64, I64, I64, P],
     "aria_rows_qkv_rope_cache": [P, P, P, P, P, P, P, P, I64, I64, I64, I64, I64, I64, P],
+    "aria_rows_experts_most": [I64, I64, I64, I32],
     "aria_rows_experts": [P, P, P, P, P, P, I64, I64, I64, I64, I64, I64, P],
     "aria_prompt_step_scratch": [P, I64],
     "aria_prompt_step": [P, P, F32, I64, P, P, P, P, I64, I64, P, I64, P, P, I64, P],

@@ -51,10 +51,7 @@ ROWS_TOKENS = 320      # x 7680 x 2560: 280 tokens 37 us, tiles 44; 320: 40, 44;
 # 120, 119; 320: 405, 212.  7680 x 4096: 96 tokens 35, 36; 128: 44, 37.  2560 x 4096: 256 tokens 30, 34; 320: 38, 36.  Level up to the line: 10240 x 2560: 200
 # tokens 39, 39; 300: 52, 51 -- by rows with 8 us of the host's time, by tiles 15; 2560 x 3328: 320 tokens 33, 34, in a model 7 us ahead (300 tokens, four layers, 2540 us against 2569).
 ROWS_PASSED, ROWS_PASSED_LONG = 52000, 26000
-# Rows of an expert on average, gate and up pairs.  Launches of one kind in turn, us by rows / tiles: 64 experts of 1664 x 2560: 6 rows 162, 182; 12 180, 184; 16 180, 186; 20 200, 187; 28 205, 192; 40
-# 230, 199.  16 of 768 x 1024: 16 rows 15.6, 16.5; 40 16.4, 18.3.  In a prompt of 280 tokens (26 rows) they take 184 us by rows; by tiles its four layers are 1998 us for 1945.
-ROWS_PER_EXPERT = 27
-ROWS_PER_EXPERT_DOWN = 10   # down projections of 64 experts: 6 rows 88.0, 89.5; 10: 89.3, 90.6; 12: 93.8, 90.7; 16: 114, 92; of 32: 8 19.5, 19.0; 12 23.4, 19.5; of 16: 10 10.5, 11.4; 16 13.1, 11.7
+ROWS_PAIR_ONLY, ROWS_PAIR, ROWS_DOWN = 0, 1, 2   # which products of experts (the C ABI's constants)
 
 
 def rows_take(M: int, K: int, N: int) -> bool:
@@ -63,16 +60,20 @@ def rows_take(M: int, K: int, N: int) -> bool:
             and (M <= 16 or (N * -(-M // 64) <= ROWS_PASSED if K <= 2560 else N * -(-M // 32) <= ROWS_PASSED_LONG)))
 
 
+def rows_experts_most(E: int, K: int, N: int, which: int) -> int:
+    """Up to how many rows of all experts their products go by rows: the line itself, and its reasons, are the library's, whose prompt step goes by it too."""
+    return hip.get_lib().cdll.aria_rows_experts_most(E, N, K, which)
+
+
 def rows_experts_take(M: int, E: int, K: int, N: int, down: bool = False) -> bool:
     """``rows_experts`` for M rows sorted by expert, w [E, N, K]"""
-    return (0 < M <= (ROWS_PER_EXPERT_DOWN if down else ROWS_PER_EXPERT) * E and E <= 256 and min(K, N) >= 512 and max(K, N) <= 2560 and K % 8 == 0
+    return (0 < M <= rows_experts_most(E, K, N, ROWS_DOWN if down else ROWS_PAIR_ONLY) and E <= 256 and min(K, N) >= 512 and max(K, N) <= 2560 and K % 8 == 0
             and N % 8 == 0)
 
 
 def experts_tiles_ahead(M: int, E: int, K: int, N: int) -> bool:
-    """Whether the gathered tiles of gate and up are ahead of the rows by expert up to ROWS_PER_EXPERT: where all of them are one round, and the weights more than a launch's ramp.
-    us by rows / tiles, rows an expert: 32 of 1024 x 1536: 8 33.1 / 34.3, 10 39.2 / 35.0, 20 42.6 / 35.8, 40 48.8 / 36.9; 16 of 768 x 1024: 12 14.1 / 16.0, 28 15.9 / 17.2."""
-    return M > 8 * E and E * K * N >= 1 << 25 and E * -(-N // 128) <= 256
+    """Whether the gathered tiles of gate and up, where they can run, are ahead of the rows by expert."""
+    return M > rows_experts_most(E, K, N, ROWS_PAIR)
 
 
 def rows_gemm(x: torch.Tensor, w: torch.Tensor, out_dtype=bf16) -> torch.Tensor:

@@ -450,7 +450,13 @@ int aria_cross_entropy(const void* logits, const int32_t* labels, float* loss_su
  * aria_rows_qkv_rope_cache: as aria_gemm_qkv_rope_cache_bf16 on caches [slots, S_cache, D]: token t is position pos[t] of slot[t] (both NULL: position t of
  *   the only slot); Q [M, D].
  * aria_rows_experts: rows sorted by expert (offsets int32 [E + 1] on the device), place i reads X row rows[i] (NULL: i); W [E, N, K]; with Wu the
- *   SwiGLU pair. */
+ *   SwiGLU pair.
+ * aria_rows_experts_most: up to how many rows of E experts together their products by weights [N, K] go by rows rather than by tiles: gate and up where their tiles
+ *   can run (PAIR) or cannot (PAIR_ONLY), down-projections. */
+#define ARIA_ROWS_PAIR_ONLY 0
+#define ARIA_ROWS_PAIR 1
+#define ARIA_ROWS_DOWN 2
+int64_t aria_rows_experts_most(int64_t E, int64_t N, int64_t K, int which);
 int aria_rows_gemm(const void* X, const void* W, void* out, int out_f32, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldo, void* stream);
 int aria_rows_swiglu(const void* X, const void* Wg, const void* Wu, void* act, int64_t M, int64_t I, int64_t K, int64_t ldx, int64_t ldact, void* stream);
 int aria_rows_qkv_rope_cache(const void* X, const void* Wqkv, void* Q, void* Kc, void* Vc, const void* freqs_cis, const int32_t* slot, const int32_t* pos,

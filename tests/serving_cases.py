@@ -588,6 +588,22 @@ def case_rows_rule():
             assert taken == sorted(taken, reverse=True)
 
 
+def case_experts_line():
+    """Rows or tiles by expert: Aria's prompts of 86 .. 288 tokens have gate and up by tiles, of 43 .. 288 the down-projections, as their outputs' bits want it; small
+    experts stay by rows; one line for the modules and the prompt step."""
+    from aria_amd import ops
+
+    E, K, N = 64, 2560, 1664
+    for tokens, pair_tiles, down_rows in ((42, False, True), (43, False, False), (85, False, False), (86, True, False), (280, True, False), (288, True, False)):
+        assert ops.rows_experts_take(6 * tokens, E, K, N) and ops.experts_tiles_ahead(6 * tokens, E, K, N) == pair_tiles, tokens
+        assert ops.rows_experts_take(6 * tokens, E, N, K, down=True) == down_rows, tokens
+    assert not ops.rows_experts_take(6 * 289, E, K, N)
+    for M, taken in ((8 * 32, False), (8 * 32 + 1, True)):      # 32 of 1024 x 1536
+        assert ops.experts_tiles_ahead(M, 32, 1536, 1024) == taken
+    assert not ops.experts_tiles_ahead(27 * 16, 16, 1024, 768) and ops.rows_experts_take(27 * 16, 16, 1024, 768)
+    assert not ops.rows_experts_take(27 * 16 + 1, 16, 1024, 768)
+
+
 def case_gptfast_packed_prompts(dev, dim=256, lens=(9, 1, 40, 17), inter=128):
     """Prompts of several requests packed into one step against each prompt alone, logits at places inside and at the end, and a step on the caches that they
     left; rounding as in ``case_gptfast_decode_batch`` (the flash kernel's probabilities included)."""

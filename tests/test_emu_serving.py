@@ -91,6 +91,10 @@ def test_rows_rule():
     C.case_rows_rule()
 
 
+def test_experts_line():
+    C.case_experts_line()
+
+
 def test_gptfast_steps_oracle(monkeypatch):
     C.case_gptfast_steps_oracle(DEV, monkeypatch, 512, 512, (3, 1, 5))
 
