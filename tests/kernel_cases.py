@@ -1134,6 +1134,47 @@ def case_cross_entropy(dev, T, V):
     close(dl, lf.grad, 2e-2, 1e-4)
 
 
+def case_cross_entropy_in_place(dev, T, V):
+    """The gradient in the logits' place, as training has it: the loss and the gradient of separate buffers, also where the label's column is rewritten first or last."""
+    from aria_amd import ops
+
+    logits = rnd(T, V, seed=42, scale=2.0).to(dev)
+    labels = torch.randint(0, V, (T,), generator=torch.Generator().manual_seed(43)).to(torch.int32)
+    labels[:4] = torch.tensor([0, V - 1, 7, V // 2], dtype=torch.int32)
+    labels[5::7] = -100
+    labels = labels.to(dev)
+    for t in range(T):   # (a row alone: its loss is one number, not a sum whose order the rows' ends decide)
+        row, dl = logits[t:t + 1].clone(), torch.empty(1, V, dtype=torch.bfloat16, device=dev)
+        want = [x.clone() for x in ops.cross_entropy(row, labels[t:t + 1], grad_scale=1.0, dlogits=dl)[:2]]
+        got = ops.cross_entropy(row, labels[t:t + 1], grad_scale=1.0, dlogits=row)[:2]
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and torch.equal(row, dl), t
+    together = logits.clone()
+    loss, n, _ = ops.cross_entropy(together, labels, grad_scale=1.0, dlogits=together)
+    apart = torch.empty_like(logits)
+    loss_apart, n_apart, _ = ops.cross_entropy(logits, labels, grad_scale=1.0, dlogits=apart)
+    assert int(n.cpu()) == int(n_apart.cpu()) == int((labels >= 0).sum())
+    assert torch.equal(together, apart)
+    close(loss.cpu(), loss_apart.cpu(), 1e-5, 0)   # (atomic sums: T roundings of 2^-24)
+
+
+def case_cross_entropy_order(dev, chunks):
+    """A row's sums are threads' over every 256th chunk of eight columns: 256 chunks of -inf in its middle, which add nothing and leave every other chunk with its thread, leave the loss
+    and the gradient as they are, bit for bit."""
+    from aria_amd import ops
+
+    V = 8 * 256 * chunks
+    for seed in range(24):
+        row = rnd(1, V, seed=100 + seed, scale=1.0) - 11   # (one column of 0: a sum of about 2, whose last bit shows in its logarithm)
+        row[0, 5] = 0
+        wide = torch.cat([row[:, :2048], torch.full((1, 2048), -float("inf"), dtype=row.dtype), row[:, 2048:]], 1)
+        out = []
+        for x in (row.to(dev), wide.to(dev)):
+            loss, _, _ = ops.cross_entropy(x, torch.tensor([5], dtype=torch.int32, device=dev), grad_scale=1.0, dlogits=x)
+            out.append((loss.cpu().clone(), x.cpu()))
+        assert torch.equal(out[0][0], out[1][0]), (seed, out[0][0], out[1][0])
+        assert torch.equal(out[0][1], torch.cat([out[1][1][:, :2048], out[1][1][:, 4096:]], 1)) and not out[1][1][:, 2048:4096].any(), seed
+
+
 def case_attention_hd72_forward(dev, B, Sq, Skv, H, masked):
     """native head_dim 72 forward (frozen ViT / projector): reduction padded to 80 in LDS, output tiles 32+32+8."""
     from aria_amd import ops

@@ -88,6 +88,16 @@ def test_cross_entropy(T, V):
     C.case_cross_entropy(DEV, T, V)
 
 
+@pytest.mark.parametrize("T,V", [(5, 8), (9, 2056), (40, 100352)])
+def test_cross_entropy_in_place(T, V):
+    C.case_cross_entropy_in_place(DEV, T, V)
+
+
+@pytest.mark.parametrize("chunks", [2, 17, 48])
+def test_cross_entropy_order(chunks):
+    C.case_cross_entropy_order(DEV, chunks)
+
+
 @pytest.mark.parametrize("B,S,H,hd,causal,use_len", [(2, 70, 2, 64, True, False), (1, 200, 1, 64, False, True),
                                                      (1, 130, 1, 128, True, False), (2, 64, 1, 64, False, False),
                                                      (2, 1024, 3, 128, True, False), (3, 1225, 2, 128, False, True),
