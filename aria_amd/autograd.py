@@ -291,6 +291,7 @@ class DecoderLayerFn(torch.autograd.Function):
         elif level is not None:
             _, c = Fn.decoder_layer_fwd(x, p, cos, sin, B, S, acfg, mcfg, eps, kv_len, save=True,
                                         attn_cache=None if c is None else c.get("attn_cache"))
+            c["mctx"]["recent"] = True
         wanted = {k for k, w in zip(_LAYER_KEYS, ctx.needs_input_grad[10:]) if w}   # frozen parameters: no weight-gradient GEMM
         dx, g = Fn.decoder_layer_bwd(_c(dout), c, p, cos, sin, None if len(wanted) == len(_LAYER_KEYS) else wanted)
         ctx.c = None
@@ -337,6 +338,7 @@ class LoraDecoderLayerFn(torch.autograd.Function):
             L = {k: LF.LoraSite(ab_in[2 * i], ab_in[2 * i + 1], ctx.hyper[i][0], ctx.hyper[i][1]) for i, k in enumerate(ctx.keys)}
             with torch.no_grad():
                 _, c = LF.decoder_layer_lora_fwd(x, p, L, cos, sin, B, S, acfg, mcfg, eps, kv_len, training, seed)
+            c["recent"] = True
             LoraDecoderLayerFn.forward_calls += 1
         n0 = 14
         need = {k for k, w in zip(_LAYER_KEYS, ctx.needs_input_grad[n0:n0 + len(_LAYER_KEYS)]) if w}

@@ -534,9 +534,9 @@ __global__ __launch_bounds__(256) void unpermute_rows_kernel(const bf16_t* eo, c
 // backward of unpermute with a compile-time row width: dout's chunks are fetched ONCE per token (the generic kernel re-reads them for each of
 // the k rows), a row's NC chunks are in flight together, and the dot product's wave sum runs on the DPP ladder instead of six ds_bpermute
 // round trips per row.  d_eo is bit-identical to the generic kernel's; dscores differs from it in the order of the 64-lane sum only (the
-// per-lane partial sums are formed in the same order), within the rounding of the bf16 it is stored in.  The forward's rows, which lie in memory since then, are read non-temporally:
-// 777 tokens 18 -> 15 us, 4096 81 -> 58, 16 384 245 -> 223.
-template <int NC, int K>
+// per-lane partial sums are formed in the same order), within the rounding of the bf16 it is stored in.
+// ONCE: rows that lie in memory, or beyond the Infinity Cache, are non-temporal (gradient_rows_once)
+template <int NC, int K, bool ONCE>
 __global__ __launch_bounds__(256) void unpermute_bwd_rows_kernel(const bf16_t* dout, const bf16_t* eo, const int32_t* inv, const bf16_t* scores,
                                                                  bf16_t* d_eo, bf16_t* dscores, int T) {
     const int l = threadIdx.x & 63;
@@ -558,7 +558,7 @@ __global__ __launch_bounds__(256) void unpermute_bwd_rows_kernel(const bf16_t* d
         for (int j = 0; j < K; ++j) {
             u32x4 v[NC];
 #pragma unroll
-            for (int i = 0; i < NC; ++i) v[i] = ld16_once(eo + (long long)rows[j] * D + (l + 64 * i) * 8);
+            for (int i = 0; i < NC; ++i) v[i] = ONCE ? ld16_once(eo + (long long)rows[j] * D + (l + 64 * i) * 8) : ld16(eo + (long long)rows[j] * D + (l + 64 * i) * 8);
             float dot = 0.f;
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
@@ -812,6 +812,32 @@ int grid_for_waves(long long n_items, int waves_per_block = 4) {
 // Whether so many rows of D that the launch before wrote are read non-temporally: more than the Infinity Cache still holds most of.  Experts' rows of 2560 back to tokens, us, plain / non-temporal:
 // 3000 tokens (92 MB) 23 / 28, 4096 29 / 34, 6144 (189 MB) 42 / 42.5, 7168 50.7 / 48.7, 8192 59 / 55, 16 384 144 / 107.
 bool rows_once(int64_t rows, int64_t D) { return 2 * rows * D >= 192ll << 20; }
+// The same in the backward pass, where a forward's rows lie in memory since then; only rows that were computed anew just before are still held.  Rows of 2560, six a token, us, plain / non-temporal,
+// from memory: 280 tokens 12.6 / 11.1, 777 18 / 14, 3000 58 / 41, 4096 77 / 54, 8192 128 / 104, 16 384 237 / 212; just written: 64 14.1 / 14.7, 777 16.1 / 19.4, 1500 18.2 / 19.4, 3000 33 / 37, 4096
+// (126 MB) 47 / 50, 6144 (189 MB) 72 / 65, 8192 100 / 83, 16 384 213 / 188.
+bool gradient_rows_once(int64_t rows, int64_t D, bool recent) { return !recent || 2 * rows * D >= 144ll << 20; }
+
+int unpermute_bwd(const void* dout, const void* expert_out, const int32_t* inv, const void* scores, void* d_expert_out, void* dscores, int64_t T, int64_t D, int64_t k, bool recent,
+                  void* stream) {
+    if (!dout || !expert_out || !inv || !scores || !d_expert_out || !dscores || T < 0 || D <= 0 || k <= 0) return ARIA_ERR_INVALID;
+    if (D & 7) return ARIA_ERR_ALIGN;
+    if (T == 0) return ARIA_OK;
+    const bf16_t *g = static_cast<const bf16_t*>(dout), *eo = static_cast<const bf16_t*>(expert_out), *sc = static_cast<const bf16_t*>(scores);
+    bf16_t *d_eo = static_cast<bf16_t*>(d_expert_out), *ds = static_cast<bf16_t*>(dscores);
+#define ARIA_ROWS(NC, K, ONCE) ARIA_LAUNCH((unpermute_bwd_rows_kernel<NC, K, ONCE>), dim3(grid_for_waves(T)), dim3(256), 0, stream, g, eo, inv, sc, d_eo, ds, int(T))
+    if (D == 2560 && k == 6 && !generic_dispatch_kernels()) {
+        if (gradient_rows_once(T * k, D, recent))
+            ARIA_ROWS(5, 6, true);
+        else
+            ARIA_ROWS(5, 6, false);
+    } else if (D == 512 && k == 2 && !generic_dispatch_kernels()) {
+        ARIA_ROWS(1, 2, false);
+    } else {
+        ARIA_LAUNCH(unpermute_bwd_kernel, dim3(grid_for_waves(T)), dim3(256), 0, stream, g, eo, inv, sc, d_eo, ds, int(T), int(D), int(k));
+    }
+#undef ARIA_ROWS
+    return aria_check_launch();
+}
 
 }  // namespace
 
@@ -938,20 +964,12 @@ int aria_moe_unpermute_res(const void* expert_out, const int32_t* inv, const voi
 
 int aria_moe_unpermute_bwd(const void* dout, const void* expert_out, const int32_t* inv, const void* scores, void* d_expert_out,
                            void* dscores, int64_t T, int64_t D, int64_t k, void* stream) {
-    if (!dout || !expert_out || !inv || !scores || !d_expert_out || !dscores || T < 0 || D <= 0 || k <= 0) return ARIA_ERR_INVALID;
-    if (D & 7) return ARIA_ERR_ALIGN;
-    if (T == 0) return ARIA_OK;
-    const bf16_t *g = static_cast<const bf16_t*>(dout), *eo = static_cast<const bf16_t*>(expert_out), *sc = static_cast<const bf16_t*>(scores);
-    if (D == 2560 && k == 6 && !generic_dispatch_kernels())
-        ARIA_LAUNCH((unpermute_bwd_rows_kernel<5, 6>), dim3(grid_for_waves(T)), dim3(256), 0, stream, g, eo, inv, sc, static_cast<bf16_t*>(d_expert_out),
-                    static_cast<bf16_t*>(dscores), int(T));
-    else if (D == 512 && k == 2 && !generic_dispatch_kernels())
-        ARIA_LAUNCH((unpermute_bwd_rows_kernel<1, 2>), dim3(grid_for_waves(T)), dim3(256), 0, stream, g, eo, inv, sc, static_cast<bf16_t*>(d_expert_out),
-                    static_cast<bf16_t*>(dscores), int(T));
-    else
-        ARIA_LAUNCH(unpermute_bwd_kernel, dim3(grid_for_waves(T)), dim3(256), 0, stream, g, eo, inv, sc, static_cast<bf16_t*>(d_expert_out),
-                    static_cast<bf16_t*>(dscores), int(T), int(D), int(k));
-    return aria_check_launch();
+    return unpermute_bwd(dout, expert_out, inv, scores, d_expert_out, dscores, T, D, k, false, stream);
+}
+
+int aria_moe_unpermute_bwd_recent(const void* dout, const void* expert_out, const int32_t* inv, const void* scores, void* d_expert_out, void* dscores, int64_t T, int64_t D,
+                                  int64_t k, void* stream) {
+    return unpermute_bwd(dout, expert_out, inv, scores, d_expert_out, dscores, T, D, k, true, stream);
 }
 
 int aria_moe_route_bwd(const void* logits, const int32_t* indices, const void* scores, const void* dscores, const int32_t* counts,

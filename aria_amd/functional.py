@@ -159,7 +159,7 @@ def moe_rematerialize(ctx, fc1, fc2) -> None:
         else:
             h1 = ops.grouped_gemm(perm, fc1, ctx["offsets"])
             act = ops.swiglu(h1)
-    ctx.update(perm=perm, h1=h1, act=act, eo=ops.grouped_gemm(act, fc2, ctx["offsets"]))
+    ctx.update(perm=perm, h1=h1, act=act, eo=ops.grouped_gemm(act, fc2, ctx["offsets"]), recent=True)
 
 
 def _want(need, *keys) -> bool:
@@ -174,7 +174,7 @@ def moe_bwd(dout, ctx, router_w, fc1, fc2, gate_w, up_w, down_w, need=None):
     x, inv, offsets = ctx["x"], ctx["inv"], ctx["offsets"]
     I2 = gate_w.shape[0]
     # routed experts
-    d_eo, dscores = ops.moe_unpermute_bwd(dout, ctx["eo"], inv, ctx["scores"], k)
+    d_eo, dscores = ops.moe_unpermute_bwd(dout, ctx["eo"], inv, ctx["scores"], k, ctx.get("recent", False))
     if ops.dglu_fusable(fc2.shape[1], fc2.shape[2]):                 # fc2's input gradient + the backward of glu in ONE launch
         d_h1 = ops.grouped_gemm_dswiglu(d_eo, fc2, offsets, ctx["h1"])
     else:

@@ -242,7 +242,7 @@ def decoder_layer_lora_bwd(dout, c, p: dict, cos, sin, need_base=None) -> Tuple[
     hn, offsets, inv = c["hn"], c["offsets"], c["inv"]
     I2 = p["gate"].shape[0]
     # ---- MoE block: routed experts
-    d_eo, dscores = ops.moe_unpermute_bwd(dout, c["eo"], inv, c["scores"], k)
+    d_eo, dscores = ops.moe_unpermute_bwd(dout, c["eo"], inv, c["scores"], k, c.get("recent", False))
     if c["c_fc2"] is None and ops.dglu_fusable(p["fc2"].shape[1], p["fc2"].shape[2]):
         d_h1 = ops.grouped_gemm_dswiglu(d_eo, p["fc2"], offsets, c["h1"])
     else:   # the adapter's input gradient belongs to d_act, in front of the SwiGLU backward

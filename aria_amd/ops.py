@@ -865,13 +865,14 @@ def moe_unpermute(expert_out: torch.Tensor, inv: torch.Tensor, scores: Optional[
     return out
 
 
-def moe_unpermute_bwd(dout: torch.Tensor, expert_out: torch.Tensor, inv: torch.Tensor, scores: torch.Tensor, k: int):
+def moe_unpermute_bwd(dout: torch.Tensor, expert_out: torch.Tensor, inv: torch.Tensor, scores: torch.Tensor, k: int, recent: bool = False):
+    """``recent``: expert_out was computed anew just before, so the caches hold it (the same results)."""
     _chk(dout, name="dout"), _chk(expert_out, name="expert_out"), _chk(scores, name="scores")
     assert dout.is_contiguous() and expert_out.is_contiguous() and scores.is_contiguous()
     T, D = dout.shape
     d_eo = torch.empty_like(expert_out)
     dscores = torch.empty_like(scores)
-    hip.get_lib().call("aria_moe_unpermute_bwd", _p(dout), _p(expert_out), _p(inv), _p(scores), _p(d_eo), _p(dscores), T, D, k,
+    hip.get_lib().call("aria_moe_unpermute_bwd_recent" if recent else "aria_moe_unpermute_bwd", _p(dout), _p(expert_out), _p(inv), _p(scores), _p(d_eo), _p(dscores), T, D, k,
                        _stream(dout))
     return d_eo, dscores
 

@@ -284,6 +284,9 @@ int aria_moe_unpermute_res(const void* expert_out, const int32_t* inv, const voi
  * dscores[t,j] = <expert_out[inv[t,j]], dout[t]> (fp32 reduce, stored bf16). */
 int aria_moe_unpermute_bwd(const void* dout, const void* expert_out, const int32_t* inv, const void* scores,
                            void* d_expert_out, void* dscores, int64_t T, int64_t D, int64_t k, void* stream);
+/* the same for an expert_out that was computed anew just before (layers that recompute), which the caches hold */
+int aria_moe_unpermute_bwd_recent(const void* dout, const void* expert_out, const int32_t* inv, const void* scores,
+                                  void* d_expert_out, void* dscores, int64_t T, int64_t D, int64_t k, void* stream);
 
 /* backward of TopKRouter.routing incl. the training-only auxiliary losses (moe_lm.py:128-166, 203-241,
  * MoEAuxLossAutoScaler :84-125): dlogits[T,E] (bf16) from dscores, z-loss and load-balancing loss.

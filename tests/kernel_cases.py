@@ -433,6 +433,18 @@ def case_unpermute_rows_form(dev, monkeypatch, T):
     assert float((got[2].double() - want[2].double()).norm() / want[2].double().norm()) < 2.0 ** -8
 
 
+def case_unpermute_bwd_recent(dev, T, D, k):
+    """Gradients of rows that were computed anew just before, on both sides of the line from which they are read past the caches too: the same bits."""
+    from aria_amd import ops
+
+    g = torch.Generator().manual_seed(T)
+    inv = torch.randperm(T * k, generator=g).to(torch.int32).to(dev)
+    eo, dout = rnd(T * k, D, seed=1).to(dev), rnd(T, D, seed=3).to(dev)
+    scores = torch.rand(T, k, generator=g).to(bf16).to(dev)
+    for a, b in zip(ops.moe_unpermute_bwd(dout, eo, inv, scores, k, recent=True), ops.moe_unpermute_bwd(dout, eo, inv, scores, k)):
+        assert torch.equal(a, b)
+
+
 def case_layernorm_two_rows_in_flight(dev, T, D):
     """r05b: ``layernorm_fwd2_kernel`` (two rows in flight per wave, compile-time row width; the frozen ViT's LayerNorms) gives the bits of the
     one-row-at-a-time kernel (ARIA_LAYERNORM_V1=1): y, mean, rstd -- odd row counts and rows past the grid's last pair included."""

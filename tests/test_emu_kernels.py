@@ -409,6 +409,11 @@ def test_dispatch_kernels_with_a_compile_time_row_width(T, E, k, D):
     C.case_dispatch_fixed_width(DEV, T, E, k, D)
 
 
+@pytest.mark.parametrize("T,D,k", [(9, 512, 2), (11, 2560, 6), (5, 128, 3)])
+def test_unpermute_bwd_recent(T, D, k):
+    C.case_unpermute_bwd_recent(DEV, T, D, k)
+
+
 @pytest.mark.parametrize("B,S,H,causal,use_len,s_rope", [(2, 70, 2, True, False, None), (1, 300, 1, False, True, 512), (1, 130, 2, True, True, None)])
 def test_attention_backward_with_the_inverse_rope_in_its_epilogue(B, S, H, causal, use_len, s_rope):
     C.case_attention_bwd_rope(DEV, B, S, H, causal, use_len, s_rope)

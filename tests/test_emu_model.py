@@ -223,6 +223,29 @@ def test_training_step_without_permuted_copy(monkeypatch):
     M.case_training_step_without_permuted_copy(DEV, layers=1)
 
 
+@pytest.mark.parametrize("lora", [False, True])
+@pytest.mark.parametrize("level", [None, "moe", "layer"])
+def test_recomputed_expert_rows_are_recent(level, lora, monkeypatch):
+    """The backward of the rows back to tokens is told whether they were computed anew just before (checkpointed layers at either level, adapted ones) or lie in memory."""
+    from aria_amd import ops
+    from aria_amd.lora import apply_lora_from_config
+    from aria_amd.moe_lm import AriaMoELMForCausalLM
+
+    monkeypatch.setenv("ARIA_RECOMPUTE_LEVEL", level or "moe")
+    lm = AriaMoELMForCausalLM(M.make_cfg(dict(hidden_size=128, num_attention_heads=2, num_key_value_heads=2, num_hidden_layers=2, vocab_size=96, moe_intermediate_size=128,
+                                              moe_num_experts=8, moe_topk=2, moe_num_shared_experts=2), gradient_checkpointing=level is not None))
+    with torch.no_grad():
+        for n, p in lm.named_parameters():
+            p.copy_(torch.ones(p.shape) if "norm" in n else (torch.randn(p.shape) * 0.08).to(torch.bfloat16))
+    if lora:
+        apply_lora_from_config(lm, dict(lora_r=8, lora_alpha=32, lora_dropout=0.0, lora_target_modules=["fc1", "fc2", "q_proj", "o_proj"]))
+    told, orig = [], ops.moe_unpermute_bwd
+    monkeypatch.setattr(ops, "moe_unpermute_bwd", lambda *a: (told.append(a[5]), orig(*a))[1])
+    ids = torch.randint(1, 96, (1, 17))
+    lm.train()(input_ids=ids, labels=ids).loss.backward()
+    assert told == [level is not None] * 2
+
+
 def test_adapted_decoder_layer_with_gradient_checkpointing():
     """recipes/config_lora.yaml runs with gradient_checkpointing: the module-by-module decoder layer recomputed in backward gives the same
     loss and the same LoRA gradients as the stored-activation run (dropout off: bit-identical)."""

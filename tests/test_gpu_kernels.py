@@ -442,6 +442,11 @@ def test_unpermute_rows_form(monkeypatch, T):
     C.case_unpermute_rows_form(DEV, monkeypatch, T)
 
 
+@pytest.mark.parametrize("T,D,k", [(1, 2560, 6), (777, 2560, 6), (4915, 2560, 6), (4916, 2560, 6), (70, 512, 2), (33, 128, 3)])
+def test_unpermute_bwd_recent(T, D, k):
+    C.case_unpermute_bwd_recent(DEV, T, D, k)
+
+
 @pytest.mark.parametrize("T,D,k", [(16384, 2560, 6), (70, 512, 2), (33, 128, 3)])
 def test_unpermute_with_the_residual_add_as_its_last_step(T, D, k):
     C.case_unpermute_with_residual(DEV, T, D, k, E=8 if k < 6 else 64)
