@@ -129,7 +129,7 @@ template <bool PAIR, class Ep>
 int launch_expert_rows(const ExpertIn& in, const ExpertLists& lists, int64_t k, int64_t T, const Ep& e, void* stream) {
     const int64_t most = (in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16) * std::min<int64_t>(lists.E, T * k);
     const dim3 grid(unsigned(std::min<int64_t>(512, most)));   // two workgroups a CU are resident
-    const bool once = in.K % 64 == 0 && in.s_ld % 64 == 0;   // (lines that do not straddle rows: rows_once)
+    const bool once = in.s_ld % 64 == 0 && experts_once(lists.E, in.N * (PAIR ? 2 : 1), in.K, 32);
 #define ARIA_ROWS(NW, KS)                                                                                                 \
     {                                                                                                                     \
         if (once)                                                                                                         \

@@ -749,7 +749,7 @@ int aria_launch_gemm4(const GemmParams& p, int a_oc, int b_oc, Gemm4Plan plan, f
     if (plan.form == 2)
         return b_oc ? launch4<false, true, 2, 2, 2, 5, 32, 5, 3, 1>(q, 1, nullptr, stream) : launch4<false, false, 4, 1, 2, 5, 64, 3, 3, 1>(q, 1, nullptr, stream);
     // Weights by expert pass the caches where a tile is the only one of its expert's rows (gemm4_kernel): a stream of 500 MB at 6.9 TB/s for 6.2.  Tensors that the Infinity Cache keeps from one use to
-    // the next lose by it: 16 experts of 1024 x 768 (25 MB) 13.8 us and 16.7.
+    // the next lose by it: 16 experts of 1024 x 768 (25 MB) 13.8 us and 16.7; their pairs (50 MB), held 11.5 and 13.6, in turn with others 15.1 and 15.5.
     const bool once = p.mode == 1 ? p.expert_mod <= 0 && (long long)p.E * p.N * p.K >= 32 << 20 : one_pass(p, 0, b_oc);
 #define ARIA_G4(BOC, VER) launch4<false, BOC, 1, 4, 4, 2, 64, 3, VER, 1>(q, split, slabs, stream)
 #define ARIA_G4E(BOC, VER) \

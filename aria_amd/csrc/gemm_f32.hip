@@ -391,10 +391,13 @@ int launch_f32(const GemmF32& p, void* stream) {
     const int64_t ntn = (int64_t(p.N) + 16 * NT - 1) / (16 * NT);
     if (ntm * ntn > 0x7fffffff) return ARIA_ERR_UNSUPPORTED;
     if constexpr (MT * NT == 1) {
-        // Weights by whole lines, non-temporal (whole_lines): read once, and enough of them or experts'.  Us, half lines / whole: 4 x 32000 x 1024 29.9 / 26.9, 16 40.3 / 35.5, 16 x 64000 x 1536 120 / 99,
-        // 4 x 2816 x 1024 5.7 / 5.4, 4 x 6656 x 2560 19.7 / 17.5; 4 x 1024 x 1024 5.0 / 5.0, 4 x 512 x 256 2.6 / 3.0; 64 experts of 1664 x 2560, 32 rows 86 / 76, 16 of 768 x 1024, 8 rows, that the
-        // Infinity Cache held 8.4 / 8.8 -- in a model's step it does not (four sequences, three layers: 1629 / 1602 with theirs whole too).
-        if (p.K % 32 == 0 && p.ldw % 32 == 0 && p.strideW % 32 == 0 && (p.offsets || (long long)p.N * p.K >= 3 << 19)) {
+        // Weights by whole lines, non-temporal (whole_lines): read once, and enough of them.  Us, half lines / whole: 4 x 32000 x 1024 29.9 / 26.9, 16 40.3 / 35.5, 16 x 64000 x 1536 120 / 99,
+        // 4 x 2816 x 1024 5.7 / 5.4, 4 x 6656 x 2560 19.7 / 17.5; 4 x 1024 x 1024 5.0 / 5.0, 4 x 512 x 256 2.6 / 3.0;
+        // By expert: 64 of 1664 x 2560, 2, 8, 16 rows each 204 / 188, 260 / 212, 334 / 275, a quarter of them with 40 rows and the rest with 2 (several tiles, each of which fetches the weights anew) 334 /
+        // 305; 32 of 1024 x 1536 36.8 / 32.5, 49 / 40, 62 / 53, 62.6 / 58.2.  16 of 768 x 1024 (50 MB), which the Infinity Cache holds: 13.6 / 13.1, 15.0 / 14.6, 16.2 / 16.3, a quarter with 24 and the
+        // rest with 8 16.1 / 16.7, with 40 and 2 18.0 / 18.5: there up to eight rows each on average.
+        if (p.K % 32 == 0 && p.ldw % 32 == 0 && p.strideW % 32 == 0 &&
+            (p.offsets ? p.M <= 8 * p.E || (long long)p.E * p.N * p.K >= 16 << 20 : (long long)p.N * p.K >= 3 << 19)) {
             ARIA_LAUNCH((gemm_f32_kernel<MT, NT, NW, FIN, true>), dim3(unsigned(ntm * ntn)), dim3(NW * 64), 0, stream, p);
             return aria_check_launch();
         }

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void row_kernel(RowsPair rp, E e) {
 // A load takes eight rows' whole cache lines (64 columns), the next one the other eight rows'; the two fragments of 16 rows and 32 columns are these with their halves
 // exchanged between the lanes of a row (whole_lines).  So the weights, which are read once, can be non-temporal: a fragment loaded as it is wanted touches half a line of 16 rows,
 // and the hint then fetches every line twice.  Reading 500 MB: half lines 87 us, non-temporal 104, whole lines 86, non-temporal 77 (6.8 TB/s); 34 MB 8.3, 10.4, 7.9, 7.4.
-// A step left over (KS odd) is a half line that another wave shares: a plain load.  !ONCE: half lines, plain (rows_once).
+// A step left over (KS odd) is a half line that another wave shares: a plain load.  !ONCE: half lines, plain (rows_once, experts_once).
 template <int NW, int MT>
 struct RowsRed {
     float v[2][NW][16 * MT][17];
@@ -320,6 +320,14 @@ inline int rows_parts(int64_t T, int64_t N) { return int(T == 1 ? (N + 7) / 8 : 
 // 15.8 / 14.9.  In several passes (found in the L2): 7680 x 2560, 280 tokens, 37.4 / 38.8.  1024 x 1024, 64 x 2560: 3.15 / 3.26, 4.8 / 4.9; 1000 x 1000 2.7 / 3.4.
 inline bool rows_once(int64_t passes, int64_t N, int64_t K) { return passes == 1 && K % 64 == 0 && N * K >= (3 << 20); }
 
+// Whether weights by expert, E times [N, K] in all, come so: lines that do not straddle rows, and at least `least` Mi weights.  Fewer are still in the Infinity Cache from the use before, which the
+// hint passes by: 32 for a step's few rows, 16 for sorted ones.  A model's steps, 16 experts of 768 x 1024 (pairs 25 M, down 12.6 M), half lines / whole: 4, 8, 16 tokens 151 / 153, 161 / 164, 176 / 179 us; 32 of 1024 x 1536: 238 / 219, 278 /
+// 254, 308 / 276.  Sorted rows, launches in turn, rows an expert: 16 of 768 x 1024, down: 12 9.7 / 10.2, 26 10.4 / 11.5, a quarter of the experts with 100 and the rest with one 15.9 / 17.1, but
+// pairs, whose two tensors are twice as many: 4 11.6 / 11.8, 12 15.2 / 13.5, 26 17.3 / 15.5, 19.9 / 19.8.  An expert of several tiles of rows fetches its weights anew for each, and is ahead or
+// level with it even so: 64 of 1664 x 2560, a quarter of the experts with 80 rows and the rest with 8: pairs 276 / 237, down 146 / 144, with 100 and one 281 / 239, 150 / 143; 32 of 1024 x 1536: 61 /
+// 53, 32.2 / 32.3, 62 / 55, 33.7 / 33.5.  Not where one expert has all rows (26 times 64): 85 / 85, 48.5 / 54.
+inline bool experts_once(int64_t E, int64_t N, int64_t K, int64_t least) { return K % 64 == 0 && E * N * K >= least << 20; }
+
 // Row groups per workgroup: one round of the 256 CUs.  More workgroups read the tokens more often (7680 x 2560, 16 tokens: 240 workgroups 10.4 us, 480
 // 13.1), fewer leave CUs idle (4448 rows: two groups each on 139 workgroups 9.5 us, one each on 278 -- a second, nearly empty round -- 12.1).
 inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std::max<int64_t>(1, (groups * problems + 255) / 256)); }
@@ -417,7 +425,7 @@ int launch_rows_of(const RowsPair& rp, int problems, int64_t T, const E& e, void
     const int per = rows_per_workgroup(groups, problems), other = rp.in[problems - 1].K;
     const int K = std::max(rp.in[0].K, other), least = std::min(rp.in[0].K, other);
     const dim3 grid(unsigned((groups + per - 1) / per), unsigned((T + 15) / 16), unsigned(problems));
-    const bool once = rows_once(grid.y, rp.in[0].N * problems, rp.in[0].K) && other % 64 == 0;
+    const bool once = rows_once(grid.y, rp.in[0].N * problems, rp.in[0].K) && other % 64 == 0;   // (a pair's 2816 x 1024 at 2, 8 tokens, half lines / whole: 5.1 / 5.5, 5.8 / 6.0)
 #define ARIA_ROWS_LONG ARIA_LAUNCH((rows_long_kernel<E, PAIR>), dim3(unsigned(long_groups), grid.y, grid.z), dim3(512), 0, stream, rp, int(T), e);
 #define ARIA_ROWS(NW, KS)                                                                                                     \
     {                                                                                                                         \

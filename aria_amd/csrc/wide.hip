@@ -130,7 +130,7 @@ int launch_sorted_rows(const ExpertRows& in, int64_t M, const Ep& e, void* strea
     const int64_t rows = (M + in.E - 1) / in.E, most = int64_t((in.N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16)) * std::min<int64_t>(in.E, M);
     const int mt = rows_tiles(in.K, 4 * rows);   // (loads differ: tiles for four times the average -- 280 tokens, 26 rows an expert on average, 63 at most)
     const dim3 grid(unsigned(std::min<int64_t>(mt > 2 ? 256 : 512, most)));
-    const bool once = in.K % 64 == 0;   // (lines that do not straddle rows: rows_once)
+    const bool once = experts_once(in.E, in.N * (PAIR ? 2 : 1), in.K, 16);
 #define ARIA_SORTED(KS, MT)                                                                                  \
     if (once)                                                                                                \
         ARIA_LAUNCH((sorted_rows_kernel<KS, MT, Ep, PAIR, true>), grid, dim3(512), 0, stream, in, e);        \

@@ -478,6 +478,23 @@ def case_rows_whole_lines(dev, M, N, K):
 UNEVEN = [[0] * 65 + [40, 0, 16, 1, 17], [33, 0, 1, 24, 0, 2, 0, 0, 4], [0, 65, 1, 129, 0, 64, 2]]
 
 
+def case_experts_whole_lines(dev, E, N, K, pair, counts=(0, 1, 2, 17, 5, 70, 16, 3)):
+    """Sorted rows whose experts' weights come by whole lines, some with several tiles, against one expert after the other by half lines (too few weights for whole ones): the same bits."""
+    from aria_amd import ops
+
+    assert E * N * (1 + pair) * K >= 16 << 20 > 2 * N * K and K % 64 == 0
+    counts = [counts[e % len(counts)] for e in range(E)]
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    x = L.rnd(sum(counts), K, seed=1).to(dev)
+    w, u = (L.rnd(E, N, K, seed=s, scale=K ** -0.5).to(dev) for s in (2, 3))
+    got = ops.rows_experts(x, w, off.to(dev), w_up=u if pair else None)
+    for e, (a, n) in enumerate(zip(off.tolist(), counts)):
+        if n == 0:
+            continue
+        one = ops.rows_experts(x[a:a + n], w[e:e + 1], torch.tensor([0, n], dtype=torch.int32, device=dev), w_up=u[e:e + 1] if pair else None)
+        assert torch.equal(got[a:a + n], one), e
+
+
 def case_rows_qkv(dev, M, D, hd, S):
     """Projection, rotation and cache write in one launch against the separate ones on the same product, bit for bit: positions 0 .. and any slots."""
     from aria_amd import gptfast as G

@@ -74,6 +74,10 @@ def test_rows_whole_lines():
     C.case_rows_whole_lines(DEV, 2, 1894, 1664)
 
 
+def test_experts_whole_lines():
+    C.case_experts_whole_lines(DEV, 16, 512, 1024, True, (1, 0, 0, 18, 0, 0, 0, 0))
+
+
 @pytest.mark.parametrize("counts", C.UNEVEN)
 def test_rows_experts_uneven(counts):
     C.case_rows_experts_uneven(DEV, counts, 20, 136)

@@ -91,6 +91,11 @@ def test_rows_whole_lines(M, N, K):
     C.case_rows_whole_lines(DEV, M, N, K)
 
 
+@pytest.mark.parametrize("E,N,K,pair", [(8, 512, 2048, True), (8, 1024, 2048, False), (16, 600, 1024, True), (9, 1250, 1536, False), (16, 300, 1792, True), (64, 1664, 2560, True)])
+def test_experts_whole_lines(E, N, K, pair):
+    C.case_experts_whole_lines(DEV, E, N, K, pair)
+
+
 @pytest.mark.parametrize("N,K", [(33, 1024), (1664, 2560), (24, 1672)])
 @pytest.mark.parametrize("counts", C.UNEVEN)
 def test_rows_experts_uneven(counts, N, K):
