@@ -29,6 +29,12 @@ def test_dyt_stream_parts(dtype):
     C.case_dyt_stream_parts(DEV, dtype, 5, 136, 5, 1)
 
 
+@pytest.mark.parametrize("dtype,T,D,k,offset", [(bf16, 530, 520, 5, 3), (bf16, 5000, 72, 2, 0), (f32, 4097, 176, 3, 1), (f32, 1400, 520, 5, 2)])
+def test_dyt_stream_eight_columns(dtype, T, D, k, offset):
+    """Beyond the lines at which a lane takes eight columns, and a wave several tokens, in either type."""
+    C.case_dyt_stream_parts(DEV, dtype, T, D, k, offset)
+
+
 @both
 def test_activations(dtype):
     C.case_activations(DEV, dtype)
