@@ -108,9 +108,8 @@ struct RowsRed {
 template <int NW, int KS, int MT, bool ONCE, class WRow, class XRow, class Out>
 __device__ __forceinline__ void stream_rows(int K, const WRow& wrow, const XRow& xrow, int g0, int g1, RowsRed<NW, MT>& red, const Out& out) {
     constexpr int P = KS / 2;                                          // ONCE: pairs of steps, and a left-over one where KS is odd
-    constexpr int SLOTS = ONCE ? KS <= 16 ? P : (P + 1) / 2 : 1;       // pairs in flight: pair p in slot p % SLOTS, in two turns at most
+    constexpr int SLOTS = ONCE ? KS <= 16 ? P : 6 : 1;   // pairs in flight: pair p in slot p % SLOTS (seven of 26 steps: an expert pair's registers spill)
     constexpr int DEPTH = ONCE ? 1 : KS <= 16 ? KS : KS / 2;           // else: fragments in flight
-    static_assert(2 * SLOTS >= P || !ONCE, "two turns");
     static_assert(KS % DEPTH == 0, "a step keeps its register");
     const int t = threadIdx.x, l = t & 63, w = t >> 6, q4 = l >> 4, c16 = l & 15;
     // the last waves' windows are moved down into the row, the columns that another wave owns zeroed in the tokens: every address is base + constant

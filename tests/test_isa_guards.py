@@ -189,3 +189,12 @@ def test_m0_has_its_wait_state(src):
     c = [s for s, _ in code(isa(src))]
     loads = [i for i, s in enumerate(c) if s.startswith("global_load_lds")]
     assert loads and not [i for i in loads if re.match(r"s_\w+ m0,", c[i - 1])]
+
+
+@pytest.mark.parametrize("src", ["batch.hip", "latent.hip"])
+def test_row_streams_stay_in_registers(src):
+    """The windows of a row stream, its weights in flight and the sums together fill most of the registers; none of its kernels may spill, the longest windows of an expert pair included."""
+    held = re.findall(r"\.name:\s+(\S+)\n(?:.*\n)*?\s*\.private_segment_fixed_size:\s*(\d+)", "\n".join(isa(src)))
+    rows = [(n, int(b)) for n, b in held if "rows_kernel" in n]
+    assert any("expert_rows_kernelILi8ELi26E" in n for n, _ in rows)
+    assert [n for n, b in rows if b] == []
