@@ -333,9 +333,13 @@ inline int rows_per_workgroup(int64_t groups, int64_t problems) { return int(std
 
 // stream_rows' shape for a reduction of K columns: CALL(waves, steps per wave).  The steps of a wave are registers (4 a step for the tokens, as many for
 // up to 16 fragments in flight), rounded up to a few values; OTHER runs beyond 6656 columns, and below 128 (a wave's window).
-// One launch, 16 tokens, this form against rows_long_kernel: 100352 x 2560 112 us (4.6 TB/s) against 147, 7680 x 2560 10.4 against 15.8, 2560 x 2560 6.7
-// against 8.9, 6656 x 2560 9.9 against 15.6; at 2 tokens 97 against 117, 9.1 against 10.6, 5.3 against 6.3, 8.5 against 10.4.  What is left beside the
-// 6.1 TB/s of a plain read is the launch itself (about 4 us until the first results) and the tokens' rows from the L2, once per workgroup.
+// One launch, 16 tokens, this form (by whole lines) against rows_long_kernel: 100352 x 2560 87 us (5.9 TB/s) against 147, 7680 x 2560 10.7 against 15.8, 2560 x 2560 7.4
+// against 8.9, 6656 x 2560 10.2 against 15.6; at 2 tokens 76 (6.7 TB/s) against 117, 9.6 against 10.6, 6.1 against 6.3, 9.1 against 10.4.  What is left beside the
+// 6.8 TB/s of a plain non-temporal read is the launch itself (about 4 us until the first results) and the tokens' rows from the L2, once per workgroup.
+// Six steps from 1025 columns on, for the seven of up to 1792, a window of which a sixth lay over another wave's there.  us, seven / six: 4608 x 1536 at 48, 200 tokens 11.4 / 10.2, 17.7 / 15.7,
+// 8192 x 1536 11.8 / 10.8, 23.4 / 20.9, 64000 x 1536 at 2, 16 32.8 / 31.7, 38.9 / 34.5, 32000 x 1536 at 16, 48 20.1 / 19.1, 27.8 / 25.9, 4096 x 1280 at 200 15.6 / 13.8, 5120 x 1088 17.6 / 15.6.
+// Duguzen's steps, 1536 wide, three layers, 2, 4, 8, 16 tokens: 190 / 186, 230 / 222, 265 / 258, 292 / 281.  The waves' sums are other ones with it; a product's error against 64 bits, seven / six
+// steps: 1088 9.1e-8 / 8.7e-8, 1280 9.3e-8 / 9.0e-8, 1536 9.5e-8 / 9.2e-8.
 #define ARIA_ROWS_SHAPE(K, CALL, OTHER) \
     if ((K) < 128)                      \
         OTHER                           \

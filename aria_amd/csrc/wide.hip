@@ -197,7 +197,7 @@ int aria_rows_qkv_rope_cache(const void* X, const void* Wqkv, void* Q, void* Kc,
 // 200 / 187, 28 205 / 192, 40 230 / 199; 32 of 1024 x 1536: 8 33.1 / 34.3, 10 39.2 / 35.0, 20 42.6 / 35.8, 40 48.8 / 36.9.  Fewer weights are a launch's ramp: 16 of 768 x 1024: 12 14.1 / 16.0, 28
 // 15.9 / 17.2, 40 16.4 / 18.3.  Down: 64 experts 6 88.0 / 89.5, 10 89.3 / 90.6, 12 93.8 / 90.7, 16 114 / 92; 32: 8 19.5 / 19.0, 12 23.4 / 19.5; 16: 10 10.5 / 11.4, 16 13.1 / 11.7.
 // A prompt's outputs hold to where the line lay when the tiles were slower, 8 and 4 rows: rows add in another order, which moves an Aria prompt's logits by 0.7 % at the same error against 64 bits.
-// Its four layers by rows up to 27 and 10 rows / by this line: 86 tokens 1706 / 1768, 130 1833 / 1858, 200 1890 / 1932, 240 1926 / 1973, 280 2060 / 2038.
+// Its four layers by rows up to 27 and 10 rows / by this line: 86 tokens 1706 / 1768, 130 1833 / 1858, 200 1890 / 1932, 240 1926 / 1973, 280 2060 / 2038 and, of another draw, 1978 / 2034.
 int64_t aria_rows_experts_most(int64_t E, int64_t N, int64_t K, int which) {
     if (which == ARIA_ROWS_DOWN) return 4 * E;
     return which == ARIA_ROWS_PAIR && E * N * K >= 1 << 25 ? 8 * E : 27 * E;
